@@ -508,6 +508,19 @@ int sgl_amd_extend_attention_ex(const void* q, void* out, const void* k_cache, c
                                 int causal, int kv_fp8, float k_scale, float v_scale, int page_size, int kv_layout_hnd,
                                 int sliding_window, float logit_cap, const void* custom_mask, const int64_t* mask_indptr, int skip_prefix_custom_mask,
                                 void* stream);
+/* Extend attention of a token-major pool (no window, cap or mask) whose longest context (prefix + new tokens) the caller knows: with few
+ * new tokens behind a long one the keys of a request are dealt over `parts` workgroups and their fp32 rows merged.
+ * sgl_amd_extend_attention_parts says how many parts pay (1: none).  For parts > 1 the caller owns ws_acc fp32
+ * [parts, num_tokens, H_q, D] and ws_ml fp32 [parts, num_tokens, H_q, 2]; num_tokens >= qo_indptr[batch]. */
+int sgl_amd_extend_attention_parts(int64_t batch, int max_extend_len, int max_kv_len, int num_q_heads, int num_kv_heads, int head_dim);
+int sgl_amd_extend_attention_kv(const void* q, void* out, const void* k_cache, const void* v_cache,
+                                const int32_t* req_to_token, int64_t req_to_token_stride,
+                                const int64_t* req_pool_indices, const int32_t* seq_lens,
+                                const int32_t* prefix_lens, const int32_t* qo_indptr, int64_t batch, int64_t num_tokens,
+                                int max_extend_len, int max_kv_len, int num_q_heads, int num_kv_heads, int head_dim,
+                                int64_t q_token_stride, int64_t out_token_stride, int64_t cache_row_stride, float sm_scale,
+                                int causal, int kv_fp8, float k_scale, float v_scale, int parts, void* ws_acc, void* ws_ml,
+                                void* stream);
 /* Test / tuning override of the extend kernel's workgroup shape (process-wide; the library never reads the
  * environment): shape 0 = automatic, 41 / 42 / 82 = waves x 16-row tiles per wave (rows per workgroup 64 / 128 / 256);
  * flags bit 0 keeps bf16 8-wave launches on the general single-image kernel, bit 1 sends them to the ping-pong

@@ -70,6 +70,11 @@ struct ExtendParams {
   const int64_t* mask_indptr;
   int mask_skip_prefix;         // the prefix part of the mask is not consulted (extend_attention.py:774 skip_prefix_custom_mask)
   int num_tiles, batch;         // the double-buffered kernel's 1-D grid: query tiles per request, requests
+  // keys split over workgroups (extend_attention_parts_kernel): part i's unnormalised fp32 rows [num_tokens, Hq, D] and (maximum, sum)
+  int parts;
+  int64_t part_rows;            // num_tokens * Hq
+  float* part_acc;
+  float* part_ml;
 };
 
 template <int D>
@@ -883,9 +888,9 @@ __device__ __forceinline__ float lane_pair_max(float x) {         // max over la
 // the products' shadow is the decision (a permlane, two ballots), four LDS writes and the barrier.
 // FP8: the pool holds e4m3 rows (8 bytes per lane and chunk, held raw in the staging registers, widened to bf16 -- exact --
 // on their way into the LDS images; k_scale rides in the softmax scale, v_scale in the epilogue).
-template <int D, int NWV, bool FP8>
-__global__ __launch_bounds__(64 * NWV, 2) void extend_attention_pipe_kernel(ExtendParams p) {
-  __shared__ SmemLadder<D> sm;
+// PARTS: the walk covers part `part` of p.parts equal pieces of the request's key tiles (extend_attention_parts_kernel below).
+template <int D, int NWV, bool FP8, bool PARTS>
+__device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadder<D>& sm) {
   constexpr int CPR = D / 8;            // 16-byte chunks per KV row
   constexpr int KS = D / 16;            // MFMA k-steps over the head dim
   constexpr int ND = D / 32;            // 32-wide output blocks over the head dim
@@ -895,10 +900,11 @@ __global__ __launch_bounds__(64 * NWV, 2) void extend_attention_pipe_kernel(Exte
   constexpr int NPV = ND * 4;           // PV products per tile
 
   // grid -> (query tile, kv head, request): as in the ping-pong kernel (heaviest tiles first, a pair stays on one XCD)
-  int tile, kvh, b;
+  // (with PARTS a pair is a (request, kv head, part): the query tiles that read the same keys)
+  int tile, kvh, b, part = 0;
   {
     const int L = blockIdx.x;
-    const int pairs = p.batch * p.num_kv_heads;
+    const int pairs = p.batch * p.num_kv_heads * (PARTS ? p.parts : 1);
     int pair, rank;
     if (pairs % 8 == 0) {
       const int per_xcd = pairs / 8;
@@ -910,6 +916,10 @@ __global__ __launch_bounds__(64 * NWV, 2) void extend_attention_pipe_kernel(Exte
       rank = L / pairs;
     }
     tile = p.num_tiles - 1 - rank;
+    if constexpr (PARTS) {
+      part = pair % p.parts;
+      pair /= p.parts;
+    }
     kvh = pair % p.num_kv_heads;
     b = pair / p.num_kv_heads;
   }
@@ -929,8 +939,22 @@ __global__ __launch_bounds__(64 * NWV, 2) void extend_attention_pipe_kernel(Exte
   int q1 = q0 + p.tokens_per_tile;
   if (q1 > ext_len) q1 = ext_len;
   const bool causal = p.causal != 0;
-  const int kv_end = causal ? (prefix + q1 < kv_len ? prefix + q1 : kv_len) : kv_len;
-  const int n_tiles = (kv_end + kKvTile - 1) / kKvTile;
+  int kv_end = causal ? (prefix + q1 < kv_len ? prefix + q1 : kv_len) : kv_len;
+  int n_tiles = (kv_end + kKvTile - 1) / kKvTile;
+  // this part's tiles become tiles 0 .. n_tiles - 1 of the walk: the row of the request table, the end and the rows' limits move
+  int part_begin = 0;
+  bool empty = false;
+  if constexpr (PARTS) {
+    const int per = (n_tiles + p.parts - 1) / p.parts;
+    const int t0 = part * per;
+    empty = t0 >= n_tiles;                                 // workgroup-uniform; such a part has no weight (below)
+    if (!empty) {
+      n_tiles = n_tiles - t0 < per ? n_tiles - t0 : per;
+      part_begin = t0 * kKvTile;
+      kv_end -= part_begin;
+      idx_base += part_begin;
+    }
+  }
 
   // ---- this lane's row (both lane halves of a row hold the same query, other head dims / keys) ----
   const int r_row = wid * 32 + l31;
@@ -940,6 +964,17 @@ __global__ __launch_bounds__(64 * NWV, 2) void extend_attention_pipe_kernel(Exte
   int row_limit = row_ok ? (causal ? prefix + q0 + r_tok + 1 : kv_len) : 0;
   if (row_limit > kv_len) row_limit = kv_len;
   const int row_off = (kvh * p.group + r_hg) * D;
+  if constexpr (PARTS) {
+    row_limit -= part_begin;
+    if (empty) {
+      if (row_ok && hi == 0) {
+        float* ml = p.part_ml + 2 * (part * p.part_rows + static_cast<int64_t>(q_begin + q0 + r_tok) * (p.num_kv_heads * p.group) + kvh * p.group + r_hg);
+        ml[0] = kNegBig;
+        ml[1] = 0.f;
+      }
+      return;
+    }
+  }
   U4 qreg[KS];                                      // Q^T operand of k-step s: dims 16 s + 8 h .. + 7 of the row
 #pragma unroll
   for (int s = 0; s < KS; ++s) {
@@ -1253,6 +1288,24 @@ __global__ __launch_bounds__(64 * NWV, 2) void extend_attention_pipe_kernel(Exte
   // c = 1, 3: eight 16-byte stores per lane instead of sixteen 8-byte ones ------------------------------------
   float l = l_run;
   l += __shfl_xor(l, 32, 64);
+  if constexpr (PARTS) {
+    if (p.parts > 1) {                                 // unnormalised rows for extend_merge_kernel
+      if (row_ok) {
+        const int64_t row = part * p.part_rows + static_cast<int64_t>(q_begin + q0 + r_tok) * (p.num_kv_heads * p.group) + kvh * p.group + r_hg;
+        float* acc = p.part_acc + row * D + 4 * hi;
+#pragma unroll
+        for (int n = 0; n < ND; ++n)
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+            *reinterpret_cast<f32x4_t*>(acc + 32 * n + 8 * c) = f32x4_t{ot[n][4 * c], ot[n][4 * c + 1], ot[n][4 * c + 2], ot[n][4 * c + 3]};
+        if (hi == 0) {
+          p.part_ml[2 * row] = m_run;
+          p.part_ml[2 * row + 1] = l;
+        }
+      }
+      return;
+    }
+  }
   const float inv = (l > 0.f) ? p.v_scale / l : 0.f;
   uint16_t* op = p.out + static_cast<int64_t>(q_begin + q0 + r_tok) * p.out_stride + row_off;
 #pragma unroll
@@ -1273,6 +1326,92 @@ __global__ __launch_bounds__(64 * NWV, 2) void extend_attention_pipe_kernel(Exte
       }
     }
   }
+}
+
+template <int D, int NWV, bool FP8>
+__global__ __launch_bounds__(64 * NWV, 2) void extend_attention_pipe_kernel(ExtendParams p) {
+  __shared__ SmemLadder<D> sm;
+  extend_pipe_body<D, NWV, FP8, false>(p, sm);
+}
+
+// The same walk by four waves (128 rows, two workgroups a CU), with a request's key tiles dealt over p.parts workgroups.  Few new tokens
+// behind a long context leave most of the chip idle otherwise, and what runs is a serial chain of tiles.  Each part leaves unnormalised
+// fp32 rows that extend_merge_kernel joins; a single part writes the output itself.
+// Measured (us; general 4-wave kernel -> this one): 203 tokens behind 3800, 32 / 8 heads: 168 -> 37 in four parts; 22 x 3 behind 4549,
+// 32 / 32 heads: 210 -> 52 in four; 1000 cold: 53 -> 27 in one part; 16 x 20 behind 500: 31 -> 19 in one.
+constexpr int kPartWaves = 4;
+
+// How many parts, from what a launch of them costs (us).  A workgroup walks its tiles in about 1.35 us each (1.05 at head dim 64) and
+// pays four more for its first fetches; up to 256 workgroups have a CU alone, two on a CU take 0.65 of the time of one behind the
+// other.  The merge is a launch (5 us), half a microsecond a part, and the parts' fp32 rows through the caches at about 6 TB/s.
+// Against the best of 1, 2, 3, 4, 6, 8 .. 32 parts this picks within 5 % on 20 of 23 measured shapes and within 12 % on the rest.
+int extend_parts(int64_t wgs, int64_t rows, int max_kv_len, int head_dim) {
+  const int tiles = (max_kv_len + kKvTile - 1) / kKvTile;
+  const double tile_us = head_dim == 128 ? 1.35 : 1.05;
+  int best = 1;
+  double best_us = 0;
+  for (int n = 1; n <= 16 && n <= tiles; ++n) {
+    const double per_cu = static_cast<double>((wgs * n + 255) / 256);
+    const double crowd = per_cu > 1 ? 0.65 * per_cu : 1.0;
+    double us = tile_us * ((tiles + n - 1) / n + 4) * crowd;
+    if (n > 1) us += 5.0 + 0.5 * n + static_cast<double>(rows) * n * head_dim * 8.0 / 6e6;
+    if (n == 1 || us < best_us) {
+      best = n;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
+// The 8-wave kernel (256 rows) or the 4-wave one for a launch of one part.  Eight waves ask for half the key rows per flop; four
+// waste fewer rows of a last tile and, two workgroups a CU, leave less of the chip idle in the last round (about 0.3 of a round
+// where eight leave up to a whole one), at 7 % more per round.  Measured at D = 128 (us, eight / four): 60 x 128 behind 896 182 / 197,
+// 6 x 2100 cold, 64 heads 521 / 550, 8 x 300 behind 1000, 32 kv heads 102 / 85, 20 x 300 behind 500 112 / 104.  At D = 64 four waves were
+// never slower (6 x 2000 cold 82 / 76, 4 x 1024 cold 29 / 23).
+bool extend_eight_waves(int64_t wgs8, int64_t wgs4, int head_dim) {
+  if (wgs8 < 256 || head_dim != 128) return false;
+  return static_cast<double>((wgs8 + 255) / 256) <= 1.07 * (static_cast<double>(wgs4) / 512.0 + 0.3);
+}
+
+template <int D, bool FP8>
+__global__ __launch_bounds__(64 * kPartWaves, 2) void extend_attention_parts_kernel(ExtendParams p) {
+  __shared__ SmemLadder<D> sm;
+  extend_pipe_body<D, kPartWaves, FP8, true>(p, sm);
+}
+
+// out = sum_i e^{m_i - m} acc_i / sum_i e^{m_i - m} l_i: a (token, head) row is D / 8 lanes, 8 dims each.  Rows outside the requests'
+// tokens stay untouched; a part without keys for the row (sum 0) is not read.
+template <int D>
+__global__ __launch_bounds__(256) void extend_merge_kernel(ExtendParams p) {
+  constexpr int LPR = D / 8;
+  const int heads = p.num_kv_heads * p.group;
+  const int64_t row = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) / LPR;
+  const int c = threadIdx.x % LPR;
+  const int64_t tok = row / heads;
+  if (row >= p.part_rows || tok < p.qo_indptr[0] || tok >= p.qo_indptr[p.batch]) return;
+  float m = kNegBig;
+  for (int i = 0; i < p.parts; ++i) m = fmaxf(m, p.part_ml[2 * (i * p.part_rows + row)]);
+  float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, l = 0.f;
+  for (int i = 0; i < p.parts; ++i) {
+    const float* ml = p.part_ml + 2 * (i * p.part_rows + row);
+    if (!(ml[1] > 0.f)) continue;
+    const float w = fast_exp2(ml[0] - m);
+    const f32x4_t* a = reinterpret_cast<const f32x4_t*>(p.part_acc + (i * p.part_rows + row) * D + c * 8);
+    const f32x4_t a0 = a[0], a1 = a[1];
+    l += ml[1] * w;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      o[j] += a0[j] * w;
+      o[4 + j] += a1[j] * w;
+    }
+  }
+  const float inv = l > 0.f ? p.v_scale / l : 0.f;
+  U4 w;
+  w.x = pack_bf2(o[0] * inv, o[1] * inv);
+  w.y = pack_bf2(o[2] * inv, o[3] * inv);
+  w.z = pack_bf2(o[4] * inv, o[5] * inv);
+  w.w = pack_bf2(o[6] * inv, o[7] * inv);
+  *reinterpret_cast<U4*>(p.out + tok * p.out_stride + (row - tok * heads) * D + c * 8) = w;
 }
 
 // Test-only probe: C[16x16] = A[16x32] . B[32x16] with the operand/result lane
@@ -1326,7 +1465,7 @@ int sgl_amd_extend_attention(const void* q, void* out, const void* k_cache, cons
                                      0, 1.0f, 1.0f, 1, 0, -1, 0.0f, nullptr, nullptr, 0, stream);
 }
 
-int sgl_amd_extend_attention_ex(const void* q, void* out, const void* k_cache, const void* v_cache,
+static int extend_attention_any(const void* q, void* out, const void* k_cache, const void* v_cache,
                                 const int32_t* req_to_token, int64_t req_to_token_stride,
                                 const int64_t* req_pool_indices, const int32_t* seq_lens,
                                 const int32_t* prefix_lens, const int32_t* qo_indptr, int64_t batch,
@@ -1335,7 +1474,8 @@ int sgl_amd_extend_attention_ex(const void* q, void* out, const void* k_cache, c
                                 int64_t k_cache_row_stride, int64_t v_cache_row_stride, float sm_scale,
                                 int causal, int kv_fp8, float k_scale, float v_scale, int page_size, int kv_layout_hnd,
                                 int sliding_window, float logit_cap, const void* custom_mask, const int64_t* mask_indptr,
-                                int skip_prefix_custom_mask, void* stream) {
+                                int skip_prefix_custom_mask, int64_t num_tokens, int max_kv_len, int parts, void* ws_acc, void* ws_ml, void* stream) {
+
   SGL_CLEAR_STALE_ERROR();
   SGL_CHECK_ARG(k_cache_row_stride == v_cache_row_stride, "extend_attention: K and V pools must share a row stride");
   SGL_CHECK_ARG(!kv_fp8 || (k_scale > 0.f && v_scale > 0.f), "extend_attention: fp8 KV needs positive k_scale / v_scale");
@@ -1350,7 +1490,7 @@ int sgl_amd_extend_attention_ex(const void* q, void* out, const void* k_cache, c
                 "extend_attention: strides must keep 16-byte row alignment");
   SGL_CHECK_ARG(batch <= 65535 && num_kv_heads <= 65535, "extend_attention: grid too large");
   if (batch == 0 || max_extend_len <= 0) return 0;
-  ExtendParams p;
+  ExtendParams p{};
   p.q = static_cast<const uint16_t*>(q);
   p.out = static_cast<uint16_t*>(out);
   p.k_cache = static_cast<const uint16_t*>(k_cache);
@@ -1368,6 +1508,9 @@ int sgl_amd_extend_attention_ex(const void* q, void* out, const void* k_cache, c
   p.num_kv_heads = num_kv_heads;
   p.group = group;
   // Workgroup shape (waves x M-tiles per wave -> rows that share one staged K/V tile):
+  //   32x32 kernels:   token-major pools without window, cap and mask: eight waves or four (extend_eight_waves), four with
+  //                    the keys dealt over workgroups (extend_parts).  Only contexts of one tile are left to the general kernel,
+  //                    whose 64-row workgroups spread them wider (37 cold tokens, 32 heads: 6.1 against 6.7 us);
   //   8 x 2 = 256 rows, two waves per SIMD and the whole register file: fewest K/V gathers per flop; measured
   //                    fastest on MI355X for every shape that gives each CU a workgroup (benchmarks/micro.py);
   //   4 x 1 =  64 rows, 3 workgroups / CU: short extends whose wider grids would leave CUs idle;
@@ -1375,6 +1518,10 @@ int sgl_amd_extend_attention_ex(const void* q, void* out, const void* k_cache, c
   const int64_t rows_total = static_cast<int64_t>(max_extend_len) * group;
   auto wgs = [&](int rows) { return ((rows_total + rows - 1) / rows) * num_kv_heads * batch; };
   int mtw = 2, nwv = 4;
+  // eligible for the 32x32 kernels (flag bit 0, or a forced shape but 8 x 2: the general kernel)
+  const bool plain = !kv_layout_hnd && sliding_window < 0 && logit_cap == 0.f && custom_mask == nullptr && (g_extend_debug_flags & 1) == 0;
+  const bool small = plain && g_extend_debug_shape == 0 && group <= 32 * kPartWaves && out_token_stride % 8 == 0 &&
+                     !extend_eight_waves(wgs(256), wgs(32 * kPartWaves), head_dim) && !(max_kv_len > 0 && max_kv_len <= kKvTile);
   if (group <= 256 && wgs(256) >= 256) { mtw = 2; nwv = 8; }
   else if (group <= 64) { mtw = 1; nwv = 4; }
   if (const int v = g_extend_debug_shape) {                   // sgl_amd_debug_extend_attention_shape(): tests / tuning
@@ -1399,8 +1546,31 @@ int sgl_amd_extend_attention_ex(const void* q, void* out, const void* k_cache, c
   hipStream_t st = as_stream(stream);
   // token-major pools (bf16 or e4m3 rows), 8-wave shape: the 32x32 two-score-set kernel (debug flag bit 1: the bf16
   // ping-pong kernel it replaced)
-  const bool fast = !kv_layout_hnd && nwv == 8 && sliding_window < 0 && logit_cap == 0.f && custom_mask == nullptr &&
-                    (g_extend_debug_flags & 1) == 0 && !(kv_fp8 && (g_extend_debug_flags & 2) != 0);
+  if (small && (g_extend_debug_flags & 2) == 0) {
+    p.tokens_per_tile = 32 * kPartWaves / group;
+    p.num_tiles = (max_extend_len + p.tokens_per_tile - 1) / p.tokens_per_tile;
+    p.batch = static_cast<int>(batch);
+    p.parts = parts > 1 ? parts : 1;
+    p.part_rows = num_tokens * num_q_heads;
+    p.part_acc = static_cast<float*>(ws_acc);
+    p.part_ml = static_cast<float*>(ws_ml);
+    const int64_t blocks = static_cast<int64_t>(p.num_tiles) * num_kv_heads * batch * p.parts;
+    SGL_CHECK_ARG(blocks < (int64_t{1} << 31), "extend_attention: grid too large");
+    const dim3 grid4(static_cast<unsigned>(blocks));
+    if (kv_fp8) {
+      if (head_dim == 128) hipLaunchKernelGGL((extend_attention_parts_kernel<128, true>), grid4, dim3(64 * kPartWaves), 0, st, p);
+      else hipLaunchKernelGGL((extend_attention_parts_kernel<64, true>), grid4, dim3(64 * kPartWaves), 0, st, p);
+    } else if (head_dim == 128) hipLaunchKernelGGL((extend_attention_parts_kernel<128, false>), grid4, dim3(64 * kPartWaves), 0, st, p);
+    else hipLaunchKernelGGL((extend_attention_parts_kernel<64, false>), grid4, dim3(64 * kPartWaves), 0, st, p);
+    if (p.parts > 1) {
+      const dim3 gridm(static_cast<unsigned>((p.part_rows * (head_dim / 8) + 255) / 256));
+      if (head_dim == 128) hipLaunchKernelGGL((extend_merge_kernel<128>), gridm, dim3(256), 0, st, p);
+      else hipLaunchKernelGGL((extend_merge_kernel<64>), gridm, dim3(256), 0, st, p);
+    }
+    SGL_CHECK_LAUNCH("extend_attention");
+    return 0;
+  }
+  const bool fast = plain && nwv == 8 && !(kv_fp8 && (g_extend_debug_flags & 2) != 0);
   if (fast) {
     p.num_tiles = tiles; p.batch = static_cast<int>(batch);
     const dim3 grid1(static_cast<unsigned>(tiles) * num_kv_heads * static_cast<unsigned>(batch));
@@ -1432,6 +1602,52 @@ int sgl_amd_extend_attention_ex(const void* q, void* out, const void* k_cache, c
 #undef SGL_LAUNCH_EXT
   SGL_CHECK_LAUNCH("extend_attention");
   return 0;
+}
+
+int sgl_amd_extend_attention_ex(const void* q, void* out, const void* k_cache, const void* v_cache,
+                                const int32_t* req_to_token, int64_t req_to_token_stride,
+                                const int64_t* req_pool_indices, const int32_t* seq_lens,
+                                const int32_t* prefix_lens, const int32_t* qo_indptr, int64_t batch,
+                                int max_extend_len, int num_q_heads, int num_kv_heads, int head_dim,
+                                int64_t q_token_stride, int64_t out_token_stride,
+                                int64_t k_cache_row_stride, int64_t v_cache_row_stride, float sm_scale,
+                                int causal, int kv_fp8, float k_scale, float v_scale, int page_size, int kv_layout_hnd,
+                                int sliding_window, float logit_cap, const void* custom_mask, const int64_t* mask_indptr,
+                                int skip_prefix_custom_mask, void* stream) {
+  return extend_attention_any(q, out, k_cache, v_cache, req_to_token, req_to_token_stride, req_pool_indices, seq_lens, prefix_lens,
+                              qo_indptr, batch, max_extend_len, num_q_heads, num_kv_heads, head_dim, q_token_stride, out_token_stride,
+                              k_cache_row_stride, v_cache_row_stride, sm_scale, causal, kv_fp8, k_scale, v_scale, page_size, kv_layout_hnd,
+                              sliding_window, logit_cap, custom_mask, mask_indptr, skip_prefix_custom_mask, 0, 0, 1, nullptr, nullptr, stream);
+}
+
+int sgl_amd_extend_attention_parts(int64_t batch, int max_extend_len, int max_kv_len, int num_q_heads, int num_kv_heads, int head_dim) {
+  if (batch <= 0 || max_extend_len <= 0 || max_kv_len <= kKvTile || num_kv_heads <= 0 || num_q_heads % num_kv_heads != 0 ||
+      (head_dim != 64 && head_dim != 128) || num_q_heads / num_kv_heads > 32 * kPartWaves || g_extend_debug_shape != 0 || g_extend_debug_flags != 0)
+    return 1;
+  const int group = num_q_heads / num_kv_heads;
+  auto wgs = [&](int rows) { return ((static_cast<int64_t>(max_extend_len) * group + rows - 1) / rows) * num_kv_heads * batch; };
+  if (extend_eight_waves(wgs(256), wgs(32 * kPartWaves), head_dim)) return 1;
+  const int tokens = 32 * kPartWaves / group;               // whole tokens a tile, as the launch deals them
+  const int64_t wgs4 = static_cast<int64_t>((max_extend_len + tokens - 1) / tokens) * num_kv_heads * batch;
+  return extend_parts(wgs4, batch * static_cast<int64_t>(max_extend_len) * num_q_heads, max_kv_len, head_dim);
+}
+
+int sgl_amd_extend_attention_kv(const void* q, void* out, const void* k_cache, const void* v_cache,
+                                const int32_t* req_to_token, int64_t req_to_token_stride,
+                                const int64_t* req_pool_indices, const int32_t* seq_lens,
+                                const int32_t* prefix_lens, const int32_t* qo_indptr, int64_t batch, int64_t num_tokens,
+                                int max_extend_len, int max_kv_len, int num_q_heads, int num_kv_heads, int head_dim,
+                                int64_t q_token_stride, int64_t out_token_stride, int64_t cache_row_stride, float sm_scale,
+                                int causal, int kv_fp8, float k_scale, float v_scale, int parts, void* ws_acc, void* ws_ml,
+                                void* stream) {
+  SGL_CLEAR_STALE_ERROR();
+  SGL_CHECK_ARG(parts >= 1 && parts <= 64 && (parts == 1 || (ws_acc && ws_ml)), "extend_attention_kv: 1..64 parts, workspaces for more than one");
+  SGL_CHECK_ARG(parts == 1 || (num_kv_heads > 0 && num_q_heads > 0 && num_tokens >= 0 && num_tokens * num_q_heads < (int64_t{1} << 31)),
+                "extend_attention_kv: num_tokens=%lld", static_cast<long long>(num_tokens));
+  return extend_attention_any(q, out, k_cache, v_cache, req_to_token, req_to_token_stride, req_pool_indices, seq_lens, prefix_lens,
+                              qo_indptr, num_tokens == 0 ? 0 : batch, max_extend_len, num_q_heads, num_kv_heads, head_dim, q_token_stride,
+                              out_token_stride, cache_row_stride, cache_row_stride, sm_scale, causal, kv_fp8, k_scale, v_scale, 1, 0, -1, 0.0f,
+                              nullptr, nullptr, 0, num_tokens, max_kv_len, parts, ws_acc, ws_ml, stream);
 }
 
 #ifdef EXT_TRACE

@@ -1,0 +1,47 @@
+"""Extend attention with the keys of a request dealt over workgroups, and the four-wave form of one part."""
+import pytest
+import torch
+
+import oracle.ops as oo
+from sglang_amd import native
+from test_kernels_gpu import BF, _random_case
+
+
+def test_rule_splits_few_rows_behind_long_contexts_only():
+    parts = native.lib().sgl_amd_extend_attention_parts
+    assert parts(1, 203, 4003, 32, 8, 128) > 1 and parts(3, 22, 4571, 32, 32, 128) > 1 and parts(1, 500, 4500, 14, 2, 64) > 1
+    for one in ((60, 128, 1024, 32, 8, 128), (6, 3107, 3107, 64, 8, 128), (1, 37, 37, 14, 2, 64), (1, 512, 512, 32, 8, 128), (1, 203, 0, 32, 8, 128),
+                (0, 5, 500, 32, 8, 128), (1, 5, 500, 32, 8, 96), (1, 5, 5000, 256, 1, 128)):
+        assert parts(*one) == 1, one
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,D,causal", [(32, 8, 128, True), (14, 2, 64, True), (4, 4, 128, True), (64, 1, 64, True), (16, 4, 128, False)])
+def test_parts_against_the_oracle(device, Hq, Hkv, D, causal, fp8):
+    """Walks of no tile, one and many, tile-straddling extends, more parts than a request has tiles, a key that dominates inside one
+    part; rows behind the requests' tokens are left alone.  Bars of the other extend tests; e4m3 rows are compared on their
+    dequantised values."""
+    prefix = [0, 896, 5, 0, 63, 64, 200, 1000] if causal else [0, 0, 0, 0]
+    extend = [130, 128, 1, 333, 65, 64, 7, 70] if causal else [50, 64, 129, 300]
+    c = _random_case(len(prefix), Hq, Hkv, D, prefix, extend, seed=Hq + D + 7, spike=True)
+    c["q"][-3] = (c["k_cache"][c["req_to_token"][c["req_pool_indices"][-1], 3].long(), 0] * 30).to(BF)
+    kc, vc = (x.to(torch.float8_e4m3fn) if fp8 else x for x in (c["k_cache"], c["v_cache"]))
+    ref = oo.extend_attention(c["q"], kc.to(BF), vc.to(BF), c["req_to_token"], c["req_pool_indices"], c["seq_lens"], c["extend_prefix_lens"],
+                              c["extend_seq_lens"], c["scaling"], causal=causal, compute_dtype=torch.float32)
+    T, spare = c["q"].shape[0], 5
+    q = torch.cat([c["q"], torch.zeros(spare, Hq, D, dtype=BF)]).to(device)
+    qo = torch.zeros(len(prefix) + 1, dtype=torch.int32)
+    qo[1:] = torch.cumsum(torch.tensor(extend), 0)
+    kc, vc = ((x.view(torch.uint8) if fp8 else x).to(device) for x in (kc, vc))
+    r2t, pool, seq, pre, qo = (c["req_to_token"].to(device), c["req_pool_indices"].to(device), c["seq_lens"].to(torch.int32).to(device),
+                               torch.tensor(prefix, dtype=torch.int32, device=device), qo.to(device))
+    for parts in (1, 2, 5, 16):
+        out = torch.full_like(q, 7.0)
+        n = (T + spare) * Hq
+        acc, ml = torch.full((parts, n, D), float("nan"), device=device), torch.full((parts, n, 2), float("nan"), device=device)
+        native.call("sgl_amd_extend_attention_kv", q.data_ptr(), out.data_ptr(), kc.data_ptr(), vc.data_ptr(), r2t.data_ptr(), r2t.stride(0), pool.data_ptr(),
+                    seq.data_ptr(), pre.data_ptr(), qo.data_ptr(), len(prefix), T + spare, max(extend), int(seq.max()), Hq, Hkv, D, q.stride(0), out.stride(0),
+                    Hkv * D, c["scaling"], int(causal), int(fp8), 1.0, 1.0, parts, acc.data_ptr(), ml.data_ptr(), torch.cuda.current_stream().cuda_stream)
+        torch.testing.assert_close(out[:T].float().cpu(), ref.float(), atol=4e-3, rtol=1e-2, msg=lambda m: f"{parts} parts: {m}")
+        assert bool((out[T:] == 7.0).all()), parts
