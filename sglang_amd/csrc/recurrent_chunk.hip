@@ -1,5 +1,8 @@
 // Mamba-2, gated-delta-rule and matrix-memory state updates in chunks of 32 tokens, for prefill-sized segments.
 //
+// 16-bit activations whose state dim is at most 128 and whose rows can be read in 16-byte pieces take the kernels of recurrent_split.hpp
+// (the same sums on the bf16 matrix cores); fp32 activations, larger states and unaligned rows are done here.
+//
 // A workgroup owns one (segment, head) and up to 64 value columns (a wave = 16 of them) and walks the segment; the state tile
 // stays in the accumulators of v_mfma_f32_16x16x4_f32 for the whole walk.  Everything is fp32: operands are widened when they
 // are staged, so the recurrence sees no 16-bit rounding beyond its inputs', and bf16 and fp32 models share one body.
@@ -20,6 +23,7 @@
 //             (S | n) = e^{m0-g_n} (S0 | n0) + sum_j e^{a_j-g_n} k_j (v_j | 1)^T,  m = c_n + g_n
 // (I + A)^-1 is formed by forward substitution in 16-token blocks, which stays accurate for repeated keys.
 #include "elem_io.hpp"
+#include "recurrent_split.hpp"
 #include "sglang_amd.h"
 
 using namespace sgl_amd;
@@ -241,6 +245,12 @@ __global__ __launch_bounds__(256, NT <= 8 ? 2 : 1) void mamba2_chunk_kernel(Mamb
       const int n = 16 * t + 4 * g + r;
       if (live && n < p.N) S[static_cast<int64_t>(n) * p.P] = s[t][r];
     }
+}
+
+template <int NU>
+__global__ __launch_bounds__(64 * (kPrepWaves + 4), 2) void mamba2_split_kernel(Mamba2ChunkParams p) {
+  __shared__ __attribute__((aligned(16))) Mamba2Split<NU> sm;
+  mamba2_split_body<Mamba2ChunkParams, NU>(p, sm);
 }
 
 struct DeltaChunkParams {
@@ -485,6 +495,12 @@ __global__ __launch_bounds__(256, NT <= 8 ? 2 : 1) void delta_chunk_kernel(Delta
     }
 }
 
+template <int NU>
+__global__ __launch_bounds__(64 * (kPrepWaves + 4), 2) void delta_split_kernel(DeltaChunkParams p) {
+  __shared__ __attribute__((aligned(16))) DeltaSplit<NU> sm;
+  delta_split_body<DeltaChunkParams, NU>(p, sm);
+}
+
 struct MemoryChunkParams {
   const void *q, *k, *v, *gi, *gf;
   int64_t stride;
@@ -705,6 +721,31 @@ int column_waves(int cols, int64_t segs_heads) {
   return w;
 }
 
+// The same for the split kernels: the preparation is repeated by every workgroup of a head, so columns are dealt over more of them only
+// while the launch stays within one workgroup a compute unit.
+int split_column_waves(int cols, int64_t segs_heads) {
+  int w = (cols + 15) / 16;
+  if (w > 4) w = 4;
+  while (w > 1 && segs_heads * ((cols + 16 * ((w + 1) / 2) - 1) / (16 * ((w + 1) / 2))) <= 256) w = (w + 1) / 2;
+  return w;
+}
+
+void launch_mamba2_split(Mamba2ChunkParams p, int segs, hipStream_t st) {
+  const int w = p.col_waves = split_column_waves(p.P, static_cast<int64_t>(segs) * p.heads);
+  const dim3 grid(p.heads, segs, (p.P + 16 * w - 1) / (16 * w)), block(64 * (kPrepWaves + w));
+  if (p.N <= 32) hipLaunchKernelGGL((mamba2_split_kernel<1>), grid, block, 0, st, p);
+  else if (p.N <= 64) hipLaunchKernelGGL((mamba2_split_kernel<2>), grid, block, 0, st, p);
+  else hipLaunchKernelGGL((mamba2_split_kernel<4>), grid, block, 0, st, p);
+}
+
+void launch_delta_split(DeltaChunkParams p, int segs, hipStream_t st) {
+  const int w = p.col_waves = split_column_waves(p.V, static_cast<int64_t>(segs) * p.heads);
+  const dim3 grid(p.heads, segs, (p.V + 16 * w - 1) / (16 * w)), block(64 * (kPrepWaves + w));
+  if (p.K <= 32) hipLaunchKernelGGL((delta_split_kernel<1>), grid, block, 0, st, p);
+  else if (p.K <= 64) hipLaunchKernelGGL((delta_split_kernel<2>), grid, block, 0, st, p);
+  else hipLaunchKernelGGL((delta_split_kernel<4>), grid, block, 0, st, p);
+}
+
 template <typename T>
 void launch_mamba2_chunk(Mamba2ChunkParams p, int segs, hipStream_t st) {
   const int w = p.col_waves = column_waves(p.P, static_cast<int64_t>(segs) * p.heads);
@@ -757,7 +798,10 @@ int sgl_amd_mamba2_chunk(int is_f32, const void* xbc, int64_t xbc_stride, const 
   const int vec = state_dim % 4 == 0 && xbc_stride % 4 == 0 && (heads * head_dim) % 4 == 0 && aligned_to(xbc, al);
   Mamba2ChunkParams p{xbc, xbc_stride, dt, dt_stride, A_log, dt_bias, D, state, slots, positions, seg_start, seg_len, y, y_stride,
                       heads, head_dim, state_dim, groups, vec, 0};
+  const bool split = !is_f32 && state_dim <= 128 && state_dim % 8 == 0 && head_dim % 8 == 0 && xbc_stride % 8 == 0 && xbc_stride < (1 << 24) && aligned_to(xbc, 16) &&
+                     y_stride % 4 == 0 && aligned_to(y, 8);
   if (is_f32) launch_mamba2_chunk<float>(p, segments, as_stream(stream));
+  else if (split) launch_mamba2_split(p, segments, as_stream(stream));
   else launch_mamba2_chunk<uint16_t>(p, segments, as_stream(stream));
   SGL_CHECK_LAUNCH("mamba2_chunk");
   return 0;
@@ -776,7 +820,10 @@ int sgl_amd_delta_chunk(int is_f32, const void* qkv, int64_t qkv_stride, const v
   const int vec = key_dim % 4 == 0 && qkv_stride % 4 == 0 && aligned_to(qkv, al);
   DeltaChunkParams p{qkv, qkv_stride, b, a, ba_stride, A_log, dt_bias, state, slots, positions, seg_start, seg_len, o, o_stride,
                      heads, kv_heads, key_dim, value_dim, vec, 0, q_scale};
+  const bool split = !is_f32 && key_dim <= 128 && key_dim % 8 == 0 && value_dim % 8 == 0 && qkv_stride % 8 == 0 && qkv_stride < (1 << 24) &&
+                     aligned_to(qkv, 16) && o_stride % 4 == 0 && aligned_to(o, 8);
   if (is_f32) launch_delta_chunk<float>(p, segments, as_stream(stream));
+  else if (split) launch_delta_split(p, segments, as_stream(stream));
   else launch_delta_chunk<uint16_t>(p, segments, as_stream(stream));
   SGL_CHECK_LAUNCH("delta_chunk");
   return 0;
