@@ -1365,12 +1365,13 @@ int extend_parts(int64_t wgs, int64_t rows, int max_kv_len, int head_dim) {
 
 // The 8-wave kernel (256 rows) or the 4-wave one for a launch of one part.  Eight waves ask for half the key rows per flop; four
 // waste fewer rows of a last tile and, two workgroups a CU, leave less of the chip idle in the last round (about 0.3 of a round
-// where eight leave up to a whole one), at 7 % more per round.  Measured at D = 128 (us, eight / four): 60 x 128 behind 896 182 / 197,
-// 6 x 2100 cold, 64 heads 521 / 550, 8 x 300 behind 1000, 32 kv heads 102 / 85, 20 x 300 behind 500 112 / 104.  At D = 64 four waves were
-// never slower (6 x 2000 cold 82 / 76, 4 x 1024 cold 29 / 23).
+// where eight leave up to a whole one), at 7 % more per round.  Past two rounds the key rows decide (44 ragged extends of 122 behind 1874
+// 289 / 302 us, 60 x 128 behind 896 182 / 197), unless the second half of a 256-row tile would be empty anyway (64 x 20 behind 3000 231 / 161).
+// Below (us, eight / four): 5 x 600 behind 1000 92 / 87, 8 x 300 behind 1000, 32 kv heads 102 / 85, 4 x 1024 cold 52 / 54.  At D = 64 four
+// waves were never slower (6 x 2000 cold 82 / 76, 4 x 1024 cold 29 / 23).
 bool extend_eight_waves(int64_t wgs8, int64_t wgs4, int head_dim) {
-  if (wgs8 < 256 || head_dim != 128) return false;
-  return static_cast<double>((wgs8 + 255) / 256) <= 1.07 * (static_cast<double>(wgs4) / 512.0 + 0.3);
+  if (wgs8 < 256 || head_dim != 128 || wgs4 * 4 <= wgs8 * 5) return false;
+  return wgs8 > 512 || static_cast<double>((wgs8 + 255) / 256) <= 1.07 * (static_cast<double>(wgs4) / 512.0 + 0.3);
 }
 
 template <int D, bool FP8>
