@@ -172,7 +172,8 @@ int sgl_amd_extend_attention(const void* q, void* out, const void* k_cache, cons
  * groups such requests; sgl_amd_cascade_decode_attention (per layer, two launches) cuts every group's
  * shared prefix and every request's private suffix into sgl_amd_cascade_chunk_tokens()-token items,
  * reads each item's K/V rows once for all its member requests (MFMA), and merges the per-item
- * partials of a (request, head) in slot order (deterministic).
+ * partials of a (request, head) in slot order (deterministic).  Behind large request tables the private
+ * tokens of the whole batch are cut into equal spans instead, one a resident workgroup.
  * plan: int32[sgl_amd_cascade_plan_ints(batch, max_items)]; ws_acc fp32 [B,Hq,slots_total,D], ws_ml fp32
  * [B,Hq,slots_total,2] with slots_total >= ceil(max_context_len / chunk) + 1; head_dim 64 or 128. */
 int sgl_amd_cascade_chunk_tokens(void);
@@ -529,7 +530,9 @@ int sgl_amd_debug_extend_attention_shape(int shape, int flags);
 /* Test / tuning override of the shared-prefix chunk kernel's launch form (process-wide; the library never reads the
  * environment).  A launch whose worst-case workgroup count (from the request table's width) is <= single_shot_units runs one
  * workgroup per (item, kv head) unit; above it a grid of loop_grid resident workgroups walks the device-built item list.
- * 0 restores a default (10240 / 1280).  Results are identical in both forms.  Not part of the reference surface. */
+ * 0 restores a default (10240 / 1280).  The switch can lower the line at which the looping form begins, not raise it: above the
+ * default one (2048 for at most 8 query heads a kv head and tables of 8 k tokens or more) the plan may cut the private tokens into
+ * spans, which only the looping form walks.  Not part of the reference surface. */
 int sgl_amd_debug_cascade_launch_form(int64_t single_shot_units, int64_t loop_grid);
 /* Test / tuning switch of the weight-streaming GEMM (process-wide; the library never reads the environment): bit 1 = the fp32
  * split-K partials are stored with plain write-back stores instead of write-through ones (the default since round 6:

@@ -39,7 +39,15 @@ constexpr float kNegBig = -1.0e30f;
 // launch-form policy of the chunk kernel (see cascade_chunk_kernel); process-wide tuning knobs behind
 // sgl_amd_debug_cascade_launch_form, like the extend kernel's shape switch
 constexpr int64_t kSingleShotHardCap = 16384;    // the largest value the switch below may take: what the plan clears for is decided against THIS, not the switch
-int64_t g_cascade_single_shot_units = 10240;   // worst-case workgroups up to which the one-workgroup-per-unit form is launched
+constexpr int64_t kSingleShotUnits = 10240;
+// ... and for requests of at most 8 query rows a kv head behind tables of at least kSpanChunks chunks, whose private tokens the plan cuts into
+// spans: the looping form.  us a layer, Llama-3-8B heads, single-shot against spans, at an 8 k-token table: 8 requests of 5 k 57 / 54, 16 of
+// 4 k 77 / 73, 2 of 7 k 25.0 / 24.0; 4 of 17 k at a 32 k-token table 82.8 / 64.6.  At tables of 1.2 and 2.5 k tokens, whose requests are
+// short: 64 of 0.9 k 51.9 / 53.1, 64 behind a shared prefix 22.5 / 23.5, 32 of 0.3 k 15.8 / 17.9.
+constexpr int64_t kSpanSingleShotUnits = 2048;
+constexpr int kSpanChunks = 64;
+inline int64_t single_shot_most(int chunks, int group) { return group <= 8 && chunks >= kSpanChunks ? kSpanSingleShotUnits : kSingleShotUnits; }
+int64_t g_cascade_single_shot_units = kSingleShotUnits;   // worst-case workgroups up to which the one-workgroup-per-unit form is launched
 int64_t g_cascade_loop_grid = 256 * 5;         // grid of the looping form: 1280 beat 1024 (= what is resident at four per CU) and equalled 2048
 
 __device__ __forceinline__ bf16x8_t as_frag(const U4& v) { return __builtin_bit_cast(bf16x8_t, v); }
@@ -87,7 +95,8 @@ struct ChunkParams {
 //   cascade_chunk_loop_kernel: a grid of kLoopGrid resident workgroups walks the list -- workgroup w takes units w, 2 G - 1 - w, 2 G + w,
 //     ... (a snake over the passes: the shared items at the head of the list are the heavy ones, the workgroups that got
 //     them in one pass get the far end of the next) below the list's end, which every workgroup knows after ONE scalar load
-//     (header[0]) that travels with its first item record.  Chosen for large request tables: the worst case of a 64-request
+//     (header[5]) that travels with its first item record.  Where the plan has cut the private tokens into spans, a unit behind the shared
+//     items is one span, piece by piece.  Chosen for large request tables: the worst case of a 64-request
 //     batch is 58 k workgroups at an 8 k-token table (Llama-3-8B's own context length under the reference's scheduler), ~1 M at
 //     128 k, and a workgroup behind the list's end costs ~0.25 ns of dispatch -- 20 -> 33.7 us per layer at 8 k, measured
 //     under the reference's scheduler (profiles/r05_sched_step_timeline_hooks.txt).  The loop keeps the thread index and the
@@ -111,13 +120,192 @@ __device__ __forceinline__ void cascade_chunk_unit(const ChunkParams& p, U4* sm,
 #include "cascade_chunk_body.inc"
 }
 
+// max over the four 16-lane rows of a wave (inline asm: with the builtin on two copies of one value hipcc kept only the first result)
+__device__ __forceinline__ float lane_rows_max(float x) {
+  float a = x, b = x;
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+  a = fmaxf(a, b);
+  b = a;
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+  return fmaxf(a, b);
+}
+
+// A unit of at most 8 query rows (a piece of a span; an e4m3 item of few members) in the looping kernel: any number of tokens, wave w
+// takes the 16-token tiles w, w + 4, ...  No barrier until the waves' (max, sum, O) sets meet: K rows are the matrix operand as they
+// come (lane = token, four lanes a row), V rows pass through the wave's own 4 KiB image and come out transposed by
+// ds_read_b64_tr_b16.  The next tile's K rows are asked for once this tile's scores are formed, its V rows once this tile's have left
+// the registers, so a wave always has rows in flight; sixteen waves a CU do the rest (16 tokens, not 32: at 32 the 128 registers spill,
+// 256 against 211 us for 32 requests of 2 k tokens in e4m3).
+// What bounds it: the gathered rows -- four layers of 37 requests of 0.9 to 5.1 k tokens in e4m3 481 -> 296 us (2.0 -> 3.3 TB/s), 128
+// requests of 1.5 k in bf16 910 -> 709 us (4.8 TB/s; a large copy reaches 4.9).  Before, a unit was 128 tokens staged through one image
+// behind six barriers.  A bf16 item of 128 tokens keeps that form: its rows come in one burst, 257 against 265 us in the shared-prefix batch.
+// Image: row (token) t at t * 2 D bytes, its 16-byte piece c in slot c ^ kSw(t): the four rows of a transposing read lie on distinct banks.
+template <int D, bool FP8, bool HND>
+__device__ __forceinline__ void cascade_few_rows_unit(const ChunkParams& p, U4* sm, float* ml_s, const int32_t* rec, const int kvh, const int tid) {
+  const int4 ra = *reinterpret_cast<const int4*>(rec), rb = *reinterpret_cast<const int4*>(rec + 4);
+  constexpr int KC = D / 32, ND = D / 16;
+  constexpr int KL = FP8 ? D / 64 : D / 32;                    // 16-byte pieces of a K row a lane holds
+  constexpr int VL = FP8 ? D / 64 : D / 32;                    // ... of the 16 V rows
+  constexpr int VPR = FP8 ? D / 16 : D / 8;                    // lanes a V row
+  typedef short v4s16_t __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) v4s16_t* lds_v4_t;
+  auto swz = [](int t) __attribute__((always_inline)) { return D == 128 ? 2 * (t & 3) : 2 * ((t >> 1) & 3); };
+  const CascadePlanView pv = cascade_plan_view(p.plan, p.batch, p.max_items);
+  const int lane = tid & 63, wid = tid >> 6, i16 = lane & 15, g = lane >> 4;
+  const int slot = __builtin_amdgcn_readfirstlane(ra.x), kv_begin = __builtin_amdgcn_readfirstlane(ra.y), kv_n = __builtin_amdgcn_readfirstlane(ra.z);
+  const int n_rows = __builtin_amdgcn_readfirstlane(ra.w) * p.group;
+  const int rec_x = __builtin_amdgcn_readfirstlane(rb.x), rec_private = __builtin_amdgcn_readfirstlane(rb.y);
+  const int32_t* idx_base = p.req_to_token + static_cast<int64_t>(__builtin_amdgcn_readfirstlane(rb.z)) * p.r2t_stride + kv_begin;
+  const int tiles = (kv_n + 15) / 16;
+  auto slot_id = [&](int t) __attribute__((always_inline)) {   // of token lane & 15 of tile t
+    const int tok = 16 * t + i16;
+    return idx_base[tok < kv_n ? tok : kv_n - 1];
+  };
+  int ids = wid < tiles ? slot_id(wid) : 0;
+  // ---- this lane's query row ----
+  const int mem_i = i16 / p.group, hg = i16 - mem_i * p.group;
+  const bool row_ok = i16 < n_rows;
+  int req = rec_x;
+  if (row_ok && !rec_private) req = pv.member_rows[rec_x + mem_i];
+  U4 qf[KC];
+#pragma unroll
+  for (int kc = 0; kc < KC; ++kc) qf[kc] = U4{0u, 0u, 0u, 0u};
+  if (row_ok) {
+    const uint16_t* qp = p.q + static_cast<int64_t>(req) * p.q_stride + (kvh * p.group + hg) * D;
+#pragma unroll
+    for (int kc = 0; kc < KC; ++kc) qf[kc] = ld16(qp + (FP8 ? (kc >> 1) * 64 + g * 16 + (kc & 1) * 8 : kc * 32 + g * 8));
+  }
+  const uint32_t row_bytes = p.fmt.page_stride;
+  const unsigned char* k_rows = reinterpret_cast<const unsigned char*>(p.k_cache) + static_cast<uint32_t>(kvh) * p.fmt.head_stride;
+  const unsigned char* v_rows = reinterpret_cast<const unsigned char*>(p.v_cache) + static_cast<uint32_t>(kvh) * p.fmt.head_stride;
+  auto row_at = [&](const unsigned char* rows, const void* pool, int id) __attribute__((always_inline)) {
+    if constexpr (HND) return kv_row(pool, p.fmt, id, kvh);
+    else return rows + static_cast<uint64_t>(static_cast<uint32_t>(id)) * row_bytes;
+  };
+  U4 kr[KL], vr[VL];
+  auto load_k = [&](int id) __attribute__((always_inline)) {
+    const unsigned char* row = row_at(k_rows, p.k_cache, id) + g * 16;
+#pragma unroll
+    for (int c = 0; c < KL; ++c) kr[c] = ld16(row + 64 * c);
+  };
+  auto load_v = [&](int id) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < VL; ++i) vr[i] = ld16(row_at(v_rows, p.v_cache, __shfl(id, lane / VPR + (64 / VPR) * i, 64)) + lane % VPR * 16);
+  };
+  f32x4_t ot[ND];
+#pragma unroll
+  for (int n = 0; n < ND; ++n) ot[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m_run = kNegBig, l_run = 0.f;                          // l: this lane's tokens
+  unsigned char* img = reinterpret_cast<unsigned char*>(sm) + wid * 4096;
+  auto put_v = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < VL; ++i) {
+      const int t = lane / VPR + (64 / VPR) * i, c = lane % VPR, sw = swz(t);
+      if constexpr (FP8) {
+        *reinterpret_cast<U4*>(img + t * (2 * D) + ((2 * c) ^ sw) * 16) = fp8x8_to_bf16x8(uint2{vr[i].x, vr[i].y});
+        *reinterpret_cast<U4*>(img + t * (2 * D) + ((2 * c + 1) ^ sw) * 16) = fp8x8_to_bf16x8(uint2{vr[i].z, vr[i].w});
+      } else {
+        *reinterpret_cast<U4*>(img + t * (2 * D) + (c ^ sw) * 16) = vr[i];
+      }
+    }
+  };
+  const int vrow = 4 * g + (i16 >> 2), vsw = swz(vrow);
+  const unsigned char* vlane = img + vrow * (2 * D) + ((i16 >> 1) & 1) * 16 + (i16 & 1) * 8;
+  if (wid < tiles) {
+    load_k(ids);
+    load_v(ids);
+  }
+  for (int t = wid; t < tiles; t += 4) {
+    const bool more = t + 4 < tiles;                           // (wave-uniform)
+    if (more) ids = slot_id(t + 4);
+    // ---- S^T: lane holds row i16, tokens 4 g + r ----
+    f32x4_t st = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kc = 0; kc < KC; ++kc) {
+      U4 kf;
+      if constexpr (FP8) {
+        const U4 w = kr[kc >> 1];
+        kf = (kc & 1) ? fp8x8_to_bf16x8(uint2{w.z, w.w}) : fp8x8_to_bf16x8(uint2{w.x, w.y});
+      } else {
+        kf = kr[kc];
+      }
+      st = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(kf), as_frag(qf[kc]), st, 0, 0, 0);
+    }
+    if (more) load_k(ids);
+    // ---- running softmax ----
+    float mx = kNegBig;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      st[r] = 16 * t + 4 * g + r < kv_n ? st[r] * p.scale_log2 : kNegBig;
+      mx = fmaxf(mx, st[r]);
+    }
+    mx = lane_rows_max(mx);
+    if (__ballot(mx > m_run) != 0ull) {
+      const float m_new = fmaxf(m_run, mx), alpha = fast_exp2(m_run - m_new);
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int n = 0; n < ND; ++n) ot[n] *= alpha;
+    }
+    float e[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      e[r] = st[r] > 0.5f * kNegBig ? fast_exp2(st[r] - m_run) : 0.f;
+      l_run += e[r];
+    }
+    const v4s16_t pf = __builtin_bit_cast(v4s16_t, uint2{pack_bf2(e[0], e[1]), pack_bf2(e[2], e[3])});
+    // ---- O^T += V^T P^T (the wave's own image: its LDS accesses complete in order) ----
+    put_v();
+    if (more) load_v(ids);
+#pragma unroll
+    for (int n = 0; n < ND; ++n) {
+      const v4s16_t vf = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4_t)(vlane + ((2 * n) ^ vsw) * 16));
+      ot[n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vf, pf, ot[n], 0, 0, 0);
+    }
+  }
+  // ---- the four waves' sets meet, each in its own image as [row < 8][dim] (another wave may still read its own) ----
+  l_run += __shfl_xor(l_run, 16, 64);
+  l_run += __shfl_xor(l_run, 32, 64);
+  if (i16 < 8) {
+#pragma unroll
+    for (int n = 0; n < ND; ++n) sm[wid * 256 + i16 * (D / 4) + 4 * n + g] = __builtin_bit_cast(U4, ot[n]);
+    if (g == 0) { ml_s[(wid * 8 + i16) * 2] = m_run; ml_s[(wid * 8 + i16) * 2 + 1] = l_run; }
+  }
+  __syncthreads();
+  constexpr int PER_ROW = D / 4;
+  const int row = tid / PER_ROW, dq = tid - row * PER_ROW;
+  if (row < n_rows) {
+    float big = kNegBig;
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+      if (ml_s[(w * 8 + row) * 2 + 1] > 0.f) big = fmaxf(big, ml_s[(w * 8 + row) * 2]);
+    f32x4_t o = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    float l = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float lw = ml_s[(w * 8 + row) * 2 + 1], sc = lw > 0.f ? fast_exp2(ml_s[(w * 8 + row) * 2] - big) : 0.f;
+      o += __builtin_bit_cast(f32x4_t, sm[w * 256 + row * PER_ROW + dq]) * sc;
+      l += lw * sc;
+    }
+    const int mi = row / p.group;
+    const int rq = rec_private ? rec_x : pv.member_rows[rec_x + mi];
+    const int64_t sl = static_cast<int64_t>(rq * p.num_q_heads + kvh * p.group + (row - mi * p.group)) * p.slots_total + slot;
+    *reinterpret_cast<f32x4_t*>(p.ws_acc + sl * D + dq * 4) = o;
+    if (dq == 0) {
+      p.ws_ml[sl * 2 + 0] = big;
+      p.ws_ml[sl * 2 + 1] = l;
+    }
+  }
+}
+
 template <int D, bool FP8, bool HND>
 __global__ __launch_bounds__(kThreads, 4) void cascade_chunk_loop_kernel(ChunkParams p) {
   __shared__ U4 sm[(kChunk / (D > 64 ? D / 64 : 1)) * (D / 8)];
   __shared__ float ml_s[64];
   __shared__ U4 side_s[D > 64 ? 4 * 8 * (D - 64) / 4 : 1];
-  int n_items = __builtin_amdgcn_readfirstlane(p.plan[0]);                   // header[0]: the list's length
-  if (n_items > p.max_items) n_items = p.max_items;
+  // one hop for all of the header that the loop needs: the list's length (shared items, then private items or spans) and what the tail is
+  const int n_items = __builtin_amdgcn_readfirstlane(p.plan[5]), n_shared = __builtin_amdgcn_readfirstlane(p.plan[3]);
+  const bool spans = __builtin_amdgcn_readfirstlane(p.plan[4]) > 0;
   const int n_units = n_items * p.num_kv_heads;
   const int G = static_cast<int>(gridDim.x), w0 = static_cast<int>(blockIdx.x);
   // The kernel's one argument sits at the start of the kernarg segment; every pass re-reads it through an address the
@@ -125,22 +313,36 @@ __global__ __launch_bounds__(kThreads, 4) void cascade_chunk_loop_kernel(ChunkPa
   // thread index as an opaque value.
   typedef const __attribute__((address_space(4))) uint64_t KernargWord;
   const uint64_t kp = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
-  for (int base = 0, pass = 0; base < n_units; base += G, ++pass) {
+  int next = 0;                                                               // > 0: the next piece of a span begun before
+  for (int base = 0, pass = 0; base < n_units;) {
     const int unit = base + ((pass & 1) ? G - 1 - w0 : w0);
-    if (unit < n_units) {                                                     // (workgroup-uniform; false only in the last pass)
-      uint64_t ka = kp;
-      asm volatile("" : "+s"(ka));
-      KernargWord* kw = reinterpret_cast<KernargWord*>(ka);
-      static_assert(sizeof(ChunkParams) % 8 == 0 && std::is_trivially_copyable<ChunkParams>::value, "kernarg image copied as 8-byte words");
-      struct Raw { uint64_t w[sizeof(ChunkParams) / 8]; } raw;
+    if (unit >= n_units) break;                                               // (workgroup-uniform; only in the last pass)
+    uint64_t ka = kp;
+    asm volatile("" : "+s"(ka));
+    KernargWord* kw = reinterpret_cast<KernargWord*>(ka);
+    static_assert(sizeof(ChunkParams) % 8 == 0 && std::is_trivially_copyable<ChunkParams>::value, "kernarg image copied as 8-byte words");
+    struct Raw { uint64_t w[sizeof(ChunkParams) / 8]; } raw;
 #pragma unroll
-      for (unsigned i = 0; i < sizeof(ChunkParams) / 8; ++i) raw.w[i] = kw[i];
-      const ChunkParams pl = __builtin_bit_cast(ChunkParams, raw);
-      int tid = threadIdx.x;
-      asm volatile("" : "+v"(tid));
-      cascade_chunk_unit<D, FP8, HND>(pl, sm, ml_s, side_s, unit, tid);
-      __syncthreads();                                                        // the image is reused by the next unit
+    for (unsigned i = 0; i < sizeof(ChunkParams) / 8; ++i) raw.w[i] = kw[i];
+    const ChunkParams pl = __builtin_bit_cast(ChunkParams, raw);
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int item = unit / pl.num_kv_heads, kvh = unit - item * pl.num_kv_heads;
+    const CascadePlanView pv = cascade_plan_view(pl.plan, pl.batch, pl.max_items);
+    const int span = item - n_shared;
+    const bool in_span = spans && span >= 0;                                  // (workgroup-uniform)
+    const int32_t* rec = pv.items + 8 * item;
+    if (in_span) {
+      const int i = next > 0 ? next : __builtin_amdgcn_readfirstlane(pv.span_first[span]);
+      rec = pv.pieces + 8 * i;
+      next = i + 1 < __builtin_amdgcn_readfirstlane(pv.span_first[span + 1]) ? i + 1 : 0;
     }
+    if (in_span || (FP8 && __builtin_amdgcn_readfirstlane(rec[3]) * pl.group <= 8))
+      cascade_few_rows_unit<D, FP8, HND>(pl, sm, ml_s, rec, kvh, tid);
+    else
+      cascade_chunk_unit<D, FP8, HND>(pl, sm, ml_s, side_s, unit, tid);
+    __syncthreads();                                                          // the image is reused by the next unit
+    if (next == 0) { base += G; ++pass; }
   }
 }
 
@@ -220,19 +422,19 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_compare_kernel(
 __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
     const int32_t* __restrict__ req_to_token, int64_t r2t_stride, const int64_t* __restrict__ req_pool_indices,
     const int32_t* __restrict__ seq_lens, int batch, int min_shared, int chunk_tokens, int tokens_per_tile,
-    int kv_tile, int max_shared, int32_t* __restrict__ plan, int max_items, int zero_items) {
+    int kv_tile, int max_shared, int32_t* __restrict__ plan, int max_items, int zero_items, int num_kv_heads, int span_units) {
   __shared__ int first_slot[kPlanMaxBatch];
   __shared__ int leader[kPlanMaxBatch];
   __shared__ int grp_min[kPlanMaxBatch];
   __shared__ int grp_cnt[kPlanMaxBatch];
   __shared__ int grp_id[kPlanMaxBatch];
-  __shared__ int scan[kPlanMaxBatch];
+  __shared__ __align__(16) int scan[kPlanMaxBatch];
   __shared__ int order[kPlanMaxBatch];
   __shared__ int g_leader[kPlanMaxBatch / 2], g_kv[kPlanMaxBatch / 2], g_first[kPlanMaxBatch / 2], g_tiles[kPlanMaxBatch / 2],
       g_rows0[kPlanMaxBatch / 2], g_members[kPlanMaxBatch / 2];
   __shared__ int n_shared_items, n_groups, n_rows;
   __shared__ int pool_row[kPlanMaxBatch], len_s[kPlanMaxBatch];   // read once: every later phase would pay the hop again
-  __shared__ int wave_tot[kPlanThreads / 64];
+  __shared__ int wave_tot[kPlanThreads / 64], wave_tiles[kPlanThreads / 64];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const CascadePlanView pv = cascade_plan_view(plan, batch, max_items);
   // members == 0 marks the end of the list for the one-workgroup-per-unit chunk kernel, whose grid never reaches beyond
@@ -308,20 +510,19 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
   }
   __syncthreads();
   // (3) members in batch order inside each group, then the ungrouped requests: a request's place is the number of
-  // earlier requests of its kind.
-  {
-    const int rows_total = n_rows;
-    int my_pos[ (kPlanMaxBatch + kPlanThreads - 1) / kPlanThreads ];
-    int k = 0;
-    for (int b = tid; b < batch; b += kPlanThreads, ++k) {
-      const int gi = grp_id[leader[b]];
-      int rank = 0;
-      for (int c = 0; c < b; ++c) rank += (grp_id[leader[c]] == gi) ? 1 : 0;   // gi < 0: all ungrouped count together
-      my_pos[k] = gi >= 0 ? g_rows0[gi] + rank : rows_total + rank;
+  // earlier requests of its kind.  (The kinds go through `scan`, dead since pass (2), so that the count is a row of independent
+  // 16-byte reads: two dependent LDS hops a request were 3 of the kernel's 9 us at 64 requests.)
+  for (int b = tid; b < batch; b += kPlanThreads) scan[b] = grp_id[leader[b]];
+  __syncthreads();
+  for (int b = tid; b < batch; b += kPlanThreads) {
+    const int gi = scan[b];
+    int rank = 0;                                      // gi < 0: all ungrouped count together
+#pragma unroll 4
+    for (int c = 0; c < b; c += 4) {
+      const int4 v = *reinterpret_cast<const int4*>(scan + c);
+      rank += (v.x == gi ? 1 : 0) + (c + 1 < b && v.y == gi ? 1 : 0) + (c + 2 < b && v.z == gi ? 1 : 0) + (c + 3 < b && v.w == gi ? 1 : 0);
     }
-    __syncthreads();                                   // `order` was scratch of pass (1)/(2) until here
-    k = 0;
-    for (int b = tid; b < batch; b += kPlanThreads, ++k) order[my_pos[k]] = b;
+    order[gi >= 0 ? g_rows0[gi] + rank : n_rows + rank] = b;   // (`order` was scratch of passes (1) and (2) until the barrier)
   }
   __syncthreads();
   // ---- write-out, all threads ----
@@ -368,21 +569,25 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
     len = len_s[tid];
     mine = len > sh ? (len - sh + chunk_tokens - 1) / chunk_tokens : 0;
   }
-  // inclusive scan: inside the wave by shuffles, across the 16 waves through LDS (three barriers, not twenty)
-  int incl = mine;
+  const int my_tiles = len > sh ? (len - sh + 63) / 64 : 0;
+  // inclusive scans of both: inside the wave by shuffles, across the 16 waves through LDS (one barrier, not twenty)
+  int incl = mine, incl_t = my_tiles;
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
-    const int v = __shfl_up(incl, off, 64);
-    if (lane >= off) incl += v;
+    const int v = __shfl_up(incl, off, 64), u = __shfl_up(incl_t, off, 64);
+    if (lane >= off) { incl += v; incl_t += u; }
   }
-  if (lane == 63) wave_tot[wid] = incl;
+  if (lane == 63) { wave_tot[wid] = incl; wave_tiles[wid] = incl_t; }
   __syncthreads();
-  int wave_base = 0;
-  for (int w = 0; w < wid; ++w) wave_base += wave_tot[w];
-  incl += wave_base;
-  scan[tid] = incl;
-  __syncthreads();
-  const int base = n_shared_items + scan[tid] - mine;
+  int n_private = 0, n_tiles = 0;
+#pragma unroll
+  for (int w = 0; w < kPlanThreads / 64; ++w) {
+    const int v = wave_tot[w], u = wave_tiles[w];
+    n_private += v;
+    n_tiles += u;
+    if (w < wid) { incl += v; incl_t += u; }
+  }
+  const int base = n_shared_items + incl - mine;
   const int first_slot_p = (sh + chunk_tokens - 1) / chunk_tokens;
   for (int j = 0; j < mine; ++j) {
     if (base + j >= max_items) break;                // cannot happen when max_items is sized by the caller
@@ -397,10 +602,53 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
     it[7] = -1;
     it[3] = 1;
   }
-  if (tid == kPlanThreads - 1) {
-    const int total = n_shared_items + scan[tid];
+  // ---- spans: the private tokens of all requests, in 64-token tiles, as ONE line cut into equal parts ----
+  // (runs of whole chunks of one request each, as many as fill the chip, left it half empty at their ends: 128 requests of 0.9 to 2.1 k tokens
+  // 813 to 929 us against 709)
+  const int total = n_shared_items + n_private;
+  int want = span_units / num_kv_heads - n_shared_items;   // the shared items hold workgroups too
+  if (want < span_units / num_kv_heads / 2) want = span_units / num_kv_heads / 2;
+  if (want < 1) want = 1;
+  const int span = span_units > 0 ? (n_tiles + want - 1) / want : 0;     // tiles of a span
+  const bool spans = span >= kMinSpanTiles;            // (uniform)
+  if (tid == 0) {
     pv.header[0] = total < max_items ? total : max_items;
+    pv.header[4] = spans ? span : 0;
+    pv.header[5] = spans ? n_shared_items + (n_tiles + span - 1) / span : total < max_items ? total : max_items;
   }
+  if (!spans) {
+    if (tid < batch) pv.req_slots[tid] = first_slot_p + mine;
+    return;
+  }
+  const int tile0 = incl_t - my_tiles;                 // this request's tiles are [tile0, incl_t) of the line
+  const int first_span = tile0 / span, my_pieces = my_tiles > 0 ? (incl_t - 1) / span - first_span + 1 : 0;
+  if (tid < batch) pv.req_slots[tid] = first_slot_p + my_pieces;
+  incl = my_pieces;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int v = __shfl_up(incl, off, 64);
+    if (lane >= off) incl += v;
+  }
+  __syncthreads();                                     // (wave_tot has been read by everybody)
+  if (lane == 63) wave_tot[wid] = incl;
+  __syncthreads();
+  for (int w = 0; w < wid; ++w) incl += wave_tot[w];
+  for (int j = 0; j < my_pieces; ++j) {                // at most one a span and one more a request
+    const int k = first_span + j, i = incl - my_pieces + j;
+    const int lo = k * span > tile0 ? k * span - tile0 : 0, hi = (k + 1) * span - tile0;     // tiles of the request
+    if (k * span >= tile0) pv.span_first[k] = i;
+    int32_t* it = pv.pieces + 8 * i;
+    const int kvb = sh + lo * 64, kve = sh + hi * 64;
+    it[0] = first_slot_p + j;
+    it[1] = kvb;
+    it[2] = (kve < len ? kve : len) - kvb;
+    it[3] = 1;
+    it[4] = tid;
+    it[5] = 1;
+    it[6] = pool_row[tid];
+    it[7] = -1;
+  }
+  if (tid == kPlanThreads - 1) pv.span_first[(n_tiles + span - 1) / span] = incl;
 }
 
 // ---- merge: slots [0, n_slots(b)) of every (request, head), in slot order ----------------------
@@ -409,7 +657,7 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
 constexpr int kMergeBlock = 16;  // slots loaded per round (all loads of a round are in flight together)
 
 __global__ __launch_bounds__(256) void cascade_merge2_kernel(const float* __restrict__ ws_acc, const float* __restrict__ ws_ml,
-                                                             const int32_t* __restrict__ plan, const int32_t* __restrict__ seq_lens,
+                                                             const int32_t* __restrict__ plan,
                                                              uint16_t* __restrict__ out, int64_t out_stride, int batch,
                                                              int max_items, int num_q_heads, int head_dim, int slots_total,
                                                              float out_scale) {
@@ -419,9 +667,7 @@ __global__ __launch_bounds__(256) void cascade_merge2_kernel(const float* __rest
   const int d = (threadIdx.x % tpd) * 4;
   if (hq >= num_q_heads) return;
   const CascadePlanView pv = cascade_plan_view(plan, batch, max_items);
-  const int sh = pv.req_shared[b];
-  const int len = seq_lens[b];
-  int n = (sh + kChunk - 1) / kChunk + (len > sh ? (len - sh + kChunk - 1) / kChunk : 0);
+  int n = pv.req_slots[b];
   if (n > slots_total) n = slots_total;
   const int64_t base = (static_cast<int64_t>(b) * num_q_heads + hq) * slots_total;
   const float2* ml = reinterpret_cast<const float2*>(ws_ml) + base;
@@ -500,7 +746,9 @@ int sgl_amd_cascade_plan(const int32_t* req_to_token, int64_t req_to_token_strid
                      // own bound, batch x (chunks + 1)) whenever such a launch is possible at ANY setting of the launch-form switch --
                      // the switch may change between the plan and the attention launches, or after graphs were captured
                      static_cast<int>(batch * (chunks + 1) * num_kv_heads <= kSingleShotHardCap
-                                          ? (batch * (chunks + 1) < max_items ? batch * (chunks + 1) : max_items) : 0));
+                                          ? (batch * (chunks + 1) < max_items ? batch * (chunks + 1) : max_items) : 0),
+                     num_kv_heads,
+                     num_q_heads / num_kv_heads <= 8 && batch * (chunks + 1) * num_kv_heads > single_shot_most(chunks, num_q_heads / num_kv_heads) ? kSpanUnits : 0);
   SGL_CHECK_LAUNCH("cascade_plan");
   return 0;
 }
@@ -566,7 +814,9 @@ int sgl_amd_cascade_decode_attention_ex(const void* q, const void* k_cache, cons
   int64_t units = batch * (chunks + 1);
   if (units > max_items) units = max_items;
   const int64_t worst = units * num_kv_heads;
-  const bool loop = worst > g_cascade_single_shot_units;
+  // (a plan of spans is only made where this is true at the switch's default: the switch can lower the line, not raise it)
+  const int64_t most = single_shot_most(chunks, p.group);
+  const bool loop = worst > (g_cascade_single_shot_units < most ? g_cascade_single_shot_units : most);
   dim3 grid(static_cast<unsigned>(loop ? (worst < g_cascade_loop_grid ? worst : g_cascade_loop_grid) : worst));
 #define SGL_LAUNCH_CASC2(D_, KERNEL_)                                                                                 \
   do {                                                                                                       \
@@ -586,7 +836,7 @@ int sgl_amd_cascade_decode_attention_ex(const void* q, const void* k_cache, cons
 #undef SGL_LAUNCH_CASC
   const int hpb = 256 / (head_dim / 4);
   hipLaunchKernelGGL(cascade_merge2_kernel, dim3(static_cast<unsigned>(batch), (num_q_heads + hpb - 1) / hpb), dim3(256), 0, st,
-                     p.ws_acc, p.ws_ml, plan, seq_lens, static_cast<uint16_t*>(out), out_token_stride, p.batch, p.max_items,
+                     p.ws_acc, p.ws_ml, plan, static_cast<uint16_t*>(out), out_token_stride, p.batch, p.max_items,
                      num_q_heads, head_dim, slots_total, kv_fp8 ? v_scale : 1.0f);
   SGL_CHECK_LAUNCH("cascade_decode_attention");
   return 0;
@@ -596,7 +846,7 @@ int sgl_amd_debug_cascade_launch_form(int64_t single_shot_units, int64_t loop_gr
   SGL_CLEAR_STALE_ERROR();
   SGL_CHECK_ARG(single_shot_units >= 0 && single_shot_units <= kSingleShotHardCap && loop_grid >= 0 && loop_grid <= (1 << 20),
                 "debug_cascade_launch_form: single_shot_units must be 0..%lld, loop_grid 0..2^20", (long long)kSingleShotHardCap);
-  g_cascade_single_shot_units = single_shot_units > 0 ? single_shot_units : 10240;
+  g_cascade_single_shot_units = single_shot_units > 0 ? single_shot_units : kSingleShotUnits;
   g_cascade_loop_grid = loop_grid > 0 ? loop_grid : 256 * 5;
   return 0;
 }
