@@ -80,15 +80,33 @@ __device__ __forceinline__ uint32_t pack_bf2(float lo, float hi) {
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // ---- wave64 reductions -----------------------------------------------------
+// The butterfly over lane ^ 32, 16, 8, 4, 2, 1 without the LDS unit (six dependent ds_bpermute are ~0.4 us of a workgroup that does
+// little else): the two lane swaps leave each half / each row pair in one register, the rest are DPP.  Once lane i and lane i ^ 8 agree,
+// a rotation by 4 inside the row of 16 reads the value of lane i ^ 4.  Same partners in the same order as __shfl_xor, so the same bits.
+// Whole waves only (every lane active).
+template <int CTRL>
+__device__ __forceinline__ float wave_dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <typename OP>
+__device__ __forceinline__ float wave_butterfly(float v, OP&& op) {
+  float a = v, b = v;                  // (asm: of the builtin's two results on one value hipcc keeps the first only; s_nop: VALU write -> lane swap)
+  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+  v = op(a, b);
+  a = v;
+  b = v;
+  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+  v = op(a, b);
+  v = op(v, wave_dpp<0x128>(v));       // row_ror:8
+  v = op(v, wave_dpp<0x124>(v));       // row_ror:4
+  v = op(v, wave_dpp<0x4e>(v));        // quad_perm [2, 3, 0, 1]
+  return op(v, wave_dpp<0xb1>(v));     // quad_perm [1, 0, 3, 2]
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+  return wave_butterfly(v, [](float x, float y) { return x + y; });
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-  return v;
+  return wave_butterfly(v, [](float x, float y) { return fmaxf(x, y); });
 }
 
 // Block-wide sum for blocks of up to 1024 threads. `scratch` = 16 floats of LDS.
