@@ -1050,7 +1050,7 @@ __global__ __launch_bounds__(kT) void sample_finish_ranges_kernel(SampleParams p
 // Sampler.forward on a decode batch used to be five launches over the [B, V] fp32 probabilities (softmax partials, normalise:
 // 33 MB written; histogram + collect: 33 MB read each; finish).  The kept set of sampler.py:574-591 is a prefix of the row's
 // descending order, and p(x) = expf(x / t - max) / sum is monotone in the bf16 logit x, so the prefix can be found on the LOGITS:
-//   candidates  grid (16 column ranges, rows), 256 threads: the softmax partials of the range (the bits of the two-launch softmax:
+//   candidates  grid (<= 16 column ranges, rows), 256 threads: the softmax partials of the range (the bits of the two-launch softmax:
 //               softmax_ranges.hpp) and an exact two-level radix select on the 16-bit order keys of the range's logits: every
 //               element >= the range's K-th largest (K = min(top_k, 64)) goes to the range's candidate list in token order
 //               (<= 127 of them: ties at the cut included), with the largest key NOT emitted -- the range's frontier;
@@ -1062,6 +1062,11 @@ __global__ __launch_bounds__(kT) void sample_finish_ranges_kernel(SampleParams p
 //   probabilities into a scratch matrix and runs the single-workgroup routine on them (no launch for rows that do not need it).
 // [64, 128256], top-k 50 / top-p 0.9: 16 MB read once from HBM instead of ~130 MB of traffic.  Same ids and kept counts as the
 // long way by construction (tests/test_sampler_gpu.py compares them on every row).
+// What bounds it: the candidates launch at many rows the vector instructions (49 a column, 22 of them the quotient and the exponential;
+// the matrix of 128 rows alone is 7 us of reading), at few rows, like the finish launch, a chain of dependent steps: 5 us until the
+// records and lists are there, 2.5 the cut, 1 the compaction, 3 rank, rules and arg-max.  us for the two launches, before this division
+// of the work (a true division per column, every column tested one by one for the list, byte-wide histograms, ranks, logs and noise all
+// by one wave) and now: [128, 128256] 53 / 42, [64, 128256] 42 / 32, [1, 128256] 34 / 23, [128, 32000] 40 / 27.
 constexpr int kFastRangesMax = 16;
 constexpr int kFastCap = 127;
 constexpr int kFastK = 64;
@@ -1071,7 +1076,7 @@ struct FastWs {
   float* partials;      // [B, S, 2]
   uint32_t* cand_val;   // [B, R, kFastCap]: the logit as fp32 bits
   int* cand_tok;        // [B, R, kFastCap]
-  int* meta;            // [B, R, 4]: candidates (-1: more than kFastCap), 1 if columns were left out, the largest of them (fp32 bits), 0
+  int* meta;            // [B, R, 4]: candidates (-1: more than kFastCap), 1 if columns were left out, the largest of them, the largest of all (fp32 bits)
   int* fallback;        // [B]: 1 = redo the row from its probabilities
 };
 __host__ __device__ inline int64_t fast_ws_bytes(int64_t batch, int splits) {
@@ -1118,6 +1123,43 @@ struct Cols4<float> {
   __device__ __forceinline__ float v(int k) const { return k == 0 ? q.x : k == 1 ? q.y : k == 2 ? q.z : q.w; }
 };
 
+// three operands at once, and no canonicalising copy of each (a signalling NaN makes the row's sum NaN either way)
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+__device__ __forceinline__ float min3(float a, float b, float c) {
+  float r;
+  asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+// fp32 bits -> unsigned that orders like the value, and back (0 = below every value)
+__device__ __forceinline__ uint32_t order32(float v) {
+  const uint32_t u = __float_as_uint(v);
+  return u ^ ((u & 0x80000000u) ? 0xffffffffu : 0x80000000u);
+}
+__device__ __forceinline__ float value_of_order32(uint32_t k) { return __uint_as_float(k ^ ((k & 0x80000000u) ? 0x80000000u : 0xffffffffu)); }
+// inclusive prefix sums over the wave's lanes (DPP row_shr 1, 2, 4, 8, then the rows' last lanes)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t moved(uint32_t v) {
+  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, ROWS, 0xf, true));
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned long long moved(unsigned long long v) {
+  return static_cast<unsigned long long>(moved<CTRL, ROWS>(static_cast<uint32_t>(v >> 32))) << 32 | moved<CTRL, ROWS>(static_cast<uint32_t>(v));
+}
+template <typename T>
+__device__ __forceinline__ T wave_prefix(T v) {
+  v += moved<0x111, 0xf>(v);
+  v += moved<0x112, 0xf>(v);
+  v += moved<0x114, 0xf>(v);
+  v += moved<0x118, 0xf>(v);
+  v += moved<0x142, 0xa>(v);
+  v += moved<0x143, 0xc>(v);
+  return v;
+}
+
 // which of 256 bins holds the K-th largest element: `c` = this thread's (tid = bin) count.  Returns through LDS `sel`:
 // [0] bin, [1] elements in the bins above it, [2] elements in it.  Needs K >= 1 and K <= the total.  256 threads.
 __device__ __forceinline__ void select_bin_256(uint32_t c, uint32_t K, uint32_t* wave_tot, int* sel) {
@@ -1156,110 +1198,132 @@ __global__ __launch_bounds__(kSplitThreads) void sample_logit_candidates_kernel(
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const IN* x = logits + static_cast<int64_t>(row) * row_stride;
   const float t = temperatures[row];
-  const int per = ((V + S - 1) / S + 3) / 4 * 4;    // (split_range_of's geometry)
+  const int per = ((V + S - 1) / S + 3) / 4 * 4;    // (split_range_of's geometry; the launch keeps S * per far below 2^31)
+  const int slots = G * J;
   // ---- one burst: every column of the workgroup ----
   Cols4<IN> q[NS];
   uint32_t on_mask = 0;                              // slot s holds four columns of this thread
-  auto slot_g = [&](int s) { return s / J; };        // (uniform)
+  auto range_begin = [&](int g) { const int b = per * (c * G + g); return b < V ? b : V; };
   auto slot_col = [&](int s) {
-    const int g = s / J, j = s - g * J;
-    int64_t b = static_cast<int64_t>(per) * (c * G + g);
-    if (b > V) b = V;
-    return static_cast<int>(b) + 1024 * j + 4 * tid;
+    const int g = (s >= J) + (s >= 2 * J) + (s >= 3 * J);
+    return range_begin(g) + 1024 * (s - g * J) + 4 * tid;
   };
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    const int g = s / J;
-    int64_t b = static_cast<int64_t>(per) * (c * G + g), e = b + per;
-    if (b > V) b = V;
-    if (e > V) e = V;
-    const int64_t e4 = b + (e - b) / 4 * 4;
-    const int i = slot_col(s);
-    const bool on = g < G && i < e4;
-    on_mask |= on ? (1u << s) : 0u;
-    if (on) q[s].load(x + i);
-    else q[s].zero();
+    q[s].zero();
+    if (s < slots) {                                 // (uniform)
+      const int g = (s >= J) + (s >= 2 * J) + (s >= 3 * J);
+      const int b = range_begin(g), e = range_begin(g + 1), i = b + 1024 * (s - g * J) + 4 * tid;
+      if (i < b + ((e - b) & ~3)) {
+        on_mask |= 1u << s;
+        q[s].load(x + i);
+      }
+    }
   }
   // (the <= 3 columns behind the last multiple of four: in the row's last range only, which is this workgroup's last if any)
-  const int tail_g = G - 1;
   int tail_i = -1;
   float tail_v = 0.f;
   {
-    int64_t b = static_cast<int64_t>(per) * (c * G + tail_g), e = b + per;
-    if (b > V) b = V;
-    if (e > V) e = V;
-    const int64_t e4 = b + (e - b) / 4 * 4;
-    if (e4 + tid < e) { tail_i = static_cast<int>(e4 + tid); tail_v = ld1(x + tail_i); }
+    const int b = range_begin(G - 1), e = range_begin(G), e4 = b + ((e - b) & ~3);
+    if (e4 + tid < e) { tail_i = e4 + tid; tail_v = ld1(x + tail_i); }
   }
-  auto val_of = [&](int s, int k) -> float { return q[s].v(k); };
   auto is_on = [&](int s) { return (on_mask >> s) & 1u; };
 
   // ---- the softmax partials of the G ranges: range_partial's arithmetic in range_partial's order (softmax_ranges.hpp), every
   // range's two workgroup reductions done side by side.  The maximum of x / t is (the maximum of x) / t for t > 0 -- a correctly
-  // rounded division is monotone -- so the first pass divides once per range, not once per column. ----
+  // rounded division is monotone -- so the first pass divides once per range, not once per column.  Slots come range by range: one
+  // running value, put away where the next range begins. ----
   const bool t_pos = t > 0.f;                        // (uniform; other temperatures: column by column, and the row goes the long way)
-  const bool t_one = t == 1.0f;                      // (uniform) x / 1 is x: the exponent pass skips 32 divisions
-  float mxg[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+  const bool t_one = t == 1.0f;                      // (uniform) x / 1 is x
+  float mxg[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY}, run = -INFINITY, lo = INFINITY;
+  auto put_away = [&](float* to, int s, float value) { // the sums of the ranges that end before slot s (uniform)
+    if (s == J) to[0] = value;
+    else if (s == 2 * J) to[1] = value;
+    else to[2] = value;
+  };
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    float m;
-    if (t_pos) m = fmaxf(fmaxf(val_of(s, 0), val_of(s, 1)), fmaxf(val_of(s, 2), val_of(s, 3)));
-    else m = fmaxf(fmaxf(val_of(s, 0) / t, val_of(s, 1) / t), fmaxf(val_of(s, 2) / t, val_of(s, 3) / t));
-    const int g = is_on(s) ? slot_g(s) : -1;
-#pragma unroll
-    for (int gg = 0; gg < 4; ++gg) mxg[gg] = g == gg ? fmaxf(mxg[gg], m) : mxg[gg];
+    if (s > 0 && (s == J || s == 2 * J || s == 3 * J) && s < slots) { put_away(mxg, s, run); run = -INFINITY; }
+    if (s < slots) {
+      const float v0 = q[s].v(0), v1 = q[s].v(1), v2 = q[s].v(2), v3 = q[s].v(3);
+      float m;
+      if (t_pos) m = max3(max3(v0, v1, v2), v3, run);
+      else m = fmaxf(fmaxf(fmaxf(v0 / t, v1 / t), fmaxf(v2 / t, v3 / t)), run);
+      lo = min3(min3(v0, v1, v2), v3, lo);
+      run = is_on(s) ? m : run;
+    }
   }
-  if (tail_i >= 0) {
-    const float m = t_pos ? tail_v : tail_v / t;
-#pragma unroll
-    for (int gg = 0; gg < 4; ++gg) mxg[gg] = tail_g == gg ? fmaxf(mxg[gg], m) : mxg[gg];
-  }
+  if (tail_i >= 0) run = fmaxf(run, t_pos ? tail_v : tail_v / t);
+  if (G == 1) mxg[0] = run;
+  else if (G == 2) mxg[1] = run;
+  else if (G == 3) mxg[2] = run;
+  else mxg[3] = run;
+  const float my_top = fmaxf(fmaxf(mxg[0], mxg[1]), fmaxf(mxg[2], mxg[3]));    // the thread's largest logit (t_pos)
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
-    const float w = wave_max(mxg[g]);
-    if (lane == 0) red[g][wid] = w;
+    if (g < G) {
+      const float w = wave_max(mxg[g]);
+      if (lane == 0) red[g][wid] = w;
+    }
   }
   __syncthreads();
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
-    const float m = fmaxf(fmaxf(red[g][0], red[g][1]), fmaxf(red[g][2], red[g][3]));
-    mxg[g] = t_pos ? m / t : m;
+    if (g < G) {
+      const float m = fmaxf(fmaxf(red[g][0], red[g][1]), fmaxf(red[g][2], red[g][3]));
+      mxg[g] = t_pos ? m / t : m;
+    }
   }
   __syncthreads();
+  // x / t with the reciprocal of t formed once.  For a correctly rounded 1 / t, one remainder step makes the quotient faithful and the
+  // second one correctly rounded (Markstein, IBM J. Res. Dev. 34, 1990): the bits of the division, at 5 operations instead of 11 and a
+  // quarter-rate reciprocal.  Needs finite operands and no overflow; columns so small that the remainder underflows are 0 beside any
+  // maximum they are compared with.  NaN stays NaN.
+  const bool by_rcp = !t_one && t >= 9.5367431640625e-7f && t <= 1048576.0f &&
+                      __ballot(!(lo >= -1e30f && my_top <= 1e30f)) == 0ull;     // (wave-uniform; masked-out columns are -inf)
+  const float rcp_t = 1.0f / t;
+  auto over_t = [&](float v) {
+    float d = v * rcp_t;
+    d = __fmaf_rn(__fmaf_rn(-t, d, v), rcp_t, d);
+    return __fmaf_rn(__fmaf_rn(-t, d, v), rcp_t, d);
+  };
   float smg[4] = {0.f, 0.f, 0.f, 0.f};
+  float mx = mxg[0];
+  run = 0.f;
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    if (is_on(s)) {
-      const int g = slot_g(s);
-      const float mx = g == 0 ? mxg[0] : g == 1 ? mxg[1] : g == 2 ? mxg[2] : mxg[3];
-      if (mx > -INFINITY) {
-        float add;
-        if (t_one) add = expf(val_of(s, 0) - mx) + expf(val_of(s, 1) - mx) + expf(val_of(s, 2) - mx) + expf(val_of(s, 3) - mx);
-        else add = expf(val_of(s, 0) / t - mx) + expf(val_of(s, 1) / t - mx) + expf(val_of(s, 2) / t - mx) + expf(val_of(s, 3) / t - mx);
-#pragma unroll
-        for (int gg = 0; gg < 4; ++gg) smg[gg] = g == gg ? smg[gg] + add : smg[gg];
-      }
+    if (s > 0 && (s == J || s == 2 * J || s == 3 * J) && s < slots) {
+      put_away(smg, s, run);
+      run = 0.f;
+      mx = s == J ? mxg[1] : s == 2 * J ? mxg[2] : mxg[3];
+    }
+    if (s < slots && mx > -INFINITY) {                // (uniform)
+      const float v0 = q[s].v(0), v1 = q[s].v(1), v2 = q[s].v(2), v3 = q[s].v(3);
+      float add;
+      if (t_one) add = expf(v0 - mx) + expf(v1 - mx) + expf(v2 - mx) + expf(v3 - mx);
+      else if (by_rcp) add = expf(over_t(v0) - mx) + expf(over_t(v1) - mx) + expf(over_t(v2) - mx) + expf(over_t(v3) - mx);
+      else add = expf(v0 / t - mx) + expf(v1 / t - mx) + expf(v2 / t - mx) + expf(v3 / t - mx);
+      if (is_on(s)) run += add;
     }
   }
-  if (tail_i >= 0) {
-    const float mx = tail_g == 0 ? mxg[0] : tail_g == 1 ? mxg[1] : tail_g == 2 ? mxg[2] : mxg[3];
-    if (mx > -INFINITY) {
-      const float add = expf(tail_v / t - mx);
-#pragma unroll
-      for (int gg = 0; gg < 4; ++gg) smg[gg] = tail_g == gg ? smg[gg] + add : smg[gg];
-    }
-  }
+  if (tail_i >= 0 && mx > -INFINITY) run += expf(tail_v / t - mx);
+  if (G == 1) smg[0] = run;
+  else if (G == 2) smg[1] = run;
+  else if (G == 3) smg[2] = run;
+  else smg[3] = run;
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
-    const float w = wave_sum(smg[g]);
-    if (lane == 0) red[g][wid] = w;
+    if (g < G) {
+      const float w = wave_sum(smg[g]);
+      if (lane == 0) red[g][wid] = w;
+    }
   }
   __syncthreads();
   if (tid < G) {
     // block_sum's association over the four wave sums: (w0 + w2) + (w1 + w3)
     const float tot = (red[tid][0] + red[tid][2]) + (red[tid][1] + red[tid][3]);
-    const float mx = tid == 0 ? mxg[0] : tid == 1 ? mxg[1] : tid == 2 ? mxg[2] : mxg[3];
-    ws.partials[(static_cast<int64_t>(row) * S + c * G + tid) * 2 + 0] = mx;
+    const float mxt = tid == 0 ? mxg[0] : tid == 1 ? mxg[1] : tid == 2 ? mxg[2] : mxg[3];
+    ws.partials[(static_cast<int64_t>(row) * S + c * G + tid) * 2 + 0] = mxt;
     ws.partials[(static_cast<int64_t>(row) * S + c * G + tid) * 2 + 1] = tot;
   }
 
@@ -1267,15 +1331,9 @@ __global__ __launch_bounds__(kSplitThreads) void sample_logit_candidates_kernel(
   int* meta = ws.meta + (static_cast<int64_t>(row) * R + c) * 4;
   int64_t top_k = top_ks ? top_ks[row] : V;
   if (top_k > V) top_k = V;
-  int n;
-  {
-    int64_t cb = static_cast<int64_t>(per) * (c * G), ce = static_cast<int64_t>(per) * (c * G + G);
-    if (cb > V) cb = V;
-    if (ce > V) ce = V;
-    n = static_cast<int>(ce - cb);
-  }
+  const int n = range_begin(G) - range_begin(0);
   if (n <= 0 || top_k <= 0) {                       // (top_k <= 0: the finish launch sends the row the long way)
-    if (tid == 0) { meta[0] = 0; meta[1] = 0; meta[2] = 0; }
+    if (tid == 0) { meta[0] = 0; meta[1] = 0; meta[2] = 0; meta[3] = static_cast<int>(0xff800000u); }
     return;
   }
   const int Kc = static_cast<int>(top_k < kFastK ? top_k : kFastK);
@@ -1299,8 +1357,11 @@ __global__ __launch_bounds__(kSplitThreads) void sample_logit_candidates_kernel(
   // everything >= the K-th largest.  (Histogramming the range cost 13 us of LDS atomics on the handful of hot bins of a softmax
   // row.)  Columns are compared as fp32 values (-0 == +0 there: a superset still; a NaN passes no test -- its row's softmax is
   // not finite and the finish launch sends it the long way).
-  float my_maxf = -INFINITY;
-  for_each_val([&](float v, int) { my_maxf = fmaxf(my_maxf, v); });
+  float my_maxf = my_top;
+  if (!t_pos) {                                       // (uniform) my_top is of quotients
+    my_maxf = -INFINITY;
+    for_each_val([&](float v, int) { my_maxf = fmaxf(my_maxf, v); });
+  }
   const int my_max = n_mine > 0 ? static_cast<int>(order_hi16(__float_as_uint(my_maxf))) : -1;
   {
     const int kw = (static_cast<int>(K) + 3) / 4;
@@ -1322,24 +1383,40 @@ __global__ __launch_bounds__(kSplitThreads) void sample_logit_candidates_kernel(
   uint32_t* out_val = ws.cand_val + (static_cast<int64_t>(row) * R + c) * kFastCap;
   int* out_tok = ws.cand_tok + (static_cast<int64_t>(row) * R + c) * kFastCap;
   // ---- emit (in no particular order: the finish launch ranks by (value, token)); the largest value left out is the frontier.
-  // Positions: hits per lane, an exclusive scan over the wave, ONE LDS atomic per wave ----
+  // Positions: a bit per column that passes, an exclusive scan of their counts over the wave, ONE LDS atomic per wave.  A lane passes
+  // a fraction of a column, so the few that pass are read again (cached) rather than each of the 32 .. 64 tested a second time ----
   float front_f = -INFINITY;
   bool any_left = false;
   auto emit = [&]() {
     const float L = kth == 0u ? -INFINITY : floor_of_key16(kth);
     front_f = -INFINITY;
-    int hits = 0;
-    for_each_val([&](float v, int) {
-      hits += v >= L;
-      front_f = fmaxf(front_f, v < L ? v : -INFINITY);
-    });
-    any_left = hits < n_mine;
-    int incl = hits;
+    uint32_t pass[NS / 8];                            // 8 slots a word, the last slot's last column in bit 0
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int o = __shfl_up(incl, off, 64);
-      if (lane >= off) incl += o;
+    for (int w = 0; w < NS / 8; ++w) {
+      pass[w] = 0u;
+#pragma unroll
+      for (int s = 8 * w; s < 8 * w + 8; ++s) {
+        if (s < slots) {                              // (uniform)
+          const uint32_t on = is_on(s);
+#pragma unroll
+          for (int k = 0; k < 4; k += 2) {
+            const float v = q[s].v(k), u = q[s].v(k + 1);
+            const bool hv = on && v >= L, hu = on && u >= L;
+            pass[w] = pass[w] << 2 | (hv ? 2u : 0u) | (hu ? 1u : 0u);
+            front_f = max3(hv || !on ? -INFINITY : v, hu || !on ? -INFINITY : u, front_f);
+          }
+        } else {
+          pass[w] <<= 4;
+        }
+      }
     }
+    const bool tail_hit = tail_i >= 0 && tail_v >= L;
+    if (tail_i >= 0 && !tail_hit) front_f = fmaxf(front_f, tail_v);
+    int hits = tail_hit ? 1 : 0;
+#pragma unroll
+    for (int w = 0; w < NS / 8; ++w) hits += __popc(pass[w]);
+    any_left = hits < n_mine;
+    const int incl = static_cast<int>(wave_prefix(static_cast<uint32_t>(hits)));
     const int total = __builtin_amdgcn_readlane(incl, 63);
     int base = 0;
     if (total > 0) {                                  // (wave-uniform)
@@ -1348,12 +1425,17 @@ __global__ __launch_bounds__(kSplitThreads) void sample_logit_candidates_kernel(
     }
     int pos = base + incl - hits;
     if (hits > 0) {
-      for_each_val([&](float v, int col) {
-        if (v >= L) {
-          if (pos < kFastCap) { out_val[pos] = __float_as_uint(v); out_tok[pos] = col; }
-          ++pos;
+      auto put = [&](float v, int col) {
+        if (pos < kFastCap) { out_val[pos] = __float_as_uint(v); out_tok[pos] = col; }
+        ++pos;
+      };
+#pragma unroll
+      for (int w = 0; w < NS / 8; ++w)
+        for (uint32_t m = pass[w]; m != 0u; m &= m - 1u) {
+          const int i = 31 - (__ffs(static_cast<int>(m)) - 1), col = slot_col(8 * w + (i >> 2)) + (i & 3);
+          put(ld1(x + col), col);
         }
-      });
+      if (tail_hit) put(tail_v, tail_i);
     }
   };
   emit();
@@ -1378,7 +1460,7 @@ __global__ __launch_bounds__(kSplitThreads) void sample_logit_candidates_kernel(
     const int n_ge = static_cast<int>(above1) + sel[1] + sel[2];
     __syncthreads();
     if (n_ge > kFastCap) {                            // (workgroup-uniform) a tie wider than the list
-      if (tid == 0) { meta[0] = -1; meta[1] = 0; meta[2] = 0; }
+      if (tid == 0) { meta[0] = -1; meta[1] = 0; meta[2] = 0; meta[3] = static_cast<int>(0xff800000u); }
       return;
     }
     if (tid == 0) sel[3] = 0;
@@ -1387,14 +1469,9 @@ __global__ __launch_bounds__(kSplitThreads) void sample_logit_candidates_kernel(
     __syncthreads();
   }
   // the largest value left out, over the workgroup (any_left: this thread left something out)
-  float fr_w = any_left ? front_f : -INFINITY;
-  int left_w = any_left ? 1 : 0;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    fr_w = fmaxf(fr_w, __shfl_xor(fr_w, off, 64));
-    left_w |= __shfl_xor(left_w, off, 64);
-  }
-  if (lane == 0) { red[0][wid] = fr_w; redi[wid] = left_w; }
+  const float fr_w = wave_max(any_left ? front_f : -INFINITY), top_w = wave_max(my_maxf);
+  const int left_w = __ballot(any_left) != 0ull ? 1 : 0;
+  if (lane == 0) { red[0][wid] = fr_w; red[1][wid] = top_w; redi[wid] = left_w; }
   __syncthreads();
   if (tid == 0) {
     const float f = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
@@ -1402,7 +1479,7 @@ __global__ __launch_bounds__(kSplitThreads) void sample_logit_candidates_kernel(
     m.x = sel[3] > kFastCap ? -1 : sel[3];            // (fp32 compares emit -0 with +0: the exact select's count is a key count)
     m.y = redi[0] | redi[1] | redi[2] | redi[3];
     m.z = static_cast<int>(__float_as_uint(f));
-    m.w = 0;
+    m.w = static_cast<int>(__float_as_uint(fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3]))));
     *reinterpret_cast<int4*>(meta) = m;
   }
 }
@@ -1411,8 +1488,8 @@ __global__ __launch_bounds__(kSplitThreads) void sample_logit_candidates_kernel(
 // arithmetic (exact_top_p_keep on fp64 inclusive prefix sums, fp64 gumbel scores, best_better) without a workgroup barrier --
 // sample_row spends ~15 us on its dozen barriers and serial LDS loops for the ~50 elements a pruned list holds.
 __device__ void finish_small_list(const SampleParams& p, const int row, const uint32_t* cand_val, const int* cand_tok, uint32_t* s_key, int* s_tok,
-                                  const int n, int64_t top_k, const float top_p, const bool has_min_p, const float min_p, const uint64_t seed,
-                                  const uint32_t pos, const Frontier* fr) {
+                                  const int n, int64_t top_k, const float top_p, const bool has_min_p, const float min_p, const int* s_part,
+                                  const double* s_log, double* s_log_sorted, const double* s_gumbel, const Frontier* fr) {
   const int lane = threadIdx.x & 63;
   const uint32_t key = lane < n ? key_of(__uint_as_float(cand_val[lane])) : 0u;
   const int tok = lane < n ? cand_tok[lane] : 0x7fffffff;
@@ -1422,14 +1499,10 @@ __device__ void finish_small_list(const SampleParams& p, const int row, const ui
     mxp = wave_max(fmaxf(mxp, 0.f));
     min_key = key_of(mxp * min_p);
   }
-  int rank = 0;                                       // descending value, ties by token id
-#pragma unroll 8
-  for (int j = 0; j < 64; ++j) {
-    const uint32_t kj = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(key), j));
-    const int tj = __builtin_amdgcn_readlane(tok, j);
-    rank += (j < n) && ((kj > key) || (kj == key && tj < tok));
-  }
-  if (lane < n) { s_key[rank] = key; s_tok[rank] = tok; }
+  int rank = 0;                                       // descending value, ties by token id: a quarter of the list by each of four waves
+#pragma unroll
+  for (int w = 0; w < 4; ++w) rank += s_part[w * 64 + lane];
+  if (lane < n) { s_key[rank] = key; s_tok[rank] = tok; s_log_sorted[rank] = s_log[lane]; }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
@@ -1451,26 +1524,18 @@ __device__ void finish_small_list(const SampleParams& p, const int row, const ui
     const bool keep_h = r0 < top_k && fr->key >= min_key && exact_top_p_keep(excl + static_cast<double>(fr->prob), fr->prob, top_p);
     if (keep_h && lane == 0) *fr->unusable = 1;
   }
-  const uint32_t hpre = murmur_prefix(seed, pos);
-  Best best{0.0, -1, 0};
   const bool keep = r < n && r < top_k && kr >= min_key && exact_top_p_keep(run, pv, top_p);
-  if (keep) {
-    best.score = log(static_cast<double>(pv)) + gumbel_from_hash(murmur_hash32(hpre, r));
-    best.rank = r;
-    best.token = tr;
-  }
-  const int kept = __popcll(__ballot(keep));
+  // arg-max of log p + gumbel over the kept ranks, the first on a tie (a kept p is a number, and so are both logs: no NaN to order)
+  const double score = keep ? s_log_sorted[r] + s_gumbel[r] : -INFINITY;
+  double best = score;
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    Best o;
-    o.score = __shfl_xor(best.score, off, 64);
-    o.rank = __shfl_xor(best.rank, off, 64);
-    o.token = __shfl_xor(best.token, off, 64);
-    if (best_better(best, o)) best = o;
-  }
+  for (int off = 32; off > 0; off >>= 1) best = fmax(best, __shfl_xor(best, off, 64));
+  const unsigned long long kept = __ballot(keep), winners = __ballot(keep && score == best);
+  const int win = winners != 0ull ? __ffsll(static_cast<long long>(winners)) - 1 : 0;
+  const int token = __builtin_amdgcn_readlane(tr, win);
   if (lane == 0) {
-    p.out_ids[row] = best.rank < 0 ? 0 : best.token;   // (empty nucleus: the reference's all -inf row argmax-es to sorted rank 0)
-    if (p.out_n_keep) p.out_n_keep[row] = kept;
+    p.out_ids[row] = kept == 0ull ? 0 : token;        // (empty nucleus: the reference's all -inf row argmax-es to sorted rank 0)
+    if (p.out_n_keep) p.out_n_keep[row] = __popcll(kept);
   }
 }
 
@@ -1478,12 +1543,12 @@ template <typename IN>
 __global__ __launch_bounds__(kT) void sample_finish_fast_kernel(SampleParams p, const IN* __restrict__ logits, int64_t logits_row_stride,
                                                                  const float* __restrict__ temperatures, int S, int R, FastWs ws) {
   __shared__ RowSmem sm;
-  __shared__ int pre[kFastRangesMax + 1];
-  __shared__ int m_cnt[kFastRangesMax], m_left[kFastRangesMax];
-  __shared__ float m_front[kFastRangesMax];
-  __shared__ int s_has_front, s_bad, s_unusable;
-  __shared__ float s_front;
+  __shared__ int m_cnt[kFastRangesMax];
+  __shared__ int s_acc, s_broken, s_unusable, s_n, s_near;
+  __shared__ uint32_t s_front, s_top;                   // order32 of the largest logit not in the list (0: none); of the largest of all
   __shared__ float s_mx, s_sum;
+  __shared__ int s_part[4 * 64];
+  __shared__ double s_gumbel[64], s_log[64], s_log_sorted[64];
   const int row = blockIdx.x, tid = threadIdx.x;
   const int lane = tid & 63, wid = tid >> 6;
   // ---- ONE round trip to memory for everything the row needs: its parameters, the R range records, the 2 S softmax partials and
@@ -1504,45 +1569,49 @@ __global__ __launch_bounds__(kT) void sample_finish_fast_kernel(SampleParams p, 
       tok[u] = ws.cand_tok[static_cast<int64_t>(row) * R * kFastCap + idx];
     }
   }
-  if (tid >= 256 && tid < 512) { sm.hist_cnt[tid - 256] = 0; sm.hist_sum[tid - 256] = 0; sm.part_cnt[tid - 256] = 0; sm.part_sum[16 + tid - 256] = 0; }
-  if (tid == 512) { sm.found_bin = -1; sm.n_eq_keep = -1; }
-  if (tid >= 64 && tid < 64 + R) {
-    const int4 m = *reinterpret_cast<const int4*>(ws.meta + (static_cast<int64_t>(row) * R + tid - 64) * 4);
-    m_cnt[tid - 64] = m.x; m_left[tid - 64] = m.y; m_front[tid - 64] = __uint_as_float(static_cast<uint32_t>(m.z));
+  sm.part_cnt[tid] = 0;
+  sm.part_sum[tid] = 0;
+  if (wid == 1) {                                       // the range records: list length, frontier, largest logit
+    int4 m = int4{0, 0, 0, static_cast<int>(0xff800000u)};
+    if (lane < R) m = *reinterpret_cast<const int4*>(ws.meta + (static_cast<int64_t>(row) * R + lane) * 4);
+    if (lane < R) m_cnt[lane] = m.x;
+    const float top = wave_max(__uint_as_float(static_cast<uint32_t>(m.w)));
+    const float front = wave_max(m.y ? __uint_as_float(static_cast<uint32_t>(m.z)) : -INFINITY);
+    const unsigned long long left = __ballot(m.y != 0), broken = __ballot(m.x < 0);
+    const uint32_t acc = wave_prefix(static_cast<uint32_t>(m.x > 0 ? m.x : 0));
+    if (lane == 63) {
+      s_acc = static_cast<int>(acc);
+      s_broken = broken != 0ull;
+      s_front = left != 0ull ? order32(front) : 0u;
+      s_top = order32(top);
+    }
   }
+  // the noise of the first 64 ranks, whatever ends up there (under the other waves' loads)
+  if (wid == 2) s_gumbel[lane] = gumbel_from_hash(murmur_hash32(murmur_prefix(seed, spos), lane));
+  if (tid == 512) { sm.found_bin = -1; sm.n_eq_keep = -1; s_unusable = 0; s_n = 0; s_near = -1; }
   if (wid == 0) {
     // the row's maximum and sum from its S partials: merge_partials' arithmetic (softmax_ranges.hpp) with the S exponentials
     // side by side; the sum itself stays a left-to-right chain over the ranges (the bits of the normalise launch)
     const float pm = lane < S ? ws.partials[(static_cast<int64_t>(row) * S + lane) * 2] : -INFINITY;
-    const float ps = lane < S ? ws.partials[(static_cast<int64_t>(row) * S + lane) * 2 + 1] : 0.f;
+    float ps = lane < S ? ws.partials[(static_cast<int64_t>(row) * S + lane) * 2 + 1] : 0.f;
+    ps = pm > -INFINITY ? ps : 0.f;
     const float mx = wave_max(pm);
     const float ex = pm > -INFINITY ? expf(pm - mx) : 0.f;
-    float sum = 0.f;
+    float sum = 0.f;                                    // (an empty range has exponential 0 and sum 0: the step adds nothing)
+#pragma unroll 8
     for (int s2 = 0; s2 < S; ++s2) {
       const float es = __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(__float_as_uint(ex)), s2)));
       const float ss = __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(__float_as_uint(ps)), s2)));
-      const float ms = __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(__float_as_uint(pm)), s2)));
-      if (ms > -INFINITY) sum = __fmaf_rn(ss, es, sum);
+      sum = __fmaf_rn(ss, es, sum);
     }
     if (lane == 0) { s_mx = mx; s_sum = sum; }
   }
   __syncthreads();
   const float mx = s_mx, sum = s_sum;
-  if (tid == 0) {
-    int acc = 0, has = 0, bad = 0;
-    float front = -INFINITY;
-    for (int c = 0; c < R; ++c) {
-      pre[c] = acc;
-      if (m_cnt[c] < 0) bad = 1; else acc += m_cnt[c];
-      if (m_left[c]) { has = 1; front = fmaxf(front, m_front[c]); }
-    }
-    pre[R] = acc;
-    if (top_k <= 0 || acc == 0 || acc >= kDirect) bad = 1;
-    if (!(t > 0.f) || !(sum > 0.f) || !(sum < INFINITY) || !(mx > -INFINITY) || !(mx < INFINITY)) bad = 1;
-    s_front = front; s_has_front = has; s_bad = bad; s_unusable = 0;
-  }
-  __syncthreads();
-  if (!s_bad) {                                         // (workgroup-uniform)
+  // (workgroup-uniform) the candidates cannot decide the row
+  const bool bad = s_broken || top_k <= 0 || s_acc == 0 || s_acc >= kDirect || !(t > 0.f) || !(sum > 0.f) || !(sum < INFINITY) || !(mx > -INFINITY) ||
+                   !(mx < INFINITY);
+  if (!bad) {
     if (top_k > p.V) top_k = p.V;
     const unsigned long long p_fix = top_p_fix_superset(top_p);
     bool have[2];
@@ -1556,13 +1625,52 @@ __global__ __launch_bounds__(kT) void sample_finish_fast_kernel(SampleParams p, 
       pbits[u] = have[u] ? __float_as_uint(softmax_prob(__uint_as_float(lb[u]), t, mx, sum)) : 0u;
     }
     // ---- prune to a prefix of the descending order that holds top_k elements or top_p (+ 2^-22) of the mass, whichever comes
-    // first: a two-level select on the 16-bit logit keys with count and fixed-point mass histograms (order-independent).  The
-    // candidates dropped here join the elements the ranges left out: the frontier rises to the largest of them. ----
+    // first, by count and fixed-point mass histograms (order-independent) over the 16-bit logit keys below the row's largest: a key a
+    // bin where the cut lies within 1023 keys of it (eight binades; nearly every row), a two-level select otherwise.  (The top byte of
+    // the key put a row's candidates into two or three bins, whose LDS atomics then queue: 4.2 -> 2 us.)  The candidates dropped here
+    // join the elements the ranges left out: the frontier rises to the largest of them. ----
     uint32_t cutkey = 0;
     bool found_any = true;
+    const uint32_t topkey = s_top >> 16;
+    int near_cut;
     {
-      // (both levels' histograms were cleared before the kernel's first barrier: level 0 in hist_cnt / hist_sum, level 1 in
-      // part_cnt[0..255] / part_sum[16..271]; three barriers per level)
+      uint32_t bin[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const uint32_t d = topkey - key16[u];           // (>= 0: no candidate is larger than the largest logit)
+        bin[u] = d < kT - 1u ? d : kT - 1u;
+        if (have[u]) {
+          atomicAdd(&sm.part_cnt[bin[u]], 1u);
+          atomicAdd(&sm.part_sum[bin[u]], static_cast<unsigned long long>(to_fix(__uint_as_float(pbits[u]))));
+        }
+      }
+      __syncthreads();
+      const uint32_t my_c = sm.part_cnt[tid];           // thread = bin
+      const unsigned long long my_s = sm.part_sum[tid];
+      uint32_t vc = wave_prefix(my_c);
+      unsigned long long vs = wave_prefix(my_s);
+      if (lane == 63) { sm.wave_a[wid] = static_cast<int>(vc); sm.hist_sum[wid] = vs; }
+      __syncthreads();
+      const uint32_t before_c = wave_prefix(lane < wid ? static_cast<uint32_t>(sm.wave_a[lane]) : 0u);
+      const unsigned long long before_s = wave_prefix(lane < wid ? sm.hist_sum[lane] : 0ull);
+      vc += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(before_c), 63));
+      vs += static_cast<unsigned long long>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(before_s >> 32), 63))) << 32 |
+            static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(before_s), 63));
+      const bool cond_incl = static_cast<int64_t>(vc) >= top_k || vs >= p_fix;
+      const bool cond_excl = static_cast<int64_t>(vc - my_c) >= top_k || vs - my_s >= p_fix;
+      if (cond_incl && !cond_excl) s_near = tid;
+      __syncthreads();
+      near_cut = s_near;
+    }
+    if (near_cut >= 0 && near_cut < kT - 1) {
+      cutkey = topkey - static_cast<uint32_t>(near_cut);
+    } else if (near_cut < 0) {
+      found_any = false;                                // the whole list is inside both limits
+    } else {
+      if (tid < 256) { sm.hist_cnt[tid] = 0; sm.hist_sum[tid] = 0; }
+      else if (tid < 512) { sm.part_cnt[tid - 256] = 0; sm.part_sum[16 + tid - 256] = 0; }
+      __syncthreads();
+      // (level 0 in hist_cnt / hist_sum, level 1 in part_cnt[0..255] / part_sum[16..271]; three barriers per level)
       uint32_t base_c = 0;
       unsigned long long base_s = 0;
 #pragma unroll
@@ -1617,61 +1725,69 @@ __global__ __launch_bounds__(kT) void sample_finish_fast_kernel(SampleParams p, 
       }
       if (!found_any) cutkey = 0;
     }
-    // ---- compact the survivors, in list order, into the row routine's candidate arrays ----
-    bool keep[2];
-    float dropped = s_has_front ? s_front : -INFINITY;   // the largest logit NOT in the list handed on: left out by a range, or dropped here
-    int any_out = s_has_front;
+    // ---- compact the survivors, in any order (the rules rank them by value and token), into the row routine's candidate arrays ----
+    float dropped = -INFINITY;                          // the largest candidate dropped here
+    bool keep[2], any_out = false;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       keep[u] = have[u] && key16[u] >= cutkey;
-      if (have[u] && !keep[u]) { dropped = fmaxf(dropped, __uint_as_float(lb[u])); any_out = 1; }
+      if (have[u] && !keep[u]) { dropped = fmaxf(dropped, __uint_as_float(lb[u])); any_out = true; }
     }
     const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     const unsigned long long b0 = __ballot(keep[0]), b1 = __ballot(keep[1]);
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      dropped = fmaxf(dropped, __shfl_xor(dropped, off, 64));
-      any_out |= __shfl_xor(any_out, off, 64);
+    if (__ballot(any_out) != 0ull) {                    // (wave-uniform)
+      dropped = wave_max(dropped);
+      if (lane == 0) atomicMax(&s_front, order32(dropped));
+    }
+    if ((b0 | b1) != 0ull) {                            // (wave-uniform)
+      int at = 0;
+      if (lane == 0) at = atomicAdd(&s_n, __popcll(b0) + __popcll(b1));
+      at = __builtin_amdgcn_readfirstlane(at);
+      if (keep[0]) { const int pos = at + __popcll(b0 & lt_mask); sm.cand_val[pos] = pbits[0]; sm.cand_tok[pos] = tok[0]; }
+      if (keep[1]) { const int pos = at + __popcll(b0) + __popcll(b1 & lt_mask); sm.cand_val[pos] = pbits[1]; sm.cand_tok[pos] = tok[1]; }
     }
     __syncthreads();
-    if (lane == 0) { sm.wave_a[wid] = __popcll(b0); sm.wave_b[wid] = __popcll(b1); sm.red[wid] = dropped; sm.s_rank[wid] = any_out; }
-    __syncthreads();
-    int off0 = 0, tot0 = 0, off1 = 0, n = 0, has_front_i = 0;
-    float front = -INFINITY;
-    for (int w = 0; w < kNW; ++w) {
-      if (w < wid) { off0 += sm.wave_a[w]; off1 += sm.wave_b[w]; }
-      tot0 += sm.wave_a[w];
-      n += sm.wave_b[w];
-      front = fmaxf(front, sm.red[w]);
-      has_front_i |= sm.s_rank[w];
-    }
-    n += tot0;
-    if (keep[0]) { const int pos = off0 + __popcll(b0 & lt_mask); sm.cand_val[pos] = pbits[0]; sm.cand_tok[pos] = tok[0]; }
-    if (keep[1]) { const int pos = tot0 + off1 + __popcll(b1 & lt_mask); sm.cand_val[pos] = pbits[1]; sm.cand_tok[pos] = tok[1]; }
+    const int n = s_n;
+    const bool has_front = s_front != 0u;
+    const float front = value_of_order32(s_front);
     Frontier fr;
     fr.unusable = &s_unusable;
     fr.prob = 0.f;
     fr.key = 0u;
-    const bool has_front = has_front_i != 0;
     if (has_front) {
       fr.prob = softmax_prob(front, t, mx, sum);
       fr.key = key_of(fr.prob);
     }
-    __syncthreads();
     // A long list that reaches neither limit (top-p over a wide nucleus without top-k) and has elements behind it: the frontier
     // test below would send the row the long way after an O(n^2) ranking of the whole list -- go there at once.
     if (!found_any && has_front && n > 256 && !p.min_ps) {
       if (tid == 0) s_unusable = 1;
     } else if (n <= 64) {                               // (workgroup-uniform) what a pruned list almost always is
+      if (wid < 4) {                                    // ranks, a quarter of the list a wave; the logs beside them
+        const uint32_t key = lane < n ? key_of(__uint_as_float(sm.cand_val[lane])) : 0u;
+        const int tk = lane < n ? sm.cand_tok[lane] : 0x7fffffff;
+        int rank = 0;
+#pragma unroll
+        for (int jj = 0; jj < 16; ++jj) {
+          const int j = 16 * wid + jj;
+          const uint32_t kj = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(key), j));
+          const int tj = __builtin_amdgcn_readlane(tk, j);
+          rank += (j < n) && ((kj > key) || (kj == key && tj < tk));
+        }
+        s_part[wid * 64 + lane] = rank;
+      } else if (wid == 4) {
+        s_log[lane] = log(static_cast<double>(lane < n ? __uint_as_float(key_of(__uint_as_float(sm.cand_val[lane]))) : 0.f));
+      }
+      __syncthreads();
       if (wid == 0)
-        finish_small_list(p, row, sm.cand_val, sm.cand_tok, sm.keys, sm.toks, n, top_k, top_p, p.min_ps != nullptr, min_p, seed, spos,
-                          has_front ? &fr : nullptr);
+        finish_small_list(p, row, sm.cand_val, sm.cand_tok, sm.keys, sm.toks, n, top_k, top_p, p.min_ps != nullptr, min_p, s_part, s_log,
+                          s_log_sorted, s_gumbel, has_front ? &fr : nullptr);
     } else {
       sample_row(p, row, sm, n, has_front ? &fr : nullptr);
     }
     __syncthreads();
   }
-  const bool redo = s_bad || s_unusable;
+  const bool redo = bad || s_unusable;
   if (tid == 0) ws.fallback[row] = redo ? 1 : 0;
   if (!redo) return;
   // ---- the long way, for this row only: its probabilities into the scratch matrix (this workgroup writes the whole row and is the
@@ -1897,11 +2013,14 @@ int sgl_amd_top_k_top_p_min_p_sample_from_logits(const void* logits, int logits_
   p.out_ids = out_ids; p.ws_keys = static_cast<uint32_t*>(ws_keys); p.ws_toks = static_cast<int32_t*>(ws_toks);
   p.out_n_keep = out_n_keep; p.filtered = 1;
   const FastWs ws = fast_ws_view(ws_fast, batch, num_splits);
-  const int G = (num_splits >= kFastRangesMax && num_splits % kFastRangesMax == 0) ? num_splits / kFastRangesMax : 1;
+  const int64_t per_range = ((vocab + num_splits - 1) / num_splits + 3) / 4 * 4;
+  int G = (num_splits >= kFastRangesMax && num_splits % kFastRangesMax == 0) ? num_splits / kFastRangesMax : 1;
+  // a workgroup's fixed work is that of about 20 columns a thread, so it takes up to 8 slots while two workgroups a CU are left
+  // ([128, 32000]: 40 -> 35 us; sixteen slots at [128, 128256] lose 1 us to the longer chain)
+  while (2 * G <= 4 && num_splits % (2 * G) == 0 && batch * (num_splits / (2 * G)) >= 512 && 2 * G * ((per_range + 1023) / 1024) <= 8) G *= 2;
   const int R = num_splits / G;
   SGL_CHECK_ARG(R <= kFastRangesMax, "sample_from_logits: num_splits must be <= 16 or a multiple of 16");
-  const int64_t per = ((vocab + num_splits - 1) / num_splits + 3) / 4 * 4;
-  const int J = static_cast<int>((per + 1023) / 1024);
+  const int J = static_cast<int>((per_range + 1023) / 1024);
   SGL_CHECK_ARG(G <= 4 && G * J <= kFastSlots, "sample_from_logits: a workgroup holds at most 16384 columns of a row (vocab / ranges too large)");
   const dim3 cgrid(R, static_cast<unsigned>(batch));
 #define SGL_LAUNCH_FAST(IN_)                                                                                                               \

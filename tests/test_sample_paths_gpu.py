@@ -1,0 +1,51 @@
+"""GPU tests of the branches inside the one-call sampler: the division by the temperature through one reciprocal, the single- and the
+two-level cut of the candidate lists, one to four softmax ranges a workgroup.  Ids and kept counts must equal those of the two calls
+(softmax over the row, then sample from the probabilities) on every row, bit for bit."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# (rows, columns): 4, 2 and 1 ranges a workgroup in 16 groups; ranges joined further for short rows; tails of 1, 2 and 3 columns
+@pytest.mark.parametrize("B,V", [(32, 128256), (64, 151936), (128, 128256), (128, 32000), (64, 65537), (128, 40002), (16, 33003), (2, 50257)])
+@pytest.mark.parametrize("fp32", [False, True])
+def test_one_call_equals_softmax_then_sample(device, B, V, fp32):
+    from sglang_amd import kernels as K
+
+    Vp = V + (-V) % 4                                   # (rows start 8- or 16-byte aligned)
+    g = torch.Generator(device=device).manual_seed(V + B)
+    rn = lambda *s: torch.randn(s, generator=g, device=device)
+    lg = rn(B, Vp) * 2.5
+    temps = torch.rand((B, 1), generator=g, device=device) + 0.4
+    temps[0] = 1.0
+    temps[1] = 1.0e-7                                   # below the reciprocal's range
+    if B >= 16:
+        temps[2] = 3.0e6                                # above it: a flat row
+        lg[3] -= 9.0                                    # the cut far (in keys) below the largest: the two-level select, across zero
+        lg[4] = -lg[4].abs() * 0.01 - 1e-4              # negative rows
+        lg[5, torch.randperm(Vp, generator=torch.Generator().manual_seed(1))[: Vp - 90].to(device)] = -float("inf")   # a masked vocabulary
+        lg[6, 1:] = -float("inf")                       # one token left
+        lg[7] *= 1e30                                   # quotients near the largest float
+        lg[8] = 0.0
+        lg[9] = lg[9].abs() * -0.0                      # -0 beside +0
+        lg[9, ::3] = 0.0
+        lg[10, 17] = float("nan")
+        lg[11, 19] = float("inf")
+        lg[12] = rn(Vp) * 1e-39                         # denormals
+    padded = lg if fp32 else lg.to(torch.bfloat16)
+    lg = padded[:, :V]
+    top_k = torch.tensor(([50, 1, 64, 40, 1 << 30, 7, 20, 60] * 16)[:B], dtype=torch.int32, device=device)
+    top_p = torch.tensor(([0.9, 1.0, 1.0, 0.95, 0.6, 0.999] * 22)[:B], device=device)
+    seeds, pos = torch.arange(B, device=device) * 977 + 5, torch.arange(B, device=device)
+    for min_p in (None, torch.full((B,), 0.02, device=device)):
+        probs = K.softmax_temperature_(padded.clone()[:, :V], temps) if fp32 else K.softmax_temperature_from_bf16(lg, temps)
+        want, want_n = K.top_k_top_p_min_p_sample(probs, top_k, top_p, min_p, seeds, pos, return_n_keep=True)
+        out = K.sample_from_logits(lg, temps, top_k, top_p, min_p, seeds, pos, return_n_keep=True, return_fallback=True)
+        assert out is not None
+        got, got_n, redone = out
+        same = (got == want) & (got_n == want_n)
+        bad = same.logical_not().nonzero().flatten().tolist()
+        assert not bad, [(r, int(got[r]), int(want[r]), int(got_n[r]), int(want_n[r]), int(redone[r])) for r in bad]
+        usual = [r for r in range(13, B) if int(top_k[r]) <= 64]
+        assert not any(redone.tolist()[r] for r in usual)          # gaussian rows are decided by their candidates
