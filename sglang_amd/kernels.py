@@ -17,7 +17,8 @@ _BF16 = torch.bfloat16
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """Handle of the current stream of the current device (without the Stream object torch.cuda.current_stream() builds: 2.8 us a launch)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -179,6 +180,15 @@ def rotary_embedding(positions: torch.Tensor, query: torch.Tensor, key: torch.Te
 
 
 # ----------------------------------------------------------------------- kv store
+def _row_width(x: torch.Tensor, n: int) -> Tuple[int, int]:
+    """(width, stride) of x.view(n, -1); the view itself is only made, or refused, for what is not [n > 1, heads, dim] with dense rows."""
+    shape, stride = x.shape, x.stride()
+    if len(shape) == 3 and shape[0] == n > 1 and shape[1] and shape[2] and stride[2] == 1 and stride[1] == shape[2]:
+        return shape[1] * shape[2], stride[0]
+    x = x.view(n, -1)
+    return x.shape[1], x.stride(0)
+
+
 def store_kv_cache(k: torch.Tensor, v: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, loc: torch.Tensor,
                    num_kv_heads: Optional[int] = None, head_dim: Optional[int] = None, kv_fp8: bool = False,
                    k_scale: float = 1.0, v_scale: float = 1.0, page_size: int = 1, hnd: bool = False) -> None:
@@ -196,11 +206,11 @@ def store_kv_cache(k: torch.Tensor, v: torch.Tensor, k_cache: torch.Tensor, v_ca
                     T, num_kv_heads, head_dim, k2.stride(0), v2.stride(0), num_kv_heads * head_dim, 1 if kv_fp8 else 0,
                     float(k_scale), float(v_scale), int(page_size), 1 if hnd else 0, _stream())
         return
-    k2, v2 = k.view(T, -1), v.view(T, -1)
-    kc, vc = k_cache.view(k_cache.shape[0], -1), v_cache.view(v_cache.shape[0], -1)
-    _need(k2.dtype == kc.dtype == _BF16 and v2.dtype == vc.dtype == _BF16, "store_kv_cache: bf16 only")
-    native.call("sgl_amd_store_kv_cache", k2.data_ptr(), v2.data_ptr(), kc.data_ptr(), vc.data_ptr(), loc.data_ptr(), T,
-                k2.shape[1], v2.shape[1], k2.stride(0), v2.stride(0), kc.stride(0), vc.stride(0), _stream())
+    _need(k.dtype == k_cache.dtype == _BF16 and v.dtype == v_cache.dtype == _BF16, "store_kv_cache: bf16 only")
+    (kw, ks), (vw, vs) = _row_width(k, T), _row_width(v, T)
+    (_, kcs), (_, vcs) = _row_width(k_cache, k_cache.shape[0]), _row_width(v_cache, v_cache.shape[0])
+    native.call("sgl_amd_store_kv_cache", k.data_ptr(), v.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), loc.data_ptr(), T,
+                kw, vw, ks, vs, kcs, vcs, _stream())
 
 
 # ----------------------------------------------------------------------- metadata
@@ -392,15 +402,15 @@ def extend_attention(q: torch.Tensor, out: torch.Tensor, k_cache: torch.Tensor, 
                     float(k_scale), float(v_scale), int(page_size), 1 if hnd else 0, int(sliding_window), float(logit_cap),
                     _ptr(custom_mask), _ptr(mask_indptr), 1 if skip_prefix_custom_mask else 0, _stream())
         return out
-    _need(q.dtype == _BF16 and k_cache.dtype == _BF16 and v_cache.dtype == _BF16 and out.dtype == _BF16, "extend_attention: bf16 only")
-    _need(seq_lens.dtype == torch.int32 and prefix_lens.dtype == torch.int32 and qo_indptr.dtype == torch.int32,
-          "extend_attention: int32 lens")
+    _need(q.dtype == k_cache.dtype == v_cache.dtype == out.dtype == _BF16, "extend_attention: bf16 only")
+    _need(seq_lens.dtype == prefix_lens.dtype == qo_indptr.dtype == torch.int32, "extend_attention: int32 lens")
     _need(req_pool_indices.dtype == torch.int64 and req_to_token.dtype == torch.int32, "extend_attention: index dtypes")
-    _need(q.stride(2) == 1 and q.stride(1) == D and out.stride(2) == 1 and out.stride(1) == D, "extend_attention: q/out head layout")
-    _need(k_cache.stride(2) == 1 and k_cache.stride(1) == D and v_cache.stride(1) == D, "extend_attention: cache layout")
-    if max_kv_len > 0 and k_cache.stride(0) == v_cache.stride(0):
+    q_s, o_s, k_s, v_s = q.stride(), out.stride(), k_cache.stride(), v_cache.stride()
+    _need(q_s[2] == 1 and q_s[1] == D and o_s[2] == 1 and o_s[1] == D, "extend_attention: q/out head layout")
+    _need(k_s[2] == 1 and k_s[1] == D and v_s[1] == D, "extend_attention: cache layout")
+    if max_kv_len > 0 and k_s[0] == v_s[0]:
         return _extend_attention_kv(q, out, k_cache, v_cache, req_to_token, req_pool_indices, seq_lens, prefix_lens, qo_indptr, max_extend_len,
-                                    max_kv_len, sm_scale, causal, False, 1.0, 1.0, k_cache.stride(0))
+                                    max_kv_len, sm_scale, causal, False, 1.0, 1.0, k_s[0])
     native.call("sgl_amd_extend_attention", q.data_ptr(), out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
                 req_to_token.data_ptr(), req_to_token.stride(0), req_pool_indices.data_ptr(), seq_lens.data_ptr(),
                 prefix_lens.data_ptr(), qo_indptr.data_ptr(), seq_lens.numel(), int(max_extend_len), Hq, Hkv, D,
@@ -414,14 +424,14 @@ def _extend_attention_kv(q, out, k_cache, v_cache, req_to_token, req_pool_indice
                          max_kv_len: int, sm_scale: float, causal: bool, kv_fp8: bool, k_scale: float, v_scale: float, row_stride: int) -> torch.Tensor:
     """extend_attention over a token-major pool whose longest context is known (arguments checked by the caller)."""
     (T, Hq, D), Hkv, B = q.shape, k_cache.shape[1], seq_lens.numel()
-    parts = 1
-    if max_kv_len > 256 and out.stride(0) % 8 == 0:          # (a split of four tiles or fewer never pays: not worth asking)
+    parts, out_stride = 1, out.stride(0)
+    if max_kv_len > 256 and out_stride % 8 == 0:          # (a split of four tiles or fewer never pays: not worth asking)
         parts = native.lib().sgl_amd_extend_attention_parts(B, int(max_extend_len), int(max_kv_len), Hq, Hkv, D)
     ws = torch.empty(parts * T * Hq * (D + 2), dtype=torch.float32, device=q.device) if parts > 1 else None
     acc = ws.data_ptr() if parts > 1 else None
     native.call("sgl_amd_extend_attention_kv", q.data_ptr(), out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), req_to_token.data_ptr(),
                 req_to_token.stride(0), req_pool_indices.data_ptr(), seq_lens.data_ptr(), prefix_lens.data_ptr(), qo_indptr.data_ptr(), B, T,
-                int(max_extend_len), int(max_kv_len), Hq, Hkv, D, q.stride(0), out.stride(0), row_stride, float(sm_scale), 1 if causal else 0,
+                int(max_extend_len), int(max_kv_len), Hq, Hkv, D, q.stride(0), out_stride, row_stride, float(sm_scale), 1 if causal else 0,
                 1 if kv_fp8 else 0, float(k_scale), float(v_scale), parts, acc, acc + 4 * parts * T * Hq * D if parts > 1 else None, _stream())
     return out
 

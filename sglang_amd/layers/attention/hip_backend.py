@@ -372,7 +372,7 @@ class HipAttnBackend(AttentionBackend):
             self._save_kv(layer, forward_batch, k, v)
         m = self.forward_metadata
         q3 = q.view(-1, layer.tp_q_head_num, layer.qk_head_dim)
-        o = torch.empty(q3.shape, dtype=q3.dtype, device=q3.device)
+        o = torch.empty_like(q3, memory_format=torch.contiguous_format)
         # (compared by VALUE: under sglang `layer` is the reference's RadixAttention and attn_type a member of the reference's
         # own AttentionType enum, radix_attention.py:58-66 -- another class than this package's look-alike)
         causal = getattr(layer.attn_type, "value", layer.attn_type) != "encoder_only"

@@ -112,7 +112,7 @@ def last_error() -> str:
 
 def call(name: str, *args) -> None:
     """Call an int-returning entry point; raise RuntimeError on a non-zero status."""
-    fn = getattr(lib(), name)
+    fn = getattr(_lib or lib(), name)
     rc = fn(*args)
     if rc != 0:
         raise RuntimeError(f"{name} failed (status {rc}): {last_error()}")
