@@ -41,8 +41,8 @@ constexpr float kNegBig = -1.0e30f;
 constexpr int64_t kSingleShotHardCap = 16384;    // the largest value the switch below may take: what the plan clears for is decided against THIS, not the switch
 constexpr int64_t kSingleShotUnits = 10240;
 // ... and for requests of at most 8 query rows a kv head behind tables of at least kSpanChunks chunks, whose private tokens the plan cuts into
-// spans: the looping form.  us a layer, Llama-3-8B heads, single-shot against spans, at an 8 k-token table: 8 requests of 5 k 57 / 54, 16 of
-// 4 k 77 / 73, 2 of 7 k 25.0 / 24.0; 4 of 17 k at a 32 k-token table 82.8 / 64.6.  At tables of 1.2 and 2.5 k tokens, whose requests are
+// spans: the looping form.  us a layer, Llama-3-8B heads, single-shot against spans, at an 8 k-token table: 8 requests of 5 k 57 / 51, 16 of
+// 4 k 77 / 70, 2 of 7 k 25.0 / 24.0; 4 of 17 k at a 32 k-token table 82.8 / 64.6.  At tables of 1.2 and 2.5 k tokens, whose requests are
 // short: 64 of 0.9 k 51.9 / 53.1, 64 behind a shared prefix 22.5 / 23.5, 32 of 0.3 k 15.8 / 17.9.
 constexpr int64_t kSpanSingleShotUnits = 2048;
 constexpr int kSpanChunks = 64;
@@ -136,8 +136,8 @@ __device__ __forceinline__ float lane_rows_max(float x) {
 // ds_read_b64_tr_b16.  The next tile's K rows are asked for once this tile's scores are formed, its V rows once this tile's have left
 // the registers, so a wave always has rows in flight; sixteen waves a CU do the rest (16 tokens, not 32: at 32 the 128 registers spill,
 // 256 against 211 us for 32 requests of 2 k tokens in e4m3).
-// What bounds it: the gathered rows -- four layers of 37 requests of 0.9 to 5.1 k tokens in e4m3 481 -> 296 us (2.0 -> 3.3 TB/s), 128
-// requests of 1.5 k in bf16 910 -> 709 us (4.8 TB/s; a large copy reaches 4.9).  Before, a unit was 128 tokens staged through one image
+// What bounds it: the gathered rows -- four layers of 37 requests of 0.9 to 5.1 k tokens in e4m3 481 -> 268 us (2.0 -> 3.6 TB/s), 128
+// requests of 1.5 k in bf16 910 -> 729 us (4.6 TB/s; a large copy reaches 4.9).  Before, a unit was 128 tokens staged through one image
 // behind six barriers.  A bf16 item of 128 tokens keeps that form: its rows come in one burst, 257 against 265 us in the shared-prefix batch.
 // Image: row (token) t at t * 2 D bytes, its 16-byte piece c in slot c ^ kSw(t): the four rows of a transposing read lie on distinct banks.
 template <int D, bool FP8, bool HND>

@@ -35,11 +35,14 @@ struct CascadePlanView {
   int32_t* pieces;
 };
 
-// (span, kv head) units that a plan of spans aims at, the shared items taken off: one a resident workgroup of the looping kernel (four a CU at
-// 128 registers), so that all of them run at once and end together.  37 requests of 0.9 to 5.1 k tokens, e4m3 rows, four layers: 296 us;
-// 2048 units 315, 1280 320 (a second, partial round).  A span of one 64-token tile would need more partial slots than context chunks + 1.
-constexpr int kSpanUnits = 1024;
-constexpr int kMinSpanTiles = 2;
+// (span, kv head) units that a plan of spans aims at, the shared items taken off: three a compute unit.  The looping kernel's registers would
+// let four run, but the chip starts about 740 of a thousand workgroups at once and the rest only as those end, a second round of a fifth of
+// the work (us for four layers at 1024 / 768 units: 37 requests of 0.9 to 5.1 k tokens in e4m3 278 / 268, 16 of 4 k in bf16 297 / 280, 64
+// behind shared prefixes, eight layers, 255 / 234; 640 and 896 units lose 4 to 8 %; with 32 kv heads of one row, where a workgroup waits
+// for its instructions more than for memory, 321 / 345).  Below three 64-token tiles a span the items' single burst is quicker
+// (32 requests of 190 tokens behind a shared prefix 93 us, 100 in spans of two).
+constexpr int kSpanUnits = 768;
+constexpr int kMinSpanTiles = 3;
 
 __host__ __device__ inline int64_t cascade_plan_ints(int64_t batch, int64_t max_items) {
   return 8 + batch + batch + (batch + 1) + batch + batch + 8 * max_items + batch + 2 * batch + batch + (kSpanUnits + 1) + 8 * (batch + kSpanUnits) + 3;

@@ -8,7 +8,7 @@ from oracle import ops as oo
 
 pytestmark = pytest.mark.gpu
 BF = torch.bfloat16
-SPAN_UNITS, MIN_TILES, TILE, CHUNK = 1024, 2, 64, 128
+SPAN_UNITS, MIN_TILES, TILE, CHUNK = 768, 3, 64, 128
 
 
 def _spans(lens, shared, n_shared_items, Hkv):
