@@ -303,9 +303,12 @@ __global__ __launch_bounds__(kThreads, 4) void cascade_chunk_loop_kernel(ChunkPa
   __shared__ U4 sm[(kChunk / (D > 64 ? D / 64 : 1)) * (D / 8)];
   __shared__ float ml_s[64];
   __shared__ U4 side_s[D > 64 ? 4 * 8 * (D - 64) / 4 : 1];
+  // the line of the workgroup's first item record travels with the header (a grid never reaches beyond max_items x kv heads)
+  const int first_rec = cascade_plan_view(p.plan, p.batch, p.max_items).items[8 * (blockIdx.x / static_cast<unsigned>(p.num_kv_heads))];
   // one hop for all of the header that the loop needs: the list's length (shared items, then private items or spans) and what the tail is
   const int n_items = __builtin_amdgcn_readfirstlane(p.plan[5]), n_shared = __builtin_amdgcn_readfirstlane(p.plan[3]);
   const bool spans = __builtin_amdgcn_readfirstlane(p.plan[4]) > 0;
+  asm volatile("" ::"v"(first_rec));
   const int n_units = n_items * p.num_kv_heads;
   const int G = static_cast<int>(gridDim.x), w0 = static_cast<int>(blockIdx.x);
   // The kernel's one argument sits at the start of the kernarg segment; every pass re-reads it through an address the
