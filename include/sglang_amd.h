@@ -511,9 +511,9 @@ int sgl_amd_extend_attention_ex(const void* q, void* out, const void* k_cache, c
                                 void* stream);
 /* Extend attention of a token-major pool (no window, cap or mask) whose longest context (prefix + new tokens) the caller knows: with few
  * new tokens behind a long one the keys of a request are dealt over `parts` workgroups and their fp32 rows merged.
- * sgl_amd_extend_attention_parts says how many parts pay (1: none).  For parts > 1 the caller owns ws_acc fp32
+ * sgl_amd_extend_attention_parts says how many parts pay (1: none; num_tokens as in the launch).  For parts > 1 the caller owns ws_acc fp32
  * [parts, num_tokens, H_q, D] and ws_ml fp32 [parts, num_tokens, H_q, 2]; num_tokens >= qo_indptr[batch]. */
-int sgl_amd_extend_attention_parts(int64_t batch, int max_extend_len, int max_kv_len, int num_q_heads, int num_kv_heads, int head_dim);
+int sgl_amd_extend_attention_parts(int64_t batch, int64_t num_tokens, int max_extend_len, int max_kv_len, int num_q_heads, int num_kv_heads, int head_dim);
 int sgl_amd_extend_attention_kv(const void* q, void* out, const void* k_cache, const void* v_cache,
                                 const int32_t* req_to_token, int64_t req_to_token_stride,
                                 const int64_t* req_pool_indices, const int32_t* seq_lens,

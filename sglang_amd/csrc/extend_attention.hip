@@ -1369,9 +1369,18 @@ int extend_parts(int64_t wgs, int64_t rows, int max_kv_len, int head_dim) {
 // 289 / 302 us, 60 x 128 behind 896 182 / 197), unless the second half of a 256-row tile would be empty anyway (64 x 20 behind 3000 231 / 161).
 // Below (us, eight / four): 5 x 600 behind 1000 92 / 87, 8 x 300 behind 1000, 32 kv heads 102 / 85, 4 x 1024 cold 52 / 54.  At D = 64 four
 // waves were never slower (6 x 2000 cold 82 / 76, 4 x 1024 cold 29 / 23).
-bool extend_eight_waves(int64_t wgs8, int64_t wgs4, int head_dim) {
-  if (wgs8 < 256 || head_dim != 128 || wgs4 * 4 <= wgs8 * 5) return false;
-  return wgs8 > 512 || static_cast<double>((wgs8 + 255) / 256) <= 1.07 * (static_cast<double>(wgs4) / 512.0 + 0.3);
+// The counts are of the longest request's tiles.  Up to two rounds of those, where the launch knows its tokens, a request's last tile is
+// taken to be half full instead (6 ragged extends of 77 .. 271 behind 2862, 32 kv heads: 110 / 115, and the padded counts say four); past
+// them ragged batches stay with eight (8 of 60 .. 314 behind 1500, 64 / 8 heads: 112 / 121, and the held counts say four).
+bool extend_eight_waves(int64_t tokens, int64_t batch, int64_t rows, int group, int kv_heads, int head_dim) {
+  auto padded = [&](int tile) { return (rows + tile - 1) / tile * batch * kv_heads; };
+  auto held = [&](int tile) {
+    const int64_t n = (2 * tokens * group + batch * tile) / (2 * tile) * kv_heads;
+    return tokens > 0 && n < padded(tile) ? n : padded(tile);
+  };
+  constexpr int kFour = 32 * kPartWaves;
+  if (padded(256) < 256 || head_dim != 128 || padded(kFour) * 4 <= padded(256) * 5) return false;
+  return padded(256) > 512 || static_cast<double>((held(256) + 255) / 256) <= 1.07 * (static_cast<double>(held(kFour)) / 512.0 + 0.3);
 }
 
 template <int D, bool FP8>
@@ -1522,7 +1531,7 @@ static int extend_attention_any(const void* q, void* out, const void* k_cache, c
   // eligible for the 32x32 kernels (flag bit 0, or a forced shape but 8 x 2: the general kernel)
   const bool plain = !kv_layout_hnd && sliding_window < 0 && logit_cap == 0.f && custom_mask == nullptr && (g_extend_debug_flags & 1) == 0;
   const bool small = plain && g_extend_debug_shape == 0 && group <= 32 * kPartWaves && out_token_stride % 8 == 0 &&
-                     !extend_eight_waves(wgs(256), wgs(32 * kPartWaves), head_dim) && !(max_kv_len > 0 && max_kv_len <= kKvTile);
+                     !extend_eight_waves(num_tokens, batch, rows_total, group, num_kv_heads, head_dim) && !(max_kv_len > 0 && max_kv_len <= kKvTile);
   if (group <= 256 && wgs(256) >= 256) { mtw = 2; nwv = 8; }
   else if (group <= 64) { mtw = 1; nwv = 4; }
   if (const int v = g_extend_debug_shape) {                   // sgl_amd_debug_extend_attention_shape(): tests / tuning
@@ -1621,13 +1630,12 @@ int sgl_amd_extend_attention_ex(const void* q, void* out, const void* k_cache, c
                               sliding_window, logit_cap, custom_mask, mask_indptr, skip_prefix_custom_mask, 0, 0, 1, nullptr, nullptr, stream);
 }
 
-int sgl_amd_extend_attention_parts(int64_t batch, int max_extend_len, int max_kv_len, int num_q_heads, int num_kv_heads, int head_dim) {
+int sgl_amd_extend_attention_parts(int64_t batch, int64_t num_tokens, int max_extend_len, int max_kv_len, int num_q_heads, int num_kv_heads, int head_dim) {
   if (batch <= 0 || max_extend_len <= 0 || max_kv_len <= kKvTile || num_kv_heads <= 0 || num_q_heads % num_kv_heads != 0 ||
       (head_dim != 64 && head_dim != 128) || num_q_heads / num_kv_heads > 32 * kPartWaves || g_extend_debug_shape != 0 || g_extend_debug_flags != 0)
     return 1;
   const int group = num_q_heads / num_kv_heads;
-  auto wgs = [&](int rows) { return ((static_cast<int64_t>(max_extend_len) * group + rows - 1) / rows) * num_kv_heads * batch; };
-  if (extend_eight_waves(wgs(256), wgs(32 * kPartWaves), head_dim)) return 1;
+  if (extend_eight_waves(num_tokens, batch, static_cast<int64_t>(max_extend_len) * group, group, num_kv_heads, head_dim)) return 1;
   const int tokens = 32 * kPartWaves / group;               // whole tokens a tile, as the launch deals them
   const int64_t wgs4 = static_cast<int64_t>((max_extend_len + tokens - 1) / tokens) * num_kv_heads * batch;
   return extend_parts(wgs4, batch * static_cast<int64_t>(max_extend_len) * num_q_heads, max_kv_len, head_dim);

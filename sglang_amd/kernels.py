@@ -426,7 +426,7 @@ def _extend_attention_kv(q, out, k_cache, v_cache, req_to_token, req_pool_indice
     (T, Hq, D), Hkv, B = q.shape, k_cache.shape[1], seq_lens.numel()
     parts, out_stride = 1, out.stride(0)
     if max_kv_len > 256 and out_stride % 8 == 0:          # (a split of four tiles or fewer never pays: not worth asking)
-        parts = native.lib().sgl_amd_extend_attention_parts(B, int(max_extend_len), int(max_kv_len), Hq, Hkv, D)
+        parts = native.lib().sgl_amd_extend_attention_parts(B, T, int(max_extend_len), int(max_kv_len), Hq, Hkv, D)
     ws = torch.empty(parts * T * Hq * (D + 2), dtype=torch.float32, device=q.device) if parts > 1 else None
     acc = ws.data_ptr() if parts > 1 else None
     native.call("sgl_amd_extend_attention_kv", q.data_ptr(), out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), req_to_token.data_ptr(),

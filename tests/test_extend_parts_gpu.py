@@ -9,10 +9,10 @@ from test_kernels_gpu import BF, _random_case
 
 def test_rule_splits_few_rows_behind_long_contexts_only():
     parts = native.lib().sgl_amd_extend_attention_parts
-    assert parts(1, 203, 4003, 32, 8, 128) > 1 and parts(3, 22, 4571, 32, 32, 128) > 1 and parts(1, 500, 4500, 14, 2, 64) > 1
+    assert parts(1, 203, 203, 4003, 32, 8, 128) > 1 and parts(3, 66, 22, 4571, 32, 32, 128) > 1 and parts(1, 500, 500, 4500, 14, 2, 64) > 1
     for one in ((60, 128, 1024, 32, 8, 128), (6, 3107, 3107, 64, 8, 128), (1, 37, 37, 14, 2, 64), (1, 512, 512, 32, 8, 128), (1, 203, 0, 32, 8, 128),
                 (0, 5, 500, 32, 8, 128), (1, 5, 500, 32, 8, 96), (1, 5, 5000, 256, 1, 128)):
-        assert parts(*one) == 1, one
+        assert parts(one[0], one[0] * one[1], *one[1:]) == 1, one
 
 
 @pytest.mark.gpu
