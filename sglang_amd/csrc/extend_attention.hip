@@ -1135,6 +1135,10 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
     put_k(t & 1, kst);
     put_v((t + 1) & 1, vst);
     EXT_T(0);
+    // (8 waves: in phase 1, where most vector instructions are, a wave goes first; the SIMD's other wave has matrix instructions to issue
+    // beside them when it is in phase 2, and the older of two waves in phase 1 no longer holds the younger back: 708 -> 663 us for 12.6 k
+    // cold tokens of six requests, 64 / 8 heads, 396 -> 384 for 4096 behind 4000.  Two workgroups of 4 waves a CU lose by it, 183 -> 203.)
+    if constexpr (NWV == 8) __builtin_amdgcn_s_setprio(1);
     // ---- phase 1 ------------------------------------------------------------------------------------------
     constexpr int KF = 3;                            // K fragment sets: reads run two products ahead (1 or 3 ahead: same time)
     constexpr int G1 = 2 * KS;                       // products (16 at D = 128)
@@ -1213,6 +1217,7 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
 #pragma unroll
       for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(pp[i].x), "+v"(pp[i].y), "+v"(pp[i].z), "+v"(pp[i].w));
     }
+    if constexpr (NWV == 8) __builtin_amdgcn_s_setprio(0);
     EXT_T(1);
     if constexpr (HAVE_NEXT) mask_tile(sn, t + 1);
     EXT_T(2);
