@@ -461,6 +461,8 @@ __global__ __launch_bounds__(kThreads2, 1) void moe_gemm256_kernel(TiledParams p
     read_x(base, 0, xf[0]);
     read_w(base, 0, 1, wf[1]);
     wait_lgkm<4>();
+    // (a wave that multiplies goes ahead of one that reads fragments or asks for tiles: 2310 -> 2240 us for both projections of 3000 tokens)
+    __builtin_amdgcn_s_setprio(1);
     products(0, wf[0], xf[0]);
     MOE256_PINNED();
     read_w(base, 1, 0, wf[0]);
@@ -478,6 +480,7 @@ __global__ __launch_bounds__(kThreads2, 1) void moe_gemm256_kernel(TiledParams p
     wait_vm<1>();                                      // in order: everything older than this step's touch, i.e. the DMA of step kt + 1
     asm volatile("" ::"v"(pf_prev));                   // the touch of the step before has certainly returned: its register is free
 #else
+    __builtin_amdgcn_s_setprio(0);
     wait_vm<0>();
 #endif
     __builtin_amdgcn_s_barrier();
