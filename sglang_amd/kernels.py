@@ -1131,16 +1131,17 @@ def moe_tile_plan(numel: int, num_experts: int, n_up: int, n_down: int):
     `numel` (token, k) pairs: the 256 x 256 x 64 form once an expert owns enough rows that the 256-row alignment's padding
     (128 rows per expert on average) costs less than the form gains (measured on Mixtral's shapes, 4096 tokens = 1024 rows
     per expert: up projection 977 vs 714 TF/s, down projection 820-870 vs 715 with its 2.25 rounds of workgroups;
-    profiles/r04_exp4_moe_gemm_ab.json).  Experts of 256 to 767 rows take it where rounds and padding together promise 9 % or more (a K step of
-    64 costs 1.9 us a 256 x 256 tile, one a CU, and 1.2 us a 128 x 128 tile, two a CU; below that the estimate is no better than the spread of the
-    experts' sizes).  Measured, both products in us, 128 / 256 rows: 8 experts of 14336 / 4096 with 750 rows each 2771 / 2308, of 7168 / 4096 with
-    750 rows 1320 / 1249, 64 of 1408 / 2048 with 562 rows 1138 / 974; not taken: 8 of 7168 / 4096 with 500 rows 940 / 996, 16 of 2048 / 2048 with 750
-    rows 440 / 456."""
+    profiles/r04_exp4_moe_gemm_ab.json).  Experts of 256 to 767 rows take it where rounds and padding together promise 9.5 % or more (a K step of
+    64 costs 1.84 us a 256 x 256 tile, one a CU, and 1.2 us a 128 x 128 tile, two a CU; below that the estimate is no better than the spread of the
+    experts' sizes).  Measured, both products in us, 128 / 256 rows: 8 experts of 14336 / 4096 with 575 rows each 2257 / 2004, with 639 2524 / 2190,
+    of 7168 / 4096 with 650 rows 1194 / 1144, 64 of 1408 / 2048 with 468 rows 988 / 871, 16 of 2048 / 2048 with 750 rows 439 / 435; not taken: 8 of
+    14336 / 4096 with 405 rows 1647 / 1761 (with 475, nearer the line, 1916 / 1759), of 7168 / 4096 with 500 rows 911 / 938, 16 of 2048 / 2048 with
+    500 rows 310 / 353."""
     rows = numel // max(1, num_experts)
     if rows >= MOE_TILE256_MIN_ROWS_PER_EXPERT:
         return 256, 256, 256
     sizes = (numel / max(1, num_experts), num_experts, n_up, n_down)
-    if rows >= 256 and _moe_tiles_us(*sizes, 256, 256, 1.9) < 0.91 * _moe_tiles_us(*sizes, 128, 512, 1.2):
+    if rows >= 256 and _moe_tiles_us(*sizes, 256, 256, 1.84) < 0.905 * _moe_tiles_us(*sizes, 128, 512, 1.2):
         return 256, 256, 256
     return 128, 128, 128
 

@@ -4,6 +4,8 @@ from sglang_amd import kernels as K
 
 def test_experts_of_middling_size():
     for pairs, experts, up, down, rows in ((2 * 3000, 8, 14336, 4096, 256), (2 * 3000, 8, 7168, 4096, 256), (6 * 6000, 64, 1408, 2048, 256),
-                                           (2 * 2000, 8, 7168, 4096, 128), (2 * 1000, 8, 14336, 4096, 128), (2 * 6000, 16, 2048, 2048, 128),
+                                           (2 * 2300, 8, 14336, 4096, 256), (2 * 6000, 16, 2048, 2048, 256),
+                                           (2 * 2000, 8, 7168, 4096, 128), (2 * 1000, 8, 14336, 4096, 128), (2 * 4000, 16, 2048, 2048, 128),
+                                           (2 * 1622, 8, 14336, 4096, 128), (2 * 2048, 8, 14336, 4096, 128),
                                            (2 * 1020, 8, 14336, 4096, 128)):
         assert K.moe_tile_plan(pairs, experts, up, down) == (rows,) * 3, (pairs, experts, up, down)
