@@ -613,7 +613,7 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
   if (want < span_units / num_kv_heads / 2) want = span_units / num_kv_heads / 2;
   if (want < 1) want = 1;
   const int span = span_units > 0 ? (n_tiles + want - 1) / want : 0;     // tiles of a span
-  const bool spans = span >= kMinSpanTiles;            // (uniform)
+  const bool spans = span >= kMinSpanTiles && static_cast<int64_t>(total) * num_kv_heads > kOneRoundUnits;      // (uniform)
   if (tid == 0) {
     pv.header[0] = total < max_items ? total : max_items;
     pv.header[4] = spans ? span : 0;

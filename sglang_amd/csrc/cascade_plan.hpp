@@ -41,7 +41,9 @@ struct CascadePlanView {
 // behind shared prefixes, eight layers, 255 / 234; 640 and 896 units lose 4 to 8 %; with 32 kv heads of one row, where a workgroup waits
 // for its instructions more than for memory, 321 / 345).  Below three 64-token tiles a span the items' single burst is quicker
 // (32 requests of 190 tokens behind a shared prefix 93 us, 100 in spans of two).
+// Nor where the items are no more than run in one round (7 requests of 585 tokens, 32 kv heads: 896 items 123 us, 768 spans 125).
 constexpr int kSpanUnits = 768;
+constexpr int kOneRoundUnits = 1024;
 constexpr int kMinSpanTiles = 3;
 
 __host__ __device__ inline int64_t cascade_plan_ints(int64_t batch, int64_t max_items) {

@@ -8,7 +8,7 @@ from oracle import ops as oo
 
 pytestmark = pytest.mark.gpu
 BF = torch.bfloat16
-SPAN_UNITS, MIN_TILES, TILE, CHUNK = 768, 3, 64, 128
+SPAN_UNITS, MIN_TILES, ONE_ROUND, TILE, CHUNK = 768, 3, 1024, 64, 128
 
 
 def _spans(lens, shared, n_shared_items, Hkv):
@@ -17,7 +17,8 @@ def _spans(lens, shared, n_shared_items, Hkv):
     per_head = SPAN_UNITS // Hkv
     want = max(per_head - n_shared_items, per_head // 2, 1)
     span = (sum(tiles) + want - 1) // want
-    if span < MIN_TILES:
+    items = n_shared_items + sum(-(-(n - s) // CHUNK) for n, s in zip(lens, shared))
+    if span < MIN_TILES or items * Hkv <= ONE_ROUND:
         return 0, [-(-s // CHUNK) + -(-(n - s) // CHUNK) for n, s in zip(lens, shared)]
     slots, at = [], 0
     for t, s in zip(tiles, shared):
