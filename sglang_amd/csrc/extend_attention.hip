@@ -943,11 +943,11 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
   int n_tiles = (kv_end + kKvTile - 1) / kKvTile;
   // this part's tiles become tiles 0 .. n_tiles - 1 of the walk: the row of the request table, the end and the rows' limits move
   int part_begin = 0;
-  bool empty = false;
+  bool empty = n_tiles <= 0;                               // workgroup-uniform: no key to read (below)
   if constexpr (PARTS) {
     const int per = (n_tiles + p.parts - 1) / p.parts;
     const int t0 = part * per;
-    empty = t0 >= n_tiles;                                 // workgroup-uniform; such a part has no weight (below)
+    empty = t0 >= n_tiles;
     if (!empty) {
       n_tiles = n_tiles - t0 < per ? n_tiles - t0 : per;
       part_begin = t0 * kKvTile;
@@ -964,16 +964,20 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
   int row_limit = row_ok ? (causal ? prefix + q0 + r_tok + 1 : kv_len) : 0;
   if (row_limit > kv_len) row_limit = kv_len;
   const int row_off = (kvh * p.group + r_hg) * D;
-  if constexpr (PARTS) {
-    row_limit -= part_begin;
-    if (empty) {
+  if constexpr (PARTS) row_limit -= part_begin;
+  if (empty) {                                             // a part without keys has no weight, a request without keys gives zeros
+    if (PARTS && p.parts > 1) {
       if (row_ok && hi == 0) {
         float* ml = p.part_ml + 2 * (part * p.part_rows + static_cast<int64_t>(q_begin + q0 + r_tok) * (p.num_kv_heads * p.group) + kvh * p.group + r_hg);
         ml[0] = kNegBig;
         ml[1] = 0.f;
       }
-      return;
+    } else if (row_ok) {
+      uint16_t* op = p.out + static_cast<int64_t>(q_begin + q0 + r_tok) * p.out_stride + row_off;
+#pragma unroll
+      for (int c = 0; c < CPR / 2; ++c) *reinterpret_cast<U4*>(op + (2 * c + hi) * 8) = U4{0u, 0u, 0u, 0u};
     }
+    return;
   }
   U4 qreg[KS];                                      // Q^T operand of k-step s: dims 16 s + 8 h .. + 7 of the row
 #pragma unroll

@@ -45,3 +45,39 @@ def test_parts_against_the_oracle(device, Hq, Hkv, D, causal, fp8):
                     Hkv * D, c["scaling"], int(causal), int(fp8), 1.0, 1.0, parts, acc.data_ptr(), ml.data_ptr(), torch.cuda.current_stream().cuda_stream)
         torch.testing.assert_close(out[:T].float().cpu(), ref.float(), atol=4e-3, rtol=1e-2, msg=lambda m: f"{parts} parts: {m}")
         assert bool((out[T:] == 7.0).all()), parts
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [0, 82])
+@pytest.mark.parametrize("Hq,Hkv,D,fp8", [(32, 8, 128, False), (14, 2, 64, True)])
+def test_request_without_keys_gives_zero_rows(device, Hq, Hkv, D, fp8, shape):
+    """Query rows of a request whose context is empty (seq_lens 0) are zeros in one part, in several and in the eight-wave form; nothing is
+    read or written for it anywhere else (one part has no partial rows), and its neighbours' rows are what they are without it."""
+    c = _random_case(3, Hq, Hkv, D, [0, 300, 70], [40, 130, 65], seed=Hq + 3)
+    kc, vc = ((x.to(torch.float8_e4m3fn).view(torch.uint8) if fp8 else x).to(device) for x in (c["k_cache"], c["v_cache"]))
+    q, r2t, pool = c["q"].to(device), c["req_to_token"].to(device), c["req_pool_indices"].to(device)
+    pre, qo = torch.tensor([0, 300, 70], dtype=torch.int32, device=device), torch.tensor([0, 40, 170, 235], dtype=torch.int32, device=device)
+
+    def run(lens, parts):
+        out = torch.full_like(q, 7.0)
+        n = q.shape[0] * Hq
+        acc, ml = torch.full((parts, n, D), float("nan"), device=device), torch.full((parts, n, 2), float("nan"), device=device)
+        ws = (acc.data_ptr(), ml.data_ptr()) if parts > 1 else (None, None)
+        seq = torch.tensor(lens, dtype=torch.int32, device=device)
+        native.call("sgl_amd_extend_attention_kv", q.data_ptr(), out.data_ptr(), kc.data_ptr(), vc.data_ptr(), r2t.data_ptr(), r2t.stride(0), pool.data_ptr(),
+                    seq.data_ptr(), pre.data_ptr(), qo.data_ptr(), 3, q.shape[0], 130, 430, Hq, Hkv, D, q.stride(0), out.stride(0), Hkv * D, D ** -0.5, 1,
+                    int(fp8), 1.0, 1.0, parts, *ws, torch.cuda.current_stream().cuda_stream)
+        return out
+
+    native.call("sgl_amd_debug_extend_attention_shape", shape, 0)
+    try:
+        for parts in (1, 2) if shape == 0 else (1,):
+            want = run([40, 430, 135], parts)
+            for empty, rows in ((0, slice(0, 40)), (1, slice(40, 170)), (2, slice(170, 235))):
+                lens = [40, 430, 135]
+                lens[empty] = 0
+                got, ref = run(lens, parts), want.clone()
+                ref[rows] = 0.0
+                assert torch.equal(got, ref), (parts, empty)
+    finally:
+        native.call("sgl_amd_debug_extend_attention_shape", 0, 0)
