@@ -1066,7 +1066,7 @@ __global__ __launch_bounds__(kT) void sample_finish_ranges_kernel(SampleParams p
 // the matrix of 128 rows alone is 7 us of reading), at few rows, like the finish launch, a chain of dependent steps: 5 us until the
 // records and lists are there, 2.5 the cut, 1 the compaction, 3 rank, rules and arg-max.  us for the two launches, before this division
 // of the work (a true division per column, every column tested one by one for the list, byte-wide histograms, ranks, logs and noise all
-// by one wave) and now: [128, 128256] 53 / 42, [64, 128256] 42 / 32, [1, 128256] 34 / 23, [128, 32000] 40 / 27.
+// by one wave) and now: [128, 128256] 53 / 42, [64, 128256] 42 / 32, [1, 128256] 34 / 23, [128, 32000] 43 / 29.
 constexpr int kFastRangesMax = 16;
 constexpr int kFastCap = 127;
 constexpr int kFastK = 64;
@@ -2014,10 +2014,9 @@ int sgl_amd_top_k_top_p_min_p_sample_from_logits(const void* logits, int logits_
   p.out_n_keep = out_n_keep; p.filtered = 1;
   const FastWs ws = fast_ws_view(ws_fast, batch, num_splits);
   const int64_t per_range = ((vocab + num_splits - 1) / num_splits + 3) / 4 * 4;
-  int G = (num_splits >= kFastRangesMax && num_splits % kFastRangesMax == 0) ? num_splits / kFastRangesMax : 1;
-  // a workgroup's fixed work is that of about 20 columns a thread, so it takes up to 8 slots while two workgroups a CU are left
-  // ([128, 32000]: 40 -> 35 us; sixteen slots at [128, 128256] lose 1 us to the longer chain)
-  while (2 * G <= 4 && num_splits % (2 * G) == 0 && batch * (num_splits / (2 * G)) >= 512 && 2 * G * ((per_range + 1023) / 1024) <= 8) G *= 2;
+  // (no more ranges a workgroup where the rows are short: a list holds its columns' 64 largest, so with four ranges to a list [128, 32000]
+  // takes 24 us in place of 28 at top-k 50, but rows that keep some hundred columns no longer fit: top-k 400 170 us in place of 78)
+  const int G = (num_splits >= kFastRangesMax && num_splits % kFastRangesMax == 0) ? num_splits / kFastRangesMax : 1;
   const int R = num_splits / G;
   SGL_CHECK_ARG(R <= kFastRangesMax, "sample_from_logits: num_splits must be <= 16 or a multiple of 16");
   const int J = static_cast<int>((per_range + 1023) / 1024);

@@ -49,3 +49,15 @@ def test_one_call_equals_softmax_then_sample(device, B, V, fp32):
         assert not bad, [(r, int(got[r]), int(want[r]), int(got_n[r]), int(want_n[r]), int(redone[r])) for r in bad]
         usual = [r for r in range(13, B) if int(top_k[r]) <= 64]
         assert not any(redone.tolist()[r] for r in usual)          # gaussian rows are decided by their candidates
+
+
+def test_rows_that_keep_some_hundred_columns_are_decided_from_the_lists(device):
+    """32000 columns in 16 lists of their ranges' 64 largest: rows that keep 400 columns need no second look at the probabilities."""
+    from sglang_amd import kernels as K
+
+    B, V = 128, 32000
+    g = torch.Generator(device=device).manual_seed(5)
+    lg = (torch.randn((B, V), generator=g, device=device) * 2.5).to(torch.bfloat16)
+    top_k, seeds, pos = torch.full((B,), 400, dtype=torch.int32, device=device), torch.arange(B, device=device), torch.arange(B, device=device)
+    out = K.sample_from_logits(lg, torch.ones((B, 1), device=device), top_k, None, None, seeds, pos, return_n_keep=True, return_fallback=True)
+    assert bool((out[1] == 400).all()) and not bool(out[2].any())
