@@ -1220,11 +1220,15 @@ __global__ __launch_bounds__(kSplitThreads) void sample_logit_candidates_kernel(
       }
     }
   }
-  // (the <= 3 columns behind the last multiple of four: in the row's last range only, which is this workgroup's last if any)
+  // (the <= 3 columns behind the last multiple of four: in the row's last range that holds any, which need not be this workgroup's last:
+  // ranges are rounded up to four columns, and short rows leave the ones at the end empty)
+  int tail_g = 0;                                    // (uniform)
+#pragma unroll
+  for (int g = 1; g < 4; ++g) tail_g += g < G && per * (c * G + g) < V ? 1 : 0;
   int tail_i = -1;
   float tail_v = 0.f;
   {
-    const int b = range_begin(G - 1), e = range_begin(G), e4 = b + ((e - b) & ~3);
+    const int b = range_begin(tail_g), e = range_begin(tail_g + 1), e4 = b + ((e - b) & ~3);
     if (e4 + tid < e) { tail_i = e4 + tid; tail_v = ld1(x + tail_i); }
   }
   auto is_on = [&](int s) { return (on_mask >> s) & 1u; };
@@ -1253,11 +1257,15 @@ __global__ __launch_bounds__(kSplitThreads) void sample_logit_candidates_kernel(
       run = is_on(s) ? m : run;
     }
   }
-  if (tail_i >= 0) run = fmaxf(run, t_pos ? tail_v : tail_v / t);
   if (G == 1) mxg[0] = run;
   else if (G == 2) mxg[1] = run;
   else if (G == 3) mxg[2] = run;
   else mxg[3] = run;
+  if (tail_i >= 0) {
+    const float m = t_pos ? tail_v : tail_v / t;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) mxg[g] = g == tail_g ? fmaxf(mxg[g], m) : mxg[g];
+  }
   const float my_top = fmaxf(fmaxf(mxg[0], mxg[1]), fmaxf(mxg[2], mxg[3]));    // the thread's largest logit (t_pos)
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
@@ -1306,11 +1314,16 @@ __global__ __launch_bounds__(kSplitThreads) void sample_logit_candidates_kernel(
       if (is_on(s)) run += add;
     }
   }
-  if (tail_i >= 0 && mx > -INFINITY) run += expf(tail_v / t - mx);
   if (G == 1) smg[0] = run;
   else if (G == 2) smg[1] = run;
   else if (G == 3) smg[2] = run;
   else smg[3] = run;
+  mx = tail_g == 0 ? mxg[0] : tail_g == 1 ? mxg[1] : tail_g == 2 ? mxg[2] : mxg[3];
+  if (tail_i >= 0 && mx > -INFINITY) {
+    const float add = expf(tail_v / t - mx);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) smg[g] = g == tail_g ? smg[g] + add : smg[g];
+  }
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
     if (g < G) {

@@ -51,6 +51,37 @@ def test_one_call_equals_softmax_then_sample(device, B, V, fp32):
         assert not any(redone.tolist()[r] for r in usual)          # gaussian rows are decided by their candidates
 
 
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("V", [101, 41, 130, 203, 515, 959])
+@pytest.mark.parametrize("B,splits", [(64, 16), (128, 16), (40, 32), (8, 48), (3, 64)])
+def test_short_rows_whose_last_ranges_are_empty(device, B, splits, V, fp32):
+    """Ranges are rounded up to four columns, so a short row's last columns may lie in any range of a workgroup.  (The Python entry leaves rows
+    below 512 columns a range to the two calls; the native one takes them.)  The largest logit sits in the last column of every second row."""
+    from sglang_amd import kernels as K, native
+
+    g = torch.Generator(device=device).manual_seed(V + B)
+    Vp = V + (-V) % 4
+    padded = torch.randn((B, Vp), generator=g, device=device) * 2.5
+    padded[::2, V - 1] = 30.0
+    padded = padded if fp32 else padded.to(torch.bfloat16)
+    lg = padded[:, :V]
+    temps = torch.rand((B, 1), generator=g, device=device) + 0.4
+    top_k, top_p = torch.full((B,), 20, dtype=torch.int32, device=device), torch.full((B,), 0.95, device=device)
+    seeds, pos = torch.arange(B, device=device) * 977 + 5, torch.arange(B, device=device)
+    probs = torch.empty((B, Vp), device=device)
+    probs[:, :V] = torch.softmax(lg.float() / temps, dim=-1)
+    want, want_n = K.top_k_top_p_min_p_sample(probs[:, :V], top_k, top_p, None, seeds, pos, return_n_keep=True)
+    got, got_n = torch.full((B,), -1, dtype=torch.int32, device=device), torch.full((B,), -1, dtype=torch.int32, device=device)
+    ws = torch.zeros(native.lib().sgl_amd_sample_from_logits_workspace_bytes(B, splits) // 8 + 2, dtype=torch.int64, device=device)
+    scratch = torch.empty((B, Vp), device=device)
+    native.call("sgl_amd_top_k_top_p_min_p_sample_from_logits", lg.data_ptr(), int(not fp32), lg.stride(0), temps.data_ptr(), scratch.data_ptr(),
+                scratch.stride(0), B, V, top_k.data_ptr(), top_p.data_ptr(), None, seeds.data_ptr(), pos.data_ptr(), got.data_ptr(), None, None,
+                got_n.data_ptr(), splits, ws.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert (got[::2] == V - 1).all() and (got_n[::2] == 1).all()
+    # (the softmax sums differ in the last bits: a row's cut may fall one column further at most, the rest is equal)
+    assert ((got_n - want_n).abs() <= 1).all() and (got == want)[got_n == want_n].all()
+
+
 def test_rows_that_keep_some_hundred_columns_are_decided_from_the_lists(device):
     """32000 columns in 16 lists of their ranges' 64 largest: rows that keep 400 columns need no second look at the probabilities."""
     from sglang_amd import kernels as K
