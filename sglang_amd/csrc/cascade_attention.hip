@@ -47,7 +47,7 @@ constexpr int64_t kSingleShotUnits = 10240;
 constexpr int64_t kSpanSingleShotUnits = 2048;
 constexpr int kSpanChunks = 64;
 inline int64_t single_shot_most(int chunks, int group) { return group <= 8 && chunks >= kSpanChunks ? kSpanSingleShotUnits : kSingleShotUnits; }
-int64_t g_cascade_single_shot_units = kSingleShotUnits;   // worst-case workgroups up to which the one-workgroup-per-unit form is launched
+int64_t g_cascade_single_shot_units = 0;       // worst-case workgroups up to which the one-workgroup-per-unit form is launched (0: the rule above)
 int64_t g_cascade_loop_grid = 256 * 5;         // grid of the looping form: 1280 beat 1024 (= what is resident at four per CU) and equalled 2048
 
 __device__ __forceinline__ bf16x8_t as_frag(const U4& v) { return __builtin_bit_cast(bf16x8_t, v); }
@@ -305,9 +305,11 @@ __global__ __launch_bounds__(kThreads, 4) void cascade_chunk_loop_kernel(ChunkPa
   __shared__ U4 side_s[D > 64 ? 4 * 8 * (D - 64) / 4 : 1];
   // the line of the workgroup's first item record travels with the header (a grid never reaches beyond max_items x kv heads)
   const int first_rec = cascade_plan_view(p.plan, p.batch, p.max_items).items[8 * (blockIdx.x / static_cast<unsigned>(p.num_kv_heads))];
-  // one hop for all of the header that the loop needs: the list's length (shared items, then private items or spans) and what the tail is
-  const int n_items = __builtin_amdgcn_readfirstlane(p.plan[5]), n_shared = __builtin_amdgcn_readfirstlane(p.plan[3]);
-  const bool spans = __builtin_amdgcn_readfirstlane(p.plan[4]) > 0;
+  // one hop for all of the header that the loop needs: the list's length (shared items, then private items or spans) and what the tail is.
+  // (Spans are walked where a kv head has at most 8 query rows, as in the merge; the items stand beside them.)
+  const bool few = p.group <= 8;
+  const int n_items = __builtin_amdgcn_readfirstlane(p.plan[few ? 5 : 0]), n_shared = __builtin_amdgcn_readfirstlane(p.plan[3]);
+  const bool spans = few && __builtin_amdgcn_readfirstlane(p.plan[4]) > 0;
   asm volatile("" ::"v"(first_rec));
   const int n_units = n_items * p.num_kv_heads;
   const int G = static_cast<int>(gridDim.x), w0 = static_cast<int>(blockIdx.x);
@@ -655,12 +657,12 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
 }
 
 // ---- merge: slots [0, n_slots(b)) of every (request, head), in slot order ----------------------
-// n_slots = shared chunks + private chunks of the request; every one of them was written this step.
+// n_slots = shared chunks + private chunks (pieces, where the launch before walked spans) of the request; every one was written this step.
 // Block = 256 / (D/4) heads x (D/4) lanes; a thread owns 4 consecutive output elements of one head.
 constexpr int kMergeBlock = 16;  // slots loaded per round (all loads of a round are in flight together)
 
 __global__ __launch_bounds__(256) void cascade_merge2_kernel(const float* __restrict__ ws_acc, const float* __restrict__ ws_ml,
-                                                             const int32_t* __restrict__ plan,
+                                                             const int32_t* __restrict__ plan, const int32_t* __restrict__ seq_lens, int walks_spans,
                                                              uint16_t* __restrict__ out, int64_t out_stride, int batch,
                                                              int max_items, int num_q_heads, int head_dim, int slots_total,
                                                              float out_scale) {
@@ -670,7 +672,13 @@ __global__ __launch_bounds__(256) void cascade_merge2_kernel(const float* __rest
   const int d = (threadIdx.x % tpd) * 4;
   if (hq >= num_q_heads) return;
   const CascadePlanView pv = cascade_plan_view(plan, batch, max_items);
-  int n = pv.req_slots[b];
+  int n;
+  if (walks_spans) {
+    n = pv.req_slots[b];
+  } else {
+    const int sh = pv.req_shared[b], len = seq_lens[b];
+    n = (sh + kChunk - 1) / kChunk + (len > sh ? (len - sh + kChunk - 1) / kChunk : 0);
+  }
   if (n > slots_total) n = slots_total;
   const int64_t base = (static_cast<int64_t>(b) * num_q_heads + hq) * slots_total;
   const float2* ml = reinterpret_cast<const float2*>(ws_ml) + base;
@@ -817,9 +825,8 @@ int sgl_amd_cascade_decode_attention_ex(const void* q, const void* k_cache, cons
   int64_t units = batch * (chunks + 1);
   if (units > max_items) units = max_items;
   const int64_t worst = units * num_kv_heads;
-  // (a plan of spans is only made where this is true at the switch's default: the switch can lower the line, not raise it)
-  const int64_t most = single_shot_most(chunks, p.group);
-  const bool loop = worst > (g_cascade_single_shot_units < most ? g_cascade_single_shot_units : most);
+  // (the plan may hold spans: the single-shot form works on its items all the same, and the merge goes by the form launched here)
+  const bool loop = worst > (g_cascade_single_shot_units > 0 ? g_cascade_single_shot_units : single_shot_most(chunks, p.group));
   dim3 grid(static_cast<unsigned>(loop ? (worst < g_cascade_loop_grid ? worst : g_cascade_loop_grid) : worst));
 #define SGL_LAUNCH_CASC2(D_, KERNEL_)                                                                                 \
   do {                                                                                                       \
@@ -839,7 +846,7 @@ int sgl_amd_cascade_decode_attention_ex(const void* q, const void* k_cache, cons
 #undef SGL_LAUNCH_CASC
   const int hpb = 256 / (head_dim / 4);
   hipLaunchKernelGGL(cascade_merge2_kernel, dim3(static_cast<unsigned>(batch), (num_q_heads + hpb - 1) / hpb), dim3(256), 0, st,
-                     p.ws_acc, p.ws_ml, plan, static_cast<uint16_t*>(out), out_token_stride, p.batch, p.max_items,
+                     p.ws_acc, p.ws_ml, plan, seq_lens, loop && p.group <= 8 ? 1 : 0, static_cast<uint16_t*>(out), out_token_stride, p.batch, p.max_items,
                      num_q_heads, head_dim, slots_total, kv_fp8 ? v_scale : 1.0f);
   SGL_CHECK_LAUNCH("cascade_decode_attention");
   return 0;
@@ -849,7 +856,7 @@ int sgl_amd_debug_cascade_launch_form(int64_t single_shot_units, int64_t loop_gr
   SGL_CLEAR_STALE_ERROR();
   SGL_CHECK_ARG(single_shot_units >= 0 && single_shot_units <= kSingleShotHardCap && loop_grid >= 0 && loop_grid <= (1 << 20),
                 "debug_cascade_launch_form: single_shot_units must be 0..%lld, loop_grid 0..2^20", (long long)kSingleShotHardCap);
-  g_cascade_single_shot_units = single_shot_units > 0 ? single_shot_units : kSingleShotUnits;
+  g_cascade_single_shot_units = single_shot_units;
   g_cascade_loop_grid = loop_grid > 0 ? loop_grid : 256 * 5;
   return 0;
 }

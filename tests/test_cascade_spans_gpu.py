@@ -104,3 +104,52 @@ def test_spans_match_oracle(device, Hq, Hkv, D, fp8, page, hnd, lens, shared):
     K.cascade_plan(ws, r2t_d, pool_d, seq_d, Hq, Hkv)
     K.cascade_decode_attention(ws, q.to(device), kd, vd, out2, r2t_d, pool_d, seq_d, D ** -0.5, bool(fp8), ks, vs, page, bool(hnd))
     assert torch.equal(out, out2)
+
+
+@pytest.mark.parametrize("fp8", [0, 1])
+@pytest.mark.parametrize("lens,plan_heads,Hq,Hkv", [([5000 + 37 * i for i in range(8)], (16, 4), 16, 4),      # spans; one workgroup a unit when asked for
+                                                   ([5000 + 37 * i for i in range(8)], (16, 4), 8, 2),       # ... and by itself, for fewer heads than the plan's
+                                                   ([130, 700, 64, 1, 1000, 333, 512, 95], (32, 8), 32, 8)])  # too few tokens for spans
+def test_every_launch_form_reads_the_plan_it_gets(device, lens, plan_heads, Hq, Hkv, fp8):
+    """Both launch forms over one plan, whether or not it holds spans, at every line of the switch: the oracle's bar each, and without
+    spans the same bits from bf16 rows (e4m3 items of few rows are cut into other tiles)."""
+    from sglang_amd import kernels as K, native
+
+    D, B, width = 128, len(lens), 8192
+    g = torch.Generator().manual_seed(Hq + B)
+    r2t = torch.zeros((B + 1, width), dtype=torch.int32)
+    perm, at = (torch.randperm(sum(lens), generator=g) + 1).int(), 0
+    for b, n in enumerate(lens):
+        r2t[b + 1, :n], at = perm[at:at + n], at + n
+    r2t[2, :min(384, lens[1] - 1)] = r2t[5, :min(384, lens[1] - 1)]                 # a shared prefix too
+    kc, vc = (torch.randn((sum(lens) + 1, Hkv, D), generator=g) * 0.5 for _ in range(2))
+    q = (torch.randn((B, Hq, D), generator=g) * 0.5).to(BF)
+    if fp8:
+        kd, vd = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+        kc, vc, kd, vd = kd.float(), vd.float(), kd.view(torch.uint8), vd.view(torch.uint8)
+    else:
+        kd, vd = kc.to(BF), vc.to(BF)
+        kc, vc = kd.float(), vd.float()
+    pool, seq = torch.arange(1, B + 1), torch.tensor(lens, dtype=torch.int32)
+    ref = oo.decode_attention(q, kc, vc, r2t, pool, seq.long(), D ** -0.5, compute_dtype=torch.float32).float()
+    bar = 2.0 ** -8 * float(vc.abs().max())                                         # as above
+    ws = K.CascadeWorkspace(B, plan_heads[0], D, width, device)
+    r2t_d, pool_d, seq_d, q_d, kd, vd = (x.to(device) for x in (r2t, pool, seq, q, kd, vd))
+    K.cascade_plan(ws, r2t_d, pool_d, seq_d, *plan_heads)
+    spans = int(ws.plan[4]) > 0
+    assert spans == (lens[0] == 5000) and K.cascade_plan_summary(ws, B)["n_shared_items"] > 0
+    outs = []
+    try:
+        for line in (0, 1, 16384):
+            native.call("sgl_amd_debug_cascade_launch_form", line, 0)
+            out = torch.empty((B, Hq, D), dtype=BF, device=device)
+            ws.ws_acc.fill_(float("nan"))
+            ws.ws_ml.fill_(float("nan"))
+            K.cascade_decode_attention(ws, q_d, kd, vd, out, r2t_d, pool_d, seq_d, D ** -0.5, bool(fp8))
+            outs.append(out)
+            err = float((out.cpu().float() - ref).abs().max())
+            assert err <= bar, (line, err, bar)
+    finally:
+        native.call("sgl_amd_debug_cascade_launch_form", 0, 0)
+    if not spans and not fp8:
+        assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
