@@ -1399,7 +1399,7 @@ __global__ __launch_bounds__(64 * kPartWaves, 2) void extend_attention_parts_ker
 }
 
 // out = sum_i e^{m_i - m} acc_i / sum_i e^{m_i - m} l_i: a (token, head) row is D / 8 lanes, 8 dims each.  Rows outside the requests'
-// tokens stay untouched; a part without keys for the row (sum 0) is not read.
+// tokens stay untouched; a part without keys for the row (sum 0) is not read, one whose sum is NaN makes the row NaN as in one part.
 template <int D>
 __global__ __launch_bounds__(256) void extend_merge_kernel(ExtendParams p) {
   constexpr int LPR = D / 8;
@@ -1413,7 +1413,7 @@ __global__ __launch_bounds__(256) void extend_merge_kernel(ExtendParams p) {
   float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, l = 0.f;
   for (int i = 0; i < p.parts; ++i) {
     const float* ml = p.part_ml + 2 * (i * p.part_rows + row);
-    if (!(ml[1] > 0.f)) continue;
+    if (ml[1] == 0.f) continue;
     const float w = fast_exp2(ml[0] - m);
     const f32x4_t* a = reinterpret_cast<const f32x4_t*>(p.part_acc + (i * p.part_rows + row) * D + c * 8);
     const f32x4_t a0 = a[0], a1 = a[1];

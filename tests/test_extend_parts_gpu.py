@@ -81,3 +81,31 @@ def test_request_without_keys_gives_zero_rows(device, Hq, Hkv, D, fp8, shape):
                 assert torch.equal(got, ref), (parts, empty)
     finally:
         native.call("sgl_amd_debug_extend_attention_shape", 0, 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_a_key_that_is_no_number_makes_its_rows_nan_in_any_number_of_parts(device, bad):
+    """Softmax over a NaN or infinite score is NaN: rows that see the key are NaN however the keys are dealt, the rest are what they are
+    without it."""
+    Hq, Hkv, D, prefix, extend = 8, 2, 128, [700, 300], [40, 30]
+    c = _random_case(2, Hq, Hkv, D, prefix, extend, seed=11)
+    qo = torch.tensor([0, 40, 70], dtype=torch.int32, device=device)
+    q, r2t, pool, seq, pre = (c["q"].to(device), c["req_to_token"].to(device), c["req_pool_indices"].to(device), c["seq_lens"].to(torch.int32).to(device),
+                              torch.tensor(prefix, dtype=torch.int32, device=device))
+    spoilt = c["k_cache"].clone()
+    spoilt[c["req_to_token"][c["req_pool_indices"][0], 710].long(), 1] = bad             # seen by tokens 10 and on of request 0, by kv head 1's rows
+    vc = c["v_cache"].to(device)
+    for parts in (1, 2, 5, 16):
+        outs = []
+        for kc in (c["k_cache"].to(device), spoilt.to(device)):
+            out, n = torch.empty_like(q), q.shape[0] * Hq
+            acc, ml = torch.empty((parts, n, D), device=device), torch.empty((parts, n, 2), device=device)
+            native.call("sgl_amd_extend_attention_kv", q.data_ptr(), out.data_ptr(), kc.data_ptr(), vc.data_ptr(), r2t.data_ptr(), r2t.stride(0), pool.data_ptr(),
+                        seq.data_ptr(), pre.data_ptr(), qo.data_ptr(), 2, 70, 40, 740, Hq, Hkv, D, q.stride(0), out.stride(0), Hkv * D, D ** -0.5, 1, 0, 1.0, 1.0,
+                        parts, acc.data_ptr(), ml.data_ptr(), torch.cuda.current_stream().cuda_stream)
+            outs.append(out)
+        nan = torch.zeros(70, Hq, dtype=torch.bool, device=device)
+        nan[10:40, 4:] = True
+        assert bool(outs[1][nan].isnan().all()), parts
+        assert torch.equal(outs[1][~nan], outs[0][~nan]), parts
