@@ -141,6 +141,12 @@ __device__ __forceinline__ double lane_f64(double v, int lane) {
                                           static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(w.y), lane))});
 }
 
+// e^v of a v that a float does not hold (rounded to one, an exponent of 50 is off by 3e-6 of the result): the rest as a first-order factor
+__device__ __forceinline__ float exp_f64(double v) {
+  const float f = static_cast<float>(v), e = expf(f);
+  return e > 0.f ? fmaf(e, static_cast<float>(v - static_cast<double>(f)), e) : e;       // (v may lie beyond the floats: 0)
+}
+
 // sum over N neighbouring lanes (4, 8 or 16; quad_perm xor 1, xor 2, then mirrors of half rows and rows), left in all of them
 template <int N>
 __device__ __forceinline__ float sum_lanes(float v) {
@@ -231,14 +237,15 @@ __device__ __forceinline__ void mamba2_split_body(const Params& p, Mamba2Split<N
       sm.cum[at][lane] = c;
       sm.dts[at][lane] = dt;
       sm.colf[at][0][lane] = lane < 48 ? expf(static_cast<float>(cm - c)) * dt : 0.f;
-      sm.colf[at][1][lane] = expf(static_cast<float>(cf - c)) * dt;          // (read only where it cannot overflow)
+      sm.colf[at][1][lane] = exp_f64(cf - c) * dt;                           // (read only where it cannot overflow)
       sm.ec[to][lane] = expf(static_cast<float>(c));
       sm.wj[to][lane] = expf(static_cast<float>(cn - c)) * dt;
       if (lane == 0) sm.fix[to][0] = expf(static_cast<float>(cn));
     };
     // Tiles on and below the diagonal of (C B^T)_ij e^{c_i - c_j} dt_j, formed transposed: a lane then holds four j of one i.  The
     // decay is e^{c_i - c_m} e^{c_m - c_j}, one exponential a lane: m is the first token behind j's tile, or the tile's own first on the
-    // diagonal, where the second factor exceeds 1 and a tile that decays by e^60 or more takes its exponentials one by one.
+    // diagonal, where the second factor exceeds 1 and a tile that decays by e^60 or more takes its exponentials one by one.  There both
+    // exponents may be many times the one of their product: they keep what a float drops (exp_f64).
     auto product = [&](int k, int ti, int tj) __attribute__((always_inline)) {
       const uint16_t* B = sm.b[k & 1] + (16 * tj + i16) * L::kLs + 8 * g;
       const uint16_t* C = sm.c[k & 1] + (16 * ti + i16) * L::kLs + 8 * g;
@@ -253,7 +260,7 @@ __device__ __forceinline__ void mamba2_split_body(const Params& p, Mamba2Split<N
       const double ci = sm.cum[at][i];
       float v[4];
       if (!diag || sm.cum[at][16 * ti] - sm.cum[at][16 * ti + 15] < 60.0) {
-        const float w = expf(static_cast<float>(ci - sm.cum[at][diag ? 16 * ti : 16 * tj + 16]));
+        const float w = exp_f64(ci - sm.cum[at][diag ? 16 * ti : 16 * tj + 16]);
         const f32x4_t e = *reinterpret_cast<const f32x4_t*>(&sm.colf[at][diag][j0]);
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = acc[r] * (w * e[r]);
@@ -521,8 +528,8 @@ __device__ __forceinline__ void delta_split_body(const Params& p, DeltaSplit<NU>
       sm.ec[at][i] = expf(static_cast<float>(c));
       sm.wj[at][i] = expf(static_cast<float>(cn - c));
       sm.colf[at][0][i] = i < 16 ? expf(static_cast<float>(cm - c)) : 0.f;
-      sm.colf[at][1][i] = expf(static_cast<float>(cf - c));                // (read only where it cannot overflow)
-      sm.rowf[at][i] = expf(static_cast<float>(c - cf));
+      sm.colf[at][1][i] = exp_f64(cf - c);                                 // (read only where it cannot overflow)
+      sm.rowf[at][i] = exp_f64(c - cf);
       if (i == 0) sm.fix[at][0] = expf(static_cast<float>(cn));
     };
     // X_i . K_j over the head dim of tile (ti, tj); `turned`: a lane holds four j of one i, else four i of one j

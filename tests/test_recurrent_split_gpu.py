@@ -72,3 +72,75 @@ def test_split_recurrence(device, rule, heads, groups, K, V, decay):
         scale = want.abs().max()
         off = (state[slots[i]].double().cpu() - want).abs().max() / scale
         assert off < 4e-6, (i, float(off), float((general[slots[i]].double().cpu() - want).abs().max() / scale))
+
+
+def _one_term(device, n, fall, seed):
+    """(split kernel's, general kernel's) relative errors of products (inverse) x (right-hand side) alone.  Only token n - 2 has a value, so U of
+    token n - 1 is one such product; its key reaches into the upper half of the head dim, where no other token's does, and the state there
+    holds that product times the (exact) key.  The keys' lengths are powers of two: what is left is the gates' and the product's."""
+    g = torch.Generator().manual_seed(seed)
+    B, heads, groups, K, V = 64, 8, 8, 64, 64
+    act = torch.randn(B, n, 2 * groups * K + heads * V, generator=g)
+    k = act[:, :, groups * K:2 * groups * K].view(B, n, groups, K)
+    k.zero_()
+    k[:, :n - 1, :, :16] = 256.0
+    k[:, n - 1, :, 8:16] = 256.0
+    k[:, n - 1, :, 32:40] = torch.randint(0, 2, (B, groups, 8), generator=g) * 512.0 - 256.0
+    act[:, torch.arange(n) != n - 2, 2 * groups * K:] = 0.0
+    gates = torch.randn(B, n, 2 * heads, generator=g)
+    gates[:, :, heads:] = fall
+    gates[:, n - 2:, heads:] = torch.randn(B, min(n, 2), heads, generator=g) - 6.0   # the last two tokens fall by little
+    act, gates = act.to(BF), gates.to(BF)
+    A_log, bias = torch.zeros(heads), torch.zeros(heads)
+    want = torch.stack([_state_want("delta", torch.zeros(heads, K, V), (act[b], gates[b]), A_log, bias, heads, groups, K, V) for b in range(B)])[:, :, 32:40]
+    pos, rows = torch.arange(n).repeat(B).to(device), torch.zeros(B * n, act.shape[-1] + 9, dtype=BF, device=device)
+    out = []
+    for odd in (0, 1):                                                               # (rows at odd addresses: the general kernel)
+        x = rows[:, odd:odd + act.shape[-1]]
+        x.copy_(act.flatten(0, 1))
+        x = x if odd else x.contiguous()
+        state, gt = torch.zeros(B, heads, K, V, device=device), gates.flatten(0, 1).to(device)
+        kernels.gated_delta_scan(x, gt[:, :heads], gt[:, heads:], A_log.to(device), bias.to(device), state, torch.arange(B, device=device), pos,
+                                 _segments([n] * B, device), groups, K ** -0.5, form="chunk")
+        err = (state[:, :, 32:40].cpu().double() - want) / want
+        out.append((float(err.mean()) * 2.0 ** 24, float(err.abs().max()) * 2.0 ** 24))
+    return out
+
+
+@pytest.mark.parametrize("n,fall", [(16, 3.9), (16, 2.0), (16, 0.5), (32, 3.9)])
+def test_decays_between_neighbours_behind_a_steep_fall(device, n, fall):
+    """The decay between the last two tokens, e^-0.003, is a product of two exponentials whose exponents are the whole tile's fall (up to e^56).
+    Largest relative error in units of 2^-24: that of the general kernel, which takes one exponential, and two for the other factor and the
+    product's rounding, plus what products of pieces leave out (7)."""
+    (_, big), (_, big0) = _one_term(device, n, fall, 1)
+    assert big < big0 + 9.0, (big, big0)
+
+
+@pytest.mark.parametrize("rule", ["mamba2", "delta"])
+def test_gates_whose_falls_leave_the_floats(device, rule):
+    """A fall of 3e38 a token: everything in front is forgotten, the sums of the falls lie beyond the largest float, nothing becomes NaN."""
+    g = torch.Generator().manual_seed(3)
+    heads, groups, K, V, T = 2, 1, 64, 64, 150
+    act, gates = torch.randn(T, heads * V + 2 * groups * K, generator=g).to(BF), torch.randn(T, 2 * heads, generator=g).to(BF)
+    gates[20:T:7] = 3.0e38
+    A_log, bias, D = torch.zeros(heads), torch.zeros(heads), torch.zeros(heads)
+    if rule == "mamba2":                                        # (its values are scaled by the same gates)
+        act[:, :heads * V] *= 1e-20
+        act[:, heads * V:] *= 1e-15
+    ref = None
+    for odd in (1, 0):
+        rows = torch.zeros(T, act.shape[1] + 9, dtype=BF, device=device)[:, odd:odd + act.shape[1]]
+        rows.copy_(act)
+        rows = rows if odd else rows.contiguous()
+        state, gt, seg, pos = torch.zeros(1, heads, K, V, device=device), gates.to(device), _segments([T], device), torch.arange(T, device=device)
+        par = [t.to(device) for t in (A_log, bias, D)]
+        if rule == "mamba2":
+            y = kernels.mamba2_scan(rows, gt[:, :heads], *par, state, torch.zeros(1, dtype=torch.int64, device=device), pos, seg, groups, form="chunk")
+        else:
+            y = kernels.gated_delta_scan(rows, gt[:, :heads], gt[:, heads:], *par[:2], state, torch.zeros(1, dtype=torch.int64, device=device), pos, seg, groups,
+                                         K ** -0.5, form="chunk")
+        assert bool(y.isfinite().all()) and bool(state.isfinite().all()), odd
+        if odd:
+            ref = y.cpu()
+    if rule == "delta":                                         # (Mamba-2: chunks of 64 here and 32 there, and small falls behind 1e38 are lost in a chunk's sum)
+        assert _err(y, ref) < 1.2e-2                            # one 16-bit rounding, as the other outputs here
