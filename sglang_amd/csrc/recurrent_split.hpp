@@ -30,8 +30,10 @@ __device__ __forceinline__ f32x4_t mfma_bf(const U4& a, const U4& b, f32x4_t c) 
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
 
-// v = h + m + l exactly (above the denormals): the leading 8 significant bits, the next 8 and the rest
+// v = h + m + l exactly (above the denormals): the leading 8 significant bits, the next 8 and the rest.  (Not contracted: of a v that is a
+// product, fma(a, b, -h) would leave more than 8 bits to l, whose end is cut off.)
 __device__ __forceinline__ void split3(float v, uint32_t& h, uint32_t& m, uint32_t& l) {
+#pragma clang fp contract(off)
   h = __float_as_uint(v) & 0xffff0000u;
   const float r = v - __uint_as_float(h);
   m = __float_as_uint(r) & 0xffff0000u;

@@ -144,3 +144,28 @@ def test_gates_whose_falls_leave_the_floats(device, rule):
             ref = y.cpu()
     if rule == "delta":                                         # (Mamba-2: chunks of 64 here and 32 there, and small falls behind 1e38 are lost in a chunk's sum)
         assert _err(y, ref) < 1.2e-2                            # one 16-bit rounding, as the other outputs here
+
+
+def _one_token_states(device, B, x, gate, dim):
+    """Mamba-2 states behind one token each, from the split kernel and from the general one (rows at odd addresses)."""
+    n, heads, V = x.shape
+    act, out = torch.cat([x.flatten(1), B.flatten(1), torch.zeros(n, dim).to(BF)], 1), []
+    zero, pos = torch.zeros(heads, device=device), torch.zeros(n, dtype=torch.int64, device=device)
+    for odd in (0, 1):
+        rows = torch.zeros(n, act.shape[1] + 9, dtype=BF, device=device)[:, odd:odd + act.shape[1]]
+        rows.copy_(act)
+        state = torch.zeros(n, heads, dim, V, device=device)
+        kernels.mamba2_scan(rows if odd else rows.contiguous(), gate.to(device), zero, zero, zero, state, torch.arange(n, device=device), pos,
+                            _segments([1] * n, device), 1, form="chunk")
+        out.append(state.cpu())
+    return out
+
+
+def test_pieces_of_a_product_add_up_to_it(device):
+    """The state behind one token is B (dt x): for B of powers of two the pieces of dt x leave exactly the float that the general kernel has."""
+    g = torch.Generator().manual_seed(2)
+    n, heads, K, V = 40, 4, 64, 64
+    B = torch.exp2(torch.randint(-3, 4, (n, 1, K), generator=g).float()).to(BF)
+    x, gate = torch.randn(n, heads, V, generator=g).to(BF), torch.randn(n, heads, generator=g).to(BF)
+    split, general = _one_token_states(device, B, x, gate, K)
+    assert torch.equal(split, general)
