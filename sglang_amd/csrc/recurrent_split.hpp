@@ -430,8 +430,9 @@ __device__ __forceinline__ void mamba2_split_body(const Params& p, Mamba2Split<N
 }
 
 // ------------------------------------------------------------------------------------------------ gated delta rule, 32 tokens a chunk
-// The products of two fp32 operands (the inverse times the right-hand side, the read-out's matrix times U) are the six products of
-// pieces above 2^-24 of the result.
+// The products of two fp32 operands (the inverse times the right-hand side, the read-out's matrix times U) are the products of their pieces
+// but the smallest, l l, below 2^-30 of the whole: of two more, m l and l m, truncated pieces make up to 7 x 2^-24 of the product, always
+// towards zero.  The matrix cores cut a product's low bits off when they add it to a larger sum, so the large term h h is summed by itself.
 template <int NU>
 struct DeltaSplit {
   static constexpr int kTok = 32, kNp = 32 * NU, kLs = kNp + 8, kVs = 64 + 8, kGs = kTok + 8, kAs = kTok + 4;
@@ -703,14 +704,18 @@ __device__ __forceinline__ void delta_split_body(const Params& p, DeltaSplit<NU>
   __syncthreads();
   __syncthreads();
   __syncthreads();
-  // the six products of two operands in pieces
-  auto mul6 = [](const U4 (&x)[3], const U4 (&y)[3], f32x4_t c) __attribute__((always_inline)) {
-    c = mfma_bf(x[2], y[0], c);
-    c = mfma_bf(x[1], y[1], c);
-    c = mfma_bf(x[0], y[2], c);
-    c = mfma_bf(x[1], y[0], c);
-    c = mfma_bf(x[0], y[1], c);
-    return mfma_bf(x[0], y[0], c);
+  // c plus the product of two operands in pieces
+  auto mul8 = [](const U4 (&x)[3], const U4 (&y)[3], f32x4_t c) __attribute__((always_inline)) {
+    f32x4_t a = {0.f, 0.f, 0.f, 0.f};
+    a = mfma_bf(x[2], y[1], a);
+    a = mfma_bf(x[1], y[2], a);
+    a = mfma_bf(x[2], y[0], a);
+    c = mfma_bf(x[0], y[0], c);
+    a = mfma_bf(x[0], y[2], a);
+    a = mfma_bf(x[1], y[1], a);
+    a = mfma_bf(x[1], y[0], a);
+    a = mfma_bf(x[0], y[1], a);
+    return c + a;
   };
   for (int k = 0; k < chunks; ++k) {
     const int c0 = k * Q, len = total - c0 < Q ? total - c0 : Q, at = k & 7;
@@ -767,7 +772,7 @@ __device__ __forceinline__ void delta_split_body(const Params& p, DeltaSplit<NU>
     split8(rhs, rp);
     f32x4_t u2[2];
 #pragma unroll
-    for (int ti = 0; ti < 2; ++ti) u2[ti] = mul6(tf[ti], rp, f32x4_t{0.f, 0.f, 0.f, 0.f});
+    for (int ti = 0; ti < 2; ++ti) u2[ti] = mul8(tf[ti], rp, f32x4_t{0.f, 0.f, 0.f, 0.f});
     // ---- S = e^{c_n} S + K^T (e^{c_n - c_j} U), O^T = e^{c_i} (Q S)^T + U^T P^T ----
 #pragma unroll
     for (int ti = 0; ti < 2; ++ti)
@@ -810,7 +815,7 @@ __device__ __forceinline__ void delta_split_body(const Params& p, DeltaSplit<NU>
 #pragma unroll
     for (int ti = 0; ti < 2; ++ti) {
       o[ti] *= sm.ec[at][16 * ti + i16] * sm.iq[at][16 * ti + i16];
-      o[ti] = mul6(up, pf[ti], o[ti]);
+      o[ti] = mul8(up, pf[ti], o[ti]);
       if (16 * ti + i16 < len && 4 * g < wide)
         *reinterpret_cast<uint2*>(to + static_cast<int64_t>(16 * ti) * p.o_stride) = uint2{pack_bf2(o[ti][0], o[ti][1]), pack_bf2(o[ti][2], o[ti][3])};
     }
