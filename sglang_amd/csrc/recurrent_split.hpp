@@ -30,6 +30,10 @@ __device__ __forceinline__ f32x4_t mfma_bf(const U4& a, const U4& b, f32x4_t c) 
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
 
+__device__ __forceinline__ f32x4_t fma4(const f32x4_t& a, float b, const f32x4_t& c) {
+  return f32x4_t{fmaf(a[0], b, c[0]), fmaf(a[1], b, c[1]), fmaf(a[2], b, c[2]), fmaf(a[3], b, c[3])};
+}
+
 // v = h + m + l exactly (above the denormals): the leading 8 significant bits, the next 8 and the rest.  (Not contracted: of a v that is a
 // product, fma(a, b, -h) would leave more than 8 bits to l, whose end is cut off.)
 __device__ __forceinline__ void split3(float v, uint32_t& h, uint32_t& m, uint32_t& l) {
@@ -375,7 +379,8 @@ __device__ __forceinline__ void mamba2_split_body(const Params& p, Mamba2Split<N
 #pragma unroll
         for (int ti = 0; ti < 4; ++ti) y[ti] = mfma_bf(sp[u & 1][q], cf[u & 1][ti], y[ti]);
     }
-    // ---- the state: S = e^{c_n} S + B^T x' (it does not wait for y) ----
+    // ---- the state: S = e^{c_n} S + B^T x' (it does not wait for y).  A chunk's addition is summed by itself: six products added to a state that is
+    // hardly forgotten lost 18 x 2^-24 of it in 2048 tokens of one sign, 2 x 2^-24 this way (fp32 products one by one: 11) ----
     U4 xp[2][3];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -386,14 +391,22 @@ __device__ __forceinline__ void mamba2_split_body(const Params& p, Mamba2Split<N
       for (int j = 0; j < 8; ++j) v[j] = ((j & 1) ? bf_hi(w[j >> 1]) : bf_lo(w[j >> 1])) * (j < 4 ? w0[j & 3] : w1[j & 3]);
       split8(v, xp[u]);
     }
-#pragma unroll
-    for (int t = 0; t < 2 * NU; ++t) s[t] *= fix;
     constexpr int W = 2 * NU < 4 ? 2 * NU : 4;                          // tiles at a time: no product waits for the one in front
     constexpr int STEPS = 2 * (2 * NU / W);
     U4 bt[2][W];
+    f32x4_t add[2][W];
     auto tiles = [&](int i) __attribute__((always_inline)) {            // step i: tokens 32 (i & 1) .., tiles W (i / 2) ..
 #pragma unroll
       for (int t = 0; t < W; ++t) bt[i & 1][t] = read_tr8(B, L::kLs, 32 * (i & 1) + 8 * g, 16 * (W * (i / 2) + t), i16);
+    };
+    auto take = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < W; ++t) s[W * j + t] = fma4(s[W * j + t], fix, add[j & 1][t]);
+    };
+    U4 gf[2][6];                                                        // tiles 0 .. 3 of tokens 0 .. 31, tiles 2 and 3 of tokens 32 .. 63
+    auto gram = [&](int q) __attribute__((always_inline)) {
+#pragma unroll
+      for (int f = 0; f < 6; ++f) gf[q & 1][f] = ld16(G + q * (Q * L::kGs) + 16 * (f < 4 ? f : f - 2) * L::kGs + 32 * (f >= 4));
     };
     tiles(0);
 #pragma unroll
@@ -401,18 +414,29 @@ __device__ __forceinline__ void mamba2_split_body(const Params& p, Mamba2Split<N
 #pragma unroll
     for (int i = 0; i < STEPS; ++i) {
       if (i + 1 < STEPS) tiles(i + 1);
+      else gram(2);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int q = 2; q >= 0; --q)
 #pragma unroll
-        for (int t = 0; t < W; ++t) s[W * (i / 2) + t] = mfma_bf(bt[i & 1][t], xp[i & 1][q], s[W * (i / 2) + t]);
+        for (int t = 0; t < W; ++t) {
+          f32x4_t& a = add[(i >> 1) & 1][t];
+          a = mfma_bf(bt[i & 1][t], xp[i & 1][q], (i & 1) == 0 && q == 2 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : a);
+        }
+      if (i >= 2 && (i & 1) == 0) take(i / 2 - 1);                      // (the products in front have landed by now)
     }
-    // ---- y += G x ----
+    // ---- y += G x: a piece's six fragments are read while the piece in front is multiplied ----
 #pragma unroll
-    for (int q = 2; q >= 0; --q)
+    for (int q = 2; q >= 0; --q) {
+      if (q > 0) gram(q - 1);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int ti = 2 * u; ti < 4; ++ti) y[ti] = mfma_bf(xf[u], ld16(G + q * (Q * L::kGs) + 16 * ti * L::kGs + 32 * u), y[ti]);
+      for (int f = 0; f < 6; ++f) {
+        const int ti = f < 4 ? f : f - 2;
+        y[ti] = mfma_bf(xf[f >= 4], gf[q & 1][f], y[ti]);
+      }
+      if (q == 2) take(STEPS / 2 - 1);
+    }
     uint16_t* to = yp + static_cast<int64_t>(c0) * p.y_stride;
 #pragma unroll
     for (int ti = 0; ti < 4; ++ti)
@@ -794,8 +818,6 @@ __device__ __forceinline__ void delta_split_body(const Params& p, DeltaSplit<NU>
       split8(u, up);
     }
     const float fix = sm.fix[at][0];
-#pragma unroll
-    for (int t = 0; t < 2 * NU; ++t) s[t] *= fix;
     constexpr int W = 2 * NU < 4 ? 2 * NU : 4;
     U4 bt[2][W];
     auto tiles = [&](int i) __attribute__((always_inline)) {
@@ -806,10 +828,13 @@ __device__ __forceinline__ void delta_split_body(const Params& p, DeltaSplit<NU>
 #pragma unroll
     for (int i = 0; i < 2 * NU / W; ++i) {
       if (i + 1 < 2 * NU / W) tiles(i + 1);
+      f32x4_t add[W];
 #pragma unroll
       for (int q = 2; q >= 0; --q)
 #pragma unroll
-        for (int t = 0; t < W; ++t) s[W * i + t] = mfma_bf(bt[i & 1][t], wp[q], s[W * i + t]);
+        for (int t = 0; t < W; ++t) add[t] = mfma_bf(bt[i & 1][t], wp[q], q == 2 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : add[t]);
+#pragma unroll
+      for (int t = 0; t < W; ++t) s[W * i + t] = fma4(s[W * i + t], fix, add[t]);
     }
     uint16_t* to = op + static_cast<int64_t>(c0) * p.o_stride;
 #pragma unroll

@@ -177,3 +177,27 @@ def test_pieces_of_a_product_add_up_to_it(device):
     x, gate = torch.randn(n, heads, V, generator=g).to(BF), torch.randn(n, heads, generator=g).to(BF)
     split, general = _one_token_states(device, B, x, gate, K)
     assert torch.equal(split, general)
+
+
+@pytest.mark.parametrize("rule", ["mamba2", "delta"])
+def test_long_memory_of_one_sign(device, rule):
+    """2500 tokens of positive values that are hardly forgotten: what every chunk's addition loses is lost with the state's sign and adds up.
+    The relative error of the state (2-norm) is no larger than the general kernel's, whose sums are fp32 products one after the other."""
+    g = torch.Generator().manual_seed(8)
+    heads, groups, K, V, T = 4, 1, 128, 64, 2500
+    act = (torch.randn(T, heads * V + 2 * groups * K, generator=g).abs() + 0.05).to(BF)
+    gates = torch.randn(T, 2 * heads, generator=g).to(BF)
+    A_log, bias, D = torch.full((heads,), -6.0), torch.full((heads,), -3.0), torch.zeros(heads)
+    want = _state_want(rule, torch.zeros(heads, K, V), (act, gates), A_log, bias, heads, groups, K, V)
+    errs = []
+    for odd in (0, 1):
+        rows = torch.zeros(T, act.shape[1] + 9, dtype=BF, device=device)[:, odd:odd + act.shape[1]]
+        rows.copy_(act)
+        rows, state, gt = rows if odd else rows.contiguous(), torch.zeros(1, heads, K, V, device=device), gates.to(device)
+        slot, pos, seg, par = torch.zeros(1, dtype=torch.int64, device=device), torch.arange(T, device=device), _segments([T], device), [t.to(device) for t in (A_log, bias, D)]
+        if rule == "mamba2":
+            kernels.mamba2_scan(rows, gt[:, :heads], *par, state, slot, pos, seg, groups, form="chunk")
+        else:
+            kernels.gated_delta_scan(rows, gt[:, :heads], gt[:, heads:], *par[:2], state, slot, pos, seg, groups, K ** -0.5, form="chunk")
+        errs.append(float((state[0].cpu().double() - want).norm() / want.norm()))
+    assert errs[0] <= errs[1], errs
