@@ -30,6 +30,11 @@ __device__ __forceinline__ f32x4_t mfma_bf(const U4& a, const U4& b, f32x4_t c) 
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
 
+// the same over 16 rows of the contraction: lane group g holds rows 4 g .. 4 g + 3
+__device__ __forceinline__ f32x4_t mfma_bf16k(const uint2& a, const uint2& b, f32x4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(split_v4s16_t, a), __builtin_bit_cast(split_v4s16_t, b), c, 0, 0, 0);
+}
+
 __device__ __forceinline__ f32x4_t fma4(const f32x4_t& a, float b, const f32x4_t& c) {
   return f32x4_t{fmaf(a[0], b, c[0]), fmaf(a[1], b, c[1]), fmaf(a[2], b, c[2]), fmaf(a[3], b, c[3])};
 }
@@ -75,6 +80,12 @@ __device__ __forceinline__ U4 read_tr8(const uint16_t* img, int stride, int r0, 
   o.x = __builtin_bit_cast(uint2, lo).x; o.y = __builtin_bit_cast(uint2, lo).y;
   o.z = __builtin_bit_cast(uint2, hi).x; o.w = __builtin_bit_cast(uint2, hi).y;
   return o;
+}
+
+// rows r0 .. r0 + 3 (r0 already the lane group's) of the 16 columns from `col` on, transposed
+__device__ __forceinline__ uint2 read_tr4(const uint16_t* img, int stride, int r0, int col, int i16) {
+  typedef __attribute__((address_space(3))) split_v4s16_t* lds_t;
+  return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_t)(img + (r0 + (i16 >> 2)) * stride + col + (i16 & 3) * 4)));
 }
 
 // the A operand in the state's slot order: columns n0 + 4 g .. + 3 and n0 + 16 + 4 g .. + 3 of one row
@@ -297,11 +308,6 @@ __device__ __forceinline__ void mamba2_split_body(const Params& p, Mamba2Split<N
       put(k, e, 0, a1);
       put(k, e, 1, a2);
     };
-    // the two tiles above the diagonal that a k-step of 32 tokens reads are zero throughout
-    for (int i = tid; i < 2 * 3 * 2 * 256; i += 64 * kPrepWaves) {
-      const int piece = i / 512, blk = (i / 256) & 1, e = i & 255;
-      sm.g[piece / 3][piece % 3][(32 * blk + (e >> 4)) * L::kGs + 32 * blk + 16 + (e & 15)] = 0;
-    }
     if (tid == 0) sm.count = 0;
     uint32_t round = 0;
     fetch(0);
@@ -360,6 +366,7 @@ __device__ __forceinline__ void mamba2_split_body(const Params& p, Mamba2Split<N
     // ---- y^T = S^T C^T (a lane holds four columns of one token): the operands of k-step u + 1 are read and split while the products of step u run ----
     f32x4_t y[4];
     U4 cf[2][4], sp[2][3], xf[2];
+    uint2 xh[2];
     auto stage = [&](int u) __attribute__((always_inline)) {
 #pragma unroll
       for (int ti = 0; ti < 4; ++ti) cf[u & 1][ti] = read_pair(C + 16 * ti * L::kLs, 32 * u, g);
@@ -368,7 +375,10 @@ __device__ __forceinline__ void mamba2_split_body(const Params& p, Mamba2Split<N
     };
     stage(0);
 #pragma unroll
-    for (int u = 0; u < 2; ++u) xf[u] = read_tr8(sm.x[at], L::kXs, 32 * u + 8 * g, cw * 16, i16);
+    for (int u = 0; u < 2; ++u) {
+      xf[u] = read_tr8(sm.x[at], L::kXs, 32 * u + 8 * g, cw * 16, i16);
+      xh[u] = read_tr4(sm.x[at], L::kXs, 32 * u + 4 * g, cw * 16, i16);
+    }
 #pragma unroll
     for (int ti = 0; ti < 4; ++ti) y[ti] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -403,10 +413,16 @@ __device__ __forceinline__ void mamba2_split_body(const Params& p, Mamba2Split<N
 #pragma unroll
       for (int t = 0; t < W; ++t) s[W * j + t] = fma4(s[W * j + t], fix, add[j & 1][t]);
     };
-    U4 gf[2][6];                                                        // tiles 0 .. 3 of tokens 0 .. 31, tiles 2 and 3 of tokens 32 .. 63
+    // tiles 1, 2 and 3 of tokens 0 .. 31 and tile 3 of tokens 32 .. 63; tiles 0 and 2 of their own 16 tokens alone: what stands beside a tile above
+    // the diagonal is not multiplied by zero, so that a value that is no number stays where it is
+    U4 gf[2][4];
+    uint2 gh[2][2];
     auto gram = [&](int q) __attribute__((always_inline)) {
+      const uint16_t* at_q = G + q * (Q * L::kGs);
 #pragma unroll
-      for (int f = 0; f < 6; ++f) gf[q & 1][f] = ld16(G + q * (Q * L::kGs) + 16 * (f < 4 ? f : f - 2) * L::kGs + 32 * (f >= 4));
+      for (int f = 0; f < 4; ++f) gf[q & 1][f] = ld16(at_q + 16 * (f < 3 ? f + 1 : 3) * L::kGs + 32 * (f == 3));
+#pragma unroll
+      for (int f = 0; f < 2; ++f) gh[q & 1][f] = *reinterpret_cast<const uint2*>(at_q - 4 * g + 32 * f * L::kGs + 32 * f);
     };
     tiles(0);
 #pragma unroll
@@ -425,18 +441,23 @@ __device__ __forceinline__ void mamba2_split_body(const Params& p, Mamba2Split<N
         }
       if (i >= 2 && (i & 1) == 0) take(i / 2 - 1);                      // (the products in front have landed by now)
     }
-    // ---- y += G x: a piece's six fragments are read while the piece in front is multiplied ----
+    // ---- y += G x: a piece's six fragments are read while the piece in front is multiplied.  (Products over 32 and over 16 rows have sums of
+    // their own: handed from the one to the other without an instruction in between, a sum lost what was in it.) ----
+    f32x4_t y2 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int q = 2; q >= 0; --q) {
       if (q > 0) gram(q - 1);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int f = 0; f < 6; ++f) {
-        const int ti = f < 4 ? f : f - 2;
-        y[ti] = mfma_bf(xf[f >= 4], gf[q & 1][f], y[ti]);
+      for (int f = 0; f < 4; ++f) {
+        const int ti = f < 3 ? f + 1 : 3;
+        y[ti] = mfma_bf(xf[f == 3], gf[q & 1][f], y[ti]);
+        if (f == 0) y[0] = mfma_bf16k(xh[0], gh[q & 1][0], y[0]);
+        if (f == 1) y2 = mfma_bf16k(xh[1], gh[q & 1][1], y2);
       }
       if (q == 2) take(STEPS / 2 - 1);
     }
+    y[2] += y2;
     uint16_t* to = yp + static_cast<int64_t>(c0) * p.y_stride;
 #pragma unroll
     for (int ti = 0; ti < 4; ++ti)
@@ -456,7 +477,7 @@ __device__ __forceinline__ void mamba2_split_body(const Params& p, Mamba2Split<N
 // ------------------------------------------------------------------------------------------------ gated delta rule, 32 tokens a chunk
 // The products of two fp32 operands (the inverse times the right-hand side, the read-out's matrix times U) are the products of their pieces
 // but the smallest, l l, below 2^-30 of the whole: of two more, m l and l m, truncated pieces make up to 7 x 2^-24 of the product, always
-// towards zero.  The matrix cores cut a product's low bits off when they add it to a larger sum, so the large term h h is summed by itself.
+// towards zero.  Rows 0 .. 15 are products over the first 16 tokens alone.  The matrix cores cut a product's low bits off when they add it to a larger sum, so the large term h h is summed by itself.
 template <int NU>
 struct DeltaSplit {
   static constexpr int kTok = 32, kNp = 32 * NU, kLs = kNp + 8, kVs = 64 + 8, kGs = kTok + 8, kAs = kTok + 4;
@@ -661,7 +682,6 @@ __device__ __forceinline__ void delta_split_body(const Params& p, DeltaSplit<NU>
 #pragma unroll
           for (int q = 0; q < 3; ++q) {
             st16(T + q * (Q * L::kGs) + lane * L::kGs + blk * 16 + 8 * c, s3[q]);
-            if (blk == 0) st16(T + q * (Q * L::kGs) + lane * L::kGs + 16 + 8 * c, U4{0u, 0u, 0u, 0u});
           }
         }
       }
@@ -680,7 +700,6 @@ __device__ __forceinline__ void delta_split_body(const Params& p, DeltaSplit<NU>
     };
     // Round k: rows of chunk k + 2 by all, A and the read-out's matrix of it by three waves, one of which scans the gates of chunks
     // k + 3 and k + 4 in odd rounds; the inverse of chunk k + 1 by the last.  The column waves are at chunk k.
-    for (int i = tid; i < 3 * 3 * 256; i += 64 * kPrepWaves) sm.p[i / 768][i / 256 % 3][((i & 255) >> 4) * L::kGs + 16 + (i & 15)] = 0;
     if (tid == 0) sm.count = 0;
     uint32_t round = 0;
     fetch(0);
@@ -728,17 +747,21 @@ __device__ __forceinline__ void delta_split_body(const Params& p, DeltaSplit<NU>
   __syncthreads();
   __syncthreads();
   __syncthreads();
-  // c plus the product of two operands in pieces
-  auto mul8 = [](const U4 (&x)[3], const U4 (&y)[3], f32x4_t c) __attribute__((always_inline)) {
+  // c plus the product of two operands in pieces (the operands' type says over how many tokens)
+  auto part = [](const auto& a, const auto& b, f32x4_t c) __attribute__((always_inline)) {
+    if constexpr (sizeof(a) == sizeof(U4)) return mfma_bf(a, b, c);
+    else return mfma_bf16k(a, b, c);
+  };
+  auto mul8 = [&](const auto& x, const auto& y, f32x4_t c) __attribute__((always_inline)) {
     f32x4_t a = {0.f, 0.f, 0.f, 0.f};
-    a = mfma_bf(x[2], y[1], a);
-    a = mfma_bf(x[1], y[2], a);
-    a = mfma_bf(x[2], y[0], a);
-    c = mfma_bf(x[0], y[0], c);
-    a = mfma_bf(x[0], y[2], a);
-    a = mfma_bf(x[1], y[1], a);
-    a = mfma_bf(x[1], y[0], a);
-    a = mfma_bf(x[0], y[1], a);
+    a = part(x[2], y[1], a);
+    a = part(x[1], y[2], a);
+    a = part(x[2], y[0], a);
+    c = part(x[0], y[0], c);
+    a = part(x[0], y[2], a);
+    a = part(x[1], y[1], a);
+    a = part(x[1], y[0], a);
+    a = part(x[0], y[1], a);
     return c + a;
   };
   for (int k = 0; k < chunks; ++k) {
@@ -774,11 +797,13 @@ __device__ __forceinline__ void delta_split_body(const Params& p, DeltaSplit<NU>
         }
     }
     // ---- U = (I + A)^-1 beta (v - e^{c_i} K S) ----
-    U4 tf[2][3], pf[2][3];
+    U4 tf[3], pf[3];
+    uint2 th[3], ph[3];
 #pragma unroll
-    for (int ti = 0; ti < 2; ++ti)
-#pragma unroll
-      for (int q = 0; q < 3; ++q) tf[ti][q] = read_pair(sm.t[k & 1][q] + (16 * ti + i16) * L::kGs, 0, g);
+    for (int q = 0; q < 3; ++q) {
+      th[q] = *reinterpret_cast<const uint2*>(sm.t[k & 1][q] + i16 * L::kGs + 4 * g);
+      tf[q] = read_pair(sm.t[k & 1][q] + (16 + i16) * L::kGs, 0, g);
+    }
     float rhs[8];
     const uint32_t* vw = reinterpret_cast<const uint32_t*>(&vf);
 #pragma unroll
@@ -795,13 +820,15 @@ __device__ __forceinline__ void delta_split_body(const Params& p, DeltaSplit<NU>
     U4 rp[3];
     split8(rhs, rp);
     f32x4_t u2[2];
-#pragma unroll
-    for (int ti = 0; ti < 2; ++ti) u2[ti] = mul8(tf[ti], rp, f32x4_t{0.f, 0.f, 0.f, 0.f});
+    const uint2 rh[3] = {uint2{rp[0].x, rp[0].y}, uint2{rp[1].x, rp[1].y}, uint2{rp[2].x, rp[2].y}};
+    u2[0] = mul8(th, rh, f32x4_t{0.f, 0.f, 0.f, 0.f});
+    u2[1] = mul8(tf, rp, f32x4_t{0.f, 0.f, 0.f, 0.f});
     // ---- S = e^{c_n} S + K^T (e^{c_n - c_j} U), O^T = e^{c_i} (Q S)^T + U^T P^T ----
 #pragma unroll
-    for (int ti = 0; ti < 2; ++ti)
-#pragma unroll
-      for (int q = 0; q < 3; ++q) pf[ti][q] = read_pair(sm.p[k % 3][q] + (16 * ti + i16) * L::kGs, 0, g);
+    for (int q = 0; q < 3; ++q) {
+      ph[q] = *reinterpret_cast<const uint2*>(sm.p[k % 3][q] + i16 * L::kGs + 4 * g);
+      pf[q] = read_pair(sm.p[k % 3][q] + (16 + i16) * L::kGs, 0, g);
+    }
     U4 up[3], wp[3];
     {
       float u[8], w[8];
@@ -817,6 +844,7 @@ __device__ __forceinline__ void delta_split_body(const Params& p, DeltaSplit<NU>
       split8(w, wp);
       split8(u, up);
     }
+    const uint2 uh[3] = {uint2{up[0].x, up[0].y}, uint2{up[1].x, up[1].y}, uint2{up[2].x, up[2].y}};
     const float fix = sm.fix[at][0];
     constexpr int W = 2 * NU < 4 ? 2 * NU : 4;
     U4 bt[2][W];
@@ -840,7 +868,8 @@ __device__ __forceinline__ void delta_split_body(const Params& p, DeltaSplit<NU>
 #pragma unroll
     for (int ti = 0; ti < 2; ++ti) {
       o[ti] *= sm.ec[at][16 * ti + i16] * sm.iq[at][16 * ti + i16];
-      o[ti] = mul8(up, pf[ti], o[ti]);
+      if (ti == 0) o[0] = mul8(uh, ph, o[0]);
+      else o[1] = mul8(up, pf, o[1]);
       if (16 * ti + i16 < len && 4 * g < wide)
         *reinterpret_cast<uint2*>(to + static_cast<int64_t>(16 * ti) * p.o_stride) = uint2{pack_bf2(o[ti][0], o[ti][1]), pack_bf2(o[ti][2], o[ti][3])};
     }

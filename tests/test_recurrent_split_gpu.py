@@ -201,3 +201,48 @@ def test_long_memory_of_one_sign(device, rule):
             kernels.gated_delta_scan(rows, gt[:, :heads], gt[:, heads:], *par[:2], state, slot, pos, seg, groups, K ** -0.5, form="chunk")
         errs.append(float((state[0].cpu().double() - want).norm() / want.norm()))
     assert errs[0] <= errs[1], errs
+
+
+@pytest.mark.parametrize("rule", ["mamba2", "delta"])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
+def test_values_that_are_no_numbers_reach_no_further(device, rule, bad):
+    """One NaN or infinity in a row of one segment, in any input, at places around the borders of tiles and chunks: the outputs and states that
+    are not finite are the general kernel's (its tile of 16 tokens, what follows, the state), and the rest is what it is without it."""
+    g = torch.Generator().manual_seed(6)
+    heads, groups, K, V, n = 2, 1, 64, 32, 150
+    places = [0, 3, 15, 16, 30, 31, 32, 47, 50, 63, 64, 100, 149]
+    inputs = ["value", "key", "query", "gate"] + ["beta"] * (rule == "delta")
+    T = n * len(places) * len(inputs)
+    act, gates = torch.randn(T, heads * V + 2 * groups * K, generator=g).to(BF), torch.randn(T, 2 * heads, generator=g).to(BF)
+    spoilt, sgates, at = act.clone(), gates.clone(), 0
+    cols = dict(value=5, key=heads * V + 9, query=heads * V + groups * K + 9) if rule == "mamba2" else dict(value=2 * groups * K + 5, key=groups * K + 9, query=9)
+    for what in inputs:
+        for p in places:
+            if what in cols:
+                spoilt[at + p, cols[what]] = bad
+            else:
+                sgates[at + p, heads if (what == "gate") == (rule == "delta") else 0] = bad
+            at += n
+    segs = len(places) * len(inputs)
+    A_log, bias, D = torch.zeros(heads), torch.zeros(heads), torch.ones(heads)
+    slots, pos, seg, par = torch.arange(segs, device=device), torch.arange(n).repeat(segs).to(device), _segments([n] * segs, device), [t.to(device) for t in (A_log, bias, D)]
+
+    def run(a, gt, odd):
+        rows = torch.zeros(T, a.shape[1] + 9, dtype=BF, device=device)[:, odd:odd + a.shape[1]]
+        rows.copy_(a)
+        rows, state, gt = rows if odd else rows.contiguous(), torch.zeros(segs, heads, K, V, device=device), gt.to(device)
+        if rule == "mamba2":
+            y = kernels.mamba2_scan(rows, gt[:, :heads], *par, state, slots, pos, seg, groups, form="chunk")
+        else:
+            y = kernels.gated_delta_scan(rows, gt[:, :heads], gt[:, heads:], *par[:2], state, slots, pos, seg, groups, K ** -0.5, form="chunk")
+        return y.view(segs, n, -1).cpu(), state.cpu()
+
+    (y, state), (y0, state0), (clean, clean_state) = run(spoilt, sgates, 0), run(spoilt, sgates, 1), run(act, gates, 0)
+    for i in range(segs):
+        where = (inputs[i // len(places)], places[i % len(places)])
+        assert torch.equal(y[i].isfinite(), y0[i].isfinite()), where
+        assert torch.equal(state[i].isfinite(), state0[i].isfinite()), where
+        ok, sok = y[i].isfinite(), state[i].isfinite()
+        assert torch.equal(y[i][ok & (torch.arange(n)[:, None] < where[1])], clean[i][ok & (torch.arange(n)[:, None] < where[1])]), where
+        assert _err(y[i][ok], y0[i][ok]) < 1.2e-2 if ok.any() else True, where
+        assert _err(state[i][sok], state0[i][sok]) < 1e-4 if sok.any() else True, where
