@@ -531,7 +531,8 @@ __device__ __forceinline__ void delta_split_body(const Params& p, DeltaSplit<NU>
       kr.fetch(rows + (p.kv_heads + kh) * p.K, len, p.K, tid);
       vr.fetch(rows + 2 * p.kv_heads * p.K + h * p.V + col0, len, cols, tid);
     };
-    // 1 / sqrt(|row|^2 + 1e-6) of the rows in flight (NP / 8 neighbouring lanes hold a row): v_rsq_f32 and a Newton step
+    // 1 / sqrt(|row|^2 + 1e-6) of the rows in flight (NP / 8 neighbouring lanes hold a row): v_rsq_f32 and a Newton step; 0 for a length
+    // beyond the floats, where the step would be inf * 0
     auto lengths = [&](const RowPieces<Q, L::kNp>& r, float* to, float scale) __attribute__((always_inline)) {
 #pragma unroll
       for (int i = 0; i < r.kPieces; ++i) {
@@ -545,7 +546,7 @@ __device__ __forceinline__ void delta_split_body(const Params& p, DeltaSplit<NU>
         }
         const float n = sum_lanes<L::kNp / 8>(ss + st) + 1e-6f;
         const float y = __builtin_amdgcn_rsqf(n), e = fmaf(-n * y, y, 1.0f);
-        if (r.col(i, tid) == 0 && r.row(i, tid) < Q) to[r.row(i, tid)] = scale * fmaf(0.5f * y, e, y);
+        if (r.col(i, tid) == 0 && r.row(i, tid) < Q) to[r.row(i, tid)] = n == INFINITY ? 0.f : scale * fmaf(0.5f * y, e, y);
       }
     };
     auto commit = [&](int k) __attribute__((always_inline)) {

@@ -246,3 +246,22 @@ def test_values_that_are_no_numbers_reach_no_further(device, rule, bad):
         assert torch.equal(y[i][ok & (torch.arange(n)[:, None] < where[1])], clean[i][ok & (torch.arange(n)[:, None] < where[1])]), where
         assert _err(y[i][ok], y0[i][ok]) < 1.2e-2 if ok.any() else True, where
         assert _err(state[i][sok], state0[i][sok]) < 1e-4 if sok.any() else True, where
+
+
+def test_rows_longer_than_the_floats(device):
+    """A key or query of finite elements whose squared length is infinite counts as zero (1 / sqrt(inf)), as in the general kernel."""
+    g = torch.Generator().manual_seed(7)
+    heads, groups, K, V, T = 2, 1, 64, 32, 150
+    act, gates = torch.randn(T, 2 * groups * K + heads * V, generator=g).to(BF), torch.randn(T, 2 * heads, generator=g).to(BF)
+    act[[5, 100], :K] = 3.0e19                                  # queries (not in one chunk with such a key in front: their product is infinite)
+    act[[20, 64, 130], K:2 * K] = -4.0e19                       # keys
+    A_log, bias, out = torch.zeros(heads, device=device), torch.zeros(heads, device=device), []
+    for odd in (0, 1):
+        rows = torch.zeros(T, act.shape[1] + 9, dtype=BF, device=device)[:, odd:odd + act.shape[1]]
+        rows.copy_(act)
+        state, gt = torch.zeros(1, heads, K, V, device=device), gates.to(device)
+        y = kernels.gated_delta_scan(rows if odd else rows.contiguous(), gt[:, :heads], gt[:, heads:], A_log, bias, state, torch.zeros(1, dtype=torch.int64, device=device),
+                                     torch.arange(T, device=device), _segments([T], device), groups, K ** -0.5, form="chunk")
+        assert bool(y.isfinite().all()) and bool(state.isfinite().all()), odd
+        out.append((y.cpu(), state.cpu()))
+    assert _err(out[0][0], out[1][0]) < 1.2e-2 and _err(out[0][1], out[1][1]) < 1e-4
