@@ -39,7 +39,7 @@ __device__ __forceinline__ f32x4_t fma4(const f32x4_t& a, float b, const f32x4_t
   return f32x4_t{fmaf(a[0], b, c[0]), fmaf(a[1], b, c[1]), fmaf(a[2], b, c[2]), fmaf(a[3], b, c[3])};
 }
 
-// v = h + m + l exactly (above the denormals): the leading 8 significant bits, the next 8 and the rest.  (Not contracted: of a v that is a
+// v = h + m + l exactly (above the denormals; an infinity becomes NaN): the leading 8 significant bits, the next 8 and the rest.  (Not contracted: of a v that is a
 // product, fma(a, b, -h) would leave more than 8 bits to l, whose end is cut off.)
 __device__ __forceinline__ void split3(float v, uint32_t& h, uint32_t& m, uint32_t& l) {
 #pragma clang fp contract(off)
@@ -198,6 +198,7 @@ struct Mamba2Split {
   double cum[2][kTok];
   float dts[2][kTok];
   float colf[2][2][kTok];                          // e^{c_m - c_j} dt_j, m the first token behind j's tile; m the first of j's tile
+  int apart[2][4];                                 // tiles whose second factor could leave the floats
   uint32_t count;
 };
 
@@ -254,15 +255,17 @@ __device__ __forceinline__ void mamba2_split_body(const Params& p, Mamba2Split<N
       sm.cum[at][lane] = c;
       sm.dts[at][lane] = dt;
       sm.colf[at][0][lane] = lane < 48 ? expf(static_cast<float>(cm - c)) * dt : 0.f;
-      sm.colf[at][1][lane] = exp_f64(cf - c) * dt;                           // (read only where it cannot overflow)
+      sm.colf[at][1][lane] = exp_f64(cf - c) * dt;                           // (read only where it cannot overflow:)
+      const unsigned long long in_range = __ballot(cf - c < 60.0 && dt < 1e12f);
+      if (i16 == 0) sm.apart[at][g] = (in_range >> (16 * g) & 0xffff) != 0xffff;
       sm.ec[to][lane] = expf(static_cast<float>(c));
       sm.wj[to][lane] = expf(static_cast<float>(cn - c)) * dt;
       if (lane == 0) sm.fix[to][0] = expf(static_cast<float>(cn));
     };
     // Tiles on and below the diagonal of (C B^T)_ij e^{c_i - c_j} dt_j, formed transposed: a lane then holds four j of one i.  The
     // decay is e^{c_i - c_m} e^{c_m - c_j}, one exponential a lane: m is the first token behind j's tile, or the tile's own first on the
-    // diagonal, where the second factor exceeds 1 and a tile that decays by e^60 or more takes its exponentials one by one.  There both
-    // exponents may be many times the one of their product: they keep what a float drops (exp_f64).
+    // diagonal, where the second factor exceeds 1 and a tile that decays by e^60 or more (or has a dt of 1e12 or more, which is part of
+    // it) takes its exponentials one by one.  There both exponents may be many times the one of their product: they keep what a float drops (exp_f64).
     auto product = [&](int k, int ti, int tj) __attribute__((always_inline)) {
       const uint16_t* B = sm.b[k & 1] + (16 * tj + i16) * L::kLs + 8 * g;
       const uint16_t* C = sm.c[k & 1] + (16 * ti + i16) * L::kLs + 8 * g;
@@ -276,7 +279,7 @@ __device__ __forceinline__ void mamba2_split_body(const Params& p, Mamba2Split<N
       const bool diag = ti == tj;
       const double ci = sm.cum[at][i];
       float v[4];
-      if (!diag || sm.cum[at][16 * ti] - sm.cum[at][16 * ti + 15] < 60.0) {
+      if (!diag || !sm.apart[at][ti]) {
         const float w = exp_f64(ci - sm.cum[at][diag ? 16 * ti : 16 * tj + 16]);
         const f32x4_t e = *reinterpret_cast<const f32x4_t*>(&sm.colf[at][diag][j0]);
 #pragma unroll

@@ -1,5 +1,7 @@
 """The chunked recurrences of 16-bit activations on the bf16 matrix cores (three-piece operands): edges of chunks, tiles and columns,
 states that must stay as exact as fp32, and agreement with the general kernels, which rows at odd addresses take."""
+import math
+
 import pytest
 import torch
 
@@ -262,6 +264,24 @@ def test_rows_longer_than_the_floats(device):
         state, gt = torch.zeros(1, heads, K, V, device=device), gates.to(device)
         y = kernels.gated_delta_scan(rows if odd else rows.contiguous(), gt[:, :heads], gt[:, heads:], A_log, bias, state, torch.zeros(1, dtype=torch.int64, device=device),
                                      torch.arange(T, device=device), _segments([T], device), groups, K ** -0.5, form="chunk")
+        assert bool(y.isfinite().all()) and bool(state.isfinite().all()), odd
+        out.append((y.cpu(), state.cpu()))
+    assert _err(out[0][0], out[1][0]) < 1.2e-2 and _err(out[0][1], out[1][1]) < 1e-4
+
+
+@pytest.mark.parametrize("dt,fall", [(1e15, 3.7), (1e12, 3.9), (1e30, 0.5), (1e11, 3.7)])
+def test_steps_so_long_that_a_factor_leaves_the_floats(device, dt, fall):
+    """dt is part of the second factor of a decay on the diagonal, which may be e^60 already: sixteen falls of 3.7 at dt = 1e15 are 8e38."""
+    g = torch.Generator().manual_seed(9)
+    heads, groups, K, V, T = 2, 1, 64, 32, 150
+    act, gates = torch.randn(T, heads * V + 2 * groups * K, generator=g).to(BF), torch.full((T, heads), dt).to(BF)
+    A_log, zero, out = torch.full((heads,), math.log(fall / dt), device=device), torch.zeros(heads, device=device), []
+    for odd in (0, 1):
+        rows = torch.zeros(T, act.shape[1] + 9, dtype=BF, device=device)[:, odd:odd + act.shape[1]]
+        rows.copy_(act)
+        state = torch.zeros(1, heads, K, V, device=device)
+        y = kernels.mamba2_scan(rows if odd else rows.contiguous(), gates.to(device), A_log, zero, zero, state, torch.zeros(1, dtype=torch.int64, device=device),
+                                torch.arange(T, device=device), _segments([T], device), groups, form="chunk")
         assert bool(y.isfinite().all()) and bool(state.isfinite().all()), odd
         out.append((y.cpu(), state.cpu()))
     assert _err(out[0][0], out[1][0]) < 1.2e-2 and _err(out[0][1], out[1][1]) < 1e-4
