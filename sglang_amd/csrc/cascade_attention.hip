@@ -612,10 +612,10 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
   // 813 to 929 us against 709)
   const int total = n_shared_items + n_private;
   int want = span_units / num_kv_heads - n_shared_items;   // the shared items hold workgroups too
-  if (want < span_units / num_kv_heads / 2) want = span_units / num_kv_heads / 2;
   if (want < 1) want = 1;
   const int span = span_units > 0 ? (n_tiles + want - 1) / want : 0;     // tiles of a span
-  const bool spans = span >= kMinSpanTiles && static_cast<int64_t>(total) * num_kv_heads > kOneRoundUnits;      // (uniform)
+  const bool spans = span >= kMinSpanTiles && static_cast<int64_t>(total) * num_kv_heads > kOneRoundUnits &&     // (uniform)
+                     2 * static_cast<int64_t>(n_shared_items) * num_kv_heads <= span_units;
   if (tid == 0) {
     pv.header[0] = total < max_items ? total : max_items;
     pv.header[4] = spans ? span : 0;

@@ -41,7 +41,10 @@ struct CascadePlanView {
 // behind shared prefixes, eight layers, 255 / 234; 640 and 896 units lose 4 to 8 %; with 32 kv heads of one row, where a workgroup waits
 // for its instructions more than for memory, 321 / 345).  Below three 64-token tiles a span the items' single burst is quicker
 // (32 requests of 190 tokens behind a shared prefix 93 us, 100 in spans of two).
-// Nor where the items are no more than run in one round (7 requests of 585 tokens, 32 kv heads: 896 items 123 us, 768 spans 125).
+// Nor where the items are no more than run in one round (7 requests of 585 tokens, 32 kv heads: 896 items 123 us, 768 spans 125), nor where the
+// shared items take more than half of these units: the spans left are long and few, and the last of them begin when shared items end (us for
+// four layers, spans / items: 128 requests of 100 tokens behind one prefix of 2 k 254 / 188, 128 of 130 in 16 groups behind 1 k 301 / 228, 100
+// of 190 behind 1 k 191 / 176, 32 kv heads, 64 of 100 behind 2 k 260 / 224; at exactly half 64 in 4 groups, 1.5 k and 300, 176 / 185).
 constexpr int kSpanUnits = 768;
 constexpr int kOneRoundUnits = 1024;
 constexpr int kMinSpanTiles = 3;

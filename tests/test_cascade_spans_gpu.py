@@ -153,3 +153,30 @@ def test_every_launch_form_reads_the_plan_it_gets(device, lens, plan_heads, Hq, 
         native.call("sgl_amd_debug_cascade_launch_form", 0, 0)
     if not spans and not fp8:
         assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
+@pytest.mark.parametrize("own,prefix,groups,want", [(100, 2000, 1, False), (130, 1000, 16, False), (190, 1100, 1, False), (300, 1000, 6, True), (100, 500, 1, True)])
+def test_no_spans_beside_shared_items_that_fill_the_chip(device, own, prefix, groups, want):
+    """96 requests, 8 kv heads: more than 48 shared items (384 units) leave the private tokens in items.  Either way the oracle's result."""
+    from sglang_amd import kernels as K
+
+    Hq, Hkv, D, B, width = 32, 8, 128, 96, 8192
+    g = torch.Generator().manual_seed(own + prefix)
+    perm = (torch.randperm(groups * prefix + B * own, generator=g) + 1).int()
+    r2t = torch.zeros((B + 1, width), dtype=torch.int32)
+    for b in range(B):
+        s = b * groups // B * prefix
+        r2t[b + 1, :prefix] = perm[s:s + prefix]
+        r2t[b + 1, prefix:prefix + own] = perm[groups * prefix + b * own:groups * prefix + (b + 1) * own]
+    kc, vc = ((torch.randn((perm.numel() + 1, Hkv, D), generator=g) * 0.5).to(BF) for _ in range(2))
+    q = (torch.randn((B, Hq, D), generator=g) * 0.5).to(BF)
+    pool, seq = torch.arange(1, B + 1), torch.full((B,), prefix + own, dtype=torch.int32)
+    ws = K.CascadeWorkspace(B, Hq, D, width, device)
+    r2t_d, pool_d, seq_d = r2t.to(device), pool.to(device), seq.to(device)
+    K.cascade_plan(ws, r2t_d, pool_d, seq_d, Hq, Hkv)
+    plan = K.cascade_plan_summary(ws, B)
+    assert (int(ws.plan[4]) > 0) == want and (plan["n_shared_items"] * Hkv <= SPAN_UNITS // 2) == want
+    out = torch.empty((B, Hq, D), dtype=BF, device=device)
+    K.cascade_decode_attention(ws, q.to(device), kc.to(device), vc.to(device), out, r2t_d, pool_d, seq_d, D ** -0.5)
+    ref = oo.decode_attention(q, kc, vc, r2t, pool, seq.long(), D ** -0.5, compute_dtype=torch.float32).float()
+    assert float((out.cpu().float() - ref).abs().max()) <= 2.0 ** -8 * float(vc.float().abs().max())      # as above
