@@ -44,9 +44,12 @@ constexpr int64_t kSingleShotUnits = 10240;
 // spans: the looping form.  us a layer, Llama-3-8B heads, single-shot against spans, at an 8 k-token table: 8 requests of 5 k 57 / 51, 16 of
 // 4 k 77 / 70, 2 of 7 k 25.0 / 24.0; 4 of 17 k at a 32 k-token table 82.8 / 64.6.  At tables of 1.2 and 2.5 k tokens, whose requests are
 // short: 64 of 0.9 k 51.9 / 53.1, 64 behind a shared prefix 22.5 / 23.5, 32 of 0.3 k 15.8 / 17.9.
+// Not for bf16 rows of head dim 64: four layers of 14 / 2 heads, 16 requests of 700 54 / 57 us, 64 of 400 66 / 69, 16 of 3 k 81 / 83, and above
+// the line items against spans 128 of 600 88 / 94, 128 of 400 behind a shared 1 k 88 / 95.  (Of e4m3 rows 64 of 1.5 k 101 / 92.)
 constexpr int64_t kSpanSingleShotUnits = 2048;
 constexpr int kSpanChunks = 64;
-inline int64_t single_shot_most(int chunks, int group) { return group <= 8 && chunks >= kSpanChunks ? kSpanSingleShotUnits : kSingleShotUnits; }
+inline int64_t single_shot_most(int chunks, bool spans) { return spans && chunks >= kSpanChunks ? kSpanSingleShotUnits : kSingleShotUnits; }
+inline bool walks_spans(int group, int head_dim, bool fp8) { return group <= 8 && (head_dim > 64 || fp8); }
 int64_t g_cascade_single_shot_units = 0;       // worst-case workgroups up to which the one-workgroup-per-unit form is launched (0: the rule above)
 int64_t g_cascade_loop_grid = 256 * 5;         // grid of the looping form: 1280 beat 1024 (= what is resident at four per CU) and equalled 2048
 
@@ -80,6 +83,7 @@ struct ChunkParams {
   int num_kv_heads;
   int slots_total;
   float scale_log2;
+  int walks_spans;              // the looping kernel takes the plan's spans, where it has any, in the place of the private items
 };
 
 // The K rows, then (after S^T) the transposed V rows, pass through ONE 16 KiB LDS image; at D = 128 it is filled twice
@@ -306,10 +310,9 @@ __global__ __launch_bounds__(kThreads, 4) void cascade_chunk_loop_kernel(ChunkPa
   // the line of the workgroup's first item record travels with the header (a grid never reaches beyond max_items x kv heads)
   const int first_rec = cascade_plan_view(p.plan, p.batch, p.max_items).items[8 * (blockIdx.x / static_cast<unsigned>(p.num_kv_heads))];
   // one hop for all of the header that the loop needs: the list's length (shared items, then private items or spans) and what the tail is.
-  // (Spans are walked where a kv head has at most 8 query rows, as in the merge; the items stand beside them.)
-  const bool few = p.group <= 8;
-  const int n_items = __builtin_amdgcn_readfirstlane(p.plan[few ? 5 : 0]), n_shared = __builtin_amdgcn_readfirstlane(p.plan[3]);
-  const bool spans = few && __builtin_amdgcn_readfirstlane(p.plan[4]) > 0;
+  // (The items stand beside the spans for a launch that does not walk these.)
+  const int n_items = __builtin_amdgcn_readfirstlane(p.plan[p.walks_spans ? 5 : 0]), n_shared = __builtin_amdgcn_readfirstlane(p.plan[3]);
+  const bool spans = p.walks_spans && __builtin_amdgcn_readfirstlane(p.plan[4]) > 0;
   asm volatile("" ::"v"(first_rec));
   const int n_units = n_items * p.num_kv_heads;
   const int G = static_cast<int>(gridDim.x), w0 = static_cast<int>(blockIdx.x);
@@ -759,7 +762,7 @@ int sgl_amd_cascade_plan(const int32_t* req_to_token, int64_t req_to_token_strid
                      static_cast<int>(batch * (chunks + 1) * num_kv_heads <= kSingleShotHardCap
                                           ? (batch * (chunks + 1) < max_items ? batch * (chunks + 1) : max_items) : 0),
                      num_kv_heads,
-                     num_q_heads / num_kv_heads <= 8 && batch * (chunks + 1) * num_kv_heads > single_shot_most(chunks, num_q_heads / num_kv_heads) ? kSpanUnits : 0);
+                     num_q_heads / num_kv_heads <= 8 && batch * (chunks + 1) * num_kv_heads > single_shot_most(chunks, true) ? kSpanUnits : 0);
   SGL_CHECK_LAUNCH("cascade_plan");
   return 0;
 }
@@ -826,7 +829,8 @@ int sgl_amd_cascade_decode_attention_ex(const void* q, const void* k_cache, cons
   if (units > max_items) units = max_items;
   const int64_t worst = units * num_kv_heads;
   // (the plan may hold spans: the single-shot form works on its items all the same, and the merge goes by the form launched here)
-  const bool loop = worst > (g_cascade_single_shot_units > 0 ? g_cascade_single_shot_units : single_shot_most(chunks, p.group));
+  p.walks_spans = walks_spans(p.group, head_dim, kv_fp8 != 0) ? 1 : 0;
+  const bool loop = worst > (g_cascade_single_shot_units > 0 ? g_cascade_single_shot_units : single_shot_most(chunks, p.walks_spans != 0));
   dim3 grid(static_cast<unsigned>(loop ? (worst < g_cascade_loop_grid ? worst : g_cascade_loop_grid) : worst));
 #define SGL_LAUNCH_CASC2(D_, KERNEL_)                                                                                 \
   do {                                                                                                       \
@@ -846,7 +850,7 @@ int sgl_amd_cascade_decode_attention_ex(const void* q, const void* k_cache, cons
 #undef SGL_LAUNCH_CASC
   const int hpb = 256 / (head_dim / 4);
   hipLaunchKernelGGL(cascade_merge2_kernel, dim3(static_cast<unsigned>(batch), (num_q_heads + hpb - 1) / hpb), dim3(256), 0, st,
-                     p.ws_acc, p.ws_ml, plan, seq_lens, loop && p.group <= 8 ? 1 : 0, static_cast<uint16_t*>(out), out_token_stride, p.batch, p.max_items,
+                     p.ws_acc, p.ws_ml, plan, seq_lens, loop && p.walks_spans ? 1 : 0, static_cast<uint16_t*>(out), out_token_stride, p.batch, p.max_items,
                      num_q_heads, head_dim, slots_total, kv_fp8 ? v_scale : 1.0f);
   SGL_CHECK_LAUNCH("cascade_decode_attention");
   return 0;
