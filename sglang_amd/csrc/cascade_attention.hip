@@ -51,7 +51,12 @@ constexpr int kSpanChunks = 64;
 inline int64_t single_shot_most(int chunks, bool spans) { return spans && chunks >= kSpanChunks ? kSpanSingleShotUnits : kSingleShotUnits; }
 inline bool walks_spans(int group, int head_dim, bool fp8) { return group <= 8 && (head_dim > 64 || fp8); }
 int64_t g_cascade_single_shot_units = 0;       // worst-case workgroups up to which the one-workgroup-per-unit form is launched (0: the rule above)
-int64_t g_cascade_loop_grid = 256 * 5;         // grid of the looping form: 1280 beat 1024 (= what is resident at four per CU) and equalled 2048
+// Grid of the looping form.  Units behind it are dealt before the launch, those inside it as workgroups end: us for four layers at 1280 / 2048
+// workgroups, 16 requests in 4 groups behind 4 k 182 / 170, 32 of them 185 / 168, 32 kv heads, 32 behind one prefix of 3 k 256 / 242; equal where
+// spans or few items are walked; 2560 and 4096 as 2048.  e4m3 items gain nothing by it, and the workgroups without a unit show (37 requests
+// of 0.9 to 5.1 k 270 / 273).
+constexpr int64_t kLoopGrid = 256 * 8, kLoopGridFp8 = 256 * 5;
+int64_t g_cascade_loop_grid = 0;               // 0: these
 
 __device__ __forceinline__ bf16x8_t as_frag(const U4& v) { return __builtin_bit_cast(bf16x8_t, v); }
 
@@ -108,7 +113,7 @@ struct ChunkParams {
 //     persistent loop died of hoisted LDS addresses), and it is given 128 registers -- four workgroups per CU, no spills --
 //     because at the 96 budget hipcc parks ~30 registers in scratch once there is a loop around the body: that instance was
 //     built and measured (profiles/r05_exp1b_cascade_forms.json): 34.1 us per layer against 26.7 at four per CU and 25.6 for
-//     the one-workgroup-per-unit form on the bench's own table; grids of 1280 / 2048 equal, 1024 (= what is resident) 28.0.
+//     the one-workgroup-per-unit form on the bench's own table; grids of 1280 / 2048 equal there, 1024 (= what is resident) 28.0.
 template <int D, bool FP8, bool HND>
 __global__ __launch_bounds__(kThreads, 5) void cascade_chunk_kernel(ChunkParams p) {
   __shared__ U4 sm[(kChunk / (D > 64 ? D / 64 : 1)) * (D / 8)];   // K: [token of the part][piece ^ swz];  V^T: [d of the part][8-token chunk ^ swz]
@@ -831,7 +836,8 @@ int sgl_amd_cascade_decode_attention_ex(const void* q, const void* k_cache, cons
   // (the plan may hold spans: the single-shot form works on its items all the same, and the merge goes by the form launched here)
   p.walks_spans = walks_spans(p.group, head_dim, kv_fp8 != 0) ? 1 : 0;
   const bool loop = worst > (g_cascade_single_shot_units > 0 ? g_cascade_single_shot_units : single_shot_most(chunks, p.walks_spans != 0));
-  dim3 grid(static_cast<unsigned>(loop ? (worst < g_cascade_loop_grid ? worst : g_cascade_loop_grid) : worst));
+  const int64_t walkers = g_cascade_loop_grid > 0 ? g_cascade_loop_grid : kv_fp8 ? kLoopGridFp8 : kLoopGrid;
+  dim3 grid(static_cast<unsigned>(loop && walkers < worst ? walkers : worst));
 #define SGL_LAUNCH_CASC2(D_, KERNEL_)                                                                                 \
   do {                                                                                                       \
     if (kv_fp8 && kv_layout_hnd) hipLaunchKernelGGL((KERNEL_<D_, true, true>), grid, dim3(kThreads), 0, st, p);   \
@@ -861,7 +867,7 @@ int sgl_amd_debug_cascade_launch_form(int64_t single_shot_units, int64_t loop_gr
   SGL_CHECK_ARG(single_shot_units >= 0 && single_shot_units <= kSingleShotHardCap && loop_grid >= 0 && loop_grid <= (1 << 20),
                 "debug_cascade_launch_form: single_shot_units must be 0..%lld, loop_grid 0..2^20", (long long)kSingleShotHardCap);
   g_cascade_single_shot_units = single_shot_units;
-  g_cascade_loop_grid = loop_grid > 0 ? loop_grid : 256 * 5;
+  g_cascade_loop_grid = loop_grid;
   return 0;
 }
 
