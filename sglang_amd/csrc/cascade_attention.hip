@@ -143,7 +143,7 @@ __device__ __forceinline__ float lane_rows_max(float x) {
 // takes the 16-token tiles w, w + 4, ...  No barrier until the waves' (max, sum, O) sets meet: K rows are the matrix operand as they
 // come (lane = token, four lanes a row), V rows pass through the wave's own 4 KiB image and come out transposed by
 // ds_read_b64_tr_b16.  The next tile's K rows are asked for once this tile's scores are formed, its V rows once this tile's have left
-// the registers, so a wave always has rows in flight; sixteen waves a CU do the rest (16 tokens, not 32: at 32 the 128 registers spill,
+// the registers, so a wave always has rows in flight; the twelve waves a CU of the spans do the rest (16 tokens, not 32: at 32 the 128 registers spill,
 // 256 against 211 us for 32 requests of 2 k tokens in e4m3).
 // What bounds it: the gathered rows -- four layers of 37 requests of 0.9 to 5.1 k tokens in e4m3 481 -> 268 us (2.0 -> 3.6 TB/s), 128
 // requests of 1.5 k in bf16 910 -> 729 us (4.6 TB/s; a large copy reaches 4.9).  Before, a unit was 128 tokens staged through one image

@@ -150,3 +150,27 @@ def test_projection_row_kernels_do_not_spill(tmp_path):
     assert sum("head_prepare_kernel" in k for k in usage) == 8 and sum("latent_down_kernel" in k for k in usage) == 4, sorted(usage)
     for name, u in usage.items():
         assert u["vgpr_spill_count"] == 0 and u["sgpr_spill_count"] == 0 and u["vgpr_count"] <= 128, (name, u)
+
+
+@pytest.mark.skipif(not Path(HIPCC).exists(), reason="hipcc not installed")
+def test_extend_parts_kernels_keep_their_registers_and_lds(tmp_path):
+    """The four-wave form is the eight-wave walk at two workgroups per CU: all of its 256 registers in the bf16 instance of head dim 128, and
+    LDS for two."""
+    usage = _resource_usage("extend_attention.hip", tmp_path)
+    inst = {k: v for k, v in usage.items() if "extend_attention_parts_kernel" in k}
+    assert len(inst) == 4, sorted(usage)                        # head dim {64, 128} x {bf16, e4m3 rows}
+    for name, u in inst.items():
+        assert u["vgpr_spill_count"] == 0 and u["sgpr_spill_count"] == 0 and u["vgpr_count"] <= 256, (name, u)
+        assert u["group_segment_fixed_size"] <= 80 * 1024, (name, u)
+
+
+@pytest.mark.skipif(not Path(HIPCC).exists(), reason="hipcc not installed")
+def test_split_recurrences_keep_their_registers_and_lds(tmp_path):
+    """Preparing and column waves share one kernel of eight waves, two per SIMD: 256 registers each, one workgroup per CU."""
+    usage = _resource_usage("recurrent_chunk.hip", tmp_path)
+    for kernel in ("mamba2_split_kernel", "delta_split_kernel"):
+        inst = {k: v for k, v in usage.items() if kernel in k}
+        assert len(inst) == 3, sorted(usage)                    # state dims of up to 32, 64 and 128
+        for name, u in inst.items():
+            assert u["vgpr_spill_count"] == 0 and u["vgpr_count"] <= 256, (name, u)
+            assert u["group_segment_fixed_size"] <= 160 * 1024, (name, u)
