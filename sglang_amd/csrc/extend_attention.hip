@@ -1140,8 +1140,8 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
     put_v((t + 1) & 1, vst);
     EXT_T(0);
     // (8 waves: in phase 1, where most vector instructions are, a wave goes first; the SIMD's other wave has matrix instructions to issue
-    // beside them when it is in phase 2, and the older of two waves in phase 1 no longer holds the younger back: 708 -> 663 us for 12.6 k
-    // cold tokens of six requests, 64 / 8 heads, 396 -> 384 for 4096 behind 4000.  Two workgroups of 4 waves a CU lose by it, 183 -> 203.)
+    // beside them when it is in phase 2, and the older of two waves in phase 1 no longer holds the younger back: 696 -> 665 us for 12.6 k
+    // cold tokens of six requests, 64 / 8 heads, 406 -> 394 for 4096 behind 4000, 171 -> 166 for 60 x 128 behind 896.  Two workgroups of 4 waves a CU lose by it, 183 -> 203.)
     if constexpr (NWV == 8) __builtin_amdgcn_s_setprio(1);
     // ---- phase 1 ------------------------------------------------------------------------------------------
     constexpr int KF = 3;                            // K fragment sets: reads run two products ahead (1 or 3 ahead: same time)
