@@ -8,11 +8,13 @@
 // the chunks: that walk is the serial chain which bounds the kernel, so everything that does not depend on the state -- rows to LDS,
 // scan of the gates, the tokens' products among themselves -- is done by the preparing waves one chunk ahead.
 //
-// What bounds it now: a round's instruction issue and LDS reads (each column wave reads all rows of the chunk), about 6 900 clocks for 64
-// tokens of Mamba-2 (1 800 of them matrix instructions of a SIMD) and 7 800 for 32 tokens of the delta rule, where the inverse's wave is the
-// longest.  Chunks of 64 suit Mamba-2 (the state is split once a chunk); the inverse and a third image of the rows keep the delta rule at 32.
-// Measured: Mamba-2 64 heads of 64 x 128, 4 segments of 1 600 - 2 460 tokens 458 -> 110 us; delta rule 32 heads of 128 x 128, 3 segments of
-// 1 290 - 1 880 tokens 751 -> 163 us.  Error of the state against 64 bits: 6.8e-8 before, 7e-8 now (relative 2-norm).
+// What bounds it now: a round's instruction issue and LDS reads (each column wave reads all rows of the chunk), 2.8 us for 64 tokens of Mamba-2
+// (1 800 clocks of them matrix instructions of a SIMD) and 2.5 us for 32 tokens of the delta rule, where the inverse's wave is the longest.
+// Chunks of 64 suit Mamba-2 (the state is split once a chunk); the inverse and a third image of the rows keep the delta rule at 32.
+// Measured: Mamba-2 64 heads of 64 x 128, 4 segments of 1 600 - 2 460 tokens 456 -> 109 us; delta rule 32 heads of 128 x 128, 3 segments of
+// 1 290 - 1 880 tokens 749 -> 156 us.  Error of the state against 64 bits (relative 2-norm, general kernel / this one, 14 draws of 17 to 1 800
+// tokens each): Mamba-2 1.0e-7 / 7.4e-8, delta rule 1.4e-7 / 1.1e-7, at most 0.85 of the general kernel's in each of them; behind 2 000 to 8 000
+// tokens of one sign that are hardly forgotten 6.4e-7 .. 1.6e-6 / 1.0e-7 .. 4.1e-7 and 5.5e-7 / 2.5e-7.
 //
 // Operand layouts of the instruction (lane = (i = lane & 15, g = lane / 16), slots j = 0..7): A[row i][8 g + j], B[8 g + j][column i],
 // result rows 4 g + r, column i.  The state's registers go into the next product as they are: tiles 2 u and 2 u + 1 fill the slots of
@@ -480,7 +482,8 @@ __device__ __forceinline__ void mamba2_split_body(const Params& p, Mamba2Split<N
 // ------------------------------------------------------------------------------------------------ gated delta rule, 32 tokens a chunk
 // The products of two fp32 operands (the inverse times the right-hand side, the read-out's matrix times U) are the products of their pieces
 // but the smallest, l l, below 2^-30 of the whole: of two more, m l and l m, truncated pieces make up to 7 x 2^-24 of the product, always
-// towards zero.  Rows 0 .. 15 are products over the first 16 tokens alone.  The matrix cores cut a product's low bits off when they add it to a larger sum, so the large term h h is summed by itself.
+// towards zero.  Rows 0 .. 15 are products over the first 16 tokens alone.  The large term h h is summed by itself: of a sum that is smaller than
+// the product added to it the matrix cores cut the low bits off, 0.17 of the result's last place on average.
 template <int NU>
 struct DeltaSplit {
   static constexpr int kTok = 32, kNp = 32 * NU, kLs = kNp + 8, kVs = 64 + 8, kGs = kTok + 8, kAs = kTok + 4;
