@@ -531,7 +531,7 @@ int sgl_amd_debug_extend_attention_shape(int shape, int flags);
  * environment).  A launch whose worst-case workgroup count (from the request table's width) is <= single_shot_units runs one
  * workgroup per (item, kv head) unit; above it a grid of loop_grid resident workgroups walks the device-built item list.
  * 0 restores a default (10240, or 2048 for at most 8 query heads a kv head and tables of 8 k tokens or more, but for bf16 rows of
- * head dim 64; 2048, of e4m3 rows 1280).  Both forms compute the
+ * head dim 64; 4096, of e4m3 rows and head dim 64 1280).  Both forms compute the
  * same; their bits agree where both cut the tokens alike, which the looping form does not where it walks spans and for e4m3 items of at
  * most 8 query rows (16-token tiles of four waves, merged).  Not part of the reference surface. */
 int sgl_amd_debug_cascade_launch_form(int64_t single_shot_units, int64_t loop_grid);

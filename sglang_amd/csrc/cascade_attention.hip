@@ -51,11 +51,11 @@ constexpr int kSpanChunks = 64;
 inline int64_t single_shot_most(int chunks, bool spans) { return spans && chunks >= kSpanChunks ? kSpanSingleShotUnits : kSingleShotUnits; }
 inline bool walks_spans(int group, int head_dim, bool fp8) { return group <= 8 && (head_dim > 64 || fp8); }
 int64_t g_cascade_single_shot_units = 0;       // worst-case workgroups up to which the one-workgroup-per-unit form is launched (0: the rule above)
-// Grid of the looping form.  Units behind it are dealt before the launch, those inside it as workgroups end: us for four layers at 1280 / 2048
-// workgroups, 16 requests in 4 groups behind 4 k 182 / 170, 32 of them 185 / 168, 32 kv heads, 32 behind one prefix of 3 k 256 / 242; equal where
-// spans or few items are walked; 2560 and 4096 as 2048.  e4m3 items gain nothing by it, and the workgroups without a unit show (37 requests
-// of 0.9 to 5.1 k 270 / 273).
-constexpr int64_t kLoopGrid = 256 * 8, kLoopGridFp8 = 256 * 5;
+// Grid of the looping form.  Units inside it are dealt as workgroups end, those behind it before the launch.  Items of bf16 rows of head dim 128 gain by
+// the first (136 batches at 1280 / 2048 / 4096 / 8192 workgroups: 5.3, 1.7, 0.6 and 0.9 % behind the best of six grids).  Beside spans, never more than
+// 1024, the workgroups without a unit cost 0.3 us a layer of 58.  That is as much beside e4m3 rows (37 requests of 0.9 to 5.1 k 270 us at 1280, 273 at
+// 2048, four layers), whose items are walked only where there are few, and rows of 64 elements gain nothing (128 of 1.2 k, 14 / 2 heads, 130 / 134).
+constexpr int64_t kLoopGrid = 256 * 16, kLoopGridSmallRows = 256 * 5;
 int64_t g_cascade_loop_grid = 0;               // 0: these
 
 __device__ __forceinline__ bf16x8_t as_frag(const U4& v) { return __builtin_bit_cast(bf16x8_t, v); }
@@ -836,7 +836,7 @@ int sgl_amd_cascade_decode_attention_ex(const void* q, const void* k_cache, cons
   // (the plan may hold spans: the single-shot form works on its items all the same, and the merge goes by the form launched here)
   p.walks_spans = walks_spans(p.group, head_dim, kv_fp8 != 0) ? 1 : 0;
   const bool loop = worst > (g_cascade_single_shot_units > 0 ? g_cascade_single_shot_units : single_shot_most(chunks, p.walks_spans != 0));
-  const int64_t walkers = g_cascade_loop_grid > 0 ? g_cascade_loop_grid : kv_fp8 ? kLoopGridFp8 : kLoopGrid;
+  const int64_t walkers = g_cascade_loop_grid > 0 ? g_cascade_loop_grid : kv_fp8 || head_dim == 64 ? kLoopGridSmallRows : kLoopGrid;
   dim3 grid(static_cast<unsigned>(loop && walkers < worst ? walkers : worst));
 #define SGL_LAUNCH_CASC2(D_, KERNEL_)                                                                                 \
   do {                                                                                                       \
