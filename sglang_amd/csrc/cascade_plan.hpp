@@ -39,7 +39,8 @@ struct CascadePlanView {
 // let four run, but the chip starts about 740 of a thousand workgroups at once and the rest only as those end, a second round of a fifth of
 // the work (us for four layers at 1024 / 768 units: 37 requests of 0.9 to 5.1 k tokens in e4m3 278 / 268, 16 of 4 k in bf16 297 / 280, 64
 // behind shared prefixes, eight layers, 255 / 234; 640 and 896 units lose 4 to 8 %; with 32 kv heads of one row, where a workgroup waits
-// for its instructions more than for memory, 321 / 345).  Below three 64-token tiles a span the items' single burst is quicker
+// for its instructions more than for memory, 321 / 345; the items are behind both there, 16 requests of 2 k 530 / 470 in 768 spans, 32 of 400
+// 280 / 241, 37 of 1 k 601 / 530).  Below three 64-token tiles a span the items' single burst is quicker
 // (32 requests of 190 tokens behind a shared prefix 93 us, 100 in spans of two).
 // Nor where the items are no more than run in one round (7 requests of 585 tokens, 32 kv heads: 896 items 123 us, 768 spans 125), nor where the
 // shared items take more than half of these units: the spans left are long and few, and the last of them begin when shared items end (us for
