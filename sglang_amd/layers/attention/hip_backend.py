@@ -24,7 +24,7 @@ from typing import Optional
 import torch
 
 from ... import kernels
-from ...mem_cache.memory_pool import KVWriteLoc, _host_scale
+from ...mem_cache.memory_pool import KVWriteLoc, MHATokenToKVPool, _host_scale
 from .base_attn_backend import AttentionBackend
 
 
@@ -403,19 +403,39 @@ class HipAttnBackend(AttentionBackend):
         out[1:] = torch.cumsum(sizes, 0)
         return out
 
+    def _riding_rows(self, layer, forward_batch, k, v):
+        """(k, v, slots) of a decode step where the attention launches can store them (cascade_decode_attention's new_rows), else None: this
+        package's pool with its own set_kv_buffer, one row a request, bf16 and 16-byte aligned."""
+        pool, loc, b = self.token_to_kv_pool, forward_batch.out_cache_loc, forward_batch.batch_size
+        if type(pool).set_kv_buffer is not MHATokenToKVPool.set_kv_buffer or "set_kv_buffer" in vars(pool):
+            return None
+        if loc.dtype != torch.int64 or loc.dim() != 1 or loc.shape[0] != b or not loc.is_contiguous():
+            return None
+        rows = (b, layer.tp_k_head_num, layer.qk_head_dim)
+        if rows[1:] != (pool.head_num, pool.head_dim):
+            return None
+        for x in (k, v):
+            if x.dtype != torch.bfloat16 or x.shape != rows or x.stride(2) != 1 or x.stride(1) != rows[2] or x.stride(0) % 8 or x.data_ptr() % 16:
+                return None
+        return k, v, loc
+
     def forward_decode(self, q, k, v, layer, forward_batch, save_kv_cache: bool = True, **kwargs):
         self._refuse_unsupported(layer, kwargs)
-        if save_kv_cache and k is not None and v is not None:
-            self._save_kv(layer, forward_batch, k, v)
         m = self.forward_metadata
+        opt = self._layer_options(layer)
+        cascade = m.cascade is not None and "sliding_window" not in opt and "logit_cap" not in opt
+        new_rows = None
+        if save_kv_cache and k is not None and v is not None:
+            new_rows = self._riding_rows(layer, forward_batch, k, v) if cascade else None
+            if new_rows is None:
+                self._save_kv(layer, forward_batch, k, v)
         q3 = q.reshape(-1, layer.tp_q_head_num, layer.qk_head_dim)
         o = torch.empty_like(q3)
-        opt = self._layer_options(layer)
-        if m.cascade is not None and "sliding_window" not in opt and "logit_cap" not in opt:
+        if cascade:
             kernels.cascade_decode_attention(m.cascade, q3, self.token_to_kv_pool.get_key_buffer(layer.layer_id),
                                              self.token_to_kv_pool.get_value_buffer(layer.layer_id), o,
                                              self.req_to_token_pool.req_to_token, self._pool_idx(forward_batch),
-                                             m.seq_lens_i32, layer.scaling, **opt)      # opt: the pool format, if any
+                                             m.seq_lens_i32, layer.scaling, new_rows=new_rows, **opt)      # opt: the pool format, if any
             return o.view(-1, layer.tp_q_head_num * layer.v_head_dim)
         kernels.decode_attention(q3, self.token_to_kv_pool.get_key_buffer(layer.layer_id),
                                  self.token_to_kv_pool.get_value_buffer(layer.layer_id), o,
