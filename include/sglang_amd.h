@@ -694,6 +694,11 @@ int sgl_amd_latent_prefill(const void* q, int64_t q_token, const void* latents, 
     const int32_t* key_first, const int64_t* positions, void* out, int64_t o_token, int heads, int dim, int rot,
     int rank, int vdim, int window, float scale, const float* sinks, void* stream);
 
+/* Inputs of a decode step into the buffers a captured graph reads (decode_cuda_graph_runner.py:1240 load_batch): `given` rows, the rest up to `padded`
+ * the padding entry (id 0, pool row 0, slot 0, length fill_len).  A NULL source: its rows stand in the buffer already. */
+int sgl_amd_stage_decode_inputs(const int64_t* input_ids, const int64_t* req_pool_indices, const int32_t* seq_lens, const int64_t* out_cache_loc,
+                                int64_t* to_input_ids, int64_t* to_req_pool_indices, int32_t* to_seq_lens, int64_t* to_out_cache_loc,
+                                int64_t given, int64_t padded, int fill_len, void* stream);
 /* ---- between a projection and attention (projection_rows.hip) ------------------------------------------------------
  * The source is rows in the activation type, or the fp32 split-K partials of a decode projection (`items` of them item_stride apart, rows
  * row_stride apart, plus `bias` in the activation type).  cos_sin fp32 [max_positions, rot_dims] = cos | sin; dimension i of the rotated

@@ -284,6 +284,21 @@ def clamp_position(seq_lens: torch.Tensor, out: Optional[torch.Tensor] = None) -
     return out
 
 
+def stage_decode_inputs(sources, buffers, given: int, padded: int, fill_len: int) -> bool:
+    """Copies the `given` (input ids, pool rows, lengths, slots) of a decode step into a captured graph's buffers and pads them to `padded` rows, in one
+    launch; a source that is its buffer already stays.  False, and nothing done, where a source is not a dense row of its buffer's type and device."""
+    ptrs, n = [], int(given)
+    for src, buf in zip(sources, buffers):
+        if src.dtype != buf.dtype or src.device != buf.device or src.shape != (n,) or (n > 1 and src.stride(0) != 1):
+            return False
+        ptrs.append(None if src.data_ptr() == buf.data_ptr() else src.data_ptr())
+    _dev(*buffers)
+    _need(n <= padded and all(b.dim() == 1 and b.numel() >= padded and b.is_contiguous() for b in buffers), "stage_decode_inputs: buffers")
+    _need([b.dtype for b in buffers] == [torch.int64, torch.int64, torch.int32, torch.int64], "stage_decode_inputs: int64 ids / rows / slots, int32 lengths")
+    native.call("sgl_amd_stage_decode_inputs", *ptrs, *(b.data_ptr() for b in buffers), n, padded, fill_len, _stream())
+    return True
+
+
 def bigram_rows(ids: torch.Tensor, positions: torch.Tensor, loc: torch.Tensor, req_to_token: torch.Tensor, req_pool_indices: torch.Tensor,
                 tok_seg: Optional[torch.Tensor], slot_ids: torch.Tensor, mul_prev: int, mul_cur: int, buckets: int) -> torch.Tensor:
     """int64 [T]: (previous token * mul_prev + token * mul_cur) mod buckets, `buckets` for a sequence's first token.  slot_ids int32 [slots]

@@ -11,7 +11,7 @@ launched on torch's current stream so they are recorded like any other node.
 What is different here: the attention backend needs no out-of-graph metadata
 refresh (it reads seq_lens / req_to_token on the device), and positions are
 recomputed inside the graph from the static seq_lens buffer, so a replay is
-exactly five small device copies + one hipGraphLaunch.
+one small launch that stages the inputs + one hipGraphLaunch.
 """
 from __future__ import annotations
 
@@ -118,15 +118,17 @@ class DecodeGraphRunner:
     def replay(self, fb: ForwardBatch) -> LogitsProcessorOutput:
         raw = fb.batch_size
         bs = next(b for b in self.capture_bs if b >= raw)
-        if bs != raw:                                     # pad: row 0 / slot 0 / fill length
-            self.input_ids[raw:bs].zero_()
-            self.req_pool_indices[raw:bs].zero_()
-            self.seq_lens[raw:bs].fill_(self.fill)
-            self.out_cache_loc[raw:bs].zero_()
         # a caller that keeps its batch state IN these buffers (harness/engine.py) has nothing to copy
-        for buf, src in ((self.input_ids, fb.input_ids), (self.req_pool_indices, fb.req_pool_indices),
-                         (self.seq_lens, fb.seq_lens), (self.out_cache_loc, fb.out_cache_loc)):
-            if src.data_ptr() != buf.data_ptr():
-                buf[:raw].copy_(src, non_blocking=True)
+        buffers = (self.input_ids, self.req_pool_indices, self.seq_lens, self.out_cache_loc)
+        sources = (fb.input_ids, fb.req_pool_indices, fb.seq_lens, fb.out_cache_loc)
+        if not kernels.stage_decode_inputs(sources, buffers, raw, bs, self.fill):
+            if bs != raw:                                 # pad: row 0 / slot 0 / fill length
+                self.input_ids[raw:bs].zero_()
+                self.req_pool_indices[raw:bs].zero_()
+                self.seq_lens[raw:bs].fill_(self.fill)
+                self.out_cache_loc[raw:bs].zero_()
+            for buf, src in zip(buffers, sources):
+                if src.data_ptr() != buf.data_ptr():
+                    buf[:raw].copy_(src, non_blocking=True)
         self.graphs[bs].replay()
         return LogitsProcessorOutput(next_token_logits=self.outputs[bs][:raw])
