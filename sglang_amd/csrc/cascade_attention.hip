@@ -375,27 +375,10 @@ __global__ __launch_bounds__(kThreads, 4) void cascade_chunk_loop_kernel(ChunkPa
 constexpr int kPlanThreads = 1024;
 constexpr int kPlanMaxBatch = 1024;
 
-// First launch of the plan: every request's leader (the lowest batch index with the same first slot) and the length of
-// the prefix it shares with that leader.  One WAVE per request, sixteen requests per workgroup: inside ONE workgroup the
-// sixteen waves walked their requests one after the other, a memory round trip each -- 26 / 183 us at 64 / 512 requests
-// (benchmarks/r03_exp7_plan_batch.py).  Results go through the plan buffer's `compare` scratch to the second launch.
-__global__ __launch_bounds__(kPlanThreads) void cascade_plan_compare_kernel(
-    const int32_t* __restrict__ req_to_token, int64_t r2t_stride, const int64_t* __restrict__ req_pool_indices,
-    const int32_t* __restrict__ seq_lens, int batch, int32_t* __restrict__ compare) {
-  __shared__ int first_slot[kPlanMaxBatch];
-  __shared__ int pool_row[kPlanMaxBatch], len_s[kPlanMaxBatch];
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  for (int b = tid; b < batch; b += kPlanThreads) {
-    const int len = seq_lens[b];
-    const int row = static_cast<int>(req_pool_indices[b]);
-    pool_row[b] = row;
-    len_s[b] = len;
-    first_slot[b] = len > 1 ? req_to_token[static_cast<int64_t>(row) * r2t_stride] : -1 - b;   // unique when too short
-  }
-  __syncthreads();
-  const int b = static_cast<int>(blockIdx.x) * (kPlanThreads / 64) + wid;
-  if (b >= batch) return;
-  int l = b;
+// One wave: request b's leader (the lowest batch index with the same first slot) and the length of the prefix it shares with that leader.
+__device__ __forceinline__ void compare_request(const int32_t* req_to_token, int64_t r2t_stride, const int* first_slot, const int* pool_row, const int* len_s,
+                                                int b, int lane, int& l, int& common) {
+  l = b;
   const int fs = first_slot[b];
   for (int c0 = 0; c0 < b; c0 += 64) {
     const int c = c0 + lane;
@@ -404,7 +387,7 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_compare_kernel(
   }
   // 2048 positions per round (32 loads in flight per lane and row)
   constexpr int kCmpLoads = 32;
-  int common = 0;
+  common = 0;
   if (l != b) {
     const int32_t* ra = req_to_token + static_cast<int64_t>(pool_row[b]) * r2t_stride;
     const int32_t* rb = req_to_token + static_cast<int64_t>(pool_row[l]) * r2t_stride;
@@ -431,12 +414,42 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_compare_kernel(
       if (first != 0x7fffffff) { common = first; break; }
     }
   }
+}
+
+// First launch of the plan: every request's leader (the lowest batch index with the same first slot) and the length of
+// the prefix it shares with that leader.  One WAVE per request, sixteen requests per workgroup: inside ONE workgroup the
+// sixteen waves walked their requests one after the other, a memory round trip each -- 26 / 183 us at 64 / 512 requests
+// (benchmarks/r03_exp7_plan_batch.py).  Results go through the plan buffer's `compare` scratch to the second launch.
+__global__ __launch_bounds__(kPlanThreads) void cascade_plan_compare_kernel(
+    const int32_t* __restrict__ req_to_token, int64_t r2t_stride, const int64_t* __restrict__ req_pool_indices,
+    const int32_t* __restrict__ seq_lens, int batch, int32_t* __restrict__ compare) {
+  __shared__ int first_slot[kPlanMaxBatch];
+  __shared__ int pool_row[kPlanMaxBatch], len_s[kPlanMaxBatch];
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  for (int b = tid; b < batch; b += kPlanThreads) {
+    const int len = seq_lens[b];
+    const int row = static_cast<int>(req_pool_indices[b]);
+    pool_row[b] = row;
+    len_s[b] = len;
+    first_slot[b] = len > 1 ? req_to_token[static_cast<int64_t>(row) * r2t_stride] : -1 - b;   // unique when too short
+  }
+  __syncthreads();
+  const int b = static_cast<int>(blockIdx.x) * (kPlanThreads / 64) + wid;
+  if (b >= batch) return;
+  int l, common;
+  compare_request(req_to_token, r2t_stride, first_slot, pool_row, len_s, b, lane, l, common);
   if (lane == 0) {
     compare[b] = l;
     compare[batch + b] = common;
   }
 }
 
+// A batch of up to kPlanOneLaunch requests, one a wave, is compared by the plan's own workgroup (ONE).  us, both launches / one: 8 requests behind
+// 500 and 3500 shared tokens 9.4 / 9.0 and 13.1 / 10.8, 16 11.7 / 10.6 and 15.9 / 12.7, and the gap between two launches; a second request a wave
+// takes it back (24: 12.9 / 12.3 and 16.5 / 15.8, 32: 13.8 / 12.8 and 15.9 / 19.1, 64: 15.0 / 21.7 and 15.9 / 32.3).
+constexpr int kPlanOneLaunch = 16;
+
+template <bool ONE>
 __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
     const int32_t* __restrict__ req_to_token, int64_t r2t_stride, const int64_t* __restrict__ req_pool_indices,
     const int32_t* __restrict__ seq_lens, int batch, int min_shared, int chunk_tokens, int tokens_per_tile,
@@ -460,17 +473,31 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
   // request table when all max_items entries were cleared (profiles/r05_exp1_cascade_table_width.json)
   for (int i = tid; i < zero_items; i += kPlanThreads) pv.items[8 * i + 3] = 0;
   for (int b = tid; b < batch; b += kPlanThreads) {
-    pool_row[b] = static_cast<int>(req_pool_indices[b]);
-    len_s[b] = seq_lens[b];
-    leader[b] = pv.compare[b];                         // first launch: leader and common prefix of every request
+    const int row = static_cast<int>(req_pool_indices[b]), len = seq_lens[b];
+    pool_row[b] = row;
+    len_s[b] = len;
+    if constexpr (ONE) {
+      first_slot[b] = len > 1 ? req_to_token[static_cast<int64_t>(row) * r2t_stride] : -1 - b;
+    } else {
+      leader[b] = pv.compare[b];                       // first launch: leader and common prefix of every request
+      scan[b] = pv.compare[batch + b];
+    }
     grp_min[b] = 0x7fffffff;
     grp_cnt[b] = 0;
   }
   __syncthreads();
+  if constexpr (ONE) {
+    for (int b = wid; b < batch; b += kPlanThreads / 64) {
+      int l, common;
+      compare_request(req_to_token, r2t_stride, first_slot, pool_row, len_s, b, lane, l, common);
+      if (lane == 0) { leader[b] = l; scan[b] = common; }
+    }
+    __syncthreads();
+  }
   for (int b = tid; b < batch; b += kPlanThreads) {
     const int l = leader[b];
     if (l != b) {
-      atomicMin(&grp_min[l], pv.compare[batch + b]);
+      atomicMin(&grp_min[l], scan[b]);
       atomicAdd(&grp_cnt[l], 1);
     }
   }
@@ -853,10 +880,12 @@ int sgl_amd_cascade_plan(const int32_t* req_to_token, int64_t req_to_token_strid
                 "cascade_plan: max_items=%lld too small for batch=%lld x %d chunks (need >= %lld)", (long long)max_items,
                 (long long)batch, chunks + 1, (long long)(2 * batch * (chunks + 1)));
   const CascadePlanView pv = cascade_plan_view(plan, batch, max_items);
-  hipLaunchKernelGGL(cascade_plan_compare_kernel, dim3(static_cast<unsigned>((batch + kPlanThreads / 64 - 1) / (kPlanThreads / 64))),
-                     dim3(kPlanThreads), 0, as_stream(stream), req_to_token, req_to_token_stride, req_pool_indices, seq_lens,
-                     static_cast<int>(batch), pv.compare);
-  hipLaunchKernelGGL(cascade_plan_kernel, dim3(1), dim3(kPlanThreads), 0, as_stream(stream), req_to_token,
+  const bool one = batch <= kPlanOneLaunch;
+  if (!one)
+    hipLaunchKernelGGL(cascade_plan_compare_kernel, dim3(static_cast<unsigned>((batch + kPlanThreads / 64 - 1) / (kPlanThreads / 64))),
+                       dim3(kPlanThreads), 0, as_stream(stream), req_to_token, req_to_token_stride, req_pool_indices, seq_lens,
+                       static_cast<int>(batch), pv.compare);
+  hipLaunchKernelGGL(one ? cascade_plan_kernel<true> : cascade_plan_kernel<false>, dim3(1), dim3(kPlanThreads), 0, as_stream(stream), req_to_token,
                      req_to_token_stride, req_pool_indices, seq_lens, static_cast<int>(batch), min_shared_len,
                      kChunk, members_per_item, 64, chunks * kChunk, plan, static_cast<int>(max_items),
                      // end-of-list markers for every item a one-workgroup-per-unit launch of THIS batch can reach (the attention entry's
