@@ -285,7 +285,7 @@ int sgl_amd_top_k_top_p_min_p_sample_ranges(const float* probs, int64_t row_stri
  * ranges: the same bits) -- ranked, filtered by the three rules and sampled.  A row whose candidates cannot decide the rules
  * (they reach the largest value a range left out: flat rows, top-p over a wide nucleus without top-k, > 127 ties, top_k <= 0, a
  * non-finite softmax) is redone inside the same call from its full probability row, written into probs_scratch for that row only.
- * Same ids and kept counts as the two calls it replaces.  num_splits: 2..16 or a multiple of 16 up to 64; ws_fast: caller-owned,
+ * Same ids and kept counts as the two calls it replaces.  num_splits: 2..64; ws_fast: caller-owned,
  * sgl_amd_sample_from_logits_workspace_bytes(batch, num_splits) bytes, 16-byte aligned, no initial state (its last `batch`
  * int32 words hold, after the call, which rows went the long way: tests / telemetry). */
 int64_t sgl_amd_sample_from_logits_workspace_bytes(int64_t batch, int num_splits);

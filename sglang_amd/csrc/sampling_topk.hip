@@ -75,6 +75,20 @@ __device__ __forceinline__ double gumbel_from_hash(uint32_t h) {
   return -log(-lx);
 }
 
+// A log p + gumbel in fp32, within kNear of the fp64 one: only elements within kNear of the largest of these can hold the largest score, and
+// the two fp64 logarithms of a score are most of what an element costs (1.5 k clocks a wave).  The noise that wins lies next to x = 1, where
+// -log(x) is taken from 1 - x (exact: the complement of the hash); the error of all of it is below 3e-4 for |log p| < 4096.
+constexpr float kNear = 0.00390625f;
+constexpr float kLn2f = 0.69314718f;
+__device__ __forceinline__ float gumbel_near(uint32_t h) {
+  const float y = static_cast<float>(~h) * 2.3283064e-10f;           // 1 - x
+  const float x = y < 0.5f ? 1.0f - y : static_cast<float>(h) * 2.3283064e-10f;
+  const float lx = y < 0.015625f ? __fmaf_rn(0.5f * y, y, y) : -kLn2f * __builtin_amdgcn_logf(x);
+  const float g = -kLn2f * __builtin_amdgcn_logf(fmaxf(lx, 2.3283064e-10f));
+  return h == 0u ? -709.0f : g;
+}
+__device__ __forceinline__ float log_near(float p) { return kLn2f * (__builtin_amdgcn_logf(p * 18446744073709551616.0f) - 64.0f); }
+
 struct Best {
   double score;
   int rank;    // sorted rank (tie-break: first)
@@ -1332,7 +1346,7 @@ __global__ __launch_bounds__(kSplitThreads) void sample_logit_candidates_kernel(
     }
   }
   __syncthreads();
-  if (tid < G) {
+  if (tid < G && c * G + tid < S) {                  // (the last list may have fewer ranges)
     // block_sum's association over the four wave sums: (w0 + w2) + (w1 + w3)
     const float tot = (red[tid][0] + red[tid][2]) + (red[tid][1] + red[tid][3]);
     const float mxt = tid == 0 ? mxg[0] : tid == 1 ? mxg[1] : tid == 2 ? mxg[2] : mxg[3];
@@ -1552,6 +1566,225 @@ __device__ void finish_small_list(const SampleParams& p, const int row, const ui
   }
 }
 
+// a condition that is the same in every lane, as a scalar
+__device__ __forceinline__ bool uniform(bool v) { return __builtin_amdgcn_readfirstlane(v ? 1 : 0) != 0; }
+
+// The three rules and the arg-max of a row whose kept columns are too many for one wave, from the COUNTS of its keys.  A bf16 logit is its 16-bit
+// key, so the columns of a key have one probability and consecutive ranks: counts below the largest key, their prefix sums and one probability a
+// key are the sorted row, and a rank's score needs nothing else.  Nothing is sorted; the winner's token is the n-th of its key's columns.
+//   LIST: the candidates in the threads' registers; else the whole row (a pass for the counts, one for the winner's key).
+//   kKeys keys below the largest (32 binades: every positive logit and more).
+// False, and nothing written, where that does not decide the row: the rules reach the frontier (LIST) or leave the keys counted, or two keys
+// have one probability (logits next to zero: their columns are ranked by token together).
+// us of the whole call, [1, 128256] / [16, 128256], before and now, gaussian logits of deviation 2.5: top-p 0.9 alone 423 / 611 and 64 / 75, min-p 0.05
+// alone 303 / 326 and 33 / 42, top-k 200 49 / 58 and 32 / 40.  Before, one workgroup sorted the nucleus (some 10 k columns) in memory, or ranked the
+// list in a loop over it, and scored every rank in fp64.  What bounds it now: the counts' LDS atomics and the ranks' hashes of one workgroup a row.
+constexpr int kKeys = 4096;
+
+template <bool LIST>
+__device__ bool finish_by_keys(const SampleParams& p, const int row, const uint16_t* x, RowSmem& sm, const uint32_t topkey, const float t, const float mx,
+                               const float sum, const int64_t top_k, const float top_p, const bool has_min_p, const float min_p, const uint32_t hpre,
+                               const bool (&keep)[2], const uint32_t (&key16)[2], const int (&tok)[2], const int listed, const Frontier* fr) {
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  uint32_t* cnt = sm.part_cnt;                                       // [kKeys] columns of key topkey - d
+  uint32_t* start = reinterpret_cast<uint32_t*>(sm.cand_tok);        // ... the rank of the first
+  float* prob = reinterpret_cast<float*>(sm.cand_val);
+  double* before = reinterpret_cast<double*>(sm.part_sum);           // the probabilities above them
+  static_assert(kHistCopies * kHistStride >= kKeys && kCand >= kKeys && kKeys == 4 * kT, "four keys a thread");
+  __syncthreads();
+  for (int d = tid; d < kKeys; d += kT) cnt[d] = 0;
+  if (tid == 0) { sm.found_bin = 0x7fffffff; sm.c_above = 0x7fffffff; sm.done_all = 0; sm.n_keep = 0; }
+  __syncthreads();
+  if constexpr (LIST) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      if (keep[u] && topkey - key16[u] < static_cast<uint32_t>(kKeys)) atomicAdd(&cnt[topkey - key16[u]], 1u);
+  } else {
+    auto count = [&](uint32_t bits) __attribute__((always_inline)) {
+      const uint32_t d = topkey - order_hi16(bits);
+      if (d < static_cast<uint32_t>(kKeys)) atomicAdd(&cnt[d], 1u);
+    };
+    const int V4 = p.V & ~3;
+    for (int i0 = 4 * tid; i0 < V4; i0 += 16 * kT) {
+      uint2 q[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (i0 + 4 * kT * u < V4) q[u] = *reinterpret_cast<const uint2*>(x + i0 + 4 * kT * u);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (i0 + 4 * kT * u < V4) { count(q[u].x << 16); count(q[u].x & 0xffff0000u); count(q[u].y << 16); count(q[u].y & 0xffff0000u); }
+    }
+    for (int i = V4 + tid; i < p.V; i += kT) count(static_cast<uint32_t>(x[i]) << 16);
+  }
+  __syncthreads();
+  // ---- ranks, probabilities and prefix sums of four keys a thread ----
+  uint32_t c[4], mine = 0;
+  float pr[4];
+  double mass = 0.0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int d = 4 * tid + j;
+    c[j] = cnt[d];
+    pr[j] = c[j] ? softmax_prob(value_of_order32((topkey - d) << 16 | (((topkey - d) & 0x8000u) ? 0u : 0xffffu)), t, mx, sum) : 0.f;
+    mine += c[j];
+    mass += static_cast<double>(c[j]) * static_cast<double>(pr[j]);
+  }
+  uint32_t upto = wave_prefix(mine);
+  if (lane == 63) sm.wave_a[wid] = static_cast<int>(upto);
+  double S = block_scan_incl(mass, sm.s_score) - mass;               // (its barriers cover wave_a)
+  uint32_t r = upto - mine;
+  int total = 0;
+  for (int w = 0; w < kNW; ++w) {
+    if (w < wid) r += static_cast<uint32_t>(sm.wave_a[w]);
+    total += sm.wave_a[w];
+  }
+  const double over = top_p > 1.001f ? INFINITY : static_cast<double>(top_p > 0.f ? top_p : 0.f) + 2.384185791015625e-07;   // (as top_p_fix_superset)
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int d = 4 * tid + j;
+    start[d] = r;
+    prob[d] = pr[j];
+    before[d] = S;
+    if (c[j]) {
+      if (S > over) atomicMin(&sm.found_bin, static_cast<int>(r));                  // ranks from here on are never kept
+      if (fr && key_of(pr[j]) <= fr->key) atomicMin(&sm.c_above, static_cast<int>(r));      // ... are not the row's own
+    }
+    r += c[j];
+    S += static_cast<double>(c[j]) * static_cast<double>(pr[j]);
+  }
+  __syncthreads();
+  auto bin_of = [&](int rank) __attribute__((always_inline)) {        // the key that holds a rank < total
+    int lo = 0, hi = kKeys - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (static_cast<int>(start[mid] + cnt[mid]) > rank) hi = mid;
+      else lo = mid + 1;
+    }
+    return lo;
+  };
+  const uint32_t min_key = has_min_p ? key_of(prob[0] * min_p) : 0u;
+  const int own = sm.c_above < total ? sm.c_above : total;            // ranks that are the row's own
+  int n = sm.found_bin < own ? sm.found_bin : own;
+  bool decided = cnt[0] != 0 && total > 0;                            // (uniform from here on)
+  if (static_cast<int64_t>(n) >= top_k) n = static_cast<int>(top_k);
+  else if (n == own && decided) {
+    // nothing but the columns behind the counted ones can be kept behind them
+    if constexpr (LIST) {
+      if (fr) {
+        const double excl = own < total ? before[bin_of(own)] : before[kKeys - 1] + static_cast<double>(cnt[kKeys - 1]) * static_cast<double>(prob[kKeys - 1]);
+        decided = !(fr->key >= min_key && exact_top_p_keep(excl + static_cast<double>(fr->prob), fr->prob, top_p));
+      }
+      if (own == total && listed > total) decided = false;
+    } else if (total < p.V) {
+      decided = has_min_p && key_of(prob[bin_of(total - 1)]) < min_key;
+    }
+  }
+  if (!uniform(decided)) return false;
+  // ---- scores: thread = a run of ranks ----
+  const int seg = (n + kT - 1) / kT, r0 = tid * seg, r1 = r0 + seg < n ? r0 + seg : n;
+  int kept = 0, first = 0;
+  bool tied = false;
+  float b1 = -INFINITY, b2 = -INFINITY;                               // the two best of the run
+  int at = -1;
+  auto next_bin = [&](int b, int q) __attribute__((always_inline)) {    // the key of rank q, which lies behind key b
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      ++b;
+      if (static_cast<int>(start[b] + cnt[b]) > q) return b;
+    }
+    return bin_of(q);
+  };
+  auto walk = [&](auto&& f, auto&& crossed) __attribute__((always_inline)) {     // f(rank, key, probability) of every kept rank of the run
+    int b = first;
+    for (int q = r0; q < r1; ++q) {
+      if (static_cast<int>(start[b] + cnt[b]) <= q) {
+        const int from = b;
+        b = next_bin(b, q);
+        crossed(from, b);
+      }
+      const float pb = prob[b];
+      const double incl = before[b] + static_cast<double>(q - static_cast<int>(start[b]) + 1) * static_cast<double>(pb);
+      if (key_of(pb) >= min_key && exact_top_p_keep(incl, pb, top_p)) f(q, b, pb);
+    }
+    return b;
+  };
+  if (r0 < r1) {
+    // columns of two keys with one probability would be ranked together: no key of the run may share its own with the one behind
+    auto compare = [&](int b, int next) __attribute__((always_inline)) { tied |= !(prob[next] < prob[b]); };
+    first = bin_of(r0);
+    const int last = walk([&](int q, int b, float pb) __attribute__((always_inline)) {
+      ++kept;
+      const float near = log_near(pb) + gumbel_near(murmur_hash32(hpre, static_cast<uint32_t>(q)));
+      if (at < 0 || near > b1) { b2 = b1; b1 = near; at = q; }
+      else b2 = fmaxf(b2, near);
+    }, compare);
+    const int end = static_cast<int>(start[last] + cnt[last]);
+    if (end <= r1 || r1 == n) {                                        // (else the next run compares)
+      if (end < total) compare(last, next_bin(last, end));
+      else tied |= LIST ? listed > total : total < p.V;
+    }
+  }
+  if (tied) sm.done_all = 1;
+  const float top = block_max(b1, sm.red);                            // (its barriers cover done_all)
+  if (uniform(sm.done_all != 0)) return false;
+  Best best{0.0, -1, 0};
+  auto score = [&](int q, int b, float pb) __attribute__((always_inline)) {
+    const Best c2{log(static_cast<double>(pb)) + gumbel_from_hash(murmur_hash32(hpre, static_cast<uint32_t>(q))), q, b};
+    if (best_better(best, c2)) best = c2;
+  };
+  if (at >= 0 && b1 >= top - kNear) {
+    if (b2 < top - kNear) {
+      const int b = bin_of(at);
+      score(at, b, prob[b]);
+    } else {
+      walk([&](int q, int b, float pb) __attribute__((always_inline)) {
+        if (log_near(pb) + gumbel_near(murmur_hash32(hpre, static_cast<uint32_t>(q))) >= top - kNear) score(q, b, pb);
+      }, [](int, int) {});
+    }
+  }
+  const int all_kept = static_cast<int>(block_sum(static_cast<float>(kept), sm.red) + 0.5f);   // (< 2^24: exact in fp32)
+  best = block_best(best, sm.s_score, sm.s_rank, sm.s_tok);
+  if (uniform(best.rank < 0)) {                                       // an empty nucleus
+    if (tid == 0) { p.out_ids[row] = 0; if (p.out_n_keep) p.out_n_keep[row] = 0; }
+    return true;
+  }
+  // ---- the winner: the (rank - start)-th token of its key ----
+  const int members = static_cast<int>(cnt[best.token]), nth = best.rank - static_cast<int>(start[best.token]);
+  const uint32_t key = topkey - static_cast<uint32_t>(best.token);
+  if (uniform(members > kLdsKeep)) return false;
+  if constexpr (LIST) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      if (keep[u] && key16[u] == key) sm.toks[atomicAdd(&sm.n_keep, 1)] = tok[u];
+  } else {
+    auto find = [&](uint32_t bits, int i) __attribute__((always_inline)) {
+      if (order_hi16(bits) == key) sm.toks[atomicAdd(&sm.n_keep, 1)] = i;
+    };
+    const int V4 = p.V & ~3;
+    for (int i0 = 4 * tid; i0 < V4; i0 += 16 * kT) {
+      uint2 q[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (i0 + 4 * kT * u < V4) q[u] = *reinterpret_cast<const uint2*>(x + i0 + 4 * kT * u);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int i = i0 + 4 * kT * u;
+        if (i < V4) { find(q[u].x << 16, i); find(q[u].x & 0xffff0000u, i + 1); find(q[u].y << 16, i + 2); find(q[u].y & 0xffff0000u, i + 3); }
+      }
+    }
+    for (int i = V4 + tid; i < p.V; i += kT) find(static_cast<uint32_t>(x[i]) << 16, i);
+  }
+  __syncthreads();
+  for (int e = tid; e < members; e += kT) {
+    const int te = sm.toks[e];
+    int below = 0;
+    for (int j = 0; j < members; ++j) below += sm.toks[j] < te;
+    if (below == nth) p.out_ids[row] = te;
+  }
+  if (tid == 0 && p.out_n_keep) p.out_n_keep[row] = all_kept;
+  return true;
+}
+
 template <typename IN>
 __global__ __launch_bounds__(kT) void sample_finish_fast_kernel(SampleParams p, const IN* __restrict__ logits, int64_t logits_row_stride,
                                                                  const float* __restrict__ temperatures, int S, int R, FastWs ws) {
@@ -1622,10 +1855,13 @@ __global__ __launch_bounds__(kT) void sample_finish_fast_kernel(SampleParams p, 
   __syncthreads();
   const float mx = s_mx, sum = s_sum;
   // (workgroup-uniform) the candidates cannot decide the row
-  const bool bad = s_broken || top_k <= 0 || s_acc == 0 || s_acc >= kDirect || !(t > 0.f) || !(sum > 0.f) || !(sum < INFINITY) || !(mx > -INFINITY) ||
-                   !(mx < INFINITY);
+  const bool by_row = uniform(s_broken || top_k <= 0 || s_acc == 0 || !(t > 0.f) || !(sum > 0.f) || !(sum < INFINITY) || !(mx > -INFINITY) || !(mx < INFINITY));
+  const bool bad = by_row || uniform(s_acc >= kDirect);
+  constexpr bool kKeyed = sizeof(IN) == 2;              // (a bf16 logit is its key)
+  const uint32_t topkey = s_top >> 16;
+  const uint32_t hpre = murmur_prefix(seed, spos);
+  if (top_k > p.V) top_k = p.V;
   if (!bad) {
-    if (top_k > p.V) top_k = p.V;
     const unsigned long long p_fix = top_p_fix_superset(top_p);
     bool have[2];
     uint32_t key16[2], pbits[2];
@@ -1644,7 +1880,6 @@ __global__ __launch_bounds__(kT) void sample_finish_fast_kernel(SampleParams p, 
     // join the elements the ranges left out: the frontier rises to the largest of them. ----
     uint32_t cutkey = 0;
     bool found_any = true;
-    const uint32_t topkey = s_top >> 16;
     int near_cut;
     {
       uint32_t bin[2];
@@ -1673,7 +1908,7 @@ __global__ __launch_bounds__(kT) void sample_finish_fast_kernel(SampleParams p, 
       const bool cond_excl = static_cast<int64_t>(vc - my_c) >= top_k || vs - my_s >= p_fix;
       if (cond_incl && !cond_excl) s_near = tid;
       __syncthreads();
-      near_cut = s_near;
+      near_cut = __builtin_amdgcn_readfirstlane(s_near);
     }
     if (near_cut >= 0 && near_cut < kT - 1) {
       cutkey = topkey - static_cast<uint32_t>(near_cut);
@@ -1730,7 +1965,7 @@ __global__ __launch_bounds__(kT) void sample_finish_fast_kernel(SampleParams p, 
           }
         }
         __syncthreads();
-        const int fb = level == 0 ? sm.found_bin : sm.n_eq_keep;
+        const int fb = __builtin_amdgcn_readfirstlane(level == 0 ? sm.found_bin : sm.n_eq_keep);
         if (fb < 0) { found_any = false; break; }       // (uniform) level 0 only: the whole list is inside both limits
         cutkey = level == 0 ? (static_cast<uint32_t>(fb) << 8) : (cutkey | static_cast<uint32_t>(fb));
         base_c = static_cast<uint32_t>(sm.c_above);
@@ -1760,8 +1995,8 @@ __global__ __launch_bounds__(kT) void sample_finish_fast_kernel(SampleParams p, 
       if (keep[1]) { const int pos = at + __popcll(b0) + __popcll(b1 & lt_mask); sm.cand_val[pos] = pbits[1]; sm.cand_tok[pos] = tok[1]; }
     }
     __syncthreads();
-    const int n = s_n;
-    const bool has_front = s_front != 0u;
+    const int n = __builtin_amdgcn_readfirstlane(s_n);
+    const bool has_front = uniform(s_front != 0u);
     const float front = value_of_order32(s_front);
     Frontier fr;
     fr.unusable = &s_unusable;
@@ -1795,14 +2030,26 @@ __global__ __launch_bounds__(kT) void sample_finish_fast_kernel(SampleParams p, 
       if (wid == 0)
         finish_small_list(p, row, sm.cand_val, sm.cand_tok, sm.keys, sm.toks, n, top_k, top_p, p.min_ps != nullptr, min_p, s_part, s_log,
                           s_log_sorted, s_gumbel, has_front ? &fr : nullptr);
+    } else if constexpr (kKeyed) {
+      const bool done = finish_by_keys<true>(p, row, nullptr, sm, topkey, t, mx, sum, top_k, top_p, p.min_ps != nullptr, min_p, hpre, keep, key16, tok, n,
+                                             has_front ? &fr : nullptr);
+      if (!done && tid == 0) s_unusable = 1;
     } else {
       sample_row(p, row, sm, n, has_front ? &fr : nullptr);
     }
     __syncthreads();
   }
-  const bool redo = bad || s_unusable;
+  const bool redo = bad || uniform(s_unusable != 0);
   if (tid == 0) ws.fallback[row] = redo ? 1 : 0;
   if (!redo) return;
+  if constexpr (kKeyed) {
+    const bool no[2] = {false, false};
+    const uint32_t no_key[2] = {0u, 0u};
+    if (!by_row && finish_by_keys<false>(p, row, logits + static_cast<int64_t>(row) * logits_row_stride, sm, topkey, t, mx, sum, top_k, top_p,
+                                         p.min_ps != nullptr, min_p, hpre, no, no_key, tok, 0, nullptr))
+      return;
+    __syncthreads();
+  }
   // ---- the long way, for this row only: its probabilities into the scratch matrix (this workgroup writes the whole row and is the
   // only one to read it), then the row routine on them ----
   {
@@ -2029,9 +2276,10 @@ int sgl_amd_top_k_top_p_min_p_sample_from_logits(const void* logits, int logits_
   const int64_t per_range = ((vocab + num_splits - 1) / num_splits + 3) / 4 * 4;
   // (no more ranges a workgroup where the rows are short: a list holds its columns' 64 largest, so with four ranges to a list [128, 32000]
   // takes 24 us in place of 28 at top-k 50, but rows that keep some hundred columns no longer fit: top-k 400 170 us in place of 78)
-  const int G = (num_splits >= kFastRangesMax && num_splits % kFastRangesMax == 0) ? num_splits / kFastRangesMax : 1;
-  const int R = num_splits / G;
-  SGL_CHECK_ARG(R <= kFastRangesMax, "sample_from_logits: num_splits must be <= 16 or a multiple of 16");
+  // (any range count: 51 ranges for 40 rows make 13 lists of four, the last of three.  Such batches took the two calls, us: 100 rows of 128256
+  // 112 / 36 at top-k 20, 358 / 58 at top-k 200; so did rows too short for 64 ranges of 512, 5 rows of 32000 66 / 27)
+  const int G = (num_splits + kFastRangesMax - 1) / kFastRangesMax;
+  const int R = (num_splits + G - 1) / G;
   const int J = static_cast<int>((per_range + 1023) / 1024);
   SGL_CHECK_ARG(G <= 4 && G * J <= kFastSlots, "sample_from_logits: a workgroup holds at most 16384 columns of a row (vocab / ranges too large)");
   const dim3 cgrid(R, static_cast<unsigned>(batch));

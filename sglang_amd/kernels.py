@@ -695,22 +695,23 @@ def top_k_top_p_min_p_sample(probs: torch.Tensor, top_ks: Optional[torch.Tensor]
 
 def sample_from_logits(logits: torch.Tensor, temperatures: torch.Tensor, top_ks: Optional[torch.Tensor],
                        top_ps: Optional[torch.Tensor], min_ps: Optional[torch.Tensor], sampling_seed: Optional[torch.Tensor],
-                       positions: Optional[torch.Tensor], return_n_keep: bool = False, return_fallback: bool = False):
+                       positions: Optional[torch.Tensor], return_n_keep: bool = False, return_fallback: bool = False, any_ranges: bool = False):
     """sampler.py:211-260 for the logits of a decode-sized batch -- bf16 (the model's dtype) or fp32 (what the reference's
     LogitsProcessor hands its Sampler) -- in one native call: softmax(logits / T) + the filtered sampler, the probabilities never
     written and the logits left as they are (sampling_topk.hip: candidates / finish; rows the candidates cannot decide are redone
     from their full probability row inside the finish launch).  Same ids and kept counts as softmax_temperature_{,from_bf16} +
-    top_k_top_p_min_p_sample.  None when the shape is not that case (the caller takes the two calls)."""
+    top_k_top_p_min_p_sample.  None when the shape is not that case (the caller takes the two calls).  any_ranges: also range counts beyond 16 that
+    are no multiple of it (40 rows: 51), and rows too short for 64 of them (32000 columns: 62, where the two calls take one workgroup a row)."""
     _dev(logits, temperatures)
     if logits.dtype not in (_BF16, torch.float32) or logits.dim() != 2 or logits.stride(1) != 1:
         return None
     B, V = logits.shape
     t = temperatures.reshape(-1)
     bf = logits.dtype == _BF16
-    splits = min(64, 2048 // max(1, B))            # the softmax's own range count: the partials are its partials
+    splits = min(64, 2048 // max(1, B), V // 512 if any_ranges else 64)            # the softmax's own range count: the partials are its partials
     per = ((V + splits - 1) // max(1, splits) + 3) // 4 * 4
-    groups = splits // 16 if (splits >= 16 and splits % 16 == 0) else 1
-    if not (B and splits >= 2 and (splits <= 16 or splits % 16 == 0) and V >= 4096 * splits // 8 and groups * ((per + 1023) // 1024) <= 16
+    groups = (splits + 15) // 16
+    if not (B and splits >= 2 and (any_ranges or splits <= 16 or splits % 16 == 0) and V >= 4096 * splits // 8 and groups * ((per + 1023) // 1024) <= 16
             and logits.data_ptr() % (8 if bf else 16) == 0 and logits.stride(0) % 4 == 0 and B <= 65535
             and t.dtype == torch.float32 and t.numel() == B and t.is_contiguous()):
         return None

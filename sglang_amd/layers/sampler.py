@@ -94,7 +94,7 @@ class Sampler(nn.Module):
                 # logits are widened inside the softmax launches (exact; no separate pass)
                 if not simple_sampling_case:
                     ids = kernels.sample_from_logits(logits, sampling_info.temperatures, sampling_info.top_ks, sampling_info.top_ps,
-                                                     min_ps, sampling_info.sampling_seed, positions)
+                                                     min_ps, sampling_info.sampling_seed, positions, any_ranges=True)
                     served["one_call_from_logits" if ids is not None else "softmax_then_sample"] += 1
                 if ids is None and logits.dtype == torch.bfloat16:
                     probs = kernels.softmax_temperature_from_bf16(logits, sampling_info.temperatures)

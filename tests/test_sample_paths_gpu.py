@@ -92,3 +92,45 @@ def test_rows_that_keep_some_hundred_columns_are_decided_from_the_lists(device):
     top_k, seeds, pos = torch.full((B,), 400, dtype=torch.int32, device=device), torch.arange(B, device=device), torch.arange(B, device=device)
     out = K.sample_from_logits(lg, torch.ones((B, 1), device=device), top_k, None, None, seeds, pos, return_n_keep=True, return_fallback=True)
     assert bool((out[1] == 400).all()) and not bool(out[2].any())
+
+
+def _rows(device, B, V, seed):
+    """bf16 logits [B, V] of several kinds, with temperatures, seeds and positions."""
+    Vp = V + (-V) % 4
+    g = torch.Generator(device=device).manual_seed(seed)
+    rn = lambda *s: torch.randn(s, generator=g, device=device)
+    lg = rn(B, Vp) * 2.5
+    temps = torch.rand((B, 1), generator=g, device=device) * 0.6 + 0.6
+    temps[0] = 1.0
+    if B >= 12:
+        lg[1] = (rn(Vp) * 8).round() / 8                            # few keys, hundreds of columns each
+        lg[2] = rn(Vp) * 0.3                                        # flat: the nucleus crosses zero
+        lg[3] = -(rn(Vp).abs() * 3 + 1)                             # no positive column
+        lg[4] = rn(Vp) * 1e-6                                       # distinct logits, equal probabilities
+        lg[4, 5] = 3.0
+        lg[5, torch.randperm(Vp, generator=torch.Generator().manual_seed(1))[: Vp - 90].to(device)] = -float("inf")
+        lg[6] = rn(Vp) * 8                                          # peaked
+        lg[7] -= 20.0
+        lg[8] = 0.0
+        lg[9, 3] = float("nan")
+        temps[10] = 4.0
+        temps[11] = 0.05
+    return lg.to(torch.bfloat16)[:, :V], temps, torch.arange(B, device=device) * 7919 + 3, torch.arange(B, device=device) + 11
+
+
+@pytest.mark.parametrize("B,V", [(1, 128256), (12, 128256), (40, 128256), (45, 50257), (100, 151936), (120, 40002), (90, 65537)])
+@pytest.mark.parametrize("top_k,top_p,min_p", [(200, 1.0, 0.0), (200, 0.7, 0.0), (65, 0.999, 0.02), (1000, 0.9, 0.0), (1 << 30, 0.9, 0.0),
+                                               (1 << 30, 0.5, 0.01), (1 << 30, 1.0, 0.05), (40, 0.9, 0.0)])
+def test_rows_decided_by_their_keys_equal_softmax_then_sample(device, B, V, top_k, top_p, min_p):
+    """Nuclei beyond one wave are decided from the counts of their 16-bit keys, from the candidate lists or from the row; any number of ranges."""
+    from sglang_amd import kernels as K
+
+    lg, temps, seeds, pos = _rows(device, B, V, V + B + top_k % 1000)
+    ks = torch.full((B,), top_k, dtype=torch.int32, device=device)
+    ps, ms = torch.full((B,), top_p, device=device), torch.full((B,), min_p, device=device) if min_p else None
+    probs = K.softmax_temperature_from_bf16(lg, temps)
+    assert probs is not None
+    want, want_n = K.top_k_top_p_min_p_sample(probs, ks, ps, ms, seeds, pos, return_n_keep=True)
+    got, got_n = K.sample_from_logits(lg, temps, ks, ps, ms, seeds, pos, return_n_keep=True, any_ranges=True)
+    bad = ((got == want) & (got_n == want_n)).logical_not().nonzero().flatten().tolist()
+    assert not bad, [(r, int(got[r]), int(want[r]), int(got_n[r]), int(want_n[r])) for r in bad]
