@@ -277,6 +277,13 @@ int sgl_amd_top_k_top_p_min_p_sample_ranges(const float* probs, int64_t row_stri
                                             const int64_t* seeds, const int64_t* positions, int32_t* out_ids,
                                             void* ws_keys, void* ws_toks, int32_t* out_n_keep, int num_ranges,
                                             void* ws_ranges, void* stream);
+/* sampling_from_probs_torch (sampler.py:732-750) for the logits of a decode-sized batch: the ids of sgl_amd_softmax_temperature_split{,_bf16}
+ * (num_splits ranges) + sgl_amd_top_k_top_p_min_p_sample(filtered = 0) without the probabilities in memory.  ws: caller-owned,
+ * sgl_amd_sample_unfiltered_from_logits_workspace_bytes(batch, num_splits) bytes, 16-byte aligned, no initial state. */
+int64_t sgl_amd_sample_unfiltered_from_logits_workspace_bytes(int64_t batch, int num_splits);
+int sgl_amd_sample_unfiltered_from_logits(const void* logits, int logits_is_bf16, int64_t logits_row_stride, const float* temperatures,
+                                          int64_t batch, int64_t vocab, const int64_t* seeds, const int64_t* positions, int32_t* out_ids,
+                                          int num_splits, void* ws, void* stream);
 /* sampler.py:211-260 in one call for the logits of a decode-sized batch -- bf16 (the model's dtype) or fp32 (what the reference's
  * LogitsProcessor hands its Sampler: logits_processor.py `.float()`) --: softmax(logits / T) followed by the filtered
  * sampler above, without ever writing the [batch, vocab] probabilities (the fp32 logits are NOT overwritten with them).  p(x) is monotone in the logit, so every column range

@@ -2130,6 +2130,118 @@ __global__ __launch_bounds__(64) void sample_unfiltered_merge_kernel(SampleParam
   }
 }
 
+// ---- the unfiltered case straight from the logits: no probabilities are written -----------------------------------------
+// Range partials of the softmax (a launch), then every range scores its columns and a wave a row takes the best range: the ids of the softmax's two
+// launches and the two above.  A column costs its quotient, its noise and two fp32 logarithms; only the columns that may hold a wave's best
+// (kNear) get the probability of the normalise launch and the score in fp64.  Rows whose softmax is not finite, or whose largest quotient is beyond
+// the fp32 estimate, score every column so.
+// us, [1, 128256] / [16, 128256] / [100, 128256]: 38 / 45 / 129 in four launches, 20 / 20 / 53 now.
+template <typename IN>
+__global__ __launch_bounds__(kSplitThreads) void logit_partials_kernel(const IN* __restrict__ logits, const float* __restrict__ temperatures, int64_t vocab,
+                                                                      int64_t row_stride, int splits, float* __restrict__ partials) {
+  __shared__ float scratch[16];
+  const int64_t row = blockIdx.y;
+  int64_t b, e;
+  split_range_of(vocab, splits, blockIdx.x, &b, &e);
+  float mx, sum;
+  range_partial<IN>(logits + row * row_stride, temperatures[row], b, e, scratch, &mx, &sum);
+  if (threadIdx.x == 0) {
+    partials[(row * splits + blockIdx.x) * 2 + 0] = mx;
+    partials[(row * splits + blockIdx.x) * 2 + 1] = sum;
+  }
+}
+
+template <typename IN>
+__global__ __launch_bounds__(kSplitThreads) void sample_logits_unfiltered_kernel(const IN* __restrict__ logits, int64_t row_stride,
+                                                                                const float* __restrict__ temperatures, const float* __restrict__ partials,
+                                                                                int V, int splits, const int64_t* __restrict__ seeds,
+                                                                                const int64_t* __restrict__ positions, PartialBest* __restrict__ bests) {
+  __shared__ float s_mx, s_sum;
+  __shared__ double w_score[kSplitThreads / 64];
+  __shared__ int w_tok[kSplitThreads / 64];
+  const int row = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const IN* x = logits + static_cast<int64_t>(row) * row_stride;
+  const float t = temperatures[row];
+  if (wid == 0) {                                      // merge_partials' arithmetic, the exponentials side by side (sample_finish_fast_kernel)
+    const float pm = lane < splits ? partials[(static_cast<int64_t>(row) * splits + lane) * 2] : -INFINITY;
+    float ps = lane < splits ? partials[(static_cast<int64_t>(row) * splits + lane) * 2 + 1] : 0.f;
+    ps = pm > -INFINITY ? ps : 0.f;
+    const float mx = wave_max(pm);
+    const float ex = pm > -INFINITY ? expf(pm - mx) : 0.f;
+    float sum = 0.f;
+    for (int s2 = 0; s2 < splits; ++s2) {
+      const float es = __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(__float_as_uint(ex)), s2)));
+      const float ss = __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(__float_as_uint(ps)), s2)));
+      sum = __fmaf_rn(ss, es, sum);
+    }
+    if (lane == 0) { s_mx = mx; s_sum = sum; }
+  }
+  __syncthreads();
+  const float mx = s_mx, sum = s_sum;
+  const uint32_t hpre = murmur_prefix(static_cast<uint64_t>(seeds[row]), positions ? static_cast<uint32_t>(positions[row] & 0xffffffffll) : 0u);
+  const bool all = !(t > 0.f) || !(sum > 0.f) || !(sum < INFINITY) || !(fabsf(mx) < 4096.f) || !(t >= 1e-30f) || !(t <= 1e30f);    // (uniform)
+  const float rt = 1.0f / t, shift = mx + log_near(sum);
+  int64_t b64, e64;
+  split_range_of(V, splits, blockIdx.x, &b64, &e64);
+  const int b = static_cast<int>(b64), e = static_cast<int>(e64);
+  Best best{0.0, -1, 0};
+  auto score = [&](float v, int i) __attribute__((always_inline)) {
+    const Best c{static_cast<double>(logf(softmax_prob(v, t, mx, sum))) + gumbel_from_hash(murmur_hash32(hpre, static_cast<uint32_t>(i))), i, i};
+    if (best_better(best, c)) best = c;
+  };
+  float near_most = -INFINITY;                         // the wave's largest estimate so far
+  constexpr int N = 2;                                 // four columns a thread and step, N steps at a time
+  for (int i0 = b + 4 * tid; i0 - 4 * tid < e; i0 += 4 * N * kSplitThreads) {
+    float v[4 * N], near[4 * N], most = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const int i = i0 + 4 * u * kSplitThreads;
+      if (i + 4 <= e) {
+        float q[4];
+        ld4<IN>(x + i, q);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[4 * u + k] = q[k];
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[4 * u + k] = i + k < e ? ld1(x + i + k) : 0.f;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4 * N; ++u) {
+      const int i = i0 + 4 * (u / 4) * kSplitThreads + (u & 3);
+      near[u] = i < e ? __fmaf_rn(v[u], rt, -shift) + gumbel_near(murmur_hash32(hpre, static_cast<uint32_t>(i))) : -INFINITY;
+      most = fmaxf(most, near[u]);
+    }
+    near_most = fmaxf(near_most, wave_max(most));
+    const float cut = near_most - kNear;
+#pragma unroll
+    for (int u = 0; u < 4 * N; ++u) {
+      const int i = i0 + 4 * (u / 4) * kSplitThreads + (u & 3);
+      if (i < e && (all || !(near[u] < cut))) score(v[u], i);
+    }
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    Best o;
+    o.score = __shfl_xor(best.score, off, 64);
+    o.rank = __shfl_xor(best.rank, off, 64);
+    o.token = __shfl_xor(best.token, off, 64);
+    if (best_better(best, o)) best = o;
+  }
+  if (lane == 0) { w_score[wid] = best.score; w_tok[wid] = best.rank; }
+  __syncthreads();
+  if (tid == 0) {
+    Best r{0.0, -1, 0};
+#pragma unroll
+    for (int w = 0; w < kSplitThreads / 64; ++w) {
+      const Best o{w_score[w], w_tok[w], w_tok[w]};
+      if (best_better(r, o)) r = o;
+    }
+    PartialBest o;
+    o.score = r.score; o.rank = r.rank; o.token = r.token;
+    bests[static_cast<int64_t>(row) * splits + blockIdx.x] = o;
+  }
+}
+
 // rank-0 token of an empty nucleus must be the arg max of the row; handled by a tiny fix-up
 // kernel so that the common path stays branch-free.
 __global__ __launch_bounds__(kT) void empty_nucleus_fixup_kernel(SampleParams p) {
@@ -2299,6 +2411,41 @@ int sgl_amd_top_k_top_p_min_p_sample_from_logits(const void* logits, int logits_
   else SGL_LAUNCH_FAST(float);
 #undef SGL_LAUNCH_FAST
   SGL_CHECK_LAUNCH("top_k_top_p_min_p_sample_from_logits");
+  return 0;
+}
+
+int64_t sgl_amd_sample_unfiltered_from_logits_workspace_bytes(int64_t batch, int num_splits) { return batch * num_splits * (16 + 8); }
+
+int sgl_amd_sample_unfiltered_from_logits(const void* logits, int logits_is_bf16, int64_t logits_row_stride, const float* temperatures, int64_t batch,
+                                          int64_t vocab, const int64_t* seeds, const int64_t* positions, int32_t* out_ids, int num_splits, void* ws,
+                                          void* stream) {
+  SGL_CLEAR_STALE_ERROR();
+  SGL_CHECK_ARG(vocab > 0 && vocab <= 0x7ffffff0LL && batch <= 65535, "sample_unfiltered_from_logits: bad shape");
+  SGL_CHECK_ARG(seeds != nullptr && temperatures != nullptr && out_ids != nullptr, "sample_unfiltered_from_logits: seeds, temperatures and ids are required");
+  SGL_CHECK_ARG(num_splits >= 1 && num_splits <= 64 && ws && (reinterpret_cast<uintptr_t>(ws) & 15) == 0,
+                "sample_unfiltered_from_logits: 1..64 ranges and a 16-byte aligned workspace");
+  SGL_CHECK_ARG(logits && (reinterpret_cast<uintptr_t>(logits) & (logits_is_bf16 ? 7 : 15)) == 0 && logits_row_stride % 4 == 0,
+                "sample_unfiltered_from_logits: needs 8-byte aligned bf16 (16-byte aligned fp32) rows");
+  if (batch == 0) return 0;
+  SampleParams p{};
+  p.V = static_cast<int>(vocab);
+  p.out_ids = out_ids;
+  PartialBest* bests = static_cast<PartialBest*>(ws);
+  float* partials = reinterpret_cast<float*>(bests + batch * num_splits);
+  const dim3 grid(num_splits, static_cast<unsigned>(batch));
+#define SGL_LAUNCH_UNFILTERED(IN_)                                                                                                            \
+  do {                                                                                                                                        \
+    const IN_* x = static_cast<const IN_*>(logits);                                                                                           \
+    hipLaunchKernelGGL(logit_partials_kernel<IN_>, grid, dim3(kSplitThreads), 0, as_stream(stream), x, temperatures, vocab, logits_row_stride, \
+                       num_splits, partials);                                                                                                 \
+    hipLaunchKernelGGL(sample_logits_unfiltered_kernel<IN_>, grid, dim3(kSplitThreads), 0, as_stream(stream), x, logits_row_stride,            \
+                       temperatures, partials, p.V, num_splits, seeds, positions, bests);                                                     \
+  } while (0)
+  if (logits_is_bf16) SGL_LAUNCH_UNFILTERED(uint16_t);
+  else SGL_LAUNCH_UNFILTERED(float);
+#undef SGL_LAUNCH_UNFILTERED
+  hipLaunchKernelGGL(sample_unfiltered_merge_kernel, dim3(static_cast<unsigned>(batch)), dim3(64), 0, as_stream(stream), p, num_splits, bests);
+  SGL_CHECK_LAUNCH("sample_unfiltered_from_logits");
   return 0;
 }
 

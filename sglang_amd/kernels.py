@@ -748,6 +748,34 @@ def sample_from_logits(logits: torch.Tensor, temperatures: torch.Tensor, top_ks:
     return out[0] if len(out) == 1 else out
 
 
+def sample_unfiltered_from_logits(logits: torch.Tensor, temperatures: torch.Tensor, sampling_seed: Optional[torch.Tensor],
+                                  positions: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """sampler.py:211-216, 732-750 for the logits (bf16 or fp32) of a decode-sized batch: the ids of softmax_temperature_{,from_bf16} +
+    top_k_top_p_min_p_sample(filtered=False), the probabilities never written and the logits left as they are.  None when the shape is not that
+    case (the caller takes the two calls)."""
+    _dev(logits, temperatures)
+    if logits.dtype not in (_BF16, torch.float32) or logits.dim() != 2 or logits.stride(1) != 1:
+        return None
+    (B, V), t, bf = logits.shape, temperatures.reshape(-1), logits.dtype == _BF16
+    splits = min(64, 2048 // max(1, B), V // 512)
+    if not (B and splits >= 2 and B <= 65535 and logits.data_ptr() % (8 if bf else 16) == 0 and logits.stride(0) % 4 == 0
+            and t.dtype == torch.float32 and t.numel() == B and t.is_contiguous()):
+        return None
+    dev = logits.device
+    if sampling_seed is None:
+        sampling_seed = torch.randint(0, 2 ** 62, (B,), dtype=torch.int64, device=dev)
+    seeds = sampling_seed.to(torch.int64) if sampling_seed.dtype != torch.int64 else sampling_seed
+    _need(seeds.numel() == B and seeds.is_contiguous(), "sample: seeds [B]")
+    if positions is not None:
+        positions = positions.to(torch.int64).contiguous()
+        _need(positions.numel() == B, "sample: positions [B]")
+    ids = torch.empty(B, dtype=torch.int32, device=dev)
+    ws = torch.empty(native.lib().sgl_amd_sample_unfiltered_from_logits_workspace_bytes(B, splits) // 8, dtype=torch.int64, device=dev)
+    native.call("sgl_amd_sample_unfiltered_from_logits", logits.data_ptr(), 1 if bf else 0, logits.stride(0), t.data_ptr(), B, V, seeds.data_ptr(),
+                _ptr(positions), ids.data_ptr(), splits, ws.data_ptr(), _stream())
+    return ids
+
+
 def sample_from_bf16_logits(logits: torch.Tensor, *args, **kwargs):
     """sample_from_logits for bf16 logits only (None otherwise)."""
     return sample_from_logits(logits, *args, **kwargs) if logits.dtype == _BF16 else None

@@ -90,12 +90,14 @@ class Sampler(nn.Module):
             if not return_logprob:
                 # The logits of a decode-sized batch (bf16, or the fp32 the reference's LogitsProcessor hands over), no logprobs asked
                 # for.  Filtered sampling: ONE native call, the probabilities are never written (and the logits not overwritten with
-                # them: sampler.py:216 does that in place, nothing downstream reads them without return_logprob); otherwise bf16
-                # logits are widened inside the softmax launches (exact; no separate pass)
+                # them: sampler.py:216 does that in place, nothing downstream reads them without return_logprob), and so for unfiltered
+                # sampling; otherwise bf16 logits are widened inside the softmax launches (exact; no separate pass)
                 if not simple_sampling_case:
                     ids = kernels.sample_from_logits(logits, sampling_info.temperatures, sampling_info.top_ks, sampling_info.top_ps,
                                                      min_ps, sampling_info.sampling_seed, positions, any_ranges=True)
                     served["one_call_from_logits" if ids is not None else "softmax_then_sample"] += 1
+                else:
+                    ids = kernels.sample_unfiltered_from_logits(logits, sampling_info.temperatures, sampling_info.sampling_seed, positions)
                 if ids is None and logits.dtype == torch.bfloat16:
                     probs = kernels.softmax_temperature_from_bf16(logits, sampling_info.temperatures)
             if ids is None:

@@ -134,3 +134,29 @@ def test_rows_decided_by_their_keys_equal_softmax_then_sample(device, B, V, top_
     got, got_n = K.sample_from_logits(lg, temps, ks, ps, ms, seeds, pos, return_n_keep=True, any_ranges=True)
     bad = ((got == want) & (got_n == want_n)).logical_not().nonzero().flatten().tolist()
     assert not bad, [(r, int(got[r]), int(want[r]), int(got_n[r]), int(want_n[r])) for r in bad]
+
+
+@pytest.mark.parametrize("B,V", [(1, 128256), (12, 32000), (33, 50257), (100, 151936), (128, 40002), (700, 33000), (3, 1025)])
+@pytest.mark.parametrize("fp32", [False, True])
+def test_unfiltered_from_logits_equals_softmax_then_sample(device, B, V, fp32):
+    from sglang_amd import kernels as K
+
+    lg, temps, seeds, pos = _rows(device, B, V, V + B)
+    lg = torch.nn.functional.pad(lg, (0, (-V) % 4))
+    lg = lg.float() if fp32 else lg
+    splits = min(64, 2048 // B, V // 512)
+    probs = torch.empty((B, lg.shape[1]), device=device)
+    ws = torch.empty(B * splits * 2, device=device)
+    from sglang_amd import native
+    if fp32:
+        probs.copy_(lg)
+        native.call("sgl_amd_softmax_temperature_split", probs.data_ptr(), temps.data_ptr(), B, V, probs.stride(0), splits, ws.data_ptr(), K._stream())
+    else:
+        native.call("sgl_amd_softmax_temperature_split_bf16", lg.data_ptr(), probs.data_ptr(), temps.data_ptr(), B, V, lg.stride(0), probs.stride(0), splits,
+                    ws.data_ptr(), K._stream())
+    want = K.top_k_top_p_min_p_sample(probs[:, :V], None, None, None, seeds, pos, filtered=False)
+    before = lg.clone()
+    got = K.sample_unfiltered_from_logits(lg[:, :V], temps, seeds, pos)
+    assert torch.equal(lg.nan_to_num(7.0), before.nan_to_num(7.0))
+    bad = (got != want).nonzero().flatten().tolist()
+    assert not bad, [(r, int(got[r]), int(want[r])) for r in bad]
