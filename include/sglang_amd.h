@@ -543,6 +543,16 @@ int sgl_amd_extend_attention_kv(const void* q, void* out, const void* k_cache, c
                                 int64_t q_token_stride, int64_t out_token_stride, int64_t cache_row_stride, float sm_scale,
                                 int causal, int kv_fp8, float k_scale, float v_scale, int parts, void* ws_acc, void* ws_ml,
                                 void* stream);
+/* sgl_amd_store_kv_cache{,_ex} of the pass's own K / V rows [num_tokens, H_kv, D] (bf16, token strides in elements) to the pool rows new_loc, then
+ * sgl_amd_extend_attention_kv over the pool: one call for both launches. */
+int sgl_amd_extend_attention_store(const void* q, void* out, void* k_cache, void* v_cache, const int32_t* req_to_token,
+                                   int64_t req_to_token_stride, const int64_t* req_pool_indices, const int32_t* seq_lens,
+                                   const int32_t* prefix_lens, const int32_t* qo_indptr, int64_t batch, int64_t num_tokens,
+                                   int max_extend_len, int max_kv_len, int num_q_heads, int num_kv_heads, int head_dim,
+                                   int64_t q_token_stride, int64_t out_token_stride, int64_t cache_row_stride, float sm_scale,
+                                   int causal, int kv_fp8, float k_scale, float v_scale, int parts, void* ws_acc, void* ws_ml,
+                                   const void* k_new, const void* v_new, const int64_t* new_loc, int64_t k_new_stride,
+                                   int64_t v_new_stride, void* stream);
 /* Test / tuning override of the extend kernel's workgroup shape (process-wide; the library never reads the
  * environment): shape 0 = automatic, 41 / 42 / 82 = waves x 16-row tiles per wave (rows per workgroup 64 / 128 / 256);
  * flags bit 0 keeps bf16 8-wave launches on the general single-image kernel, bit 1 sends them to the ping-pong

@@ -1668,6 +1668,23 @@ int sgl_amd_extend_attention_kv(const void* q, void* out, const void* k_cache, c
                               nullptr, nullptr, 0, num_tokens, max_kv_len, parts, ws_acc, ws_ml, stream);
 }
 
+int sgl_amd_extend_attention_store(const void* q, void* out, void* k_cache, void* v_cache, const int32_t* req_to_token, int64_t req_to_token_stride,
+                                   const int64_t* req_pool_indices, const int32_t* seq_lens, const int32_t* prefix_lens, const int32_t* qo_indptr,
+                                   int64_t batch, int64_t num_tokens, int max_extend_len, int max_kv_len, int num_q_heads, int num_kv_heads,
+                                   int head_dim, int64_t q_token_stride, int64_t out_token_stride, int64_t cache_row_stride, float sm_scale, int causal,
+                                   int kv_fp8, float k_scale, float v_scale, int parts, void* ws_acc, void* ws_ml, const void* k_new,
+                                   const void* v_new, const int64_t* new_loc, int64_t k_new_stride, int64_t v_new_stride, void* stream) {
+  const int row = num_kv_heads * head_dim;
+  const int rc = kv_fp8 ? sgl_amd_store_kv_cache_ex(k_new, v_new, k_cache, v_cache, new_loc, num_tokens, num_kv_heads, head_dim, k_new_stride,
+                                                    v_new_stride, cache_row_stride, 1, k_scale, v_scale, 1, 0, stream)
+                        : sgl_amd_store_kv_cache(k_new, v_new, k_cache, v_cache, new_loc, num_tokens, row, row, k_new_stride, v_new_stride,
+                                                 cache_row_stride, cache_row_stride, stream);
+  if (rc != 0) return rc;
+  return sgl_amd_extend_attention_kv(q, out, k_cache, v_cache, req_to_token, req_to_token_stride, req_pool_indices, seq_lens, prefix_lens, qo_indptr,
+                                     batch, num_tokens, max_extend_len, max_kv_len, num_q_heads, num_kv_heads, head_dim, q_token_stride,
+                                     out_token_stride, cache_row_stride, sm_scale, causal, kv_fp8, k_scale, v_scale, parts, ws_acc, ws_ml, stream);
+}
+
 #ifdef EXT_TRACE
 int sgl_amd_debug_ext_trace(void* buf) {
   uint64_t* p = static_cast<uint64_t*>(buf);
