@@ -1194,7 +1194,7 @@ def _moe_tiles_us(rows_per_expert: float, num_experts: int, n_up: int, n_down: i
 
 def moe_tile_plan(numel: int, num_experts: int, n_up: int, n_down: int):
     """(align block, tile rows of the up projection, tile rows of the down projection) for a prefill-sized batch of
-    `numel` (token, k) pairs: the 256 x 256 x 64 form once an expert owns enough rows that the 256-row alignment's padding
+    `numel` (token, k) pairs, where whole tiles decide (moe_tiles): the 256 x 256 x 64 form once an expert owns enough rows that the 256-row alignment's padding
     (128 rows per expert on average) costs less than the form gains (measured on Mixtral's shapes, 4096 tokens = 1024 rows
     per expert: up projection 977 vs 714 TF/s, down projection 820-870 vs 715 with its 2.25 rounds of workgroups;
     profiles/r04_exp4_moe_gemm_ab.json).  Experts of 256 to 767 rows take it where rounds and padding together promise 9.5 % or more (a K step of
@@ -1210,6 +1210,24 @@ def moe_tile_plan(numel: int, num_experts: int, n_up: int, n_down: int):
     if rows >= 256 and _moe_tiles_us(*sizes, 256, 256, 1.84) < 0.905 * _moe_tiles_us(*sizes, 128, 512, 1.2):
         return 256, 256, 256
     return 128, 128, 128
+
+
+MOE_HALF_TILE_MIN_ROWS, MOE_HALF_TILE_MIN_WORKGROUPS = 240, 5 * 256
+
+
+def moe_tiles(numel: int, num_experts: int, n_up: int, n_down: int):
+    """moe_tile_plan, and the 256-row form also where only its half tiles pay: an expert's last tile with 128 rows or fewer takes two thirds of a whole
+    one, so that experts of 240 rows and more gain once the up projection fills five rounds of workgroups.  Both products in us, 128 / 256 rows, for
+    three routings each: 8 experts of 14336 / 4096 with 250 rows 1191 / 1116, 1206 / 1091, 1147 / 1131, with 400 1639 / 1282, 1624 / 1275, 1617 / 1294,
+    with 440 1730 / 1741, 1799 / 1753, 1795 / 1707, with 520 2178 / 1895, 2088 / 1885, 2007 / 1736; 32 of 7168 / 4096 with 260 2292 / 2239, 2234 / 2031,
+    2264 / 2043; 64 of 1408 / 2048 with 350 757 / 672, 759 / 676, 765 / 673.  Below the lines: 64 of 4096 / 2048 with 200 rows 1175 / 1212, 8 of 7168 /
+    4096 (four rounds) with 400 786 / 700, 794 / 903, 784 / 692, 16 of 2048 / 2048 (two) with 500 325 / 353."""
+    plan = moe_tile_plan(numel, num_experts, n_up, n_down)
+    rows = numel / max(1, num_experts)
+    workgroups = num_experts * (rows / 256 + 0.5) * -(-n_up // 128)
+    if plan[0] == 128 and rows >= MOE_HALF_TILE_MIN_ROWS and workgroups >= MOE_HALF_TILE_MIN_WORKGROUPS:
+        return 256, 256, 256
+    return plan
 
 
 def moe_grouped_gemm(a: torch.Tensor, w: torch.Tensor, c: torch.Tensor, sorted_token_ids: torch.Tensor,
@@ -1327,7 +1345,7 @@ def fused_experts(hidden_states: torch.Tensor, w13: torch.Tensor, w2: torch.Tens
         return out
     if numel // E >= MOE_TILED_MIN_ROWS_PER_EXPERT and K % 64 == 0 and N % 64 == 0:
         # prefill-sized batch: row-tiled MFMA kernels, every expert's weights read once per 128 / 256 of its rows
-        block_m, up_rows, down_rows = moe_tile_plan(numel, E, N, K) if K % 64 == 0 else (128, 128, 128)
+        block_m, up_rows, down_rows = moe_tiles(numel, E, N, K)
         if MOE_TILE_OVERRIDE is not None:
             block_m, up_rows, down_rows = MOE_TILE_OVERRIDE
         sorted_ids, expert_ids, post = moe_align_block_size(topk_ids, block_m, E)

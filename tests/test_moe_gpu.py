@@ -312,3 +312,24 @@ def test_tiled_grouped_gemm_row_gather_and_scale(device):
                 * tw.flatten()[:, None])
         d = (c.cpu().float() - want).abs()
         assert bool((d <= want.abs() * 2.0 ** -7 + 1e-3).all()), float(d.max())
+
+
+@pytest.mark.parametrize("loads", [(128, 129, 1, 127), (256, 257, 384, 385), (0, 300, 512, 64), (640, 0, 0, 641)])
+@pytest.mark.parametrize("fuse_silu", [True, False])
+def test_256_row_tiles_whose_second_half_is_empty(device, loads, fuse_silu):
+    """An expert's last 256-row tile leaves out its second half where that has no rows: loads on both sides of the halves, an expert with none.
+    Rows are compared with the 128-row form's (the same products summed in the same order)."""
+    K = _k()
+    g = torch.Generator().manual_seed(sum(loads) + loads[0])
+    M, E, N, Kd = sum(loads), len(loads), 320, 384
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(loads))[torch.randperm(M, generator=g)].to(torch.int32).view(M, 1).to(device)
+    a = torch.randn((M, Kd), generator=g).to(BF).to(device)
+    w = (torch.randn((E, N * (2 if fuse_silu else 1), Kd), generator=g) * 0.05).to(BF).to(device)
+    outs = []
+    for rows in (128, 256):
+        s, e, post = K.moe_align_block_size(ids, 256, E)
+        c = torch.full((M, N), float("nan"), dtype=BF, device=device)
+        K.moe_tiled_gemm(a, w, c, s, e, post, None, False, 1, M, 256, fuse_silu=fuse_silu, tile_rows=rows)
+        outs.append(c)
+    assert bool(torch.isfinite(outs[1].float()).all())
+    assert torch.equal(outs[0], outs[1])

@@ -9,3 +9,11 @@ def test_experts_of_middling_size():
                                            (2 * 1622, 8, 14336, 4096, 128), (2 * 2048, 8, 14336, 4096, 128),
                                            (2 * 1020, 8, 14336, 4096, 128)):
         assert K.moe_tile_plan(pairs, experts, up, down) == (rows,) * 3, (pairs, experts, up, down)
+
+
+def test_experts_that_half_tiles_pay_for():
+    for pairs, experts, up, down, rows in ((2 * 1000, 8, 14336, 4096, 256), (2 * 1622, 8, 14336, 4096, 256), (2 * 2048, 8, 14336, 4096, 256),
+                                           (2 * 3000, 8, 14336, 4096, 256), (32 * 260, 32, 7168, 4096, 256), (64 * 350, 64, 1408, 2048, 256),
+                                           (2 * 950, 8, 14336, 4096, 128), (2 * 1600, 8, 7168, 4096, 128), (16 * 500, 16, 2048, 2048, 128),
+                                           (64 * 200, 64, 4096, 2048, 128)):
+        assert K.moe_tiles(pairs, experts, up, down) == (rows,) * 3, (pairs, experts, up, down)
