@@ -1178,7 +1178,18 @@ def moe_tiled_gemm(a: torch.Tensor, w: torch.Tensor, c: torch.Tensor, sorted_tok
 
 
 MOE_TILE_OVERRIDE = None                # tests / benchmarks: (align block, up tile rows, down tile rows)
-MOE_TILED_MIN_ROWS_PER_EXPERT = 96     # above this an expert fills most of a 128-row tile: the MFMA-bound form wins
+# From here on the row-tiled form: the weight-streaming one takes 64 rows at a time, and an expert with more reads its weights again.  us, both products,
+# streaming / 128-row tiles, two routings each: 8 experts of 14336 / 4096 with 48 rows 613 / 592, 600 / 575, with 60 710 / 595, 699 / 578, with 90 922 / 620,
+# 911 / 599; of 7168 / 4096 with 48 281 / 316, 271 / 309, with 70 400 / 326, 394 / 320; 64 of 1408 / 2048 with 48 287 / 282, 301 / 283, with 70 372 / 301.
+# Only from 96 rows on where the up projection has fewer than 256 such tiles: 4 experts of 1024 / 1024 with 58 to 76 rows 41 / 45.
+MOE_TILED_MIN_ROWS_PER_EXPERT, MOE_TILED_MIN_ROWS_FEW_TILES = 56, 96
+
+
+def _row_tiled(numel: int, num_experts: int, n_up: int) -> bool:
+    rows = numel // num_experts
+    return rows >= MOE_TILED_MIN_ROWS_PER_EXPERT and (num_experts * n_up >= 256 * 64 or rows >= MOE_TILED_MIN_ROWS_FEW_TILES)
+
+
 MOE_TILE256_MIN_ROWS_PER_EXPERT = 768  # above this the 256-row alignment's padding (128 rows per expert on average) is
                                        # worth the 256 x 256 x 64 form's rate
 
@@ -1343,7 +1354,7 @@ def fused_experts(hidden_states: torch.Tensor, w13: torch.Tensor, w2: torch.Tens
         out = torch.empty((M, K), dtype=_BF16, device=dev)
     if M == 0:
         return out
-    if numel // E >= MOE_TILED_MIN_ROWS_PER_EXPERT and K % 64 == 0 and N % 64 == 0:
+    if _row_tiled(numel, E, N) and K % 64 == 0 and N % 64 == 0:
         # prefill-sized batch: row-tiled MFMA kernels, every expert's weights read once per 128 / 256 of its rows
         block_m, up_rows, down_rows = moe_tiles(numel, E, N, K)
         if MOE_TILE_OVERRIDE is not None:
@@ -2099,7 +2110,7 @@ def routed_experts(h: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, ids: to
         return _experts_plain(_experts_plain(h, w13, ids, True, act), w2, ids, False).view(T, top, W)
     inter = torch.empty((numel, N), dtype=_BF16, device=h.device)
     down = torch.empty((numel, W), dtype=_BF16, device=h.device)
-    if numel // E >= MOE_TILED_MIN_ROWS_PER_EXPERT and W % 64 == 0 and N % 64 == 0:
+    if _row_tiled(numel, E, N) and W % 64 == 0 and N % 64 == 0:
         block_m, up_rows, down_rows = moe_tile_plan(numel, E, N, W) if MOE_TILE_OVERRIDE is None else MOE_TILE_OVERRIDE
         s = moe_align_block_size(ids, block_m, E)
         moe_tiled_gemm(h, w13, inter, *s, None, False, top, numel, block_m, fuse_silu=act.gated, tile_rows=up_rows, act=act)

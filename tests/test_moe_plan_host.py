@@ -17,3 +17,9 @@ def test_experts_that_half_tiles_pay_for():
                                            (2 * 950, 8, 14336, 4096, 128), (2 * 1600, 8, 7168, 4096, 128), (16 * 500, 16, 2048, 2048, 128),
                                            (64 * 200, 64, 4096, 2048, 128)):
         assert K.moe_tiles(pairs, experts, up, down) == (rows,) * 3, (pairs, experts, up, down)
+
+
+def test_where_the_row_tiles_begin():
+    for pairs, experts, up, tiled in ((8 * 56, 8, 14336, True), (8 * 55, 8, 14336, False), (4 * 95, 4, 1024, False), (4 * 96, 4, 1024, True),
+                                      (8 * 56, 8, 2048, True), (8 * 1000, 8, 64, True)):
+        assert K._row_tiled(pairs, experts, up) == tiled, (pairs, experts, up)
