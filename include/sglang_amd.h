@@ -544,7 +544,10 @@ int sgl_amd_extend_attention_kv(const void* q, void* out, const void* k_cache, c
                                 int causal, int kv_fp8, float k_scale, float v_scale, int parts, void* ws_acc, void* ws_ml,
                                 void* stream);
 /* sgl_amd_store_kv_cache{,_ex} of the pass's own K / V rows [num_tokens, H_kv, D] (bf16, token strides in elements) to the pool rows new_loc, then
- * sgl_amd_extend_attention_kv over the pool: one call for both launches. */
+ * sgl_amd_extend_attention_kv over the pool: one call for both launches.  sgl_amd_extend_attention_store_parts says how many parts pay here
+ * (sum_kv_len: the sum of the contexts, 0 if the caller does not know it); 0: workgroups that stay and take their query tiles, the longest contexts
+ * first, from eight counters, ws_ml (32 bytes of the caller's, zeroed by the call; ws_acc unused). */
+int sgl_amd_extend_attention_store_parts(int64_t batch, int64_t num_tokens, int64_t sum_kv_len, int max_extend_len, int max_kv_len, int num_q_heads, int num_kv_heads, int head_dim);
 int sgl_amd_extend_attention_store(const void* q, void* out, void* k_cache, void* v_cache, const int32_t* req_to_token,
                                    int64_t req_to_token_stride, const int64_t* req_pool_indices, const int32_t* seq_lens,
                                    const int32_t* prefix_lens, const int32_t* qo_indptr, int64_t batch, int64_t num_tokens,

@@ -294,13 +294,15 @@ __global__ void rope_kernel(const int64_t* __restrict__ positions, uint16_t* __r
 // ---------------------------------------------------------------------------
 // KV-row scatter: k_cache[loc[t], :] = k[t, :], same for v.  16 B per lane.
 // ---------------------------------------------------------------------------
+template <bool ZERO>
 __global__ void store_kv_kernel(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
                                 uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache,
                                 const int64_t* __restrict__ loc, int row_elems, int v_row_elems,
                                 int64_t k_stride, int64_t v_stride, int64_t kc_stride,
-                                int64_t vc_stride) {
+                                int64_t vc_stride, unsigned* zero8) {
   const int64_t tok = blockIdx.x;
   const int64_t slot = loc[tok];
+  if (ZERO && tok == 0 && threadIdx.x < 8) zero8[threadIdx.x] = 0u;      // counters of the launch behind this one
   const uint16_t* ks = k + tok * k_stride;
   const uint16_t* vs = v + tok * v_stride;
   uint16_t* kd = k_cache + slot * kc_stride;
@@ -311,12 +313,13 @@ __global__ void store_kv_kernel(const uint16_t* __restrict__ k, const uint16_t* 
 
 // The same scatter for any pool layout / element format: one workgroup per token, a thread per 8 elements of the
 // token's [H_kv, D] row; fp8 rows hold x / scale rounded to OCP e4m3 (memory_pool.py:2364-2374).
-template <bool FP8>
+template <bool FP8, bool ZERO>
 __global__ void store_kv_fmt_kernel(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
                                     void* __restrict__ k_cache, void* __restrict__ v_cache,
                                     const int64_t* __restrict__ loc, int num_kv_heads, int head_dim,
-                                    int64_t k_stride, int64_t v_stride, KvFormat fmt, float inv_k_scale, float inv_v_scale) {
+                                    int64_t k_stride, int64_t v_stride, KvFormat fmt, float inv_k_scale, float inv_v_scale, unsigned* zero8) {
   const int64_t tok = blockIdx.x;
+  if (ZERO && tok == 0 && threadIdx.x < 8) zero8[threadIdx.x] = 0u;
   const int slot = static_cast<int>(loc[tok]);
   const int per_head = head_dim >> 3;
   for (int e = threadIdx.x; e < num_kv_heads * per_head; e += blockDim.x) {
@@ -491,10 +494,10 @@ int sgl_amd_rotary_embedding(const int64_t* positions, void* q, void* k, const v
   return 0;
 }
 
-int sgl_amd_store_kv_cache(const void* k, const void* v, void* k_cache, void* v_cache,
-                           const int64_t* loc, int64_t num_tokens, int k_row_elems,
-                           int v_row_elems, int64_t k_token_stride, int64_t v_token_stride,
-                           int64_t k_cache_row_stride, int64_t v_cache_row_stride, void* stream) {
+static int store_kv_plain(const void* k, const void* v, void* k_cache, void* v_cache,
+                          const int64_t* loc, int64_t num_tokens, int k_row_elems,
+                          int v_row_elems, int64_t k_token_stride, int64_t v_token_stride,
+                          int64_t k_cache_row_stride, int64_t v_cache_row_stride, unsigned* zero8, void* stream) {
   SGL_CLEAR_STALE_ERROR();
   SGL_CHECK_ARG(k_row_elems % 8 == 0 && v_row_elems % 8 == 0, "store_kv_cache: row sizes must be multiples of 8 elements (16 B)");
   SGL_CHECK_ARG(k_token_stride % 8 == 0 && v_token_stride % 8 == 0 && k_cache_row_stride % 8 == 0 && v_cache_row_stride % 8 == 0,
@@ -505,19 +508,19 @@ int sgl_amd_store_kv_cache(const void* k, const void* v, void* k_cache, void* v_
   int threads = ((maxrow / 8 + 63) / 64) * 64;
   if (threads > 256) threads = 256;
   if (threads < 64) threads = 64;
-  hipLaunchKernelGGL(store_kv_kernel, dim3(num_tokens), dim3(threads), 0, as_stream(stream),
+  hipLaunchKernelGGL(zero8 ? store_kv_kernel<true> : store_kv_kernel<false>, dim3(num_tokens), dim3(threads), 0, as_stream(stream),
                      static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v),
                      static_cast<uint16_t*>(k_cache), static_cast<uint16_t*>(v_cache), loc,
                      k_row_elems, v_row_elems, k_token_stride, v_token_stride, k_cache_row_stride,
-                     v_cache_row_stride);
+                     v_cache_row_stride, zero8);
   SGL_CHECK_LAUNCH("store_kv_cache");
   return 0;
 }
 
-int sgl_amd_store_kv_cache_ex(const void* k, const void* v, void* k_cache, void* v_cache, const int64_t* loc,
-                              int64_t num_tokens, int num_kv_heads, int head_dim, int64_t k_token_stride,
-                              int64_t v_token_stride, int64_t cache_row_stride, int kv_fp8, float k_scale, float v_scale,
-                              int page_size, int kv_layout_hnd, void* stream) {
+static int store_kv_any(const void* k, const void* v, void* k_cache, void* v_cache, const int64_t* loc,
+                        int64_t num_tokens, int num_kv_heads, int head_dim, int64_t k_token_stride,
+                        int64_t v_token_stride, int64_t cache_row_stride, int kv_fp8, float k_scale, float v_scale,
+                        int page_size, int kv_layout_hnd, unsigned* zero8, void* stream) {
   SGL_CLEAR_STALE_ERROR();
   SGL_CHECK_ARG(head_dim % 8 == 0 && num_kv_heads > 0, "store_kv_cache: head_dim must be a multiple of 8");
   SGL_CHECK_ARG(k_token_stride % 8 == 0 && v_token_stride % 8 == 0 && cache_row_stride % 8 == 0,
@@ -530,15 +533,42 @@ int sgl_amd_store_kv_cache_ex(const void* k, const void* v, void* k_cache, void*
   int threads = ((num_kv_heads * head_dim / 8 + 63) / 64) * 64;
   if (threads > 256) threads = 256;
   if (kv_fp8)
-    hipLaunchKernelGGL(store_kv_fmt_kernel<true>, dim3(num_tokens), dim3(threads), 0, as_stream(stream),
+    hipLaunchKernelGGL((zero8 ? store_kv_fmt_kernel<true, true> : store_kv_fmt_kernel<true, false>), dim3(num_tokens), dim3(threads), 0, as_stream(stream),
                        static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v), k_cache, v_cache, loc, num_kv_heads,
-                       head_dim, k_token_stride, v_token_stride, fmt, 1.0f / k_scale, 1.0f / v_scale);
+                       head_dim, k_token_stride, v_token_stride, fmt, 1.0f / k_scale, 1.0f / v_scale, zero8);
   else
-    hipLaunchKernelGGL(store_kv_fmt_kernel<false>, dim3(num_tokens), dim3(threads), 0, as_stream(stream),
+    hipLaunchKernelGGL((store_kv_fmt_kernel<false, false>), dim3(num_tokens), dim3(threads), 0, as_stream(stream),
                        static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v), k_cache, v_cache, loc, num_kv_heads,
-                       head_dim, k_token_stride, v_token_stride, fmt, 1.0f, 1.0f);
+                       head_dim, k_token_stride, v_token_stride, fmt, 1.0f, 1.0f, zero8);
   SGL_CHECK_LAUNCH("store_kv_cache_ex");
   return 0;
 }
 
+int sgl_amd_store_kv_cache(const void* k, const void* v, void* k_cache, void* v_cache,
+                           const int64_t* loc, int64_t num_tokens, int k_row_elems,
+                           int v_row_elems, int64_t k_token_stride, int64_t v_token_stride,
+                           int64_t k_cache_row_stride, int64_t v_cache_row_stride, void* stream) {
+  return store_kv_plain(k, v, k_cache, v_cache, loc, num_tokens, k_row_elems, v_row_elems, k_token_stride, v_token_stride, k_cache_row_stride,
+                        v_cache_row_stride, nullptr, stream);
+}
+
+int sgl_amd_store_kv_cache_ex(const void* k, const void* v, void* k_cache, void* v_cache, const int64_t* loc,
+                              int64_t num_tokens, int num_kv_heads, int head_dim, int64_t k_token_stride,
+                              int64_t v_token_stride, int64_t cache_row_stride, int kv_fp8, float k_scale, float v_scale,
+                              int page_size, int kv_layout_hnd, void* stream) {
+  return store_kv_any(k, v, k_cache, v_cache, loc, num_tokens, num_kv_heads, head_dim, k_token_stride, v_token_stride, cache_row_stride, kv_fp8,
+                      k_scale, v_scale, page_size, kv_layout_hnd, nullptr, stream);
+}
+
 }  // extern "C"
+
+// The same for a token-major pool, in front of a launch that needs eight zeroed counters (null: none).
+int sgl_amd::store_kv_rows(const void* k, const void* v, void* k_cache, void* v_cache, const int64_t* loc, int64_t num_tokens, int num_kv_heads, int head_dim,
+                           int64_t k_token_stride, int64_t v_token_stride, int64_t cache_row_stride, int kv_fp8, float k_scale, float v_scale,
+                           unsigned* zero8, void* stream) {
+  const int row = num_kv_heads * head_dim;
+  return kv_fp8 ? store_kv_any(k, v, k_cache, v_cache, loc, num_tokens, num_kv_heads, head_dim, k_token_stride, v_token_stride, cache_row_stride, 1, k_scale,
+                               v_scale, 1, 0, zero8, stream)
+                : store_kv_plain(k, v, k_cache, v_cache, loc, num_tokens, row, row, k_token_stride, v_token_stride, cache_row_stride, cache_row_stride,
+                                 zero8, stream);
+}

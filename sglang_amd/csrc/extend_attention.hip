@@ -75,6 +75,7 @@ struct ExtendParams {
   int64_t part_rows;            // num_tokens * Hq
   float* part_acc;
   float* part_ml;
+  unsigned* grabbed;            // extend_attention_walk_kernel: tiles taken so far, per XCD
 };
 
 template <int D>
@@ -879,6 +880,105 @@ __device__ __forceinline__ float lane_pair_max(float x) {         // max over la
   return fmaxf(a, b);
 }
 
+__device__ __forceinline__ float lane_pair_sum(float x) {         // the sum of the same two
+  float a = x, b = x;
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+  return a + b;
+}
+
+// The query tiles of a launch as workgroups that stay take them (extend_attention_walk_kernel): one list per XCD (tile L goes to list L mod 8, as
+// launched workgroups would), longest contexts first.  A request's tiles stand at consecutive levels, tile t behind a prefix of whole tiles at
+// level prefix / tokens + t; a level lists its requests' kv heads, so that neighbours in the list read the same heads' rows on the same XCD.
+struct WalkQueue {
+  static constexpr int kRequests = 512, kThreads = 512, kLevels = 4096;
+  int next;                                         // the tile taken next, for all waves
+  int sums[kThreads / 64];
+  int32_t ids[4 * kKvTile];                         // slots of its first four key tiles
+  int first[kRequests], tiles[kRequests];           // levels [first, first + tiles)
+  int q_begin[kRequests], len[kRequests], kv_len[kRequests], prefix[kRequests], row[kRequests];
+  int below[kLevels];                               // tiles in front of the i-th level from the top
+
+  // every thread of the workgroup; returns the top level
+  __device__ __forceinline__ int fill(const ExtendParams& p, int tid) {
+    const int lane = tid & 63, wid = tid >> 6;
+    int f = 0, n = 0;
+    if (tid < p.batch) {
+      const int at = p.qo_indptr[tid], l = p.qo_indptr[tid + 1] - at, pre = p.prefix_lens[tid];
+      n = l > 0 ? min((l + p.tokens_per_tile - 1) / p.tokens_per_tile, kLevels) : 0;
+      f = min(pre / p.tokens_per_tile, kLevels - n);  // (longer contexts stand at the top together)
+      q_begin[tid] = at;
+      len[tid] = l;
+      kv_len[tid] = p.seq_lens[tid];
+      prefix[tid] = pre;
+      row[tid] = static_cast<int>(p.req_pool_indices[tid]);
+    }
+    first[tid] = f;
+    tiles[tid] = n;
+    int top = n > 0 ? f + n - 1 : -1;
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) top = max(top, __shfl_xor(top, d, 64));
+    if (lane == 0) sums[wid] = top;
+    __syncthreads();
+    top = -1;
+#pragma unroll
+    for (int w = 0; w < kThreads / 64; ++w) top = max(top, sums[w]);
+    top = __builtin_amdgcn_readfirstlane(top);
+    __syncthreads();
+    const int per = (top + kThreads) / kThreads;    // levels of a thread: per tid .. from the top, 1 up to 32 k tokens in tiles of 64
+    int mine = 0;
+    for (int i = 0; i < per; ++i) {
+      const int level = top - (per * tid + i);
+      int c = 0;
+      if (level >= 0)
+        for (int r = 0; r < p.batch; ++r) c += level >= first[r] && level - first[r] < tiles[r] ? p.num_kv_heads : 0;
+      if (per * tid + i < kLevels) below[per * tid + i] = mine;
+      mine += c;
+    }
+    int upto = mine;                                // of the wave's threads so far
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int o = __shfl_up(upto, d, 64);
+      if (lane >= d) upto += o;
+    }
+    if (lane == 63) sums[wid] = upto;
+    __syncthreads();
+    int front = upto - mine;
+    for (int w = 0; w < wid; ++w) front += sums[w];
+    for (int i = 0; i < per; ++i)
+      if (per * tid + i < kLevels) below[per * tid + i] += front;
+    if (tid == kThreads - 1) next = front + mine;   // all tiles
+    __syncthreads();
+    return top;
+  }
+
+  // request, kv head and query tile of tile L of the list (one that exists)
+  __device__ __forceinline__ void find(int L, int top, int batch, int heads, int lane, int& b, int& kvh, int& tile) const {
+    int at = 0;                                     // the last level with below[] <= L: 64 of them at a time, then one of 64
+    for (int c = 64; c <= top; c += 64 * 64) {
+      const int i = c + 64 * lane;
+      at += 64 * __popcll(__ballot(i <= top && below[i <= top ? i : 0] <= L));
+    }
+    const int i = at + lane;
+    at += __popcll(__ballot(i <= top && below[i <= top ? i : 0] <= L)) - 1;
+    const int level = top - at, rest = L - __builtin_amdgcn_readfirstlane(below[at]);
+    int nth = rest / heads;
+    kvh = rest - nth * heads;
+    b = 0;
+    for (int c = 0; c < batch; c += 64) {
+      const bool in = level >= first[c + lane] && level - first[c + lane] < tiles[c + lane];
+      const unsigned long long m = __ballot(in);
+      const int n = __popcll(m);
+      if (nth < n) {
+        const int rank = __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(m >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(m), 0u));
+        b = c + __ffsll(__ballot(in && rank == nth)) - 1;
+        break;
+      }
+      nth -= n;
+    }
+    tile = level - __builtin_amdgcn_readfirstlane(first[b]);
+  }
+};
+
 // A step of the walk is two phases of products with the vector work of the NEIGHBOURING tiles spread between them:
 //     phase 1:  S^T(t + 1) = K(t + 1) . Q^T   ||  P(t) = exp2(S(t) scale - m)  and the row requests of the tiles ahead
 //     phase 2:  O^T += V^T(t) . P^T(t)        ||  mask + row maxima of S(t + 1)
@@ -889,8 +989,9 @@ __device__ __forceinline__ float lane_pair_max(float x) {         // max over la
 // FP8: the pool holds e4m3 rows (8 bytes per lane and chunk, held raw in the staging registers, widened to bf16 -- exact --
 // on their way into the LDS images; k_scale rides in the softmax scale, v_scale in the epilogue).
 // PARTS: the walk covers part `part` of p.parts equal pieces of the request's key tiles (extend_attention_parts_kernel below).
-template <int D, int NWV, bool FP8, bool PARTS>
-__device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadder<D>& sm) {
+// STAYS: the workgroup takes query tiles from the queue until there are none (extend_attention_walk_kernel below).
+template <int D, int NWV, bool FP8, bool PARTS, bool STAYS = false>
+__device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadder<D>& sm, WalkQueue* queue = nullptr) {
   constexpr int CPR = D / 8;            // 16-byte chunks per KV row
   constexpr int KS = D / 16;            // MFMA k-steps over the head dim
   constexpr int ND = D / 32;            // 32-wide output blocks over the head dim
@@ -899,48 +1000,105 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
   constexpr int VSUB = SmemLadder<D>::kVSub;
   constexpr int NPV = ND * 4;           // PV products per tile
 
+  // (STAYS: formed anew for each query tile, as is what only the passage from tile to tile needs: kept across the outer loop, all the addresses
+  // made of them would take registers from the walk)
+  auto thread = [&]() __attribute__((always_inline)) {
+    int x = threadIdx.x;
+    if constexpr (STAYS) asm volatile("" : "+v"(x));
+    return x;
+  };
+  int tid, lane, wid, l31, hi;
+  auto lanes = [&]() __attribute__((always_inline)) {
+    tid = thread();
+    lane = tid & 63;
+    wid = tid >> 6;
+    l31 = lane & 31;
+    hi = lane >> 5;
+  };
+  lanes();
   // grid -> (query tile, kv head, request): as in the ping-pong kernel (heaviest tiles first, a pair stays on one XCD)
   // (with PARTS a pair is a (request, kv head, part): the query tiles that read the same keys)
   int tile, kvh, b, part = 0;
-  {
-    const int L = blockIdx.x;
-    const int pairs = p.batch * p.num_kv_heads * (PARTS ? p.parts : 1);
-    int pair, rank;
-    if (pairs % 8 == 0) {
-      const int per_xcd = pairs / 8;
-      const int j = L >> 3;
-      pair = (j % per_xcd) * 8 + (L & 7);
-      rank = j / per_xcd;
-    } else {
-      pair = L % pairs;
-      rank = L / pairs;
+  int q_begin, ext_len, kv_len, prefix;
+  const int32_t* idx_base;
+  int top = 0, all = 0;                                // of the queue: its top level, its tiles
+  auto of_queue = [&](int r, int t) __attribute__((always_inline)) {       // request r's figures
+    q_begin = __builtin_amdgcn_readfirstlane(queue->q_begin[r]);
+    ext_len = __builtin_amdgcn_readfirstlane(queue->len[r]);
+    kv_len = __builtin_amdgcn_readfirstlane(queue->kv_len[r]);
+    prefix = __builtin_amdgcn_readfirstlane(queue->prefix[r]);
+    idx_base = p.req_to_token + __builtin_amdgcn_readfirstlane(queue->row[r]) * p.r2t_stride;
+    tile = t;
+  };
+  if constexpr (STAYS) {
+    static_assert(64 * NWV == WalkQueue::kThreads && WalkQueue::kRequests == WalkQueue::kThreads, "one request a thread");
+    top = queue->fill(p, tid);
+    all = __builtin_amdgcn_readfirstlane(queue->next);
+    if (static_cast<int>(blockIdx.x) >= all) return;
+    queue->find(blockIdx.x, top, p.batch, p.num_kv_heads, lane, b, kvh, tile);
+    of_queue(b, tile);
+  } else {
+    {
+      // (the arguments in one round trip, not piece by piece in front of their first uses)
+      asm volatile("" ::"s"(p.q), "s"(p.k_cache), "s"(p.v_cache), "s"(p.req_to_token), "s"(p.req_pool_indices), "s"(p.seq_lens), "s"(p.prefix_lens), "s"(p.qo_indptr),
+                   "s"(p.q_stride), "s"(p.r2t_stride), "s"(p.fmt.page_stride), "s"(p.fmt.head_stride), "s"(p.scale_log2), "s"(p.group), "s"(p.causal),
+                   "s"(p.parts), "s"(p.part_rows), "s"(p.part_ml));
+      const int L = blockIdx.x;
+      const int pairs = p.batch * p.num_kv_heads * (PARTS ? p.parts : 1);
+      int pair, rank;
+      if (pairs % 8 == 0) {
+        const int per_xcd = pairs / 8;
+        const int j = L >> 3;
+        pair = (j % per_xcd) * 8 + (L & 7);
+        rank = j / per_xcd;
+      } else {
+        pair = L % pairs;
+        rank = L / pairs;
+      }
+      tile = p.num_tiles - 1 - rank;
+      if constexpr (PARTS) {
+        part = pair % p.parts;
+        pair /= p.parts;
+      }
+      kvh = pair % p.num_kv_heads;
+      b = pair / p.num_kv_heads;
     }
-    tile = p.num_tiles - 1 - rank;
-    if constexpr (PARTS) {
-      part = pair % p.parts;
-      pair /= p.parts;
-    }
-    kvh = pair % p.num_kv_heads;
-    b = pair / p.num_kv_heads;
+    q_begin = p.qo_indptr[b];
+    ext_len = p.qo_indptr[b + 1] - q_begin;
+    kv_len = p.seq_lens[b];
+    prefix = p.prefix_lens[b];
+    const int64_t row = p.req_pool_indices[b];
+    // (one round trip for all five: left to itself the compiler sinks the last three below the branch)
+    asm volatile("" ::"s"(ext_len), "s"(kv_len), "s"(prefix), "s"(row));
+    idx_base = p.req_to_token + row * p.r2t_stride;
+    if (tile * p.tokens_per_tile >= ext_len) return;
   }
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wid = tid >> 6;
-  const int l31 = lane & 31;
-  const int hi = lane >> 5;
 
-  const int q_begin = p.qo_indptr[b];
-  const int ext_len = p.qo_indptr[b + 1] - q_begin;
-  const int kv_len = p.seq_lens[b];
-  const int prefix = p.prefix_lens[b];
-  const int32_t* idx_base = p.req_to_token + p.req_pool_indices[b] * p.r2t_stride;
-  const int q0 = tile * p.tokens_per_tile;
-  if (q0 >= ext_len) return;
-  int q1 = q0 + p.tokens_per_tile;
-  if (q1 > ext_len) q1 = ext_len;
+  // ---- the query tile: its tokens, its keys, this lane's row (both lane halves of a row hold the same query, other head dims / keys) ----
   const bool causal = p.causal != 0;
-  int kv_end = causal ? (prefix + q1 < kv_len ? prefix + q1 : kv_len) : kv_len;
-  int n_tiles = (kv_end + kKvTile - 1) / kKvTile;
+  int r_tok, r_hg;
+  auto row_of = [&](int x) __attribute__((always_inline)) {
+    const int r_row = (x >> 6) * 32 + (x & 31);
+    int group = p.group;
+    if constexpr (STAYS || PARTS) asm volatile("" : "+s"(group));
+    r_tok = r_row / group;
+    r_hg = r_row - r_tok * group;
+  };
+  int q0, q1, kv_end, n_tiles, row_limit, row_off;
+  bool row_ok;
+  auto place = [&]() __attribute__((always_inline)) {
+    row_of(thread());
+    q0 = tile * p.tokens_per_tile;
+    q1 = q0 + p.tokens_per_tile;
+    if (q1 > ext_len) q1 = ext_len;
+    kv_end = causal ? (prefix + q1 < kv_len ? prefix + q1 : kv_len) : kv_len;
+    n_tiles = (kv_end + kKvTile - 1) / kKvTile;
+    row_ok = (r_tok < p.tokens_per_tile) && (q0 + r_tok < q1);
+    row_limit = row_ok ? (causal ? prefix + q0 + r_tok + 1 : kv_len) : 0;
+    if (row_limit > kv_len) row_limit = kv_len;
+    row_off = (kvh * p.group + r_hg) * D;
+  };
+  place();
   // this part's tiles become tiles 0 .. n_tiles - 1 of the walk: the row of the request table, the end and the rows' limits move
   int part_begin = 0;
   bool empty = n_tiles <= 0;                               // workgroup-uniform: no key to read (below)
@@ -954,48 +1112,47 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
       kv_end -= part_begin;
       idx_base += part_begin;
     }
+    row_limit -= part_begin;
   }
-
-  // ---- this lane's row (both lane halves of a row hold the same query, other head dims / keys) ----
-  const int r_row = wid * 32 + l31;
-  const int r_tok = r_row / p.group;
-  const int r_hg = r_row - r_tok * p.group;
-  const bool row_ok = (r_tok < p.tokens_per_tile) && (q0 + r_tok < q1);
-  int row_limit = row_ok ? (causal ? prefix + q0 + r_tok + 1 : kv_len) : 0;
-  if (row_limit > kv_len) row_limit = kv_len;
-  const int row_off = (kvh * p.group + r_hg) * D;
-  if constexpr (PARTS) row_limit -= part_begin;
-  if (empty) {                                             // a part without keys has no weight, a request without keys gives zeros
+  auto put_zeros = [&]() __attribute__((always_inline)) {
+    uint16_t* op = p.out + static_cast<int64_t>(q_begin + q0 + r_tok) * p.out_stride + row_off;
+#pragma unroll
+    for (int c = 0; c < CPR / 2; ++c) *reinterpret_cast<U4*>(op + (2 * c + hi) * 8) = U4{0u, 0u, 0u, 0u};
+  };
+  if (!STAYS && empty) {                                   // a part without keys has no weight, a request without keys gives zeros
     if (PARTS && p.parts > 1) {
       if (row_ok && hi == 0) {
         float* ml = p.part_ml + 2 * (part * p.part_rows + static_cast<int64_t>(q_begin + q0 + r_tok) * (p.num_kv_heads * p.group) + kvh * p.group + r_hg);
         ml[0] = kNegBig;
         ml[1] = 0.f;
       }
-    } else if (row_ok) {
-      uint16_t* op = p.out + static_cast<int64_t>(q_begin + q0 + r_tok) * p.out_stride + row_off;
-#pragma unroll
-      for (int c = 0; c < CPR / 2; ++c) *reinterpret_cast<U4*>(op + (2 * c + hi) * 8) = U4{0u, 0u, 0u, 0u};
-    }
+    } else if (row_ok) put_zeros();
     return;
   }
   U4 qreg[KS];                                      // Q^T operand of k-step s: dims 16 s + 8 h .. + 7 of the row
+  if constexpr (!STAYS) {
 #pragma unroll
-  for (int s = 0; s < KS; ++s) {
-    U4 qf = U4{0u, 0u, 0u, 0u};
-    if (row_ok) qf = ld16(p.q + static_cast<int64_t>(q_begin + q0 + r_tok) * p.q_stride + row_off + s * 16 + hi * 8);
-    qreg[s] = qf;
+    for (int s = 0; s < KS; ++s) {
+      U4 qf = U4{0u, 0u, 0u, 0u};
+      if (row_ok) qf = ld16(p.q + static_cast<int64_t>(q_begin + q0 + r_tok) * p.q_stride + row_off + s * 16 + hi * 8);
+      qreg[s] = qf;
+    }
   }
 
   f32x16_t ot[ND];
+  float m_run, l_run;                               // l: this lane's share of the row sum
+  auto fresh = [&]() __attribute__((always_inline)) {
+    m_run = kNegBig;
+    l_run = 0.f;
 #pragma unroll
-  for (int n = 0; n < ND; ++n)
+    for (int n = 0; n < ND; ++n)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) ot[n][r] = 0.f;
-  float m_run = kNegBig, l_run = 0.f;               // l: this lane's share of the row sum
+      for (int r = 0; r < 16; ++r) ot[n][r] = 0.f;
+  };
+  if constexpr (!STAYS) fresh();
 
   // ---- staging: thread = (row st_r + ROWS_PER_PASS i, 16-byte chunk st_c) of a K tile and of a V tile ----
-  const int st_c = tid % CPR, st_r = tid / CPR;
+  int st_c, st_r;
   int32_t idx_k[LOADS], idx_v[LOADS];
   typedef typename std::conditional<FP8, uint2, U4>::type Stage;   // a gathered 8-dim piece as it travels: raw bytes
   Stage kst[LOADS], vst[LOADS];
@@ -1016,14 +1173,36 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
       dst[i] = idx_base[tok];
     }
   };
-  const unsigned char* k_rows = reinterpret_cast<const unsigned char*>(p.k_cache) + static_cast<uint64_t>(kvh) * p.fmt.head_stride + st_c * (FP8 ? 8 : 16);
-  const unsigned char* v_rows = reinterpret_cast<const unsigned char*>(p.v_cache) + static_cast<uint64_t>(kvh) * p.fmt.head_stride + st_c * (FP8 ? 8 : 16);
   // V^T operand reads: lane i of 16-lane group g points at token row 4 (g >> 1) + (i >> 2), dims 16 (g & 1) + 4 (i & 3)
-  const int v_lane = (4 * hi + ((lane & 15) >> 2)) * 64 + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
+  int v_lane;
+  auto staging = [&]() __attribute__((always_inline)) {
+    if constexpr (STAYS) lanes();
+    st_c = tid % CPR;
+    st_r = tid / CPR;
+    v_lane = (4 * hi + ((lane & 15) >> 2)) * 64 + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
+  };
+  if constexpr (STAYS) {
+    staging();
+  } else {
+    st_c = tid % CPR;
+    st_r = tid / CPR;
+  }
+  auto head_rows = [&](const uint16_t* cache, int head) __attribute__((always_inline)) {
+    return reinterpret_cast<const unsigned char*>(cache) + static_cast<uint64_t>(head) * p.fmt.head_stride + st_c * (FP8 ? 8 : 16);
+  };
+  const unsigned char* k_rows = head_rows(p.k_cache, kvh);
+  const unsigned char* v_rows = head_rows(p.v_cache, kvh);
+  if constexpr (!STAYS) v_lane = (4 * hi + ((lane & 15) >> 2)) * 64 + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
 
+  // (STAYS: a stride widened in front of the outer loop would be multiplied in 64 x 32 bits, two quarter-rate instructions a row for one)
+  auto row_stride = [&]() __attribute__((always_inline)) {
+    uint32_t x = p.fmt.page_stride;
+    if constexpr (STAYS) asm volatile("" : "+s"(x));
+    return x;
+  };
   auto load_rows = [&](const unsigned char* base, const int32_t (&ids)[LOADS], Stage (&dst)[LOADS]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) dst[i] = ld_stage(base + static_cast<uint64_t>(static_cast<uint32_t>(ids[i])) * p.fmt.page_stride);
+    for (int i = 0; i < LOADS; ++i) dst[i] = ld_stage(base + static_cast<uint64_t>(static_cast<uint32_t>(ids[i])) * row_stride());
   };
   auto put_k = [&](int buf, const Stage (&src)[LOADS]) __attribute__((always_inline)) {
 #pragma unroll
@@ -1039,24 +1218,133 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
   };
   // ---- prologue: K(0), K(1), V(0) go to LDS in one round trip; K(2) and V(1) are asked for; ids of tiles 2 / 3 held.
   // (Tiles behind the end of the walk: load_idx clamps to the walk's last row, nobody reads those images.) ----------
-  {
-    int32_t i0[LOADS], i1[LOADS];
-    Stage k0[LOADS], k1[LOADS], v0[LOADS];
-    load_idx(0, i0);
-    load_idx(1, i1);
-    load_rows(k_rows, i0, k0);
-    load_rows(k_rows, i1, k1);
-    load_rows(v_rows, i0, v0);
+  // STAYS: the next query tile's rows (kst, k1st, vst) and queries are asked for while this one is walked.
+  int32_t id1[LOADS];
+  Stage k1st[LOADS];
+  auto first_rows = [&](int head, int64_t q_at, int q_len) __attribute__((always_inline)) {      // (queue->ids holds the slots)
+    const unsigned char* kr = head_rows(p.k_cache, head);
+    const unsigned char* vr = head_rows(p.v_cache, head);
+    int32_t id0[LOADS];
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int32_t* ids = queue->ids + thread() / CPR + ROWS_PER_PASS * i;
+      id0[i] = ids[0];
+      id1[i] = ids[kKvTile];
+      idx_v[i] = ids[2 * kKvTile];
+      idx_k[i] = ids[3 * kKvTile];
+    }
+    load_rows(kr, id0, kst);
+    load_rows(kr, id1, k1st);
+    load_rows(vr, id0, vst);
+    // (a row beyond the tile's tokens takes its last token's queries: all its keys are masked)
+    row_of(thread());
+    const uint16_t* qp = p.q + (q_at + (r_tok < q_len ? r_tok : q_len - 1)) * p.q_stride + (head * p.group + r_hg) * D + (thread() >> 5 & 1) * 8;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qreg[s] = ld16(qp + s * 16);
+  };
+  if constexpr (!STAYS) {
+    Stage k0[LOADS], v0[LOADS];
+    int32_t id0[LOADS];
+    load_idx(0, id0);
+    load_idx(1, id1);
+    load_rows(k_rows, id0, k0);
+    load_rows(k_rows, id1, k1st);
+    load_rows(v_rows, id0, v0);
     load_idx(2, idx_v);
     load_idx(3, idx_k);
     put_k(0, k0);
-    put_k(1, k1);
+    put_k(1, k1st);
     put_v(0, v0);
     load_rows(k_rows, idx_v, kst);                   // K(2): written at the top of step 0
-    load_rows(v_rows, i1, vst);                      // V(1): same
+    load_rows(v_rows, id1, vst);                     // V(1): same
+    __syncthreads();
   }
-  __syncthreads();
 
+  // ---- STAYS: the tile taken next.  Taken eight to nine steps before the end of this one, handed to all waves two steps later, looked up another
+  // two later, its slots left in LDS another two later; its rows travel under the last step and the epilogue. ----
+  bool more = false;                                 // there is one
+  int n_b = 0, n_kvh = 0, n_tile = 0;
+  int32_t held = 0;                                  // what is on its way: the count of tiles taken (thread 0), a slot id
+  auto take = [&]() __attribute__((always_inline)) {
+    if (thread() == 0) held = static_cast<int32_t>(__hip_atomic_fetch_add(p.grabbed + (blockIdx.x & 7), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  };
+  auto hand = [&]() __attribute__((always_inline)) {
+    if (thread() == 0) queue->next = 8 * (static_cast<int>(gridDim.x / 8) + held) + static_cast<int>(blockIdx.x & 7);
+  };
+  int n_q0 = 0, n_len = 0;                           // its tokens
+  int64_t n_at = 0;
+  auto slot_of = [&](const int32_t* base, int end) __attribute__((always_inline)) {
+    const int x = thread(), tok = x < 4 * kKvTile ? x : 0;
+    held = base[tok < end ? tok : end - 1];
+  };
+  auto look = [&]() __attribute__((always_inline)) {
+    const int L = __builtin_amdgcn_readfirstlane(queue->next);
+    more = L < all;
+    if (more) queue->find(L, top, p.batch, p.num_kv_heads, thread() & 63, n_b, n_kvh, n_tile);
+    const int32_t* base = idx_base;
+    int end = 0;
+    if (more) {
+      const int len = __builtin_amdgcn_readfirstlane(queue->len[n_b]), keys = __builtin_amdgcn_readfirstlane(queue->kv_len[n_b]);
+      const int pre = __builtin_amdgcn_readfirstlane(queue->prefix[n_b]);
+      base = p.req_to_token + __builtin_amdgcn_readfirstlane(queue->row[n_b]) * p.r2t_stride;
+      n_q0 = n_tile * p.tokens_per_tile;
+      n_len = len - n_q0 < p.tokens_per_tile ? len - n_q0 : p.tokens_per_tile;
+      n_at = __builtin_amdgcn_readfirstlane(queue->q_begin[n_b]) + n_q0;
+      end = causal && pre + n_q0 + n_len < keys ? pre + n_q0 + n_len : keys;
+    }
+    if (end <= 0) {                                  // nothing to read ahead: this tile's own rows once more
+      base = idx_base;
+      end = kv_end;
+      n_len = q1 - q0;
+      n_at = q_begin + q0;
+      if (!more) n_kvh = kvh;
+    }
+    if (end > 0) slot_of(base, end);
+  };
+  auto leave = [&]() __attribute__((always_inline)) {
+    const int x = thread();
+    if (x < 4 * kKvTile) queue->ids[x] = held;
+  };
+  auto from_scratch = [&]() __attribute__((always_inline)) {                // this tile's first rows, nothing read ahead
+    if (n_tiles > 0) {
+      staging();
+      slot_of(idx_base, kv_end);
+      leave();
+      __syncthreads();
+      first_rows(kvh, q_begin + q0, q1 - q0);
+    }
+  };
+  if constexpr (STAYS) from_scratch();
+
+  for (;;) {                                         // (STAYS: the tiles of the workgroup)
+  if constexpr (STAYS) {
+    if (empty) {                                     // no key: zeros, and the next tile from scratch
+      if (row_ok) put_zeros();
+      take();
+      hand();
+      __syncthreads();
+      look();
+      __syncthreads();
+      if (!more) return;
+      kvh = n_kvh;
+      of_queue(n_b, n_tile);
+      place();
+      empty = n_tiles <= 0;
+      from_scratch();
+      continue;
+    }
+    staging();
+    if (n_tiles < 9) take();                         // too few steps to hide it all
+    k_rows = head_rows(p.k_cache, kvh);
+    v_rows = head_rows(p.v_cache, kvh);
+    put_k(0, kst);
+    put_k(1, k1st);
+    put_v(0, vst);
+    load_rows(k_rows, idx_v, kst);
+    load_rows(v_rows, id1, vst);
+    __syncthreads();
+  }
+  if constexpr (STAYS) fresh();
   f32x16_t s_a[2], s_b[2];                           // the two score sets: tile t and tile t + 1 trade places every step
   U4 pp[4];                                          // bf16(P(t)): [2 blk + ks] -> the 16 keys of one PV k-step
 #pragma unroll
@@ -1136,8 +1424,11 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
     // ---- what was asked for a step ago goes to LDS: K(t + 2), V(t + 1) -- images nobody reads before the barrier below.
     // (Between the phases instead, with the requests beside the phase-2 products: same time per tile, the wait moves
     // with the writes; and the registers no longer fit.)
-    put_k(t & 1, kst);
-    put_v((t + 1) & 1, vst);
+    // (STAYS: in the last step kst and vst hold the next query tile's rows)
+    if constexpr (!STAYS || HAVE_NEXT) {
+      put_k(t & 1, kst);
+      put_v((t + 1) & 1, vst);
+    }
     EXT_T(0);
     // (8 waves: in phase 1, where most vector instructions are, a wave goes first; the SIMD's other wave has matrix instructions to issue
     // beside them when it is in phase 2, and the older of two waves in phase 1 no longer holds the younger back: 696 -> 665 us for 12.6 k
@@ -1157,13 +1448,13 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
       static_assert(NREQ * RSTRIDE <= G1, "requests fit the products of phase 1");
       auto request = [&](int j) __attribute__((always_inline)) {
         if (j < LOADS) {
-          vst[j] = ld_stage(v_rows + static_cast<uint64_t>(static_cast<uint32_t>(idx_v[j])) * p.fmt.page_stride);
+          vst[j] = ld_stage(v_rows + static_cast<uint64_t>(static_cast<uint32_t>(idx_v[j])) * row_stride());
         } else if (j < 2 * LOADS) {
           if (j == LOADS) {
 #pragma unroll
             for (int i = 0; i < LOADS; ++i) idx_v[i] = idx_k[i];          // the ids of K(t + 3) are those of V(t + 3) a step on
           }
-          kst[j - LOADS] = ld_stage(k_rows + static_cast<uint64_t>(static_cast<uint32_t>(idx_k[j - LOADS])) * p.fmt.page_stride);
+          kst[j - LOADS] = ld_stage(k_rows + static_cast<uint64_t>(static_cast<uint32_t>(idx_k[j - LOADS])) * row_stride());
         } else {
           const int last = kv_end - 1;
           const int tok = (t + 4) * kKvTile + st_r + ROWS_PER_PASS * (j - 2 * LOADS);
@@ -1213,7 +1504,7 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
         if (i >= 1) stage_c(i - 1);
         stage_b();
         if (i + 1 < G1) stage_a(i + 1);
-        if constexpr (HAVE_NEXT) __builtin_amdgcn_sched_barrier(0);   // groups stay as written
+        if constexpr (HAVE_NEXT || STAYS) __builtin_amdgcn_sched_barrier(0);   // groups stay as written
       }
       stage_c(G1 - 1);
       // P(t) and its sum are "used" here: hipcc otherwise sinks the exponential stream below later branches
@@ -1258,8 +1549,8 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
 #pragma unroll
             for (int j = PER * (i - LSTART); j < PER * (i - LSTART + 1); ++j) link(sn, m4, j);
           }
-          __builtin_amdgcn_sched_barrier(0);
         }
+        if constexpr (HAVE_NEXT || STAYS) __builtin_amdgcn_sched_barrier(0);
       }
     }
     EXT_T(3);
@@ -1272,11 +1563,42 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
   };
   {
     int t = 0;
+    const int t_take = n_tiles >= 9 ? (n_tiles - 9) & ~1 : -8;
+    if constexpr (STAYS) {
+      if (n_tiles < 9) {                               // (taken in front of the first scores)
+        hand();
+        __syncthreads();
+        look();
+        leave();
+        __syncthreads();
+      }
+      staging();
+    }
     for (; t + 2 < n_tiles; t += 2) {
+      if constexpr (STAYS) {
+        if (__builtin_expect(t >= t_take, 0)) {
+          if (t == t_take) take();
+          else if (t == t_take + 2) hand();
+          else if (t == t_take + 4) look();
+          else if (t == t_take + 6) leave();
+        }
+      }
       step(t, s_a, s_b, std::true_type{});
       step(t + 1, s_b, s_a, std::true_type{});
     }
-    if (n_tiles - t == 2) {
+    if constexpr (STAYS) {                             // (one last step for both: a copy of the scores costs less than its code twice)
+      staging();
+      if (n_tiles - t == 2) {
+        step(t, s_a, s_b, std::true_type{});
+        s_a[0] = s_b[0];
+        s_a[1] = s_b[1];
+        ++t;
+        staging();
+      }
+      first_rows(n_kvh, n_at, n_len);
+      __builtin_amdgcn_sched_barrier(0);
+      step(t, s_a, s_b, std::false_type{});
+    } else if (n_tiles - t == 2) {
       step(t, s_a, s_b, std::true_type{});
       step(t + 1, s_b, s_a, std::false_type{});
     } else {
@@ -1295,8 +1617,14 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
   // ---- epilogue: lane (q, h) holds O^T[d = 32 n + 8 c + 4 h + e][q], c = 0..3, e = 0..3.  The lane halves trade
   // 4-dim pieces (v_permlane32_swap on the packed words) so that h = 0 owns the 8 dims of c = 0, 2 and h = 1 those of
   // c = 1, 3: eight 16-byte stores per lane instead of sixteen 8-byte ones ------------------------------------
-  float l = l_run;
-  l += __shfl_xor(l, 32, 64);
+  const float l = lane_pair_sum(l_run);
+  if constexpr (STAYS || PARTS) {                    // (again: not kept across the walk)
+    int x = threadIdx.x;
+    asm volatile("" : "+v"(x));
+    row_of(x);
+    row_ok = r_tok < q1 - q0;
+    row_off = (kvh * p.group + r_hg) * D;
+  }
   if constexpr (PARTS) {
     if (p.parts > 1) {                                 // unnormalised rows for extend_merge_kernel
       if (row_ok) {
@@ -1335,12 +1663,33 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
       }
     }
   }
+  if (!STAYS || !more) return;
+  kvh = n_kvh;
+  of_queue(n_b, n_tile);
+  place();
+  empty = n_tiles <= 0;
+  }
 }
 
 template <int D, int NWV, bool FP8>
 __global__ __launch_bounds__(64 * NWV, 2) void extend_attention_pipe_kernel(ExtendParams p) {
   __shared__ SmemLadder<D> sm;
   extend_pipe_body<D, NWV, FP8, false>(p, sm);
+}
+
+// 256 workgroups that stay and take the query tiles of a large launch of mixed contexts from the queue, longest contexts first.  A launch deals its
+// workgroups by query tile alone, whatever stands in front of them, and hands out empty ones for the shorter requests; a workgroup of this shape has its CU
+// alone, so that nothing covers its prologue (lengths, slot ids, rows, one behind the other: 10 000 clocks beside a walk of 60 000 to 76 000).  Here the next
+// tile's slots, rows and queries travel under the walk of this one and the longest contexts end first.  The same instructions a tile, the same bits.
+// p.grabbed: eight counters, zero at the launch.  Figures at extend_ragged().  Formed anew for each tile (thread(), staging()): lane constants and what the
+// compiler makes of them; kept across the outer loop they spilled 20 to 400 registers around the walk.
+template <bool FP8>
+__global__ __launch_bounds__(512, 2) void extend_attention_walk_kernel(ExtendParams p) {
+  __shared__ struct {
+    SmemLadder<128> sm;
+    WalkQueue queue;
+  } lds;
+  extend_pipe_body<128, 8, FP8, false, true>(p, lds.sm, &lds.queue);
 }
 
 // The same walk by four waves (128 rows, two workgroups a CU), with a request's key tiles dealt over p.parts workgroups.  Few new tokens
@@ -1390,6 +1739,21 @@ bool extend_eight_waves(int64_t tokens, int64_t batch, int64_t rows, int group, 
   constexpr int kFour = 32 * kPartWaves;
   if (padded(256) < 256 || head_dim != 128 || padded(kFour) * 4 <= padded(256) * 5) return false;
   return padded(256) > 512 || static_cast<double>((held(256) + 255) / 256) <= 1.07 * (static_cast<double>(held(kFour)) / 512.0 + 0.3);
+}
+
+// Whether a launch of eight waves can be one of workgroups that stay: more query tiles than CUs (ragged batches counted as held() does above).
+int64_t extend_held(int64_t tokens, int64_t batch, int group, int kv_heads) { return (2 * tokens * group + batch * 256) / 512 * kv_heads; }
+bool extend_walks(int64_t tokens, int64_t batch, int64_t rows, int group, int kv_heads, int head_dim) {
+  if (head_dim != 128 || tokens <= 0 || batch > WalkQueue::kRequests || group > 256 || !extend_eight_waves(tokens, batch, rows, group, kv_heads, head_dim)) return false;
+  return extend_held(tokens, batch, group, kv_heads) > 256;
+}
+// Whether it pays.  Not while all contexts are about as long, where a step costs 3 % more than is saved between the tiles: us, launched / staying, by mean over
+// longest context: 0.98 to 1.0 549 / 539 .. 311 / 309, 0.91 (8 cold prompts of 1350 - 1650) 214 / 219, 0.91 (24 of 450 - 550, 64 heads) 240 / 228, 0.9 (20 extends
+// of 150 - 450 behind 1000) 344 / 314, 0.84 (4 of 2000 - 3400) 416 / 354, 0.67 (6 of 1.1 - 3.1 k) 662 / 606, 0.4 (12 of 60 - 3000 behind 10 - 6000) 1322 / 745,
+// 0.2 (60 of 200 behind 10 - 6000) 695 / 572.  Nor where walks are over before the next tile has arrived (eight key tiles and fewer), unless many rounds
+// leave something to balance: 16 x 237 cold 41 / 45, 40 x 237 83 / 86, 30 x 200 behind 300 91 / 99; 24 x 350 84 / 81, 36 x 380, 64 heads, 267 / 234.
+bool extend_ragged(int64_t held, int64_t batch, int64_t sum_kv_len, int max_kv_len) {
+  return sum_kv_len > 0 && sum_kv_len * 100 <= batch * max_kv_len * 92 && (max_kv_len >= 640 || (max_kv_len >= 400 && held >= 1024));
 }
 
 template <int D, bool FP8>
@@ -1493,7 +1857,8 @@ static int extend_attention_any(const void* q, void* out, const void* k_cache, c
                                 int64_t k_cache_row_stride, int64_t v_cache_row_stride, float sm_scale,
                                 int causal, int kv_fp8, float k_scale, float v_scale, int page_size, int kv_layout_hnd,
                                 int sliding_window, float logit_cap, const void* custom_mask, const int64_t* mask_indptr,
-                                int skip_prefix_custom_mask, int64_t num_tokens, int max_kv_len, int parts, void* ws_acc, void* ws_ml, void* stream) {
+                                int skip_prefix_custom_mask, int64_t num_tokens, int max_kv_len, int parts, void* ws_acc, void* ws_ml, void* stream,
+                                unsigned* grabbed = nullptr) {
 
   SGL_CLEAR_STALE_ERROR();
   SGL_CHECK_ARG(k_cache_row_stride == v_cache_row_stride, "extend_attention: K and V pools must share a row stride");
@@ -1592,6 +1957,13 @@ static int extend_attention_any(const void* q, void* out, const void* k_cache, c
   const bool fast = plain && nwv == 8 && !(kv_fp8 && (g_extend_debug_flags & 2) != 0);
   if (fast) {
     p.num_tiles = tiles; p.batch = static_cast<int>(batch);
+    if (grabbed != nullptr && g_extend_debug_flags == 0 && extend_walks(num_tokens, batch, rows_total, group, num_kv_heads, head_dim)) {
+      p.grabbed = grabbed;
+      if (kv_fp8) hipLaunchKernelGGL((extend_attention_walk_kernel<true>), dim3(256), dim3(512), 0, st, p);
+      else hipLaunchKernelGGL((extend_attention_walk_kernel<false>), dim3(256), dim3(512), 0, st, p);
+      SGL_CHECK_LAUNCH("extend_attention");
+      return 0;
+    }
     const dim3 grid1(static_cast<unsigned>(tiles) * num_kv_heads * static_cast<unsigned>(batch));
     if ((g_extend_debug_flags & 2) != 0) {
       if (head_dim == 128) hipLaunchKernelGGL((extend_attention_dbuf_kernel<128>), grid1, dim3(512), 0, st, p);
@@ -1674,15 +2046,31 @@ int sgl_amd_extend_attention_store(const void* q, void* out, void* k_cache, void
                                    int head_dim, int64_t q_token_stride, int64_t out_token_stride, int64_t cache_row_stride, float sm_scale, int causal,
                                    int kv_fp8, float k_scale, float v_scale, int parts, void* ws_acc, void* ws_ml, const void* k_new,
                                    const void* v_new, const int64_t* new_loc, int64_t k_new_stride, int64_t v_new_stride, void* stream) {
-  const int row = num_kv_heads * head_dim;
-  const int rc = kv_fp8 ? sgl_amd_store_kv_cache_ex(k_new, v_new, k_cache, v_cache, new_loc, num_tokens, num_kv_heads, head_dim, k_new_stride,
-                                                    v_new_stride, cache_row_stride, 1, k_scale, v_scale, 1, 0, stream)
-                        : sgl_amd_store_kv_cache(k_new, v_new, k_cache, v_cache, new_loc, num_tokens, row, row, k_new_stride, v_new_stride,
-                                                 cache_row_stride, cache_row_stride, stream);
+  SGL_CHECK_ARG(parts >= 0 && (parts > 0 || (ws_ml && max_kv_len > 0 && num_kv_heads > 0 && num_q_heads % num_kv_heads == 0)),
+                "extend_attention_store: counters for workgroups that stay");
+  unsigned* grabbed = parts == 0 ? static_cast<unsigned*>(ws_ml) : nullptr;
+  const int rc = store_kv_rows(k_new, v_new, k_cache, v_cache, new_loc, num_tokens, num_kv_heads, head_dim, k_new_stride, v_new_stride, cache_row_stride, kv_fp8,
+                               k_scale, v_scale, grabbed, stream);
   if (rc != 0) return rc;
-  return sgl_amd_extend_attention_kv(q, out, k_cache, v_cache, req_to_token, req_to_token_stride, req_pool_indices, seq_lens, prefix_lens, qo_indptr,
-                                     batch, num_tokens, max_extend_len, max_kv_len, num_q_heads, num_kv_heads, head_dim, q_token_stride,
-                                     out_token_stride, cache_row_stride, sm_scale, causal, kv_fp8, k_scale, v_scale, parts, ws_acc, ws_ml, stream);
+  if (parts > 0)
+    return sgl_amd_extend_attention_kv(q, out, k_cache, v_cache, req_to_token, req_to_token_stride, req_pool_indices, seq_lens, prefix_lens, qo_indptr,
+                                       batch, num_tokens, max_extend_len, max_kv_len, num_q_heads, num_kv_heads, head_dim, q_token_stride,
+                                       out_token_stride, cache_row_stride, sm_scale, causal, kv_fp8, k_scale, v_scale, parts, ws_acc, ws_ml, stream);
+  return extend_attention_any(q, out, k_cache, v_cache, req_to_token, req_to_token_stride, req_pool_indices, seq_lens, prefix_lens,
+                              qo_indptr, num_tokens == 0 ? 0 : batch, max_extend_len, num_q_heads, num_kv_heads, head_dim, q_token_stride,
+                              out_token_stride, cache_row_stride, cache_row_stride, sm_scale, causal, kv_fp8, k_scale, v_scale, 1, 0, -1, 0.0f,
+                              nullptr, nullptr, 0, num_tokens, max_kv_len, 1, nullptr, nullptr, stream, grabbed);
+}
+
+int sgl_amd_extend_attention_store_parts(int64_t batch, int64_t num_tokens, int64_t sum_kv_len, int max_extend_len, int max_kv_len, int num_q_heads,
+                                         int num_kv_heads, int head_dim) {
+  if (batch > 0 && max_extend_len > 0 && max_kv_len > kKvTile && num_kv_heads > 0 && num_q_heads % num_kv_heads == 0 && g_extend_debug_shape == 0 &&
+      g_extend_debug_flags == 0) {
+    const int group = num_q_heads / num_kv_heads;
+    if (extend_ragged(extend_held(num_tokens, batch, group, num_kv_heads), batch, sum_kv_len, max_kv_len) &&
+        extend_walks(num_tokens, batch, static_cast<int64_t>(max_extend_len) * group, group, num_kv_heads, head_dim)) return 0;
+  }
+  return sgl_amd_extend_attention_parts(batch, num_tokens, max_extend_len, max_kv_len, num_q_heads, num_kv_heads, head_dim);
 }
 
 #ifdef EXT_TRACE

@@ -102,4 +102,9 @@ __device__ __forceinline__ float soft_cap_log2(float x, float cap_log2, float in
   return cap_log2 * th;
 }
 
+// store_kv_cache of [num_tokens, H_kv, D] rows to a token-major pool; zero8: eight counters that the launch behind it needs zeroed (null: none).
+int store_kv_rows(const void* k, const void* v, void* k_cache, void* v_cache, const int64_t* loc, int64_t num_tokens, int num_kv_heads, int head_dim,
+                  int64_t k_token_stride, int64_t v_token_stride, int64_t cache_row_stride, int kv_fp8, float k_scale, float v_scale, unsigned* zero8,
+                  void* stream);
+
 }  // namespace sgl_amd

@@ -389,10 +389,10 @@ def extend_attention(q: torch.Tensor, out: torch.Tensor, k_cache: torch.Tensor, 
                      causal: bool = True, kv_fp8: bool = False, k_scale: float = 1.0, v_scale: float = 1.0,
                      page_size: int = 1, hnd: bool = False, sliding_window: int = -1, logit_cap: float = 0.0,
                      custom_mask: Optional[torch.Tensor] = None, mask_indptr: Optional[torch.Tensor] = None,
-                     skip_prefix_custom_mask: bool = False, max_kv_len: int = 0, new_rows=None) -> torch.Tensor:
+                     skip_prefix_custom_mask: bool = False, max_kv_len: int = 0, new_rows=None, sum_kv_len: int = 0) -> torch.Tensor:
     """q/out [T, Hq, D]; k_cache/v_cache [slots, Hkv, D] (HND / fp8 as in decode_attention); int32
-    seq_lens/prefix_lens/qo_indptr; custom_mask uint8 / bool flat, mask_indptr int64 [B + 1].  max_kv_len: the longest of seq_lens where the
-    caller knows it on the host (0: unknown); it decides how the work is dealt, never what is computed.  new_rows: (k, v, loc), the pass's rows
+    seq_lens/prefix_lens/qo_indptr; custom_mask uint8 / bool flat, mask_indptr int64 [B + 1].  max_kv_len, sum_kv_len: the longest of seq_lens and
+    their sum where the caller knows them on the host (0: unknown); they decide how the work is dealt, never what is computed.  new_rows: (k, v, loc), the pass's rows
     [T, Hkv, D] and their slots (int64 [T]), stored in front as store_kv_cache would (max_kv_len known; no hnd, window, cap or mask)."""
     _dev(q, out, k_cache, v_cache, req_to_token, req_pool_indices, seq_lens, prefix_lens, qo_indptr)
     T, Hq, D = q.shape
@@ -405,7 +405,7 @@ def extend_attention(q: torch.Tensor, out: torch.Tensor, k_cache: torch.Tensor, 
         _need(q.stride(2) == 1 and q.stride(1) == D and out.stride(2) == 1 and out.stride(1) == D, "extend_attention: q/out head layout")
         if max_kv_len > 0 and not hnd and sliding_window < 0 and logit_cap <= 0 and custom_mask is None:
             return _extend_attention_kv(q, out, k_cache, v_cache, req_to_token, req_pool_indices, seq_lens, prefix_lens, qo_indptr, max_extend_len,
-                                        max_kv_len, sm_scale, causal, kv_fp8, k_scale, v_scale, Hkv * D, new_rows)
+                                        max_kv_len, sm_scale, causal, kv_fp8, k_scale, v_scale, Hkv * D, new_rows, sum_kv_len)
         _need(new_rows is None, "extend_attention: new rows in this form")
         if custom_mask is not None:
             _dev(custom_mask, mask_indptr)
@@ -427,7 +427,7 @@ def extend_attention(q: torch.Tensor, out: torch.Tensor, k_cache: torch.Tensor, 
     _need(k_s[2] == 1 and k_s[1] == D and v_s[1] == D, "extend_attention: cache layout")
     if max_kv_len > 0 and k_s[0] == v_s[0]:
         return _extend_attention_kv(q, out, k_cache, v_cache, req_to_token, req_pool_indices, seq_lens, prefix_lens, qo_indptr, max_extend_len,
-                                    max_kv_len, sm_scale, causal, False, 1.0, 1.0, k_s[0], new_rows)
+                                    max_kv_len, sm_scale, causal, False, 1.0, 1.0, k_s[0], new_rows, sum_kv_len)
     _need(new_rows is None, "extend_attention: new rows in this form")
     native.call("sgl_amd_extend_attention", q.data_ptr(), out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
                 req_to_token.data_ptr(), req_to_token.stride(0), req_pool_indices.data_ptr(), seq_lens.data_ptr(),
@@ -440,18 +440,21 @@ def extend_attention(q: torch.Tensor, out: torch.Tensor, k_cache: torch.Tensor, 
 
 def _extend_attention_kv(q, out, k_cache, v_cache, req_to_token, req_pool_indices, seq_lens, prefix_lens, qo_indptr, max_extend_len: int,
                          max_kv_len: int, sm_scale: float, causal: bool, kv_fp8: bool, k_scale: float, v_scale: float, row_stride: int,
-                         new_rows=None) -> torch.Tensor:
+                         new_rows=None, sum_kv_len: int = 0) -> torch.Tensor:
     """extend_attention over a token-major pool whose longest context is known (arguments checked by the caller)."""
     (T, Hq, D), Hkv, B = q.shape, k_cache.shape[1], seq_lens.numel()
     parts, out_stride = 1, out.stride(0)
     if max_kv_len > 256 and out_stride % 8 == 0:          # (a split of four tiles or fewer never pays: not worth asking)
-        parts = native.lib().sgl_amd_extend_attention_parts(B, T, int(max_extend_len), int(max_kv_len), Hq, Hkv, D)
-    ws = torch.empty(parts * T * Hq * (D + 2), dtype=torch.float32, device=q.device) if parts > 1 else None
-    acc = ws.data_ptr() if parts > 1 else None
+        shape = (int(max_extend_len), int(max_kv_len), Hq, Hkv, D)
+        parts = (native.lib().sgl_amd_extend_attention_parts(B, T, *shape) if new_rows is None
+                 else native.lib().sgl_amd_extend_attention_store_parts(B, T, int(sum_kv_len), *shape))
+    # (0 parts: workgroups that stay, eight counters)
+    ws = torch.empty(parts * T * Hq * (D + 2) or 8, dtype=torch.float32, device=q.device) if parts != 1 else None
+    acc = ws.data_ptr() if parts != 1 else None
     args = (q.data_ptr(), out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), req_to_token.data_ptr(),
             req_to_token.stride(0), req_pool_indices.data_ptr(), seq_lens.data_ptr(), prefix_lens.data_ptr(), qo_indptr.data_ptr(), B, T,
             int(max_extend_len), int(max_kv_len), Hq, Hkv, D, q.stride(0), out_stride, row_stride, float(sm_scale), 1 if causal else 0,
-            1 if kv_fp8 else 0, float(k_scale), float(v_scale), parts, acc, acc + 4 * parts * T * Hq * D if parts > 1 else None)
+            1 if kv_fp8 else 0, float(k_scale), float(v_scale), parts, acc, acc + 4 * parts * T * Hq * D if parts != 1 else None)
     if new_rows is None:
         native.call("sgl_amd_extend_attention_kv", *args, _stream())
         return out

@@ -50,7 +50,8 @@ class _Meta:
     qo_indptr: Optional[torch.Tensor] = None
     prefix_lens_i32: Optional[torch.Tensor] = None
     max_extend_len: int = 0
-    max_kv_len: int = 0                      # extend: the longest context of the batch, where the host knows it
+    max_kv_len: int = 0                      # extend: the longest context of the batch and the sum of all, where the host knows them
+    sum_kv_len: int = 0
     cascade: Optional["kernels.CascadeWorkspace"] = None   # shared-prefix decode plan + split slots
     mask_indptr: Optional[torch.Tensor] = None             # TARGET_VERIFY: offsets of the requests' blocks in the flat mask
     verify_mask: Optional[torch.Tensor] = None             # TARGET_VERIFY: the persistent copy of this step's flat tree mask
@@ -305,7 +306,8 @@ class HipAttnBackend(AttentionBackend):
             self.forward_metadata = _Meta(seq_i32, qo_indptr=qo.to(self.device, non_blocking=True),
                                           prefix_lens_i32=fb.extend_prefix_lens.to(torch.int32),
                                           max_extend_len=max(ext) if ext else 0,
-                                          max_kv_len=int(fb.seq_lens_cpu.max()) if fb.seq_lens_cpu is not None and len(fb.seq_lens_cpu) else 0)
+                                          **(dict(max_kv_len=int(fb.seq_lens_cpu.max()), sum_kv_len=int(fb.seq_lens_cpu.sum()))
+                                             if fb.seq_lens_cpu is not None and len(fb.seq_lens_cpu) else {}))
         else:
             self.forward_metadata = None
 
@@ -396,7 +398,7 @@ class HipAttnBackend(AttentionBackend):
         kernels.extend_attention(q3, o, self.token_to_kv_pool.get_key_buffer(layer.layer_id),
                                  self.token_to_kv_pool.get_value_buffer(layer.layer_id),
                                  self.req_to_token_pool.req_to_token, self._pool_idx(forward_batch), m.seq_lens_i32,
-                                 m.prefix_lens_i32, m.qo_indptr, m.max_extend_len, layer.scaling, causal, max_kv_len=m.max_kv_len, new_rows=new_rows, **opt)
+                                 m.prefix_lens_i32, m.qo_indptr, m.max_extend_len, layer.scaling, causal, max_kv_len=m.max_kv_len, sum_kv_len=m.sum_kv_len, new_rows=new_rows, **opt)
         return o.view(-1, layer.tp_q_head_num * layer.v_head_dim)
 
     @staticmethod

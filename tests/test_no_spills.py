@@ -76,6 +76,17 @@ def test_extend_eight_wave_kernels_keep_their_registers_and_lds(tmp_path):
 
 
 @pytest.mark.skipif(not Path(HIPCC).exists(), reason="hipcc not installed")
+def test_extend_workgroups_that_stay_keep_their_registers(tmp_path):
+    """The walk of the 8-wave kernel inside a loop over query tiles: what that loop keeps alive is a reload in the walk."""
+    usage = _resource_usage("extend_attention.hip", tmp_path)
+    inst = {k: v for k, v in usage.items() if "extend_attention_walk_kernel" in k or "extend_attention_parts_kernel" in k}
+    assert len(inst) == 6, sorted(usage)
+    for name, u in inst.items():
+        assert u["vgpr_spill_count"] == 0 and u["sgpr_spill_count"] == 0 and u["vgpr_count"] <= 256, (name, u)
+        assert u["group_segment_fixed_size"] <= (160 if "walk" in name else 80) * 1024, (name, u)
+
+
+@pytest.mark.skipif(not Path(HIPCC).exists(), reason="hipcc not installed")
 def test_general_extend_kernels_do_not_spill(tmp_path):
     """Every instance of the general extend kernel (fp8 / paged pools, sliding window, soft cap, custom mask; the 4-wave
     shapes of short extends): a spill would sit inside the KV-tile loop."""
