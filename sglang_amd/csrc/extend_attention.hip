@@ -1038,13 +1038,12 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
     queue->find(blockIdx.x, top, p.batch, p.num_kv_heads, lane, b, kvh, tile);
     of_queue(b, tile);
   } else {
+    int heads = p.num_kv_heads;
+    int64_t table_stride = p.r2t_stride;
+    asm("" : "+s"(heads), "+s"(table_stride));             // (asked for with the first arguments, not in a round trip of its own behind the lengths)
     {
-      // (the arguments in one round trip, not piece by piece in front of their first uses)
-      asm volatile("" ::"s"(p.q), "s"(p.k_cache), "s"(p.v_cache), "s"(p.req_to_token), "s"(p.req_pool_indices), "s"(p.seq_lens), "s"(p.prefix_lens), "s"(p.qo_indptr),
-                   "s"(p.q_stride), "s"(p.r2t_stride), "s"(p.fmt.page_stride), "s"(p.fmt.head_stride), "s"(p.scale_log2), "s"(p.group), "s"(p.causal),
-                   "s"(p.parts), "s"(p.part_rows), "s"(p.part_ml));
       const int L = blockIdx.x;
-      const int pairs = p.batch * p.num_kv_heads * (PARTS ? p.parts : 1);
+      const int pairs = p.batch * heads * (PARTS ? p.parts : 1);
       int pair, rank;
       if (pairs % 8 == 0) {
         const int per_xcd = pairs / 8;
@@ -1060,17 +1059,17 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
         part = pair % p.parts;
         pair /= p.parts;
       }
-      kvh = pair % p.num_kv_heads;
-      b = pair / p.num_kv_heads;
+      kvh = pair % heads;
+      b = pair / heads;
     }
     q_begin = p.qo_indptr[b];
     ext_len = p.qo_indptr[b + 1] - q_begin;
     kv_len = p.seq_lens[b];
     prefix = p.prefix_lens[b];
-    const int64_t row = p.req_pool_indices[b];
-    // (one round trip for all five: left to itself the compiler sinks the last three below the branch)
-    asm volatile("" ::"s"(ext_len), "s"(kv_len), "s"(prefix), "s"(row));
-    idx_base = p.req_to_token + row * p.r2t_stride;
+    int64_t row = p.req_pool_indices[b];
+    // (one round trip for all five: left to itself the compiler sinks the last three below the branch.  Not volatile: behind that they would be vector loads)
+    asm("" : "+s"(ext_len), "+s"(kv_len), "+s"(prefix), "+s"(row));
+    idx_base = p.req_to_token + row * table_stride;
     if (tile * p.tokens_per_tile >= ext_len) return;
   }
 
