@@ -1744,6 +1744,7 @@ bool extend_eight_waves(int64_t tokens, int64_t batch, int64_t rows, int group, 
 int64_t extend_held(int64_t tokens, int64_t batch, int group, int kv_heads) { return (2 * tokens * group + batch * 256) / 512 * kv_heads; }
 bool extend_walks(int64_t tokens, int64_t batch, int64_t rows, int group, int kv_heads, int head_dim) {
   if (head_dim != 128 || tokens <= 0 || batch > WalkQueue::kRequests || group > 256 || !extend_eight_waves(tokens, batch, rows, group, kv_heads, head_dim)) return false;
+  if (rows / group > static_cast<int64_t>(256 / group) * WalkQueue::kLevels) return false;       // a request's tiles stand at levels of their own
   return extend_held(tokens, batch, group, kv_heads) > 256;
 }
 // Whether it pays.  Not while all contexts are about as long, where a step costs 3 % more than is saved between the tiles: us, launched / staying, by mean over

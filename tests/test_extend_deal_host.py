@@ -11,6 +11,10 @@ from sglang_amd import native
     ([1100, 3100, 2000, 1500, 2700, 2200], [0] * 6, 14, 2, 64, False),   # head dim 64: four waves
     ([20, 300, 100], [0] * 3, 32, 8, 128, False),                        # fewer tiles than CUs
     ([150 + i for i in range(513)], [7 * i for i in range(513)], 32, 8, 128, False),
+    ([40000, 100], [0, 0], 32, 8, 128, True),
+    ([300000, 100], [0, 0], 32, 8, 128, False),                          # more tiles of 64 tokens than levels
+    ([262144, 100], [0, 0], 32, 8, 128, True),
+    ([262145, 100], [0, 0], 32, 8, 128, False),
     ([150 + i % 40 for i in range(512)], [7 * i for i in range(512)], 32, 8, 128, True),
 ])
 def test_rule(lens, pre, hq, hkv, d, stays):
