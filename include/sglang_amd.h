@@ -205,20 +205,6 @@ int sgl_amd_cascade_decode_attention_ex(const void* q, const void* k_cache, cons
                                         float sm_scale, int64_t max_context_len, int slots_total,
                                         void* ws_acc, void* ws_ml, int kv_fp8, float k_scale, float v_scale,
                                         int page_size, int kv_layout_hnd, void* stream);
-/* The same with the store of the step's K / V rows in it (set_kv_buffer before forward_decode, memory_pool.py:2331-2456): k_new / v_new
- * [B, H_kv, D] bf16 (token strides in elements, 16-byte aligned) go to the pool rows new_loc[b] while the requests attend.  A request whose
- * last token's slot is new_loc[b] sees its new row; every other slot is read as the pool held it before the call.  k_new NULL: no store. */
-int sgl_amd_cascade_decode_attention_store(const void* q, void* k_cache, void* v_cache, void* out,
-                                           const int32_t* req_to_token, int64_t req_to_token_stride,
-                                           const int64_t* req_pool_indices, const int32_t* seq_lens,
-                                           const int32_t* plan, int64_t batch, int64_t max_items,
-                                           int num_q_heads, int num_kv_heads, int head_dim,
-                                           int64_t q_token_stride, int64_t out_token_stride,
-                                           int64_t k_cache_row_stride, int64_t v_cache_row_stride,
-                                           float sm_scale, int64_t max_context_len, int slots_total,
-                                           void* ws_acc, void* ws_ml, int kv_fp8, float k_scale, float v_scale,
-                                           int page_size, int kv_layout_hnd, const void* k_new, const void* v_new, const int64_t* new_loc,
-                                           int64_t k_new_stride, int64_t v_new_stride, void* stream);
 
 /* ---- Sampling (reference: srt/layers/sampler.py:98-260,567-750;
  *      kernels/ops/sampling/murmur_hash.py:51-121) ------------------------------- */

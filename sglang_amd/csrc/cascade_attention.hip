@@ -89,11 +89,7 @@ struct ChunkParams {
   int slots_total;
   float scale_log2;
   int walks_spans;              // the looping kernel takes the plan's spans, where it has any, in the place of the private items
-  int last_apart;               // the merge takes every request's last token (from the step's new rows): items end in front of it
 };
-
-// tokens of an item whose record ends in (kv tokens, ..., field 7)
-__device__ __forceinline__ int item_tokens(const ChunkParams& p, int kv_n, int field7) { return kv_n - (p.last_apart && field7 == kHoldsLast ? 1 : 0); }
 
 // The K rows, then (after S^T) the transposed V rows, pass through ONE 16 KiB LDS image; at D = 128 it is filled twice
 // per operand: K by token halves (64 tokens x 128 dims: each score tile is complete inside its half), V^T by head-dim
@@ -165,8 +161,7 @@ __device__ __forceinline__ void cascade_few_rows_unit(const ChunkParams& p, U4* 
   auto swz = [](int t) __attribute__((always_inline)) { return D == 128 ? 2 * (t & 3) : 2 * ((t >> 1) & 3); };
   const CascadePlanView pv = cascade_plan_view(p.plan, p.batch, p.max_items);
   const int lane = tid & 63, wid = tid >> 6, i16 = lane & 15, g = lane >> 4;
-  const int slot = __builtin_amdgcn_readfirstlane(ra.x), kv_begin = __builtin_amdgcn_readfirstlane(ra.y),
-            kv_n = item_tokens(p, __builtin_amdgcn_readfirstlane(ra.z), __builtin_amdgcn_readfirstlane(rb.w));     // (none left: an empty set)
+  const int slot = __builtin_amdgcn_readfirstlane(ra.x), kv_begin = __builtin_amdgcn_readfirstlane(ra.y), kv_n = __builtin_amdgcn_readfirstlane(ra.z);
   const int n_rows = __builtin_amdgcn_readfirstlane(ra.w) * p.group;
   const int rec_x = __builtin_amdgcn_readfirstlane(rb.x), rec_private = __builtin_amdgcn_readfirstlane(rb.y);
   const int32_t* idx_base = p.req_to_token + static_cast<int64_t>(__builtin_amdgcn_readfirstlane(rb.z)) * p.r2t_stride + kv_begin;
@@ -659,7 +654,7 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
     it[4] = tid;                                     // the request itself
     it[5] = 1;                                       // private item
     it[6] = pool_row[tid];
-    it[7] = j + 1 < mine ? -1 : kHoldsLast;
+    it[7] = -1;
     it[3] = 1;
   }
   // ---- spans: the private tokens of all requests, in 64-token tiles, as ONE line cut into equal parts ----
@@ -706,7 +701,7 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
     it[4] = tid;
     it[5] = 1;
     it[6] = pool_row[tid];
-    it[7] = j + 1 < my_pieces ? -1 : kHoldsLast;
+    it[7] = -1;
   }
   if (tid == kPlanThreads - 1) pv.span_first[(n_tiles + span - 1) / span] = incl;
 }
@@ -714,77 +709,26 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
 // ---- merge: slots [0, n_slots(b)) of every (request, head), in slot order ----------------------
 // n_slots = shared chunks + private chunks (pieces, where the launch before walked spans) of the request; every one was written this step.
 // Block = 256 / (D/4) heads x (D/4) lanes; a thread owns 4 consecutive output elements of one head.
-// The step's own K / V rows may come with the launch (NewRows): the last token of every request is then a set of its own here -- one score, one V
-// row -- and its rows go to the pool from these registers.  A store launch in front of the chunk kernel was 1 to 2 us of a layer (us: four layers of two
-// requests of 420 tokens, 32 kv heads, 66 -> 61; 64 requests behind four prefixes of 896, eight layers, 234 -> 221; 37 of 0.9 to 5.1 k in e4m3, four
-// layers, 270 -> 263).  Inside the chunk kernel the newest row, read in the place of a
-// pool row, cost the walk of e4m3 rows as much as that.  Nothing here waits for one another but the row's slot for its table entry: the row is taken
-// as the pool held it where that is another slot.
 constexpr int kMergeBlock = 16;  // slots loaded per round (all loads of a round are in flight together)
 
-struct NewRows {
-  const uint16_t* k;               // [B, Hkv, D]; null: the rows are in the pool
-  const uint16_t* v;
-  const uint16_t* q;
-  void* k_cache;
-  void* v_cache;
-  const int64_t* loc;
-  const int32_t* req_to_token;
-  const int64_t* req_pool_indices;
-  int64_t q_stride, k_stride, v_stride, r2t_stride;
-  int group;
-  float scale_log2, inv_k_scale, inv_v_scale;
-  KvFormat fmt;
-};
-
-// four bf16 values of a row as the pool holds them: the bytes in `kept` (two dwords of bf16, one of e4m3), the values in `x`
-__device__ __forceinline__ void as_kept(const uint2& w, int fp8, float inv_scale, uint2& kept, float (&x)[4]) {
-  x[0] = bf_lo(w.x); x[1] = bf_hi(w.x); x[2] = bf_lo(w.y); x[3] = bf_hi(w.y);
-  kept = w;
-  if (fp8) {
-    const uint2 e = bf16x8_to_fp8x8(U4{w.x, w.y, 0u, 0u}, inv_scale);
-    kept = uint2{e.x, 0u};
-    const U4 b = fp8x8_to_bf16x8(e);
-    x[0] = bf_lo(b.x); x[1] = bf_hi(b.x); x[2] = bf_lo(b.y); x[3] = bf_hi(b.y);
-  }
-}
-
-template <bool NEW>
 __global__ __launch_bounds__(256) void cascade_merge2_kernel(const float* __restrict__ ws_acc, const float* __restrict__ ws_ml,
                                                              const int32_t* __restrict__ plan, const int32_t* __restrict__ seq_lens, int walks_spans,
                                                              uint16_t* __restrict__ out, int64_t out_stride, int batch,
                                                              int max_items, int num_q_heads, int head_dim, int slots_total,
-                                                             float out_scale, NewRows nr) {
+                                                             float out_scale) {
   const int tpd = head_dim >> 2;
   const int b = blockIdx.x;
   const int hq = blockIdx.y * (256 / tpd) + threadIdx.x / tpd;
   const int d = (threadIdx.x % tpd) * 4;
   if (hq >= num_q_heads) return;
   const CascadePlanView pv = cascade_plan_view(plan, batch, max_items);
-  // (everything the partials' addresses and the row's slot follow from is asked for at once: one hop after another cost 0.3 us)
+  // (everything the partials' addresses follow from is asked for at once: one hop after another cost 0.3 us)
   const int span_slots = pv.req_slots[b], sh = pv.req_shared[b], len = seq_lens[b];
-  int64_t loc = 0, pool_row = 0;
-  uint2 kw, vw, qw;
-  int kvh = 0;
-  if constexpr (NEW) {
-    loc = nr.loc[b];
-    pool_row = nr.req_pool_indices[b];
-    kvh = hq / nr.group;
-    qw = *reinterpret_cast<const uint2*>(nr.q + static_cast<int64_t>(b) * nr.q_stride + static_cast<int64_t>(hq) * head_dim + d);
-    kw = *reinterpret_cast<const uint2*>(nr.k + static_cast<int64_t>(b) * nr.k_stride + static_cast<int64_t>(kvh) * head_dim + d);
-    vw = *reinterpret_cast<const uint2*>(nr.v + static_cast<int64_t>(b) * nr.v_stride + static_cast<int64_t>(kvh) * head_dim + d);
-  }
   int n = walks_spans ? span_slots : (sh + kChunk - 1) / kChunk + (len > sh ? (len - sh + kChunk - 1) / kChunk : 0);
   if (n > slots_total) n = slots_total;
   const int64_t base = (static_cast<int64_t>(b) * num_q_heads + hq) * slots_total;
   const float2* ml = reinterpret_cast<const float2*>(ws_ml) + base;
   const float* accp = ws_acc + base * head_dim + d;
-  int own = 0;
-  if constexpr (NEW) {
-    int lane0 = 0;                                         // (a vector load: a scalar one would be waited for with whatever scalar comes next)
-    asm volatile("" : "+v"(lane0));
-    own = nr.req_to_token[pool_row * nr.r2t_stride + (len > 0 ? len - 1 : 0) + lane0];
-  }
   float m_run = kNegBig, l = 0.f;
   float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
   for (int s0 = 0; s0 < n; s0 += kMergeBlock) {
@@ -810,52 +754,6 @@ __global__ __launch_bounds__(256) void cascade_merge2_kernel(const float* __rest
         l += mlv[i].y * sc;
         o.x += av[i].x * sc; o.y += av[i].y * sc; o.z += av[i].z * sc; o.w += av[i].w * sc;
       }
-    }
-  }
-  // ---- the last token's own set (scored behind the partials: in front of them, while the first are on their way, it was 0.3 us slower) ----
-  float kx[4], vx[4], score = 0.f;
-  auto score_of = [&]() __attribute__((always_inline)) {
-    float s = bf_lo(qw.x) * kx[0];
-    s = fmaf(bf_hi(qw.x), kx[1], s);
-    s = fmaf(bf_lo(qw.y), kx[2], s);
-    s = fmaf(bf_hi(qw.y), kx[3], s);
-    for (int lanes = tpd >> 1; lanes > 0; lanes >>= 1) s += __shfl_xor(s, lanes, 64);
-    return s * nr.scale_log2;
-  };
-  if constexpr (NEW) {
-    uint2 kk, vk;
-    as_kept(kw, nr.fmt.fp8, nr.inv_k_scale, kk, kx);
-    as_kept(vw, nr.fmt.fp8, nr.inv_v_scale, vk, vx);
-    if (hq % nr.group == 0) {
-      unsigned char* kd = const_cast<unsigned char*>(kv_row(nr.k_cache, nr.fmt, static_cast<int>(loc), kvh));
-      unsigned char* vd = const_cast<unsigned char*>(kv_row(nr.v_cache, nr.fmt, static_cast<int>(loc), kvh));
-      if (nr.fmt.fp8) {
-        *reinterpret_cast<uint32_t*>(kd + d) = kk.x;
-        *reinterpret_cast<uint32_t*>(vd + d) = vk.x;
-      } else {
-        *reinterpret_cast<uint2*>(kd + 2 * d) = kk;
-        *reinterpret_cast<uint2*>(vd + 2 * d) = vk;
-      }
-    }
-    score = score_of();
-    if (len > 0 && own != loc) {                           // (uniform in the workgroup)
-      const unsigned char* ks = kv_row(nr.k_cache, nr.fmt, own, kvh);
-      const unsigned char* vs = kv_row(nr.v_cache, nr.fmt, own, kvh);
-      if (nr.fmt.fp8) {
-        const U4 a = fp8x8_to_bf16x8(uint2{*reinterpret_cast<const uint32_t*>(ks + d), *reinterpret_cast<const uint32_t*>(vs + d)});
-        kx[0] = bf_lo(a.x); kx[1] = bf_hi(a.x); kx[2] = bf_lo(a.y); kx[3] = bf_hi(a.y);
-        vx[0] = bf_lo(a.z); vx[1] = bf_hi(a.z); vx[2] = bf_lo(a.w); vx[3] = bf_hi(a.w);
-      } else {
-        const uint2 a = *reinterpret_cast<const uint2*>(ks + 2 * d), c = *reinterpret_cast<const uint2*>(vs + 2 * d);
-        kx[0] = bf_lo(a.x); kx[1] = bf_hi(a.x); kx[2] = bf_lo(a.y); kx[3] = bf_hi(a.y);
-        vx[0] = bf_lo(c.x); vx[1] = bf_hi(c.x); vx[2] = bf_lo(c.y); vx[3] = bf_hi(c.y);
-      }
-      score = score_of();
-    }
-    if (len > 0 && score > 0.5f * kNegBig) {               // (a score that is no number counts for nothing, as in the chunk kernel)
-      const float m_new = fmaxf(m_run, score), alpha = exp2f(m_run - m_new), e = exp2f(score - m_new);
-      l = l * alpha + e;
-      o.x = o.x * alpha + vx[0] * e; o.y = o.y * alpha + vx[1] * e; o.z = o.z * alpha + vx[2] * e; o.w = o.w * alpha + vx[3] * e;
     }
   }
   const float inv = (l > 0.f) ? out_scale / l : 0.f;       // out_scale: v_scale of an fp8 pool, else 1
@@ -940,22 +838,6 @@ int sgl_amd_cascade_decode_attention_ex(const void* q, const void* k_cache, cons
                                         int64_t v_cache_row_stride, float sm_scale, int64_t max_context_len,
                                         int slots_total, void* ws_acc, void* ws_ml, int kv_fp8, float k_scale, float v_scale,
                                         int page_size, int kv_layout_hnd, void* stream) {
-  return sgl_amd_cascade_decode_attention_store(q, const_cast<void*>(k_cache), const_cast<void*>(v_cache), out, req_to_token, req_to_token_stride, req_pool_indices,
-                                                seq_lens, plan, batch, max_items, num_q_heads, num_kv_heads, head_dim, q_token_stride,
-                                                out_token_stride, k_cache_row_stride, v_cache_row_stride, sm_scale, max_context_len, slots_total,
-                                                ws_acc, ws_ml, kv_fp8, k_scale, v_scale, page_size, kv_layout_hnd, nullptr, nullptr, nullptr, 0, 0,
-                                                stream);
-}
-
-int sgl_amd_cascade_decode_attention_store(const void* q, void* k_cache, void* v_cache, void* out,
-                                        const int32_t* req_to_token, int64_t req_to_token_stride,
-                                        const int64_t* req_pool_indices, const int32_t* seq_lens, const int32_t* plan,
-                                        int64_t batch, int64_t max_items, int num_q_heads, int num_kv_heads, int head_dim,
-                                        int64_t q_token_stride, int64_t out_token_stride, int64_t k_cache_row_stride,
-                                        int64_t v_cache_row_stride, float sm_scale, int64_t max_context_len,
-                                        int slots_total, void* ws_acc, void* ws_ml, int kv_fp8, float k_scale, float v_scale,
-                                        int page_size, int kv_layout_hnd, const void* k_new, const void* v_new, const int64_t* new_loc,
-                                           int64_t k_new_stride, int64_t v_new_stride, void* stream) {
   SGL_CLEAR_STALE_ERROR();
   SGL_CHECK_ARG(head_dim == 64 || head_dim == 128, "cascade_decode_attention: head_dim=%d not supported (64/128)", head_dim);
   SGL_CHECK_ARG(num_kv_heads > 0 && num_q_heads % num_kv_heads == 0 && num_q_heads / num_kv_heads <= kRowsPerItem,
@@ -968,13 +850,6 @@ int sgl_amd_cascade_decode_attention_store(const void* q, void* k_cache, void* v
   SGL_CHECK_ARG(batch >= 1 && batch <= 1024 && max_items >= 1 && plan && ws_acc && ws_ml, "cascade_decode_attention: bad batch / workspace");
   const int chunks = static_cast<int>((max_context_len + kChunk - 1) / kChunk);
   SGL_CHECK_ARG(slots_total >= chunks + 1, "cascade_decode_attention: slots_total=%d < %d (context chunks + 1)", slots_total, chunks + 1);
-  if (k_new != nullptr) {
-    SGL_CHECK_ARG(v_new && new_loc, "cascade_decode_attention: new rows need K, V and slots");
-    SGL_CHECK_ARG(k_new_stride % 8 == 0 && v_new_stride % 8 == 0 &&
-                      ((reinterpret_cast<uintptr_t>(k_new) | reinterpret_cast<uintptr_t>(v_new) | reinterpret_cast<uintptr_t>(k_cache) |
-                        reinterpret_cast<uintptr_t>(v_cache)) & 15u) == 0,
-                  "cascade_decode_attention: new rows and pools must be 16-byte aligned");
-  }
   hipStream_t st = as_stream(stream);
   ChunkParams p{};
   p.q = static_cast<const uint16_t*>(q);
@@ -1001,13 +876,6 @@ int sgl_amd_cascade_decode_attention_store(const void* q, void* k_cache, void* v
   // (the plan may hold spans: the single-shot form works on its items all the same, and the merge goes by the form launched here)
   p.walks_spans = walks_spans(p.group, head_dim, kv_fp8 != 0) ? 1 : 0;
   const bool loop = worst > (g_cascade_single_shot_units > 0 ? g_cascade_single_shot_units : single_shot_most(chunks, p.walks_spans != 0));
-  NewRows nr{};
-  if (k_new != nullptr) {
-    p.last_apart = 1;
-    nr = NewRows{static_cast<const uint16_t*>(k_new), static_cast<const uint16_t*>(v_new), p.q, k_cache, v_cache, new_loc, req_to_token, req_pool_indices,
-                 q_token_stride, k_new_stride, v_new_stride, req_to_token_stride, p.group, p.scale_log2,
-                 kv_fp8 ? 1.0f / k_scale : 1.0f, kv_fp8 ? 1.0f / v_scale : 1.0f, p.fmt};
-  }
   const int64_t walkers = g_cascade_loop_grid > 0 ? g_cascade_loop_grid : kv_fp8 || head_dim == 64 ? kLoopGridSmallRows : kLoopGrid;
   dim3 grid(static_cast<unsigned>(loop && walkers < worst ? walkers : worst));
 #define SGL_LAUNCH_CASC2(D_, KERNEL_)                                                                                 \
@@ -1027,15 +895,9 @@ int sgl_amd_cascade_decode_attention_store(const void* q, void* k_cache, void* v
 #undef SGL_LAUNCH_CASC2
 #undef SGL_LAUNCH_CASC
   const int hpb = 256 / (head_dim / 4);
-  const dim3 merge_grid(static_cast<unsigned>(batch), (num_q_heads + hpb - 1) / hpb);
-  const int by_spans = loop && p.walks_spans ? 1 : 0;
-  const float out_scale = kv_fp8 ? v_scale : 1.0f;
-#define SGL_LAUNCH_MERGE(NEW_)                                                                                                               \
-  hipLaunchKernelGGL(cascade_merge2_kernel<NEW_>, merge_grid, dim3(256), 0, st, p.ws_acc, p.ws_ml, plan, seq_lens, by_spans,                 \
-                     static_cast<uint16_t*>(out), out_token_stride, p.batch, p.max_items, num_q_heads, head_dim, slots_total, out_scale, nr)
-  if (k_new != nullptr) SGL_LAUNCH_MERGE(true);
-  else SGL_LAUNCH_MERGE(false);
-#undef SGL_LAUNCH_MERGE
+  hipLaunchKernelGGL(cascade_merge2_kernel, dim3(static_cast<unsigned>(batch), (num_q_heads + hpb - 1) / hpb), dim3(256), 0, st,
+                     p.ws_acc, p.ws_ml, plan, seq_lens, loop && p.walks_spans ? 1 : 0, static_cast<uint16_t*>(out), out_token_stride, p.batch, p.max_items,
+                     num_q_heads, head_dim, slots_total, kv_fp8 ? v_scale : 1.0f);
   SGL_CHECK_LAUNCH("cascade_decode_attention");
   return 0;
 }

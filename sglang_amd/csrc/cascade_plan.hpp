@@ -9,8 +9,7 @@
 //   group_pool_row[B]    req_to_token row of the group's leader
 //   group_kvlen[B]       shared kv length of the group (multiple of the kv tile)
 //   items[8 * max_items] self-contained records: (group, kv chunk, row tile, members, first member_rows
-//                        index, kv tokens, req_to_token row of the leader, group; of a private item kHoldsLast where it ends in its request's
-//                        last token, else -1); members == 0: unused entry
+//                        index, kv tokens, req_to_token row of the leader, 0); members == 0: unused entry
 //   batch_order[B]       permutation of the batch: grouped requests (group by group) first, then the rest
 //   req_slots[B]         partial slots of request b: its shared chunks, then its private items or pieces
 //   span_first[kSpanUnits + 1], pieces[8 * (B + kSpanUnits)]   (header[4] > 0) span k is pieces span_first[k] .. span_first[k + 1] - 1, records like
@@ -35,9 +34,6 @@ struct CascadePlanView {
   int32_t* span_first;
   int32_t* pieces;
 };
-
-// what record field 7 of a private item says where the item ends in the last token of its request
-constexpr int kHoldsLast = -2;
 
 // (span, kv head) units that a plan of spans aims at, the shared items taken off: three a compute unit.  The looping kernel's registers would
 // let four run, but the chip starts about 740 of a thousand workgroups at once and the rest only as those end, a second round of a fifth of

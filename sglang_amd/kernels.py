@@ -504,10 +504,9 @@ def cascade_plan(ws: CascadeWorkspace, req_to_token: torch.Tensor, req_pool_indi
 def cascade_decode_attention(ws: CascadeWorkspace, q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                              out: torch.Tensor, req_to_token: torch.Tensor, req_pool_indices: torch.Tensor,
                              seq_lens: torch.Tensor, sm_scale: float, kv_fp8: bool = False, k_scale: float = 1.0,
-                             v_scale: float = 1.0, page_size: int = 1, hnd: bool = False, new_rows=None) -> torch.Tensor:
+                             v_scale: float = 1.0, page_size: int = 1, hnd: bool = False) -> torch.Tensor:
     """Per layer, after cascade_plan(): q/out [B, Hq, D]; pools as in decode_attention (bf16 or uint8 e4m3 rows,
-    [slots, Hkv, D] or [pages, Hkv, page_size, D] with hnd).  new_rows: (k, v, loc), the step's rows [B, Hkv, D] and their slots (int64 [B]),
-    stored as store_kv_cache would before."""
+    [slots, Hkv, D] or [pages, Hkv, page_size, D] with hnd)."""
     _dev(q, k_cache, v_cache, out)
     B, Hq, D = q.shape
     Hkv = k_cache.shape[1]
@@ -521,19 +520,11 @@ def cascade_decode_attention(ws: CascadeWorkspace, q: torch.Tensor, k_cache: tor
         _need(k_cache.stride(2) == 1 and k_cache.stride(1) == D and v_cache.stride(1) == D
               and k_cache.stride(0) == v_cache.stride(0), "cascade: cache layout")
         row = k_cache.stride(0)
-    kn, vn, loc, kns, vns = None, None, None, 0, 0
-    if new_rows is not None:
-        k, v, loc = new_rows
-        _dev(k, v, loc)
-        _need(k.dtype == _BF16 and v.dtype == _BF16 and loc.dtype == torch.int64 and loc.is_contiguous() and loc.numel() == B, "cascade: new rows")
-        for x in (k, v):
-            _need(x.shape == (B, Hkv, D) and x.stride(2) == 1 and (Hkv == 1 or x.stride(1) == D), "cascade: new rows [B, Hkv, D]")
-        kn, vn, loc, kns, vns = k.data_ptr(), v.data_ptr(), loc.data_ptr(), k.stride(0), v.stride(0)
-    native.call("sgl_amd_cascade_decode_attention_store", q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(),
+    native.call("sgl_amd_cascade_decode_attention_ex", q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(),
                 req_to_token.data_ptr(), req_to_token.stride(0), req_pool_indices.data_ptr(), seq_lens.data_ptr(),
                 ws.plan.data_ptr(), B, ws.max_items, Hq, Hkv, D, q.stride(0), out.stride(0), row, row,
                 float(sm_scale), ws.max_context_len, ws.slots, ws.ws_acc.data_ptr(), ws.ws_ml.data_ptr(),
-                1 if kv_fp8 else 0, float(k_scale), float(v_scale), int(page_size), 1 if hnd else 0, kn, vn, loc, kns, vns, _stream())
+                1 if kv_fp8 else 0, float(k_scale), float(v_scale), int(page_size), 1 if hnd else 0, _stream())
     return out
 
 

@@ -412,8 +412,8 @@ class HipAttnBackend(AttentionBackend):
         return out
 
     def _riding_rows(self, layer, forward_batch, k, v, tokens: int):
-        """(k, v, slots) of a step where the attention call can store them (new_rows of cascade_decode_attention and extend_attention), else None:
-        this package's pool with its own set_kv_buffer, `tokens` rows, bf16 and 16-byte aligned."""
+        """(k, v, slots) of a pass where the attention call can store them (new_rows of extend_attention), else None: this package's pool with
+        its own set_kv_buffer, `tokens` rows, bf16 and 16-byte aligned."""
         pool, loc = self.token_to_kv_pool, forward_batch.out_cache_loc
         if type(pool).set_kv_buffer is not MHATokenToKVPool.set_kv_buffer or "set_kv_buffer" in vars(pool):
             return None
@@ -430,21 +430,17 @@ class HipAttnBackend(AttentionBackend):
 
     def forward_decode(self, q, k, v, layer, forward_batch, save_kv_cache: bool = True, **kwargs):
         self._refuse_unsupported(layer, kwargs)
-        m = self.forward_metadata
-        opt = self._layer_options(layer)
-        cascade = m.cascade is not None and "sliding_window" not in opt and "logit_cap" not in opt
-        new_rows = None
         if save_kv_cache and k is not None and v is not None:
-            new_rows = self._riding_rows(layer, forward_batch, k, v, forward_batch.batch_size) if cascade else None
-            if new_rows is None:
-                self._save_kv(layer, forward_batch, k, v)
+            self._save_kv(layer, forward_batch, k, v)
+        m = self.forward_metadata
         q3 = q.reshape(-1, layer.tp_q_head_num, layer.qk_head_dim)
         o = torch.empty_like(q3)
-        if cascade:
+        opt = self._layer_options(layer)
+        if m.cascade is not None and "sliding_window" not in opt and "logit_cap" not in opt:
             kernels.cascade_decode_attention(m.cascade, q3, self.token_to_kv_pool.get_key_buffer(layer.layer_id),
                                              self.token_to_kv_pool.get_value_buffer(layer.layer_id), o,
                                              self.req_to_token_pool.req_to_token, self._pool_idx(forward_batch),
-                                             m.seq_lens_i32, layer.scaling, new_rows=new_rows, **opt)      # opt: the pool format, if any
+                                             m.seq_lens_i32, layer.scaling, **opt)      # opt: the pool format, if any
             return o.view(-1, layer.tp_q_head_num * layer.v_head_dim)
         kernels.decode_attention(q3, self.token_to_kv_pool.get_key_buffer(layer.layer_id),
                                  self.token_to_kv_pool.get_value_buffer(layer.layer_id), o,
