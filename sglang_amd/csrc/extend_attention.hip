@@ -897,6 +897,7 @@ struct WalkQueue {
   int first[kRequests], tiles[kRequests];           // levels [first, first + tiles)
   int q_begin[kRequests], len[kRequests], kv_len[kRequests], prefix[kRequests], row[kRequests];
   int below[kLevels];                               // tiles in front of the i-th level from the top
+  int all;                                          // tiles of the launch
 
   // every thread of the workgroup; returns the top level
   __device__ __forceinline__ int fill(const ExtendParams& p, int tid) {
@@ -946,7 +947,7 @@ struct WalkQueue {
     for (int w = 0; w < wid; ++w) front += sums[w];
     for (int i = 0; i < per; ++i)
       if (per * tid + i < kLevels) below[per * tid + i] += front;
-    if (tid == kThreads - 1) next = front + mine;   // all tiles
+    if (tid == kThreads - 1) all = front + mine;
     __syncthreads();
     return top;
   }
@@ -1033,7 +1034,7 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
   if constexpr (STAYS) {
     static_assert(64 * NWV == WalkQueue::kThreads && WalkQueue::kRequests == WalkQueue::kThreads, "one request a thread");
     top = queue->fill(p, tid);
-    all = __builtin_amdgcn_readfirstlane(queue->next);
+    all = __builtin_amdgcn_readfirstlane(queue->all);   // (not in `next`: a first tile without keys has no barrier in front of hand())
     if (static_cast<int>(blockIdx.x) >= all) return;
     queue->find(blockIdx.x, top, p.batch, p.num_kv_heads, lane, b, kvh, tile);
     of_queue(b, tile);

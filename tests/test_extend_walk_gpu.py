@@ -30,7 +30,18 @@ SHAPES = {
 @pytest.mark.parametrize("kv_fp8", [False, True])
 @pytest.mark.parametrize("name", list(SHAPES))
 def test_walked_extends_give_the_same_bits(name, kv_fp8, monkeypatch):
-    lens, pre, hq, hkv = SHAPES[name]
+    _walked_and_launched(name, *SHAPES[name], kv_fp8, monkeypatch)
+
+
+# Requests that have new tokens and no keys (their rows are zeros): the first tile that every workgroup takes (the longest prefixes stand first), tiles in the
+# middle of the list, behind one another and between others, and all of them.
+@pytest.mark.parametrize("kv_fp8", [False, True])
+@pytest.mark.parametrize("name,without", [("first", lambda i: i >= 44), ("middle", lambda i: 9 < i < 14), ("every other", lambda i: i % 2 == 0), ("all", lambda i: True)])
+def test_requests_without_keys(name, without, kv_fp8, monkeypatch):
+    _walked_and_launched(name, [100 + i for i in range(64)], [40 * i for i in range(64)], 32, 8, kv_fp8, monkeypatch, [i for i in range(64) if without(i)])
+
+
+def _walked_and_launched(name, lens, pre, hq, hkv, kv_fp8, monkeypatch, no_keys=()):
     d, b, t = 128, len(lens), sum(lens)
     g = torch.Generator(device="cuda")
     g.manual_seed(len(name))
@@ -49,7 +60,7 @@ def test_walked_extends_give_the_same_bits(name, kv_fp8, monkeypatch):
     qkv = torch.randn((t, (hq + 2 * hkv) * d), device="cuda", generator=g).to(BF)
     q, k, v = (x.reshape(t, -1, d) for x in qkv.split([hq * d, hkv * d, hkv * d], dim=-1))
     pool = [torch.randn((slots, hkv, d), device="cuda", generator=g).to(FP8 if kv_fp8 else BF) for _ in range(2)]
-    seq, prefix = (torch.tensor(x, dtype=torch.int32, device="cuda") for x in (total, pre))
+    seq, prefix = (torch.tensor(x, dtype=torch.int32, device="cuda") for x in ([0 if i in no_keys else n for i, n in enumerate(total)], pre))
     indptr = torch.tensor([0] + lens, dtype=torch.int32, device="cuda").cumsum(0, dtype=torch.int32)
     for causal in (True, False):
         outs, pools = [], []
@@ -71,3 +82,5 @@ def test_walked_extends_give_the_same_bits(name, kv_fp8, monkeypatch):
             pools.append((kc, vc))
         assert torch.equal(outs[0], outs[1]), (name, causal, (outs[0] != outs[1]).any(-1).any(-1).nonzero().flatten()[:8].tolist())
         assert all(torch.equal(a, c) for a, c in zip(*pools))
+        for i in no_keys:
+            assert not outs[0][sum(lens[:i]):sum(lens[:i + 1])].any()
