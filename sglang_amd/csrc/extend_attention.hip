@@ -1748,13 +1748,23 @@ bool extend_walks(int64_t tokens, int64_t batch, int64_t rows, int group, int kv
   if (rows / group > static_cast<int64_t>(256 / group) * WalkQueue::kLevels) return false;       // a request's tiles stand at levels of their own
   return extend_held(tokens, batch, group, kv_heads) > 256;
 }
-// Whether it pays.  Not while all contexts are about as long, where a step costs 3 % more than is saved between the tiles: us, launched / staying, by mean over
-// longest context: 0.98 to 1.0 549 / 539 .. 311 / 309, 0.91 (8 cold prompts of 1350 - 1650) 214 / 219, 0.91 (24 of 450 - 550, 64 heads) 240 / 228, 0.9 (20 extends
-// of 150 - 450 behind 1000) 344 / 314, 0.84 (4 of 2000 - 3400) 416 / 354, 0.67 (6 of 1.1 - 3.1 k) 662 / 606, 0.4 (12 of 60 - 3000 behind 10 - 6000) 1322 / 745,
-// 0.2 (60 of 200 behind 10 - 6000) 695 / 572.  Nor where walks are over before the next tile has arrived (eight key tiles and fewer), unless many rounds
-// leave something to balance: 16 x 237 cold 41 / 45, 40 x 237 83 / 86, 30 x 200 behind 300 91 / 99; 24 x 350 84 / 81, 36 x 380, 64 heads, 267 / 234.
-bool extend_ragged(int64_t held, int64_t batch, int64_t sum_kv_len, int max_kv_len) {
-  return sum_kv_len > 0 && sum_kv_len * 100 <= batch * max_kv_len * 92 && (max_kv_len >= 640 || (max_kv_len >= 400 && held >= 1024));
+// Whether it pays, from the sums that the caller has.  It saves the wait for a long context that a launch deals last, empty workgroups and hidden prologues;
+// it costs 3 % a step, and where walks are over before the next tile has arrived (eight key tiles and fewer) two barriers and a look at the list a tile.
+// So: never while all contexts are about as long (mean over longest above 0.92); where the longest prefix stands 512 keys and more above the mean one;
+// else where a CU walks key tiles enough to pay for the ends: 12, or 24 with less to balance (mean over longest above 0.7).  A
+// query head to a kv head, whose heads share no rows: only where the longest prefix stands apart by 1024 (without that -3 to +2 %).
+// us, launched / staying: 6 cold prompts of 1.1 - 3.1 k, 64 / 8 heads, 662 / 606, 12 of 60 - 3000 behind 10 - 6000 1322 / 745, 30 of 200 behind 10 - 1000 87 / 80,
+// 40 of 237 and 200 behind 1500 126 / 89, 24 of 140 - 560 93 / 83.  Launched: 30 of 200 behind 300 and a cold one of 700 111 / 115, 8 of 490 - 910, 32 / 32
+// heads, 113 / 119.  The lines cannot tell every batch: of 2400 drawn ones (3 to 90 requests of 60 to 1600 new tokens, cold, behind one prefix, behind
+// log-uniform ones, one long request among short ones; three in ten in e4m3) 3.4 % are slower than launched by more than 2 %, worst 0.89 (8.9 % and 0.79 with
+// lines on the longest context, at 640 and 400 tokens); over all of them launching takes 1.057 times as long.
+bool extend_ragged(int64_t held, int64_t batch, int64_t num_tokens, int64_t sum_kv_len, int max_extend_len, int max_kv_len, int group) {
+  const int64_t longest = batch * max_kv_len;
+  if (sum_kv_len <= 0 || sum_kv_len * 100 > longest * 92) return false;
+  const int64_t apart = longest - batch * max_extend_len - (sum_kv_len - num_tokens);            // times batch
+  const int64_t walked = held * (2 * sum_kv_len - num_tokens) / (batch * 2 * kKvTile * 256);      // key tiles a CU: the mean prefix and half of the mean extend
+  if (group == 1) return apart >= 1024 * batch;
+  return (apart >= 512 * batch && walked >= 8) || walked >= (sum_kv_len * 100 <= longest * 70 ? 12 : 24);
 }
 
 template <int D, bool FP8>
@@ -2068,7 +2078,7 @@ int sgl_amd_extend_attention_store_parts(int64_t batch, int64_t num_tokens, int6
   if (batch > 0 && max_extend_len > 0 && max_kv_len > kKvTile && num_kv_heads > 0 && num_q_heads % num_kv_heads == 0 && g_extend_debug_shape == 0 &&
       g_extend_debug_flags == 0) {
     const int group = num_q_heads / num_kv_heads;
-    if (extend_ragged(extend_held(num_tokens, batch, group, num_kv_heads), batch, sum_kv_len, max_kv_len) &&
+    if (extend_ragged(extend_held(num_tokens, batch, group, num_kv_heads), batch, num_tokens, sum_kv_len, max_extend_len, max_kv_len, group) &&
         extend_walks(num_tokens, batch, static_cast<int64_t>(max_extend_len) * group, group, num_kv_heads, head_dim)) return 0;
   }
   return sgl_amd_extend_attention_parts(batch, num_tokens, max_extend_len, max_kv_len, num_q_heads, num_kv_heads, head_dim);

@@ -16,6 +16,13 @@ from sglang_amd import native
     ([262144, 100], [0, 0], 32, 8, 128, True),
     ([262145, 100], [0, 0], 32, 8, 128, False),
     ([150 + i % 40 for i in range(512)], [7 * i for i in range(512)], 32, 8, 128, True),
+    # one request that stands out does not put a batch of short walks into the queue, a long prefix that would be dealt last does
+    ([200] * 30 + [700], [300] * 30 + [0], 32, 8, 128, False),
+    ([200] * 12 + [700], [200] * 12 + [0], 32, 8, 128, False),
+    ([200] * 31, [300] * 30 + [1500], 32, 8, 128, True),
+    ([237] * 40 + [200], [0] * 40 + [1500], 32, 8, 128, True),
+    ([700, 910, 500, 800, 600, 900, 490, 700], [0] * 8, 32, 32, 128, False),      # a query head to a kv head
+    ([150] * 16, [100] * 15 + [3000], 32, 32, 128, True),
 ])
 def test_rule(lens, pre, hq, hkv, d, stays):
     total = [p + n for p, n in zip(pre, lens)]
