@@ -75,9 +75,11 @@ __device__ __forceinline__ double gumbel_from_hash(uint32_t h) {
   return -log(-lx);
 }
 
-// A log p + gumbel in fp32, within kNear of the fp64 one: only elements within kNear of the largest of these can hold the largest score, and
-// the two fp64 logarithms of a score are most of what an element costs (1.5 k clocks a wave).  The noise that wins lies next to x = 1, where
-// -log(x) is taken from 1 - x (exact: the complement of the hash); the error of all of it is below 3e-4 for |log p| < 4096.
+// A log p + gumbel in fp32: only elements within kNear of the largest of these can hold the largest score, and the two fp64 logarithms of a score are most of
+// what an element costs (1.5 k clocks a wave).  kNear is more than twice the error.  The noise: it wins next to x = 1, where -log(x) is taken as y + y^2 / 2 of
+// y = 1 - x (the complement of the hash), y^2 / 3 < 8.2e-5 short of it at y = 1/64, in all below 1.1e-4.  log_near(): 1e-5 (the logarithm's last bit at 64).
+// The unfiltered kernel's v / t - (mx + log sum), |mx| < 4096 and log p > -87: 2.5e-4 from the reciprocal, 2.5e-4 from the rounded sum, and 2.5e-4 of the
+// quotient it stands for, together with the noise 8.7e-4.
 constexpr float kNear = 0.00390625f;
 constexpr float kLn2f = 0.69314718f;
 __device__ __forceinline__ float gumbel_near(uint32_t h) {
@@ -85,7 +87,7 @@ __device__ __forceinline__ float gumbel_near(uint32_t h) {
   const float x = y < 0.5f ? 1.0f - y : static_cast<float>(h) * 2.3283064e-10f;
   const float lx = y < 0.015625f ? __fmaf_rn(0.5f * y, y, y) : -kLn2f * __builtin_amdgcn_logf(x);
   const float g = -kLn2f * __builtin_amdgcn_logf(fmaxf(lx, 2.3283064e-10f));
-  return h == 0u ? -709.0f : g;
+  return h == 0u ? -709.7827f : g;                                   // -log(DBL_MAX)
 }
 __device__ __forceinline__ float log_near(float p) { return kLn2f * (__builtin_amdgcn_logf(p * 18446744073709551616.0f) - 64.0f); }
 
@@ -2110,13 +2112,7 @@ __global__ __launch_bounds__(kT) void sample_unfiltered_ranges_kernel(SamplePara
   }
 }
 
-__global__ __launch_bounds__(64) void sample_unfiltered_merge_kernel(SampleParams p, int splits, const PartialBest* __restrict__ partials) {
-  const int row = blockIdx.x, lane = threadIdx.x;
-  Best r{0.0, -1, 0};
-  if (lane < splits) {
-    const PartialBest o = partials[static_cast<int64_t>(row) * splits + lane];
-    r.score = o.score; r.rank = o.rank; r.token = o.token;
-  }
+__device__ __forceinline__ Best wave_best(Best r) {
   for (int off = 32; off > 0; off >>= 1) {
     Best o;
     o.score = __shfl_xor(r.score, off, 64);
@@ -2124,9 +2120,23 @@ __global__ __launch_bounds__(64) void sample_unfiltered_merge_kernel(SampleParam
     o.token = __shfl_xor(r.token, off, 64);
     if (best_better(r, o)) r = o;
   }
-  if (lane == 0) {
-    p.out_ids[row] = r.rank < 0 ? 0 : r.token;
-    if (p.out_n_keep) p.out_n_keep[row] = p.V;
+  return r;
+}
+
+__device__ __forceinline__ Best best_of_ranges(const PartialBest* partials, int row, int splits, int lane) {
+  Best r{0.0, -1, 0};
+  if (lane < splits) {
+    const PartialBest o = partials[static_cast<int64_t>(row) * splits + lane];
+    r.score = o.score; r.rank = o.rank; r.token = o.token;
+  }
+  return wave_best(r);
+}
+
+__global__ __launch_bounds__(64) void sample_unfiltered_merge_kernel(SampleParams p, int splits, const PartialBest* __restrict__ partials) {
+  const Best r = best_of_ranges(partials, blockIdx.x, splits, threadIdx.x);
+  if (threadIdx.x == 0) {
+    p.out_ids[blockIdx.x] = r.rank < 0 ? 0 : r.token;
+    if (p.out_n_keep) p.out_n_keep[blockIdx.x] = p.V;
   }
 }
 
@@ -2134,7 +2144,9 @@ __global__ __launch_bounds__(64) void sample_unfiltered_merge_kernel(SampleParam
 // Range partials of the softmax (a launch), then every range scores its columns and a wave a row takes the best range: the ids of the softmax's two
 // launches and the two above.  A column costs its quotient, its noise and two fp32 logarithms; only the columns that may hold a wave's best
 // (kNear) get the probability of the normalise launch and the score in fp64.  Rows whose softmax is not finite, or whose largest quotient is beyond
-// the fp32 estimate, score every column so.
+// the fp32 estimate, score every column so.  The estimate knows nothing of a probability below the least normal float, whose score is below -64; a row's
+// largest probability is no less than 1 / V, so that only one with hash 0 there (noise -709.8) can have such a best score: the wave that joins the ranges
+// scores it again, every column.
 // us, [1, 128256] / [16, 128256] / [100, 128256]: 38 / 45 / 129 in four launches, 20 / 20 / 53 now.
 template <typename IN>
 __global__ __launch_bounds__(kSplitThreads) void logit_partials_kernel(const IN* __restrict__ logits, const float* __restrict__ temperatures, int64_t vocab,
@@ -2151,6 +2163,21 @@ __global__ __launch_bounds__(kSplitThreads) void logit_partials_kernel(const IN*
   }
 }
 
+// One wave: merge_partials' arithmetic, the exponentials side by side (sample_finish_fast_kernel).
+__device__ __forceinline__ void softmax_of_ranges(const float* partials, int row, int splits, int lane, float& mx, float& sum) {
+  const float pm = lane < splits ? partials[(static_cast<int64_t>(row) * splits + lane) * 2] : -INFINITY;
+  float ps = lane < splits ? partials[(static_cast<int64_t>(row) * splits + lane) * 2 + 1] : 0.f;
+  ps = pm > -INFINITY ? ps : 0.f;
+  mx = wave_max(pm);
+  const float ex = pm > -INFINITY ? expf(pm - mx) : 0.f;
+  sum = 0.f;
+  for (int s2 = 0; s2 < splits; ++s2) {
+    const float es = __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(__float_as_uint(ex)), s2)));
+    const float ss = __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(__float_as_uint(ps)), s2)));
+    sum = __fmaf_rn(ss, es, sum);
+  }
+}
+
 template <typename IN>
 __global__ __launch_bounds__(kSplitThreads) void sample_logits_unfiltered_kernel(const IN* __restrict__ logits, int64_t row_stride,
                                                                                 const float* __restrict__ temperatures, const float* __restrict__ partials,
@@ -2162,18 +2189,9 @@ __global__ __launch_bounds__(kSplitThreads) void sample_logits_unfiltered_kernel
   const int row = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const IN* x = logits + static_cast<int64_t>(row) * row_stride;
   const float t = temperatures[row];
-  if (wid == 0) {                                      // merge_partials' arithmetic, the exponentials side by side (sample_finish_fast_kernel)
-    const float pm = lane < splits ? partials[(static_cast<int64_t>(row) * splits + lane) * 2] : -INFINITY;
-    float ps = lane < splits ? partials[(static_cast<int64_t>(row) * splits + lane) * 2 + 1] : 0.f;
-    ps = pm > -INFINITY ? ps : 0.f;
-    const float mx = wave_max(pm);
-    const float ex = pm > -INFINITY ? expf(pm - mx) : 0.f;
-    float sum = 0.f;
-    for (int s2 = 0; s2 < splits; ++s2) {
-      const float es = __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(__float_as_uint(ex)), s2)));
-      const float ss = __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(__float_as_uint(ps)), s2)));
-      sum = __fmaf_rn(ss, es, sum);
-    }
+  if (wid == 0) {
+    float mx, sum;
+    softmax_of_ranges(partials, row, splits, lane, mx, sum);
     if (lane == 0) { s_mx = mx; s_sum = sum; }
   }
   __syncthreads();
@@ -2220,13 +2238,7 @@ __global__ __launch_bounds__(kSplitThreads) void sample_logits_unfiltered_kernel
       if (i < e && (all || !(near[u] < cut))) score(v[u], i);
     }
   }
-  for (int off = 32; off > 0; off >>= 1) {
-    Best o;
-    o.score = __shfl_xor(best.score, off, 64);
-    o.rank = __shfl_xor(best.rank, off, 64);
-    o.token = __shfl_xor(best.token, off, 64);
-    if (best_better(best, o)) best = o;
-  }
+  best = wave_best(best);
   if (lane == 0) { w_score[wid] = best.score; w_tok[wid] = best.rank; }
   __syncthreads();
   if (tid == 0) {
@@ -2240,6 +2252,28 @@ __global__ __launch_bounds__(kSplitThreads) void sample_logits_unfiltered_kernel
     o.score = r.score; o.rank = r.rank; o.token = r.token;
     bests[static_cast<int64_t>(row) * splits + blockIdx.x] = o;
   }
+}
+
+template <typename IN>
+__global__ __launch_bounds__(64) void sample_logits_unfiltered_merge_kernel(SampleParams p, const IN* __restrict__ logits, int64_t row_stride,
+                                                                           const float* __restrict__ temperatures, const float* __restrict__ partials,
+                                                                           int splits, const PartialBest* __restrict__ bests) {
+  const int row = blockIdx.x, lane = threadIdx.x;
+  Best r = best_of_ranges(bests, row, splits, lane);
+  if (uniform(r.score < -64.0)) {
+    const IN* x = logits + static_cast<int64_t>(row) * row_stride;
+    const float t = temperatures[row];
+    float mx, sum;
+    softmax_of_ranges(partials, row, splits, lane, mx, sum);
+    const uint32_t hpre = murmur_prefix(static_cast<uint64_t>(p.seeds[row]), p.positions ? static_cast<uint32_t>(p.positions[row] & 0xffffffffll) : 0u);
+    r = Best{0.0, -1, 0};
+    for (int i = lane; i < p.V; i += 64) {
+      const Best c{static_cast<double>(logf(softmax_prob(ld1(x + i), t, mx, sum))) + gumbel_from_hash(murmur_hash32(hpre, static_cast<uint32_t>(i))), i, i};
+      if (best_better(r, c)) r = c;
+    }
+    r = wave_best(r);
+  }
+  if (lane == 0) p.out_ids[row] = r.rank < 0 ? 0 : r.token;
 }
 
 // rank-0 token of an empty nucleus must be the arg max of the row; handled by a tiny fix-up
@@ -2429,6 +2463,8 @@ int sgl_amd_sample_unfiltered_from_logits(const void* logits, int logits_is_bf16
   if (batch == 0) return 0;
   SampleParams p{};
   p.V = static_cast<int>(vocab);
+  p.seeds = seeds;
+  p.positions = positions;
   p.out_ids = out_ids;
   PartialBest* bests = static_cast<PartialBest*>(ws);
   float* partials = reinterpret_cast<float*>(bests + batch * num_splits);
@@ -2440,11 +2476,12 @@ int sgl_amd_sample_unfiltered_from_logits(const void* logits, int logits_is_bf16
                        num_splits, partials);                                                                                                 \
     hipLaunchKernelGGL(sample_logits_unfiltered_kernel<IN_>, grid, dim3(kSplitThreads), 0, as_stream(stream), x, logits_row_stride,            \
                        temperatures, partials, p.V, num_splits, seeds, positions, bests);                                                     \
+    hipLaunchKernelGGL(sample_logits_unfiltered_merge_kernel<IN_>, dim3(static_cast<unsigned>(batch)), dim3(64), 0, as_stream(stream), p, x,   \
+                       logits_row_stride, temperatures, partials, num_splits, bests);                                                         \
   } while (0)
   if (logits_is_bf16) SGL_LAUNCH_UNFILTERED(uint16_t);
   else SGL_LAUNCH_UNFILTERED(float);
 #undef SGL_LAUNCH_UNFILTERED
-  hipLaunchKernelGGL(sample_unfiltered_merge_kernel, dim3(static_cast<unsigned>(batch)), dim3(64), 0, as_stream(stream), p, num_splits, bests);
   SGL_CHECK_LAUNCH("sample_unfiltered_from_logits");
   return 0;
 }

@@ -160,3 +160,61 @@ def test_unfiltered_from_logits_equals_softmax_then_sample(device, B, V, fp32):
     assert torch.equal(lg.nan_to_num(7.0), before.nan_to_num(7.0))
     bad = (got != want).nonzero().flatten().tolist()
     assert not bad, [(r, int(got[r]), int(want[r])) for r in bad]
+
+
+def _seed_with_hash(col, want=0):
+    """The seed (its upper half and the position 0) whose hash of column `col` is `want`: every step of the hash can be undone."""
+    M = 0xffffffff
+    inv = lambda x: pow(x, -1, 1 << 32)
+    rotr = lambda x, r: (x >> r) | (x << (32 - r)) & M
+
+    def unshift(h, r):
+        x = h
+        for _ in range(32 // r + 1):
+            x = h ^ (x >> r)
+        return x
+
+    def scramble(k):
+        k = k * 0xCC9E2D51 & M
+        return ((k << 15 | k >> 17) & M) * 0x1B873593 & M
+
+    def unmix(h, k):                                              # h in front of mm_mix(h, k)
+        return rotr((h - 0xE6546B64) * inv(5) & M, 13) ^ scramble(k)
+
+    h = unshift(want, 16) * inv(0xC2B2AE35) & M
+    h = unshift(h, 13) * inv(0x85EBCA6B) & M
+    h = unmix(unmix(unmix(unshift(h, 16) ^ 16, col), 0), 0)       # column, position, upper half
+    k = rotr((h - 0xE6546B64) * inv(5) & M, 13)                    # scramble(lower half) ^ 0
+    return rotr(k * inv(0x1B873593) & M, 15) * inv(0xCC9E2D51) & M
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("below", [85, 97, 103, 120])
+def test_unfiltered_rows_whose_largest_probability_has_hash_0(device, fp32, below):
+    """Its noise is -709.8, so that a column of the far tail wins: probabilities below the least normal float, whole binades apart or zero."""
+    from sglang_amd import kernels as K
+
+    B, V = 48, 32000
+    g = torch.Generator().manual_seed(below)
+    lg = 30.0 - below + torch.randn((B, V), generator=g) * 2.0
+    top = torch.randint(0, V, (B,), generator=g)
+    lg[torch.arange(B), top] = 30.0
+    lg = lg.to(torch.bfloat16).to(device)
+    lg = lg.float() if fp32 else lg
+    seeds = torch.tensor([_seed_with_hash(int(c)) for c in top], device=device)
+    temps, pos = torch.ones((B, 1), device=device), torch.zeros(B, dtype=torch.int64, device=device)
+    probs = torch.empty((B, V), device=device)
+    ws = torch.empty(B * 64 * 2, device=device)
+    from sglang_amd import native
+    splits = min(64, 2048 // B, V // 512)
+    if fp32:
+        probs.copy_(lg)
+        native.call("sgl_amd_softmax_temperature_split", probs.data_ptr(), temps.data_ptr(), B, V, V, splits, ws.data_ptr(), K._stream())
+    else:
+        native.call("sgl_amd_softmax_temperature_split_bf16", lg.data_ptr(), probs.data_ptr(), temps.data_ptr(), B, V, V, V, splits, ws.data_ptr(), K._stream())
+    want = K.top_k_top_p_min_p_sample(probs, None, None, None, seeds, pos, filtered=False)
+    if below < 120:                                               # (of 120 all others are zero and the largest wins)
+        assert not bool((want.cpu() == top).any())
+    got = K.sample_unfiltered_from_logits(lg, temps, seeds, pos)
+    bad = (got != want).nonzero().flatten().tolist()
+    assert not bad, [(r, int(got[r]), int(want[r])) for r in bad]
