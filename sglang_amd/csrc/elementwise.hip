@@ -545,7 +545,7 @@ static int store_kv_any(const void* k, const void* v, void* k_cache, void* v_cac
                        static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v), k_cache, v_cache, loc, num_kv_heads,
                        head_dim, k_token_stride, v_token_stride, fmt, 1.0f / k_scale, 1.0f / v_scale, zero8);
   else
-    hipLaunchKernelGGL((store_kv_fmt_kernel<false, false>), dim3(num_tokens), dim3(threads), 0, as_stream(stream),
+    hipLaunchKernelGGL((zero8 ? store_kv_fmt_kernel<false, true> : store_kv_fmt_kernel<false, false>), dim3(num_tokens), dim3(threads), 0, as_stream(stream),
                        static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v), k_cache, v_cache, loc, num_kv_heads,
                        head_dim, k_token_stride, v_token_stride, fmt, 1.0f, 1.0f, zero8);
   SGL_CHECK_LAUNCH("store_kv_cache_ex");
