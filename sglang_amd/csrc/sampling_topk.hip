@@ -1860,10 +1860,8 @@ __global__ __launch_bounds__(kT) void sample_finish_fast_kernel(SampleParams p, 
   const bool by_row = uniform(s_broken || top_k <= 0 || s_acc == 0 || !(t > 0.f) || !(sum > 0.f) || !(sum < INFINITY) || !(mx > -INFINITY) || !(mx < INFINITY));
   const bool bad = by_row || uniform(s_acc >= kDirect);
   constexpr bool kKeyed = sizeof(IN) == 2;              // (a bf16 logit is its key)
-  const uint32_t topkey = s_top >> 16;
-  const uint32_t hpre = murmur_prefix(seed, spos);
-  if (top_k > p.V) top_k = p.V;
   if (!bad) {
+    if (top_k > p.V) top_k = p.V;
     const unsigned long long p_fix = top_p_fix_superset(top_p);
     bool have[2];
     uint32_t key16[2], pbits[2];
@@ -1882,6 +1880,7 @@ __global__ __launch_bounds__(kT) void sample_finish_fast_kernel(SampleParams p, 
     // join the elements the ranges left out: the frontier rises to the largest of them. ----
     uint32_t cutkey = 0;
     bool found_any = true;
+    const uint32_t topkey = s_top >> 16;
     int near_cut;
     {
       uint32_t bin[2];
@@ -2033,8 +2032,8 @@ __global__ __launch_bounds__(kT) void sample_finish_fast_kernel(SampleParams p, 
         finish_small_list(p, row, sm.cand_val, sm.cand_tok, sm.keys, sm.toks, n, top_k, top_p, p.min_ps != nullptr, min_p, s_part, s_log,
                           s_log_sorted, s_gumbel, has_front ? &fr : nullptr);
     } else if constexpr (kKeyed) {
-      const bool done = finish_by_keys<true>(p, row, nullptr, sm, topkey, t, mx, sum, top_k, top_p, p.min_ps != nullptr, min_p, hpre, keep, key16, tok, n,
-                                             has_front ? &fr : nullptr);
+      const bool done = finish_by_keys<true>(p, row, nullptr, sm, topkey, t, mx, sum, top_k, top_p, p.min_ps != nullptr, min_p, murmur_prefix(seed, spos), keep,
+                                             key16, tok, n, has_front ? &fr : nullptr);
       if (!done && tid == 0) s_unusable = 1;
     } else {
       sample_row(p, row, sm, n, has_front ? &fr : nullptr);
@@ -2047,8 +2046,8 @@ __global__ __launch_bounds__(kT) void sample_finish_fast_kernel(SampleParams p, 
   if constexpr (kKeyed) {
     const bool no[2] = {false, false};
     const uint32_t no_key[2] = {0u, 0u};
-    if (!by_row && finish_by_keys<false>(p, row, logits + static_cast<int64_t>(row) * logits_row_stride, sm, topkey, t, mx, sum, top_k, top_p,
-                                         p.min_ps != nullptr, min_p, hpre, no, no_key, tok, 0, nullptr))
+    if (!by_row && finish_by_keys<false>(p, row, logits + static_cast<int64_t>(row) * logits_row_stride, sm, s_top >> 16, t, mx, sum,
+                                         top_k < p.V ? top_k : p.V, top_p, p.min_ps != nullptr, min_p, murmur_prefix(seed, spos), no, no_key, tok, 0, nullptr))
       return;
     __syncthreads();
   }
