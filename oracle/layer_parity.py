@@ -29,7 +29,22 @@ class _Patch:
         self._saved.clear()
 
 
-def ulp_stats(got: torch.Tensor, ref: torch.Tensor) -> dict:
+def _whose_error(g2, r2, a, third) -> dict:
+    """Which rows and columns are beyond one ulp (first, last, how many), and, where `third(rows)` gives those rows of another evaluation (fp64 on the
+    CPU), which of the two sides is away from it: a record of one run then tells a tile of a product from a strip of rows, and the result from its reference."""
+    off = (a > 1).cpu()
+    rows, cols = off.any(1).nonzero().flatten(), off.any(0).nonzero().flatten()
+    out = dict(off=int(off.sum()), rows=[int(rows[0]), int(rows[-1]), len(rows)], cols=[int(cols[0]), int(cols[-1]), len(cols)])
+    if third is not None:
+        worst = off.sum(1).topk(min(8, off.shape[0])).indices.sort().values
+        t = third(worst.to(g2.device)).cpu().double()
+        unit = bf16_ulp(torch.maximum(t.abs(), t.pow(2).mean(-1, keepdim=True).sqrt()).float()).double()
+        away = {who: float(((x[worst.to(x.device)].cpu().double() - t) / unit).abs()[off[worst]].max()) for who, x in (("result", g2), ("reference", r2))}
+        out.update(rows_looked_at=worst.tolist(), ulps_from_fp64=away, odd=max(away, key=away.get))
+    return out
+
+
+def ulp_stats(got: torch.Tensor, ref: torch.Tensor, third=None) -> dict:
     got, ref = got.float(), ref.float()
     assert got.shape == ref.shape, (got.shape, ref.shape)
     g2, r2 = got.reshape(-1, got.shape[-1]), ref.reshape(-1, ref.shape[-1])
@@ -40,7 +55,9 @@ def ulp_stats(got: torch.Tensor, ref: torch.Tensor) -> dict:
     # the floored figures so that the floor's effect can be read off (elements that cancel towards zero carry the
     # absolute noise of the sum they came from and count as many "plain" ulps in ANY evaluation, the reference's own too)
     ap = ((g2 - r2) / bf16_ulp(r2)).abs()
-    return dict(n=int(a.numel()), frac_identical=float((g2 == r2).float().mean()), frac_within_1ulp=float((a <= 1).float().mean()),
+    within = float((a <= 1).float().mean())
+    more = dict(where=_whose_error(g2, r2, a, third)) if third is not None and (within < 0.999 or float(a.max()) > 3.0) else {}
+    return dict(more, n=int(a.numel()), frac_identical=float((g2 == r2).float().mean()), frac_within_1ulp=within,
                 frac_within_1ulp_plain_unit=float((ap <= 1).float().mean()), frac_within_2ulp_plain_unit=float((ap <= 2).float().mean()),
                 frac_within_2ulp=float((a <= 2).float().mean()), max_ulp=float(a.max()), mean_signed_ulp=float(e.mean()),
                 rms_ulp=float(e.pow(2).mean().sqrt()), max_abs=float((g2 - r2).abs().max()), ref_rms=float(r2.pow(2).mean().sqrt()))
@@ -158,12 +175,16 @@ def run_layer_parity(cfg, device, prompt_lens, monkeypatch, operator_surface=Fal
         fused = tag == "decode_fused"
         key = f"layer{i}.{tag}"
         bias = A.qkv_proj.bias.data if A.qkv_proj.bias is not None else None
+
+        def product(x, linear):                      # rows of x . W^T (+ b) in fp64, for a stage beyond its bars
+            return lambda rows: oo.linear64(x[rows], linear.weight.data, linear.bias.data if linear.bias is not None else None)
+
         # 1. qkv_proj -> rope -> KV-row store
         if fused:
             q = K.wstream_qkv_rope(lr["normed"].clone(), A.qkv_proj.weight.data, bias, positions, A.rotary_emb.cos_sin_cache,
                                    Hq, Hkv, D, kb, vb, loc)
         else:
-            stages[f"{key}.qkv_proj"] = ulp_stats(A.qkv_proj(lr["normed"].clone()), lr["qkv"])
+            stages[f"{key}.qkv_proj"] = ulp_stats(A.qkv_proj(lr["normed"].clone()), lr["qkv"], product(lr["normed"], A.qkv_proj))
             q, k, v = (t.contiguous() for t in lr["qkv"].split([Hq * D, Hkv * D, Hkv * D], dim=-1))
             A.rotary_emb(positions, q, k, fused_set_kv_buffer_arg=FusedSetKVBufferArg(value=v, k_buffer=kb, v_buffer=vb, cache_loc=loc))
         stages[f"{key}.rope_q"] = ulp_stats(q.reshape(T, Hq, D), lr["q_rot"].reshape(T, Hq, D))
@@ -182,7 +203,7 @@ def run_layer_parity(cfg, device, prompt_lens, monkeypatch, operator_surface=Fal
             stages[f"{key}.o_proj_add_norm"] = ulp_stats(K.unblock(x), lr["post_normed"])
             stages[f"{key}.o_proj_add_norm.residual"] = ulp_stats(res, lr["res_out"])
         else:
-            stages[f"{key}.o_proj"] = ulp_stats(A.o_proj(attn_in), lr["o_proj"])
+            stages[f"{key}.o_proj"] = ulp_stats(A.o_proj(attn_in), lr["o_proj"], product(attn_in, A.o_proj))
             x, res = layer.post_attention_layernorm(lr["o_proj"].clone(), lr["residual"].clone())
             stages[f"{key}.post_norm"] = ulp_stats(x, lr["post_normed"])
             stages[f"{key}.post_norm.residual"] = ulp_stats(res, lr["res_out"])
@@ -194,7 +215,8 @@ def run_layer_parity(cfg, device, prompt_lens, monkeypatch, operator_surface=Fal
             stages[f"{key}.experts"] = ulp_stats(out, lr["out"])
             return
         act = layer.mlp.gate_up_act(lr["post_normed"].clone(), out_blocked=fused)
-        stages[f"{key}.gate_up_silu"] = ulp_stats(K.unblock(act), lr["act"])
+        gate_up = product(lr["post_normed"], layer.mlp.gate_up_proj)
+        stages[f"{key}.gate_up_silu"] = ulp_stats(K.unblock(act), lr["act"], lambda rows: oo.silu_and_mul(gate_up(rows)))
         if fused:
             nxt = layer_rec(i + 1)
             norm = model.layers[i + 1].input_layernorm if nxt is not None else model.norm
@@ -203,7 +225,7 @@ def run_layer_parity(cfg, device, prompt_lens, monkeypatch, operator_surface=Fal
             stages[f"{key}.down_add_norm"] = ulp_stats(K.unblock(x), nxt["normed"] if nxt is not None else rec["final_normed"])
             stages[f"{key}.down_add_norm.residual"] = ulp_stats(res, nxt["residual"] if nxt is not None else rec["final_residual"])
         else:
-            stages[f"{key}.down_proj"] = ulp_stats(layer.mlp.down_proj(lr["act"].clone()), lr["out"])
+            stages[f"{key}.down_proj"] = ulp_stats(layer.mlp.down_proj(lr["act"].clone()), lr["out"], product(lr["act"], layer.mlp.down_proj))
 
     # ---- product layers fed with the oracle's inputs
     def wrap_layer(i, layer):

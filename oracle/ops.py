@@ -46,6 +46,12 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
     return F.silu(x[..., :d]) * x[..., d:]
 
 
+def linear64(x: torch.Tensor, weight: torch.Tensor, bias=None) -> torch.Tensor:
+    """F.linear in fp64 on the CPU (some rows of a product that two library calls disagree about)."""
+    y = x.cpu().double() @ weight.cpu().double().t()
+    return y if bias is None else y + bias.cpu().double()
+
+
 # ---------------------------------------------------------------- RoPE
 def rope_inv_freq(rotary_dim: int, base: float) -> torch.Tensor:
     """srt/layers/rotary_embedding/base.py:153-171 (_compute_inv_freq)."""

@@ -54,17 +54,17 @@ def _assert_bars(report, stages, noise, moe=False):
         # whose P is rounded to bf16 ahead of PV exactly like the reference's literal bf16 SDPA; >= 99.999 % for every
         # GEMM / norm / rope / activation stage, most of them bit-identical), none beyond 3 (a silu(gate) * up whose
         # gate flipped one rounding), no systematic sign
-        assert st["frac_within_1ulp"] >= 0.999, (k, st)
-        assert st["max_ulp"] <= 3.0, (k, st)
-        assert abs(st["mean_signed_ulp"]) < 0.01, (k, st)
+        assert st["frac_within_1ulp"] >= 0.999, f"{k}: {st}"
+        assert st["max_ulp"] <= 3.0, f"{k}: {st}"
+        assert abs(st["mean_signed_ulp"]) < 0.01, f"{k}: {st}"
         if not k.endswith(".attention"):
-            assert st["frac_identical"] >= 0.985, (k, st)
+            assert st["frac_identical"] >= 0.985, f"{k}: {st}"
     for k, st in report.items():
-        assert abs(st["mean_signed_ulp"]) < 0.05, (k, st)
+        assert abs(st["mean_signed_ulp"]) < 0.05, f"{k}: {st}"
         ref = noise[k]
-        assert st["rms_ulp"] <= 1.25 * ref["rms_ulp"] + 0.02, (k, st, ref)
-        assert st["max_ulp"] <= 1.5 * ref["max_ulp"] + 1.0, (k, st, ref)
-        assert st["frac_within_1ulp"] >= ref["frac_within_1ulp"] - 0.02, (k, st, ref)
+        assert st["rms_ulp"] <= 1.25 * ref["rms_ulp"] + 0.02, f"{k}: {st}, reference against itself: {ref}"
+        assert st["max_ulp"] <= 1.5 * ref["max_ulp"] + 1.0, f"{k}: {st}, reference against itself: {ref}"
+        assert st["frac_within_1ulp"] >= ref["frac_within_1ulp"] - 0.02, f"{k}: {st}, reference against itself: {ref}"
 
 
 SHAPES = {

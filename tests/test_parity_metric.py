@@ -40,3 +40,21 @@ def test_ulp_stats_counts_in_units_of_the_reference_value_floored_at_the_row_rms
     rms = float(ref2.float().pow(2).mean().sqrt())
     assert s2["max_ulp"] == abs(float(got2[0, 3].float() - ref2[0, 3].float())) / float(bf16_ulp(torch.tensor(rms)))
     assert s2["max_ulp"] < 0.02
+
+
+def test_a_stage_beyond_its_bars_says_where_and_whose():
+    """A mistake planted in one tile of the result, or of the reference: rows and columns of the tile, and the side that a third evaluation in fp64 disagrees with."""
+    from oracle import ops
+
+    g = torch.Generator().manual_seed(3)
+    x, w = torch.randn((96, 64), generator=g).to(BF), torch.randn((160, 64), generator=g).to(BF)
+    right = (x.double() @ w.double().t()).to(BF)
+    wrong = right.clone()
+    wrong[16:80, 32:128] = (x[16:80, :56].double() @ w[32:128, :56].double().t()).to(BF)       # a part of the sum left out
+    third = lambda rows: ops.linear64(x[rows], w)
+    for got, ref, odd in ((wrong, right, "result"), (right, wrong, "reference")):
+        s = ulp_stats(got, ref, third)["where"]
+        assert s["odd"] == odd and s["rows"] == [16, 79, 64] and s["cols"] == [32, 127, 96], s
+        assert s["ulps_from_fp64"][odd] > 3.0 and min(s["ulps_from_fp64"].values()) <= 0.5
+        assert all(16 <= r < 80 for r in s["rows_looked_at"])
+    assert "where" not in ulp_stats(right, right, third)
