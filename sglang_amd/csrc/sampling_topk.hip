@@ -1573,11 +1573,12 @@ __device__ __forceinline__ bool uniform(bool v) { return __builtin_amdgcn_readfi
 
 // The three rules and the arg-max of a row whose kept columns are too many for one wave, from the COUNTS of its keys.  A bf16 logit is its 16-bit
 // key, so the columns of a key have one probability and consecutive ranks: counts below the largest key, their prefix sums and one probability a
-// key are the sorted row, and a rank's score needs nothing else.  Nothing is sorted; the winner's token is the n-th of its key's columns.
+// key are the sorted row, and a rank's score needs nothing else.  Nothing is sorted; the winner's token is the n-th of the columns of its probability (logits
+// next to zero or far below the largest: several keys have one).
 //   LIST: the candidates in the threads' registers; else the whole row (a pass for the counts, one for the winner's key).
 //   kKeys keys below the largest (32 binades: every positive logit and more).
-// False, and nothing written, where that does not decide the row: the rules reach the frontier (LIST) or leave the keys counted, or two keys
-// have one probability (logits next to zero: their columns are ranked by token together).
+// False, and nothing written, where that does not decide the row: the rules reach the frontier (LIST) or leave the keys counted, or the winner's
+// probability may be that of columns that are not counted.
 // us of the whole call, [1, 128256] / [16, 128256], before and now, gaussian logits of deviation 2.5: top-p 0.9 alone 423 / 611 and 64 / 75, min-p 0.05
 // alone 303 / 326 and 33 / 42, top-k 200 49 / 58 and 32 / 40.  Before, one workgroup sorted the nucleus (some 10 k columns) in memory, or ranked the
 // list in a loop over it, and scored every rank in fp64.  What bounds it now: the counts' LDS atomics and the ranks' hashes of one workgroup a row.
@@ -1595,7 +1596,7 @@ __device__ bool finish_by_keys(const SampleParams& p, const int row, const uint1
   static_assert(kHistCopies * kHistStride >= kKeys && kCand >= kKeys && kKeys == 4 * kT, "four keys a thread");
   __syncthreads();
   for (int d = tid; d < kKeys; d += kT) cnt[d] = 0;
-  if (tid == 0) { sm.found_bin = 0x7fffffff; sm.c_above = 0x7fffffff; sm.done_all = 0; sm.n_keep = 0; }
+  if (tid == 0) { sm.found_bin = 0x7fffffff; sm.c_above = 0x7fffffff; sm.n_keep = 0; }
   __syncthreads();
   if constexpr (LIST) {
 #pragma unroll
@@ -1696,39 +1697,26 @@ __device__ bool finish_by_keys(const SampleParams& p, const int row, const uint1
     }
     return bin_of(q);
   };
-  auto walk = [&](auto&& f, auto&& crossed) __attribute__((always_inline)) {     // f(rank, key, probability) of every kept rank of the run
+  auto walk = [&](auto&& f) __attribute__((always_inline)) {           // f(rank, key, probability) of every kept rank of the run
     int b = first;
     for (int q = r0; q < r1; ++q) {
-      if (static_cast<int>(start[b] + cnt[b]) <= q) {
-        const int from = b;
-        b = next_bin(b, q);
-        crossed(from, b);
-      }
+      if (static_cast<int>(start[b] + cnt[b]) <= q) b = next_bin(b, q);
       const float pb = prob[b];
       const double incl = before[b] + static_cast<double>(q - static_cast<int>(start[b]) + 1) * static_cast<double>(pb);
       if (key_of(pb) >= min_key && exact_top_p_keep(incl, pb, top_p)) f(q, b, pb);
     }
-    return b;
   };
   if (r0 < r1) {
-    // columns of two keys with one probability would be ranked together: no key of the run may share its own with the one behind
-    auto compare = [&](int b, int next) __attribute__((always_inline)) { tied |= !(prob[next] < prob[b]); };
     first = bin_of(r0);
-    const int last = walk([&](int q, int b, float pb) __attribute__((always_inline)) {
+    walk([&](int q, int b, float pb) __attribute__((always_inline)) {
       ++kept;
       const float near = log_near(pb) + gumbel_near(murmur_hash32(hpre, static_cast<uint32_t>(q)));
       if (at < 0 || near > b1) { b2 = b1; b1 = near; at = q; }
       else b2 = fmaxf(b2, near);
-    }, compare);
-    const int end = static_cast<int>(start[last] + cnt[last]);
-    if (end <= r1 || r1 == n) {                                        // (else the next run compares)
-      if (end < total) compare(last, next_bin(last, end));
-      else tied |= LIST ? listed > total : total < p.V;
-    }
+    });
   }
-  if (tied) sm.done_all = 1;
-  const float top = block_max(b1, sm.red);                            // (its barriers cover done_all)
-  if (uniform(sm.done_all != 0)) return false;
+  const float top = block_max(b1, sm.red);                            // (its barriers stand behind the reads of the three words, those below in front of their use)
+  if (tid == 0) { sm.found_bin = 0x7fffffff; sm.c_above = -1; sm.n_eq_keep = 0; }
   Best best{0.0, -1, 0};
   auto score = [&](int q, int b, float pb) __attribute__((always_inline)) {
     const Best c2{log(static_cast<double>(pb)) + gumbel_from_hash(murmur_hash32(hpre, static_cast<uint32_t>(q))), q, b};
@@ -1741,7 +1729,7 @@ __device__ bool finish_by_keys(const SampleParams& p, const int row, const uint1
     } else {
       walk([&](int q, int b, float pb) __attribute__((always_inline)) {
         if (log_near(pb) + gumbel_near(murmur_hash32(hpre, static_cast<uint32_t>(q))) >= top - kNear) score(q, b, pb);
-      }, [](int, int) {});
+      });
     }
   }
   const int all_kept = static_cast<int>(block_sum(static_cast<float>(kept), sm.red) + 0.5f);   // (< 2^24: exact in fp32)
@@ -1750,17 +1738,23 @@ __device__ bool finish_by_keys(const SampleParams& p, const int row, const uint1
     if (tid == 0) { p.out_ids[row] = 0; if (p.out_n_keep) p.out_n_keep[row] = 0; }
     return true;
   }
-  // ---- the winner: the (rank - start)-th token of its key ----
-  const int members = static_cast<int>(cnt[best.token]), nth = best.rank - static_cast<int>(start[best.token]);
-  const uint32_t key = topkey - static_cast<uint32_t>(best.token);
-  if (uniform(members > kLdsKeep)) return false;
+  // ---- the winner: the (rank - start)-th token of the keys lo .. hi that have its probability ----
+  const float won = prob[best.token];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (c[j] && pr[j] == won) { atomicMin(&sm.found_bin, 4 * tid + j); atomicMax(&sm.c_above, 4 * tid + j); atomicAdd(&sm.n_eq_keep, static_cast<int>(c[j])); }
+  __syncthreads();
+  const int lo = __builtin_amdgcn_readfirstlane(sm.found_bin), hi = __builtin_amdgcn_readfirstlane(sm.c_above);
+  const int members = __builtin_amdgcn_readfirstlane(sm.n_eq_keep), nth = best.rank - static_cast<int>(start[lo]);
+  if (uniform(members > kLdsKeep || (static_cast<int>(start[hi] + cnt[hi]) == total && (LIST ? listed > total : total < p.V)))) return false;
+  const uint32_t key_most = topkey - static_cast<uint32_t>(lo), keys_less = static_cast<uint32_t>(hi - lo);
   if constexpr (LIST) {
 #pragma unroll
     for (int u = 0; u < 2; ++u)
-      if (keep[u] && key16[u] == key) sm.toks[atomicAdd(&sm.n_keep, 1)] = tok[u];
+      if (keep[u] && key_most - key16[u] <= keys_less) sm.toks[atomicAdd(&sm.n_keep, 1)] = tok[u];
   } else {
     auto find = [&](uint32_t bits, int i) __attribute__((always_inline)) {
-      if (order_hi16(bits) == key) sm.toks[atomicAdd(&sm.n_keep, 1)] = i;
+      if (key_most - order_hi16(bits) <= keys_less) sm.toks[atomicAdd(&sm.n_keep, 1)] = i;
     };
     const int V4 = p.V & ~3;
     for (int i0 = 4 * tid; i0 < V4; i0 += 16 * kT) {

@@ -136,6 +136,27 @@ def test_rows_decided_by_their_keys_equal_softmax_then_sample(device, B, V, top_
     assert not bad, [(r, int(got[r]), int(want[r]), int(got_n[r]), int(want_n[r])) for r in bad]
 
 
+@pytest.mark.parametrize("top_k", [100, 300, 700])
+@pytest.mark.parametrize("V", [33000, 65536])
+def test_kept_columns_of_one_probability_are_decided_from_their_counts(device, V, top_k):
+    """Peaked rows that keep columns of many keys whose probabilities are all zero: nothing is sorted in memory."""
+    from sglang_amd import kernels as K
+
+    B, g = 32, torch.Generator(device=device).manual_seed(V + top_k)
+    lg = (torch.randn((B, V), generator=g, device=device) * 6.0).to(torch.bfloat16)
+    temps, pos = torch.linspace(0.03, 0.12, B, device=device)[:, None], torch.arange(B, device=device)
+    args = (torch.full((B,), top_k, dtype=torch.int32, device=device), None, None, pos * 31, pos)
+    probs = K.softmax_temperature_from_bf16(lg, temps)
+    assert bool(((probs > 0).sum(-1) < top_k).any())
+    want, want_n = K.top_k_top_p_min_p_sample(probs, *args, return_n_keep=True)
+    K.sample_from_logits(lg, temps, *args)
+    scratch = K._SAMPLE_WS["from_logits", B, V, 64, str(lg.device)][1]               # rows that go the long way are written here as probabilities
+    scratch.fill_(-1.0)
+    got, got_n = K.sample_from_logits(lg, temps, *args, return_n_keep=True)
+    assert torch.equal(got, want) and torch.equal(got_n, want_n)
+    assert bool((scratch == -1.0).all()), (scratch != -1.0).any(-1).nonzero().flatten().tolist()
+
+
 @pytest.mark.parametrize("B,V", [(1, 128256), (12, 32000), (33, 50257), (100, 151936), (128, 40002), (700, 33000), (3, 1025)])
 @pytest.mark.parametrize("fp32", [False, True])
 def test_unfiltered_from_logits_equals_softmax_then_sample(device, B, V, fp32):
