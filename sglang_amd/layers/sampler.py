@@ -58,6 +58,15 @@ class LogitsProcessorOutput:
 served = {"one_call_from_logits": 0, "softmax_then_sample": 0}
 
 
+def any_ranges(logits: torch.Tensor, need_top_k: bool) -> bool:
+    """Whether batches whose softmax has an odd number of ranges take the one call too (kernels.sample_from_logits).  Not where many rows end on its long way,
+    one workgroup a row, which the two calls are ahead of: nuclei without a top-k in rows of less than 16384 columns (us, two calls / one, flat bf16 rows:
+    [5, 4096] top-p 0.9 74 / 115, [128, 4096] min-p 0.05 82 / 133; from 16384 on 5 to 10 % where flat, one half to one seventh else), in fp32 rows of any width
+    ([33, 64000] min-p 0.05 112 / 372, [40, 128256] top-p 0.9 419 / 465), whose lists alone decide them, and top-k in short fp32 rows ([256, 2048] top-k 300 58 / 118)."""
+    wide = logits.shape[-1] >= 16384
+    return (need_top_k and wide) if logits.dtype == torch.float32 else (need_top_k or wide)
+
+
 class Sampler(nn.Module):
     """sampler.py:71-300.  Dtypes follow the reference: greedy ids are int64 (torch.argmax, :139), sampled ids
     int32 (sampling_from_probs_torch / the torch top-k/top-p path).  Unseeded sampling draws one fresh 62-bit seed
@@ -94,9 +103,10 @@ class Sampler(nn.Module):
                 # sampling; otherwise bf16 logits are widened inside the softmax launches (exact; no separate pass)
                 if not simple_sampling_case:
                     ids = kernels.sample_from_logits(logits, sampling_info.temperatures, sampling_info.top_ks, sampling_info.top_ps,
-                                                     min_ps, sampling_info.sampling_seed, positions, any_ranges=True)
+                                                     min_ps, sampling_info.sampling_seed, positions,
+                                                     any_ranges=any_ranges(logits, sampling_info.need_top_k_sampling))
                     served["one_call_from_logits" if ids is not None else "softmax_then_sample"] += 1
-                else:
+                elif logits.dtype == torch.bfloat16 or logits.shape[-1] >= 8192:        # (short fp32 rows: 23 us in two calls, 23 to 26 in one)
                     ids = kernels.sample_unfiltered_from_logits(logits, sampling_info.temperatures, sampling_info.sampling_seed, positions)
                 if ids is None and logits.dtype == torch.bfloat16:
                     probs = kernels.softmax_temperature_from_bf16(logits, sampling_info.temperatures)
