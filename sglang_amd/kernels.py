@@ -706,7 +706,7 @@ def sample_from_logits(logits: torch.Tensor, temperatures: torch.Tensor, top_ks:
     """sampler.py:211-260 for the logits of a decode-sized batch -- bf16 (the model's dtype) or fp32 (what the reference's
     LogitsProcessor hands its Sampler) -- in one native call: softmax(logits / T) + the filtered sampler, the probabilities never
     written and the logits left as they are (sampling_topk.hip: candidates / finish; rows the candidates cannot decide are redone
-    from their full probability row inside the finish launch).  Same ids and kept counts as softmax_temperature_{,from_bf16} +
+    from their full probability row inside the finish launch).  Same ids and kept counts as softmax_temperature_split{,_bf16} over the same ranges +
     top_k_top_p_min_p_sample.  None when the shape is not that case (the caller takes the two calls).  any_ranges: also range counts beyond 16 that
     are no multiple of it (40 rows: 51), and rows too short for 64 of them (32000 columns: 62, where the two calls take one workgroup a row)."""
     _dev(logits, temperatures)
@@ -757,9 +757,9 @@ def sample_from_logits(logits: torch.Tensor, temperatures: torch.Tensor, top_ks:
 
 def sample_unfiltered_from_logits(logits: torch.Tensor, temperatures: torch.Tensor, sampling_seed: Optional[torch.Tensor],
                                   positions: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
-    """sampler.py:211-216, 732-750 for the logits (bf16 or fp32) of a decode-sized batch: the ids of softmax_temperature_{,from_bf16} +
-    top_k_top_p_min_p_sample(filtered=False), the probabilities never written and the logits left as they are.  None when the shape is not that
-    case (the caller takes the two calls)."""
+    """sampler.py:211-216, 732-750 for the logits (bf16 or fp32) of a decode-sized batch: the ids of softmax_temperature_split{,_bf16} over the same ranges +
+    top_k_top_p_min_p_sample(filtered=False), the probabilities never written and the logits left as they are (softmax_temperature_ takes one workgroup
+    a row for some of these shapes: another order of the row's sum).  None when the shape is not that case (the caller takes the two calls)."""
     _dev(logits, temperatures)
     if logits.dtype not in (_BF16, torch.float32) or logits.dim() != 2 or logits.stride(1) != 1:
         return None
@@ -2105,6 +2105,7 @@ def routed_experts(h: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, ids: to
     inter = torch.empty((numel, N), dtype=_BF16, device=h.device)
     down = torch.empty((numel, W), dtype=_BF16, device=h.device)
     if _row_tiled(numel, E, N) and W % 64 == 0 and N % 64 == 0:
+        # (not moe_tiles: its line for half tiles was measured on fused_experts' shapes alone)
         block_m, up_rows, down_rows = moe_tile_plan(numel, E, N, W) if MOE_TILE_OVERRIDE is None else MOE_TILE_OVERRIDE
         s = moe_align_block_size(ids, block_m, E)
         moe_tiled_gemm(h, w13, inter, *s, None, False, top, numel, block_m, fuse_silu=act.gated, tile_rows=up_rows, act=act)
