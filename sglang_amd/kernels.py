@@ -448,7 +448,7 @@ def _extend_attention_kv(q, out, k_cache, v_cache, req_to_token, req_pool_indice
         shape = (int(max_extend_len), int(max_kv_len), Hq, Hkv, D)
         parts = (native.lib().sgl_amd_extend_attention_parts(B, T, *shape) if new_rows is None
                  else native.lib().sgl_amd_extend_attention_store_parts(B, T, int(sum_kv_len), *shape))
-    # (0 parts: workgroups that stay, eight counters)
+    # (0 parts: workgroups that stay, eight counters, zeroed by the store's launch: only where there are new rows)
     ws = torch.empty(parts * T * Hq * (D + 2) or 8, dtype=torch.float32, device=q.device) if parts != 1 else None
     acc = ws.data_ptr() if parts != 1 else None
     args = (q.data_ptr(), out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), req_to_token.data_ptr(),
