@@ -867,12 +867,27 @@ __global__ __launch_bounds__(512, 2) void extend_attention_dbuf_kernel(ExtendPar
 // two-workgroups-per-CU variant (slower again: twice the row requests per flop) were measured and dropped.
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
-template <int D>
+// (FP8: rows that are widened on their way in, written by the threads: V in one sub-image per 32 head dims with a bank skew between them)
+template <int D, bool FP8>
 struct SmemLadder {
   static constexpr int kVSub = 64 * 64 + (D == 128 ? 64 : 128);   // bytes of one 32-dim V sub-image + bank skew
-  U4 k[2][kKvTile * D / 8];                                       // [token][chunk ^ swz]
-  U4 v[2][(D / 32) * kVSub / 16];
+  U4 k[2][kKvTile * D / 8];                                       // [token][chunk ^ k_swz]
+  U4 v[2][FP8 ? (D / 32) * kVSub / 16 : kKvTile * D / 8];         // [dims / 32][token][chunk] or [token][chunk ^ v_swz]
+  // The scores' operand: 16 consecutive tokens at one chunk cover all chunk slots of the 256 bytes of banks.
+  __device__ __forceinline__ static int k_swz(int row) { return (row * (D / 8) / 16) & (D / 8 - 1); }
+  // The values' operand: four consecutive tokens at 64 bytes each (a transposing read of half a wave) cover the banks once.
+  __device__ __forceinline__ static int v_swz(int row) { return D == 128 ? (row & 3) << 2 : (row & 2) << 1; }
 };
+
+// 16 bytes a lane from memory to 1 KiB of LDS at `to`, behind the compiler's back: it would wait for all of these in front of the next read
+// of LDS.  Whoever issues them waits (rows_landed) and meets the others at a barrier before any of it is read.  No registers are written, and
+// nothing else here uses M0.  Rows that went through registers cost a step 300 of its 3900 clocks: all waves write LDS behind the barrier while
+// no product runs.  us, through registers / straight to LDS: 60 x 128 behind 896, 32 / 8 heads, 166 / 162, six cold prompts of 1.1 to 3.1 k, 64 / 8
+// heads, 619 / 603 (both at a lower clock in turn: power), 6 x 2000 cold, 14 / 2 heads of 64, 79 / 68, 1000 cold 26.0 / 23.5, 203 behind 3800 35.2 / 33.2.
+__device__ __forceinline__ void rows_to_lds(const unsigned char* from, uint32_t to) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(from), "s"(to) : "memory");
+}
+__device__ __forceinline__ void rows_landed() { asm volatile("s_waitcnt vmcnt(0)" : : : "memory"); }
 
 __device__ __forceinline__ float lane_pair_max(float x) {         // max over lanes l and l ^ 32
   float a = x, b = x;
@@ -986,19 +1001,21 @@ struct WalkQueue {
 //     then the rescale decision for tile t + 1 (everything exponentiated against the old maximum -- P(t) -- is inside
 //     O and l by then), and ONE barrier.
 // Every product carries <= 7 vector instructions, none of them waiting for the product next to it; what is left outside
-// the products' shadow is the decision (a permlane, two ballots), four LDS writes and the barrier.
+// the products' shadow is the decision (a permlane, two ballots), with e4m3 rows four LDS writes, and the barrier.
 // FP8: the pool holds e4m3 rows (8 bytes per lane and chunk, held raw in the staging registers, widened to bf16 -- exact --
 // on their way into the LDS images; k_scale rides in the softmax scale, v_scale in the epilogue).
 // PARTS: the walk covers part `part` of p.parts equal pieces of the request's key tiles (extend_attention_parts_kernel below).
 // STAYS: the workgroup takes query tiles from the queue until there are none (extend_attention_walk_kernel below).
 template <int D, int NWV, bool FP8, bool PARTS, bool STAYS = false>
-__device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadder<D>& sm, WalkQueue* queue = nullptr) {
+__device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadder<D, FP8>& sm, WalkQueue* queue = nullptr) {
   constexpr int CPR = D / 8;            // 16-byte chunks per KV row
   constexpr int KS = D / 16;            // MFMA k-steps over the head dim
   constexpr int ND = D / 32;            // 32-wide output blocks over the head dim
   constexpr int ROWS_PER_PASS = 64 * NWV / CPR;
   constexpr int LOADS = kKvTile / ROWS_PER_PASS;     // 16-byte loads per thread per operand per tile (2 at D = 128, 8 waves)
-  constexpr int VSUB = SmemLadder<D>::kVSub;
+  typedef SmemLadder<D, FP8> Lds;
+  constexpr bool DMA = !FP8;                         // rows go from memory to LDS as they are (rows_to_lds)
+  static_assert(ROWS_PER_PASS % 16 == 0 && (64 * NWV) % CPR == 0, "a thread's rows share their swizzles");
   constexpr int NPV = ND * 4;           // PV products per tile
 
   // (STAYS: formed anew for each query tile, as is what only the passage from tile to tile needs: kept across the outer loop, all the addresses
@@ -1153,7 +1170,7 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
 
   // ---- staging: thread = (row st_r + ROWS_PER_PASS i, 16-byte chunk st_c) of a K tile and of a V tile ----
   int st_c, st_r;
-  int32_t idx_k[LOADS], idx_v[LOADS];
+  int32_t idx_k[LOADS], idx_v[LOADS], idx_n[LOADS];
   typedef typename std::conditional<FP8, uint2, U4>::type Stage;   // a gathered 8-dim piece as it travels: raw bytes
   Stage kst[LOADS], vst[LOADS];
   auto ld_stage = [&](const unsigned char* ptr) __attribute__((always_inline)) -> Stage {
@@ -1173,26 +1190,43 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
       dst[i] = idx_base[tok];
     }
   };
-  // V^T operand reads: lane i of 16-lane group g points at token row 4 (g >> 1) + (i >> 2), dims 16 (g & 1) + 4 (i & 3)
-  int v_lane;
+  // V^T operand reads: lane i of 16-lane group g points at token row 4 (g >> 1) + (i >> 2), dims 16 (g & 1) + 4 (i & 3) of a 32-dim block
+  int v_lane[DMA ? ND : 1];
+  uint32_t to_lds = 0;                              // the wave's 1 KiB of a pass, from the images' start
+  auto v_lanes = [&]() __attribute__((always_inline)) {
+    const int r = 4 * hi + ((lane & 15) >> 2), in = ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
+    if constexpr (DMA) {
+#pragma unroll
+      for (int n = 0; n < ND; ++n) v_lane[n] = r * (2 * D) + (((4 * n) ^ Lds::v_swz(r)) << 4) + in;
+    } else {
+      v_lane[0] = r * 64 + in;
+    }
+  };
+  auto pieces = [&]() __attribute__((always_inline)) {
+    st_c = tid % CPR;
+    st_r = tid / CPR;
+  };
   auto staging = [&]() __attribute__((always_inline)) {
-    if constexpr (STAYS) lanes();
-    st_c = tid % CPR;
-    st_r = tid / CPR;
-    v_lane = (4 * hi + ((lane & 15) >> 2)) * 64 + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
+    if constexpr (STAYS) {
+      lanes();
+      pieces();
+    }
+    v_lanes();
+    to_lds = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(wid)) * 1024u;
   };
-  if constexpr (STAYS) {
-    staging();
-  } else {
-    st_c = tid % CPR;
-    st_r = tid / CPR;
-  }
-  auto head_rows = [&](const uint16_t* cache, int head) __attribute__((always_inline)) {
-    return reinterpret_cast<const unsigned char*>(cache) + static_cast<uint64_t>(head) * p.fmt.head_stride + st_c * (FP8 ? 8 : 16);
+  if constexpr (STAYS) staging();
+  else pieces();
+  auto head_rows = [&](const uint16_t* cache, int head, int c) __attribute__((always_inline)) {
+    return reinterpret_cast<const unsigned char*>(cache) + static_cast<uint64_t>(head) * p.fmt.head_stride + c * (FP8 ? 8 : 16);
   };
-  const unsigned char* k_rows = head_rows(p.k_cache, kvh);
-  const unsigned char* v_rows = head_rows(p.v_cache, kvh);
-  if constexpr (!STAYS) v_lane = (4 * hi + ((lane & 15) >> 2)) * 64 + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
+  // (DMA: a thread writes chunk slot st_c of its rows, so that it fetches the chunk that belongs there)
+  const unsigned char *k_rows, *v_rows;
+  auto rows_of = [&](int head) __attribute__((always_inline)) {
+    k_rows = head_rows(p.k_cache, head, DMA ? st_c ^ Lds::k_swz(st_r) : st_c);
+    v_rows = head_rows(p.v_cache, head, DMA ? st_c ^ Lds::v_swz(st_r) : st_c);
+  };
+  rows_of(kvh);
+  if constexpr (!STAYS) staging();
 
   // (STAYS: a stride widened in front of the outer loop would be multiplied in 64 x 32 bits, two quarter-rate instructions a row for one)
   auto row_stride = [&]() __attribute__((always_inline)) {
@@ -1208,30 +1242,45 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
       const int row = st_r + ROWS_PER_PASS * i;
-      sm.k[buf][row * CPR + (st_c ^ ((row * CPR / 16) & (CPR - 1)))] = widen(src[i]);
+      sm.k[buf][row * CPR + (st_c ^ Lds::k_swz(row))] = widen(src[i]);
     }
   };
   auto put_v = [&](int buf, const Stage (&src)[LOADS]) __attribute__((always_inline)) {
-    unsigned char* base = reinterpret_cast<unsigned char*>(sm.v[buf]) + (st_c >> 2) * VSUB + (st_c & 3) * 16;
+    unsigned char* base = reinterpret_cast<unsigned char*>(sm.v[buf]) + (DMA ? (st_c ^ Lds::v_swz(st_r)) * 16 : (st_c >> 2) * Lds::kVSub + (st_c & 3) * 16);
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) *reinterpret_cast<U4*>(base + (st_r + ROWS_PER_PASS * i) * 64) = widen(src[i]);
+    for (int i = 0; i < LOADS; ++i) *reinterpret_cast<U4*>(base + (st_r + ROWS_PER_PASS * i) * (DMA ? 2 * D : 64)) = widen(src[i]);
+  };
+  // (behind rows_landed(): the compiler takes ids to be on their way still, and would wait in the next step for what that has asked for since)
+  auto held_ids = [&](int32_t (&ids)[LOADS]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) asm volatile("" : "+v"(ids[i]));
+  };
+  // piece i of the rows `ids` of one image, asked for
+  auto send = [&](const unsigned char* base, int32_t id, const U4* image, int i) __attribute__((always_inline)) {
+    typedef __attribute__((address_space(3))) const U4* lds_t;
+    uint32_t wave = to_lds;
+    if constexpr (STAYS) asm volatile("" : "+s"(wave));
+    rows_to_lds(base + static_cast<uint64_t>(static_cast<uint32_t>(id)) * row_stride(),
+                static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_t)(image))) + wave + i * (64 * NWV * 16));
   };
   // ---- prologue: K(0), K(1), V(0) go to LDS in one round trip; K(2) and V(1) are asked for; ids of tiles 2 / 3 held.
+  // (DMA: a step asks for V(t + 1) and K(t + 2) itself, the ids of tiles 1 / 2 are held.)
   // (Tiles behind the end of the walk: load_idx clamps to the walk's last row, nobody reads those images.) ----------
   // STAYS: the next query tile's rows (kst, k1st, vst) and queries are asked for while this one is walked.
   int32_t id1[LOADS];
   Stage k1st[LOADS];
   auto first_rows = [&](int head, int64_t q_at, int q_len) __attribute__((always_inline)) {      // (queue->ids holds the slots)
-    const unsigned char* kr = head_rows(p.k_cache, head);
-    const unsigned char* vr = head_rows(p.v_cache, head);
+    const int c = thread() % CPR;
+    const unsigned char* kr = head_rows(p.k_cache, head, c);
+    const unsigned char* vr = head_rows(p.v_cache, head, c);
     int32_t id0[LOADS];
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
       const int32_t* ids = queue->ids + thread() / CPR + ROWS_PER_PASS * i;
       id0[i] = ids[0];
       id1[i] = ids[kKvTile];
-      idx_v[i] = ids[2 * kKvTile];
-      idx_k[i] = ids[3 * kKvTile];
+      (DMA ? idx_k : idx_v)[i] = ids[2 * kKvTile];
+      if constexpr (!DMA) idx_k[i] = ids[3 * kKvTile];
     }
     load_rows(kr, id0, kst);
     load_rows(kr, id1, k1st);
@@ -1242,7 +1291,22 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
 #pragma unroll
     for (int s = 0; s < KS; ++s) qreg[s] = ld16(qp + s * 16);
   };
-  if constexpr (!STAYS) {
+  if constexpr (!STAYS && DMA) {
+    int32_t id0[LOADS];
+    load_idx(0, id0);
+    load_idx(1, idx_v);
+    load_idx(2, idx_k);
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) send(k_rows, id0[i], sm.k[0], i);
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) send(k_rows, idx_v[i], sm.k[1], i);
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) send(v_rows, id0[i], sm.v[0], i);
+    rows_landed();
+    held_ids(idx_v);
+    held_ids(idx_k);
+    __syncthreads();
+  } else if constexpr (!STAYS) {
     Stage k0[LOADS], v0[LOADS];
     int32_t id0[LOADS];
     load_idx(0, id0);
@@ -1335,13 +1399,18 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
     }
     staging();
     if (n_tiles < 9) take();                         // too few steps to hide it all
-    k_rows = head_rows(p.k_cache, kvh);
-    v_rows = head_rows(p.v_cache, kvh);
+    rows_of(kvh);
     put_k(0, kst);
     put_k(1, k1st);
     put_v(0, vst);
-    load_rows(k_rows, idx_v, kst);
-    load_rows(v_rows, id1, vst);
+    if constexpr (DMA) {
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) idx_v[i] = id1[i];
+      held_ids(idx_k);
+    } else {
+      load_rows(k_rows, idx_v, kst);
+      load_rows(v_rows, id1, vst);
+    }
     __syncthreads();
   }
   if constexpr (STAYS) fresh();
@@ -1357,7 +1426,7 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
 
   auto read_k = [&](const U4* kimg, int i) __attribute__((always_inline)) {   // product i = (block i & 1, k-step i >> 1)
     const int row = (i & 1) * 32 + l31;
-    return kimg[row * CPR + ((2 * (i >> 1) + hi) ^ ((row * CPR / 16) & (CPR - 1)))];
+    return kimg[row * CPR + ((2 * (i >> 1) + hi) ^ Lds::k_swz(row))];
   };
   // mask (when the tile needs it), the row maximum of the lane pair, and the rescale decision for tile t: m_run, l_run
   // and O move to the new maximum together.  `links_done`: the in-lane maxima of registers 4..15 are in m4 already.
@@ -1425,7 +1494,7 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
     // (Between the phases instead, with the requests beside the phase-2 products: same time per tile, the wait moves
     // with the writes; and the registers no longer fit.)
     // (STAYS: in the last step kst and vst hold the next query tile's rows)
-    if constexpr (!STAYS || HAVE_NEXT) {
+    if constexpr (!DMA && (!STAYS || HAVE_NEXT)) {
       put_k(t & 1, kst);
       put_v((t + 1) & 1, vst);
     }
@@ -1447,7 +1516,16 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
       constexpr int RSTRIDE = G1 / NREQ > 0 ? G1 / NREQ : 1;
       static_assert(NREQ * RSTRIDE <= G1, "requests fit the products of phase 1");
       auto request = [&](int j) __attribute__((always_inline)) {
-        if (j < LOADS) {
+        if constexpr (DMA) {                            // ids of tile t + 3, V(t + 1), K(t + 2): landed in front of the barrier
+          if (j < LOADS) {
+            const int last = kv_end - 1, tok = (t + 3) * kKvTile + st_r + ROWS_PER_PASS * j;
+            idx_n[j] = idx_base[tok > last ? last : tok];
+          } else if (j < 2 * LOADS) {
+            send(v_rows, idx_v[j - LOADS], sm.v[(t + 1) & 1], j - LOADS);
+          } else {
+            send(k_rows, idx_k[j - 2 * LOADS], sm.k[t & 1], j - 2 * LOADS);
+          }
+        } else if (j < LOADS) {
           vst[j] = ld_stage(v_rows + static_cast<uint64_t>(static_cast<uint32_t>(idx_v[j])) * row_stride());
         } else if (j < 2 * LOADS) {
           if (j == LOADS) {
@@ -1519,12 +1597,13 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
     // ---- phase 2 ------------------------------------------------------------------------------------------
     float m4[4];
     {
-      const unsigned char* vbase = reinterpret_cast<const unsigned char*>(sm.v[t & 1]) + v_lane;
+      const unsigned char* vbase = reinterpret_cast<const unsigned char*>(sm.v[t & 1]);
       typedef __attribute__((address_space(3))) v4s16_t* lds_v4_t;
       auto read_v = [&](int i) __attribute__((always_inline)) {   // product i = (output block i % ND, k-step i / ND of the tile)
-        const unsigned char* a = vbase + (i % ND) * VSUB + (i / ND) * (16 * 64);
+        constexpr int kRow = DMA ? 2 * D : 64;       // bytes from token to token
+        const unsigned char* a = vbase + (DMA ? v_lane[DMA ? i % ND : 0] : v_lane[0] + (i % ND) * Lds::kVSub) + (i / ND) * (16 * kRow);
         const v4s16_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4_t)(a));
-        const v4s16_t hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4_t)(a + 8 * 64));
+        const v4s16_t hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4_t)(a + 8 * kRow));
         U4 o;
         o.x = __builtin_bit_cast(uint2, lo).x; o.y = __builtin_bit_cast(uint2, lo).y;
         o.z = __builtin_bit_cast(uint2, hi4).x; o.w = __builtin_bit_cast(uint2, hi4).y;
@@ -1558,6 +1637,15 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
     if constexpr (HAVE_NEXT) decide(m4, psum);
     else l_run += psum;
     EXT_T(4);
+    if constexpr (DMA && HAVE_NEXT) {
+      rows_landed();
+      held_ids(idx_n);
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        idx_v[i] = idx_k[i];
+        idx_k[i] = idx_n[i];
+      }
+    }
     __syncthreads();
     EXT_T(5);
   };
@@ -1673,7 +1761,7 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
 
 template <int D, int NWV, bool FP8>
 __global__ __launch_bounds__(64 * NWV, 2) void extend_attention_pipe_kernel(ExtendParams p) {
-  __shared__ SmemLadder<D> sm;
+  __shared__ SmemLadder<D, FP8> sm;
   extend_pipe_body<D, NWV, FP8, false>(p, sm);
 }
 
@@ -1686,7 +1774,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void extend_attention_pipe_kernel(Exte
 template <bool FP8>
 __global__ __launch_bounds__(512, 2) void extend_attention_walk_kernel(ExtendParams p) {
   __shared__ struct {
-    SmemLadder<128> sm;
+    SmemLadder<128, FP8> sm;
     WalkQueue queue;
   } lds;
   extend_pipe_body<128, 8, FP8, false, true>(p, lds.sm, &lds.queue);
@@ -1695,14 +1783,16 @@ __global__ __launch_bounds__(512, 2) void extend_attention_walk_kernel(ExtendPar
 // The same walk by four waves (128 rows, two workgroups a CU), with a request's key tiles dealt over p.parts workgroups.  Few new tokens
 // behind a long context leave most of the chip idle otherwise, and what runs is a serial chain of tiles.  Each part leaves unnormalised
 // fp32 rows that extend_merge_kernel joins; a single part writes the output itself.
-// Measured (us; general 4-wave kernel -> this one): 203 tokens behind 3800, 32 / 8 heads: 168 -> 37 in four parts; 22 x 3 behind 4549,
-// 32 / 32 heads: 210 -> 52 in four; 1000 cold: 53 -> 27 in one part; 16 x 20 behind 500: 31 -> 19 in one.
+// Measured (us; general 4-wave kernel -> this one): 203 tokens behind 3800, 32 / 8 heads: 168 -> 33 in four parts; 22 x 3 behind 4549,
+// 32 / 32 heads: 210 -> 53 in five; 1000 cold: 53 -> 23.5 in one part; 16 x 20 behind 500: 31 -> 18.5 in one.
+// (Two groups of four waves a workgroup, half of a part's tiles each, joined in LDS: 63 tiles in one part 80 -> 65, but two waves a SIMD need 4300 clocks for
+// two tiles where one needs 2700 for one, and with parts to choose from 90 drawn launches gained 0.8 %.)
 constexpr int kPartWaves = 4;
 
-// How many parts, from what a launch of them costs (us).  A workgroup walks its tiles in about 1.35 us each (1.05 at head dim 64) and
-// pays four more for its first fetches; up to 256 workgroups have a CU alone, two on a CU take 0.65 of the time of one behind the
+// How many parts, from what a launch of them costs (us).  A workgroup walks its tiles in about 1.35 us each (1.05 at head dim 64; bf16 rows a tenth
+// less) and pays four more for its first fetches; up to 256 workgroups have a CU alone, two on a CU take 0.65 of the time of one behind the
 // other.  The merge is a launch (5 us), half a microsecond a part, and the parts' fp32 rows through the caches at about 6 TB/s.
-// Against the best of 1, 2, 3, 4, 6, 8 .. 32 parts this picks within 5 % on 20 of 23 measured shapes and within 12 % on the rest.
+// Against the best of 1, 2, 3, 4, 5, 6, 8 .. 16 parts this picks 1.8 % above it on the mean of 90 drawn launches, 14 % at worst.
 int extend_parts(int64_t wgs, int64_t rows, int max_kv_len, int head_dim) {
   const int tiles = (max_kv_len + kKvTile - 1) / kKvTile;
   const double tile_us = head_dim == 128 ? 1.35 : 1.05;
@@ -1768,8 +1858,8 @@ bool extend_ragged(int64_t held, int64_t batch, int64_t num_tokens, int64_t sum_
 }
 
 template <int D, bool FP8>
-__global__ __launch_bounds__(64 * kPartWaves, 2) void extend_attention_parts_kernel(ExtendParams p) {
-  __shared__ SmemLadder<D> sm;
+__global__ __launch_bounds__(64 * kPartWaves, D > 64 ? 2 : 3) void extend_attention_parts_kernel(ExtendParams p) {
+  __shared__ SmemLadder<D, FP8> sm;
   extend_pipe_body<D, kPartWaves, FP8, true>(p, sm);
 }
 
@@ -1914,7 +2004,9 @@ static int extend_attention_any(const void* q, void* out, const void* k_cache, c
   auto wgs = [&](int rows) { return ((rows_total + rows - 1) / rows) * num_kv_heads * batch; };
   int mtw = 2, nwv = 4;
   // eligible for the 32x32 kernels (flag bit 0, or a forced shape but 8 x 2: the general kernel)
-  const bool plain = !kv_layout_hnd && sliding_window < 0 && logit_cap == 0.f && custom_mask == nullptr && (g_extend_debug_flags & 1) == 0;
+  // (rows_to_lds() takes whole 16-byte pieces: bf16 pools that do not begin at one stay with the general kernel)
+  const bool plain = !kv_layout_hnd && sliding_window < 0 && logit_cap == 0.f && custom_mask == nullptr && (g_extend_debug_flags & 1) == 0 &&
+                     (kv_fp8 || ((reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache)) & 15) == 0);
   const bool small = plain && g_extend_debug_shape == 0 && group <= 32 * kPartWaves && out_token_stride % 8 == 0 &&
                      !extend_eight_waves(num_tokens, batch, rows_total, group, num_kv_heads, head_dim) && !(max_kv_len > 0 && max_kv_len <= kKvTile);
   if (group <= 256 && wgs(256) >= 256) { mtw = 2; nwv = 8; }

@@ -3,7 +3,7 @@ import pytest
 import torch
 
 import oracle.ops as oo
-from sglang_amd import native
+from sglang_amd import kernels, native
 from test_kernels_gpu import BF, _random_case
 
 
@@ -109,3 +109,26 @@ def test_a_key_that_is_no_number_makes_its_rows_nan_in_any_number_of_parts(devic
         nan[10:40, 4:] = True
         assert bool(outs[1][nan].isnan().all()), parts
         assert torch.equal(outs[1][~nan], outs[0][~nan]), parts
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hq,Hkv,D,extend,max_kv", [(32, 8, 128, [130, 7], 0), (14, 2, 64, [300, 65], 365), (64, 8, 128, [700, 900], 1000)])
+def test_pool_that_does_not_begin_at_a_16_byte_piece(device, Hq, Hkv, D, extend, max_kv):
+    """Rows go to LDS in whole 16-byte pieces only where the pool begins at one; other pools give the same result another way."""
+    prefix = [0, 100]
+    c = _random_case(2, Hq, Hkv, D, prefix, extend, seed=Hq + D)
+    ref = oo.extend_attention(c["q"], c["k_cache"], c["v_cache"], c["req_to_token"], c["req_pool_indices"], c["seq_lens"], c["extend_prefix_lens"],
+                              c["extend_seq_lens"], c["scaling"], causal=True, compute_dtype=torch.float32)
+
+    def shifted(x, by):
+        flat = torch.empty(x.numel() + by, dtype=x.dtype, device=device)
+        flat[by:] = x.reshape(-1).to(device)
+        return flat[by:].view(x.shape)
+
+    q = c["q"].to(device)
+    qo = torch.tensor([0, extend[0], sum(extend)], dtype=torch.int32, device=device)
+    args = (c["req_to_token"].to(device), c["req_pool_indices"].to(device), c["seq_lens"].to(torch.int32).to(device),
+            torch.tensor(prefix, dtype=torch.int32, device=device), qo, max(extend), c["scaling"])
+    for k_by, v_by in ((0, 0), (4, 0), (0, 4), (2, 4)):
+        out = kernels.extend_attention(q, torch.empty_like(q), shifted(c["k_cache"], k_by), shifted(c["v_cache"], v_by), *args, max_kv_len=max_kv)
+        torch.testing.assert_close(out.float().cpu(), ref.float(), atol=4e-3, rtol=1e-2, msg=lambda m: f"{k_by}, {v_by}: {m}")
