@@ -23,6 +23,7 @@
 //             (S | n) = e^{m0-g_n} (S0 | n0) + sum_j e^{a_j-g_n} k_j (v_j | 1)^T,  m = c_n + g_n
 // (I + A)^-1 is formed by forward substitution in 16-token blocks, which stays accurate for repeated keys.
 #include "elem_io.hpp"
+#include "delta_walk.hpp"
 #include "recurrent_split.hpp"
 #include "sglang_amd.h"
 
@@ -267,6 +268,8 @@ struct DeltaChunkParams {
   int64_t o_stride;
   int heads, kv_heads, K, V, vec, col_waves;
   float q_scale;
+  void* ws;                     // two launches: what the first leaves to the second, and for how many chunks of a head there is room
+  int64_t units;
 };
 
 template <typename T, int NT>
@@ -499,6 +502,24 @@ template <int NU>
 __global__ __launch_bounds__(64 * (kPrepWaves + 4), 2) void delta_split_kernel(DeltaChunkParams p) {
   __shared__ __attribute__((aligned(16))) DeltaSplit<NU> sm;
   delta_split_body<DeltaChunkParams, NU>(p, sm);
+}
+
+template <int NU>
+__global__ __launch_bounds__(64 * kDeltaPrepWaves, 4) void delta_prepare_kernel(DeltaChunkParams p) {
+  __shared__ __attribute__((aligned(16))) DeltaPrep sm[kDeltaPrepWaves];
+  delta_prepare_body<DeltaChunkParams, NU>(p, sm[threadIdx.x >> 6]);
+}
+
+template <int NU>
+__global__ __launch_bounds__(64 * 5, 2) void delta_walk_kernel(DeltaChunkParams p) {
+  __shared__ __attribute__((aligned(1024))) DeltaWalk<NU> sm[2];
+  delta_walk_body<DeltaChunkParams, NU, false>(p, sm);
+}
+
+template <int NU>
+__global__ __launch_bounds__(64 * 4, 2) void delta_walk_self_kernel(DeltaChunkParams p) {
+  __shared__ __attribute__((aligned(1024))) DeltaWalk<NU> sm[2];
+  delta_walk_body<DeltaChunkParams, NU, true>(p, sm);
 }
 
 struct MemoryChunkParams {
@@ -746,6 +767,36 @@ void launch_delta_split(DeltaChunkParams p, int segs, hipStream_t st) {
   else hipLaunchKernelGGL((delta_split_kernel<4>), grid, block, 0, st, p);
 }
 
+// Two launches (delta_walk.hpp) where the walk is long enough for what they cost more in front of it: one launch takes about 7.6 us and 2.45 a chunk of the
+// longest segment (4.6 for two workgroups of a compute unit, one behind the other), two take 11.5 and 2.0 (3.1 side by side).  us, one launch / two: 3 x 40
+// tokens 14.0 / 17.6, 2 of up to 290 31.3 / 31.6, 300 tokens 31.5 / 30.1, 1500 119 / 96; of more workgroups than compute units 8 x 33 26.1 / 24.0, 16 x 100
+// 75 / 54.  And while the first launch leaves no more than this to the second.
+constexpr int kDeltaWalkChunks = 9, kDeltaWalkCrowdedChunks = 3;
+constexpr int64_t kDeltaWalkBytes = int64_t{1} << 30;
+// What the first of two launches leaves to the second: chunks of 32 tokens a segment, DeltaUnit a chunk and head.
+int64_t delta_units(int64_t tokens, int64_t segs) { return tokens / 32 + segs; }
+
+void launch_delta_walk(DeltaChunkParams p, int segs, int max_len, hipStream_t st) {
+  const int w = p.col_waves = split_column_waves(p.V, static_cast<int64_t>(segs) * p.heads);
+  const int chunks = (max_len + 31) / 32;
+  const dim3 prep((p.heads + kDeltaPrepWaves - 1) / kDeltaPrepWaves, chunks < 1 ? 1 : chunks > 65535 ? 65535 : chunks, segs), block0(64 * kDeltaPrepWaves);
+  const dim3 grid(p.heads, segs, (p.V + 16 * w - 1) / (16 * w));
+  // (up to one workgroup a compute unit a fifth wave fetches: 3 of 1.3 - 1.9 k, 32 heads of 128 x 128, 134 us against 147; past that two workgroups share a
+  // compute unit and their waves fetch: 16 x 512 194 -> 171, 6 x 1400 217 -> 200)
+  const bool self = w == 4 && static_cast<int64_t>(grid.x) * grid.y * grid.z > 256;
+  const dim3 block(64 * (self ? w : 1 + w));
+#define SGL_LAUNCH_WALK(NU_)                                                                       \
+  do {                                                                                             \
+    hipLaunchKernelGGL((delta_prepare_kernel<NU_>), prep, block0, 0, st, p);                       \
+    if (self) hipLaunchKernelGGL((delta_walk_self_kernel<NU_>), grid, block, 0, st, p);            \
+    else hipLaunchKernelGGL((delta_walk_kernel<NU_>), grid, block, 0, st, p);                      \
+  } while (0)
+  if (p.K <= 32) SGL_LAUNCH_WALK(1);
+  else if (p.K <= 64) SGL_LAUNCH_WALK(2);
+  else SGL_LAUNCH_WALK(4);
+#undef SGL_LAUNCH_WALK
+}
+
 template <typename T>
 void launch_mamba2_chunk(Mamba2ChunkParams p, int segs, hipStream_t st) {
   const int w = p.col_waves = column_waves(p.P, static_cast<int64_t>(segs) * p.heads);
@@ -807,10 +858,18 @@ int sgl_amd_mamba2_chunk(int is_f32, const void* xbc, int64_t xbc_stride, const 
   return 0;
 }
 
-int sgl_amd_delta_chunk(int is_f32, const void* qkv, int64_t qkv_stride, const void* b, const void* a, int64_t ba_stride,
+int64_t sgl_amd_delta_chunk_workspace(int64_t tokens, int segments, int max_len, int heads, int key_dim, int value_dim) {
+  if (tokens <= 0 || segments <= 0 || heads <= 0 || key_dim <= 0 || key_dim > 128 || value_dim <= 0 || max_len <= 0) return 0;
+  const int64_t chunks = (static_cast<int64_t>(max_len) + 31) / 32, wgs = static_cast<int64_t>(segments) * heads * ((value_dim + 63) / 64), rounds = (wgs + 255) / 256;
+  if (chunks * rounds < (rounds > 1 ? kDeltaWalkCrowdedChunks : kDeltaWalkChunks)) return 0;
+  const int64_t bytes = delta_units(tokens, segments) * heads * static_cast<int64_t>(sizeof(DeltaUnit));
+  return bytes <= kDeltaWalkBytes ? bytes : 0;
+}
+
+int sgl_amd_delta_chunk_ws(int is_f32, const void* qkv, int64_t qkv_stride, const void* b, const void* a, int64_t ba_stride,
                         const float* A_log, const float* dt_bias, float* state, const int64_t* slots, const int64_t* positions,
                         const int32_t* seg_start, const int32_t* seg_len, void* o, int64_t o_stride, int segments, int heads, int kv_heads,
-                        int key_dim, int value_dim, float q_scale, void* stream) {
+                        int key_dim, int value_dim, float q_scale, int64_t tokens, int max_len, void* ws, int64_t ws_bytes, void* stream) {
   SGL_CLEAR_STALE_ERROR();
   SGL_CHECK_ARG(qkv && b && a && A_log && dt_bias && state && slots && positions && seg_start && seg_len && o, "delta_chunk: null operand");
   SGL_CHECK_ARG(kv_heads > 0 && heads > 0 && heads % kv_heads == 0 && value_dim > 0 && key_dim > 0 && key_dim <= 192 && segments <= 65535,
@@ -822,11 +881,25 @@ int sgl_amd_delta_chunk(int is_f32, const void* qkv, int64_t qkv_stride, const v
                      heads, kv_heads, key_dim, value_dim, vec, 0, q_scale};
   const bool split = !is_f32 && key_dim <= 128 && key_dim % 8 == 0 && value_dim % 8 == 0 && qkv_stride % 8 == 0 && qkv_stride < (1 << 24) &&
                      aligned_to(qkv, 16) && o_stride % 4 == 0 && aligned_to(o, 8);
-  if (is_f32) launch_delta_chunk<float>(p, segments, as_stream(stream));
+  if (split && ws) {
+    SGL_CHECK_ARG(aligned_to(ws, 16) && tokens >= 0 && ws_bytes >= delta_units(tokens, segments) * heads * static_cast<int64_t>(sizeof(DeltaUnit)),
+                  "delta_chunk: workspace of %lld bytes", static_cast<long long>(ws_bytes));
+    p.ws = ws;
+    p.units = delta_units(tokens, segments);
+    launch_delta_walk(p, segments, max_len, as_stream(stream));
+  } else if (is_f32) launch_delta_chunk<float>(p, segments, as_stream(stream));
   else if (split) launch_delta_split(p, segments, as_stream(stream));
   else launch_delta_chunk<uint16_t>(p, segments, as_stream(stream));
   SGL_CHECK_LAUNCH("delta_chunk");
   return 0;
+}
+
+int sgl_amd_delta_chunk(int is_f32, const void* qkv, int64_t qkv_stride, const void* b, const void* a, int64_t ba_stride,
+                        const float* A_log, const float* dt_bias, float* state, const int64_t* slots, const int64_t* positions,
+                        const int32_t* seg_start, const int32_t* seg_len, void* o, int64_t o_stride, int segments, int heads, int kv_heads,
+                        int key_dim, int value_dim, float q_scale, void* stream) {
+  return sgl_amd_delta_chunk_ws(is_f32, qkv, qkv_stride, b, a, ba_stride, A_log, dt_bias, state, slots, positions, seg_start, seg_len, o, o_stride, segments, heads,
+                                kv_heads, key_dim, value_dim, q_scale, 0, 0, nullptr, 0, stream);
 }
 
 int sgl_amd_memory_chunk(int is_f32, const void* q, const void* k, const void* v, const void* gate_i, const void* gate_f, int64_t stride,

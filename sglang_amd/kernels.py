@@ -1697,9 +1697,15 @@ def gated_delta_scan(qkv: torch.Tensor, b: torch.Tensor, a: torch.Tensor, A_log:
     _need(qkv.shape[1] == 2 * kv_heads * K + H * V and b.shape == a.shape == (T, H) and b.stride(0) == a.stride(0)
           and A_log.numel() == dt_bias.numel() == H, "gated_delta_scan: shapes")
     o = torch.empty((T, H * V), dtype=qkv.dtype, device=qkv.device)
-    native.call("sgl_amd_delta_chunk" if _chunked(seg, K, form) else "sgl_amd_delta_step", _is_f32(qkv, b, a), qkv.data_ptr(), qkv.stride(0), b.data_ptr(), a.data_ptr(), b.stride(0),
-                A_log.data_ptr(), dt_bias.data_ptr(), state.data_ptr(), slots.data_ptr(), positions.data_ptr(), _ptr(seg.start), _ptr(seg.len),
-                o.data_ptr(), o.stride(0), B, H, kv_heads, K, V, float(q_scale), _stream())
+    is_f32 = _is_f32(qkv, b, a)
+    args = (is_f32, qkv.data_ptr(), qkv.stride(0), b.data_ptr(), a.data_ptr(), b.stride(0), A_log.data_ptr(), dt_bias.data_ptr(), state.data_ptr(),
+            slots.data_ptr(), positions.data_ptr(), _ptr(seg.start), _ptr(seg.len), o.data_ptr(), o.stride(0), B, H, kv_heads, K, V, float(q_scale))
+    if not _chunked(seg, K, form):
+        native.call("sgl_amd_delta_step", *args, _stream())
+        return o
+    size = 0 if is_f32 else native.lib().sgl_amd_delta_chunk_workspace(T, B, int(seg.max_len), H, K, V)
+    ws = torch.empty(size, dtype=torch.uint8, device=qkv.device) if size else None
+    native.call("sgl_amd_delta_chunk_ws", *args, T, int(seg.max_len), _ptr(ws), size, _stream())
     return o
 
 

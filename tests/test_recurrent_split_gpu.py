@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from oracle import hybrid as oh
-from sglang_amd import kernels
+from sglang_amd import kernels, native
 from test_hybrid_kernels_gpu import _err, _segments
 
 pytestmark = pytest.mark.gpu
@@ -285,3 +285,72 @@ def test_steps_so_long_that_a_factor_leaves_the_floats(device, dt, fall):
         assert bool(y.isfinite().all()) and bool(state.isfinite().all()), odd
         out.append((y.cpu(), state.cpu()))
     assert _err(out[0][0], out[1][0]) < 1.2e-2 and _err(out[0][1], out[1][1]) < 1e-4
+
+
+def test_rule_of_two_launches():
+    """Where the first launch pays: from so many chunks of the longest segment on, fewer where workgroups stand behind each other."""
+    size = native.lib().sgl_amd_delta_chunk_workspace
+    assert size(1500, 1, 1500, 32, 128, 128) == (1500 // 32 + 1) * 32 * 10240
+    for args, two in (((288, 1, 288, 32, 128, 128), True), ((256, 1, 256, 32, 128, 128), False), ((8 * 33, 8, 33, 32, 128, 128), True), ((4 * 33, 4, 33, 32, 128, 128), False),
+                      ((512, 16, 32, 32, 128, 128), True), ((256, 8, 32, 32, 128, 128), False), ((1500, 1, 1500, 32, 136, 128), False), ((0, 1, 1500, 32, 128, 128), False),
+                      ((200000, 4, 50000, 32, 128, 128), False)):
+        assert (size(*args) > 0) == two, args
+
+
+@pytest.mark.parametrize("heads,groups,K,V,decay,copies", [(2, 1, 128, 128, 0.0, 1), (4, 2, 64, 64, 0.0, 1), (2, 2, 32, 16, 0.0, 1), (3, 3, 40, 24, -1.0, 1),
+                                                           (2, 1, 72, 136, -2.0, 1), (4, 2, 8, 8, 0.5, 1), (2, 1, 104, 72, 4.0, 1), (7, 7, 128, 64, 0.0, 3), (8, 4, 56, 72, 4.0, 2)])
+def test_delta_rule_in_two_launches(device, heads, groups, K, V, decay, copies):
+    """The same bars as the one launch (test_split_recurrence), at the edges of chunks, tiles and columns; several copies: more workgroups than compute units.
+    A workspace full of NaN: nothing is read that the first launch does not write.  Empty segments change nothing."""
+    g = torch.Generator().manual_seed(heads * K + V)
+    lens = ([0] + LENS + [0, 300]) * copies
+    T, width = sum(lens), heads * V + 2 * groups * K
+    act, gates = torch.randn(T, width, generator=g).to(BF), torch.randn(T, 2 * heads, generator=g).to(BF)
+    A_log, bias = torch.randn(heads, generator=g) * 0.5 + decay, torch.randn(heads, generator=g) * 0.5 - 1.0
+    state0 = torch.randn(len(lens) + 1, heads, K, V, generator=g) * 0.3
+    slots = torch.randperm(len(lens), generator=g) + 1
+    spans, pos, at = [], [], 0
+    for i, n in enumerate(lens):
+        if i % 2 and n:
+            act[at:at + n, groups * K:2 * groups * K] = act[at, groups * K:2 * groups * K].clone()
+        spans.append((at, at + n))
+        pos.append(torch.arange(n) + (7 if i % 2 == 0 else 0))
+        at += n
+    start = torch.tensor([min(lo, T - 1) for lo, _ in spans], dtype=torch.int32, device=device)
+    length, pos = torch.tensor(lens, dtype=torch.int32, device=device), torch.cat(pos).to(device)
+    dev = [t.to(device) for t in (A_log, bias, slots)]
+    gt, stream = gates.to(device), torch.cuda.current_stream().cuda_stream
+    units = (T // 32 + len(lens)) * heads * 10240
+
+    def run(rows, two):
+        state, o = state0.to(device), torch.full((T, heads * V), 7.0, dtype=BF, device=device)
+        a = gt[:, heads:]
+        args = (0, rows.data_ptr(), rows.stride(0), gt.data_ptr(), a.data_ptr(), gt.stride(0), dev[0].data_ptr(), dev[1].data_ptr(), state.data_ptr(), dev[2].data_ptr(),
+                pos.data_ptr(), start.data_ptr(), length.data_ptr(), o.data_ptr(), o.stride(0), len(lens), heads, groups, K, V, K ** -0.5)
+        if two:
+            ws = torch.full((units // 2,), float("nan"), dtype=BF, device=device)
+            native.call("sgl_amd_delta_chunk_ws", *args, T, max(lens), ws.data_ptr(), units, stream)
+        else:
+            native.call("sgl_amd_delta_chunk", *args, stream)
+        return o, state
+
+    y, state = run(act.to(device), True)
+    odd = torch.zeros(T, width + 9, dtype=BF, device=device)
+    odd[:, 1:1 + width] = act.to(device)
+    y0, general = run(odd[:, 1:1 + width], False)                        # rows at odd addresses: the general kernel
+    assert _err(y, y0.cpu()) < 1.2e-2 and torch.equal(state[0].cpu(), state0[0])
+    for i, (lo, hi) in enumerate(spans):
+        if lo == hi:
+            assert torch.equal(state[slots[i]].cpu(), state0[slots[i]])
+            continue
+        if i >= len(LENS) + 3:                                           # (copies: against the general kernel alone)
+            off = (state[slots[i]] - general[slots[i]]).abs().max() / general[slots[i]].abs().max()
+            assert off < 8e-6, (i, float(off))
+            continue
+        begin = state0[slots[i]] if i % 2 == 0 else torch.zeros(heads, K, V)
+        want = _state_want("delta", begin, (act[lo:hi], gates[lo:hi]), A_log, bias, heads, groups, K, V)
+        off = (state[slots[i]].double().cpu() - want).abs().max() / want.abs().max()
+        assert off < 4e-6, (i, float(off), float((general[slots[i]].double().cpu() - want).abs().max() / want.abs().max()))
+    # the same bits every time
+    again, state2 = run(act.to(device), True)
+    assert torch.equal(again, y) and torch.equal(state2, state)
