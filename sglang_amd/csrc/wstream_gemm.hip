@@ -36,6 +36,7 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 
+constexpr int kNumCus = 256;
 constexpr int kKC = 128;              // K elements per chunk (256 B of every weight row)
 constexpr int kKSteps = kKC / 32;     // MFMA k-steps per chunk
 constexpr int kSlotsPerRow = kKC / 8; // 16-byte slots per staged activation row
@@ -276,7 +277,7 @@ __global__ __launch_bounds__(64 * NW, 1) void wstream_gemm_kernel(WsParams p) {
   constexpr int WCH = NW * WWAVE;                       // weight bytes per chunk
   constexpr int CH = WCH + XPIECES * 1024;              // ring slot: [weights of wave 0..NW) | activations]
   static_assert(PD >= 3 && PD * CH + 1024 <= 160 * 1024, "LDS ring does not fit");
-  static_assert((PD - 1) * WPC + (PD - 2) * XP < 64, "vmcnt range");
+  static_assert((PD - 1) * WPC + (PD - 2) * XP + MT * TPW < 64, "vmcnt range");
   __shared__ __attribute__((aligned(1024))) unsigned char ring[PD * CH + 1024];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -285,8 +286,11 @@ __global__ __launch_bounds__(64 * NW, 1) void wstream_gemm_kernel(WsParams p) {
   const int r16 = lane & 15, g = lane >> 4;
   const int wtiles = p.ntiles / TPW;                    // tiles a wave index ranges over
   const int bx = blockIdx.x, by = GROUPED ? 0 : blockIdx.y;
-  const int tile = bx * NW + wid;
-  const bool active = tile < wtiles;
+  int tile = bx * NW + wid;
+  // Without split-K a workgroup stays where there are more groups of NW wave tiles than compute units: it takes every gridDim.x-th
+  // group and asks for the next one's first chunks while it multiplies the last ones of this (launch_main()).
+  const int tile_step = GROUPED ? 0 : static_cast<int>(gridDim.x) * NW;
+  const int groups = GROUPED ? 1 : ((wtiles + NW - 1) / NW - bx + static_cast<int>(gridDim.x) - 1) / static_cast<int>(gridDim.x);
   const int split = by;
   const int rb = GROUPED ? blockIdx.y : 0;              // row block (grouped form)
   const uint16_t* wbase = p.w;
@@ -306,16 +310,19 @@ __global__ __launch_bounds__(64 * NW, 1) void wstream_gemm_kernel(WsParams p) {
   // is applied on the global side, each row's 256 B still move as two whole cache lines.
   const int q4 = lane >> 4, s16 = lane & 15;
   const uint16_t* wsrc[TPW][kKSteps];
+  auto weights_of = [&](int wave_tile) {
 #pragma unroll
-  for (int t = 0; t < TPW; ++t)
+    for (int t = 0; t < TPW; ++t)
 #pragma unroll
-    for (int j = 0; j < kKSteps; ++j) {
-      const int row = 4 * j + q4;
-      const int64_t tl = active ? tile : wtiles - 1;
-      const int64_t wrow = (TPW == 1 && p.pair_silu == 2) ? (row < 8 ? 0 : p.N / 2) + tl * 8 + (row & 7)
-                                                          : (tl + static_cast<int64_t>(t) * wtiles) * 16 + row;
-      wsrc[t][j] = wbase + wrow * p.w_stride + ((s16 ^ row) & 15) * 8 + static_cast<int64_t>(cb) * kKC;
-    }
+      for (int j = 0; j < kKSteps; ++j) {
+        const int row = 4 * j + q4;
+        const int64_t tl = wave_tile < wtiles ? wave_tile : wtiles - 1;
+        const int64_t wrow = (TPW == 1 && p.pair_silu == 2) ? (row < 8 ? 0 : p.N / 2) + tl * 8 + (row & 7)
+                                                            : (tl + static_cast<int64_t>(t) * wtiles) * 16 + row;
+        wsrc[t][j] = wbase + wrow * p.w_stride + ((s16 ^ row) & 15) * 8 + static_cast<int64_t>(cb) * kKC;
+      }
+  };
+  weights_of(tile);
   const uint16_t* xsrc[XP];
   int xoff[XP];                                          // wave-uniform LDS offset inside a ring slot
 #pragma unroll
@@ -346,29 +353,40 @@ __global__ __launch_bounds__(64 * NW, 1) void wstream_gemm_kernel(WsParams p) {
   // stride (a multiple of 8 KiB) maps onto a few memory channels (gate_up 46.5 -> 38.6 us).  Split-K launches already
   // start at `splits` different columns and measured 0.3-1 us slower staggered.
   const int rot = p.splits == 1 && n > 1 ? static_cast<int>((static_cast<int64_t>(bx) * n) / gridDim.x) : 0;
-  auto issue_w = [&](int c_rel, int slot) {
-    if (c_rel < n) {
-      const int cr = c_rel + rot < n ? c_rel + rot : c_rel + rot - n;
+  // The next chunk to ask for, of the weights and of the activations: its place in the K range and the groups left, its own included.
+  int w_c = 0, w_left = groups, w_tile = tile, x_c = 0, x_left = groups;
+  auto issue_w = [&](int slot) {
+    if (w_left > 0) {
+      const int cr = w_c + rot < n ? w_c + rot : w_c + rot - n;
       const int koff = cr * kKC;
       const int base = slot * CH + wid * WWAVE;
 #pragma unroll
       for (int t = 0; t < TPW; ++t)
 #pragma unroll
         for (int j = 0; j < kKSteps; ++j) dma16<2>(wsrc[t][j] + koff, (lds_ptr_t)(ring3 + base + t * 4096 + j * 1024));
+      if (++w_c == n) {
+        w_c = 0;
+        w_tile += tile_step;
+        if (--w_left > 0) weights_of(w_tile);
+      }
     } else {
 #pragma unroll
       for (int i = 0; i < WPC; ++i) dma16<0>(dummy_src, dummy_dst);
     }
   };
-  auto issue_x = [&](int c_rel, int slot) {
-    if (c_rel < n) {
-      const int cr = c_rel + rot < n ? c_rel + rot : c_rel + rot - n;
+  auto issue_x = [&](int slot) {
+    if (x_left > 0) {
+      const int cr = x_c + rot < n ? x_c + rot : x_c + rot - n;
       const int64_t koff = cr * p.x_cstride;
       const int base = slot * CH;
 #pragma unroll
       for (int i = 0; i < XP; ++i) {
         const int off = xoff[i] >= 0 ? base + xoff[i] : PD * CH;
         dma16<0>(xsrc[i] + koff, (lds_ptr_t)(ring3 + off));
+      }
+      if (++x_c == n) {
+        x_c = 0;
+        --x_left;
       }
     } else {
 #pragma unroll
@@ -383,10 +401,6 @@ __global__ __launch_bounds__(64 * NW, 1) void wstream_gemm_kernel(WsParams p) {
   for (int kk = 0; kk < kKSteps; ++kk) foff[kk] = r16 * 256 + (((kk * 4 + g) ^ r16) & 15) * 16;
 
   f32x4_t acc[TPW][MT];
-#pragma unroll
-  for (int t = 0; t < TPW; ++t)
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[t][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   // activation fragments of one "stage": up to 64 rows the stage is a whole k-step (all B tiles); beyond, a k-step is
   // two stages (first half of the B tiles, then the second half) so that the reads of two consecutive stages stay
@@ -403,7 +417,7 @@ __global__ __launch_bounds__(64 * NW, 1) void wstream_gemm_kernel(WsParams p) {
     if constexpr (H > 2) b[2] = lds_rd<WCH + 8192>(bd);
     if constexpr (H > 3) b[3] = lds_rd<WCH + 12288>(bd);
   };
-  auto compute = [&](int slot, int c) {
+  auto compute = [&](int slot) {
     const uint32_t slot_addr = ring_addr + slot * CH;
     u32x4_t a[kKSteps][TPW], b[2][H];                    // a: the wave's weight tiles of the chunk; b: by stage parity
 #pragma unroll
@@ -417,7 +431,7 @@ __global__ __launch_bounds__(64 * NW, 1) void wstream_gemm_kernel(WsParams p) {
     for (int kk = 0; kk < kKSteps; ++kk)
 #pragma unroll
       for (int t = 0; t < TPW; ++t) pin(a[kk][t]);
-    issue_w(c + PD, slot);                               // the tiles just copied out are free: refill them now
+    issue_w(slot);                                       // the tiles just copied out are free: refill them now
 #pragma unroll
     for (int st = 0; st < NST; ++st) {
       const int kk = WIDE ? st >> 1 : st;
@@ -441,124 +455,146 @@ __global__ __launch_bounds__(64 * NW, 1) void wstream_gemm_kernel(WsParams p) {
     }
   };
 
+  // lane holds C[m = 16 mt + r16][n = 16 tile + 4 g + r]
+  auto write_out = [&]() {
+    const int n0 = tile * 16 + g * 4;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      int64_t m = mt * 16 + r16;                           // output row
+      float scale = 1.f;
+      if constexpr (GROUPED) {
+        const int id = p.sorted_ids[rb * (16 * MT) + mt * 16 + r16];
+        if (id >= p.M) continue;
+        m = id;
+        if (p.row_scale) scale = p.row_scale[id];
+      } else {
+        if (m >= p.M) continue;
+      }
+      // one 4-wide piece of an output row: partial, or bias / router weight and the store
+      auto put = [&](float (&o)[4], int nn, bool plain) {
+        if (plain && !GROUPED && p.bias) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[r] += bf2f(p.bias[nn + r]);
+        }
+        if (plain && act_pointwise(p.glu.kind)) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[r] = squared_relu(o[r]);
+        }
+        if (GROUPED && p.row_scale) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[r] = (p.round_before_scale ? rbf(o[r]) : o[r]) * scale;
+        }
+        if (GROUPED && p.out_f32) {
+          *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(p.y) + m * p.y_stride + nn) = f32x4_t{o[0], o[1], o[2], o[3]};
+        } else {
+          uint2 w2;
+          w2.x = pack_bf2(o[0], o[1]);
+          w2.y = pack_bf2(o[2], o[3]);
+          *reinterpret_cast<uint2*>(p.y + blocked_off(m, nn, p.y_stride, p.y_cstride)) = w2;
+        }
+      };
+      if (TPW == 1 && !GROUPED && p.pair_silu == 2) {
+        // lanes g = 0, 1 hold the gate values of columns 8 tile + 4 g + r, lanes g = 2, 3 the up values of the same columns
+        float o[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float mine = acc[0][mt][r];
+          const float other = __shfl_xor(mine, 32, 64);
+          float gv = g < 2 ? mine : other, uv = g < 2 ? other : mine;
+          if (p.bias) {
+            const int c = tile * 8 + (g & 1) * 4 + r;
+            gv += bf2f(p.bias[c]);
+            uv += bf2f(p.bias[p.N / 2 + c]);
+          }
+          o[r] = glu<true>(p.glu, gv, uv);
+        }
+        if (g < 2) put(o, tile * 8 + g * 4, false);
+        continue;
+      }
+      if (TPW == 2 && p.pair_silu) {
+        // linear -> bf16, silu -> bf16, product -> bf16 (activation.py:141-143)
+        float o[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float gv = acc[0][mt][r], uv = acc[TPW - 1][mt][r];
+          if (!GROUPED && p.bias) {
+            gv += bf2f(p.bias[n0 + r]);
+            uv += bf2f(p.bias[p.N / 2 + n0 + r]);
+          }
+          o[r] = glu<true>(p.glu, gv, uv);
+        }
+        put(o, n0, false);
+        continue;
+      }
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) {                      // plain form: tile t of the wave is output tile `tile + t * wtiles`
+        const int nn = n0 + t * wtiles * 16;
+        if (!GROUPED && p.part) {
+          const int64_t e = (static_cast<int64_t>(split) * p.M + m) * p.N + nn;
+          if (!(p.dbg & 2)) {   // write-through (sc1): the partials leave the L2 while the stream runs, not at the kernel boundary
+                                // (qkv 18.7 -> 17.0, o 15.2 -> 14.7, down 29.1 -> 28.6 us per GEMM + combine pair: profiles/r06_exp2_gemm_ab.json)
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(p.part, 0, static_cast<int>(static_cast<int64_t>(p.splits) * p.M * p.N * 4), 0x00020000);
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc[t][mt]), r, static_cast<int>(e * 4), 0, 16);
+          } else {
+            *reinterpret_cast<f32x4_t*>(p.part + e) = acc[t][mt];
+          }
+          continue;
+        }
+        float o[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = acc[t][mt][r];
+        put(o, nn, true);
+      }
+    }
+  };
+
   // ---- pipeline: weights PD chunks ahead, activations PD - 1, one barrier per chunk ----
 #pragma unroll
   for (int u = 0; u < PD - 1; ++u) {
-    issue_w(u, u);
-    issue_x(u, u);
+    issue_w(u);
+    issue_x(u);
   }
-  issue_w(PD - 1, PD - 1);
+  issue_w(PD - 1);
   int slot = 0, nslot = PD - 1;                          // slot of chunk c, slot of chunk c - 1 (= c + PD - 1)
-  for (int c = 0; c < n; ++c) {
-    // chunk c has landed once only the DMAs issued after its activations are outstanding:
-    // weights of c+1 .. c+PD-1 and activations of c+1 .. c+PD-2
-    wait_vm<(PD - 1) * WPC + (PD - 2) * XP>();
-    __builtin_amdgcn_s_barrier();                        // everyone's pieces of chunk c are visible,
-                                                         // everyone is done reading the activations of chunk c - 1
-    issue_x(c + PD - 1, nslot);
-#ifdef WS_TRACE
-    if (c == 0) WS_STAMP(1);
-#endif
-    compute(slot, c);
-    slot = slot + 1 == PD ? 0 : slot + 1;
-    nslot = nslot + 1 == PD ? 0 : nslot + 1;
-  }
-
-  WS_STAMP(2);
-#ifdef WS_TRACE
-  struct StampAtExit { __device__ ~StampAtExit() { __builtin_amdgcn_s_waitcnt(0); WS_STAMP(3); } } stamp_at_exit;
-#endif
-  if (!active) return;
-  // lane holds C[m = 16 mt + r16][n = 16 tile + 4 g + r]
-  const int n0 = tile * 16 + g * 4;
+  // The output stores of a group go out behind the requests of the next one's first chunks and count among what is outstanding.
+  // Every wave with a tile makes exactly this many (a 16-row tile of the launched MT has a row below M).
+  const int stores = TPW == 2 && p.pair_silu ? MT : MT * TPW;
+  int behind = 0;                                        // stores that the first PD - 1 waits of this group may leave outstanding
+  for (int gr = 0; gr < groups; ++gr, tile += tile_step) {
+    const bool active = tile < wtiles;
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    int64_t m = mt * 16 + r16;                           // output row
-    float scale = 1.f;
-    if constexpr (GROUPED) {
-      const int id = p.sorted_ids[rb * (16 * MT) + mt * 16 + r16];
-      if (id >= p.M) continue;
-      m = id;
-      if (p.row_scale) scale = p.row_scale[id];
-    } else {
-      if (m >= p.M) continue;
-    }
-    // one 4-wide piece of an output row: partial, or bias / router weight and the store
-    auto put = [&](float (&o)[4], int nn, bool plain) {
-      if (plain && !GROUPED && p.bias) {
+    for (int t = 0; t < TPW; ++t)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] += bf2f(p.bias[nn + r]);
-      }
-      if (plain && act_pointwise(p.glu.kind)) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = squared_relu(o[r]);
-      }
-      if (GROUPED && p.row_scale) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = (p.round_before_scale ? rbf(o[r]) : o[r]) * scale;
-      }
-      if (GROUPED && p.out_f32) {
-        *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(p.y) + m * p.y_stride + nn) = f32x4_t{o[0], o[1], o[2], o[3]};
+      for (int mt = 0; mt < MT; ++mt) acc[t][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < n; ++c) {
+      // chunk c has landed once only the DMAs issued after its activations are outstanding:
+      // weights of c+1 .. c+PD-1 and activations of c+1 .. c+PD-2
+      constexpr int AHEAD = (PD - 1) * WPC + (PD - 2) * XP;
+      if (!GROUPED && MT <= 4 && behind == MT * TPW && c < PD - 1) {
+        wait_vm<AHEAD + MT * TPW>();
+      } else if (!GROUPED && MT <= 4 && behind == MT && c < PD - 1) {
+        wait_vm<AHEAD + MT>();
       } else {
-        uint2 w2;
-        w2.x = pack_bf2(o[0], o[1]);
-        w2.y = pack_bf2(o[2], o[3]);
-        *reinterpret_cast<uint2*>(p.y + blocked_off(m, nn, p.y_stride, p.y_cstride)) = w2;
+        wait_vm<AHEAD>();
       }
-    };
-    if (TPW == 1 && !GROUPED && p.pair_silu == 2) {
-      // lanes g = 0, 1 hold the gate values of columns 8 tile + 4 g + r, lanes g = 2, 3 the up values of the same columns
-      float o[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float mine = acc[0][mt][r];
-        const float other = __shfl_xor(mine, 32, 64);
-        float gv = g < 2 ? mine : other, uv = g < 2 ? other : mine;
-        if (p.bias) {
-          const int c = tile * 8 + (g & 1) * 4 + r;
-          gv += bf2f(p.bias[c]);
-          uv += bf2f(p.bias[p.N / 2 + c]);
-        }
-        o[r] = glu<true>(p.glu, gv, uv);
-      }
-      if (g < 2) put(o, tile * 8 + g * 4, false);
-      continue;
+      __builtin_amdgcn_s_barrier();                      // everyone's pieces of chunk c are visible,
+                                                         // everyone is done reading the activations of chunk c - 1
+      issue_x(nslot);
+#ifdef WS_TRACE
+      if (c == 0) WS_STAMP(1);
+#endif
+      compute(slot);
+      slot = slot + 1 == PD ? 0 : slot + 1;
+      nslot = nslot + 1 == PD ? 0 : nslot + 1;
     }
-    if (TPW == 2 && p.pair_silu) {
-      // linear -> bf16, silu -> bf16, product -> bf16 (activation.py:141-143)
-      float o[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float gv = acc[0][mt][r], uv = acc[TPW - 1][mt][r];
-        if (!GROUPED && p.bias) {
-          gv += bf2f(p.bias[n0 + r]);
-          uv += bf2f(p.bias[p.N / 2 + n0 + r]);
-        }
-        o[r] = glu<true>(p.glu, gv, uv);
-      }
-      put(o, n0, false);
-      continue;
-    }
-#pragma unroll
-    for (int t = 0; t < TPW; ++t) {                      // plain form: tile t of the wave is output tile `tile + t * wtiles`
-      const int nn = n0 + t * wtiles * 16;
-      if (!GROUPED && p.part) {
-        const int64_t e = (static_cast<int64_t>(split) * p.M + m) * p.N + nn;
-        if (!(p.dbg & 2)) {   // write-through (sc1): the partials leave the L2 while the stream runs, not at the kernel boundary
-                              // (qkv 18.7 -> 17.0, o 15.2 -> 14.7, down 29.1 -> 28.6 us per GEMM + combine pair: profiles/r06_exp2_gemm_ab.json)
-          const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(p.part, 0, static_cast<int>(static_cast<int64_t>(p.splits) * p.M * p.N * 4), 0x00020000);
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc[t][mt]), r, static_cast<int>(e * 4), 0, 16);
-        } else {
-          *reinterpret_cast<f32x4_t*>(p.part + e) = acc[t][mt];
-        }
-        continue;
-      }
-      float o[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] = acc[t][mt][r];
-      put(o, nn, true);
-    }
+    WS_STAMP(2);
+    behind = active ? stores : 0;
+    if (active) write_out();
   }
+#ifdef WS_TRACE
+  __builtin_amdgcn_s_waitcnt(0);
+  WS_STAMP(3);
+#endif
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -705,7 +741,11 @@ __global__ __launch_bounds__(256) void prefetch_head_kernel(const uint16_t* __re
 template <int MT, int NW, int TPW>
 int launch_main(const WsParams& p, hipStream_t st, int row_blocks = 0) {
   if constexpr (ring_depth(MT, NW, TPW) >= 3) {
-    dim3 grid((p.ntiles / TPW + NW - 1) / NW, row_blocks ? row_blocks : p.splits);
+    const int groups = (p.ntiles / TPW + NW - 1) / NW;
+    // One workgroup fits on a compute unit.  More groups than compute units, in rounds of workgroups, let the ring run dry at every round's
+    // end; workgroups that stay keep it filled across groups: [64, 128256, 4096] 184 -> 177 us (one row 169 -> 156), [64, 151936, 896]
+    // 66.1 -> 56.5 (49 -> 43), silu [16, 57344, 8192] 157 -> 142.  A launch of fewer groups has nothing to stay for.
+    dim3 grid(p.splits == 1 && !row_blocks && groups > kNumCus ? kNumCus : groups, row_blocks ? row_blocks : p.splits);
     if (row_blocks) {
       if constexpr (MT <= 4) hipLaunchKernelGGL((wstream_gemm_kernel<MT, NW, TPW, true>), grid, dim3(64 * NW), 0, st, p);
       else return -1;

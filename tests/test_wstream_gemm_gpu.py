@@ -316,6 +316,33 @@ def test_wstream_two_tiles_per_wave_plain_epilogues(device, M, N, K, nw, splits)
         assert torch.equal(K_.unblock(blk), got)
 
 
+@pytest.mark.parametrize("M", [1, 16, 50, 64, 100])
+@pytest.mark.parametrize("N,K,nw,tpw,silu", [(16400, 128, 4, 1, False), (50000, 896, 4, 1, False), (33312, 256, 5, 1, False), (32800, 128, 4, 2, False),
+                                             (70016, 384, 4, 2, False), (20000, 640, 2, 2, False), (49184, 384, 3, 2, True), (33056, 896, 8, 1, True)])
+def test_wstream_workgroups_that_take_several_groups(device, M, N, K, nw, tpw, silu):
+    """More groups of tiles than compute units, without split-K: rounds that end within a group, fewer chunks than the ring has slots,
+    bias loads and stores between two groups' requests; with and without a bias."""
+    K_ = _k()
+    if M > 64 and (nw > 5 or (nw > 2 and tpw == 2)):
+        pytest.skip("beyond 64 rows the wide groups have no ring")
+    g = torch.Generator().manual_seed(M + N + K)
+    x = (torch.randn((M, K), generator=g) * 0.5).to(BF).to(device)
+    w = (torch.randn((N, K), generator=g) * 0.05).to(BF).to(device)
+    for bias in (None, torch.randn(N, generator=g).to(BF).to(device)):
+        got = K_.wstream_gemm(x, w, bias=bias, epilogue="silu_and_mul" if silu else "none", waves_per_group=nw, tiles_per_wave=tpw, splits=1)
+        ref = _ref_linear(x, w, bias)
+        if not silu:
+            _check(got, ref)
+            continue
+        h = ref.to(BF).double()
+        h, up = h[:, :N // 2], h[:, N // 2:]
+        # the product is rounded three times (gate and up, silu, product): an ulp of bf16 (2^-8 of the value) each, and that of gate times
+        # silu's slope relative to its value, at most (1 + |gate|)
+        want = torch.nn.functional.silu(h) * up
+        tol = want.abs() * 2.0 ** -8 * (4 + h.abs()) + 1e-3
+        assert bool(((got.double() - want).abs() <= tol).all())
+
+
 def test_wstream_auto_decomposition_is_what_the_model_runs(device):
     """No explicit decomposition: choose_wstream_decomposition (two-tile waves for the wide single-split launches)."""
     K_ = _k()
