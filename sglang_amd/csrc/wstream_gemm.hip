@@ -23,6 +23,8 @@
 //   * split-K partials are plain row-major fp32 [split][M][N]; one combine kernel sums them in
 //     split order (deterministic) and applies the epilogue the next operator would have been:
 //     bias, silu(gate)*up, or residual-add + RMSNorm, with the torch-native bf16 rounding points.
+#include <type_traits>
+
 #include "common.hpp"
 #include "glu.hpp"
 #include "kv_format.hpp"
@@ -38,8 +40,6 @@ typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kNumCus = 256;
 constexpr int kKC = 128;              // K elements per chunk (256 B of every weight row)
-constexpr int kKSteps = kKC / 32;     // MFMA k-steps per chunk
-constexpr int kSlotsPerRow = kKC / 8; // 16-byte slots per staged activation row
 
 __device__ __forceinline__ bf16x8_t as_frag(const U4& v) { return __builtin_bit_cast(bf16x8_t, v); }
 
@@ -193,6 +193,10 @@ struct WsParams {
   int64_t x_cstride;     // elements between consecutive 128-wide K chunks of an x row (128 for a row-major x)
   int64_t y_cstride;     // the same for the 128-wide column blocks of y (bf16 outputs)
   int M, N, K, splits, ntiles;
+  int width;             // wave tiles of a group (launch_main())
+  int turns, full;       // a workgroup's groups: turns, and one less from workgroup `full` on
+  int chunks_each, chunks_over; // K chunks / splits and what is left over
+  float inv_splits, inv_grid;   // 1 / splits, 1 / gridDim.x (a division of two integers takes some hundred clocks in front of the first request)
   // grouped (mixture-of-experts) form: blockIdx.y = row block of moe_align_block_size's output, rows gathered /
   // scattered through sorted_ids, weights of expert expert_ids[block]; M = number of valid (token, k) pair ids
   const int32_t* sorted_ids;    // [>= blocks * 16 MT]  pair ids, padding >= M
@@ -253,11 +257,16 @@ __device__ __forceinline__ void pin(u32x4_t& v) { asm volatile("" : "+v"(v)); }
 template <int N>
 __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
-// ring depth: as many chunk slots as fit the 160 KiB LDS (1 KiB is the dummy landing zone), at most 6
-constexpr int ring_depth(int mt, int nw, int tpw) {
-  const int slot = nw * tpw * 4096 + mt * 4 * 1024;
-  const int d = (160 * 1024 - 1024) / slot;
-  return d > 6 ? 6 : d;
+// K elements of a ring chunk: 128, and 64 for the groups of eight two-tile waves, whose 256 rows of weights would leave room for one chunk of 128
+constexpr int ring_chunk(int nw, int tpw) { return nw * tpw > 8 ? 64 : 128; }
+// ring depth: as many chunk slots as fit the 160 KiB LDS, at most 6, and no more than the 6 bits that count a wave's requests
+constexpr int ring_depth(int mt, int nw, int tpw, bool grouped) {
+  const int kc = ring_chunk(nw, tpw);
+  int d = (grouped ? 159 : 160) * 1024 / ((nw * tpw + mt) * 32 * kc);
+  if (d > 6) d = 6;
+  const int wpc = tpw * kc / 32, xp = (mt * kc / 32 + nw - 1) / nw;
+  while ((d - 1) * wpc + (d - 2) * xp + mt * tpw > 63) --d;
+  return d;
 }
 
 // TPW = 16-row weight tiles per wave.  TPW == 2: the wave owns tiles t and t + ntiles/2 (half the activation reads
@@ -269,16 +278,23 @@ constexpr int ring_depth(int mt, int nw, int tpw) {
 // 224 x 4 waves: 32 CUs idle).  Gate and up of a column sit 32 lanes apart in the accumulator: one lane swap in the epilogue.
 template <int MT, int NW, int TPW, bool GROUPED>
 __global__ __launch_bounds__(64 * NW, 1) void wstream_gemm_kernel(WsParams p) {
-  constexpr int PD = ring_depth(MT, NW, TPW);
-  constexpr int XPIECES = MT * 4;                       // 1 KiB pieces (4 rows x 256 B) of an activation chunk
-  constexpr int XP = (XPIECES + NW - 1) / NW;           // pieces each wave fetches (surplus -> dummy slot)
-  constexpr int WPC = TPW * kKSteps;                    // weight DMA instructions per wave per chunk
-  constexpr int WWAVE = TPW * 4096;                     // weight bytes per wave per chunk
+  constexpr int PD = ring_depth(MT, NW, TPW, GROUPED);
+  constexpr int KC = ring_chunk(NW, TPW);               // K elements per chunk
+  constexpr int KSTEPS = KC / 32;                       // MFMA k-steps per chunk
+  constexpr int SLOTS = KC / 8;                         // 16-byte slots of a staged row
+  constexpr int PROWS = 64 / SLOTS;                     // rows of a 1 KiB piece
+  constexpr int TILE = 32 * KC;                         // bytes of 16 staged rows
+  constexpr int TPIECES = 16 / PROWS;                   // pieces of 16 staged rows
+  constexpr int XPIECES = MT * TPIECES;                 // pieces of an activation chunk
+  constexpr int XP = (XPIECES + NW - 1) / NW;           // pieces each wave fetches, ...
+  constexpr int XS = XPIECES / NW;                      // ... or those that are left without a last one
+  constexpr int WPC = TPW * TPIECES;                    // weight DMA instructions per wave per chunk
+  constexpr int WWAVE = TPW * TILE;                     // weight bytes per wave per chunk
   constexpr int WCH = NW * WWAVE;                       // weight bytes per chunk
   constexpr int CH = WCH + XPIECES * 1024;              // ring slot: [weights of wave 0..NW) | activations]
-  static_assert(PD >= 3 && PD * CH + 1024 <= 160 * 1024, "LDS ring does not fit");
+  static_assert(PD >= 3 && PD * CH <= 160 * 1024, "LDS ring does not fit");
   static_assert((PD - 1) * WPC + (PD - 2) * XP + MT * TPW < 64, "vmcnt range");
-  __shared__ __attribute__((aligned(1024))) unsigned char ring[PD * CH + 1024];
+  __shared__ __attribute__((aligned(1024))) unsigned char ring[PD * CH];
 
   const int tid = threadIdx.x, lane = tid & 63;
   WS_STAMP(0);
@@ -286,11 +302,11 @@ __global__ __launch_bounds__(64 * NW, 1) void wstream_gemm_kernel(WsParams p) {
   const int r16 = lane & 15, g = lane >> 4;
   const int wtiles = p.ntiles / TPW;                    // tiles a wave index ranges over
   const int bx = blockIdx.x, by = GROUPED ? 0 : blockIdx.y;
-  int tile = bx * NW + wid;
-  // Without split-K a workgroup stays where there are more groups of NW wave tiles than compute units: it takes every gridDim.x-th
-  // group and asks for the next one's first chunks while it multiplies the last ones of this (launch_main()).
-  const int tile_step = GROUPED ? 0 : static_cast<int>(gridDim.x) * NW;
-  const int groups = GROUPED ? 1 : ((wtiles + NW - 1) / NW - bx + static_cast<int>(gridDim.x) - 1) / static_cast<int>(gridDim.x);
+  // The tiles are dealt out in groups of p.width.  Where there are more groups than workgroups in a row of the grid (launch_main()), a
+  // workgroup stays: it takes every gridDim.x-th group and asks for the next one's first chunks while it multiplies the last ones of this.
+  const int groups = GROUPED ? 1 : p.turns - (bx >= p.full);
+  const int tile_step = static_cast<int>(gridDim.x) * p.width;
+  int tile = bx * p.width + wid;
   const int split = by;
   const int rb = GROUPED ? blockIdx.y : 0;              // row block (grouped form)
   const uint16_t* wbase = p.w;
@@ -300,36 +316,40 @@ __global__ __launch_bounds__(64 * NW, 1) void wstream_gemm_kernel(WsParams p) {
     if (e < 0) return;                                  // filtered expert (EP): its rows stay untouched
     wbase += static_cast<int64_t>(e) * p.w_expert_stride;
   }
-  const int nch = p.K / kKC;
-  const int cb = static_cast<int>(static_cast<int64_t>(split) * nch / p.splits);
-  const int ce = static_cast<int>(static_cast<int64_t>(split + 1) * nch / p.splits);
+  const int nch = p.K / KC;
+  // split s begins at chunk floor(s nch / splits)
+  auto begin_of = [&](int sp) {
+    return sp == p.splits ? nch : sp * p.chunks_each + static_cast<int>((static_cast<float>(sp * p.chunks_over) + 0.5f) * p.inv_splits);
+  };
+  const int cb = GROUPED ? 0 : begin_of(split);
+  const int ce = GROUPED ? nch : begin_of(split + 1);
   const int n = ce - cb;
 
-  // ---- DMA roles.  A 1 KiB piece = 4 rows x 16 slots; the lane at (row q, slot s) of the LDS image
-  // fetches global slot s ^ (row & 15): the XOR swizzle that makes the fragment reads conflict-free
-  // is applied on the global side, each row's 256 B still move as two whole cache lines.
-  const int q4 = lane >> 4, s16 = lane & 15;
-  const uint16_t* wsrc[TPW][kKSteps];
+  // ---- DMA roles.  A 1 KiB piece = PROWS rows x SLOTS slots; the lane at (row q, slot s) of the LDS image
+  // fetches global slot s ^ swz(row): the XOR swizzle that makes the fragment reads conflict-free
+  // is applied on the global side, each row's 256 or 128 B still move as whole cache lines.
+  const int qrow = lane / SLOTS, qslot = lane % SLOTS;
+  auto swz = [](int row) { return SLOTS == 16 ? row & 15 : (row >> 1) & 7; };
+  const uint16_t* wsrc[TPW][TPIECES];
   auto weights_of = [&](int wave_tile) {
 #pragma unroll
     for (int t = 0; t < TPW; ++t)
 #pragma unroll
-      for (int j = 0; j < kKSteps; ++j) {
-        const int row = 4 * j + q4;
+      for (int j = 0; j < TPIECES; ++j) {
+        const int row = PROWS * j + qrow;
         const int64_t tl = wave_tile < wtiles ? wave_tile : wtiles - 1;
         const int64_t wrow = (TPW == 1 && p.pair_silu == 2) ? (row < 8 ? 0 : p.N / 2) + tl * 8 + (row & 7)
                                                             : (tl + static_cast<int64_t>(t) * wtiles) * 16 + row;
-        wsrc[t][j] = wbase + wrow * p.w_stride + ((s16 ^ row) & 15) * 8 + static_cast<int64_t>(cb) * kKC;
+        wsrc[t][j] = wbase + wrow * p.w_stride + (qslot ^ swz(row)) * 8 + static_cast<int64_t>(cb) * KC;
       }
   };
   weights_of(tile);
   const uint16_t* xsrc[XP];
-  int xoff[XP];                                          // wave-uniform LDS offset inside a ring slot
+  const bool all_pieces = wid + NW * (XP - 1) < XPIECES;
 #pragma unroll
   for (int i = 0; i < XP; ++i) {
     const int piece = wid + NW * i;
-    const bool real = piece < XPIECES;
-    const int row = real ? 4 * piece + q4 : 0;
+    const int row = piece < XPIECES ? PROWS * piece + qrow : 0;
     int srow;
     if constexpr (GROUPED) {
       const int id = p.sorted_ids[rb * (16 * MT) + row];
@@ -337,68 +357,54 @@ __global__ __launch_bounds__(64 * NW, 1) void wstream_gemm_kernel(WsParams p) {
     } else {
       srow = row < p.M ? row : p.M - 1;
     }
-    xsrc[i] = p.x + static_cast<int64_t>(srow) * p.x_stride + ((s16 ^ row) & 15) * 8 + static_cast<int64_t>(cb) * p.x_cstride;
-    xoff[i] = real ? WCH + piece * 1024 : -1;
+    xsrc[i] = p.x + static_cast<int64_t>(srow) * p.x_stride + (qslot ^ swz(row)) * 8;
   }
   lds_bytes_t ring3 = (lds_bytes_t)(ring);
   // Chunk c lives in ring slot c % PD.  A wave's weight tiles of a slot are private to it: the wave copies them to
   // registers (TPW * 4 fragments) at the top of compute() and refills the slot with chunk c + PD at once, so all PD
   // slots' worth of weights stay in flight; the activation image is shared, so chunk c + PD - 1's goes into slot
-  // c - 1 after the barrier that retires it.  Behind the end of the K range a dummy DMA (L2-resident source, the
-  // 1 KiB landing zone) is issued instead, which keeps the in-order vmcnt arithmetic the same in every iteration.
-  const uint16_t* dummy_src = p.x + s16 * 8;
-  lds_ptr_t dummy_dst = (lds_ptr_t)(ring3 + PD * CH);
+  // c - 1 after the barrier that retires it.
   // Without split-K the workgroups walk the K range from staggered starting chunks (wrapping around): launched
   // together they would otherwise all pull the same 256-byte column of their rows at the same moment, which the row
   // stride (a multiple of 8 KiB) maps onto a few memory channels (gate_up 46.5 -> 38.6 us).  Split-K launches already
   // start at `splits` different columns and measured 0.3-1 us slower staggered.
-  const int rot = p.splits == 1 && n > 1 ? static_cast<int>((static_cast<int64_t>(bx) * n) / gridDim.x) : 0;
+  const int rot = p.splits == 1 ? min(static_cast<int>(static_cast<float>(bx * n) * p.inv_grid), n - 1) : 0;
   // The next chunk to ask for, of the weights and of the activations: its place in the K range and the groups left, its own included.
   int w_c = 0, w_left = groups, w_tile = tile, x_c = 0, x_left = groups;
   auto issue_w = [&](int slot) {
-    if (w_left > 0) {
-      const int cr = w_c + rot < n ? w_c + rot : w_c + rot - n;
-      const int koff = cr * kKC;
-      const int base = slot * CH + wid * WWAVE;
+    if (w_left == 0) return;
+    const int cr = w_c + rot < n ? w_c + rot : w_c + rot - n;
+    const int koff = cr * KC;
+    const int base = slot * CH + wid * WWAVE;
 #pragma unroll
-      for (int t = 0; t < TPW; ++t)
+    for (int t = 0; t < TPW; ++t)
 #pragma unroll
-        for (int j = 0; j < kKSteps; ++j) dma16<2>(wsrc[t][j] + koff, (lds_ptr_t)(ring3 + base + t * 4096 + j * 1024));
-      if (++w_c == n) {
-        w_c = 0;
-        w_tile += tile_step;
-        if (--w_left > 0) weights_of(w_tile);
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < WPC; ++i) dma16<0>(dummy_src, dummy_dst);
+      for (int j = 0; j < TPIECES; ++j) dma16<2>(wsrc[t][j] + koff, (lds_ptr_t)(ring3 + base + t * TILE + j * 1024));
+    if (++w_c == n) {
+      w_c = 0;
+      w_tile += tile_step;
+      if (--w_left > 0) weights_of(w_tile);
     }
   };
   auto issue_x = [&](int slot) {
-    if (x_left > 0) {
-      const int cr = x_c + rot < n ? x_c + rot : x_c + rot - n;
-      const int64_t koff = cr * p.x_cstride;
-      const int base = slot * CH;
+    if (x_left == 0) return;
+    const int cr = cb + (x_c + rot < n ? x_c + rot : x_c + rot - n);
+    const int64_t koff = KC == kKC ? cr * p.x_cstride : (cr >> 1) * p.x_cstride + (cr & 1) * KC;
+    const int base = slot * CH;
 #pragma unroll
-      for (int i = 0; i < XP; ++i) {
-        const int off = xoff[i] >= 0 ? base + xoff[i] : PD * CH;
-        dma16<0>(xsrc[i] + koff, (lds_ptr_t)(ring3 + off));
-      }
-      if (++x_c == n) {
-        x_c = 0;
-        --x_left;
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < XP; ++i) dma16<0>(dummy_src, dummy_dst);
+    for (int i = 0; i < XP; ++i)
+      if (i < XS || all_pieces) dma16<0>(xsrc[i] + koff, (lds_ptr_t)(ring3 + base + WCH + (wid + NW * i) * 1024));
+    if (++x_c == n) {
+      x_c = 0;
+      --x_left;
     }
   };
 
   // ---- fragment read addresses (bytes, LDS address space) ----
   const uint32_t ring_addr = (uint32_t)(uintptr_t)(ring3);
-  uint32_t foff[kKSteps];
+  uint32_t foff[KSTEPS];
 #pragma unroll
-  for (int kk = 0; kk < kKSteps; ++kk) foff[kk] = r16 * 256 + (((kk * 4 + g) ^ r16) & 15) * 16;
+  for (int kk = 0; kk < KSTEPS; ++kk) foff[kk] = r16 * (2 * KC) + ((kk * 4 + g) ^ swz(r16)) * 16;
 
   f32x4_t acc[TPW][MT];
 
@@ -407,28 +413,28 @@ __global__ __launch_bounds__(64 * NW, 1) void wstream_gemm_kernel(WsParams p) {
   // inside the 4-bit lgkmcnt while one stage is always read ahead of the MFMAs
   constexpr bool WIDE = MT > 4;
   constexpr int H = WIDE ? MT / 2 : MT;                // B tiles per stage
-  constexpr int NST = WIDE ? 2 * kKSteps : kKSteps;    // stages per chunk
+  constexpr int NST = WIDE ? 2 * KSTEPS : KSTEPS;    // stages per chunk
   auto read_stage = [&](uint32_t slot_addr, int st, u32x4_t (&b)[H]) {
     const int kk = WIDE ? st >> 1 : st;
     const int half = WIDE ? st & 1 : 0;
-    const uint32_t bd = slot_addr + foff[kk] + half * (H * 4096);
+    const uint32_t bd = slot_addr + foff[kk] + half * (H * TILE);
     b[0] = lds_rd<WCH>(bd);
-    if constexpr (H > 1) b[1] = lds_rd<WCH + 4096>(bd);
-    if constexpr (H > 2) b[2] = lds_rd<WCH + 8192>(bd);
-    if constexpr (H > 3) b[3] = lds_rd<WCH + 12288>(bd);
+    if constexpr (H > 1) b[1] = lds_rd<WCH + TILE>(bd);
+    if constexpr (H > 2) b[2] = lds_rd<WCH + 2 * TILE>(bd);
+    if constexpr (H > 3) b[3] = lds_rd<WCH + 3 * TILE>(bd);
   };
   auto compute = [&](int slot) {
     const uint32_t slot_addr = ring_addr + slot * CH;
-    u32x4_t a[kKSteps][TPW], b[2][H];                    // a: the wave's weight tiles of the chunk; b: by stage parity
+    u32x4_t a[KSTEPS][TPW], b[2][H];                    // a: the wave's weight tiles of the chunk; b: by stage parity
 #pragma unroll
-    for (int kk = 0; kk < kKSteps; ++kk) {
+    for (int kk = 0; kk < KSTEPS; ++kk) {
       a[kk][0] = lds_rd<0>(slot_addr + foff[kk] + wid * WWAVE);
-      if constexpr (TPW > 1) a[kk][1] = lds_rd<4096>(slot_addr + foff[kk] + wid * WWAVE);
+      if constexpr (TPW > 1) a[kk][1] = lds_rd<TILE>(slot_addr + foff[kk] + wid * WWAVE);
     }
     read_stage(slot_addr, 0, b[0]);
     wait_lgkm<H>();                                      // LDS returns in order: the weight fragments are in
 #pragma unroll
-    for (int kk = 0; kk < kKSteps; ++kk)
+    for (int kk = 0; kk < KSTEPS; ++kk)
 #pragma unroll
       for (int t = 0; t < TPW; ++t) pin(a[kk][t]);
     issue_w(slot);                                       // the tiles just copied out are free: refill them now
@@ -549,17 +555,58 @@ __global__ __launch_bounds__(64 * NW, 1) void wstream_gemm_kernel(WsParams p) {
   };
 
   // ---- pipeline: weights PD chunks ahead, activations PD - 1, one barrier per chunk ----
+  int slot = 0, nslot = PD - 1;                          // slot of chunk c, slot of chunk c - 1 (= c + PD - 1)
+  int left = groups * n;                                 // the chunks of all groups not yet multiplied
+  if (!GROUPED && wid >= p.width) {                      // a wave beyond the groups' width only helps with the activations
+    for (int u = 0; u < PD - 1; ++u) issue_x(u);
+    for (; left > 0; --left) {
+      if (left < PD) wait_vm<0>();
+      else if (XS == XP || all_pieces) wait_vm<(PD - 2) * XP>();
+      else wait_vm<(PD - 2) * XS>();
+      __builtin_amdgcn_s_barrier();
+      issue_x(nslot);
+      nslot = nslot + 1 == PD ? 0 : nslot + 1;
+    }
+    return;
+  }
 #pragma unroll
   for (int u = 0; u < PD - 1; ++u) {
     issue_w(u);
     issue_x(u);
   }
   issue_w(PD - 1);
-  int slot = 0, nslot = PD - 1;                          // slot of chunk c, slot of chunk c - 1 (= c + PD - 1)
   // The output stores of a group go out behind the requests of the next one's first chunks and count among what is outstanding.
   // Every wave with a tile makes exactly this many (a 16-row tile of the launched MT has a row below M).
   const int stores = TPW == 2 && p.pair_silu ? MT : MT * TPW;
   int behind = 0;                                        // stores that the first PD - 1 waits of this group may leave outstanding
+  // Chunk c has landed once only the requests made behind its activations are outstanding: weights of c+1 .. c+PD-1 and activations of
+  // c+1 .. c+PD-2, or of as many as are left (where waves differ in the pieces that they bring, at least so many).
+  auto wait_ahead = [&](auto pieces, int c) {
+    constexpr int AHEAD = (PD - 1) * WPC + (PD - 2) * decltype(pieces)::value;
+    if (!GROUPED && MT <= 4 && behind == MT * TPW && c < PD - 1) {
+      wait_vm<AHEAD + MT * TPW>();
+    } else if (!GROUPED && MT <= 4 && behind == MT && c < PD - 1) {
+      wait_vm<AHEAD + MT>();
+    } else {
+      wait_vm<AHEAD>();
+    }
+  };
+  auto wait_chunk = [&](int c) {
+    if (left >= PD - 1) {
+      if (XS == XP || all_pieces) wait_ahead(std::integral_constant<int, XP>{}, c);
+      else wait_ahead(std::integral_constant<int, XS>{}, c);
+    } else if (left == 0) {
+      wait_vm<0>();
+    } else if (left == 1) {
+      wait_vm<WPC + XS>();
+    } else if (PD > 3 && left == 2) {
+      wait_vm<2 * (WPC + XS)>();
+    } else if (PD > 4 && left == 3) {
+      wait_vm<3 * (WPC + XS)>();
+    } else if (PD > 5 && left == 4) {
+      wait_vm<4 * (WPC + XS)>();
+    }
+  };
   for (int gr = 0; gr < groups; ++gr, tile += tile_step) {
     const bool active = tile < wtiles;
 #pragma unroll
@@ -567,16 +614,8 @@ __global__ __launch_bounds__(64 * NW, 1) void wstream_gemm_kernel(WsParams p) {
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) acc[t][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     for (int c = 0; c < n; ++c) {
-      // chunk c has landed once only the DMAs issued after its activations are outstanding:
-      // weights of c+1 .. c+PD-1 and activations of c+1 .. c+PD-2
-      constexpr int AHEAD = (PD - 1) * WPC + (PD - 2) * XP;
-      if (!GROUPED && MT <= 4 && behind == MT * TPW && c < PD - 1) {
-        wait_vm<AHEAD + MT * TPW>();
-      } else if (!GROUPED && MT <= 4 && behind == MT && c < PD - 1) {
-        wait_vm<AHEAD + MT>();
-      } else {
-        wait_vm<AHEAD>();
-      }
+      --left;
+      wait_chunk(c);
       __builtin_amdgcn_s_barrier();                      // everyone's pieces of chunk c are visible,
                                                          // everyone is done reading the activations of chunk c - 1
       issue_x(nslot);
@@ -739,13 +778,25 @@ __global__ __launch_bounds__(256) void prefetch_head_kernel(const uint16_t* __re
 
 // the activation image of a chunk grows with M: beyond 64 rows only the narrower groups keep a 3-deep ring
 template <int MT, int NW, int TPW>
-int launch_main(const WsParams& p, hipStream_t st, int row_blocks = 0) {
-  if constexpr (ring_depth(MT, NW, TPW) >= 3) {
-    const int groups = (p.ntiles / TPW + NW - 1) / NW;
+int launch_main(WsParams p, hipStream_t st, int row_blocks = 0) {
+  if constexpr (ring_depth(MT, NW, TPW, false) >= 3 && (NW * TPW + MT <= 13 || (NW == 8 && TPW == 2 && MT <= 4))) {
     // One workgroup fits on a compute unit.  More groups than compute units, in rounds of workgroups, let the ring run dry at every round's
-    // end; workgroups that stay keep it filled across groups: [64, 128256, 4096] 184 -> 177 us (one row 169 -> 156), [64, 151936, 896]
-    // 66.1 -> 56.5 (49 -> 43), silu [16, 57344, 8192] 157 -> 142.  A launch of fewer groups has nothing to stay for.
-    dim3 grid(p.splits == 1 && !row_blocks && groups > kNumCus ? kNumCus : groups, row_blocks ? row_blocks : p.splits);
+    // end; workgroups that stay keep it filled: [64, 128256, 4096] 184 -> 177 us (one row 169 -> 156), silu [16, 57344, 8192] 157 -> 142.
+    // Groups are as narrow as the number of rounds allows, so that the last round is as full as the others: silu [24, 9728, 896] 10.9 -> 8.9
+    // (76 groups of four pairs / 152 of two), [64, 32000, 4096] in eight waves 56.4 -> 41.8.
+    const int wtiles = p.ntiles / TPW;
+    const bool stays = p.splits == 1 && !row_blocks;
+    const int rounds = ((wtiles + NW - 1) / NW + kNumCus - 1) / kNumCus;
+    p.width = stays ? (wtiles + kNumCus * rounds - 1) / (kNumCus * rounds) : NW;
+    const int groups = (wtiles + p.width - 1) / p.width;
+    dim3 grid(stays && groups > kNumCus ? kNumCus : groups, row_blocks ? row_blocks : p.splits);
+    p.turns = (groups + static_cast<int>(grid.x) - 1) / static_cast<int>(grid.x);
+    p.full = groups - (p.turns - 1) * static_cast<int>(grid.x);
+    const int nch = p.K / ring_chunk(NW, TPW);
+    p.chunks_each = nch / p.splits;
+    p.chunks_over = nch - p.chunks_each * p.splits;
+    p.inv_splits = 1.f / static_cast<float>(p.splits);
+    p.inv_grid = 1.f / static_cast<float>(grid.x);
     if (row_blocks) {
       if constexpr (MT <= 4) hipLaunchKernelGGL((wstream_gemm_kernel<MT, NW, TPW, true>), grid, dim3(64 * NW), 0, st, p);
       else return -1;
@@ -764,7 +815,18 @@ int launch_nw(const WsParams& p, int nw, bool two_tiles, hipStream_t st, int row
     switch (nw) {
       case 2: return launch_main<MT, 2, 2>(p, st, row_blocks);
       case 3: return launch_main<MT, 3, 2>(p, st, row_blocks);
-      case 4: return launch_main<MT, 4, 2>(p, st, row_blocks);
+      case 4:
+        // Groups of four waves or of eight.  The chip is bound by the requests that a compute unit's vector cache keeps in flight (115 to
+        // 130 of a line, of 0.9 to 1.2 k clocks each) as much as by HBM, and every turn asks for the activations anew: 256 rows of weights
+        // a turn in the place of 128 make them a fifth of the requests and not a third.  us, four waves / eight: [64, 128256, 4096]
+        // 177.5 / 168, silu [64, 57344, 8192] 152 / 141, silu [64, 37888, 3584] 58 / 46.6, [64, 32000, 4096] 43.8 / 41.8.  Up to 3.75 pairs of tiles
+        // a workgroup the eight find too little to do (silu [64, 28672, 4096] 40.3 / 41.3, [16, 9728, 896] 7.7 / 8.3); over several turns few rows are
+        // read quicker in 256 bytes of a row at a time (one row of [128256, 4096] 156 / 162, 24 rows of [151936, 896] 47.3 / 49.6).
+        if constexpr (MT <= 4) {
+          const int pairs = p.ntiles / 2;
+          if (p.splits == 1 && !row_blocks && pairs * 4 > 15 * kNumCus && (pairs <= 8 * kNumCus || MT > 2)) return launch_main<MT, 8, 2>(p, st);
+        }
+        return launch_main<MT, 4, 2>(p, st, row_blocks);
       default: return -1;
     }
   }

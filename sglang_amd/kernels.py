@@ -911,7 +911,7 @@ def choose_wstream_config(M: int, N: int, K: int, need_combine: bool = False, fu
     if fused_silu:                    # one pass, each wave owns a gate tile and its up tile: no split-K
         tiles //= 2
     wide = M > 64                     # a 128-row activation image leaves room for fewer weight waves
-    for nw in (((2,) if wide else (4, 3, 2)) if fused_silu else ((5, 4) if wide else (8, 7, 6, 5, 4))):
+    for nw in (((2,) if wide else (4,)) if fused_silu else ((5, 4) if wide else (8, 7, 6, 5, 4))):
         groups = (tiles + nw - 1) // nw
         for s in range(1, 2 if fused_silu else max(1, min(nch // 2, 32)) + 1):
             wgs = groups * s
@@ -952,10 +952,18 @@ def unblock(x: torch.Tensor) -> torch.Tensor:
 def choose_wstream_decomposition(M: int, N: int, K: int, need_combine: bool = False, fused_silu: bool = False) -> Tuple[int, int, int]:
     """(waves_per_group, tiles_per_wave, k_splits).  On top of choose_wstream_config(): a launch without split-K
     whose rows fit 64 may give every wave two output tiles (t and t + N/32) -- half the activation traffic per weight
-    byte: lm_head 200 -> 174 us, the unfused gate_up 39.6 -> 39.1 (benchmarks/gemm_sweep.py --blocked).  With split-K
-    the two-tile forms measured no faster (down 27.8 vs 27.5 us), so those keep one tile per wave."""
+    byte: lm_head 200 -> 174 us, the unfused gate_up 39.6 -> 39.1 (benchmarks/gemm_sweep.py --blocked); four such waves are
+    launched as eight where that reads quicker (launch_nw() in wstream_gemm.hip).  With split-K the two-tile forms measured no
+    faster (down 27.8 vs 27.5 us), so those keep one tile per wave."""
     nw, s = choose_wstream_config(M, N, K, need_combine, fused_silu)
     nch = K // 128
+
+    def pairs_time() -> float:
+        # up to 64 rows the launch deals the pairs of tiles out in the narrowest groups that the number of rounds allows
+        pairs, waves = N // 32, nw if M > 64 else 4
+        rounds = -(-pairs // (waves * _NUM_CUS))
+        width = waves if M > 64 else -(-pairs // (rounds * _NUM_CUS))
+        return rounds_time(-(-pairs // width), width * nch * 8192, 6.0e12, 26e9)
 
     def rounds_time(groups: int, wg_bytes: int, chip: float, per_cu: float) -> float:
         full, rem = divmod(groups, _NUM_CUS)
@@ -969,7 +977,7 @@ def choose_wstream_decomposition(M: int, N: int, K: int, need_combine: bool = Fa
         # (nw, 1) = every wave ONE tile of 8 gate + 8 up rows (N / 16 tiles).  The second one exists for the widths whose pairs
         # do not make whole rounds of the chip: Llama-3-8B gate_up has 896 pairs = 224 workgroups of 4 waves (32 CUs idle)
         # but 1792 tiles = 256 workgroups of 7 waves (measured equal: see WSTREAM_SILU_INTERLEAVED)
-        best = (rounds_time((N // 32 + nw - 1) // nw, nw * nch * 8192, 6.0e12, 26e9), nw, 2)
+        best = (pairs_time(), nw, 2)
         if WSTREAM_SILU_INTERLEAVED and M <= 64 and N % 16 == 0:
             for nw1 in (8, 7, 6, 5, 4):
                 t1 = rounds_time((N // 16 + nw1 - 1) // nw1, nw1 * nch * 4096, 6.4e12, 26e9)
@@ -980,12 +988,7 @@ def choose_wstream_decomposition(M: int, N: int, K: int, need_combine: bool = Fa
         return nw, 1, s
 
     one = rounds_time((N // 16 + nw - 1) // nw, nw * nch * 4096, 5.3e12, 24e9)
-    best = (one, nw, 1)
-    for nw2 in (4, 3, 2):
-        two = rounds_time((N // 32 + nw2 - 1) // nw2, nw2 * nch * 8192, 6.0e12, 26e9)
-        if two < best[0] * 0.98:
-            best = (two, nw2, 2)
-    return best[1], best[2], 1
+    return (4, 2, 1) if pairs_time() < one * 0.98 else (nw, 1, 1)
 
 
 def wstream_gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, epilogue: str = "none",

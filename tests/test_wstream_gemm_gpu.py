@@ -318,10 +318,12 @@ def test_wstream_two_tiles_per_wave_plain_epilogues(device, M, N, K, nw, splits)
 
 @pytest.mark.parametrize("M", [1, 16, 50, 64, 100])
 @pytest.mark.parametrize("N,K,nw,tpw,silu", [(16400, 128, 4, 1, False), (50000, 896, 4, 1, False), (33312, 256, 5, 1, False), (32800, 128, 4, 2, False),
-                                             (70016, 384, 4, 2, False), (20000, 640, 2, 2, False), (49184, 384, 3, 2, True), (33056, 896, 8, 1, True)])
+                                             (70016, 384, 4, 2, False), (20000, 640, 2, 2, False), (49184, 384, 3, 2, True), (33056, 896, 8, 1, True),
+                                             (36896, 384, 4, 2, True), (12832, 640, 4, 2, False), (9728, 896, 4, 2, True)])
 def test_wstream_workgroups_that_take_several_groups(device, M, N, K, nw, tpw, silu):
     """More groups of tiles than compute units, without split-K: rounds that end within a group, fewer chunks than the ring has slots,
-    bias loads and stores between two groups' requests; with and without a bias."""
+    bias loads and stores between two groups' requests, groups of four and of eight two-tile waves and narrower ones; with and without a
+    bias, rows and chunk-major."""
     K_ = _k()
     if M > 64 and (nw > 5 or (nw > 2 and tpw == 2)):
         pytest.skip("beyond 64 rows the wide groups have no ring")
@@ -329,7 +331,9 @@ def test_wstream_workgroups_that_take_several_groups(device, M, N, K, nw, tpw, s
     x = (torch.randn((M, K), generator=g) * 0.5).to(BF).to(device)
     w = (torch.randn((N, K), generator=g) * 0.05).to(BF).to(device)
     for bias in (None, torch.randn(N, generator=g).to(BF).to(device)):
-        got = K_.wstream_gemm(x, w, bias=bias, epilogue="silu_and_mul" if silu else "none", waves_per_group=nw, tiles_per_wave=tpw, splits=1)
+        how = dict(bias=bias, epilogue="silu_and_mul" if silu else "none", waves_per_group=nw, tiles_per_wave=tpw, splits=1)
+        got = K_.wstream_gemm(x, w, **how)
+        assert torch.equal(got, K_.wstream_gemm(x.view(M, K // 128, 128).transpose(0, 1).contiguous(), w, **how))
         ref = _ref_linear(x, w, bias)
         if not silu:
             _check(got, ref)
