@@ -34,14 +34,47 @@ __device__ __forceinline__ float squared_relu(float v) {
   return v * v;
 }
 
+// silu(g) of a g that is a bf16 value.  Up to |g| = 80 nothing over- or underflows, and a gate costs 12 instructions in the place of the 60 of
+// expf and a division for all cases: log2 e in two parts (Cody and Waite), the first of 16 bits, so that its product with the 8 bits of g is exact
+// and v_exp_f32 takes it as it is; the reciprocal's quotient once corrected.  Rounded to bf16 it equals silu_any() for every g.
+// us: 3000 tokens over 8 experts (64 outputs a lane at the end of a tile) 2243 -> 2194, 48 tokens 429 -> 426.6, a decode step of four layers 720 -> 716.
+__device__ __forceinline__ float silu_near(float g) {                      // |g| <= 80, or no number
+  const float e = fast_exp2(g * -0x1.7154p+0f);
+  const float d = 1.0f + __builtin_fmaf(e, g * -0x1.480fb6p-18f, e);
+  const float r = __builtin_amdgcn_rcpf(d);
+  const float q = g * r;
+  return __builtin_fmaf(__builtin_fmaf(-d, q, g), r, q);
+}
+__device__ __forceinline__ float silu_any(float g) { return g / (1.0f + expf(-g)); }
+
 // kRound: silu keeps the rounding points of 16-bit activations (projection -> bf16, silu -> bf16); the other kinds stay in fp32
 template <bool kRound>
 __device__ __forceinline__ float glu(const GluParams& p, float g, float u) {
   if (p.kind == kGluGeluTanh) return gelu_tanh_glu(g, u);
   if (p.kind == kGluClampedSwish) return clamped_swish_glu(p, g, u);
-  if (!kRound) return g / (1.0f + expf(-g)) * u;
+  if (!kRound) return silu_any(g) * u;
   const float gb = rbf(g);
-  return rbf(gb / (1.0f + expf(-gb))) * rbf(u);
+  return rbf(fabsf(gb) > 80.f ? silu_any(gb) : silu_near(gb)) * rbf(u);
+}
+// four outputs of glu<true>, the kind and the range looked at once
+__device__ __forceinline__ void glu4(const GluParams& p, const float (&g)[4], const float (&u)[4], float (&o)[4]) {
+  if (p.kind != kGluSilu) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r] = glu<true>(p, g[r], u[r]);
+    return;
+  }
+  float gb[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) gb[r] = rbf(g[r]);
+  if (fmaxf(fmaxf(fabsf(gb[0]), fabsf(gb[1])), fmaxf(fabsf(gb[2]), fabsf(gb[3]))) > 80.f) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r] = silu_any(gb[r]);
+  } else {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r] = silu_near(gb[r]);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) o[r] = rbf(o[r]) * rbf(u[r]);
 }
 
 }  // namespace sgl_amd

@@ -183,11 +183,10 @@ __global__ __launch_bounds__(kThreads, 2) void moe_tiled_gemm_kernel(TiledParams
       for (int i = 0; i < 2; ++i) {
         const int col = nt0 * 64 + wn * 32 + i * 16 + g * 4;
         if (col >= p.N) continue;
+        const float gv[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+        const float uv[4] = {acc[i + 2][j][0], acc[i + 2][j][1], acc[i + 2][j][2], acc[i + 2][j][3]};
         float o[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          o[r] = glu<true>(p.glu, acc[i][j][r], acc[i + 2][j][r]);
-        }
+        glu4(p.glu, gv, uv, o);
         uint2 w2;
         w2.x = pack_bf2(o[0], o[1]); w2.y = pack_bf2(o[2], o[3]);
         *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.c) + static_cast<int64_t>(id) * p.c_stride + col) = w2;
@@ -460,11 +459,10 @@ __global__ __launch_bounds__(kThreads2, 1) void moe_gemm256_kernel(TiledParams p
       for (int i = 0; i < 4; ++i) {
         const int col = nt0 * 128 + wr * 64 + i * 16 + g * 4;
         if (col >= p.N) continue;
+        const float gv[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+        const float uv[4] = {acc[i + 4][j][0], acc[i + 4][j][1], acc[i + 4][j][2], acc[i + 4][j][3]};
         float o[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          o[r] = glu<true>(p.glu, acc[i][j][r], acc[i + 4][j][r]);
-        }
+        glu4(p.glu, gv, uv, o);
         uint2 w2;
         w2.x = pack_bf2(o[0], o[1]); w2.y = pack_bf2(o[2], o[3]);
         *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.c) + static_cast<int64_t>(sid) * p.c_stride + col) = w2;

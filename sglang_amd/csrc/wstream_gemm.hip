@@ -501,34 +501,36 @@ __global__ __launch_bounds__(64 * NW, 1) void wstream_gemm_kernel(WsParams p) {
       };
       if (TPW == 1 && !GROUPED && p.pair_silu == 2) {
         // lanes g = 0, 1 hold the gate values of columns 8 tile + 4 g + r, lanes g = 2, 3 the up values of the same columns
-        float o[4];
+        float gv[4], uv[4], o[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const float mine = acc[0][mt][r];
           const float other = __shfl_xor(mine, 32, 64);
-          float gv = g < 2 ? mine : other, uv = g < 2 ? other : mine;
+          gv[r] = g < 2 ? mine : other;
+          uv[r] = g < 2 ? other : mine;
           if (p.bias) {
             const int c = tile * 8 + (g & 1) * 4 + r;
-            gv += bf2f(p.bias[c]);
-            uv += bf2f(p.bias[p.N / 2 + c]);
+            gv[r] += bf2f(p.bias[c]);
+            uv[r] += bf2f(p.bias[p.N / 2 + c]);
           }
-          o[r] = glu<true>(p.glu, gv, uv);
         }
+        glu4(p.glu, gv, uv, o);
         if (g < 2) put(o, tile * 8 + g * 4, false);
         continue;
       }
       if (TPW == 2 && p.pair_silu) {
         // linear -> bf16, silu -> bf16, product -> bf16 (activation.py:141-143)
-        float o[4];
+        float gv[4], uv[4], o[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          float gv = acc[0][mt][r], uv = acc[TPW - 1][mt][r];
+          gv[r] = acc[0][mt][r];
+          uv[r] = acc[TPW - 1][mt][r];
           if (!GROUPED && p.bias) {
-            gv += bf2f(p.bias[n0 + r]);
-            uv += bf2f(p.bias[p.N / 2 + n0 + r]);
+            gv[r] += bf2f(p.bias[n0 + r]);
+            uv[r] += bf2f(p.bias[p.N / 2 + n0 + r]);
           }
-          o[r] = glu<true>(p.glu, gv, uv);
         }
+        glu4(p.glu, gv, uv, o);
         put(o, n0, false);
         continue;
       }
@@ -686,11 +688,13 @@ __global__ __launch_bounds__(256) void wstream_combine_silu_kernel(CombineParams
   const float* row = p.part + static_cast<int64_t>(m) * p.N;
   const f32x4_t gt = sum_splits(row + j0, ss, p.splits);
   const f32x4_t up = sum_splits(row + half + j0, ss, p.splits);
-  float o[4];
+  float gv[4], uv[4], o[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    o[r] = glu<true>(p.glu, p.bias ? gt[r] + bf2f(p.bias[j0 + r]) : gt[r], p.bias ? up[r] + bf2f(p.bias[half + j0 + r]) : up[r]);
+    gv[r] = p.bias ? gt[r] + bf2f(p.bias[j0 + r]) : gt[r];
+    uv[r] = p.bias ? up[r] + bf2f(p.bias[half + j0 + r]) : up[r];
   }
+  glu4(p.glu, gv, uv, o);
   uint2 w2;
   w2.x = pack_bf2(o[0], o[1]);
   w2.y = pack_bf2(o[2], o[3]);

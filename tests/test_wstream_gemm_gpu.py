@@ -347,6 +347,27 @@ def test_wstream_workgroups_that_take_several_groups(device, M, N, K, nw, tpw, s
         assert bool(((got.double() - want).abs() <= tol).all())
 
 
+def test_silu_of_every_bf16_gate(device):
+    """One-hot gate rows and an up column of 1 (its bias): out = bf16(silu(x)) for every finite bf16 x.  An fp32 evaluation errs by a few
+    2^-24 of the value, so it may round to the other neighbour only where the 64-bit value lies within 2^-21 of its own size of the middle
+    between two; below 2^-120 the fp32 exponential of the gate overflows and the quotient is 0."""
+    K_ = _k()
+    v = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(BF)
+    v = v[torch.isfinite(v.float())]
+    v = torch.cat([v, torch.zeros((-v.numel()) % 8192, dtype=BF)]).view(-1, 64, 128).to(device)
+    w, b = torch.zeros((256, 128), dtype=BF, device=device), torch.zeros(256, dtype=BF, device=device)
+    w[:128], b[128:] = torch.eye(128, dtype=BF, device=device), 1.0
+    for x in v:
+        got = K_.wstream_gemm(x, w, bias=b, epilogue="silu_and_mul").cpu()
+        gate = K_.wstream_gemm(x, w, bias=b)[:, :128].cpu().double()
+        want = gate / (1.0 + torch.exp(-gate))
+        near = want.to(BF)
+        off = (got != near) & (want.abs() > 2.0 ** -120)
+        tie = (got.double() + near.double()) / 2
+        assert bool(((want - tie).abs()[off] <= want.abs()[off] * 2.0 ** -21).all())
+        assert bool((got.double() - want).abs()[want.abs() <= 2.0 ** -120].le(2.0 ** -120).all())
+
+
 def test_wstream_auto_decomposition_is_what_the_model_runs(device):
     """No explicit decomposition: choose_wstream_decomposition (two-tile waves for the wide single-split launches)."""
     K_ = _k()
