@@ -47,7 +47,7 @@ for M in (2048, 4096, 7680, 16384):
     K.MOE_TILED_MIN_ROWS_PER_EXPERT = 1 << 30
     t_stream = graph_time(lambda: K.fused_experts(x, w13, w2, tw, ti), reps=2)
     K.MOE_TILED_MIN_ROWS_PER_EXPERT = old
-    res[M] = {"tiled_ms": t_tiled * 1e3, "tiled_tflops": flops / t_tiled / 1e12, "plan": K.moe_tiles(M * topk, E, N, Kd),
+    res[M] = {"tiled_ms": t_tiled * 1e3, "tiled_tflops": flops / t_tiled / 1e12, "plan": K.moe_rows(M * topk, E, N, Kd),
               "plans": plans, "wstream_ms": t_stream * 1e3, "wstream_tflops": flops / t_stream / 1e12}
     print(M, res[M])
 Path("gpurun_out").mkdir(exist_ok=True)

@@ -1148,7 +1148,7 @@ def moe_tiled_gemm(a: torch.Tensor, w: torch.Tensor, c: torch.Tensor, sorted_tok
                    mul_routed_weight: bool, top_k_div: int, num_valid_ids: int, block_m: int, fuse_silu: bool = False,
                    round_before_scale: bool = False, tile_rows: Optional[int] = None, act: Glu = SILU) -> torch.Tensor:
     """moe_grouped_gemm on the row-tiled MFMA kernels (prefill-sized batches): block_m = the align block size (128 or
-    256), tile_rows = rows of an expert per workgroup tile (128, or 256 over a 256 alignment: the 256 x 256 x 64 form);
+    256), tile_rows = rows of an expert per workgroup tile (128, or 256 over a 256 alignment: even tiles of up to 320 rows);
     a [rows, K] bf16, w [E, N(or 2N), K] bf16, c [num_valid_ids, N] bf16 or fp32."""
     _dev(a, w, c, sorted_token_ids, expert_ids, num_tokens_post_padded)
     tile_rows = block_m if tile_rows is None else tile_rows
@@ -1236,6 +1236,19 @@ def moe_tiles(numel: int, num_experts: int, n_up: int, n_down: int):
     if plan[0] == 128 and rows >= MOE_HALF_TILE_MIN_ROWS and workgroups >= MOE_HALF_TILE_MIN_WORKGROUPS:
         return 256, 256, 256
     return plan
+
+
+def moe_rows(numel: int, num_experts: int, n_up: int, n_down: int):
+    """moe_tiles, and the 256-row alignment, whose experts are cut into even tiles of up to 320 rows (moe_rows_kernel), also for smaller experts where
+    the up projection has tiles for the chip: from 140 rows on with 640 column tiles of 128 over all experts, from 300 on with 256.  Both products
+    in us, 128 rows / even: 64 experts of 1408 / 2048 (704) with 120 rows 349 / 355, with 140 387 / 375, with 230 528 / 477; 8 of 14336 / 4096 (896) with
+    140 857 / 854, with 200 939 / 852, with 230 1186 / 923; 32 of 7168 / 4096 with 100 1281 / 1279, with 150 1569 / 1363; 128 of 768 / 2048 (768) with 150
+    503 / 492, with 260 758 / 629; 32 of 2048 / 2048 (512) with 230 334 / 361, with 300 412 / 388; 16 of 2048 / 2048 (256) with 260 199 / 207, with 300
+    218 / 216, with 400 262 / 241; 4 of 1024 / 1024 (32) with 600 53 / 74."""
+    rows, tiles = numel / max(1, num_experts), num_experts * -(-n_up // 128)
+    if (tiles >= 640 and rows >= 140) or (tiles >= 256 and rows >= 300):
+        return 256, 256, 256
+    return moe_tiles(numel, num_experts, n_up, n_down)
 
 
 def moe_grouped_gemm(a: torch.Tensor, w: torch.Tensor, c: torch.Tensor, sorted_token_ids: torch.Tensor,
@@ -1353,7 +1366,7 @@ def fused_experts(hidden_states: torch.Tensor, w13: torch.Tensor, w2: torch.Tens
         return out
     if _row_tiled(numel, E, N) and K % 64 == 0 and N % 64 == 0:
         # prefill-sized batch: row-tiled MFMA kernels, every expert's weights read once per 128 / 256 of its rows
-        block_m, up_rows, down_rows = moe_tiles(numel, E, N, K)
+        block_m, up_rows, down_rows = moe_rows(numel, E, N, K)
         if MOE_TILE_OVERRIDE is not None:
             block_m, up_rows, down_rows = MOE_TILE_OVERRIDE
         sorted_ids, expert_ids, post = moe_align_block_size(topk_ids, block_m, E)

@@ -333,3 +333,53 @@ def test_256_row_tiles_whose_second_half_is_empty(device, loads, fuse_silu):
         outs.append(c)
     assert bool(torch.isfinite(outs[1].float()).all())
     assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("loads,N,Kd", [((159, 160, 161, 15, 16, 17), 128, 64), ((319, 320, 321, 0, 641, 1), 260, 128), ((1000, 33, 0, 255, 256, 257), 1000, 192),
+                                        (tuple(range(0, 200, 2)), 256, 64), ((2500, 170), 2048, 320)])
+@pytest.mark.parametrize("fuse_silu", [True, False])
+def test_even_row_tiles(device, loads, N, Kd, fuse_silu):
+    """Experts cut into even tiles of up to 320 rows: loads at the edges of a 16-row unit, of the fewest and the most units of a tile, none, more
+    experts than a wave has lanes, more tiles than compute units, one and two K steps, ragged columns; rows gathered two to a source row.
+    Bit for bit the 128-row form's (the same products summed in the same order)."""
+    K = _k()
+    g = torch.Generator().manual_seed(sum(loads) + N)
+    M, E = sum(loads), len(loads)
+    N = N // 32 * 32 if fuse_silu else N
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(loads))[torch.randperm(M, generator=g)].to(torch.int32).view(M, 1).to(device)
+    a = torch.randn(((M + 1) // 2, Kd), generator=g).to(BF).to(device)
+    w = (torch.randn((E, N * (2 if fuse_silu else 1), Kd), generator=g) * 0.05).to(BF).to(device)
+    tw = torch.rand(M, generator=g).to(device)
+    s, e, post = K.moe_align_block_size(ids, 256, E)
+    outs = []
+    for rows in (128, 256):
+        c = torch.full((M, N), float("nan"), dtype=BF if fuse_silu else torch.float32, device=device)
+        K.moe_tiled_gemm(a, w, c, s, e, post, None if fuse_silu else tw, not fuse_silu, 2, M, 256, fuse_silu=fuse_silu, round_before_scale=not fuse_silu, tile_rows=rows)
+        outs.append(c)
+    assert bool(torch.isfinite(outs[1].float()).all())
+    assert torch.equal(outs[0], outs[1])
+
+
+def test_even_row_tiles_of_filtered_experts_and_of_too_many_runs(device):
+    """Blocks of an expert below 0 stay untouched; metadata with more runs of blocks than the launch's table holds (experts that take turns) is
+    multiplied block by block."""
+    K = _k()
+    g = torch.Generator().manual_seed(3)
+    for experts, per in (((0, 0, -1, 1, 1, 1, -1, -1, 2, 0), 200), (tuple(i % 2 for i in range(1100)), 3)):
+        blocks, N, Kd = len(experts), 96, 128
+        s = torch.full((blocks, 256), blocks * per, dtype=torch.int32)
+        s[:, :per] = torch.randperm(blocks * per, generator=g).to(torch.int32).view(blocks, per)
+        if per == 200:
+            s[0] = torch.arange(blocks * per, blocks * per + 256)                   # (rows of an expert: whole blocks, then the rest)
+            s[[0, 3, 4]] = torch.randperm(3 * 256, generator=g).to(torch.int32).view(3, 256)
+            s[[1, 2, 5, 6, 7, 8, 9], :] = blocks * per
+            for i, b in enumerate((1, 2, 5, 6, 7, 8, 9)):
+                s[b, :per] = torch.arange(3 * 256 + i * per, 3 * 256 + (i + 1) * per, dtype=torch.int32).clamp(max=blocks * per)
+        M = blocks * per
+        a, w = torch.randn((M, Kd), generator=g).to(BF).to(device), (torch.randn((3, N, Kd), generator=g) * 0.05).to(BF).to(device)
+        e, post, outs = torch.tensor(experts, dtype=torch.int32, device=device), torch.tensor([blocks * 256], dtype=torch.int32, device=device), []
+        for rows in (128, 256):
+            c = torch.full((M, N), 7.0, dtype=BF, device=device)
+            K.moe_tiled_gemm(a, w, c, s.view(-1).to(device), e, post, None, False, 1, M, 256, tile_rows=rows)
+            outs.append(c)
+        assert torch.equal(outs[0], outs[1])

@@ -19,6 +19,13 @@ def test_experts_that_half_tiles_pay_for():
         assert K.moe_tiles(pairs, experts, up, down) == (rows,) * 3, (pairs, experts, up, down)
 
 
+def test_experts_that_even_tiles_pay_for():
+    for pairs, experts, up, down, rows in ((64 * 140, 64, 1408, 2048, 256), (64 * 139, 64, 1408, 2048, 128), (8 * 140, 8, 14336, 4096, 256),
+                                           (8 * 100, 8, 14336, 4096, 128), (32 * 230, 32, 2048, 2048, 128), (16 * 300, 16, 2048, 2048, 256),
+                                           (16 * 299, 16, 2048, 2048, 128), (4 * 600, 4, 1024, 1024, 128), (8 * 1024, 8, 14336, 4096, 256)):
+        assert K.moe_rows(pairs, experts, up, down) == (rows,) * 3, (pairs, experts, up, down)
+
+
 def test_where_the_row_tiles_begin():
     for pairs, experts, up, tiled in ((8 * 56, 8, 14336, True), (8 * 55, 8, 14336, False), (4 * 95, 4, 1024, False), (4 * 96, 4, 1024, True),
                                       (8 * 56, 8, 2048, True), (8 * 1000, 8, 64, True)):
