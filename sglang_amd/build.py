@@ -10,8 +10,11 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
+import tempfile
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
+from typing import Optional
 
 PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
@@ -115,6 +118,29 @@ def build(force: bool = False, verbose: bool = False, group: str = "all") -> Pat
         res = subprocess.run(cmd, capture_output=True, text=True)
         if res.returncode != 0:
             raise RuntimeError(f"link failed:\n{res.stdout}\n{res.stderr}")
+    build_calls()
+    return out
+
+
+def build_calls(out: Optional[Path] = None, header: Optional[Path] = None) -> Optional[Path]:
+    """Compile the Python calls of the C ABI (binding/calls.cpp) for this interpreter; None where its headers are not installed (native.call() then
+    goes through ctypes)."""
+    from . import native
+
+    include = Path(sysconfig.get_paths()["include"])
+    if not (include / "Python.h").exists():
+        return None
+    header, out = header or native.HEADER_PATH, out or native.CALLS_PATH
+    out.parent.mkdir(exist_ok=True)
+    names = "".join(f" X({i}, {n})" for i, n in enumerate(native.parse_header(header)))
+    with tempfile.TemporaryDirectory() as tmp:
+        listing = Path(tmp) / "names.h"
+        listing.write_text(f'#define SGL_AMD_NAMES(X){names}\n#define SGL_AMD_HEADER_DIGEST "{native.header_digest(header)}"\n')
+        cmd = [_hipcc(), "-x", "c++", "-O2", "-std=c++17", "-shared", "-fPIC", "-include", str(listing), f"-I{header.parent}", f"-I{include}",
+               str(PKG / "binding" / "calls.cpp"), "-o", str(out), "-ldl"]
+        res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"the C ABI's calls did not compile:\n{res.stdout}\n{res.stderr}")
     return out
 
 

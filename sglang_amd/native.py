@@ -6,6 +6,9 @@ If the shared object is missing or a call fails, a RuntimeError is raised.
 from __future__ import annotations
 
 import ctypes
+import hashlib
+import importlib.machinery
+import importlib.util
 import os
 import re
 from pathlib import Path
@@ -23,13 +26,33 @@ LIB_PATH = PKG / "lib" / "libsglang_amd.so"
 HEADER_PATH = next((h for h in (PKG / "include" / "sglang_amd.h", PKG.parent / "include" / "sglang_amd.h") if h.exists()),
                    PKG / "include" / "sglang_amd.h")
 
+CALLS_PATH = PKG / "lib" / "_calls.so"
+
 _lib = None
 _sigs: Dict[str, List] = {}
+_calls: Dict[str, object] = {}          # name -> the entry point as a Python function (binding/calls.cpp)
 
 
-def _parse_header() -> Dict[str, List]:
-    """Derive argtypes from include/sglang_amd.h so the binding cannot drift."""
-    text = HEADER_PATH.read_text()
+def header_digest(header: Path) -> str:
+    return hashlib.sha256(header.read_bytes()).hexdigest()
+
+
+def _load_calls(library: Path) -> Dict[str, object]:
+    """The entry points of `library` without ctypes, or none: not built for this interpreter, or for another header than this one."""
+    if not CALLS_PATH.exists():
+        return {}
+    loader = importlib.machinery.ExtensionFileLoader("_calls", str(CALLS_PATH))
+    try:
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_calls", loader))
+        loader.exec_module(module)
+    except ImportError:
+        return {}
+    return module.bind(str(library)) if module.header_digest == header_digest(HEADER_PATH) else {}
+
+
+def parse_header(header: Path) -> Dict[str, List]:
+    """{name: [return type, argtypes]} of a C header, so the binding cannot drift."""
+    text = header.read_text()
     text = re.sub(r"/\*.*?\*/", "", text, flags=re.S)
     sigs: Dict[str, List] = {}
     for m in re.finditer(r"\b(int64_t|int|const char\*)\s+(sgl_amd_\w+)\s*\(([^;]*?)\)\s*;", text, flags=re.S):
@@ -53,7 +76,7 @@ def _parse_header() -> Dict[str, List]:
 
 
 def declared_symbols() -> List[str]:
-    return sorted(_parse_header().keys())
+    return sorted(parse_header(HEADER_PATH).keys())
 
 
 _group = "all"
@@ -72,7 +95,7 @@ def ensure(group: str = "all") -> None:
 
 
 def lib() -> ctypes.CDLL:
-    global _lib, _sigs
+    global _lib, _sigs, _calls
     if _lib is not None:
         return _lib
     # ORDER MATTERS: torch bundles its own libamdhip64.so (SONAME libamdhip64.so.7).  It must be
@@ -91,7 +114,7 @@ def lib() -> ctypes.CDLL:
             "There is no CPU/torch fallback for this path."
         )
     cdll = ctypes.CDLL(str(path))
-    _sigs = _parse_header()
+    _sigs = parse_header(HEADER_PATH)
     for name, (ret, argtypes) in _sigs.items():
         try:
             fn = getattr(cdll, name)
@@ -101,6 +124,7 @@ def lib() -> ctypes.CDLL:
             raise RuntimeError(f"{path} does not export {name} (declared in sglang_amd.h)") from e
         fn.argtypes = argtypes
         fn.restype = {"int": ctypes.c_int, "int64_t": ctypes.c_int64}.get(ret, ctypes.c_char_p)
+    _calls = _load_calls(path)
     _lib = cdll
     return cdll
 
@@ -112,7 +136,9 @@ def last_error() -> str:
 
 def call(name: str, *args) -> None:
     """Call an int-returning entry point; raise RuntimeError on a non-zero status."""
-    fn = getattr(_lib or lib(), name)
-    rc = fn(*args)
+    fn = _calls.get(name)
+    rc = NotImplemented if fn is None else fn(*args)
+    if rc is NotImplemented:
+        rc = getattr(_lib or lib(), name)(*args)
     if rc != 0:
         raise RuntimeError(f"{name} failed (status {rc}): {last_error()}")
