@@ -586,9 +586,8 @@ __global__ __launch_bounds__(kThreads2, 1) void moe_rows_kernel(TiledParams p) {
         tiles += __shfl_xor(tiles, off, 64);
         fullest = max(fullest, __shfl_xor(fullest, off, 64));
       }
-      // a step's clocks in units of 128: the products of the pairs of 16-row tiles of both halves of the rows and 1.1 k beside them, and what its requests take
-      const int pairs = (((fullest + 1) / 2 + 1) / 2) + ((fullest / 2 + 1) / 2);
-      if (lane == 0) scratch[16 + m] = (tiles * cols + kNumCus - 1) / kNumCus * max(24, 2 * pairs + 9);
+      // a step's clocks in units of 128: the products of the fullest tile and 1.1 k beside them, or what its requests take
+      if (lane == 0) scratch[16 + m] = (tiles * cols + kNumCus - 1) / kNumCus * max(24, fullest + 9);
     }
     __syncthreads();
     int least = 0x7fffffff;
@@ -723,12 +722,12 @@ __global__ __launch_bounds__(kThreads2, 1) void moe_rows_kernel(TiledParams p) {
     wf[0] = lds_rd<0>(ad); wf[1] = lds_rd<2048>(ad); wf[2] = lds_rd<4096>(ad); wf[3] = lds_rd<6144>(ad);
   };
   const int nk = p.K / kBK;
-  // The steps of a wave with PAIRS pairs of token tiles (the last one maybe of one).  Issue the next step's tiles, read and multiply this step's, wait,
+  // The steps of a wave with TILES token tiles, two at a time.  Issue the next step's tiles, read and multiply this step's, wait,
   // barrier.  The fragments of a pair are read a pair ahead of its eight products.  (Of 256-row tiles, measured equal to 5 % slower: a barrier ahead of the last
   // quarter with the next stage's first fragments read behind it.  Touching a step's 64 lines one to three steps ahead, so that they wait in L2: 5
   // to 7 % slower, first-touch latency is not what the walk waits for -- profiles/r04_exp4_moe_gemm_ab.json.  Products of 32 x 32: 7 % slower.)
-  auto walk = [&](auto pairs_of, uint32_t x_base) __attribute__((always_inline)) {
-    constexpr int PAIRS = decltype(pairs_of)::value;
+  auto walk = [&](auto tiles_of, uint32_t x_base) __attribute__((always_inline)) {
+    constexpr int TILES = decltype(tiles_of)::value, PAIRS = (TILES + 1) / 2;
 #pragma clang loop unroll(disable)
     for (int kt = 0; kt < nk; ++kt) {
       const int stage = kt & 1;
@@ -739,7 +738,7 @@ __global__ __launch_bounds__(kThreads2, 1) void moe_rows_kernel(TiledParams p) {
         auto read_x = [&](auto n) __attribute__((always_inline)) {                    // pair n of both halves of the step
           constexpr int KK = decltype(n)::value / PAIRS, JP = decltype(n)::value % PAIRS;
           xf[decltype(n)::value & 1][0] = lds_rd<JP * 4096>(xa + foff[KK]);
-          xf[decltype(n)::value & 1][1] = lds_rd<JP * 4096 + 2048>(xa + foff[KK]);
+          if constexpr (2 * JP + 1 < TILES) xf[decltype(n)::value & 1][1] = lds_rd<JP * 4096 + 2048>(xa + foff[KK]);
         };
         read_w(wa + foff[0], wf[0]);
         read_x(std::integral_constant<int, 0>{});
@@ -750,16 +749,16 @@ __global__ __launch_bounds__(kThreads2, 1) void moe_rows_kernel(TiledParams p) {
           if constexpr (NN + 1 < 2 * PAIRS) {
             if constexpr (NN + 1 == PAIRS) read_w(wa + foff[1], wf[1]);
             read_x(std::integral_constant<int, NN + 1>{});
-            wait_lgkm<NN + 1 == PAIRS ? 6 : 2>();
+            wait_lgkm<(NN + 1 == PAIRS ? 4 : 0) + (2 * ((NN + 1) % PAIRS) + 1 < TILES ? 2 : 1)>();
           } else {
             wait_lgkm<0>();
           }
 #pragma unroll
           for (int i = 0; i < 4; ++i) pin(wf[KK][i]);
           pin(xf[NN & 1][0]);
-          pin(xf[NN & 1][1]);
+          if constexpr (2 * JP + 1 < TILES) pin(xf[NN & 1][1]);
 #pragma unroll
-          for (int j = 0; j < 2; ++j)
+          for (int j = 0; j < (2 * JP + 1 < TILES ? 2 : 1); ++j)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
               acc[i][2 * JP + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[KK][i]), __builtin_bit_cast(bf16x8_t, xf[NN & 1][j]),
@@ -811,7 +810,12 @@ __global__ __launch_bounds__(kThreads2, 1) void moe_rows_kernel(TiledParams p) {
 #pragma unroll
         for (int j = 0; j < MOST; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       const uint32_t x_base = sm_addr + kOpW + (wh ? half0 * 2048 : 0);
-      switch ((mine + 1) >> 1) {
+      switch (mine) {
+        case 10: walk(std::integral_constant<int, 10>{}, x_base); break;
+        case 9: walk(std::integral_constant<int, 9>{}, x_base); break;
+        case 8: walk(std::integral_constant<int, 8>{}, x_base); break;
+        case 7: walk(std::integral_constant<int, 7>{}, x_base); break;
+        case 6: walk(std::integral_constant<int, 6>{}, x_base); break;
         case 5: walk(std::integral_constant<int, 5>{}, x_base); break;
         case 4: walk(std::integral_constant<int, 4>{}, x_base); break;
         case 3: walk(std::integral_constant<int, 3>{}, x_base); break;
