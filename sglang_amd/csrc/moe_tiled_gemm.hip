@@ -523,7 +523,7 @@ __device__ __forceinline__ u32x4_t lds_quad(uint32_t addr) {
 // quarters of a whole tile's time).  One workgroup a compute unit, and it stays: in rounds of workgroups there were 2.4 us in front of a tile's steps
 // (100 us of K = 4096), 14 behind and the 10 to 15 until the next workgroup ran.  The next tile's first two stages are asked for in front of the
 // outputs, its rows and expert a tile before.
-// us, tiles of 256 in rounds of workgroups / these: 8 experts of 14336 / 4096, 3000 tokens 2303 / 2014, 2048 1814 / 1595, 1500 1213 / 1195, 1000 1133 / 929.
+// us, tiles of 256 in rounds of workgroups / these: 8 experts of 14336 / 4096, 3000 tokens 2303 / 1990, 2048 1814 / 1595, 1500 1213 / 1181, 1000 1133 / 919.
 __global__ __launch_bounds__(kThreads2, 1) void moe_rows_kernel(TiledParams p) {
   __shared__ __attribute__((aligned(1024))) unsigned char smem[2 * kStage3 + kRuns * 16];
   const int tid = threadIdx.x, lane = tid & 63;
