@@ -787,7 +787,9 @@ int launch_main(WsParams p, hipStream_t st, int row_blocks = 0) {
     // One workgroup fits on a compute unit.  More groups than compute units, in rounds of workgroups, let the ring run dry at every round's
     // end; workgroups that stay keep it filled: [64, 128256, 4096] 184 -> 177 us (one row 169 -> 156), silu [16, 57344, 8192] 157 -> 142.
     // Groups are as narrow as the number of rounds allows, so that the last round is as full as the others: silu [24, 9728, 896] 10.9 -> 8.9
-    // (76 groups of four pairs / 152 of two), [64, 32000, 4096] in eight waves 56.4 -> 41.8.
+    // (76 groups of four pairs / 152 of two), [64, 32000, 4096] in eight waves 56.4 -> 41.8.  At least two pairs a group would be
+    // slower: silu of 16 rows, one / two, [8192, 4096] 16.6 / 19.1, [5120, 14336] 47.3 / 51.2, [2048, 1024] 5.6 / 6.0.  Launches of two waves, with a deeper
+    // ring, are no quicker either: silu of 64 rows, four / two, [8192, 4096] 23.2 / 24.5, [4096, 896] 8.5 / 8.8.
     const int wtiles = p.ntiles / TPW;
     const bool stays = p.splits == 1 && !row_blocks;
     const int rounds = ((wtiles + NW - 1) / NW + kNumCus - 1) / kNumCus;
