@@ -33,6 +33,7 @@
 
 #include "common.hpp"
 #include "glu.hpp"
+#include "row_tiles.hpp"
 #include "sglang_amd.h"
 
 using namespace sgl_amd;
@@ -657,9 +658,9 @@ __global__ __launch_bounds__(kThreads2, 1) void moe_rows_kernel(TiledParams p) {
       const int first = __builtin_amdgcn_readfirstlane(t.x), all = __builtin_amdgcn_readfirstlane(t.y);
       const int tiles = (all + most - 1) / most, in = at - first * cols;
       w.nt = in / tiles;
-      const int k = in - w.nt * tiles, from = k * all / tiles;
-      w.units = (k + 1) * all / tiles - from;
-      w.row0 = (__builtin_amdgcn_readfirstlane(t.z) + from) * 16;
+      const RowTile tile = even_tile(all, tiles, in - w.nt * tiles);
+      w.units = tile.units;
+      w.row0 = (__builtin_amdgcn_readfirstlane(t.z) + tile.from) * 16;
       w.e = __builtin_amdgcn_readfirstlane(t.w);
     } else {
       w.nt = at - rt * cols;
