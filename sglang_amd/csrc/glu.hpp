@@ -36,14 +36,15 @@ __device__ __forceinline__ float squared_relu(float v) {
 
 // silu(g) of a g that is a bf16 value.  Up to |g| = 80 nothing over- or underflows, and a gate costs 12 instructions in the place of the 60 of
 // expf and a division for all cases: log2 e in two parts (Cody and Waite), the first of 16 bits, so that its product with the 8 bits of g is exact
-// and v_exp_f32 takes it as it is; the reciprocal's quotient once corrected.  Rounded to bf16 it equals silu_any() for every g.
-// us: 3000 tokens over 8 experts (64 outputs a lane at the end of a tile) 2243 -> 2194, 48 tokens 429 -> 426.6, a decode step of four layers 720 -> 716.
+// and v_exp_f32 takes it as it is; the reciprocal's quotient once corrected.  Rounded to bf16 it has silu_any()'s bits for all 65 536 g, -0 among them
+// (compared on the device; of a g that is no number the sign may differ).
+// us: 3000 tokens over 8 experts (64 outputs a lane at the end of a tile) 2243 -> 2194, a decode step of four layers 720 -> 716; 48 tokens the same.
 __device__ __forceinline__ float silu_near(float g) {                      // |g| <= 80, or no number
   const float e = fast_exp2(g * -0x1.7154p+0f);
   const float d = 1.0f + __builtin_fmaf(e, g * -0x1.480fb6p-18f, e);
   const float r = __builtin_amdgcn_rcpf(d);
   const float q = g * r;
-  return __builtin_fmaf(__builtin_fmaf(-d, q, g), r, q);
+  return __builtin_fmaf(-__builtin_fmaf(d, q, -g), r, q);                  // (this way round a gate of -0 keeps its sign)
 }
 __device__ __forceinline__ float silu_any(float g) { return g / (1.0f + expf(-g)); }
 
