@@ -670,7 +670,8 @@ int sgl_amd_delta_chunk(int is_f32, const void* qkv, int64_t qkv_stride, const v
     const int32_t* seg_start, const int32_t* seg_len, void* o, int64_t o_stride, int segments, int heads, int kv_heads,
     int key_dim, int value_dim, float q_scale, void* stream);
 /* The same in two launches over a workspace (16-bit rows; others take what sgl_amd_delta_chunk does).  _workspace: bytes for `tokens` packed tokens in
-   `segments` segments whose longest has max_len, 0: one launch is as good, or the workspace would be too large.  The segments do not overlap. */
+   `segments` segments whose longest has max_len, 0: one launch is as good, or the workspace would be too large.  The segments do not overlap.
+   A segment that `tokens` leaves no room for has no numbers (NaN) for outputs, and its state stays as it is. */
 int64_t sgl_amd_delta_chunk_workspace(int64_t tokens, int segments, int max_len, int heads, int key_dim, int value_dim);
 int sgl_amd_delta_chunk_ws(int is_f32, const void* qkv, int64_t qkv_stride, const void* b, const void* a, int64_t ba_stride,
     const float* A_log, const float* dt_bias, float* state, const int64_t* slots, const int64_t* positions,

@@ -63,7 +63,13 @@ __device__ __forceinline__ void delta_prepare_body(const Params& p, DeltaPrep& s
   const int chunks = (total + Q - 1) / Q;
   if (static_cast<int>(blockIdx.y) >= chunks) return;
   const int64_t tok0 = p.seg_start[b], first = delta_units_before(p.seg_len, b, threadIdx.x & 63);
-  if (first + chunks > p.units) return;
+  if (first + chunks > p.units) {                // more tokens than the caller said: the walk leaves the segment out, and nobody takes its outputs for results
+    uint16_t* o = static_cast<uint16_t*>(p.o) + tok0 * p.o_stride + h * p.V;
+    for (int k = blockIdx.y; k < chunks; k += gridDim.y)
+      for (int t = k * Q; t < total && t < (k + 1) * Q; ++t)
+        for (int v = threadIdx.x & 63; v < p.V; v += 64) o[t * p.o_stride + v] = 0x7fc0;
+    return;
+  }
   const float a = -expf(p.A_log[h]), dtb = p.dt_bias[h];
   for (int k = blockIdx.y; k < chunks; k += gridDim.y) {       // (once, but for segments beyond two million tokens)
     int lane = threadIdx.x & 63;

@@ -354,3 +354,41 @@ def test_delta_rule_in_two_launches(device, heads, groups, K, V, decay, copies):
     # the same bits every time
     again, state2 = run(act.to(device), True)
     assert torch.equal(again, y) and torch.equal(state2, state)
+
+
+@pytest.mark.parametrize("V,copies", [(128, 1), (72, 1), (128, 70)])
+def test_segments_that_the_callers_tokens_leave_no_room_for(device, V, copies):
+    """More tokens in the segments than the call says: what has room is computed as ever, the rest has no numbers for outputs (and never the buffer's old ones) and
+    keeps its state; by the fetching wave's form and by the one of more workgroups than compute units."""
+    heads, K, lens = 2, 64, [64] * copies + [320, 5]
+    g = torch.Generator().manual_seed(V + copies)
+    T = sum(lens)
+    qkv = torch.randn(T, 2 * heads * K + heads * V, generator=g).to(BF).to(device)
+    gt = torch.randn(T, 2 * heads, generator=g).to(BF).to(device)
+    A_log, bias = (torch.randn(heads, generator=g).to(device) for _ in range(2))
+    state0 = torch.randn(len(lens), heads, K, V, generator=g).to(device)
+    slots = torch.arange(len(lens), device=device)
+    length = torch.tensor(lens, dtype=torch.int32, device=device)
+    start = (length.cumsum(0) - length).to(torch.int32)
+    pos = torch.cat([torch.arange(n) + 1 for n in lens]).to(device)
+    outs = []
+    for tokens in (T, 32 * (2 * copies + 3 - len(lens))):                 # (room for all; for three chunks more than the copies have)
+        state, o = state0.clone(), torch.full((T, heads * V), 7.0, dtype=BF, device=device)
+        units = (tokens // 32 + len(lens)) * heads * 10240
+        ws = torch.empty(units, dtype=torch.uint8, device=device)
+        native.call("sgl_amd_delta_chunk_ws", 0, qkv.data_ptr(), qkv.stride(0), gt.data_ptr(), gt[:, heads:].data_ptr(), gt.stride(0), A_log.data_ptr(), bias.data_ptr(),
+                    state.data_ptr(), slots.data_ptr(), pos.data_ptr(), start.data_ptr(), length.data_ptr(), o.data_ptr(), o.stride(0), len(lens), heads, heads, K, V,
+                    K ** -0.5, tokens, max(lens), ws.data_ptr(), units, torch.cuda.current_stream().cuda_stream)
+        outs.append((o, state))
+    (o, state), (o2, state2) = outs
+    assert bool(o.isfinite().all())
+    room, at, cut = tokens // 32 + len(lens), 0, []
+    for n in lens:
+        at += -(-n // 32)
+        cut.append(at > room)
+    assert any(cut) and not cut[0]
+    for i, (lo, n) in enumerate(zip(start.tolist(), lens)):
+        if cut[i]:
+            assert bool(o2[lo:lo + n].isnan().all()) and torch.equal(state2[i], state0[i]), i
+        else:
+            assert torch.equal(o2[lo:lo + n], o[lo:lo + n]) and torch.equal(state2[i], state[i]), i
