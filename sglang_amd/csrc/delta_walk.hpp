@@ -277,7 +277,8 @@ struct DeltaWalk {
   }
 };
 
-// 16 bytes a lane from memory to 1 KiB of LDS at `to`; the issuing wave waits (vmcnt) in front of the barrier behind which they are read
+// 16 bytes a lane from memory to 1 KiB of LDS at `to`; the issuing wave waits (vmcnt) in front of the barrier behind which they are read.
+// (Nothing else here may use M0, which cannot be named as overwritten: test_no_spills.py looks for it in the listing.)
 __device__ __forceinline__ void piece_to_lds(const void* from, uint32_t to) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(from), "s"(to) : "memory");
 }

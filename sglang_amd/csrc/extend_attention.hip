@@ -881,7 +881,7 @@ struct SmemLadder {
 
 // 16 bytes a lane from memory to 1 KiB of LDS at `to`, behind the compiler's back: it would wait for all of these in front of the next read
 // of LDS.  Whoever issues them waits (rows_landed) and meets the others at a barrier before any of it is read.  No registers are written, and
-// nothing else here uses M0.  Rows that went through registers cost a step 300 of its 3900 clocks: all waves write LDS behind the barrier while
+// nothing else here uses M0 (which cannot be named as overwritten; test_no_spills.py looks for other users of it in the listing).  Rows that went through registers cost a step 300 of its 3900 clocks: all waves write LDS behind the barrier while
 // no product runs.  us, through registers / straight to LDS: 60 x 128 behind 896, 32 / 8 heads, 166 / 162, six cold prompts of 1.1 to 3.1 k, 64 / 8
 // heads, 619 / 603 (both at a lower clock in turn: power), 6 x 2000 cold, 14 / 2 heads of 64, 79 / 68, 1000 cold 26.0 / 23.5, 203 behind 3800 35.2 / 33.2.
 __device__ __forceinline__ void rows_to_lds(const unsigned char* from, uint32_t to) {

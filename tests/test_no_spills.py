@@ -185,3 +185,28 @@ def test_split_recurrences_keep_their_registers_and_lds(tmp_path):
         for name, u in inst.items():
             assert u["vgpr_spill_count"] == 0 and u["vgpr_count"] <= 256, (name, u)
             assert u["group_segment_fixed_size"] <= 160 * 1024, (name, u)
+
+
+@pytest.mark.skipif(not Path(HIPCC).exists(), reason="hipcc not installed")
+@pytest.mark.parametrize("src,kernels", [("extend_attention.hip", ("extend_attention_pipe_kernel", "extend_attention_walk_kernel", "extend_attention_parts_kernel")),
+                                         ("recurrent_chunk.hip", ("delta_walk_kernel", "delta_walk_self_kernel"))])
+def test_requests_into_lds_are_alone_with_m0(tmp_path, src, kernels):
+    """The requests written in assembly set M0, which the compiler does not let a statement name as overwritten: a value of its own that it
+    kept there across one would be lost.  So these kernels hold no other instruction that writes or needs it."""
+    usage, at, inside, seen = _resource_usage(src, tmp_path), None, False, {}
+    for line in (tmp_path / "k.s").read_text().splitlines():
+        m = re.match(r"(_Z\w+):", line)
+        if m:
+            at, inside = next((k for k in kernels if re.search(rf"\d{k}I", m.group(1))), None), False
+        elif line.startswith(".Lfunc_end"):
+            at = None
+        elif at is not None:
+            code = line.split(";")[0]
+            if "#ASMSTART" in line or "#ASMEND" in line:
+                inside = "#ASMSTART" in line
+            elif re.search(r"\bm0\b", code) or "_load_lds" in code:
+                assert inside, (at, line)
+                seen[at] = seen.get(at, 0) + 1
+            else:
+                assert not re.match(r"\s*(s_sendmsg|s_movrel|v_movrel|v_interp|ds_gws|ds_ordered|s_ttrace|buffer_load\S*.*\blds\b)", code), (at, line)
+    assert usage and all(seen.get(k, 0) >= 2 for k in kernels), seen
