@@ -26,7 +26,8 @@ LIB_PATH = PKG / "lib" / "libsglang_amd.so"
 HEADER_PATH = next((h for h in (PKG / "include" / "sglang_amd.h", PKG.parent / "include" / "sglang_amd.h") if h.exists()),
                    PKG / "include" / "sglang_amd.h")
 
-CALLS_PATH = PKG / "lib" / "_calls.so"
+# (named for the interpreter that it was built for: CPython does not look whether a file that it is told to load is for another one)
+CALLS_PATH = PKG / "lib" / ("_calls" + importlib.machinery.EXTENSION_SUFFIXES[0])
 
 _lib = None
 _sigs: Dict[str, List] = {}

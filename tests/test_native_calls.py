@@ -1,6 +1,7 @@
 """The C ABI's Python calls (binding/calls.cpp) convert every argument as ctypes does, and step aside where they cannot."""
 import ctypes
 import subprocess
+import sysconfig
 
 import pytest
 
@@ -72,3 +73,7 @@ def test_what_is_left_to_ctypes(both):
         assert calls["sgl_amd_wide"](odd) is NotImplemented
     buf = (ctypes.c_int64 * 12)()
     assert calls["sgl_amd_echo"](ctypes.byref(buf), *([0] * 12)) is NotImplemented and calls["sgl_amd_echo"](0, 1.0, *([0] * 11)) is NotImplemented
+
+
+def test_another_interpreters_module_is_not_looked_at():
+    assert native.CALLS_PATH.name == "_calls" + sysconfig.get_config_var("EXT_SUFFIX") and sysconfig.get_config_var("SOABI") in native.CALLS_PATH.name
