@@ -118,29 +118,34 @@ def build(force: bool = False, verbose: bool = False, group: str = "all") -> Pat
         res = subprocess.run(cmd, capture_output=True, text=True)
         if res.returncode != 0:
             raise RuntimeError(f"link failed:\n{res.stdout}\n{res.stderr}")
-    build_calls()
+    build_calls(force=force)
     return out
 
 
-def build_calls(out: Optional[Path] = None, header: Optional[Path] = None) -> Optional[Path]:
-    """Compile the Python calls of the C ABI (binding/calls.cpp) for this interpreter; None where its headers are not installed (native.call() then
-    goes through ctypes)."""
+def build_calls(out: Optional[Path] = None, header: Optional[Path] = None, force: bool = False) -> Optional[Path]:
+    """Compile (if stale) the Python calls of the C ABI (binding/calls.cpp) for this interpreter; None where its headers are not installed (native.call()
+    then goes through ctypes).  The file appears whole: a process that loads or builds it meanwhile finds the old one or the new one."""
     from . import native
 
     include = Path(sysconfig.get_paths()["include"])
     if not (include / "Python.h").exists():
         return None
     header, out = header or native.HEADER_PATH, out or native.CALLS_PATH
+    source = PKG / "binding" / "calls.cpp"
+    made_of = (source, header, Path(__file__), Path(native.__file__), include / "Python.h")
+    if not force and out.exists() and out.stat().st_mtime >= max(f.stat().st_mtime for f in made_of):
+        return out
     out.parent.mkdir(exist_ok=True)
     names = "".join(f" X({i}, {n})" for i, n in enumerate(native.parse_header(header)))
-    with tempfile.TemporaryDirectory() as tmp:
-        listing = Path(tmp) / "names.h"
+    with tempfile.TemporaryDirectory(dir=out.parent) as tmp:
+        listing, made = Path(tmp) / "names.h", Path(tmp) / "calls"
         listing.write_text(f'#define SGL_AMD_NAMES(X){names}\n#define SGL_AMD_HEADER_DIGEST "{native.header_digest(header)}"\n')
         cmd = [_hipcc(), "-x", "c++", "-O2", "-std=c++17", "-shared", "-fPIC", "-include", str(listing), f"-I{header.parent}", f"-I{include}",
-               str(PKG / "binding" / "calls.cpp"), "-o", str(out), "-ldl"]
+               str(source), "-o", str(made), "-ldl"]
         res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode != 0:
-        raise RuntimeError(f"the C ABI's calls did not compile:\n{res.stdout}\n{res.stderr}")
+        if res.returncode != 0:
+            raise RuntimeError(f"the C ABI's calls did not compile:\n{res.stdout}\n{res.stderr}")
+        os.replace(made, out)
     return out
 
 

@@ -1,5 +1,6 @@
 """The C ABI's Python calls (binding/calls.cpp) convert every argument as ctypes does, and step aside where they cannot."""
 import ctypes
+import os
 import subprocess
 import sysconfig
 
@@ -77,3 +78,24 @@ def test_what_is_left_to_ctypes(both):
 
 def test_another_interpreters_module_is_not_looked_at():
     assert native.CALLS_PATH.name == "_calls" + sysconfig.get_config_var("EXT_SUFFIX") and sysconfig.get_config_var("SOABI") in native.CALLS_PATH.name
+
+
+def test_the_module_is_built_where_it_is_stale_and_replaced_whole(tmp_path, monkeypatch):
+    (tmp_path / "sglang_amd.h").write_text(HEADER)
+    header, out = tmp_path / "sglang_amd.h", tmp_path / "_calls.so"
+    if build.build_calls(out, header) is None:
+        pytest.skip("no Python headers")
+    first = out.stat()
+    assert build.build_calls(out, header) == out and out.stat() == first                # nothing to do
+    os.utime(header, (first.st_atime + 2, first.st_mtime + 2))
+    with out.open("rb") as reader:                                                      # (holds the old file)
+        monkeypatch.setenv("HIPCC", "/bin/false")
+        with pytest.raises(RuntimeError):
+            build.build_calls(out, header)
+        assert out.stat() == first                                                      # a failure leaves the old one
+        monkeypatch.delenv("HIPCC")
+        build.build_calls(out, header)
+        assert out.stat().st_ino != first.st_ino and os.fstat(reader.fileno()).st_ino == first.st_ino
+    made = out.stat()
+    build.build_calls(out, header, force=True)
+    assert out.stat().st_ino != made.st_ino and sorted(p.name for p in tmp_path.iterdir()) == ["_calls.so", "sglang_amd.h"]
