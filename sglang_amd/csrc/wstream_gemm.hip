@@ -813,7 +813,7 @@ int launch_main(WsParams p, hipStream_t st, int row_blocks = 0) {
     p.inv_splits = 1.f / static_cast<float>(p.splits);
     p.inv_grid = 1.f / static_cast<float>(grid.x);
     if (row_blocks) {
-      if constexpr (MT <= 4) hipLaunchKernelGGL((wstream_gemm_kernel<MT, NW, TPW, true>), grid, dim3(64 * NW), 0, st, p);
+      if constexpr (MT <= 4 && NW * TPW <= 8) hipLaunchKernelGGL((wstream_gemm_kernel<MT, NW, TPW, true>), grid, dim3(64 * NW), 0, st, p);
       else return -1;
     } else {
       hipLaunchKernelGGL((wstream_gemm_kernel<MT, NW, TPW, false>), grid, dim3(64 * NW), 0, st, p);
