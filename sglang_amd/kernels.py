@@ -959,10 +959,9 @@ def choose_wstream_decomposition(M: int, N: int, K: int, need_combine: bool = Fa
     nch = K // 128
 
     def pairs_time() -> float:
-        # up to 64 rows the launch deals the pairs of tiles out in the narrowest groups that the number of rounds allows
-        pairs, waves = N // 32, nw if M > 64 else 4
-        rounds = -(-pairs // (waves * _NUM_CUS))
-        width = waves if M > 64 else -(-pairs // (rounds * _NUM_CUS))
+        # the launch deals the pairs of tiles out in the narrowest groups that the number of rounds allows (compared only up to 64 rows: four waves)
+        pairs = N // 32
+        width = -(-pairs // (-(-pairs // (4 * _NUM_CUS)) * _NUM_CUS))
         return rounds_time(-(-pairs // width), width * nch * 8192, 6.0e12, 26e9)
 
     def rounds_time(groups: int, wg_bytes: int, chip: float, per_cu: float) -> float:
@@ -1202,12 +1201,14 @@ def _moe_tiles_us(rows_per_expert: float, num_experts: int, n_up: int, n_down: i
 
 def moe_tile_plan(numel: int, num_experts: int, n_up: int, n_down: int):
     """(align block, tile rows of the up projection, tile rows of the down projection) for a prefill-sized batch of
-    `numel` (token, k) pairs, where whole tiles decide (moe_tiles): the 256 x 256 x 64 form once an expert owns enough rows that the 256-row alignment's padding
+    `numel` (token, k) pairs, by lines that were fitted to whole 256 x 256 x 64 tiles (moe_gemm256_kernel).  Sizes past them run on moe_rows_kernel, whose even
+    tiles of up to 320 rows pay earlier: fused_experts asks moe_rows in front of this; for routed_experts, whose products of few rows those lines were not measured on, this
+    decides alone.  Whole tiles: once an expert owns enough rows that the 256-row alignment's padding
     (128 rows per expert on average) costs less than the form gains (measured on Mixtral's shapes, 4096 tokens = 1024 rows
     per expert: up projection 977 vs 714 TF/s, down projection 820-870 vs 715 with its 2.25 rounds of workgroups;
     profiles/r04_exp4_moe_gemm_ab.json).  Experts of 256 to 767 rows take it where rounds and padding together promise 9.5 % or more (a K step of
-    64 costs 1.84 us a 256 x 256 tile, one a CU, and 1.2 us a 128 x 128 tile, two a CU; below that the estimate is no better than the spread of the
-    experts' sizes).  Measured, both products in us, 128 / 256 rows: 8 experts of 14336 / 4096 with 575 rows each 2257 / 2004, with 639 2524 / 2190,
+    64 cost 1.84 us a whole tile, one a CU, and 1.2 us a 128 x 128 tile, two a CU; below that the estimate is no better than the spread of the
+    experts' sizes).  Measured, both products in us, 128 rows / whole tiles of 256: 8 experts of 14336 / 4096 with 575 rows each 2257 / 2004, with 639 2524 / 2190,
     of 7168 / 4096 with 650 rows 1194 / 1144, 64 of 1408 / 2048 with 468 rows 988 / 871, 16 of 2048 / 2048 with 750 rows 439 / 435; not taken: 8 of
     14336 / 4096 with 405 rows 1647 / 1761 (with 475, nearer the line, 1916 / 1759), of 7168 / 4096 with 500 rows 911 / 938, 16 of 2048 / 2048 with
     500 rows 310 / 353."""
@@ -1224,8 +1225,9 @@ MOE_HALF_TILE_MIN_ROWS, MOE_HALF_TILE_MIN_WORKGROUPS = 240, 5 * 256
 
 
 def moe_tiles(numel: int, num_experts: int, n_up: int, n_down: int):
-    """moe_tile_plan, and the 256-row form also where only its half tiles pay: an expert's last tile with 128 rows or fewer takes two thirds of a whole
-    one, so that experts of 240 rows and more gain once the up projection fills five rounds of workgroups.  Both products in us, 128 / 256 rows, for
+    """moe_tile_plan, and the 256-row form also where only the half tiles of moe_gemm256_kernel paid: an expert's last tile with 128 rows or fewer took two thirds of a
+    whole one, so that experts of 240 rows and more gained once the up projection filled five rounds of workgroups.  (moe_rows' lines lie below this one
+    everywhere: behind them it decides nothing.)  Both products in us, 128 rows / tiles of 256, for
     three routings each: 8 experts of 14336 / 4096 with 250 rows 1191 / 1116, 1206 / 1091, 1147 / 1131, with 400 1639 / 1282, 1624 / 1275, 1617 / 1294,
     with 440 1730 / 1741, 1799 / 1753, 1795 / 1707, with 520 2178 / 1895, 2088 / 1885, 2007 / 1736; 32 of 7168 / 4096 with 260 2292 / 2239, 2234 / 2031,
     2264 / 2043; 64 of 1408 / 2048 with 350 757 / 672, 759 / 676, 765 / 673.  Below the lines: 64 of 4096 / 2048 with 200 rows 1175 / 1212, 8 of 7168 /
@@ -1239,7 +1241,7 @@ def moe_tiles(numel: int, num_experts: int, n_up: int, n_down: int):
 
 
 def moe_rows(numel: int, num_experts: int, n_up: int, n_down: int):
-    """moe_tiles, and the 256-row alignment, whose experts are cut into even tiles of up to 320 rows (moe_rows_kernel), also for smaller experts where
+    """The plan of fused_experts: moe_tile_plan, and the 256-row alignment, whose experts are cut into even tiles of up to 320 rows (moe_rows_kernel), also for smaller experts where
     the up projection has tiles for the chip: from 140 rows on with 640 column tiles of 128 over all experts, from 300 on with 256.  Both products
     in us, 128 rows / even: 64 experts of 1408 / 2048 (704) with 120 rows 349 / 355, with 140 387 / 375, with 230 528 / 477; 8 of 14336 / 4096 (896) with
     140 857 / 854, with 200 939 / 852, with 230 1186 / 923; 32 of 7168 / 4096 with 100 1281 / 1279, with 150 1569 / 1363; 128 of 768 / 2048 (768) with 150
@@ -1248,7 +1250,7 @@ def moe_rows(numel: int, num_experts: int, n_up: int, n_down: int):
     rows, tiles = numel / max(1, num_experts), num_experts * -(-n_up // 128)
     if (tiles >= 640 and rows >= 140) or (tiles >= 256 and rows >= 300):
         return 256, 256, 256
-    return moe_tiles(numel, num_experts, n_up, n_down)
+    return moe_tile_plan(numel, num_experts, n_up, n_down)
 
 
 def moe_grouped_gemm(a: torch.Tensor, w: torch.Tensor, c: torch.Tensor, sorted_token_ids: torch.Tensor,
@@ -2127,7 +2129,7 @@ def routed_experts(h: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, ids: to
     inter = torch.empty((numel, N), dtype=_BF16, device=h.device)
     down = torch.empty((numel, W), dtype=_BF16, device=h.device)
     if _row_tiled(numel, E, N) and W % 64 == 0 and N % 64 == 0:
-        # (not moe_tiles: its line for half tiles was measured on fused_experts' shapes alone)
+        # (not moe_rows: its lines were measured on fused_experts' shapes alone)
         block_m, up_rows, down_rows = moe_tile_plan(numel, E, N, W) if MOE_TILE_OVERRIDE is None else MOE_TILE_OVERRIDE
         s = moe_align_block_size(ids, block_m, E)
         moe_tiled_gemm(h, w13, inter, *s, None, False, top, numel, block_m, fuse_silu=act.gated, tile_rows=up_rows, act=act)
