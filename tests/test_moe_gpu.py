@@ -265,7 +265,7 @@ def test_fused_experts_prefill_sized_batches_take_the_tiled_form(device, M, E, k
 @pytest.mark.parametrize("plan", [(256, 256, 256), (256, 256, 128), (256, 128, 128)])
 @pytest.mark.parametrize("M,E,k,N,Kd", [(4096, 8, 2, 7168, 4096), (3000, 4, 2, 448, 320), (1100, 2, 1, 1024, 1024)])
 def test_fused_experts_256_row_tiles(device, monkeypatch, plan, M, E, k, N, Kd):
-    """The 256 x 256 x 64 form (moe_gemm256_kernel: 8 waves, two LDS-DMA stages, XCD-patched order) for the up projection
+    """The 256-row alignment (moe_rows_kernel: even tiles of up to 320 rows by workgroups that stay) for the up projection
     (silu epilogue), the down projection (router weight, fp32), or -- over the same 256-row alignment -- the 128-row tiles;
     (4096, 8, 2, 7168, 4096) is one TP=2 rank of Mixtral-8x7B, the others have ragged column tiles, K = 5 steps and a
     last row block that is mostly padding.  Same bars as the 128-row form, and the forms agree to one ulp."""
@@ -317,7 +317,8 @@ def test_tiled_grouped_gemm_row_gather_and_scale(device):
 @pytest.mark.parametrize("loads", [(128, 129, 1, 127), (256, 257, 384, 385), (0, 300, 512, 64), (640, 0, 0, 641)])
 @pytest.mark.parametrize("fuse_silu", [True, False])
 def test_256_row_tiles_whose_second_half_is_empty(device, loads, fuse_silu):
-    """An expert's last 256-row tile leaves out its second half where that has no rows: loads on both sides of the halves, an expert with none.
+    """Loads on both sides of the halves of a 256-row block, an expert with none, over the 256-row alignment (the whole tiles, which leave out an empty
+    second half, have test_256_row_tiles_of_operands_beyond_32_bits).
     Rows are compared with the 128-row form's (the same products summed in the same order)."""
     K = _k()
     g = torch.Generator().manual_seed(sum(loads) + loads[0])
@@ -383,3 +384,55 @@ def test_even_row_tiles_of_filtered_experts_and_of_too_many_runs(device):
             K.moe_tiled_gemm(a, w, c, s.view(-1).to(device), e, post, None, False, 1, M, 256, tile_rows=rows)
             outs.append(c)
         assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("kind", ["gelu_tanh", "clamped_swish", "squared_relu"])
+def test_even_row_tiles_of_every_activation(device, kind):
+    """The other gated activations and the pointwise one on even tiles, bit for bit the 128-row form's."""
+    K = _k()
+    act = K.Pointwise(kind) if kind == "squared_relu" else K.Glu(kind, 7.0, 1.702)
+    g = torch.Generator().manual_seed(len(kind))
+    loads, N, Kd = (159, 321, 0, 641, 17), 160, 192
+    M, E = sum(loads), len(loads)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(loads))[torch.randperm(M, generator=g)].to(torch.int32).view(M, 1).to(device)
+    a = torch.randn((M, Kd), generator=g).to(BF).to(device)
+    w = (torch.randn((E, N * (2 if act.gated else 1), Kd), generator=g) * 0.2).to(BF).to(device)
+    s, e, post = K.moe_align_block_size(ids, 256, E)
+    outs = []
+    for rows in (128, 256):
+        c = torch.full((M, N), float("nan"), dtype=BF, device=device)
+        K.moe_tiled_gemm(a, w, c, s, e, post, None, False, 1, M, 256, fuse_silu=act.gated, tile_rows=rows, act=act)
+        outs.append(c)
+    assert bool(torch.isfinite(outs[1].float()).all()) and bool((outs[1] != 0).any())
+    assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("wide", ["rows", "weights"])
+@pytest.mark.parametrize("fuse_silu", [True, False])
+def test_256_row_tiles_of_operands_beyond_32_bits(device, wide, fuse_silu):
+    """Rows, or an expert's weights, that lie further apart than 32 bits count bytes: whole tiles of 256 rows (moe_gemm256_kernel), with
+    second halves that have no rows, ragged columns and an expert with none.  Bit for bit the 128-row form's."""
+    K = _k()
+    g = torch.Generator().manual_seed(11)
+    loads, N, Kd = ((128, 0, 129, 300), 160, 192) if wide == "rows" else ((300,), 288, 192)
+    M, E, columns = sum(loads), len(loads), N * (2 if fuse_silu else 1)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(loads))[torch.randperm(M, generator=g)].to(torch.int32).view(M, 1).to(device)
+
+    def apart(x, count):                                   # rows at least 4 GiB from the first to behind the last
+        step = (2 ** 31 // count + 7) // 8 * 8
+        view = torch.empty(count * step, dtype=BF, device=device).view(count, step)[:, :Kd]
+        return view.copy_(x)
+
+    a = torch.randn((M, Kd), generator=g).to(BF).to(device)
+    w = (torch.randn((E, columns, Kd), generator=g) * 0.1).to(BF).to(device)
+    far = (apart(a, M), w) if wide == "rows" else (a, apart(w[0], columns).unsqueeze(0))
+    assert max(far[0].stride(0) * M, far[1].stride(1) * columns) * 2 >= 2 ** 32
+    tw = torch.rand(M, generator=g).to(device)
+    s, e, post = K.moe_align_block_size(ids, 256, E)
+    outs = []
+    for x, y, rows in ((a, w, 128), (*far, 256)):
+        c = torch.full((M, N), float("nan"), dtype=BF if fuse_silu else torch.float32, device=device)
+        K.moe_tiled_gemm(x, y, c, s, e, post, None if fuse_silu else tw, not fuse_silu, 1, M, 256, fuse_silu=fuse_silu, round_before_scale=not fuse_silu, tile_rows=rows)
+        outs.append(c)
+    assert bool(torch.isfinite(outs[1].float()).all())
+    assert torch.equal(outs[0], outs[1])

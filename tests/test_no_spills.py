@@ -108,6 +108,13 @@ def test_moe_256_tile_kernel_keeps_its_registers_and_lds(tmp_path):
         assert u["vgpr_spill_count"] == 0 and u["sgpr_spill_count"] == 0, (name, u)
         assert u["vgpr_count"] <= 256, (name, u)
         assert u["group_segment_fixed_size"] == 128 * 1024, (name, u)
+    # moe_rows_kernel: 160 accumulators + fragments and the next tile's row pointers, all of its 256 registers.  Up to 36 scalars are parked in lanes of vector
+    # registers (eleven copies of the walk beside the next tile's addresses and the arguments), none of them between a walk's products; LDS = two 72 KiB stages and the table of runs
+    rows = {k: v for k, v in usage.items() if "moe_rows_kernel" in k}
+    assert len(rows) == 1, sorted(usage)
+    for name, u in rows.items():
+        assert u["vgpr_spill_count"] == 0 and u["sgpr_spill_count"] <= 36 and u["vgpr_count"] <= 256, (name, u)
+        assert u["group_segment_fixed_size"] == 160 * 1024, (name, u)
     k128 = {k: v for k, v in usage.items() if "moe_tiled_gemm_kernel" in k}
     assert len(k128) == 1
     for name, u in k128.items():
@@ -184,6 +191,26 @@ def test_split_recurrences_keep_their_registers_and_lds(tmp_path):
         assert len(inst) == 3, sorted(usage)                    # state dims of up to 32, 64 and 128
         for name, u in inst.items():
             assert u["vgpr_spill_count"] == 0 and u["vgpr_count"] <= 256, (name, u)
+            assert u["group_segment_fixed_size"] <= 160 * 1024, (name, u)
+    # the two launches: four preparing waves a SIMD; the walk alone on a compute unit with a fetching wave, or two workgroups of four waves
+    for kernel, registers, lds in (("delta_prepare_kernel", 128, 40), ("delta_walk_kernel", 256, 160), ("delta_walk_self_kernel", 256, 80)):
+        inst = {k: v for k, v in usage.items() if kernel in k}
+        assert len(inst) == 3, sorted(usage)
+        for name, u in inst.items():
+            assert u["vgpr_spill_count"] == 0 and u["sgpr_spill_count"] == 0 and u["vgpr_count"] <= registers, (name, u)
+            assert u["group_segment_fixed_size"] <= lds * 1024, (name, u)
+
+
+@pytest.mark.skipif(not Path(HIPCC).exists(), reason="hipcc not installed")
+def test_weight_streams_of_eight_two_tile_waves_do_not_spill(tmp_path):
+    """The widest groups, and those of four such waves: accumulators, a chunk's fragments and the weights' pointers stay in registers; no scratch, one workgroup a
+    compute unit.  Experts' rows never take the groups of eight: no such kernel is compiled."""
+    usage = _resource_usage("wstream_gemm.hip", tmp_path)
+    for form, n in (("Li8ELi2ELb0E", 4), ("Li4ELi2ELb0E", 4), ("Li8ELi2ELb1E", 0)):
+        inst = {k: v for k, v in usage.items() if "wstream_gemm_kernel" in k and form in k}
+        assert len(inst) == n, sorted(inst)
+        for name, u in inst.items():
+            assert u["vgpr_spill_count"] == 0 and u["sgpr_spill_count"] == 0 and u["vgpr_count"] <= 256, (name, u)
             assert u["group_segment_fixed_size"] <= 160 * 1024, (name, u)
 
 
