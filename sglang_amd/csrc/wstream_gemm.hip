@@ -797,8 +797,8 @@ int launch_main(WsParams p, hipStream_t st, int row_blocks = 0) {
     // end; workgroups that stay keep it filled: [64, 128256, 4096] 184 -> 177 us (one row 169 -> 156), silu [16, 57344, 8192] 157 -> 142.
     // Groups are as narrow as the number of rounds allows, so that the last round is as full as the others: silu [24, 9728, 896] 10.9 -> 8.9
     // (76 groups of four pairs / 152 of two), [64, 32000, 4096] in eight waves 56.4 -> 41.8.  At least two pairs a group would be
-    // slower: silu of 16 rows, one / two, [8192, 4096] 16.6 / 19.1, [5120, 14336] 47.3 / 51.2, [2048, 1024] 5.6 / 6.0.  Launches of two waves, with a deeper
-    // ring, are no quicker either: silu of 64 rows, four / two, [8192, 4096] 23.2 / 24.5, [4096, 896] 8.5 / 8.8.
+    // slower: silu of 16 rows, one / two, [8192, 4096] 14.3 / 18.1, [5120, 14336] 40.0 / 46.7, [2048, 1024] 5.5 / 6.1.  Launches of two waves, with a deeper
+    // ring, are no quicker either: silu of 64 rows, four / two, [8192, 4096] 21.8 / 22.3, [4096, 896] 8.0 / 8.5.
     const int wtiles = p.ntiles / TPW;
     const bool stays = p.splits == 1 && !row_blocks;
     const int rounds = ((wtiles + NW - 1) / NW + kNumCus - 1) / kNumCus;
@@ -834,9 +834,10 @@ int launch_nw(const WsParams& p, int nw, bool two_tiles, hipStream_t st, int row
         // Groups of four waves or of eight.  The chip is bound by the requests that a compute unit's vector cache keeps in flight (115 to
         // 130 of a line, of 0.9 to 1.2 k clocks each) as much as by HBM, and every turn asks for the activations anew: 256 rows of weights
         // a turn in the place of 128 make them a fifth of the requests and not a third.  us, four waves / eight: [64, 128256, 4096]
-        // 177.5 / 168, silu [64, 57344, 8192] 152 / 141, silu [64, 37888, 3584] 58 / 46.6, [64, 32000, 4096] 43.8 / 41.8.  Up to 3.75 pairs of tiles
-        // a workgroup the eight find too little to do (silu [64, 28672, 4096] 40.3 / 41.3, [16, 9728, 896] 7.7 / 8.3); over several turns few rows are
-        // read quicker in 256 bytes of a row at a time (one row of [128256, 4096] 156 / 162, 24 rows of [151936, 896] 47.3 / 49.6).
+        // 184 / 175, silu [64, 57344, 8192] 157 / 148, silu [64, 37888, 3584] 59.5 / 48.7, [64, 32000, 4096] 45.1 / 44.9.  Up to 3.75 pairs of tiles
+        // a workgroup the eight find too little to do (silu [64, 28672, 4096] 39.0 / 40.1, [16, 9728, 896] 6.9 / 7.5); over several turns few rows are
+        // read quicker in 256 bytes of a row at a time (one row of [128256, 4096] 161 / 167, 24 rows of [151936, 896] 47.0 / 49.6).  Of 16 rows in one
+        // turn most widths gain ([57344, 4096] 73.7 / 71.5, [61440, 8192] 172 / 161, [32768, 896] 11.6 / 11.4), a few lose ([49152, 4096] 64.4 / 67.3, [45056, 4096] 57.4 / 59.1).
         if constexpr (MT <= 4) {
           const int pairs = p.ntiles / 2;
           if (p.splits == 1 && !row_blocks && pairs * 4 > 15 * kNumCus && (pairs <= 8 * kNumCus || MT > 2)) return launch_main<MT, 8, 2>(p, st);
