@@ -91,6 +91,85 @@ struct ChunkParams {
   int walks_spans;              // the looping kernel takes the plan's spans, where it has any, in the place of the private items
 };
 
+// A pointer that came as a bare word, known to lie in device memory.  Left generic, all 650 loads of the looping kernels were flat ones: those count as LDS
+// accesses too, so that every wait for the image drained the rows on their way.  us for four layers: 100 requests of 0.6 to 1.4 k, 32 / 8 heads, 433 -> 415,
+// 8 of 5 k, 64 / 8 heads, 196 -> 188, 16 of 1 k, 32 kv heads, 272 -> 263, 64 of 1.5 k in e4m3 252 -> 249.
+template <typename T>
+__device__ __forceinline__ T* global_ptr(T* x) {
+  return (T*)(__attribute__((address_space(1))) T*)(uint64_t)x;
+}
+
+// ---- The rows of the step itself (sgl_amd_cascade_decode_attention_store).  A launch of their own in front of every layer's attention is little more than launch, so
+// each row is stored by the one unit of a kv head that reads it as its request's newest token: by every wave of the unit that reads it, before it does (the
+// accesses of a wave to one address complete in order, and what the other waves store is the same).  Nobody else reads the slot, unless a table holds
+// another row's new slot; the plan looks for that once a step (cascade_check_rows), and then every wave stores all rows of its kv head first, the later of two
+// with one slot.
+// us of attention a step, store launch / this: 64 requests behind shared prefixes, 32 / 8 heads, 8 layers, 233 / 219; 37 of 0.9 to 5.1 k in e4m3, 4 layers,
+// 267 / 258; 21 of 180 in e4m3, 64 / 8 heads, 4 layers, 70 / 61.  What is left of the launch: 1 us a layer in units of 128 tokens (with nothing stored 209).
+struct NewRows {
+  const uint16_t* k;            // [B, Hkv, D]
+  const uint16_t* v;
+  const int64_t* loc;
+  int64_t k_stride, v_stride;
+  float inv_k_scale, inv_v_scale;
+};
+struct StoreParams {
+  ChunkParams chunk;
+  NewRows rows;
+};
+constexpr int kNewest = -2, kOlder = -1;              // word 7 of a private item's or piece's record: it ends in the request's newest token, or not
+enum RowsToStore { kInPool = 0, kOwnRow = 1, kAllRows = 2 };
+
+// a lane's piece of request b's new rows of a kv head: asked for, stored (K by the first D / 8 lanes, V by the next)
+template <int D>
+__device__ __forceinline__ U4 ask_new_row(const NewRows& rows, const int b, const int kvh, const int lane) {
+  return ld16((lane & (D / 8) ? rows.v + b * rows.v_stride : rows.k + b * rows.k_stride) + kvh * D + (lane & (D / 8 - 1)) * 8);
+}
+template <int D, bool FP8>
+__device__ __forceinline__ void put_new_row(const ChunkParams& p, const NewRows& rows, const U4& x, const int slot, const int kvh, const int lane) {
+  const bool of_v = (lane & (D / 8)) != 0;
+  unsigned char* to = const_cast<unsigned char*>(kv_row(of_v ? p.v_cache : p.k_cache, p.fmt, slot, kvh));
+  if (lane < D / 4) put_kv8<FP8>(to, lane & (D / 8 - 1), x, of_v ? rows.inv_v_scale : rows.inv_k_scale);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+template <int D, bool FP8>
+__device__ __forceinline__ void put_own_row(const ChunkParams& p, const NewRows& rows, const int b, const int kvh, const int lane) {
+  const int slot = static_cast<int>(rows.loc[b]);
+  put_new_row<D, FP8>(p, rows, ask_new_row<D>(rows, b, kvh, lane), slot, kvh, lane);
+}
+template <int D, bool FP8>
+__device__ __forceinline__ void put_all_rows(const ChunkParams& p, const NewRows& rows, const int kvh, const int lane) {
+#pragma clang loop unroll(disable)
+  for (int b = 0; b < p.batch; ++b) {
+    const int64_t slot = rows.loc[b];
+    bool again = false;
+#pragma clang loop unroll(disable)
+    for (int c = b + 1 + lane; c < p.batch; c += 64) again |= rows.loc[c] == slot;
+    if (__ballot(again) == 0ull) put_new_row<D, FP8>(p, rows, ask_new_row<D>(rows, b, kvh, lane), static_cast<int>(slot), kvh, lane);
+  }
+}
+
+// Whether all rows have to be stored first: a table holds a new slot elsewhere, or the plan does not know these slots (every wave for itself).
+// The first 64 requests' slots and the words are asked for by ask(), beside what else a kernel begins with: behind it they are a round trip of their own.
+struct RowsMeet {
+  int word, planned, now;
+  __device__ __forceinline__ void ask(const ChunkParams& p, const NewRows& rows, const int lane) {
+    const CascadePlanView pv = cascade_plan_view(p.plan, p.batch, p.max_items);
+    const int first = lane < p.batch ? lane : p.batch - 1;
+    word = pv.meet[lane];
+    planned = pv.new_slots[first];
+    now = static_cast<int32_t>(rows.loc[first]);
+  }
+  __device__ __forceinline__ int answer(const ChunkParams& p, const NewRows& rows, const int lane) const {
+    bool meet = (word != 0) | (planned != now);
+    if (p.batch > 64) {
+      const CascadePlanView pv = cascade_plan_view(p.plan, p.batch, p.max_items);
+      for (int b = 64 + lane; b < p.batch; b += 64) meet |= pv.new_slots[b] != static_cast<int32_t>(rows.loc[b]);
+    }
+    return __ballot(meet) != 0ull ? kAllRows : kOwnRow;
+  }
+};
+
 // The K rows, then (after S^T) the transposed V rows, pass through ONE 16 KiB LDS image; at D = 128 it is filled twice
 // per operand: K by token halves (64 tokens x 128 dims: each score tile is complete inside its half), V^T by head-dim
 // halves (64 dims x 128 tokens: each output tile is complete inside its half).  With <= 96 VGPRs that makes five
@@ -121,11 +200,35 @@ __global__ __launch_bounds__(kThreads, 5) void cascade_chunk_kernel(ChunkParams 
   __shared__ U4 side_s[D > 64 ? 4 * 8 * (D - 64) / 4 : 1];        // ... and their O^T partials of every V^T part but the last
   const int unit = blockIdx.x;
   const int tid = threadIdx.x;
+  constexpr bool STORE = false;
+  const NewRows new_rows{};
+  RowsMeet meet;
+#define CASC_ONE_SHOT
 #include "cascade_chunk_body.inc"
+#undef CASC_ONE_SHOT
 }
 
-template <int D, bool FP8, bool HND>
-__device__ __forceinline__ void cascade_chunk_unit(const ChunkParams& p, U4* sm, float* ml_s, U4* side_s, const int unit, const int tid) {
+// ... with the step's rows to store (token-major pools)
+template <int D, bool FP8>
+__global__ __launch_bounds__(kThreads, 5) void cascade_store_kernel(StoreParams sp) {
+  __shared__ U4 sm[(kChunk / (D > 64 ? D / 64 : 1)) * (D / 8)];
+  __shared__ float ml_s[64];
+  __shared__ U4 side_s[D > 64 ? 4 * 8 * (D - 64) / 4 : 1];
+  const ChunkParams& p = sp.chunk;
+  const NewRows& new_rows = sp.rows;
+  const int unit = blockIdx.x;
+  const int tid = threadIdx.x;
+  constexpr bool HND = false, STORE = true;
+  RowsMeet meet;
+  meet.ask(p, new_rows, tid & 63);
+#define CASC_ONE_SHOT
+#include "cascade_chunk_body.inc"
+#undef CASC_ONE_SHOT
+}
+
+template <int D, bool FP8, bool HND, bool STORE>
+__device__ __forceinline__ void cascade_chunk_unit(const ChunkParams& p, const NewRows& new_rows, U4* sm, float* ml_s, U4* side_s, const int unit, const int tid,
+                                                   const int store_rows) {
 #include "cascade_chunk_body.inc"
 }
 
@@ -149,8 +252,9 @@ __device__ __forceinline__ float lane_rows_max(float x) {
 // requests of 1.5 k in bf16 910 -> 729 us (4.6 TB/s; a large copy reaches 4.9).  Before, a unit was 128 tokens staged through one image
 // behind six barriers.  A bf16 item of 128 tokens keeps that form: its rows come in one burst, 257 against 265 us in the shared-prefix batch.
 // Image: row (token) t at t * 2 D bytes, its 16-byte piece c in slot c ^ kSw(t): the four rows of a transposing read lie on distinct banks.
-template <int D, bool FP8, bool HND>
-__device__ __forceinline__ void cascade_few_rows_unit(const ChunkParams& p, U4* sm, float* ml_s, const int32_t* rec, const int kvh, const int tid) {
+template <int D, bool FP8, bool HND, bool STORE>
+__device__ __forceinline__ void cascade_few_rows_unit(const ChunkParams& p, const NewRows& new_rows, U4* sm, float* ml_s, const int32_t* rec, const int kvh,
+                                                      const int tid, const int store_rows) {
   const int4 ra = *reinterpret_cast<const int4*>(rec), rb = *reinterpret_cast<const int4*>(rec + 4);
   constexpr int KC = D / 32, ND = D / 16;
   constexpr int KL = FP8 ? D / 64 : D / 32;                    // 16-byte pieces of a K row a lane holds
@@ -220,10 +324,19 @@ __device__ __forceinline__ void cascade_few_rows_unit(const ChunkParams& p, U4* 
   };
   const int vrow = 4 * g + (i16 >> 2), vsw = swz(vrow);
   const unsigned char* vlane = img + vrow * (2 * D) + ((i16 >> 1) & 1) * 16 + (i16 & 1) * 8;
+  // The newest token is in the last tile: its wave alone reads it, and stores it behind the requests for its first tile's rows where that is another one (in front
+  // of them the wait for it was 4 us of a launch of 57).
+  const bool mine = STORE && store_rows == kOwnRow && __builtin_amdgcn_readfirstlane(rb.w) == kNewest && wid < tiles && ((tiles - 1 - wid) & 3) == 0;
+  U4 own;
+  if (mine) {
+    if (tiles - 1 == wid) put_own_row<D, FP8>(p, new_rows, rec_x, kvh, lane);
+    else own = ask_new_row<D>(new_rows, rec_x, kvh, lane);
+  }
   if (wid < tiles) {
     load_k(ids);
     load_v(ids);
   }
+  if (mine && tiles - 1 != wid) put_new_row<D, FP8>(p, new_rows, own, static_cast<int>(new_rows.loc[rec_x]), kvh, lane);
   for (int t = wid; t < tiles; t += 4) {
     const bool more = t + 4 < tiles;                           // (wave-uniform)
     if (more) ids = slot_id(t + 4);
@@ -307,19 +420,15 @@ __device__ __forceinline__ void cascade_few_rows_unit(const ChunkParams& p, U4* 
   }
 }
 
-// A pointer that came as a bare word, known to lie in device memory.  Left generic, all 650 loads of the looping kernels were flat ones: those count as LDS
-// accesses too, so that every wait for the image drained the rows on their way.  us for four layers: 100 requests of 0.6 to 1.4 k, 32 / 8 heads, 433 -> 415,
-// 8 of 5 k, 64 / 8 heads, 196 -> 188, 16 of 1 k, 32 kv heads, 272 -> 263, 64 of 1.5 k in e4m3 252 -> 249.
-template <typename T>
-__device__ __forceinline__ T* global_ptr(T* x) {
-  return (T*)(__attribute__((address_space(1))) T*)(uint64_t)x;
-}
-
-template <int D, bool FP8, bool HND>
-__global__ __launch_bounds__(kThreads, 4) void cascade_chunk_loop_kernel(ChunkParams p) {
+// The looping form's walk; ARG: the kernel's one argument, a ChunkParams or what begins with one.
+template <int D, bool FP8, bool HND, typename ARG>
+__device__ __forceinline__ void cascade_chunk_loop(const ChunkParams& p, const NewRows* new_rows) {
+  constexpr bool STORE = std::is_same<ARG, StoreParams>::value;
   __shared__ U4 sm[(kChunk / (D > 64 ? D / 64 : 1)) * (D / 8)];
   __shared__ float ml_s[64];
   __shared__ U4 side_s[D > 64 ? 4 * 8 * (D - 64) / 4 : 1];
+  RowsMeet meet;
+  if constexpr (STORE) meet.ask(p, *new_rows, threadIdx.x & 63);
   // the line of the workgroup's first item record travels with the header (a grid never reaches beyond max_items x kv heads)
   const int first_rec = cascade_plan_view(p.plan, p.batch, p.max_items).items[8 * (blockIdx.x / static_cast<unsigned>(p.num_kv_heads))];
   // one hop for all of the header that the loop needs: the list's length (shared items, then private items or spans) and what the tail is.
@@ -329,6 +438,12 @@ __global__ __launch_bounds__(kThreads, 4) void cascade_chunk_loop_kernel(ChunkPa
   asm volatile("" ::"v"(first_rec));
   const int n_units = n_items * p.num_kv_heads;
   const int G = static_cast<int>(gridDim.x), w0 = static_cast<int>(blockIdx.x);
+  int store_rows = kInPool;
+  if constexpr (STORE) {
+    asm volatile("" : "+v"(meet.word), "+v"(meet.planned), "+v"(meet.now));
+    store_rows = __builtin_amdgcn_readfirstlane(meet.answer(p, *new_rows, threadIdx.x & 63));
+    if (n_units == 0 && w0 < p.num_kv_heads) put_all_rows<D, FP8>(p, *new_rows, w0, threadIdx.x & 63);    // nobody reads anything
+  }
   // The kernel's one argument sits at the start of the kernarg segment; every pass re-reads it through an address the
   // compiler cannot see through, exactly as a fresh launch would (scalar loads, served by the scalar cache), and takes the
   // thread index as an opaque value.
@@ -341,11 +456,22 @@ __global__ __launch_bounds__(kThreads, 4) void cascade_chunk_loop_kernel(ChunkPa
     uint64_t ka = kp;
     asm volatile("" : "+s"(ka));
     KernargWord* kw = reinterpret_cast<KernargWord*>(ka);
-    static_assert(sizeof(ChunkParams) % 8 == 0 && std::is_trivially_copyable<ChunkParams>::value, "kernarg image copied as 8-byte words");
-    struct Raw { uint64_t w[sizeof(ChunkParams) / 8]; } raw;
+    static_assert(sizeof(ARG) % 8 == 0 && std::is_trivially_copyable<ARG>::value, "kernarg image copied as 8-byte words");
+    struct Raw { uint64_t w[sizeof(ARG) / 8]; } raw;
 #pragma unroll
-    for (unsigned i = 0; i < sizeof(ChunkParams) / 8; ++i) raw.w[i] = kw[i];
-    ChunkParams pl = __builtin_bit_cast(ChunkParams, raw);
+    for (unsigned i = 0; i < sizeof(ARG) / 8; ++i) raw.w[i] = kw[i];
+    ARG arg = __builtin_bit_cast(ARG, raw);
+    NewRows nr{};
+    ChunkParams pl;
+    if constexpr (STORE) {
+      pl = arg.chunk;
+      nr = arg.rows;
+      nr.k = global_ptr(nr.k);
+      nr.v = global_ptr(nr.v);
+      nr.loc = global_ptr(nr.loc);
+    } else {
+      pl = arg;
+    }
     pl.q = global_ptr(pl.q);
     pl.k_cache = global_ptr(pl.k_cache);
     pl.v_cache = global_ptr(pl.v_cache);
@@ -359,6 +485,9 @@ __global__ __launch_bounds__(kThreads, 4) void cascade_chunk_loop_kernel(ChunkPa
     const CascadePlanView pv = cascade_plan_view(pl.plan, pl.batch, pl.max_items);
     const int span = item - n_shared;
     const bool in_span = spans && span >= 0;                                  // (workgroup-uniform)
+    if constexpr (STORE) {
+      if (store_rows == kAllRows) put_all_rows<D, FP8>(pl, nr, kvh, tid & 63);
+    }
     const int32_t* rec = pv.items + 8 * item;
     if (in_span) {
       const int i = next > 0 ? next : __builtin_amdgcn_readfirstlane(pv.span_first[span]);
@@ -366,12 +495,21 @@ __global__ __launch_bounds__(kThreads, 4) void cascade_chunk_loop_kernel(ChunkPa
       next = i + 1 < __builtin_amdgcn_readfirstlane(pv.span_first[span + 1]) ? i + 1 : 0;
     }
     if (in_span || (FP8 && __builtin_amdgcn_readfirstlane(rec[3]) * pl.group <= 8))
-      cascade_few_rows_unit<D, FP8, HND>(pl, sm, ml_s, rec, kvh, tid);
+      cascade_few_rows_unit<D, FP8, HND, STORE>(pl, nr, sm, ml_s, rec, kvh, tid, store_rows);
     else
-      cascade_chunk_unit<D, FP8, HND>(pl, sm, ml_s, side_s, unit, tid);
+      cascade_chunk_unit<D, FP8, HND, STORE>(pl, nr, sm, ml_s, side_s, unit, tid, store_rows);
     __syncthreads();                                                          // the image is reused by the next unit
     if (next == 0) { base += G; ++pass; }
   }
+}
+
+template <int D, bool FP8, bool HND>
+__global__ __launch_bounds__(kThreads, 4) void cascade_chunk_loop_kernel(ChunkParams p) {
+  cascade_chunk_loop<D, FP8, HND, ChunkParams>(p, nullptr);
+}
+template <int D, bool FP8>
+__global__ __launch_bounds__(kThreads, 4) void cascade_store_loop_kernel(StoreParams p) {
+  cascade_chunk_loop<D, FP8, false, StoreParams>(p.chunk, &p.rows);
 }
 
 // ---- cascade plan: group the requests of a decode batch that share a KV prefix ----------------
@@ -459,10 +597,68 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_compare_kernel(
 // takes it back (24: 12.9 / 12.3 and 16.5 / 15.8, 32: 13.8 / 12.8 and 15.9 / 19.1, 64: 15.0 / 21.7 and 15.9 / 32.3).
 constexpr int kPlanOneLaunch = 16;
 
+// Whether a request's table holds the slot of a row of this step anywhere but at its own newest token, looked up by workgroups beside the plan's own (one
+// launch; they take less time than it).  The new slots are bits of two hashes in LDS; what both hold is compared with every slot.  Slot 0 is the sink of padded
+// entries, which may share it.  A request without tokens counts as well: no unit would store its row.
+__device__ __forceinline__ void cascade_check_rows(const int32_t* req_to_token, int64_t r2t_stride, const int64_t* req_pool_indices, const int32_t* seq_lens,
+                                                   const int64_t* new_loc, int batch, int checker, int checkers, uint32_t* bits0, uint32_t* bits1, int* slots,
+                                                   const CascadePlanView& pv) {
+  const int tid = threadIdx.x;
+  for (int i = tid; i < 1024; i += kPlanThreads) bits0[i] = bits1[i] = 0u;
+  __syncthreads();
+  auto hash = [](uint32_t s) { return (s * 0x9e3779b1u) >> 17; };
+  bool meet = false, seen[kPlanMaxBatch / kPlanThreads];
+#pragma unroll
+  for (int i = 0; i < kPlanMaxBatch / kPlanThreads; ++i) {
+    const int b = tid + i * kPlanThreads;
+    seen[i] = false;
+    if (b < batch) {
+      const uint32_t s = static_cast<uint32_t>(new_loc[b]), h = hash(s);
+      slots[b] = static_cast<int>(s);
+      seen[i] = (atomicOr(&bits0[(s & 32767u) >> 5], 1u << (s & 31u)) >> (s & 31u)) & 1u;
+      atomicOr(&bits1[h >> 5], 1u << (h & 31u));
+      if (checker == 0) pv.new_slots[b] = static_cast<int>(s);
+    }
+  }
+  __syncthreads();
+  auto among = [&](int s, int but) {
+    bool found = false;
+    for (int c = 0; c < batch; ++c) found |= slots[c] == s && c != but;
+    return found;
+  };
+#pragma unroll
+  for (int i = 0; i < kPlanMaxBatch / kPlanThreads; ++i)
+    if (checker == 0 && seen[i] && slots[tid + i * kPlanThreads] != 0) meet |= among(slots[tid + i * kPlanThreads], tid + i * kPlanThreads);
+  constexpr int kAhead = 8;
+  for (int b = checker; b < batch; b += checkers) {
+    const int32_t* row = req_to_token + req_pool_indices[b] * r2t_stride;
+    const int len = seq_lens[b], own = slots[b];
+    meet |= len < 1;
+    for (int t0 = tid; t0 < len; t0 += kAhead * kPlanThreads) {
+      int s[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int t = t0 + u * kPlanThreads;
+        s[u] = row[t < len ? t : len - 1];
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const uint32_t x = static_cast<uint32_t>(s[u]), h = hash(x);
+        if ((bits0[(x & 32767u) >> 5] >> (x & 31u)) & (bits1[h >> 5] >> (h & 31u)) & 1u) {
+          const bool newest = t0 + u * kPlanThreads >= len - 1;                  // (or behind it: that token again)
+          if (!(newest && s[u] == own) && among(s[u], -1)) meet = true;
+        }
+      }
+    }
+  }
+  if (__syncthreads_or(meet) && tid == 0) pv.meet[checker] = 1;
+  else if (tid == 0) pv.meet[checker] = 0;
+}
+
 template <bool ONE>
 __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
     const int32_t* __restrict__ req_to_token, int64_t r2t_stride, const int64_t* __restrict__ req_pool_indices,
-    const int32_t* __restrict__ seq_lens, int batch, int min_shared, int chunk_tokens, int tokens_per_tile,
+    const int32_t* __restrict__ seq_lens, const int64_t* __restrict__ new_loc, int batch, int min_shared, int chunk_tokens, int tokens_per_tile,
     int kv_tile, int max_shared, int32_t* __restrict__ plan, int max_items, int zero_items, int num_kv_heads, int span_units) {
   __shared__ int first_slot[kPlanMaxBatch];
   __shared__ int leader[kPlanMaxBatch];
@@ -478,6 +674,12 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
   __shared__ int wave_tot[kPlanThreads / 64], wave_tiles[kPlanThreads / 64];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const CascadePlanView pv = cascade_plan_view(plan, batch, max_items);
+  if (blockIdx.x > 0) {
+    static_assert(kPlanMaxBatch == 1024, "the arrays hold 32768 bits");
+    cascade_check_rows(req_to_token, r2t_stride, req_pool_indices, seq_lens, new_loc, batch, static_cast<int>(blockIdx.x) - 1, static_cast<int>(gridDim.x) - 1,
+                       reinterpret_cast<uint32_t*>(first_slot), reinterpret_cast<uint32_t*>(leader), grp_min, pv);
+    return;
+  }
   // members == 0 marks the end of the list for the one-workgroup-per-unit chunk kernel, whose grid never reaches beyond
   // zero_items entries (the looping form reads the list's length from the header): 13.8 -> 98 us per step at a 128 k-token
   // request table when all max_items entries were cleared (profiles/r05_exp1_cascade_table_width.json)
@@ -616,6 +818,8 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
     pv.header[2] = rows;
     pv.header[3] = n_shared_items;
   }
+  // (no word of a workgroup that looked: 1 where there are none, so that a plan without the slots says what one that found some says)
+  if (tid < kCheckers && tid >= static_cast<int>(gridDim.x) - 1) pv.meet[tid] = gridDim.x == 1 ? 1 : 0;
   // ---- private chunks of every request, appended behind the shared items (block-wide exclusive scan) ----
   int mine = 0, sh = 0, len = 0;
   if (tid < batch) {
@@ -654,7 +858,7 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
     it[4] = tid;                                     // the request itself
     it[5] = 1;                                       // private item
     it[6] = pool_row[tid];
-    it[7] = -1;
+    it[7] = kvb + chunk_tokens < len ? kOlder : kNewest;
     it[3] = 1;
   }
   // ---- spans: the private tokens of all requests, in 64-token tiles, as ONE line cut into equal parts ----
@@ -701,7 +905,7 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
     it[4] = tid;
     it[5] = 1;
     it[6] = pool_row[tid];
-    it[7] = -1;
+    it[7] = kve < len ? kOlder : kNewest;
   }
   if (tid == kPlanThreads - 1) pv.span_first[(n_tiles + span - 1) / span] = incl;
 }
@@ -781,6 +985,13 @@ int64_t sgl_amd_cascade_plan_ints(int64_t batch, int64_t max_items) { return cas
 int sgl_amd_cascade_plan(const int32_t* req_to_token, int64_t req_to_token_stride, const int64_t* req_pool_indices,
                          const int32_t* seq_lens, int64_t batch, int num_q_heads, int num_kv_heads,
                          int min_shared_len, int64_t max_context_len, int32_t* plan, int64_t max_items, void* stream) {
+  return sgl_amd_cascade_plan_new_rows(req_to_token, req_to_token_stride, req_pool_indices, seq_lens, nullptr, batch, num_q_heads, num_kv_heads, min_shared_len,
+                                       max_context_len, plan, max_items, stream);
+}
+
+int sgl_amd_cascade_plan_new_rows(const int32_t* req_to_token, int64_t req_to_token_stride, const int64_t* req_pool_indices,
+                                  const int32_t* seq_lens, const int64_t* new_loc, int64_t batch, int num_q_heads, int num_kv_heads,
+                                  int min_shared_len, int64_t max_context_len, int32_t* plan, int64_t max_items, void* stream) {
   SGL_CLEAR_STALE_ERROR();
   SGL_CHECK_ARG(batch >= 1 && batch <= kPlanMaxBatch, "cascade_plan: batch=%lld (supported: 1..%d)", (long long)batch, kPlanMaxBatch);
   SGL_CHECK_ARG(num_kv_heads > 0 && num_q_heads % num_kv_heads == 0 && num_q_heads / num_kv_heads <= kRowsPerItem, "cascade_plan: bad head counts");
@@ -798,8 +1009,9 @@ int sgl_amd_cascade_plan(const int32_t* req_to_token, int64_t req_to_token_strid
     hipLaunchKernelGGL(cascade_plan_compare_kernel, dim3(static_cast<unsigned>((batch + kPlanThreads / 64 - 1) / (kPlanThreads / 64))),
                        dim3(kPlanThreads), 0, as_stream(stream), req_to_token, req_to_token_stride, req_pool_indices, seq_lens,
                        static_cast<int>(batch), pv.compare);
-  hipLaunchKernelGGL(one ? cascade_plan_kernel<true> : cascade_plan_kernel<false>, dim3(1), dim3(kPlanThreads), 0, as_stream(stream), req_to_token,
-                     req_to_token_stride, req_pool_indices, seq_lens, static_cast<int>(batch), min_shared_len,
+  const unsigned checkers = new_loc == nullptr ? 0 : static_cast<unsigned>(batch < kCheckers ? batch : kCheckers);
+  hipLaunchKernelGGL(one ? cascade_plan_kernel<true> : cascade_plan_kernel<false>, dim3(1 + checkers), dim3(kPlanThreads), 0, as_stream(stream), req_to_token,
+                     req_to_token_stride, req_pool_indices, seq_lens, new_loc, static_cast<int>(batch), min_shared_len,
                      kChunk, members_per_item, 64, chunks * kChunk, plan, static_cast<int>(max_items),
                      // end-of-list markers for every item a one-workgroup-per-unit launch of THIS batch can reach (the attention entry's
                      // own bound, batch x (chunks + 1)) whenever such a launch is possible at ANY setting of the launch-form switch --
@@ -838,7 +1050,22 @@ int sgl_amd_cascade_decode_attention_ex(const void* q, const void* k_cache, cons
                                         int64_t v_cache_row_stride, float sm_scale, int64_t max_context_len,
                                         int slots_total, void* ws_acc, void* ws_ml, int kv_fp8, float k_scale, float v_scale,
                                         int page_size, int kv_layout_hnd, void* stream) {
+  return sgl_amd_cascade_decode_attention_store(q, const_cast<void*>(k_cache), const_cast<void*>(v_cache), out, req_to_token, req_to_token_stride, req_pool_indices,
+                                                seq_lens, plan, batch, max_items, num_q_heads, num_kv_heads, head_dim, q_token_stride, out_token_stride,
+                                                k_cache_row_stride, v_cache_row_stride, sm_scale, max_context_len, slots_total, ws_acc, ws_ml, kv_fp8, k_scale,
+                                                v_scale, page_size, kv_layout_hnd, nullptr, nullptr, nullptr, 0, 0, stream);
+}
+
+int sgl_amd_cascade_decode_attention_store(const void* q, void* k_cache, void* v_cache, void* out, const int32_t* req_to_token, int64_t req_to_token_stride,
+                                           const int64_t* req_pool_indices, const int32_t* seq_lens, const int32_t* plan, int64_t batch, int64_t max_items,
+                                           int num_q_heads, int num_kv_heads, int head_dim, int64_t q_token_stride, int64_t out_token_stride,
+                                           int64_t k_cache_row_stride, int64_t v_cache_row_stride, float sm_scale, int64_t max_context_len, int slots_total,
+                                           void* ws_acc, void* ws_ml, int kv_fp8, float k_scale, float v_scale, int page_size, int kv_layout_hnd,
+                                           const void* k_new, const void* v_new, const int64_t* new_loc, int64_t k_new_stride, int64_t v_new_stride, void* stream) {
   SGL_CLEAR_STALE_ERROR();
+  SGL_CHECK_ARG((k_new == nullptr) == (v_new == nullptr) && (k_new == nullptr) == (new_loc == nullptr), "cascade_decode_attention: new rows without a part");
+  SGL_CHECK_ARG(((reinterpret_cast<uintptr_t>(k_new) | reinterpret_cast<uintptr_t>(v_new)) & 15) == 0 && k_new_stride % 8 == 0 && v_new_stride % 8 == 0,
+                "cascade_decode_attention: new rows must be 16-byte aligned");
   SGL_CHECK_ARG(head_dim == 64 || head_dim == 128, "cascade_decode_attention: head_dim=%d not supported (64/128)", head_dim);
   SGL_CHECK_ARG(num_kv_heads > 0 && num_q_heads % num_kv_heads == 0 && num_q_heads / num_kv_heads <= kRowsPerItem,
                 "cascade_decode_attention: bad head counts (%d / %d)", num_q_heads, num_kv_heads);
@@ -876,6 +1103,13 @@ int sgl_amd_cascade_decode_attention_ex(const void* q, const void* k_cache, cons
   // (the plan may hold spans: the single-shot form works on its items all the same, and the merge goes by the form launched here)
   p.walks_spans = walks_spans(p.group, head_dim, kv_fp8 != 0) ? 1 : 0;
   const bool loop = worst > (g_cascade_single_shot_units > 0 ? g_cascade_single_shot_units : single_shot_most(chunks, p.walks_spans != 0));
+  if (k_new && kv_layout_hnd) {
+    // (a launch for the step's rows all the same: beside the addresses of head-major pages the looping form has no scalar registers left for theirs)
+    const int rc = sgl_amd_store_kv_cache_ex(k_new, v_new, k_cache, v_cache, new_loc, batch, num_kv_heads, head_dim, k_new_stride, v_new_stride,
+                                             k_cache_row_stride, kv_fp8, k_scale, v_scale, page_size, kv_layout_hnd, stream);
+    if (rc != 0) return rc;
+    k_new = nullptr;
+  }
   const int64_t walkers = g_cascade_loop_grid > 0 ? g_cascade_loop_grid : kv_fp8 || head_dim == 64 ? kLoopGridSmallRows : kLoopGrid;
   dim3 grid(static_cast<unsigned>(loop && walkers < worst ? walkers : worst));
 #define SGL_LAUNCH_CASC2(D_, KERNEL_)                                                                                 \
@@ -890,7 +1124,19 @@ int sgl_amd_cascade_decode_attention_ex(const void* q, const void* k_cache, cons
     if (loop) SGL_LAUNCH_CASC2(D_, cascade_chunk_loop_kernel);    \
     else SGL_LAUNCH_CASC2(D_, cascade_chunk_kernel);              \
   } while (0)
-  if (head_dim == 128) SGL_LAUNCH_CASC(128);
+  if (k_new) {
+    StoreParams sp;
+    sp.chunk = p;
+    sp.rows = NewRows{static_cast<const uint16_t*>(k_new), static_cast<const uint16_t*>(v_new), new_loc, k_new_stride, v_new_stride, 1.0f / k_scale, 1.0f / v_scale};
+#define SGL_LAUNCH_STORE(KERNEL_)                                                                                                   \
+  do {                                                                                                                              \
+    if (kv_fp8) hipLaunchKernelGGL((head_dim == 128 ? KERNEL_<128, true> : KERNEL_<64, true>), grid, dim3(kThreads), 0, st, sp);    \
+    else hipLaunchKernelGGL((head_dim == 128 ? KERNEL_<128, false> : KERNEL_<64, false>), grid, dim3(kThreads), 0, st, sp);         \
+  } while (0)
+    if (loop) SGL_LAUNCH_STORE(cascade_store_loop_kernel);
+    else SGL_LAUNCH_STORE(cascade_store_kernel);
+#undef SGL_LAUNCH_STORE
+  } else if (head_dim == 128) SGL_LAUNCH_CASC(128);
   else SGL_LAUNCH_CASC(64);
 #undef SGL_LAUNCH_CASC2
 #undef SGL_LAUNCH_CASC

@@ -15,6 +15,8 @@
 //   span_first[kSpanUnits + 1], pieces[8 * (B + kSpanUnits)]   (header[4] > 0) span k is pieces span_first[k] .. span_first[k + 1] - 1, records like
 //                        the items'; they stand in the place of the private items for the looping attention kernel
 //   compare[2 B]         scratch between the plan's two launches: leader of request b, its common prefix with the leader
+//   new_slots[B]         the slots that the plan was told the step's rows go to (if it was)
+//   meet[kCheckers]      whether a request reads one of them that is not its own newest token's, a word a workgroup that looked (it was not told: 1)
 #pragma once
 #include <stdint.h>
 
@@ -33,6 +35,8 @@ struct CascadePlanView {
   int32_t* req_slots;
   int32_t* span_first;
   int32_t* pieces;
+  int32_t* new_slots;
+  int32_t* meet;
 };
 
 // (span, kv head) units that a plan of spans aims at, the shared items taken off: three a compute unit.  The looping kernel's registers would
@@ -49,9 +53,11 @@ struct CascadePlanView {
 constexpr int kSpanUnits = 768;
 constexpr int kOneRoundUnits = 1024;
 constexpr int kMinSpanTiles = 3;
+constexpr int kCheckers = 64;        // workgroups that look through the request tables for the new slots, one word each
 
 __host__ __device__ inline int64_t cascade_plan_ints(int64_t batch, int64_t max_items) {
-  return 8 + batch + batch + (batch + 1) + batch + batch + 8 * max_items + batch + 2 * batch + batch + (kSpanUnits + 1) + 8 * (batch + kSpanUnits) + 3;
+  return 8 + batch + batch + (batch + 1) + batch + batch + 8 * max_items + batch + 2 * batch + batch + (kSpanUnits + 1) + 8 * (batch + kSpanUnits) + 3 + batch +
+         kCheckers;
 }
 
 __host__ __device__ inline CascadePlanView cascade_plan_view(const int32_t* plan, int64_t batch, int64_t max_items) {
@@ -69,6 +75,8 @@ __host__ __device__ inline CascadePlanView cascade_plan_view(const int32_t* plan
   v.req_slots = p; p += batch;
   v.span_first = p; p += kSpanUnits + 1;
   v.pieces = v.header + ((p - v.header + 3) & ~static_cast<int64_t>(3));   // 16-byte records
+  v.new_slots = v.pieces + 8 * (batch + kSpanUnits);
+  v.meet = v.new_slots + batch;
   return v;
 }
 

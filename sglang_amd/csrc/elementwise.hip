@@ -328,21 +328,8 @@ __global__ void store_kv_fmt_kernel(const uint16_t* __restrict__ k, const uint16
     const U4 vv8 = ld16(v + tok * v_stride + static_cast<int64_t>(h) * head_dim + c * 8);
     unsigned char* kd = const_cast<unsigned char*>(kv_row(k_cache, fmt, slot, h));
     unsigned char* vd = const_cast<unsigned char*>(kv_row(v_cache, fmt, slot, h));
-    if constexpr (FP8) {
-      const uint32_t kw[4] = {kv8.x, kv8.y, kv8.z, kv8.w}, vw[4] = {vv8.x, vv8.y, vv8.z, vv8.w};
-      float kf[8], vf[8];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        // (K / k_scale) is a bf16 division in the reference (cache_k.div_(k_scale) on a bf16 tensor) before the cast
-        kf[2 * j] = rbf(bf_lo(kw[j]) * inv_k_scale); kf[2 * j + 1] = rbf(bf_hi(kw[j]) * inv_k_scale);
-        vf[2 * j] = rbf(bf_lo(vw[j]) * inv_v_scale); vf[2 * j + 1] = rbf(bf_hi(vw[j]) * inv_v_scale);
-      }
-      *reinterpret_cast<uint2*>(kd + c * 8) = f32x8_to_fp8x8(kf, 1.0f);
-      *reinterpret_cast<uint2*>(vd + c * 8) = f32x8_to_fp8x8(vf, 1.0f);
-    } else {
-      st16(kd + c * 16, kv8);
-      st16(vd + c * 16, vv8);
-    }
+    put_kv8<FP8>(kd, c, kv8, inv_k_scale);
+    put_kv8<FP8>(vd, c, vv8, inv_v_scale);
   }
 }
 

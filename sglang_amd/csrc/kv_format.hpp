@@ -81,6 +81,24 @@ __device__ __forceinline__ uint2 f32x8_to_fp8x8(const float* v, float inv_scale)
   return o;
 }
 
+// 8 bf16 elements of a new row to piece c of a pool row.  e4m3: (K / k_scale) is a bf16 division in the reference (cache_k.div_(k_scale) on a bf16
+// tensor) before the cast (memory_pool.py:2364-2374).
+template <bool FP8>
+__device__ __forceinline__ void put_kv8(unsigned char* row, int c, const U4& x, float inv_scale) {
+  if constexpr (FP8) {
+    const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+    float f[8];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      f[2 * j] = rbf(bf_lo(w[j]) * inv_scale);
+      f[2 * j + 1] = rbf(bf_hi(w[j]) * inv_scale);
+    }
+    *reinterpret_cast<uint2*>(row + c * 8) = f32x8_to_fp8x8(f, 1.0f);
+  } else {
+    st16(row + c * 16, x);
+  }
+}
+
 // logit soft cap in the log2 domain: x = s * log2(e) with s the scaled score; returns cap * tanh(s / cap) * log2(e)
 __device__ __forceinline__ float soft_cap_log2(float x, float cap_log2, float inv_cap_log2) {
   const float t = x * inv_cap_log2;                      // s / cap

@@ -488,25 +488,29 @@ class CascadeWorkspace:
 
 
 def cascade_plan(ws: CascadeWorkspace, req_to_token: torch.Tensor, req_pool_indices: torch.Tensor, seq_lens: torch.Tensor,
-                 num_q_heads: int, num_kv_heads: int, min_shared: int = CASCADE_MIN_SHARED) -> None:
-    """Once per decode step: group the batch by shared KV prefix (device only, graph safe)."""
+                 num_q_heads: int, num_kv_heads: int, min_shared: int = CASCADE_MIN_SHARED, new_loc: Optional[torch.Tensor] = None) -> None:
+    """Once per decode step: group the batch by shared KV prefix (device only, graph safe).  new_loc: the slots (int64 [B]) of the step's rows, for
+    layers that store them in the attention's launch (cascade_decode_attention's new_rows)."""
     _dev(req_to_token, req_pool_indices, seq_lens)
     B = seq_lens.numel()
     _need(B <= ws.max_batch, "cascade_plan: batch larger than the workspace")
     _need(seq_lens.dtype == torch.int32 and req_pool_indices.dtype == torch.int64 and req_to_token.dtype == torch.int32,
           "cascade_plan: dtypes")
     # NOTE: the plan / slot layout is addressed with the ACTUAL batch size B
-    native.call("sgl_amd_cascade_plan", req_to_token.data_ptr(), req_to_token.stride(0), req_pool_indices.data_ptr(),
-                seq_lens.data_ptr(), B, num_q_heads, num_kv_heads, min_shared, ws.max_context_len, ws.plan.data_ptr(),
+    if new_loc is not None:
+        _need(new_loc.dtype == torch.int64 and new_loc.shape == (B,) and new_loc.is_contiguous() and new_loc.is_cuda, "cascade_plan: int64 slots [B]")
+    native.call("sgl_amd_cascade_plan_new_rows", req_to_token.data_ptr(), req_to_token.stride(0), req_pool_indices.data_ptr(),
+                seq_lens.data_ptr(), _ptr(new_loc), B, num_q_heads, num_kv_heads, min_shared, ws.max_context_len, ws.plan.data_ptr(),
                 ws.max_items, _stream())
 
 
 def cascade_decode_attention(ws: CascadeWorkspace, q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                              out: torch.Tensor, req_to_token: torch.Tensor, req_pool_indices: torch.Tensor,
                              seq_lens: torch.Tensor, sm_scale: float, kv_fp8: bool = False, k_scale: float = 1.0,
-                             v_scale: float = 1.0, page_size: int = 1, hnd: bool = False) -> torch.Tensor:
+                             v_scale: float = 1.0, page_size: int = 1, hnd: bool = False, new_rows=None) -> torch.Tensor:
     """Per layer, after cascade_plan(): q/out [B, Hq, D]; pools as in decode_attention (bf16 or uint8 e4m3 rows,
-    [slots, Hkv, D] or [pages, Hkv, page_size, D] with hnd)."""
+    [slots, Hkv, D] or [pages, Hkv, page_size, D] with hnd).  new_rows: (k, v, loc), the step's rows [B, Hkv, D] and their slots (int64 [B]),
+    stored as by store_kv_cache in front, in the same launch (quick where the plan was given loc)."""
     _dev(q, k_cache, v_cache, out)
     B, Hq, D = q.shape
     Hkv = k_cache.shape[1]
@@ -520,11 +524,19 @@ def cascade_decode_attention(ws: CascadeWorkspace, q: torch.Tensor, k_cache: tor
         _need(k_cache.stride(2) == 1 and k_cache.stride(1) == D and v_cache.stride(1) == D
               and k_cache.stride(0) == v_cache.stride(0), "cascade: cache layout")
         row = k_cache.stride(0)
-    native.call("sgl_amd_cascade_decode_attention_ex", q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(),
+    new = (None, None, None, 0, 0)
+    if new_rows is not None:
+        k, v, loc = new_rows
+        _need(k.shape == (B, Hkv, D) and v.shape == (B, Hkv, D) and k.dtype == v.dtype == _BF16 and loc.dtype == torch.int64 and loc.shape == (B,),
+              "cascade: new rows bf16 [B, Hkv, D], int64 slots [B]")
+        (ks, kh, kd), (vs, vh, vd) = k.stride(), v.stride()
+        _need(kh == vh == D and kd == vd == 1 and k.is_cuda and v.is_cuda and loc.is_cuda and loc.is_contiguous(), "cascade: new rows' layout")
+        new = (k.data_ptr(), v.data_ptr(), loc.data_ptr(), ks, vs)
+    native.call("sgl_amd_cascade_decode_attention_store", q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(),
                 req_to_token.data_ptr(), req_to_token.stride(0), req_pool_indices.data_ptr(), seq_lens.data_ptr(),
                 ws.plan.data_ptr(), B, ws.max_items, Hq, Hkv, D, q.stride(0), out.stride(0), row, row,
                 float(sm_scale), ws.max_context_len, ws.slots, ws.ws_acc.data_ptr(), ws.ws_ml.data_ptr(),
-                1 if kv_fp8 else 0, float(k_scale), float(v_scale), int(page_size), 1 if hnd else 0, _stream())
+                1 if kv_fp8 else 0, float(k_scale), float(v_scale), int(page_size), 1 if hnd else 0, *new, _stream())
     return out
 
 
