@@ -467,6 +467,39 @@ def _extend_attention_kv(q, out, k_cache, v_cache, req_to_token, req_pool_indice
     return out
 
 
+def extend_attention_layer(q, k, v, loc, k_cache, v_cache, req_to_token, req_pool_indices, seq_lens, prefix_lens, qo_indptr, max_extend_len: int, max_kv_len: int,
+                           sum_kv_len: int, num_q_heads: int, sm_scale: float, causal: bool, kv_fp8: bool, k_scale: float, v_scale: float) -> Optional[torch.Tensor]:
+    """extend_attention of q [T, Hq * D] with new_rows (k, v, loc), every argument looked at once: what a short prompt's layer waits for is this thread (37 cold
+    tokens, 14 / 2 heads: 20.7 us a call through the views and checks of the general wrappers, 16.4 here).  None, and nothing done, where an argument is not of the
+    plainest form: the general wrappers say what of it is wrong, or take it."""
+    shape, rows, pool = q.shape, k.shape, k_cache.stride()
+    if len(shape) != 2 or len(rows) != 3:
+        return None
+    T, Hkv, D = rows
+    row, (qs, q1), (ks, kh, kd), (vs, vh, vd) = Hkv * D, q.stride(), k.stride(), v.stride()
+    kp, vp = k.data_ptr(), v.data_ptr()
+    if not (shape == (T, num_q_heads * D) and v.shape == rows and q1 == kd == vd == 1 and kh == vh == D and ks % 8 == vs % 8 == 0 and kp % 16 == vp % 16 == 0
+            and q.dtype is k.dtype is v.dtype is _BF16 and k_cache.dtype is v_cache.dtype is (torch.uint8 if kv_fp8 else _BF16)
+            and pool == v_cache.stride() == (row, D, 1) and k_cache.shape[1:] == v_cache.shape[1:] == rows[1:]
+            and loc.dtype is req_pool_indices.dtype is torch.int64 and loc.shape == (T,) and loc.stride(0) == 1
+            and req_to_token.dtype is seq_lens.dtype is prefix_lens.dtype is qo_indptr.dtype is torch.int32
+            and q.is_cuda and k.is_cuda and v.is_cuda and loc.is_cuda and k_cache.is_cuda and v_cache.is_cuda and req_to_token.is_cuda
+            and req_pool_indices.is_cuda and seq_lens.is_cuda and prefix_lens.is_cuda and qo_indptr.is_cuda):
+        return None
+    B, parts, ws = seq_lens.shape[0], 1, 0
+    out = q.new_empty(shape)
+    if max_kv_len > 256:                                  # (a split of four tiles or fewer never pays: not worth asking)
+        parts = native.lib().sgl_amd_extend_attention_store_parts(B, T, sum_kv_len, max_extend_len, max_kv_len, num_q_heads, Hkv, D)
+        if parts != 1:                                    # (0 parts: eight counters)
+            held = torch.empty(parts * T * num_q_heads * (D + 2) or 8, dtype=torch.float32, device=q.device)
+            ws = held.data_ptr()
+    native.call("sgl_amd_extend_attention_store", q.data_ptr(), out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), req_to_token.data_ptr(), req_to_token.stride(0),
+                req_pool_indices.data_ptr(), seq_lens.data_ptr(), prefix_lens.data_ptr(), qo_indptr.data_ptr(), B, T, max_extend_len, max_kv_len, num_q_heads, Hkv, D,
+                qs, num_q_heads * D, row, float(sm_scale), 1 if causal else 0, 1 if kv_fp8 else 0, k_scale, v_scale, parts, ws, ws + 4 * parts * T * num_q_heads * D if ws else 0,
+                kp, vp, loc.data_ptr(), ks, vs, _stream())
+    return out
+
+
 # ------------------------------------------------------------- shared-prefix (cascade) decode
 CASCADE_MIN_SHARED = 128
 

@@ -25,6 +25,7 @@ import torch
 
 from ... import kernels
 from ...mem_cache.memory_pool import KVWriteLoc, MHATokenToKVPool, _host_scale
+from ..radix_attention import AttentionType, RadixAttention
 from .base_attn_backend import AttentionBackend
 
 
@@ -372,7 +373,25 @@ class HipAttnBackend(AttentionBackend):
         if layer.qk_head_dim != layer.v_head_dim:
             raise NotImplementedError(f"hip_mi355x attention backend: qk_head_dim {layer.qk_head_dim} != v_head_dim {layer.v_head_dim} (MLA layouts)")
 
+    def _extend_plain(self, q, k, v, layer, forward_batch):
+        """forward_extend of this package's own layer and pool without any of their switches, or None."""
+        pool, m, loc = self.token_to_kv_pool, self.forward_metadata, forward_batch.out_cache_loc
+        if (type(layer) is not RadixAttention or not isinstance(loc, torch.Tensor) or type(pool) is not MHATokenToKVPool or pool.use_hnd or "set_kv_buffer" in vars(pool) or m.max_kv_len <= 0
+                or layer.logit_cap or layer.sliding_window_size != -1 or layer.is_cross_attention or "xai_temperature_len" in vars(layer)
+                or layer.qk_head_dim != layer.v_head_dim or layer.qk_head_dim != pool.head_dim or getattr(forward_batch, "spec_info", None) is not None):
+            return None
+        i, fp8, kind = layer.layer_id, pool.is_fp8, layer.attn_type
+        return kernels.extend_attention_layer(q, k, v, loc, pool.get_key_buffer(i), pool.get_value_buffer(i),
+                                              self.req_to_token_pool.req_to_token, self._pool_idx(forward_batch), m.seq_lens_i32, m.prefix_lens_i32, m.qo_indptr,
+                                              m.max_extend_len, m.max_kv_len, m.sum_kv_len, layer.tp_q_head_num, layer.scaling,
+                                              kind is AttentionType.DECODER or getattr(kind, "value", kind) != "encoder_only", fp8,
+                                              _host_scale(layer, "k_scale") if fp8 else 1.0, _host_scale(layer, "v_scale") if fp8 else 1.0)
+
     def forward_extend(self, q, k, v, layer, forward_batch, save_kv_cache: bool = True, **kwargs):
+        if save_kv_cache and not kwargs and k is not None and v is not None:
+            o = self._extend_plain(q, k, v, layer, forward_batch)
+            if o is not None:
+                return o
         self._refuse_unsupported(layer, kwargs)
         m = self.forward_metadata
         opt = self._layer_options(layer)
