@@ -606,6 +606,17 @@ int sgl_amd_moe_tiled_gemm_ex(const void* a, const void* w, void* c, const int32
                               int64_t max_m_blocks, int glu_kind, float glu_limit, float glu_alpha, int out_f32, int align_block_m, int tile_rows,
                               void* stream);
 
+/* Experts cut into even tiles, over a 256-row alignment for products that the weights bound: most_rows = rows of a tile, 320 with two
+ * stages of a step, or 240 with three of the weights (at most 256 row blocks then).  max_splits = 0: c is bf16 rows, with the activation.  max_splits 1 .. 4: K is cut into as many parts as
+ * suit the experts' rows, fp32 sums of part s at c + s * part_stride, *splits says how many; sgl_amd_moe_sum_parts then gives
+ * out[m,:] = bf16(routed_scaling_factor * sum_k topk_weights[m,k] * bf16(sum of the parts)).  Operands below 4 GiB of offsets. */
+int sgl_amd_moe_rows_gemm(const void* a, const void* w, void* c, const int32_t* sorted_token_ids, const int32_t* expert_ids,
+                          const int32_t* num_tokens_post_padded, int top_k_div, int64_t num_valid_ids, int64_t N, int64_t K, int64_t a_row_stride,
+                          int64_t w_row_stride, int64_t w_expert_stride, int64_t c_row_stride, int64_t max_m_blocks, int glu_kind, float glu_limit,
+                          float glu_alpha, int most_rows, int max_splits, int64_t part_stride, int32_t* splits, void* stream);
+int sgl_amd_moe_sum_parts(const float* parts, const int32_t* splits, int64_t part_stride, const float* topk_weights, void* output, int64_t num_tokens, int topk,
+                          int hidden, int64_t in_row_stride, int64_t out_row_stride, float routed_scaling_factor, void* stream);
+
 /* ---- fp32 residual stream and gated norms (residual_norm.hip) -----------------------------------------------
  * sgl_amd_residual_norm: one launch between two sublayers.  mode 0: x = table[ids] * scale; 1: x += LayerNorm(y; w1, b1);
  * 2: x = y + step; y may be given as split-K partials (fp32 [splits, rows, width] + optional bias, epilogue 3 of

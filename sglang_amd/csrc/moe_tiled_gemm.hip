@@ -66,6 +66,9 @@ struct TiledParams {
   GluParams glu;
   int eid_shift;                // expert_ids is indexed by (row block >> eid_shift): 128-row tiles over a 256-row alignment
   int n_tiles;                  // 256-form: output-column tiles (its grid is one-dimensional)
+  int max_splits, part_cost;    // moe_rows_kernel in parts of K: most parts, what another part costs (in its unit of clocks)
+  int64_t part_stride;          // elements between two parts of c
+  int32_t* splits;              // how many parts there are
 };
 
 __device__ __forceinline__ void dma16(const uint16_t* src, lds_ptr_t dst) {
@@ -500,11 +503,10 @@ __global__ __launch_bounds__(kThreads2, 1) void moe_gemm256_kernel(TiledParams p
 // LDS-DMA; the ds_read_b128 fragment reads of a 16-lane group then cover all 16 slots of a 256-byte bank row).
 // ---------------------------------------------------------------------------------------------------------------------
 constexpr int kOpW = kT2 * kBK * 2;                  // 32 KiB of weights
-constexpr int kMostUnits = 20;                       // token rows of a tile, in units of 16
-constexpr int kOpX = kMostUnits * 16 * kBK * 2;      // 40 KiB of token rows
-constexpr int kStage3 = kOpW + kOpX;
+constexpr int kMostParts = 4;
 constexpr int kRuns = 1024;                          // experts that a launch can cut into even tiles (moe_align_block_size takes fewer)
-constexpr int kLeastUnits = 10;
+constexpr int kWholeUnits = 20, kFewUnits = 15;      // most units of 16 token rows a tile has
+constexpr int kFewRuns = 256;
 
 // One dword / four dwords of LDS, waited for at once: a read that the compiler sees waits for every store and request to memory.
 __device__ __forceinline__ uint32_t lds_word(uint32_t addr) {
@@ -525,364 +527,24 @@ __device__ __forceinline__ u32x4_t lds_quad(uint32_t addr) {
 // (100 us of K = 4096), 14 behind and the 10 to 15 until the next workgroup ran.  The next tile's first two stages are asked for in front of the
 // outputs, its rows and expert a tile before.
 // us, tiles of 256 in rounds of workgroups / these: 8 experts of 14336 / 4096, 3000 tokens 2303 / 1990, 2048 1814 / 1595, 1500 1213 / 1181, 1000 1133 / 919.
+//
+// FEW units: with one tile an expert every weight comes from behind L2, and a step of 320-row tiles is then 4.8 k clocks, the time that its weights take to
+// arrive.  Where a tile has 240 rows or fewer, LDS holds three stages of weights: they are asked for two steps ahead, and the token rows, which L2 has, one (two
+// ahead as well, 160 rows a tile: no faster).  And all workgroups at one place of K read rows 8 KiB apart, which few memory channels hold: an XCD's workgroups begin
+// an eighth of K behind those of the XCD in front (a place for each column tile: token rows then miss L2, 1000 tokens 860 -> 888).
+// PARTS: the down projection of few rows has fewer tiles than there are compute units (8 experts, 16 column tiles of 4096: 128) and the longest K.  K is cut into
+// up to max_splits parts, as many as make the rounds of parts shortest, by the same estimate as the tiles; their sums are left in fp32, and moe_sum_parts
+// adds them, rounds and weighs as the epilogue here would have.
+// us, both products of 8 experts of 14336 / 4096, 128-row tiles or 320 / PARTS with 320 / three stages / and the turn: 441 tokens 734 / 692 / 621 / 567, 640 873 / 739 / 657 / 656,
+// 800 895 / 772 / 742 / 780 (other rows an expert), 1000 947 / 880 / 862 / 860.  The weights alone are 428 us.
 __global__ __launch_bounds__(kThreads2, 1) void moe_rows_kernel(TiledParams p) {
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[2 * kStage3 + kRuns * 16];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  lds_bytes_t sm3 = (lds_bytes_t)(smem);
-  const uint32_t sm_addr = (uint32_t)(uintptr_t)(sm3);
-  const uint32_t tab_addr = sm_addr + 2 * kStage3;
-  const int blocks = p.num_post_pad[0] / kT2;
-  const int cols_per_tile = p.fuse_silu ? 128 : 256;
-
-  // ---- the row tiles.  A run of an expert's alignment blocks holds its rows, the padding behind them.  Table of runs: first row tile | units of 16 rows |
-  // first unit | expert.  The most units of a tile are the same for all runs: of 10 to 20 the number with which the rounds of tiles over the compute
-  // units, times the clocks of the fullest tile's step, are least.  Every workgroup works this out for itself, in about 4 us. ----
-  int runs = 0;
-  {
-    int* const tab = reinterpret_cast<int*>(smem + 2 * kStage3);
-    int* const scratch = reinterpret_cast<int*>(smem);                     // (the stages are not in use yet)
-    for (int b0 = 0; b0 < blocks; b0 += kThreads2) {
-      const int b = b0 + tid;
-      const int e = b < blocks ? p.expert_ids[b] : -1, before = b > 0 && b < blocks ? p.expert_ids[b - 1] : -2;
-      const unsigned long long starts = __ballot(b < blocks && e != before);
-      if (lane == 0) scratch[wid] = __popcll(starts);
-      __syncthreads();
-      int at = runs + __popcll(starts & ((1ull << lane) - 1ull));
-#pragma unroll
-      for (int w = 0; w < kThreads2 / 64; ++w) {
-        const int n = scratch[w];
-        if (w < wid) at += n;
-        runs += n;
-      }
-      if ((starts >> lane & 1ull) && at < kRuns) {
-        tab[4 * at + 2] = b;
-        tab[4 * at + 3] = e;
-      }
-      __syncthreads();
-    }
-  }
-  const bool even = runs <= kRuns;                     // (more experts than that: tiles are the alignment blocks)
-  int row_tiles = blocks, most = kT2 / 16;
-  if (even) {
-    int* const tab = reinterpret_cast<int*>(smem + 2 * kStage3);
-    int* const scratch = reinterpret_cast<int*>(smem);
-    for (int i = tid; i < runs; i += kThreads2) {
-      const int b0 = tab[4 * i + 2], last = (i + 1 < runs ? tab[4 * i + 6] : blocks) - 1;
-      int units = (last - b0) * (kT2 / 16);
-#pragma unroll
-      for (int u = 0; u < kT2 / 16; ++u) units += p.sorted_ids[last * kT2 + 16 * u] < p.num_valid ? 1 : 0;
-      tab[4 * i + 1] = tab[4 * i + 3] < 0 ? 0 : units;                     // (a filtered expert has no tiles)
-    }
-    __syncthreads();
-    const int cols = (p.N + cols_per_tile - 1) / cols_per_tile;
-    for (int m = kLeastUnits + wid; m <= kMostUnits; m += kThreads2 / 64) {
-      int tiles = 0, fullest = 0;
-      for (int i = lane; i < runs; i += 64) {
-        const int units = tab[4 * i + 1], n = (units + m - 1) / m;
-        tiles += n;
-        if (n > 0) fullest = max(fullest, (units + n - 1) / n);
-      }
-      for (int off = 32; off > 0; off >>= 1) {
-        tiles += __shfl_xor(tiles, off, 64);
-        fullest = max(fullest, __shfl_xor(fullest, off, 64));
-      }
-      // a step's clocks in units of 128: the products of the fullest tile and 1.1 k beside them, or what its requests take
-      if (lane == 0) scratch[16 + m] = (tiles * cols + kNumCus - 1) / kNumCus * max(24, fullest + 9);
-    }
-    __syncthreads();
-    int least = 0x7fffffff;
-    for (int m = kMostUnits; m >= kLeastUnits; --m) {
-      const int cost = scratch[16 + m];
-      if (cost < least) { least = cost; most = m; }
-    }
-    if (wid == 0) {
-      int sum = 0;
-      for (int i0 = 0; i0 < runs; i0 += 64) {
-        const int i = i0 + lane, n = i < runs ? (tab[4 * i + 1] + most - 1) / most : 0;
-        int incl = n;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-          const int v = __shfl_up(incl, off, 64);
-          if (lane >= off) incl += v;
-        }
-        if (i < runs) {
-          tab[4 * i] = sum + incl - n;
-          tab[4 * i + 2] *= kT2 / 16;
-        }
-        sum += __shfl(incl, 63, 64);
-      }
-      if (lane == 0) scratch[0] = sum;
-    }
-    __syncthreads();
-    row_tiles = __builtin_amdgcn_readfirstlane(scratch[0]);
-    most = __builtin_amdgcn_readfirstlane(most);
-    __syncthreads();                                   // (the stages take the place of the scratch)
-  }
-
-  // ---- workgroup -> (row tile, column tile).  All tiles are one line: expert by expert, within one column tile by column tile, within that the row tiles.
-  // Workgroups go to the XCDs round robin by their linear index; XCD x takes the pieces x, x + 8, ... of 32 tiles of the line, so that its
-  // 32 workgroups work on a few column tiles of one expert and its L2 fetches each operand row once for most of them.
-  const int cols = (p.N + cols_per_tile - 1) / cols_per_tile;
-  const int total = row_tiles * cols;
-  const int piece_tiles = total >= kNumCus ? 32 : (total + 7) / 8;
-  const int xcd = blockIdx.x & 7;
-  int place = blockIdx.x >> 3;                         // in the piece
-  if (place >= piece_tiles) return;
-  int at_tile = xcd * piece_tiles + place;
-  if (at_tile >= total) return;
-  // This wave: weight rows 64 wq .., and one half of the tile's token rows; the two waves of a SIMD (wid, wid + 4) share the weight rows.
-  const int wq = wid & 3, wh = wid >> 2;
-  const int r16 = lane & 15, g = lane >> 4;
-
-  // ---- DMA roles: piece j of an operand tile is its rows 8j .. 8j+7 (lane i -> row 8j + i/8, slot i%8, global
-  // piece slot ^ (row & 7)); wave w issues the pieces 4w .. 4w+3 of the W tile and w, w + 8, ... of the X tile's 2 `units`.
-  const int dr = lane >> 3, ds = lane & 7;
-  constexpr int XP = kMostUnits / 4;
-  uint32_t aoff[XP];                                   // token rows (X tile), bytes behind p.a
-  uint32_t boff[4];                                    // weight rows (W tile), bytes behind the expert's
-  const unsigned char* wbase;
-  // the tile whose stages are asked for
-  int nt0, units, row0;
-  bool valid;
-  // what the next tile's pointers follow from
-  struct Wanted { int e, nt, units, row0, sid[XP]; };
-  auto want = [&](int at, Wanted& w) {
-    const int rt = at / cols;                          // (a run's first tile of the line is `cols` times its first row tile)
-    if (even) {
-      // the last run that begins at this row tile or in front of it, in two looks of a lane a run
-      auto begins = [&](int i, bool on) { return __ballot(on && i < runs && static_cast<int>(lds_word(tab_addr + 16 * (i < runs ? i : 0))) <= rt); };
-      const int sixteen = 16 * (__popcll(begins(16 * lane, true)) - 1);
-      const int run = sixteen + __popcll(begins(sixteen + lane, lane < 16)) - 1;
-      const u32x4_t t = lds_quad(tab_addr + 16 * run);
-      const int first = __builtin_amdgcn_readfirstlane(t.x), all = __builtin_amdgcn_readfirstlane(t.y);
-      const int tiles = (all + most - 1) / most, in = at - first * cols;
-      w.nt = in / tiles;
-      const RowTile tile = even_tile(all, tiles, in - w.nt * tiles);
-      w.units = tile.units;
-      w.row0 = (__builtin_amdgcn_readfirstlane(t.z) + tile.from) * 16;
-      w.e = __builtin_amdgcn_readfirstlane(t.w);
-    } else {
-      w.nt = at - rt * cols;
-      w.row0 = rt * kT2;
-      w.units = __popcll(__ballot(lane < kT2 / 16 && p.sorted_ids[w.row0 + 16 * (lane & 15)] < p.num_valid));
-      w.e = p.expert_ids[rt];
-    }
-#pragma unroll
-    for (int u = 0; u < XP; ++u) {
-      const int j = wid + 8 * u;
-      w.sid[u] = j < 2 * w.units ? p.sorted_ids[w.row0 + 8 * j + dr] : 0;
-    }
-  };
-  auto set_tile = [&](const Wanted& w) {
-    nt0 = w.nt;
-    units = w.units;
-    row0 = w.row0;
-    valid = w.e >= 0 && w.units > 0;         // (a filtered expert)
-    wbase = reinterpret_cast<const unsigned char*>(p.w + static_cast<int64_t>(valid ? w.e : 0) * p.w_expert_stride);
-    const int piece = (ds ^ dr) * 16;
-#pragma unroll
-    for (int u = 0; u < XP; ++u) {
-      const int srow = w.sid[u] < p.num_valid ? w.sid[u] / p.topk_div : 0;      // padding rows read row 0, their outputs are dropped
-      aoff[u] = static_cast<uint32_t>(srow) * static_cast<uint32_t>(2 * p.a_stride) + piece;
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int row = (wid * 4 + u) * 8 + dr;          // 0..255
-      int wrow;
-      if (p.fuse_silu) {
-        // tile rows: per quarter of 64, [32 gate | 32 up] of output columns nt0 * 128 + quarter * 32 + c
-        const int in = row & 63, col = nt0 * 128 + (row >> 6) * 32 + (in & 31);
-        wrow = (in < 32 ? 0 : p.N) + (col < p.N ? col : p.N - 1);
-      } else {
-        const int col = nt0 * 256 + row;
-        wrow = col < p.N ? col : p.N - 1;
-      }
-      boff[u] = static_cast<uint32_t>(wrow) * static_cast<uint32_t>(2 * p.w_row_stride) + piece;
-    }
-  };
-  auto issue = [&](int kt, int stage) {
-    const unsigned char* wk = wbase + kt * (2 * kBK);
-    const unsigned char* ak = reinterpret_cast<const unsigned char*>(p.a) + kt * (2 * kBK);
-#pragma unroll
-    for (int u = 0; u < 4; ++u) dma16(reinterpret_cast<const uint16_t*>(wk + boff[u]), (lds_ptr_t)(sm3 + stage * kStage3 + (wid * 4 + u) * 1024));
-#pragma unroll
-    for (int u = 0; u < XP; ++u)
-      if (wid + 8 * u < 2 * units) dma16(reinterpret_cast<const uint16_t*>(ak + aoff[u]), (lds_ptr_t)(sm3 + stage * kStage3 + kOpW + (wid + 8 * u) * 1024));
-  };
-
-  uint32_t foff[2];
-#pragma unroll
-  for (int kk = 0; kk < 2; ++kk) foff[kk] = r16 * 128 + (((kk * 4 + g) ^ (r16 & 7)) & 7) * 16;
-  const uint32_t w_base = sm_addr + wq * (64 * 128);   // this wave's 64 weight rows of the W tile
-
-  constexpr int MOST = kMostUnits / 2;                 // 16-row token tiles of a wave
-  f32x4_t acc[4][MOST];                                // [weight 16-row tile][token 16-row tile]
-
-  auto read_w = [&](uint32_t ad, u32x4_t (&wf)[4]) {
-    wf[0] = lds_rd<0>(ad); wf[1] = lds_rd<2048>(ad); wf[2] = lds_rd<4096>(ad); wf[3] = lds_rd<6144>(ad);
-  };
-  const int nk = p.K / kBK;
-  // The steps of a wave with TILES token tiles, two at a time.  Issue the next step's tiles, read and multiply this step's, wait,
-  // barrier.  The fragments of a pair are read a pair ahead of its eight products.  (Of 256-row tiles, measured equal to 5 % slower: a barrier ahead of the last
-  // quarter with the next stage's first fragments read behind it.  Touching a step's 64 lines one to three steps ahead, so that they wait in L2: 5
-  // to 7 % slower, first-touch latency is not what the walk waits for -- profiles/r04_exp4_moe_gemm_ab.json.  Products of 32 x 32: 7 % slower.)
-  auto walk = [&](auto tiles_of, uint32_t x_base) __attribute__((always_inline)) {
-    constexpr int TILES = decltype(tiles_of)::value, PAIRS = (TILES + 1) / 2;
-#pragma clang loop unroll(disable)
-    for (int kt = 0; kt < nk; ++kt) {
-      const int stage = kt & 1;
-      if (kt > 0 && kt + 1 < nk) issue(kt + 1, stage ^ 1);
-      if constexpr (PAIRS > 0) {
-        u32x4_t wf[2][4], xf[2][2];
-        const uint32_t wa = w_base + stage * kStage3, xa = x_base + stage * kStage3;
-        auto read_x = [&](auto n) __attribute__((always_inline)) {                    // pair n of both halves of the step
-          constexpr int KK = decltype(n)::value / PAIRS, JP = decltype(n)::value % PAIRS;
-          xf[decltype(n)::value & 1][0] = lds_rd<JP * 4096>(xa + foff[KK]);
-          if constexpr (2 * JP + 1 < TILES) xf[decltype(n)::value & 1][1] = lds_rd<JP * 4096 + 2048>(xa + foff[KK]);
-        };
-        read_w(wa + foff[0], wf[0]);
-        read_x(std::integral_constant<int, 0>{});
-        // (a wave that multiplies goes ahead of one that reads fragments or asks for tiles: 2310 -> 2240 us for both projections of 3000 tokens)
-        __builtin_amdgcn_s_setprio(1);
-        auto pair = [&](auto n) __attribute__((always_inline)) {
-          constexpr int NN = decltype(n)::value, KK = NN / PAIRS, JP = NN % PAIRS;
-          if constexpr (NN + 1 < 2 * PAIRS) {
-            if constexpr (NN + 1 == PAIRS) read_w(wa + foff[1], wf[1]);
-            read_x(std::integral_constant<int, NN + 1>{});
-            wait_lgkm<(NN + 1 == PAIRS ? 4 : 0) + (2 * ((NN + 1) % PAIRS) + 1 < TILES ? 2 : 1)>();
-          } else {
-            wait_lgkm<0>();
-          }
-#pragma unroll
-          for (int i = 0; i < 4; ++i) pin(wf[KK][i]);
-          pin(xf[NN & 1][0]);
-          if constexpr (2 * JP + 1 < TILES) pin(xf[NN & 1][1]);
-#pragma unroll
-          for (int j = 0; j < (2 * JP + 1 < TILES ? 2 : 1); ++j)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              acc[i][2 * JP + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[KK][i]), __builtin_bit_cast(bf16x8_t, xf[NN & 1][j]),
-                                                                          acc[i][2 * JP + j], 0, 0, 0);
-          __builtin_amdgcn_sched_barrier(0);
-        };
-        pair(std::integral_constant<int, 0>{});
-        pair(std::integral_constant<int, 1>{});
-        if constexpr (PAIRS > 1) { pair(std::integral_constant<int, 2>{}); pair(std::integral_constant<int, 3>{}); }
-        if constexpr (PAIRS > 2) { pair(std::integral_constant<int, 4>{}); pair(std::integral_constant<int, 5>{}); }
-        if constexpr (PAIRS > 3) { pair(std::integral_constant<int, 6>{}); pair(std::integral_constant<int, 7>{}); }
-        if constexpr (PAIRS > 4) { pair(std::integral_constant<int, 8>{}); pair(std::integral_constant<int, 9>{}); }
-        __builtin_amdgcn_s_setprio(0);
-      }
-      if (kt > 0) wait_vm<0>();                        // (stage 1 landed with stage 0)
-      __builtin_amdgcn_s_barrier();
-    }
-  };
-
-  // What the tile after the next one asks for is looked up while the next one's first stages are on their way and waited for with them: a load that
-  // the compiler sees on its way would be waited for within the steps.
-  auto landed = [&](Wanted& w) {
-    wait_vm<0>();
-    __builtin_amdgcn_s_waitcnt(0x0f70);                // vmcnt(0) once more, as the compiler knows it: it counts nothing as on its way from here
-#pragma unroll
-    for (int u = 0; u < XP; ++u) asm volatile("" : "+v"(w.sid[u]));
-  };
-  const int stride = 8 * piece_tiles;
-  Wanted next;
-  want(at_tile, next);
-  set_tile(next);
-  if (valid) {
-    issue(0, 0);
-    if (nk > 1) issue(1, 1);
-  }
-  if (at_tile + stride < total) want(at_tile + stride, next);
-  landed(next);
-  while (true) {
-    __builtin_amdgcn_s_barrier();                      // this tile's first two stages are in LDS
-    const int tnt = nt0;
-    const bool tvalid = valid;
-    const bool more = at_tile + stride < total;
-    // this wave's 16-row token tiles: the first half of them, rounded up, or the rest
-    const int half0 = (units + 1) >> 1, mine = tvalid ? (wh ? units - half0 : half0) : 0;
-    const int trow0 = row0 + (wh ? half0 * 16 : 0);
-    if (tvalid) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < MOST; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      const uint32_t x_base = sm_addr + kOpW + (wh ? half0 * 2048 : 0);
-      switch (mine) {
-        case 10: walk(std::integral_constant<int, 10>{}, x_base); break;
-        case 9: walk(std::integral_constant<int, 9>{}, x_base); break;
-        case 8: walk(std::integral_constant<int, 8>{}, x_base); break;
-        case 7: walk(std::integral_constant<int, 7>{}, x_base); break;
-        case 6: walk(std::integral_constant<int, 6>{}, x_base); break;
-        case 5: walk(std::integral_constant<int, 5>{}, x_base); break;
-        case 4: walk(std::integral_constant<int, 4>{}, x_base); break;
-        case 3: walk(std::integral_constant<int, 3>{}, x_base); break;
-        case 2: walk(std::integral_constant<int, 2>{}, x_base); break;
-        case 1: walk(std::integral_constant<int, 1>{}, x_base); break;
-        default: walk(std::integral_constant<int, 0>{}, x_base); break;
-      }
-    }
-    at_tile += stride;
-    if (more) {
-      set_tile(next);
-      if (valid) {
-        issue(0, 0);
-        if (nk > 1) issue(1, 1);
-      }
-      if (at_tile + stride < total) want(at_tile + stride, next);
-    }
-    // ---- outputs: lane holds C^T[n = 16 i + 4 g + r][m = 16 j + r16].  The next tile's stages are waited for ahead of the stores, so that nobody waits
-    // for these: before they return, two steps of the next tile go by. ----
-    const int lane_now = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), m16 = lane_now & 15, n4 = (lane_now >> 4) * 4;   // (r16 and 4 g, kept by nobody)
-    int row_sid[MOST];
-#pragma unroll
-    for (int j = 0; j < MOST; ++j) row_sid[j] = j < mine ? p.sorted_ids[trow0 + j * 16 + m16] : p.num_valid;
-    landed(next);
-#pragma unroll
-    for (int j = 0; j < MOST; ++j) {
-      if (j >= mine) continue;
-      const int sid = row_sid[j];
-      const bool real = sid < p.num_valid;
-      if (p.fuse_silu) {
-        // weight tiles 0, 1 = gate columns [0, 32) of this wave's quarter, tiles 2, 3 = the matching up columns
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const int col = tnt * 128 + wq * 32 + i * 16 + n4;
-          const float gv[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
-          const float uv[4] = {acc[i + 2][j][0], acc[i + 2][j][1], acc[i + 2][j][2], acc[i + 2][j][3]};
-          float o[4];
-          glu4(p.glu, gv, uv, o);
-          uint2 w2;
-          w2.x = pack_bf2(o[0], o[1]); w2.y = pack_bf2(o[2], o[3]);
-          if (real && col < p.N) *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.c) + static_cast<int64_t>(sid) * p.c_stride + col) = w2;
-        }
-      } else {
-        const float scale = p.row_scale && real ? p.row_scale[sid] : 1.f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int col = tnt * 256 + wq * 64 + i * 16 + n4;
-          float o[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float v = act_pointwise(p.glu.kind) ? squared_relu(acc[i][j][r]) : acc[i][j][r];
-            o[r] = p.row_scale ? (p.round_before_scale ? rbf(v) : v) * scale : v;
-          }
-          if (!real || col >= p.N) continue;
-          if (p.out_f32) {
-            *reinterpret_cast<f32x4_t*>(static_cast<float*>(p.c) + static_cast<int64_t>(sid) * p.c_stride + col) = f32x4_t{o[0], o[1], o[2], o[3]};
-          } else {
-            uint2 w2;
-            w2.x = pack_bf2(o[0], o[1]); w2.y = pack_bf2(o[2], o[3]);
-            *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.c) + static_cast<int64_t>(sid) * p.c_stride + col) = w2;
-          }
-        }
-      }
-    }
-    if (!more) return;
-  }
+  constexpr int UNITS = kWholeUnits;
+  constexpr bool PARTS = false;
+#include "moe_rows_body.inc"
+}
+template <int UNITS, bool PARTS>
+__global__ __launch_bounds__(kThreads2, 1) void moe_weight_bound_kernel(TiledParams p) {
+#include "moe_rows_body.inc"
 }
 
 }  // namespace
@@ -954,6 +616,50 @@ int sgl_amd_moe_tiled_gemm_ex(const void* a, const void* w, void* c, const int32
   dim3 grid(static_cast<unsigned>((N + cols_per_tile - 1) / cols_per_tile), static_cast<unsigned>(m_blocks));
   hipLaunchKernelGGL(moe_tiled_gemm_kernel, grid, dim3(kThreads), 0, as_stream(stream), p);
   SGL_CHECK_LAUNCH("moe_tiled_gemm");
+  return 0;
+}
+
+int sgl_amd_moe_rows_gemm(const void* a, const void* w, void* c, const int32_t* sorted_token_ids, const int32_t* expert_ids,
+                          const int32_t* num_tokens_post_padded, int top_k_div, int64_t num_valid_ids, int64_t N, int64_t K, int64_t a_row_stride,
+                          int64_t w_row_stride, int64_t w_expert_stride, int64_t c_row_stride, int64_t max_m_blocks, int glu_kind, float glu_limit,
+                          float glu_alpha, int most_rows, int max_splits, int64_t part_stride, int32_t* splits, void* stream) {
+  SGL_CLEAR_STALE_ERROR();
+  SGL_CHECK_ARG(glu_kind >= kGluNone && glu_kind < kActKinds, "moe_rows_gemm: no activation %d", glu_kind);
+  const int gated = act_gated(glu_kind);
+  SGL_CHECK_ARG(N > 0 && N % 4 == 0 && K >= kBK && K % kBK == 0, "moe_rows_gemm: need N %% 4 == 0 and K %% %d == 0 (got N=%lld K=%lld)", kBK, (long long)N, (long long)K);
+  SGL_CHECK_ARG(!gated || N % 32 == 0, "moe_rows_gemm: the gated form needs N %% 32 == 0");
+  SGL_CHECK_ARG(a_row_stride % 8 == 0 && w_row_stride % 8 == 0 && c_row_stride % 4 == 0, "moe_rows_gemm: row strides must keep 16-byte (a, w) / 8-byte (c) alignment");
+  SGL_CHECK_ARG(top_k_div >= 1 && num_valid_ids >= 0 && num_valid_ids <= 0x7fffffffLL && max_m_blocks >= 0, "moe_rows_gemm: bad top_k_div / sizes");
+  SGL_CHECK_ARG(max_splits >= 0 && max_splits <= kMostParts && (max_splits == 0 || (splits != nullptr && glu_kind == kGluNone && K / kBK >= max_splits && part_stride % 4 == 0 &&
+                                                                                  part_stride >= num_valid_ids * c_row_stride)),
+                "moe_rows_gemm: parts of K need a count, no activation, a step each and room (max_splits %d)", max_splits);
+  SGL_CHECK_ARG(most_rows == 16 * kFewUnits || most_rows == 16 * kWholeUnits, "moe_rows_gemm: tiles of 240 or 320 rows (got %d)", most_rows);
+  SGL_CHECK_ARG(most_rows == 16 * kWholeUnits || max_m_blocks <= kFewRuns, "moe_rows_gemm: more than %d row blocks are not cut into tiles of few rows", kFewRuns);
+  if (max_m_blocks == 0 || num_valid_ids == 0) return 0;
+  const int64_t w_rows = gated ? 2 * N : N, a_rows = (num_valid_ids + top_k_div - 1) / top_k_div, col_tiles = (N + (gated ? 127 : 255)) / (gated ? 128 : 256);
+  SGL_CHECK_ARG(w_rows * w_row_stride * 2 < (int64_t{1} << 32) && a_rows * a_row_stride * 2 < (int64_t{1} << 32) &&
+                    col_tiles * 4 * max_m_blocks * (max_splits > 1 ? max_splits : 1) <= 0x3fffffffLL,
+                "moe_rows_gemm: operands past 4 GiB of offsets");
+  TiledParams p{};
+  p.a = static_cast<const uint16_t*>(a); p.w = static_cast<const uint16_t*>(w); p.c = c;
+  p.sorted_ids = sorted_token_ids; p.expert_ids = expert_ids; p.num_post_pad = num_tokens_post_padded;
+  p.a_stride = a_row_stride; p.w_row_stride = w_row_stride; p.w_expert_stride = w_expert_stride; p.c_stride = c_row_stride;
+  p.num_valid = static_cast<int>(num_valid_ids); p.N = static_cast<int>(N); p.K = static_cast<int>(K); p.topk_div = top_k_div;
+  p.fuse_silu = gated; p.glu = GluParams{glu_kind, glu_limit, glu_alpha};
+  p.max_splits = max_splits;
+  // another part is written and read once more in fp32: 8 bytes a number at 5 TB/s and 2.4 GHz, in units of 128 clocks
+  const double part_cost = 3e-5 * static_cast<double>(num_valid_ids) * static_cast<double>(N);
+  p.part_cost = part_cost < 1e8 ? static_cast<int>(part_cost) : 100000000;
+  p.part_stride = part_stride; p.splits = splits;
+  const dim3 grid(kNumCus), block(kThreads2);
+  if (most_rows == 16 * kFewUnits) {
+    if (max_splits) hipLaunchKernelGGL((moe_weight_bound_kernel<kFewUnits, true>), grid, block, 0, as_stream(stream), p);
+    else hipLaunchKernelGGL((moe_weight_bound_kernel<kFewUnits, false>), grid, block, 0, as_stream(stream), p);
+  } else {
+    if (max_splits) hipLaunchKernelGGL((moe_weight_bound_kernel<kWholeUnits, true>), grid, block, 0, as_stream(stream), p);
+    else hipLaunchKernelGGL(moe_rows_kernel, grid, block, 0, as_stream(stream), p);
+  }
+  SGL_CHECK_LAUNCH("moe_rows_gemm");
   return 0;
 }
 

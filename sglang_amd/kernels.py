@@ -1218,6 +1218,46 @@ def moe_tiled_gemm(a: torch.Tensor, w: torch.Tensor, c: torch.Tensor, sorted_tok
     return c
 
 
+def moe_rows_gemm(a: torch.Tensor, w: torch.Tensor, c: torch.Tensor, sorted_token_ids: torch.Tensor, expert_ids: torch.Tensor,
+                  num_tokens_post_padded: torch.Tensor, top_k_div: int, num_valid_ids: int, most_rows: int, act: Optional[Glu] = None,
+                  splits: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """moe_tiled_gemm for experts whose weights bound a product, over the 256-row alignment: c [num_valid_ids, N] bf16 with the activation `act`, or,
+    with `splits` (int32 [1], says how many), the fp32 sums of up to four parts of K, c [parts, num_valid_ids, N], for moe_sum_parts."""
+    _dev(a, w, c, sorted_token_ids, expert_ids, num_tokens_post_padded)
+    _need(a.dtype == _BF16 and w.dtype == _BF16 and w.dim() == 3 and a.dim() == 2, "moe_rows_gemm: bf16 a, w [E, N, K]")
+    _need(sorted_token_ids.dtype == torch.int32 and expert_ids.dtype == torch.int32 and num_tokens_post_padded.dtype == torch.int32, "moe_rows_gemm: int32 metadata")
+    E, WN, K = w.shape
+    gated = act is not None and act.gated
+    N = WN // 2 if gated else WN
+    if splits is None:
+        _need(c.dtype == _BF16 and c.dim() == 2, "moe_rows_gemm: bf16 rows")
+    else:
+        _need(act is None and c.dtype == torch.float32 and c.dim() == 3 and 1 <= c.shape[0] <= 4 and c.is_contiguous() and splits.dtype == torch.int32 and splits.numel() == 1,
+              "moe_rows_gemm: fp32 parts and their count")
+        _dev(splits)
+    _need(c.shape[-2:] == (num_valid_ids, N) and a.shape[1] == K and a.stride(1) == 1 and w.stride(2) == 1 and c.stride(-1) == 1
+          and a.shape[0] * top_k_div >= num_valid_ids, "moe_rows_gemm: shapes / contiguity")
+    max_m_blocks = expert_ids.numel()
+    _need(sorted_token_ids.numel() >= max_m_blocks * 256, "moe_rows_gemm: sorted_token_ids too short")
+    native.call("sgl_amd_moe_rows_gemm", a.data_ptr(), w.data_ptr(), c.data_ptr(), sorted_token_ids.data_ptr(), expert_ids.data_ptr(),
+                num_tokens_post_padded.data_ptr(), top_k_div, num_valid_ids, N, K, a.stride(0), w.stride(1), w.stride(0), c.stride(-2), max_m_blocks,
+                *(NO_GLU if act is None else act.args), int(most_rows), 0 if splits is None else c.shape[0], 0 if splits is None else c.stride(0),
+                _ptr(splits), _stream())
+    return c
+
+
+def moe_sum_parts(parts: torch.Tensor, splits: torch.Tensor, topk_weights: torch.Tensor, out: torch.Tensor, routed_scaling_factor: float = 1.0) -> torch.Tensor:
+    """out [M, H] of the parts [S, M * topk, H] that moe_rows_gemm left: each row's sum in bf16 times its weight, summed over topk."""
+    _dev(parts, splits, topk_weights, out)
+    _need(parts.dtype == torch.float32 and parts.is_contiguous() and topk_weights.dtype == torch.float32 and topk_weights.is_contiguous() and topk_weights.dim() == 2
+          and splits.dtype == torch.int32, "moe_sum_parts: fp32 parts and weights")
+    M, topk = topk_weights.shape
+    _need(parts.shape[1] == M * topk and out.dtype == _BF16 and out.shape == (M, parts.shape[2]) and out.stride(1) == 1, "moe_sum_parts: shapes")
+    native.call("sgl_amd_moe_sum_parts", parts.data_ptr(), splits.data_ptr(), parts.stride(0), topk_weights.data_ptr(), out.data_ptr(), M, topk, parts.shape[2],
+                parts.stride(1), out.stride(0), float(routed_scaling_factor), _stream())
+    return out
+
+
 MOE_TILE_OVERRIDE = None                # tests / benchmarks: (align block, up tile rows, down tile rows)
 # From here on the row-tiled form: the weight-streaming one takes 64 rows at a time, and an expert with more reads its weights again.  us, both products,
 # streaming / 128-row tiles, two routings each: 8 experts of 14336 / 4096 with 48 rows 613 / 592, 600 / 575, with 60 710 / 595, 699 / 578, with 90 922 / 620,
@@ -1296,6 +1336,34 @@ def moe_rows(numel: int, num_experts: int, n_up: int, n_down: int):
     if (tiles >= 640 and rows >= 140) or (tiles >= 256 and rows >= 300):
         return 256, 256, 256
     return moe_tile_plan(numel, num_experts, n_up, n_down)
+
+
+MOE_PARTS_OVERRIDE = None               # tests / benchmarks: (most rows of a tile, most parts of K)
+
+
+def moe_weight_bound(numel: int, num_experts: int, n_up: int, n_down: int):
+    """(most rows of a tile, most parts of K of the down projection) where moe_rows_gemm takes both products of fused_experts; (320, 0): it doesn't.
+    Tiles of 240 rows from 50 or 56 rows an expert on, where weights no longer stream for one block of rows, to 330, where products bound both forms; in front of
+    320-row tiles without parts, 128-row tiles and streams.  us, those / these: 8 experts of 14336 / 4096 with 40 rows 590 / 530, 50 640 / 541, 64 587 / 539, 90 709 / 543, 130 820 / 598,
+    180 860 / 673, 240 923 / 823, 300 1063 / 967, 440 1231 / 1281; of 7168 / 4096 with 50 269 / 280, 64 315 / 285, 130 414 / 313, 240 566 / 451, 300 557 / 530, 360 579 / 596;
+    of 3584 / 4096 (224 column tiles of the up projection, the line) with 64 169 / 159, 130 217 / 191, 300 351 / 288; 64 of 1408 / 2048 with 50 280 / 250, 130 367 / 317, 300 534 /
+    491; 32 of 7168 / 4096 with 50 1114 / 1007, 130 1437 / 1184, 240 1664 / 1633, 300 1919 / 1967 (past 1024 column tiles 256 rows are the line); 128 of 768 / 2048 with 50 330 / 309, 240
+    605 / 539; 16 of 2048 / 2048 with 64 113 / 113, 130 149 / 139, 180 156 / 158, 300 221 / 195; 4 of 1024 / 1024 (32) with 130 45 / 49.
+    Tiles of 320 rows with the down projection in two parts from 480 rows on while that has up to two rounds of tiles and a long K: 8 of 14336 / 4096 with 440 1240 / 1231,
+    with 560 1651 / 1561, 750 1986 / 1942, 1000 2440 / 2386; of 7168 / 4096 with 750 1014 / 993, with 1000 1272 / 1297.
+    No more parts than give four rounds of tiles: another part is another fp32 copy of the rows."""
+    rows, col_tiles, down = numel / max(1, num_experts), num_experts * -(-n_up // 128), num_experts * -(-n_down // 256)
+    blocks = (numel + (num_experts + 1) * 255 + 255) // 256      # moe_align_block_size's
+    if blocks <= 256 and col_tiles >= 224 and (50 if col_tiles >= 640 else 56) <= rows <= (330 if col_tiles <= 1024 else 256):
+        return 240, max(1, min(4, 1024 // (down * -(-int(rows) // 240))))
+    if rows >= 480 and n_up >= 8192 and col_tiles >= 640 and down * -(-int(rows) // 320) <= 512:
+        return 320, 2
+    return 320, 0
+
+
+def _offsets_fit(*rows_strides) -> bool:
+    """Whether all of (rows, row stride in elements) stay below 4 GiB of bf16."""
+    return all(2 * rows * stride < 1 << 32 for rows, stride in rows_strides)
 
 
 def moe_grouped_gemm(a: torch.Tensor, w: torch.Tensor, c: torch.Tensor, sorted_token_ids: torch.Tensor,
@@ -1411,6 +1479,17 @@ def fused_experts(hidden_states: torch.Tensor, w13: torch.Tensor, w2: torch.Tens
         out = torch.empty((M, K), dtype=_BF16, device=dev)
     if M == 0:
         return out
+    most, parts = MOE_PARTS_OVERRIDE or ((320, 0) if MOE_TILE_OVERRIDE is not None else moe_weight_bound(numel, E, N, K))
+    if (parts > 0 and K % 64 == 0 and N % 64 == 0
+            and _offsets_fit((N2, w13.stride(1)), (K, w2.stride(1)), (M, hidden_states.stride(0)), (numel, N))):
+        # an expert's weights take longer than its products: read once for all of its rows
+        sorted_ids, expert_ids, post = moe_align_block_size(topk_ids, 256, E)
+        inter = torch.empty((numel, N), dtype=_BF16, device=dev)
+        moe_rows_gemm(hidden_states, w13, inter, sorted_ids, expert_ids, post, topk, numel, most, act=SILU)
+        down = torch.empty((parts, numel, K), dtype=torch.float32, device=dev)
+        splits = torch.empty(1, dtype=torch.int32, device=dev)
+        moe_rows_gemm(inter, w2, down, sorted_ids, expert_ids, post, 1, numel, most, splits=splits)
+        return moe_sum_parts(down, splits, topk_weights.reshape(M, topk).contiguous(), out, routed_scaling_factor)
     if _row_tiled(numel, E, N) and K % 64 == 0 and N % 64 == 0:
         # prefill-sized batch: row-tiled MFMA kernels, every expert's weights read once per 128 / 256 of its rows
         block_m, up_rows, down_rows = moe_rows(numel, E, N, K)

@@ -1,0 +1,89 @@
+"""Experts whose weights bound their products (moe_weight_bound_kernel, moe_sum_parts): tiles of 240 rows with three stages of weights, K of the down projection in
+parts, against float64."""
+import pytest
+import torch
+
+from sglang_amd import kernels as K
+
+BF = torch.bfloat16
+
+
+def test_where_these_tiles_are_taken():
+    for rows, experts, up, down, most in ((49, 8, 14336, 4096, 320), (50, 8, 14336, 4096, 240), (55, 8, 7168, 4096, 320), (56, 8, 7168, 4096, 240), (330, 8, 14336, 4096, 240),
+                                          (331, 8, 14336, 4096, 320), (256, 32, 7168, 4096, 240), (257, 32, 7168, 4096, 320), (130, 4, 1024, 1024, 320),
+                                          (254, 128, 768, 2048, 240), (258, 128, 768, 2048, 320)):
+        assert K.moe_weight_bound(rows * experts, experts, up, down)[0] == most, (rows, experts)
+    assert K.moe_weight_bound(8 * 130, 8, 14336, 4096) == (240, 4) and K.moe_weight_bound(64 * 130, 64, 1408, 2048) == (240, 2)
+    assert K.moe_weight_bound(6000, 8, 14336, 4096) == (320, 2)
+    for pairs, experts, up, down in ((8 * 479, 8, 14336, 4096), (8 * 1281, 8, 14336, 4096), (8 * 750, 8, 7168, 4096)):
+        assert K.moe_weight_bound(pairs, experts, up, down) == (320, 0)
+
+
+def _pairs(loads, topk, g):
+    """Pairs of every expert in no order, `topk` a token."""
+    ids = torch.repeat_interleave(torch.arange(len(loads)), torch.tensor(loads))
+    return ids[torch.randperm(ids.numel(), generator=g)].to(torch.int32).view(-1, topk).cuda()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("most", [240, 320])
+@pytest.mark.parametrize("loads,N,Kd", [((1, 16, 17, 0), 64, 64), ((239, 240, 241, 2), 320, 128), ((15, 241, 480, 481), 288, 192), ((225, 224, 0, 33), 576, 512),
+                                        ((320, 321, 640, 7), 256, 832)])
+def test_products_of_few_rows(most, loads, N, Kd):
+    g = torch.Generator().manual_seed(sum(loads) + N)
+    E, numel = len(loads), sum(loads)
+    ids = _pairs(loads, 2 if numel % 2 == 0 else 1, g)
+    M, topk = ids.shape
+    flat = ids.flatten().long()
+    s, e, post = K.moe_align_block_size(ids, 256, E)
+    x = torch.randn((M, Kd), generator=g).to(BF).cuda()
+    rows = x[torch.arange(numel, device="cuda") // topk]
+    # gated up projection: the activation's argument is one fp32 sum, its value rounded to bf16 twice (2^-8 of it each) and once more with `up`
+    w13 = (torch.randn((E, 2 * N, Kd), generator=g) * 0.05).to(BF).cuda()
+    up = torch.empty((numel, N), dtype=BF, device="cuda")
+    K.moe_rows_gemm(x, w13, up, s, e, post, topk, numel, most, act=K.SILU)
+    want = torch.empty((numel, 2 * N), dtype=torch.float64, device="cuda")
+    for i in range(E):
+        want[flat == i] = rows[flat == i].double() @ w13[i].double().T.contiguous()
+    want = torch.nn.functional.silu(want[:, :N]) * want[:, N:]
+    assert bool(((up.double() - want).abs() <= 2.0 ** -6 * want.abs() + 1e-3).all())
+    # parts of K: fp32 sums of Kd products in any order
+    w2 = (torch.randn((E, N, Kd), generator=g) * 0.05).to(BF).cuda()
+    want, bound = torch.empty((numel, N), dtype=torch.float64, device="cuda"), torch.empty((numel, N), dtype=torch.float64, device="cuda")
+    for i in range(E):
+        want[flat == i] = rows[flat == i].double() @ w2[i].double().T.contiguous()
+        bound[flat == i] = rows[flat == i].double().abs() @ w2[i].double().abs().T.contiguous() * (Kd + 4) * 2.0 ** -24
+    tw = torch.rand((M, topk), generator=g).cuda()
+    for most_parts in {1, min(4, Kd // 64)}:
+        parts = torch.full((most_parts, numel, N), float("nan"), device="cuda")
+        splits = torch.zeros(1, dtype=torch.int32, device="cuda")
+        K.moe_rows_gemm(x, w2, parts, s, e, post, topk, numel, most, splits=splits)
+        n = int(splits)
+        assert 1 <= n <= most_parts
+        assert bool(((parts[:n].double().sum(0) - want).abs() <= bound).all())
+        out = torch.empty((M, N), dtype=BF, device="cuda")
+        K.moe_sum_parts(parts, splits, tw, out, 0.5)
+        total = parts[0].clone()
+        for i in range(1, n):
+            total += parts[i]
+        acc = torch.zeros((M, N), device="cuda")
+        for k in range(topk):
+            acc += total.to(BF).float().view(M, topk, N)[:, k] * tw[:, k:k + 1]
+        assert torch.equal(out, (acc * 0.5).to(BF))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("override", [(240, 4), (320, 2)])
+def test_the_layer_agrees_with_the_other_tiles(monkeypatch, override):
+    """Same products, other order of their fp32 sums: bf16 results differ by an ulp where one of three roundings falls the other way."""
+    g = torch.Generator().manual_seed(3)
+    M, E, N, H = 500, 8, 768, 1024
+    x = torch.randn((M, H), generator=g).to(BF).cuda()
+    w13, w2 = (torch.randn((E, 2 * N, H), generator=g) * 0.03).to(BF).cuda(), (torch.randn((E, H, N), generator=g) * 0.03).to(BF).cuda()
+    tw, ids = torch.randn((M, E), generator=g).softmax(-1).topk(2)
+    tw, ids = tw.float().contiguous().cuda(), ids.int().contiguous().cuda()
+    monkeypatch.setattr(K, "MOE_TILE_OVERRIDE", (128, 128, 128))
+    base = K.fused_experts(x, w13, w2, tw, ids).float()
+    monkeypatch.setattr(K, "MOE_PARTS_OVERRIDE", override)
+    d = (K.fused_experts(x, w13, w2, tw, ids).float() - base).abs()
+    assert float((d > 2.0 ** -7 * base.abs() + 1e-3).float().mean()) < 1e-3
