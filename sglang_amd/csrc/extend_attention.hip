@@ -1095,7 +1095,9 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
   const bool causal = p.causal != 0;
   int r_tok, r_hg;
   auto row_of = [&](int x) __attribute__((always_inline)) {
-    const int r_row = (x >> 6) * 32 + (x & 31);
+    // (PARTS: of two workgroups on a compute unit, the launch's w and w + 256, one takes its rows from the last wave on, so that waves without rows stand on
+    // different SIMDs)
+    const int r_row = ((x >> 6) ^ (PARTS && DMA ? (blockIdx.x >> 8 & 1) * (NWV - 1) : 0)) * 32 + (x & 31);
     int group = p.group;
     if constexpr (STAYS || PARTS) asm volatile("" : "+s"(group));
     r_tok = r_row / group;
@@ -1488,6 +1490,54 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
   }
   __syncthreads();
 
+  // request j of step t (of 3 LOADS)
+  auto request_of = [&](int t, int j) __attribute__((always_inline)) {
+    if constexpr (DMA) {                            // ids of tile t + 3, V(t + 1), K(t + 2): landed in front of the barrier
+      if (j < LOADS) {
+        const int last = kv_end - 1, tok = (t + 3) * kKvTile + st_r + ROWS_PER_PASS * j;
+        idx_n[j] = idx_base[tok > last ? last : tok];
+      } else if (j < 2 * LOADS) {
+        send(v_rows, idx_v[j - LOADS], sm.v[(t + 1) & 1], j - LOADS);
+      } else {
+        send(k_rows, idx_k[j - 2 * LOADS], sm.k[t & 1], j - 2 * LOADS);
+      }
+    } else if (j < LOADS) {
+      vst[j] = ld_stage(v_rows + static_cast<uint64_t>(static_cast<uint32_t>(idx_v[j])) * row_stride());
+    } else if (j < 2 * LOADS) {
+      if (j == LOADS) {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) idx_v[i] = idx_k[i];          // the ids of K(t + 3) are those of V(t + 3) a step on
+      }
+      kst[j - LOADS] = ld_stage(k_rows + static_cast<uint64_t>(static_cast<uint32_t>(idx_k[j - LOADS])) * row_stride());
+    } else {
+      const int last = kv_end - 1;
+      const int tok = (t + 4) * kKvTile + st_r + ROWS_PER_PASS * (j - 2 * LOADS);
+      idx_k[j - 2 * LOADS] = idx_base[tok > last ? last : tok];
+    }
+  };
+
+  // A wave without rows (behind the last token of a request's last tile; 44 tokens of one query head leave two of four) asks for its rows of the tiles and
+  // leaves its SIMD to the other workgroup's.  us, all waves walking / this: 30 x 44 behind one prefix of 833, 32 / 32 heads, 66.9 / 64.3; where the rows of the keys
+  // bound (16 x 40 behind 1500 each) equal.  (Not for e4m3 rows: 109 registers spilled, 74 behind 5452 39 / 42.)
+  if constexpr (PARTS && DMA) {
+    if (__ballot(row_ok) == 0ull) {                  // (wave-uniform)
+      for (int t = 0; t + 1 < n_tiles; ++t) {
+#pragma unroll
+        for (int j = 0; j < 3 * LOADS; ++j) request_of(t, j);
+        rows_landed();
+        held_ids(idx_n);
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+          idx_v[i] = idx_k[i];
+          idx_k[i] = idx_n[i];
+        }
+        __syncthreads();
+      }
+      __syncthreads();
+      return;
+    }
+  }
+
   auto step = [&](int t, f32x16_t (&sc)[2], f32x16_t (&sn)[2], auto have_next_tag) __attribute__((always_inline)) {
     constexpr bool HAVE_NEXT = decltype(have_next_tag)::value;
     // ---- what was asked for a step ago goes to LDS: K(t + 2), V(t + 1) -- images nobody reads before the barrier below.
@@ -1515,30 +1565,7 @@ __device__ __forceinline__ void extend_pipe_body(const ExtendParams& p, SmemLadd
       constexpr int NREQ = 3 * LOADS;
       constexpr int RSTRIDE = G1 / NREQ > 0 ? G1 / NREQ : 1;
       static_assert(NREQ * RSTRIDE <= G1, "requests fit the products of phase 1");
-      auto request = [&](int j) __attribute__((always_inline)) {
-        if constexpr (DMA) {                            // ids of tile t + 3, V(t + 1), K(t + 2): landed in front of the barrier
-          if (j < LOADS) {
-            const int last = kv_end - 1, tok = (t + 3) * kKvTile + st_r + ROWS_PER_PASS * j;
-            idx_n[j] = idx_base[tok > last ? last : tok];
-          } else if (j < 2 * LOADS) {
-            send(v_rows, idx_v[j - LOADS], sm.v[(t + 1) & 1], j - LOADS);
-          } else {
-            send(k_rows, idx_k[j - 2 * LOADS], sm.k[t & 1], j - 2 * LOADS);
-          }
-        } else if (j < LOADS) {
-          vst[j] = ld_stage(v_rows + static_cast<uint64_t>(static_cast<uint32_t>(idx_v[j])) * row_stride());
-        } else if (j < 2 * LOADS) {
-          if (j == LOADS) {
-#pragma unroll
-            for (int i = 0; i < LOADS; ++i) idx_v[i] = idx_k[i];          // the ids of K(t + 3) are those of V(t + 3) a step on
-          }
-          kst[j - LOADS] = ld_stage(k_rows + static_cast<uint64_t>(static_cast<uint32_t>(idx_k[j - LOADS])) * row_stride());
-        } else {
-          const int last = kv_end - 1;
-          const int tok = (t + 4) * kKvTile + st_r + ROWS_PER_PASS * (j - 2 * LOADS);
-          idx_k[j - 2 * LOADS] = idx_base[tok > last ? last : tok];
-        }
-      };
+      auto request = [&](int j) __attribute__((always_inline)) { request_of(t, j); };
       // the exponentials as a three-stage software pipeline:  A(i) scale + subtract,  B(i) exp2,  C(i) sum + pack
       float ta[SPP], eb[SPP];
       auto stage_a = [&](int i) __attribute__((always_inline)) {
