@@ -74,6 +74,9 @@ struct TiledParams {
 __device__ __forceinline__ void dma16(const uint16_t* src, lds_ptr_t dst) {
   __builtin_amdgcn_global_load_lds((glb_ptr_t)(src), dst, 16, 0, 0);
 }
+__device__ __forceinline__ void dma16_once(const uint16_t* src, lds_ptr_t dst) {      // nt: not kept in the caches
+  __builtin_amdgcn_global_load_lds((glb_ptr_t)(src), dst, 16, 0, 2);
+}
 template <int OFF>
 __device__ __forceinline__ u32x4_t lds_rd(uint32_t addr) {
   u32x4_t v;
@@ -532,6 +535,7 @@ __device__ __forceinline__ u32x4_t lds_quad(uint32_t addr) {
 // arrive.  Where a tile has 240 rows or fewer, LDS holds three stages of weights: they are asked for two steps ahead, and the token rows, which L2 has, one (two
 // ahead as well, 160 rows a tile: no faster).  And all workgroups at one place of K read rows 8 KiB apart, which few memory channels hold: an XCD's workgroups begin
 // an eighth of K behind those of the XCD in front (a place for each column tile: token rows then miss L2, 1000 tokens 860 -> 888).
+// Weights that one tile alone reads stay out of the caches (nt): 200 tokens 541 -> 502, 441 587 -> 548, 800 783 -> 766; for all tiles 1000 851 -> 867.
 // PARTS: the down projection of few rows has fewer tiles than there are compute units (8 experts, 16 column tiles of 4096: 128) and the longest K.  K is cut into
 // up to max_splits parts, as many as make the rounds of parts shortest, by the same estimate as the tiles; their sums are left in fp32, and moe_sum_parts
 // adds them, rounds and weighs as the epilogue here would have.

@@ -1343,18 +1343,19 @@ MOE_PARTS_OVERRIDE = None               # tests / benchmarks: (most rows of a ti
 
 def moe_weight_bound(numel: int, num_experts: int, n_up: int, n_down: int):
     """(most rows of a tile, most parts of K of the down projection) where moe_rows_gemm takes both products of fused_experts; (320, 0): it doesn't.
-    Tiles of 240 rows from 50 or 56 rows an expert on, where weights no longer stream for one block of rows, to 330, where products bound both forms; in front of
-    320-row tiles without parts, 128-row tiles and streams.  us, those / these: 8 experts of 14336 / 4096 with 40 rows 590 / 530, 50 640 / 541, 64 587 / 539, 90 709 / 543, 130 820 / 598,
-    180 860 / 673, 240 923 / 823, 300 1063 / 967, 440 1231 / 1281; of 7168 / 4096 with 50 269 / 280, 64 315 / 285, 130 414 / 313, 240 566 / 451, 300 557 / 530, 360 579 / 596;
-    of 3584 / 4096 (224 column tiles of the up projection, the line) with 64 169 / 159, 130 217 / 191, 300 351 / 288; 64 of 1408 / 2048 with 50 280 / 250, 130 367 / 317, 300 534 /
-    491; 32 of 7168 / 4096 with 50 1114 / 1007, 130 1437 / 1184, 240 1664 / 1633, 300 1919 / 1967 (past 1024 column tiles 256 rows are the line); 128 of 768 / 2048 with 50 330 / 309, 240
-    605 / 539; 16 of 2048 / 2048 with 64 113 / 113, 130 149 / 139, 180 156 / 158, 300 221 / 195; 4 of 1024 / 1024 (32) with 130 45 / 49.
+    Tiles of 240 rows from 40 rows an expert on (below, the weight streams are quicker wherever no expert has more rows than their block: 33 rows 474 / 484) to 330, where products bound
+    both forms.  us, streams, 128-row tiles or 320-row tiles without parts / these, routings of uneven experts: 8 experts of 14336 / 4096 with 16 rows 443 / 478, 24 570 / 488, 32 594 / 492, 40 488 / 485, 64 586 /
+    502, 90 601 / 505, 130 832 / 561, 180 910 / 674, 240 955 / 830, 300 1006 / 977, 440 1261 / 1348; of 7168 / 4096 with 24 236 / 253, 32 249 / 254, 64 314 / 261, 130 397 / 294, 300 578 / 532, 360 599
+    / 600; of 3584 / 4096 (224 column tiles of the up projection, the line) with 24 124 / 129, 32 148 / 133, 130 219 / 173, 360 380 / 306, 440 423 / 418; 64 of 1408 / 2048 with 16 208 / 213, 32 234 /
+    224, 130 364 / 305, 360 606 / 560; 32 of 7168 / 4096 with 32 975 / 895, 130 1439 / 1215, 240 1716 / 1653, 300 1893 / 1926 (past 1024 column tiles 256 rows are the line); 128 of 768 / 2048 with
+    32 276 / 261, 240 605 / 536; 16 of 2048 / 2048 with 32 116 / 92, 130 154 / 138, 180 155 / 161, 300 227 / 192; 4 of 1024 / 1024 (32) with 130 46 / 51.
     Tiles of 320 rows with the down projection in two parts from 480 rows on while that has up to two rounds of tiles and a long K: 8 of 14336 / 4096 with 440 1240 / 1231,
     with 560 1651 / 1561, 750 1986 / 1942, 1000 2440 / 2386; of 7168 / 4096 with 750 1014 / 993, with 1000 1272 / 1297.
     No more parts than give four rounds of tiles: another part is another fp32 copy of the rows."""
     rows, col_tiles, down = numel / max(1, num_experts), num_experts * -(-n_up // 128), num_experts * -(-n_down // 256)
     blocks = (numel + (num_experts + 1) * 255 + 255) // 256      # moe_align_block_size's
-    if blocks <= 256 and col_tiles >= 224 and (50 if col_tiles >= 640 else 56) <= rows <= (330 if col_tiles <= 1024 else 256):
+    most = 256 if col_tiles > 1024 else 330 if n_up * n_down > 1 << 24 else 400
+    if blocks <= 256 and col_tiles >= 224 and 40 <= rows <= most:
         return 240, max(1, min(4, 1024 // (down * -(-int(rows) // 240))))
     if rows >= 480 and n_up >= 8192 and col_tiles >= 640 and down * -(-int(rows) // 320) <= 512:
         return 320, 2

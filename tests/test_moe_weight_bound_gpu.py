@@ -9,8 +9,8 @@ BF = torch.bfloat16
 
 
 def test_where_these_tiles_are_taken():
-    for rows, experts, up, down, most in ((49, 8, 14336, 4096, 320), (50, 8, 14336, 4096, 240), (55, 8, 7168, 4096, 320), (56, 8, 7168, 4096, 240), (330, 8, 14336, 4096, 240),
-                                          (331, 8, 14336, 4096, 320), (256, 32, 7168, 4096, 240), (257, 32, 7168, 4096, 320), (130, 4, 1024, 1024, 320),
+    for rows, experts, up, down, most in ((39, 8, 14336, 4096, 320), (40, 8, 14336, 4096, 240), (39, 8, 7168, 4096, 320), (40, 8, 7168, 4096, 240), (330, 8, 14336, 4096, 240),
+                                          (331, 8, 14336, 4096, 320), (256, 32, 7168, 4096, 240), (257, 32, 7168, 4096, 320), (130, 4, 1024, 1024, 320), (400, 32, 2048, 2048, 240),
                                           (254, 128, 768, 2048, 240), (258, 128, 768, 2048, 320)):
         assert K.moe_weight_bound(rows * experts, experts, up, down)[0] == most, (rows, experts)
     assert K.moe_weight_bound(8 * 130, 8, 14336, 4096) == (240, 4) and K.moe_weight_bound(64 * 130, 64, 1408, 2048) == (240, 2)
