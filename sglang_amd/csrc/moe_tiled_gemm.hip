@@ -534,7 +534,8 @@ __device__ __forceinline__ u32x4_t lds_quad(uint32_t addr) {
 // FEW units: with one tile an expert every weight comes from behind L2, and a step of 320-row tiles is then 4.8 k clocks, the time that its weights take to
 // arrive.  Where a tile has 240 rows or fewer, LDS holds three stages of weights: they are asked for two steps ahead, and the token rows, which L2 has, one (two
 // ahead as well, 160 rows a tile: no faster).  And all workgroups at one place of K read rows 8 KiB apart, which few memory channels hold: an XCD's workgroups begin
-// an eighth of K behind those of the XCD in front (a place for each column tile: token rows then miss L2, 1000 tokens 860 -> 888).
+// an eighth of K behind those of the XCD in front (a place for each column tile: token rows then miss L2, 1000 tokens 860 -> 888;
+// with 320-row tiles an eighth takes 1 %: 1700 tokens 1220 -> 1209, 3000 1924 -> 1902).
 // Weights that one tile alone reads stay out of the caches (nt): 200 tokens 541 -> 502, 441 587 -> 548, 800 783 -> 766; for all tiles 1000 851 -> 867.
 // PARTS: the down projection of few rows has fewer tiles than there are compute units (8 experts, 16 column tiles of 4096: 128) and the longest K.  K is cut into
 // up to max_splits parts, as many as make the rounds of parts shortest, by the same estimate as the tiles; their sums are left in fp32, and moe_sum_parts
@@ -543,11 +544,12 @@ __device__ __forceinline__ u32x4_t lds_quad(uint32_t addr) {
 // 800 895 / 772 / 742 / 780 (other rows an expert), 1000 947 / 880 / 862 / 860.  The weights alone are 428 us.
 __global__ __launch_bounds__(kThreads2, 1) void moe_rows_kernel(TiledParams p) {
   constexpr int UNITS = kWholeUnits;
-  constexpr bool PARTS = false;
+  constexpr bool PARTS = false, TURN = false;          // (its sums are those of the 128-row tiles, bit by bit)
 #include "moe_rows_body.inc"
 }
 template <int UNITS, bool PARTS>
 __global__ __launch_bounds__(kThreads2, 1) void moe_weight_bound_kernel(TiledParams p) {
+  constexpr bool TURN = true;
 #include "moe_rows_body.inc"
 }
 
@@ -661,7 +663,7 @@ int sgl_amd_moe_rows_gemm(const void* a, const void* w, void* c, const int32_t* 
     else hipLaunchKernelGGL((moe_weight_bound_kernel<kFewUnits, false>), grid, block, 0, as_stream(stream), p);
   } else {
     if (max_splits) hipLaunchKernelGGL((moe_weight_bound_kernel<kWholeUnits, true>), grid, block, 0, as_stream(stream), p);
-    else hipLaunchKernelGGL(moe_rows_kernel, grid, block, 0, as_stream(stream), p);
+    else hipLaunchKernelGGL((moe_weight_bound_kernel<kWholeUnits, false>), grid, block, 0, as_stream(stream), p);
   }
   SGL_CHECK_LAUNCH("moe_rows_gemm");
   return 0;
