@@ -1454,12 +1454,14 @@ def moe_sum_reduce(x: torch.Tensor, out: torch.Tensor, routed_scaling_factor: fl
 
 
 def choose_moe_block_m(num_pairs: int, num_experts: int) -> int:
-    """Row-block height of the grouped GEMM: the smallest of 16/32/48/64 that holds 1.5x an average expert's
-    rows -- an expert whose rows spill into a second block streams its weights twice, padded rows cost nothing
-    (the kernel is bound by the weight stream)."""
+    """Row-block height of the grouped GEMM: an expert whose rows spill into a second block streams its weights twice, padded rows cost next to nothing
+    (the kernel is bound by the weight stream): 16 rows for up to 6 an expert, 32 for up to 16, 48 for up to 32.  us, means of eight routings of uneven experts, the next
+    smaller block / this: 7 rows an expert on average, 8 experts of 14336 / 4096 420 / 418, of 7168 / 4096 226 / 221, 128 of 768 / 2048 220 / 209, 64 of 1408 / 2048 190 / 188; 10 rows 461 / 421, 230 / 222, 234 /
+    218, 205 / 193; 17 rows 438 / 439, 229 / 229, 243 / 236, 211 / 206; 21 rows 457 / 446, 247 / 232, 252 / 245, 227 / 213; one routing at worst 0.984 and at best 1.22 of the time.  Even
+    experts: at most 1.5 % more."""
     avg = (num_pairs + num_experts - 1) // max(1, num_experts)
-    for bm in (16, 32, 48):
-        if avg + avg // 2 <= bm:
+    for most, bm in ((6, 16), (16, 32), (32, 48)):
+        if avg <= most:
             return bm
     return 64
 
