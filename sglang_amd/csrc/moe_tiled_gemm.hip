@@ -540,8 +540,8 @@ __device__ __forceinline__ u32x4_t lds_quad(uint32_t addr) {
 // PARTS: the down projection of few rows has fewer tiles than there are compute units (8 experts, 16 column tiles of 4096: 128) and the longest K.  K is cut into
 // up to max_splits parts, as many as make the rounds of parts shortest, by the same estimate as the tiles; their sums are left in fp32, and moe_sum_parts
 // adds them, rounds and weighs as the epilogue here would have.
-// us, both products of 8 experts of 14336 / 4096, 128-row tiles or 320 / PARTS with 320 / three stages / and the turn: 441 tokens 734 / 692 / 621 / 567, 640 873 / 739 / 657 / 656,
-// 800 895 / 772 / 742 / 780 (other rows an expert), 1000 947 / 880 / 862 / 860.  The weights alone are 428 us.
+// us, both products of 8 experts of 14336 / 4096, 128-row tiles or 320 / PARTS with 320 / three stages / and the turn / and nt: 441 tokens 734 / 692 / 621 / 567 / 560,
+// 640 873 / 739 / 657 / 656 / 634, 1000 947 / 880 / 862 / 860 / 860.  The weights alone are 428 us.
 __global__ __launch_bounds__(kThreads2, 1) void moe_rows_kernel(TiledParams p) {
   constexpr int UNITS = kWholeUnits;
   constexpr bool PARTS = false, TURN = false;          // (its sums are those of the 128-row tiles, bit by bit)
