@@ -1351,12 +1351,12 @@ def moe_weight_bound(numel: int, num_experts: int, n_up: int, n_down: int):
     32 276 / 261, 240 605 / 536; 16 of 2048 / 2048 with 32 116 / 92, 130 154 / 138, 180 155 / 161, 300 227 / 192; 4 of 1024 / 1024 (32) with 130 46 / 51.
     Tiles of 320 rows with the down projection in two parts from 480 rows on while that has up to two rounds of tiles and a long K: 8 of 14336 / 4096 with 440 1240 / 1231,
     with 560 1651 / 1561, 750 1986 / 1942, 1000 2440 / 2386; of 7168 / 4096 with 750 1014 / 993, with 1000 1272 / 1297.
-    No more parts than give four rounds of tiles: another part is another fp32 copy of the rows."""
+    No more parts than give four rounds of tiles: another part is another fp32 copy of the rows; nor than the down projection's K has steps of 64."""
     rows, col_tiles, down = numel / max(1, num_experts), num_experts * -(-n_up // 128), num_experts * -(-n_down // 256)
     blocks = (numel + (num_experts + 1) * 255 + 255) // 256      # moe_align_block_size's
     most = 256 if col_tiles > 1024 else 330 if n_up * n_down > 1 << 24 else 400
     if blocks <= 256 and col_tiles >= 224 and 40 <= rows <= most:
-        return 240, max(1, min(4, 1024 // (down * -(-int(rows) // 240))))
+        return 240, max(1, min(4, n_up // 64, 1024 // (down * -(-int(rows) // 240))))
     if rows >= 480 and n_up >= 8192 and col_tiles >= 640 and down * -(-int(rows) // 320) <= 512:
         return 320, 2
     return 320, 0

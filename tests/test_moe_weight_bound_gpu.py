@@ -19,6 +19,38 @@ def test_where_these_tiles_are_taken():
         assert K.moe_weight_bound(pairs, experts, up, down) == (320, 0)
 
 
+def test_no_more_parts_than_steps():
+    """A part of K has a step of 64 at least (sgl_amd_moe_rows_gemm refuses others): intermediate sizes of few steps over all that the rule takes."""
+    taken = 0
+    for experts in (64, 112, 128, 160, 192, 220):
+        for up in (64, 128, 192, 256, 320):
+            for down in (64, 256, 512, 1024, 2048):
+                for rows in (40, 56, 90, 130, 250):
+                    most, parts = K.moe_weight_bound(rows * experts, experts, up, down)
+                    taken += parts > 0
+                    assert parts <= up // 64, (experts, up, down, rows)
+    assert taken > 20
+
+
+@pytest.mark.gpu
+def test_a_layer_of_three_steps():
+    """128 experts of 192 / 512 with 56 rows: four parts would suit its tiles, its K has three steps."""
+    g = torch.Generator().manual_seed(11)
+    M, E, N, H, top = 896, 128, 192, 512, 8
+    x = torch.randn((M, H), generator=g).to(BF).cuda()
+    w13, w2 = (torch.randn((E, 2 * N, H), generator=g) * 0.05).to(BF).cuda(), (torch.randn((E, H, N), generator=g) * 0.05).to(BF).cuda()
+    tw, ids = torch.randn((M, E), generator=g).softmax(-1).topk(top)
+    tw, ids = tw.float().contiguous().cuda(), ids.int().contiguous().cuda()
+    assert K.moe_weight_bound(M * top, E, N, H)[1] > 0
+    got, want = K.fused_experts(x, w13, w2, tw, ids), torch.zeros((M, H), dtype=torch.float64, device="cuda")
+    for i in range(E):
+        tok, k = (ids == i).nonzero(as_tuple=True)
+        gu = x[tok].double() @ w13[i].double().T.contiguous()
+        want.index_add_(0, tok, (torch.nn.functional.silu(gu[:, :N]) * gu[:, N:]) @ w2[i].double().T.contiguous() * tw[tok, k].double()[:, None])
+    # bf16 roundings of gate and activation, of their product, of a pair's row and of the result, 2^-9 each
+    assert float((got.double() - want).norm() / want.norm()) < 5 * 2.0 ** -9
+
+
 def _pairs(loads, topk, g):
     """Pairs of every expert in no order, `topk` a token."""
     ids = torch.repeat_interleave(torch.arange(len(loads)), torch.tensor(loads))
