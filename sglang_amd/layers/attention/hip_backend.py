@@ -451,10 +451,11 @@ class HipAttnBackend(AttentionBackend):
 
     def _new_slots(self, forward_batch, tokens: int):
         """The slots of a pass's `tokens` rows where the attention's call can store them, else None: this package's pool with its own set_kv_buffer."""
-        pool, loc = self.token_to_kv_pool, forward_batch.out_cache_loc
-        if type(pool).set_kv_buffer is not MHATokenToKVPool.set_kv_buffer or "set_kv_buffer" in vars(pool):
+        # (a step whose rows are in the pool already needs neither slots on the device nor a pool that takes rows)
+        pool, loc = self.token_to_kv_pool, getattr(forward_batch, "out_cache_loc", None)
+        if getattr(type(pool), "set_kv_buffer", None) is not MHATokenToKVPool.set_kv_buffer or "set_kv_buffer" in vars(pool):
             return None
-        return loc if isinstance(loc, torch.Tensor) and loc.dtype == torch.int64 and loc.shape == (tokens,) and loc.is_contiguous() else None
+        return loc if isinstance(loc, torch.Tensor) and loc.is_cuda and loc.dtype == torch.int64 and loc.shape == (tokens,) and loc.is_contiguous() else None
 
     def forward_decode(self, q, k, v, layer, forward_batch, save_kv_cache: bool = True, **kwargs):
         self._refuse_unsupported(layer, kwargs)

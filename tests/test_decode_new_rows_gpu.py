@@ -135,6 +135,40 @@ def test_replays_with_other_slots(device):
         assert torch.equal(out, want) and torch.equal(kc, k1) and torch.equal(vc, v1), (n, meet)
 
 
+def _planned_slots(monkeypatch, pool, fb, **attrs):
+    """new_loc of the plan that a decode step of `fb` makes over `pool`."""
+    from types import SimpleNamespace
+
+    from sglang_amd.layers.attention import hip_backend as H
+
+    b, got = H.HipAttnBackend.__new__(H.HipAttnBackend), []
+    vars(b).update(token_to_kv_pool=pool, req_to_token_pool=SimpleNamespace(req_to_token=None), num_q_heads=8, num_kv_heads=2, _seq_src=None,
+                   forward_metadata=H._Meta(torch.ones(3, dtype=torch.int32), cascade=object()), **attrs)
+    monkeypatch.setattr(H.kernels, "cascade_plan", lambda *a, new_loc=None, **k: got.append(new_loc))
+    b.init_forward_metadata_in_graph(fb)
+    assert b.forward_metadata.slots_planned == (got[0] is not None)
+    return got[0]
+
+
+@pytest.mark.parametrize("what", ["no_slots", "slots_none", "slots_on_the_host", "pool_takes_no_rows"])
+def test_steps_whose_rows_are_in_the_pool_need_no_slots(monkeypatch, what):
+    """A model that stores its rows itself plans a step whatever its batch says of slots, over pools that take no rows."""
+    from types import SimpleNamespace
+
+    from sglang_amd.mem_cache.memory_pool import MHATokenToKVPool
+    from sglang_amd.model_executor.forward_batch_info import ForwardMode
+
+    fb = SimpleNamespace(forward_mode=ForwardMode.DECODE, req_pool_indices=torch.zeros(3, dtype=torch.int64), out_cache_loc=torch.zeros(3, dtype=torch.int64))
+    pool = MHATokenToKVPool.__new__(MHATokenToKVPool)
+    if what == "no_slots":
+        del fb.out_cache_loc
+    elif what == "slots_none":
+        fb.out_cache_loc = None
+    elif what == "pool_takes_no_rows":
+        pool = SimpleNamespace()
+    assert _planned_slots(monkeypatch, pool, fb) is None
+
+
 @pytest.mark.skipif(not Path(HIPCC).exists(), reason="hipcc not installed")
 def test_registers(tmp_path):
     usage = _resource_usage("cascade_attention.hip", tmp_path)
