@@ -1483,7 +1483,8 @@ def fused_experts(hidden_states: torch.Tensor, w13: torch.Tensor, w2: torch.Tens
     if M == 0:
         return out
     most, parts = MOE_PARTS_OVERRIDE or ((320, 0) if MOE_TILE_OVERRIDE is not None else moe_weight_bound(numel, E, N, K))
-    if (parts > 0 and K % 64 == 0 and N % 64 == 0
+    # (ids, weights or an output of more rows than there are tokens, and strides that moe_sum_reduce refuses, are left to the forms below)
+    if (parts > 0 and K % 64 == 0 and N % 64 == 0 and topk_ids.shape[0] == M and topk_weights.numel() == numel and out.shape == (M, K) and out.stride(0) % 8 == 0
             and _offsets_fit((N2, w13.stride(1)), (K, w2.stride(1)), (M, hidden_states.stride(0)), (numel, N))):
         # an expert's weights take longer than its products: read once for all of its rows
         sorted_ids, expert_ids, post = moe_align_block_size(topk_ids, 256, E)

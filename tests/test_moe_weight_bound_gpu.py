@@ -105,6 +105,33 @@ def test_products_of_few_rows(most, loads, N, Kd):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("form", ["rows_of_out", "columns_of_out", "rows_of_ids", "stride_of_out"])
+def test_what_the_other_tiles_take_or_refuse(form):
+    """Outputs, ids and weights with more rows than there are tokens, as padded buffers have, and an output whose rows are not 16 bytes apart."""
+    g = torch.Generator().manual_seed(12)
+    M, E, N, H, top = 250, 8, 3584, 256, 2
+    x = torch.randn((M, H), generator=g).to(BF).cuda()
+    w13, w2 = (torch.randn((E, 2 * N, H), generator=g) * 0.05).to(BF).cuda(), (torch.randn((E, H, N), generator=g) * 0.05).to(BF).cuda()
+    tw, ids = torch.randn((M + 9, E), generator=g).softmax(-1).topk(top)
+    tw, ids = tw.float().contiguous().cuda(), ids.int().contiguous().cuda()
+    assert K.moe_weight_bound(M * top, E, N, H)[1] > 0
+    want = K.fused_experts(x, w13, w2, tw[:M].contiguous(), ids[:M].contiguous()).float()
+    if form == "stride_of_out":
+        with pytest.raises(RuntimeError, match="multiples of 8"):
+            K.fused_experts(x, w13, w2, tw[:M].contiguous(), ids[:M].contiguous(), out=torch.empty((M, H + 4), dtype=BF, device="cuda")[:, :H])
+        return
+    if form == "rows_of_ids":
+        got = K.fused_experts(x, w13, w2, tw, ids)
+    else:
+        out = torch.full((M + (5 if form == "rows_of_out" else 0), H + (8 if form == "columns_of_out" else 0)), 7.0, dtype=BF, device="cuda")
+        got = K.fused_experts(x, w13, w2, tw[:M].contiguous(), ids[:M].contiguous(), out=out)
+        assert got is out and bool((out[M:] == 7).all()) and bool((out[:, H:] == 7).all())
+        got = got[:M, :H]
+    d = (got.float() - want).abs()                     # (other tiles: an ulp where one of three roundings falls the other way)
+    assert float((d > 2.0 ** -7 * want.abs() + 1e-3).float().mean()) < 1e-3
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("override", [(240, 4), (320, 2)])
 def test_the_layer_agrees_with_the_other_tiles(monkeypatch, override):
     """Same products, other order of their fp32 sums: bf16 results differ by an ulp where one of three roundings falls the other way."""
