@@ -384,7 +384,15 @@ class CausalLM(nn.Module):
                                 self.config.num_hidden_layers, device, use_hnd=use_hnd)
 
     def create_attn_backend(self, runner):
-        return HipAttnBackend(runner)
+        return HipAttnBackend(runner, self.brings_rows)
+
+    def brings_rows(self, pool, rows: int) -> bool:
+        """Whether LlamaAttention hands the rows of a decode step to the backend: bf16 rows in token order, and all that the weight-streaming projection writes, are in the
+        pool before."""
+        if not getattr(pool, "is_fp8", False) and not getattr(pool, "use_hnd", False):
+            return False
+        attn = self.layers[0].self_attn
+        return OPERATOR_SURFACE_ONLY or not attn.rotary_emb.is_neox_style or not kernels.wstream_preferred(rows, *attn.qkv_proj.weight.shape)
 
     def forward_hidden(self, input_ids: torch.Tensor, positions: torch.Tensor, forward_batch) -> torch.Tensor:
         embeds = getattr(forward_batch, "input_embeds", None)

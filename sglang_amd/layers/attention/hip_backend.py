@@ -132,7 +132,11 @@ class HipAttnBackend(AttentionBackend):
     # qo_indptr / lens are sized per forward, never preallocated at (req pool + 1) (base_attn_backend.py:117-122)
     extend_dummy_seqs_capped_by_req_pool = False
 
-    def __init__(self, model_runner):
+    _brings_rows = None
+
+    def __init__(self, model_runner, brings_rows=None):
+        """brings_rows(pool, rows): whether the layers of a decode step of `rows` requests hand their new rows to forward_decode to be stored (None: they may)."""
+        self._brings_rows = brings_rows
         """Reads what the reference backends read of a ModelRunner (triton_backend.py:145-206,
         torch_native_backend.py:20-33): `device`, `req_to_token_pool`, `token_to_kv_pool`, and for the head
         counts `model_config` + the attention TP size -- or the harness runner's per-rank fields."""
@@ -328,8 +332,11 @@ class HipAttnBackend(AttentionBackend):
         if m is not None and self._seq_src is not None and forward_batch.forward_mode.is_decode():
             m.seq_lens_i32.copy_(forward_batch.seq_lens)         # int64 -> int32, recorded into the graph
         if m is not None and m.cascade is not None and forward_batch.forward_mode.is_decode():
-            # (the layers may then store the step's rows in the attention's launch)
-            loc = self._new_slots(forward_batch, m.seq_lens_i32.numel())
+            # (the layers may then store the step's rows in the attention's launch: not where they bring none, and over head-major pages by a launch all the same)
+            rows, pool = m.seq_lens_i32.numel(), self.token_to_kv_pool
+            loc = self._new_slots(forward_batch, rows)
+            if loc is not None and (pool_kernel_format(pool)["hnd"] or not (self._brings_rows is None or self._brings_rows(pool, rows))):
+                loc = None
             m.slots_planned = loc is not None
             kernels.cascade_plan(m.cascade, self.req_to_token_pool.req_to_token, self._pool_idx(forward_batch),
                                  m.seq_lens_i32, self.num_q_heads, self.num_kv_heads, new_loc=loc)

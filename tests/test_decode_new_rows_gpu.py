@@ -169,6 +169,29 @@ def test_steps_whose_rows_are_in_the_pool_need_no_slots(monkeypatch, what):
     assert _planned_slots(monkeypatch, pool, fb) is None
 
 
+@pytest.mark.parametrize("fp8,hnd,page,streams,looks", [(False, False, 1, True, False), (False, False, 1, False, False), (True, False, 1, True, False), (True, False, 1, False, True),
+                                                        (False, True, 16, False, False), (True, True, 16, False, False)])
+def test_the_plan_looks_only_where_a_layer_stores_with_it(monkeypatch, fp8, hnd, page, streams, looks):
+    """The package's own model stores its rows itself over bf16 pools and where the projection streams; over head-major pages the store keeps its launch."""
+    from types import SimpleNamespace
+
+    from sglang_amd.harness import models
+    from sglang_amd.layers.attention.hip_backend import HipAttnBackend
+    from sglang_amd.mem_cache.memory_pool import MHATokenToKVPool
+    from sglang_amd.model_executor.forward_batch_info import ForwardMode
+
+    pool, loc = MHATokenToKVPool.__new__(MHATokenToKVPool), torch.zeros(3, dtype=torch.int64)
+    vars(pool).update(dtype=FP8 if fp8 else BF, is_fp8=fp8, use_hnd=hnd, page_size=page)
+    monkeypatch.setattr(HipAttnBackend, "_new_slots", lambda *a: loc)
+    monkeypatch.setattr(models.kernels, "wstream_preferred", lambda *a: streams)
+    attn = SimpleNamespace(rotary_emb=SimpleNamespace(is_neox_style=True), qkv_proj=SimpleNamespace(weight=torch.zeros(1, 1)))
+    model = SimpleNamespace(layers=[SimpleNamespace(self_attn=attn)])
+    fb = SimpleNamespace(forward_mode=ForwardMode.DECODE, req_pool_indices=loc)
+    got = _planned_slots(monkeypatch, pool, fb, _brings_rows=lambda *a: models.CausalLM.brings_rows(model, *a))
+    assert (got is loc) == looks
+    assert (_planned_slots(monkeypatch, pool, fb) is loc) == (not hnd)      # a backend that is not told
+
+
 @pytest.mark.skipif(not Path(HIPCC).exists(), reason="hipcc not installed")
 def test_registers(tmp_path):
     usage = _resource_usage("cascade_attention.hip", tmp_path)
