@@ -103,7 +103,7 @@ __device__ __forceinline__ T* global_ptr(T* x) {
 // each row is stored by the one unit of a kv head that reads it as its request's newest token: by every wave of the unit that reads it, before it does (the
 // accesses of a wave to one address complete in order, and what the other waves store is the same).  Nobody else reads the slot, unless a table holds
 // another row's new slot; the plan looks for that once a step (cascade_check_rows), and then every wave stores all rows of its kv head first, the later of two
-// with one slot.
+// with one slot.  The row of a request without tokens, which no unit reads, is stored by the first workgroup of its kv head.
 // us of attention a step, store launch / this: 64 requests behind shared prefixes, 32 / 8 heads, 8 layers, 233 / 219; 37 of 0.9 to 5.1 k in e4m3, 4 layers,
 // 267 / 258; 21 of 180 in e4m3, 64 / 8 heads, 4 layers, 70 / 61.  What is left of the launch: 1 us a layer in units of 128 tokens (with nothing stored 209).
 struct NewRows {
@@ -149,6 +149,18 @@ __device__ __forceinline__ void put_all_rows(const ChunkParams& p, const NewRows
   }
 }
 
+// The rows of the requests without tokens (a call for the whole batch, of one workgroup a kv head, where the plan found any).  As a meeting of slots, which every wave
+// answers by storing all rows, one such request among 64 of 1 k took a layer from 50 to 105 us.
+template <int D, bool FP8>
+__device__ __forceinline__ void put_unread_rows(const ChunkParams& p, const NewRows& rows, const int kvh, const int lane) {
+#pragma clang loop unroll(disable)
+  for (int b0 = 0; b0 < p.batch; b0 += 64) {
+    unsigned long long todo = __ballot(b0 + lane < p.batch && p.seq_lens[b0 + lane < p.batch ? b0 + lane : 0] < 1);
+#pragma clang loop unroll(disable)
+    for (; todo != 0ull; todo &= todo - 1) put_own_row<D, FP8>(p, rows, b0 + __ffsll(static_cast<long long>(todo)) - 1, kvh, lane);
+  }
+}
+
 // Whether all rows have to be stored first: a table holds a new slot elsewhere, or the plan does not know these slots (every wave for itself).
 // The first 64 requests' slots and the words are asked for by ask(), beside what else a kernel begins with: behind it they are a round trip of their own.
 struct RowsMeet {
@@ -161,13 +173,14 @@ struct RowsMeet {
     now = static_cast<int32_t>(rows.loc[first]);
   }
   __device__ __forceinline__ int answer(const ChunkParams& p, const NewRows& rows, const int lane) const {
-    bool meet = (word != 0) | (planned != now);
+    bool meet = (word & kPlanMeet) | (planned != now);
     if (p.batch > 64) {
       const CascadePlanView pv = cascade_plan_view(p.plan, p.batch, p.max_items);
       for (int b = 64 + lane; b < p.batch; b += 64) meet |= pv.new_slots[b] != static_cast<int32_t>(rows.loc[b]);
     }
     return __ballot(meet) != 0ull ? kAllRows : kOwnRow;
   }
+  __device__ __forceinline__ bool unread() const { return __ballot(word & kPlanUnread) != 0ull; }
 };
 
 // The K rows, then (after S^T) the transposed V rows, pass through ONE 16 KiB LDS image; at D = 128 it is filled twice
@@ -442,7 +455,7 @@ __device__ __forceinline__ void cascade_chunk_loop(const ChunkParams& p, const N
   if constexpr (STORE) {
     asm volatile("" : "+v"(meet.word), "+v"(meet.planned), "+v"(meet.now));
     store_rows = __builtin_amdgcn_readfirstlane(meet.answer(p, *new_rows, threadIdx.x & 63));
-    if (n_units == 0 && w0 < p.num_kv_heads) put_all_rows<D, FP8>(p, *new_rows, w0, threadIdx.x & 63);    // nobody reads anything
+    if (meet.unread() && (store_rows == kOwnRow || n_units == 0) && w0 < p.num_kv_heads) put_unread_rows<D, FP8>(p, *new_rows, w0, threadIdx.x & 63);
   }
   // The kernel's one argument sits at the start of the kernarg segment; every pass re-reads it through an address the
   // compiler cannot see through, exactly as a fresh launch would (scalar loads, served by the scalar cache), and takes the
@@ -599,7 +612,7 @@ constexpr int kPlanOneLaunch = 16;
 
 // Whether a request's table holds the slot of a row of this step anywhere but at its own newest token, looked up by workgroups beside the plan's own (one
 // launch; they take less time than it).  The new slots are bits of two hashes in LDS; what both hold is compared with every slot.  Slot 0 is the sink of padded
-// entries, which may share it.  A request without tokens counts as well: no unit would store its row.
+// entries, which may share it.  Requests without tokens, whose row no unit would store, are found by the way.
 __device__ __forceinline__ void cascade_check_rows(const int32_t* req_to_token, int64_t r2t_stride, const int64_t* req_pool_indices, const int32_t* seq_lens,
                                                    const int64_t* new_loc, int batch, int checker, int checkers, uint32_t* bits0, uint32_t* bits1, int* slots,
                                                    const CascadePlanView& pv) {
@@ -607,7 +620,7 @@ __device__ __forceinline__ void cascade_check_rows(const int32_t* req_to_token, 
   for (int i = tid; i < 1024; i += kPlanThreads) bits0[i] = bits1[i] = 0u;
   __syncthreads();
   auto hash = [](uint32_t s) { return (s * 0x9e3779b1u) >> 17; };
-  bool meet = false, seen[kPlanMaxBatch / kPlanThreads];
+  bool meet = false, unread = false, seen[kPlanMaxBatch / kPlanThreads];
 #pragma unroll
   for (int i = 0; i < kPlanMaxBatch / kPlanThreads; ++i) {
     const int b = tid + i * kPlanThreads;
@@ -633,7 +646,7 @@ __device__ __forceinline__ void cascade_check_rows(const int32_t* req_to_token, 
   for (int b = checker; b < batch; b += checkers) {
     const int32_t* row = req_to_token + req_pool_indices[b] * r2t_stride;
     const int len = seq_lens[b], own = slots[b];
-    meet |= len < 1;
+    unread |= len < 1;
     for (int t0 = tid; t0 < len; t0 += kAhead * kPlanThreads) {
       int s[kAhead];
 #pragma unroll
@@ -651,8 +664,8 @@ __device__ __forceinline__ void cascade_check_rows(const int32_t* req_to_token, 
       }
     }
   }
-  if (__syncthreads_or(meet) && tid == 0) pv.meet[checker] = 1;
-  else if (tid == 0) pv.meet[checker] = 0;
+  const int found = (__syncthreads_or(meet) ? kPlanMeet : 0) | (__syncthreads_or(unread) ? kPlanUnread : 0);
+  if (tid == 0) pv.meet[checker] = found;
 }
 
 template <bool ONE>
@@ -818,8 +831,8 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
     pv.header[2] = rows;
     pv.header[3] = n_shared_items;
   }
-  // (no word of a workgroup that looked: 1 where there are none, so that a plan without the slots says what one that found some says)
-  if (tid < kCheckers && tid >= static_cast<int>(gridDim.x) - 1) pv.meet[tid] = gridDim.x == 1 ? 1 : 0;
+  // (no word of a workgroup that looked: both bits where there are none, so that a plan without the slots says what one that found both says)
+  if (tid < kCheckers && tid >= static_cast<int>(gridDim.x) - 1) pv.meet[tid] = gridDim.x == 1 ? kPlanMeet | kPlanUnread : 0;
   // ---- private chunks of every request, appended behind the shared items (block-wide exclusive scan) ----
   int mine = 0, sh = 0, len = 0;
   if (tid < batch) {

@@ -16,7 +16,7 @@
 //                        the items'; they stand in the place of the private items for the looping attention kernel
 //   compare[2 B]         scratch between the plan's two launches: leader of request b, its common prefix with the leader
 //   new_slots[B]         the slots that the plan was told the step's rows go to (if it was)
-//   meet[kCheckers]      whether a request reads one of them that is not its own newest token's, a word a workgroup that looked (it was not told: 1)
+//   meet[kCheckers]      what was found of them, a word of PlanFound bits a workgroup that looked (it was not told: both bits)
 #pragma once
 #include <stdint.h>
 
@@ -54,6 +54,7 @@ constexpr int kSpanUnits = 768;
 constexpr int kOneRoundUnits = 1024;
 constexpr int kMinSpanTiles = 3;
 constexpr int kCheckers = 64;        // workgroups that look through the request tables for the new slots, one word each
+enum PlanFound { kPlanMeet = 1, kPlanUnread = 2 };   // a request reads a new slot that is not its own newest token's, or two rows have one; a request has no tokens
 
 __host__ __device__ inline int64_t cascade_plan_ints(int64_t batch, int64_t max_items) {
   return 8 + batch + batch + (batch + 1) + batch + batch + 8 * max_items + batch + 2 * batch + batch + (kSpanUnits + 1) + 8 * (batch + kSpanUnits) + 3 + batch +

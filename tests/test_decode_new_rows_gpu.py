@@ -89,6 +89,54 @@ def test_the_bits_of_both_calls(device, Hq, Hkv, D, fp8, page, hnd, width, lens,
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("without", ["every_third", "all", "the_last_two_of_one_slot", "one_whose_slot_is_read"])
+@pytest.mark.parametrize("Hq,Hkv,D,fp8,width,B", [(32, 8, 128, 0, 16384, 26), (32, 8, 128, 0, 512, 26), (14, 2, 64, 0, 512, 130), (32, 8, 128, 1, 16384, 70), (16, 4, 64, 1, 512, 5)])
+def test_requests_without_tokens(device, Hq, Hkv, D, fp8, width, B, without):
+    """Their rows are stored though no unit reads them, and the plan says no more of them than that: other rows are then not stored by every wave."""
+    from sglang_amd import kernels
+
+    g = torch.Generator().manual_seed(B + Hq)
+    lens = [EDGES[b % len(EDGES)] + (b > 20) * 200 for b in range(B)]
+    slots = sum(lens) + 1
+    table, at, perm = torch.zeros((B + 1, width), dtype=torch.int32), 0, torch.randperm(slots - 1, generator=g).int() + 1
+    for b, n in enumerate(lens):
+        table[b + 1, :n] = perm[at:at + n]
+        at += n
+    loc = torch.tensor([int(table[b + 1, n - 1]) for b, n in enumerate(lens)])
+    empty = {"every_third": range(0, B, 3), "all": range(B), "the_last_two_of_one_slot": [B - 2, B - 1], "one_whose_slot_is_read": [1]}[without]
+    for b in empty:
+        lens[b] = 0
+    found = 2                                                        # kPlanUnread
+    if without == "the_last_two_of_one_slot":
+        loc[B - 2], found = loc[B - 1], 3                            # and kPlanMeet
+    if without == "one_whose_slot_is_read":
+        table[3, 4], found = loc[1], 3
+    pools = [(torch.randn((slots, Hkv, D), generator=g) * 0.5).to(FP8 if fp8 else BF) for _ in range(2)]
+    pools = [(x.view(torch.uint8) if fp8 else x).to(device) for x in pools]
+    q, k, v = ((torch.randn((B, h, D), generator=g) * 0.7).to(BF).to(device) for h in (Hq, Hkv, Hkv))
+    table, loc, seq, rows = table.to(device), loc.to(device), torch.tensor(lens, dtype=torch.int32, device=device), torch.arange(1, B + 1, device=device)
+    fmt = dict(kv_fp8=True, k_scale=0.75, v_scale=1.25) if fp8 else {}
+    ws, got = kernels.CascadeWorkspace(B, Hq, D, width, device), []
+    for riding in (False, True):
+        kc, vc = (x.clone() for x in pools)
+        out = torch.zeros((B, Hq, D), dtype=BF, device=device)
+        kernels.cascade_plan(ws, table, rows, seq, Hq, Hkv, new_loc=loc)
+        if not riding:
+            # (of two rows with one slot a launch of both may leave either; the attention's own keeps the later one)
+            keep = slice(0, B) if without != "the_last_two_of_one_slot" else [b for b in range(B) if b != B - 2]
+            kernels.store_kv_cache(k[keep].contiguous(), v[keep].contiguous(), kc, vc, loc[keep].contiguous(), **(dict(num_kv_heads=Hkv, head_dim=D, **fmt) if fp8 else {}))
+        kernels.cascade_decode_attention(ws, q, kc, vc, out, table, rows, seq, D ** -0.5, **fmt, **(dict(new_rows=(k, v, loc)) if riding else {}))
+        got += [out, kc, vc]
+    assert all(torch.equal(a, b) for a, b in zip(got[:3], got[3:]))
+    words = 9 + 9 * B + 8 * ws.max_items + 769                        # cascade_plan_view (cascade_plan.hpp): ints in front of the pieces ...
+    words = (words + 3) // 4 * 4 + 8 * (B + 768) + B                 # ... and of what was found
+    bits = 0
+    for x in ws.plan[words:words + 64].tolist():
+        bits |= x
+    assert bits == found
+
+
+@pytest.mark.gpu
 def test_replays_with_other_slots(device):
     """A captured step whose slots, lengths and tables change between replays, among them to ones that meet and back."""
     from sglang_amd import kernels
