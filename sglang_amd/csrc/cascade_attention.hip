@@ -102,8 +102,9 @@ __device__ __forceinline__ T* global_ptr(T* x) {
 // ---- The rows of the step itself (sgl_amd_cascade_decode_attention_store).  A launch of their own in front of every layer's attention is little more than launch, so
 // each row is stored by the one unit of a kv head that reads it as its request's newest token: by every wave of the unit that reads it, before it does (the
 // accesses of a wave to one address complete in order, and what the other waves store is the same).  Nobody else reads the slot, unless a table holds
-// another row's new slot; the plan looks for that once a step (cascade_check_rows), and then every wave stores all rows of its kv head first, the later of two
-// with one slot.  The row of a request without tokens, which no unit reads, is stored by the first workgroup of its kv head.
+// another row's new slot; the plan looks for that once a step (cascade_check_rows), and then every wave stores the rows that it found first (put_rows_first), the later
+// of two with one slot; all rows, where the plan was not made for these slots.  The row of a request without tokens, which no unit reads, is stored by the first
+// workgroup of its kv head.
 // us of attention a step, store launch / this: 64 requests behind shared prefixes, 32 / 8 heads, 8 layers, 233 / 219; 37 of 0.9 to 5.1 k in e4m3, 4 layers,
 // 267 / 258; 21 of 180 in e4m3, 64 / 8 heads, 4 layers, 70 / 61.  What is left of the launch: 1 us a layer in units of 128 tokens (with nothing stored 209).
 struct NewRows {
@@ -118,7 +119,7 @@ struct StoreParams {
   NewRows rows;
 };
 constexpr int kNewest = -2, kOlder = -1;              // word 7 of a private item's or piece's record: it ends in the request's newest token, or not
-enum RowsToStore { kInPool = 0, kOwnRow = 1, kAllRows = 2 };
+enum RowsToStore { kInPool = 0, kOwnRow = 1, kMetRows = 2, kAllRows = 3 };
 
 // a lane's piece of request b's new rows of a kv head: asked for, stored (K by the first D / 8 lanes, V by the next)
 template <int D>
@@ -137,15 +138,32 @@ __device__ __forceinline__ void put_own_row(const ChunkParams& p, const NewRows&
   const int slot = static_cast<int>(rows.loc[b]);
   put_new_row<D, FP8>(p, rows, ask_new_row<D>(rows, b, kvh, lane), slot, kvh, lane);
 }
+// whether no later row of the step has request b's slot
+__device__ __forceinline__ bool latest_row(const ChunkParams& p, const NewRows& rows, const int b, const int lane) {
+  const int64_t slot = rows.loc[b];
+  bool again = false;
+#pragma clang loop unroll(disable)
+  for (int c = b + 1 + lane; c < p.batch; c += 64) again |= rows.loc[c] == slot;
+  return __ballot(again) == 0ull;
+}
+// In front of all units where others may read some rows, or the plan was made for other slots: the rows that the plan found, or all.  us a layer, a launch for
+// the rows / all of them in front of every unit / these: 64 requests of 1 k 52 / 107 / 59, 1024 of 300 304 / 16058 / 370.
 template <int D, bool FP8>
-__device__ __forceinline__ void put_all_rows(const ChunkParams& p, const NewRows& rows, const int kvh, const int lane) {
+__device__ __forceinline__ void put_rows_first(const ChunkParams& p, const NewRows& rows, const bool all, const int first_kvh, const int end_kvh, const int lane) {
+  const CascadePlanView pv = cascade_plan_view(p.plan, p.batch, p.max_items);
+  const bool found = pv.meet[lane] != 0;
 #pragma clang loop unroll(disable)
-  for (int b = 0; b < p.batch; ++b) {
-    const int64_t slot = rows.loc[b];
-    bool again = false;
+  for (int b0 = 0; b0 < p.batch; b0 += 32) {
+    uint32_t some = found ? pv.met_rows[32 * lane + (b0 >> 5)] : 0u;
+    for (int off = 32; off > 0; off >>= 1) some |= __shfl_xor(some, off, 64);
+    if (all) some = b0 + 32 <= p.batch ? ~0u : (1u << (p.batch - b0)) - 1u;
 #pragma clang loop unroll(disable)
-    for (int c = b + 1 + lane; c < p.batch; c += 64) again |= rows.loc[c] == slot;
-    if (__ballot(again) == 0ull) put_new_row<D, FP8>(p, rows, ask_new_row<D>(rows, b, kvh, lane), static_cast<int>(slot), kvh, lane);
+    for (uint32_t todo = __builtin_amdgcn_readfirstlane(some); todo != 0u; todo &= todo - 1u) {
+      const int b = b0 + __ffs(static_cast<int>(todo)) - 1;
+      if (!latest_row(p, rows, b, lane)) continue;
+#pragma clang loop unroll(disable)
+      for (int kvh = first_kvh; kvh < end_kvh; ++kvh) put_own_row<D, FP8>(p, rows, b, kvh, lane);
+    }
   }
 }
 
@@ -161,7 +179,7 @@ __device__ __forceinline__ void put_unread_rows(const ChunkParams& p, const NewR
   }
 }
 
-// Whether all rows have to be stored first: a table holds a new slot elsewhere, or the plan does not know these slots (every wave for itself).
+// Whether rows have to be stored first: a table holds a new slot elsewhere, or the plan does not know these slots (every wave for itself).
 // The first 64 requests' slots and the words are asked for by ask(), beside what else a kernel begins with: behind it they are a round trip of their own.
 struct RowsMeet {
   int word, planned, now;
@@ -173,12 +191,13 @@ struct RowsMeet {
     now = static_cast<int32_t>(rows.loc[first]);
   }
   __device__ __forceinline__ int answer(const ChunkParams& p, const NewRows& rows, const int lane) const {
-    bool meet = (word & kPlanMeet) | (planned != now);
+    bool other = (word & kPlanUntold) | (planned != now);
     if (p.batch > 64) {
       const CascadePlanView pv = cascade_plan_view(p.plan, p.batch, p.max_items);
-      for (int b = 64 + lane; b < p.batch; b += 64) meet |= pv.new_slots[b] != static_cast<int32_t>(rows.loc[b]);
+      for (int b = 64 + lane; b < p.batch; b += 64) other |= pv.new_slots[b] != static_cast<int32_t>(rows.loc[b]);
     }
-    return __ballot(meet) != 0ull ? kAllRows : kOwnRow;
+    if (__ballot(other | (word & kPlanMeet)) == 0ull) return kOwnRow;
+    return __ballot(other) != 0ull ? kAllRows : kMetRows;
   }
   __device__ __forceinline__ bool unread() const { return __ballot(word & kPlanUnread) != 0ull; }
 };
@@ -339,7 +358,8 @@ __device__ __forceinline__ void cascade_few_rows_unit(const ChunkParams& p, cons
   const unsigned char* vlane = img + vrow * (2 * D) + ((i16 >> 1) & 1) * 16 + (i16 & 1) * 8;
   // The newest token is in the last tile: its wave alone reads it, and stores it behind the requests for its first tile's rows where that is another one (in front
   // of them the wait for it was 4 us of a launch of 57).
-  const bool mine = STORE && store_rows == kOwnRow && __builtin_amdgcn_readfirstlane(rb.w) == kNewest && wid < tiles && ((tiles - 1 - wid) & 3) == 0;
+  bool mine = STORE && __builtin_amdgcn_readfirstlane(rb.w) == kNewest && wid < tiles && ((tiles - 1 - wid) & 3) == 0;
+  if (mine && store_rows != kOwnRow) mine = latest_row(p, new_rows, rec_x, lane);
   U4 own;
   if (mine) {
     if (tiles - 1 == wid) put_own_row<D, FP8>(p, new_rows, rec_x, kvh, lane);
@@ -455,7 +475,8 @@ __device__ __forceinline__ void cascade_chunk_loop(const ChunkParams& p, const N
   if constexpr (STORE) {
     asm volatile("" : "+v"(meet.word), "+v"(meet.planned), "+v"(meet.now));
     store_rows = __builtin_amdgcn_readfirstlane(meet.answer(p, *new_rows, threadIdx.x & 63));
-    if (meet.unread() && (store_rows == kOwnRow || n_units == 0) && w0 < p.num_kv_heads) put_unread_rows<D, FP8>(p, *new_rows, w0, threadIdx.x & 63);
+    if (store_rows != kOwnRow) put_rows_first<D, FP8>(p, *new_rows, store_rows == kAllRows, 0, p.num_kv_heads, threadIdx.x & 63);
+    else if (meet.unread() && w0 < p.num_kv_heads) put_unread_rows<D, FP8>(p, *new_rows, w0, threadIdx.x & 63);
   }
   // The kernel's one argument sits at the start of the kernarg segment; every pass re-reads it through an address the
   // compiler cannot see through, exactly as a fresh launch would (scalar loads, served by the scalar cache), and takes the
@@ -498,9 +519,6 @@ __device__ __forceinline__ void cascade_chunk_loop(const ChunkParams& p, const N
     const CascadePlanView pv = cascade_plan_view(pl.plan, pl.batch, pl.max_items);
     const int span = item - n_shared;
     const bool in_span = spans && span >= 0;                                  // (workgroup-uniform)
-    if constexpr (STORE) {
-      if (store_rows == kAllRows) put_all_rows<D, FP8>(pl, nr, kvh, tid & 63);
-    }
     const int32_t* rec = pv.items + 8 * item;
     if (in_span) {
       const int i = next > 0 ? next : __builtin_amdgcn_readfirstlane(pv.span_first[span]);
@@ -615,8 +633,9 @@ constexpr int kPlanOneLaunch = 16;
 // entries, which may share it.  Requests without tokens, whose row no unit would store, are found by the way.
 __device__ __forceinline__ void cascade_check_rows(const int32_t* req_to_token, int64_t r2t_stride, const int64_t* req_pool_indices, const int32_t* seq_lens,
                                                    const int64_t* new_loc, int batch, int checker, int checkers, uint32_t* bits0, uint32_t* bits1, int* slots,
-                                                   const CascadePlanView& pv) {
+                                                   uint32_t* met, const CascadePlanView& pv) {
   const int tid = threadIdx.x;
+  if (tid < kPlanMaxBatch / 32) met[tid] = 0u;
   for (int i = tid; i < 1024; i += kPlanThreads) bits0[i] = bits1[i] = 0u;
   __syncthreads();
   auto hash = [](uint32_t s) { return (s * 0x9e3779b1u) >> 17; };
@@ -634,19 +653,32 @@ __device__ __forceinline__ void cascade_check_rows(const int32_t* req_to_token, 
     }
   }
   __syncthreads();
-  auto among = [&](int s, int but) {
+  auto mark = [&](int b) { atomicOr(&met[b >> 5], 1u << (b & 31)); };
+  auto mark_rows_of = [&](int s, int but) {
     bool found = false;
-    for (int c = 0; c < batch; ++c) found |= slots[c] == s && c != but;
+    for (int c = 0; c < batch; ++c)
+      if (slots[c] == s && c != but) {
+        mark(c);
+        found = true;
+      }
     return found;
   };
 #pragma unroll
-  for (int i = 0; i < kPlanMaxBatch / kPlanThreads; ++i)
-    if (checker == 0 && seen[i] && slots[tid + i * kPlanThreads] != 0) meet |= among(slots[tid + i * kPlanThreads], tid + i * kPlanThreads);
+  for (int i = 0; i < kPlanMaxBatch / kPlanThreads; ++i) {
+    const int b = tid + i * kPlanThreads;
+    if (checker == 0 && seen[i] && slots[b] != 0 && mark_rows_of(slots[b], b)) {
+      mark(b);
+      meet = true;
+    }
+  }
   constexpr int kAhead = 8;
   for (int b = checker; b < batch; b += checkers) {
     const int32_t* row = req_to_token + req_pool_indices[b] * r2t_stride;
     const int len = seq_lens[b], own = slots[b];
-    unread |= len < 1;
+    if (len < 1 && tid == 0) {
+      mark(b);
+      unread = true;
+    }
     for (int t0 = tid; t0 < len; t0 += kAhead * kPlanThreads) {
       int s[kAhead];
 #pragma unroll
@@ -659,13 +691,14 @@ __device__ __forceinline__ void cascade_check_rows(const int32_t* req_to_token, 
         const uint32_t x = static_cast<uint32_t>(s[u]), h = hash(x);
         if ((bits0[(x & 32767u) >> 5] >> (x & 31u)) & (bits1[h >> 5] >> (h & 31u)) & 1u) {
           const bool newest = t0 + u * kPlanThreads >= len - 1;                  // (or behind it: that token again)
-          if (!(newest && s[u] == own) && among(s[u], -1)) meet = true;
+          if (!(newest && s[u] == own) && mark_rows_of(s[u], -1)) meet = true;
         }
       }
     }
   }
   const int found = (__syncthreads_or(meet) ? kPlanMeet : 0) | (__syncthreads_or(unread) ? kPlanUnread : 0);
   if (tid == 0) pv.meet[checker] = found;
+  if (found != 0 && tid < kPlanMaxBatch / 32) pv.met_rows[kPlanMaxBatch / 32 * checker + tid] = static_cast<int>(met[tid]);
 }
 
 template <bool ONE>
@@ -690,7 +723,7 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
   if (blockIdx.x > 0) {
     static_assert(kPlanMaxBatch == 1024, "the arrays hold 32768 bits");
     cascade_check_rows(req_to_token, r2t_stride, req_pool_indices, seq_lens, new_loc, batch, static_cast<int>(blockIdx.x) - 1, static_cast<int>(gridDim.x) - 1,
-                       reinterpret_cast<uint32_t*>(first_slot), reinterpret_cast<uint32_t*>(leader), grp_min, pv);
+                       reinterpret_cast<uint32_t*>(first_slot), reinterpret_cast<uint32_t*>(leader), grp_min, reinterpret_cast<uint32_t*>(grp_cnt), pv);
     return;
   }
   // members == 0 marks the end of the list for the one-workgroup-per-unit chunk kernel, whose grid never reaches beyond
@@ -831,8 +864,8 @@ __global__ __launch_bounds__(kPlanThreads) void cascade_plan_kernel(
     pv.header[2] = rows;
     pv.header[3] = n_shared_items;
   }
-  // (no word of a workgroup that looked: both bits where there are none, so that a plan without the slots says what one that found both says)
-  if (tid < kCheckers && tid >= static_cast<int>(gridDim.x) - 1) pv.meet[tid] = gridDim.x == 1 ? kPlanMeet | kPlanUnread : 0;
+  // (no word of a workgroup that looked)
+  if (tid < kCheckers && tid >= static_cast<int>(gridDim.x) - 1) pv.meet[tid] = gridDim.x == 1 ? kPlanUntold : 0;
   // ---- private chunks of every request, appended behind the shared items (block-wide exclusive scan) ----
   int mine = 0, sh = 0, len = 0;
   if (tid < batch) {

@@ -16,7 +16,8 @@
 //                        the items'; they stand in the place of the private items for the looping attention kernel
 //   compare[2 B]         scratch between the plan's two launches: leader of request b, its common prefix with the leader
 //   new_slots[B]         the slots that the plan was told the step's rows go to (if it was)
-//   meet[kCheckers]      what was found of them, a word of PlanFound bits a workgroup that looked (it was not told: both bits)
+//   meet[kCheckers]      what was found of them, a word of PlanFound bits a workgroup that looked (it was not told: kPlanUntold)
+//   met_rows[kCheckers * 32]  the rows of the step that such a workgroup found something of, a bit each, where its word is not 0
 #pragma once
 #include <stdint.h>
 
@@ -37,6 +38,7 @@ struct CascadePlanView {
   int32_t* pieces;
   int32_t* new_slots;
   int32_t* meet;
+  int32_t* met_rows;
 };
 
 // (span, kv head) units that a plan of spans aims at, the shared items taken off: three a compute unit.  The looping kernel's registers would
@@ -54,11 +56,11 @@ constexpr int kSpanUnits = 768;
 constexpr int kOneRoundUnits = 1024;
 constexpr int kMinSpanTiles = 3;
 constexpr int kCheckers = 64;        // workgroups that look through the request tables for the new slots, one word each
-enum PlanFound { kPlanMeet = 1, kPlanUnread = 2 };   // a request reads a new slot that is not its own newest token's, or two rows have one; a request has no tokens
+enum PlanFound { kPlanMeet = 1, kPlanUnread = 2, kPlanUntold = 4 };   // a request reads a new slot that is not its own newest token's, or two rows have one; a request has no tokens
 
 __host__ __device__ inline int64_t cascade_plan_ints(int64_t batch, int64_t max_items) {
   return 8 + batch + batch + (batch + 1) + batch + batch + 8 * max_items + batch + 2 * batch + batch + (kSpanUnits + 1) + 8 * (batch + kSpanUnits) + 3 + batch +
-         kCheckers;
+         kCheckers + kCheckers * 32;
 }
 
 __host__ __device__ inline CascadePlanView cascade_plan_view(const int32_t* plan, int64_t batch, int64_t max_items) {
@@ -78,6 +80,7 @@ __host__ __device__ inline CascadePlanView cascade_plan_view(const int32_t* plan
   v.pieces = v.header + ((p - v.header + 3) & ~static_cast<int64_t>(3));   // 16-byte records
   v.new_slots = v.pieces + 8 * (batch + kSpanUnits);
   v.meet = v.new_slots + batch;
+  v.met_rows = v.meet + kCheckers;
   return v;
 }
 
