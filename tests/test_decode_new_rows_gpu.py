@@ -183,7 +183,7 @@ def test_replays_with_other_slots(device):
         assert torch.equal(out, want) and torch.equal(kc, k1) and torch.equal(vc, v1), (n, meet)
 
 
-def _planned_slots(monkeypatch, pool, fb, **attrs):
+def _planned_slots(monkeypatch, pool, fb, requests=3, **attrs):
     """new_loc of the plan that a decode step of `fb` makes over `pool`."""
     from types import SimpleNamespace
 
@@ -191,7 +191,7 @@ def _planned_slots(monkeypatch, pool, fb, **attrs):
 
     b, got = H.HipAttnBackend.__new__(H.HipAttnBackend), []
     vars(b).update(token_to_kv_pool=pool, req_to_token_pool=SimpleNamespace(req_to_token=None), num_q_heads=8, num_kv_heads=2, _seq_src=None,
-                   forward_metadata=H._Meta(torch.ones(3, dtype=torch.int32), cascade=object()), **attrs)
+                   forward_metadata=H._Meta(torch.ones(requests, dtype=torch.int32), cascade=object()), **attrs)
     monkeypatch.setattr(H.kernels, "cascade_plan", lambda *a, new_loc=None, **k: got.append(new_loc))
     b.init_forward_metadata_in_graph(fb)
     assert b.forward_metadata.slots_planned == (got[0] is not None)
@@ -238,6 +238,7 @@ def test_the_plan_looks_only_where_a_layer_stores_with_it(monkeypatch, fp8, hnd,
     got = _planned_slots(monkeypatch, pool, fb, _brings_rows=lambda *a: models.CausalLM.brings_rows(model, *a))
     assert (got is loc) == looks
     assert (_planned_slots(monkeypatch, pool, fb) is loc) == (not hnd)      # a backend that is not told
+    assert (_planned_slots(monkeypatch, pool, fb, 512) is loc) == (not hnd) and _planned_slots(monkeypatch, pool, fb, 513) is None
 
 
 @pytest.mark.skipif(not Path(HIPCC).exists(), reason="hipcc not installed")
