@@ -1078,12 +1078,12 @@ __global__ __launch_bounds__(kT) void sample_finish_ranges_kernel(SampleParams p
 //   probabilities into a scratch matrix and runs the single-workgroup routine on them (no launch for rows that do not need it).
 // [64, 128256], top-k 50 / top-p 0.9: 16 MB read once from HBM instead of ~130 MB of traffic.  Same ids and kept counts as the
 // long way by construction (tests/test_sampler_gpu.py compares them on every row).
-// What bounds it: the candidates launch at many rows the vector instructions (45 a column, 18 of them the quotient and the exponential;
+// What bounds it: the candidates launch at many rows the vector instructions (47 a column, 20 of them the quotient and the exponential;
 // the matrix of 128 rows alone is 7 us of reading), at few rows, like the finish launch, a chain of dependent steps: 5 us until the
 // records and lists are there, 2.5 the cut, 1 the compaction, 3 rank, rules and arg-max.  us for the two launches, before this division
 // of the work (a true division per column, every column tested one by one for the list, byte-wide histograms, ranks, logs and noise all
 // by one wave) and now: [128, 128256] 53 / 41, [64, 128256] 42 / 32, [1, 128256] 34 / 23, [128, 32000] 43 / 29.  (A second
-// remainder step of the quotient and expf's test for overflow: the candidates launch 30.7 / 29.4.  Four columns tested for the list by their largest, the few
+// remainder step of the quotient: the candidates launch 30.6 / 30.0.  Four columns tested for the list by their largest, the few
 // that pass looked at again: 15 % fewer instructions, and the launch 1 us longer by the dependent reads.)
 constexpr int kFastRangesMax = 16;
 constexpr int kFastCap = 127;
@@ -1197,16 +1197,6 @@ __device__ __forceinline__ void select_bin_256(uint32_t c, uint32_t K, uint32_t*
   __syncthreads();
 }
 
-// expf for arguments that are not positive (or NaN), with expf's bits: 2^(x log2 e), the exponent as a product of two floats, without the test for
-// results beyond the floats (all 2^31 of them give expf's bits).
-__device__ __forceinline__ float exp_to_one(float x) {
-#pragma clang fp contract(off)
-  constexpr float kLog2e = 0x1.715476p+0f, kRest = 0x1.4ae0bep-26f;
-  const float p = x * kLog2e, rest = __builtin_fmaf(x, kRest, __builtin_fmaf(x, kLog2e, -p)), n = __builtin_rintf(p);
-  const float e = __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((p - n) + rest), static_cast<int>(n));
-  return x < -0x1.9d1da0p+6f ? 0.f : e;               // 0xc2ce8ed0: log 2^-149
-}
-
 constexpr int kFastSlots = 16;     // 1024-column steps of a workgroup's columns (4 per thread and step): <= 16384 columns
 
 // A workgroup's columns live in REGISTERS (one round trip to L2 / HBM for the whole range: a pass over them from memory cost
@@ -1318,8 +1308,7 @@ __global__ __launch_bounds__(kSplitThreads) void sample_logit_candidates_kernel(
   const bool by_rcp = !t_one && t >= 9.5367431640625e-7f && t <= 1048576.0f &&
                       __ballot(!(lo >= -1e30f && my_top <= 1e30f)) == 0ull;     // (wave-uniform; masked-out columns are -inf)
   const float rcp_t = 1.0f / t;
-  // (bf16 logits: the first step rounds correctly already, all 2^7 significands over all 2^23 of t were looked at:
-  // tests/test_sampler_quotient_host.py)
+  // (bf16 logits: the first step rounds correctly already, all 2^7 significands over all 2^23 of t: tests/test_sampler_quotient_host.py)
   auto over_t = [&](float v) {
     float d = v * rcp_t;
     d = __fmaf_rn(__fmaf_rn(-t, d, v), rcp_t, d);
@@ -1339,8 +1328,8 @@ __global__ __launch_bounds__(kSplitThreads) void sample_logit_candidates_kernel(
     if (s < slots && mx > -INFINITY) {                // (uniform)
       const float v0 = q[s].v(0), v1 = q[s].v(1), v2 = q[s].v(2), v3 = q[s].v(3);
       float add;
-      if (t_one) add = exp_to_one(v0 - mx) + exp_to_one(v1 - mx) + exp_to_one(v2 - mx) + exp_to_one(v3 - mx);
-      else if (by_rcp) add = exp_to_one(over_t(v0) - mx) + exp_to_one(over_t(v1) - mx) + exp_to_one(over_t(v2) - mx) + exp_to_one(over_t(v3) - mx);
+      if (t_one) add = expf(v0 - mx) + expf(v1 - mx) + expf(v2 - mx) + expf(v3 - mx);
+      else if (by_rcp) add = expf(over_t(v0) - mx) + expf(over_t(v1) - mx) + expf(over_t(v2) - mx) + expf(over_t(v3) - mx);
       else add = expf(v0 / t - mx) + expf(v1 / t - mx) + expf(v2 / t - mx) + expf(v3 / t - mx);
       if (is_on(s)) run += add;
     }
