@@ -1455,12 +1455,14 @@ def moe_sum_reduce(x: torch.Tensor, out: torch.Tensor, routed_scaling_factor: fl
 
 def choose_moe_block_m(num_pairs: int, num_experts: int) -> int:
     """Row-block height of the grouped GEMM: an expert whose rows spill into a second block streams its weights twice, padded rows cost next to nothing
-    (the kernel is bound by the weight stream): 16 rows for up to 6 an expert, 32 for up to 16, 48 for up to 32.  us, means of eight routings of uneven experts, the next
-    smaller block / this: 7 rows an expert on average, 8 experts of 14336 / 4096 420 / 418, of 7168 / 4096 226 / 221, 128 of 768 / 2048 220 / 209, 64 of 1408 / 2048 190 / 188; 10 rows 461 / 421, 230 / 222, 234 /
-    218, 205 / 193; 17 rows 438 / 439, 229 / 229, 243 / 236, 211 / 206; 21 rows 457 / 446, 247 / 232, 252 / 245, 227 / 213; one routing at worst 0.984 and at best 1.22 of the time.  Even
-    experts: at most 1.5 % more."""
+    (the kernel is bound by the weight stream): 16 rows for up to 7 an expert, 32 for up to 18, 48 for up to 32.  The next smaller block's time over this one's, even
+    experts / uneven ones of two kinds, three routings each: 8 experts of 14336 / 4096 with 8 rows an expert 1.000 / 1.002, 1.059, with 19 1.000 / 0.995, 0.998, with 21 0.993 / 0.996, 0.994; of
+    7168 / 4096 with 8 0.998 / 1.000, 1.049, with 19 0.991 / 0.992, 0.990, with 21 0.992 / 0.996, 1.067; 64 of 1408 / 2048 with 8 0.991 / 0.994, 1.027, with 19 0.983 / 0.980, 1.021, with 21 0.985 /
+    0.995, 1.041; 128 of 768 / 2048 with 8 0.996 / 1.014, 1.051, with 19 0.982 / 1.015, 1.043, with 21 0.987 / 1.018, 1.040; 16 of 2048 / 2048 with 8 0.996 / 0.992, 1.058, with 19 0.984 / 0.988, 1.135,
+    with 21 0.979 / 0.993, 1.087: padded rows are 1 to 2 % where nothing would spill.  Not from 7 and 17 rows on, where that is most of what the larger block does: 8 of 7168 / 4096 0.999 / 1.000,
+    1.000 and 0.995 / 0.991, 0.992, 16 of 2048 / 2048 0.987 / 0.987, 0.996 and 0.991 / 0.989, 1.035.  Without weights (routed_experts) the same within 1 %."""
     avg = (num_pairs + num_experts - 1) // max(1, num_experts)
-    for most, bm in ((6, 16), (16, 32), (32, 48)):
+    for most, bm in ((7, 16), (18, 32), (32, 48)):
         if avg <= most:
             return bm
     return 64

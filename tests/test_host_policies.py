@@ -95,16 +95,24 @@ def test_kernels_refuse_cpu_tensors():
         K.rmsnorm(x, torch.ones(256, dtype=torch.bfloat16), 1e-5)
 
 
-def test_moe_block_height_holds_one_and_a_half_average_experts():
+def test_moe_block_height_of_the_batches_it_was_made_for():
     """choose_moe_block_m: an expert whose rows spill into a second row block streams its weights twice."""
     assert K.choose_moe_block_m(2, 8) == 16            # one token, top-2
     assert K.choose_moe_block_m(32, 8) == 16           # 4 rows per expert on average
-    assert K.choose_moe_block_m(128, 8) == 32          # the 64-token Mixtral decode batch: 16 on average -> 24 -> 32
+    assert K.choose_moe_block_m(128, 8) == 32          # the 64-token Mixtral decode batch: 16 on average
     assert K.choose_moe_block_m(256, 8) == 48
     assert K.choose_moe_block_m(8192, 8) == 64
     for pairs in range(1, 600, 7):
         for experts in (4, 8, 64, 256):
             assert K.choose_moe_block_m(pairs, experts) in (16, 32, 48, 64)
+
+
+@pytest.mark.parametrize("experts", [4, 8, 64, 256])
+def test_moe_block_height_on_both_sides_of_its_lines(experts):
+    """Taller blocks from 8, 19 and 33 rows an expert on, the mean rounded up."""
+    for most, block, taller in ((7, 16, 32), (18, 32, 48), (32, 48, 64)):
+        assert K.choose_moe_block_m(most * experts, experts) == block
+        assert K.choose_moe_block_m(most * experts + 1, experts) == K.choose_moe_block_m((most + 1) * experts, experts) == taller
 
 
 def test_req_token_arrays():
