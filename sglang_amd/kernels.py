@@ -1260,7 +1260,8 @@ def moe_sum_parts(parts: torch.Tensor, splits: torch.Tensor, topk_weights: torch
 
 MOE_TILE_OVERRIDE = None                # tests / benchmarks: (align block, up tile rows, down tile rows)
 # From here on the row-tiled form: the weight-streaming one takes 64 rows at a time, and an expert with more reads its weights again.  us, both products,
-# streaming / 128-row tiles, two routings each: 8 experts of 14336 / 4096 with 48 rows 613 / 592, 600 / 575, with 60 710 / 595, 699 / 578, with 90 922 / 620,
+# streaming / 128-row tiles, two routings each, at sizes of which fused_experts now gives most to moe_weight_bound in front of this (what is left to it: routed_experts, fewer than 224 column
+# tiles, more than 256 row blocks): 8 experts of 14336 / 4096 with 48 rows 613 / 592, 600 / 575, with 60 710 / 595, 699 / 578, with 90 922 / 620,
 # 911 / 599; of 7168 / 4096 with 48 281 / 316, 271 / 309, with 70 400 / 326, 394 / 320; 64 of 1408 / 2048 with 48 287 / 282, 301 / 283, with 70 372 / 301.
 # Only from 96 rows on where the up projection has fewer than 256 such tiles: 4 experts of 1024 / 1024 with 58 to 76 rows 41 / 45.
 MOE_TILED_MIN_ROWS_PER_EXPERT, MOE_TILED_MIN_ROWS_FEW_TILES = 56, 96
@@ -1344,18 +1345,24 @@ MOE_PARTS_OVERRIDE = None               # tests / benchmarks: (most rows of a ti
 def moe_weight_bound(numel: int, num_experts: int, n_up: int, n_down: int):
     """(most rows of a tile, most parts of K of the down projection) where moe_rows_gemm takes both products of fused_experts; (320, 0): it doesn't.
     Tiles of 240 rows from 40 rows an expert on (below, the weight streams are quicker wherever no expert has more rows than their block: 33 rows 474 / 484) to 330, where products bound
-    both forms.  us, streams, 128-row tiles or 320-row tiles without parts / these, routings of uneven experts: 8 experts of 14336 / 4096 with 16 rows 443 / 478, 24 570 / 488, 32 594 / 492, 40 488 / 485, 64 586 /
-    502, 90 601 / 505, 130 832 / 561, 180 910 / 674, 240 955 / 830, 300 1006 / 977, 440 1261 / 1348; of 7168 / 4096 with 24 236 / 253, 32 249 / 254, 64 314 / 261, 130 397 / 294, 300 578 / 532, 360 599
-    / 600; of 3584 / 4096 (224 column tiles of the up projection, the line) with 24 124 / 129, 32 148 / 133, 130 219 / 173, 360 380 / 306, 440 423 / 418; 64 of 1408 / 2048 with 16 208 / 213, 32 234 /
-    224, 130 364 / 305, 360 606 / 560; 32 of 7168 / 4096 with 32 975 / 895, 130 1439 / 1215, 240 1716 / 1653, 300 1893 / 1926 (past 1024 column tiles 256 rows are the line); 128 of 768 / 2048 with
-    32 276 / 261, 240 605 / 536; 16 of 2048 / 2048 with 32 116 / 92, 130 154 / 138, 180 155 / 161, 300 227 / 192; 4 of 1024 / 1024 (32) with 130 46 / 51.
-    Tiles of 320 rows with the down projection in two parts from 480 rows on while that has up to two rounds of tiles and a long K: 8 of 14336 / 4096 with 440 1240 / 1231,
-    with 560 1651 / 1561, 750 1986 / 1942, 1000 2440 / 2386; of 7168 / 4096 with 750 1014 / 993, with 1000 1272 / 1297.
-    No more parts than give four rounds of tiles: another part is another fp32 copy of the rows; nor than the down projection's K has steps of 64."""
+    both forms.  us, streams, 128-row tiles or 320-row tiles without parts / these, means of routings of three kinds from nearly even to uneven: 8 experts of 14336 / 4096 with 40 rows 557 / 495, 60 618 /
+    515, 100 664 / 524, 130 824 / 589, 180 892 / 668, 245 960 / 819, 300 1027 / 901; of 7168 / 4096 with 40 280 / 258, 60 324 / 272, 130 409 / 317, 245 547 / 449, 328 579 / 535; of 3584 / 4096 (224 column
+    tiles of the up projection, the line) with 60 170 / 144, 130 229 / 180, 300 337 / 278, 395 406 / 335; 64 of 1408 / 2048 with 44 259 / 229, 130 373 / 304, 245 477 / 444, 395 656 / 596; 32 of 7168 / 4096
+    with 40 1013 / 911, 130 1468 / 1168, 220 1636 / 1512, 256 1760 / 1702 (even 1603 / 1654; past 1024 column tiles the line); 128 of 768 / 2048 with 40 291 / 261, 130 451 / 376, 245 615 / 566; 16 of 2048 /
+    2048 with 40 108 / 100, 130 152 / 122, 180 160 / 142, 300 220 / 190, 395 234 / 230; 16 of 2048 / 7168 with 40 292 / 270, 130 429 / 334, 395 704 / 649; 4 of 1024 / 1024 (32) with 130 46 / 51.
+    From 50 rows on where few experts have few column tiles or a down projection has a short K: 8 of 4096 / 6144 with 40 237 / 235 (even 229 / 233), 48 246 / 238 (even 231 / 235), 60 299 / 229; 96 of 384 /
+    4096 with 40 244 / 239 (even 236 / 247), 48 264 / 253 (even 245 / 253), 60 293 / 267, 245 713 / 528.
+    Tiles of 320 rows with the down projection in two parts from 480 rows on while that has up to two rounds of tiles and a long K: 8 of 14336 / 4096 with 480 1389 / 1332, 640 1828 / 1671, 800 2059 /
+    1983, 1280 3086 / 3073; of 10240 / 4096 with 480 949 / 940, 640 1307 / 1223, 960 1709 / 1696; of 16384 / 6144 with 480 2349 / 2152, 640 2827 / 2778; of 12288 / 8192 with 480 2158 / 2141; of 14336 / 2048 with 480
+    856 / 754 (uneven 881 / 897), 960 1280 / 1269; 16 of 8192 / 4096 with 480 1596 / 1564; of 8192 / 2048 with 640 1166 / 1082, 1280 1960 / 1930; 4 of 20480 / 4096 with 480 1100 / 887, 640 1281 / 1289, 1280 2416 /
+    2191; not of 7168 / 4096: with 750 1014 / 993, with 1000 1272 / 1297.
+    No more parts than give four rounds of tiles: another part is another fp32 copy of the rows, with tiles of 240 some 250 MB in all where there are two parts or more, with tiles of 320 336 MB; nor than the
+    down projection's K has steps of 64."""
     rows, col_tiles, down = numel / max(1, num_experts), num_experts * -(-n_up // 128), num_experts * -(-n_down // 256)
     blocks = (numel + (num_experts + 1) * 255 + 255) // 256      # moe_align_block_size's
     most = 256 if col_tiles > 1024 else 330 if n_up * n_down > 1 << 24 else 400
-    if blocks <= 256 and col_tiles >= 224 and 40 <= rows <= most:
+    least = 50 if n_up < 768 or (num_experts <= 8 and col_tiles < 448) else 40
+    if blocks <= 256 and col_tiles >= 224 and least <= rows <= most:
         return 240, max(1, min(4, n_up // 64, 1024 // (down * -(-int(rows) // 240))))
     if rows >= 480 and n_up >= 8192 and col_tiles >= 640 and down * -(-int(rows) // 320) <= 512:
         return 320, 2

@@ -19,6 +19,26 @@ def test_where_these_tiles_are_taken():
         assert K.moe_weight_bound(pairs, experts, up, down) == (320, 0)
 
 
+def test_from_how_many_rows_on():
+    """Few column tiles of few experts, and a short K of the down projection, from 50 rows an expert on; others from 40."""
+    for experts, up, down, least in ((8, 4096, 6144, 50), (8, 3584, 4096, 50), (96, 384, 4096, 50), (16, 2048, 7168, 40), (16, 2048, 2048, 40), (4, 14336, 4096, 40), (60, 1408, 2048, 40)):
+        assert K.moe_weight_bound((least - 1) * experts, experts, up, down)[1] == 0 and K.moe_weight_bound(least * experts, experts, up, down)[0] == 240
+
+
+def test_copies_of_the_rows_are_bounded():
+    """fp32 copies that the parts of the down projection take: 256 MiB with tiles of 240 rows, 320 with tiles of 320; one copy, as the other tiles have, without a bound."""
+    seen = set()
+    for experts in (4, 8, 16, 32, 64, 100, 128, 200):
+        for up in (384, 768, 1408, 2048, 4096, 7168, 8192, 14336, 20480):
+            for down in (1024, 2048, 4096, 6144, 8192):
+                for rows in (40, 56, 130, 240, 241, 330, 400, 480, 481, 640, 960, 1280):
+                    most, parts = K.moe_weight_bound(rows * experts, experts, up, down)
+                    if parts > 1:
+                        seen.add((most, parts))
+                        assert parts * rows * experts * down * 4 <= (256 if most == 240 else 320) << 20, (experts, up, down, rows)
+    assert {(240, 2), (240, 4), (320, 2)} <= seen
+
+
 def test_no_more_parts_than_steps():
     """A part of K has a step of 64 at least (sgl_amd_moe_rows_gemm refuses others): intermediate sizes of few steps over all that the rule takes."""
     taken = 0
