@@ -77,6 +77,22 @@ def _pairs(loads, topk, g):
     return ids[torch.randperm(ids.numel(), generator=g)].to(torch.int32).view(-1, topk).cuda()
 
 
+def _estimate(loads, N, Kd, most, max_parts, gated):
+    """(parts of K, tiles of a part) that the kernel chooses for a product: the number of units of 16 rows and of parts whose rounds of tiles over 256 compute units take least."""
+    best, nk, cols = None, Kd // 64, -(-N // (128 if gated else 256))
+    units = [-(-n // 16) for n in loads if n]
+    for m in range(most // 16, most // 32 - 1, -1):
+        tiles = [-(-u // m) for u in units]
+        fullest = max(-(-u // t) for u, t in zip(units, tiles))
+        step = max(12 + fullest * 3 // 4 if most == 240 else 24, fullest + 9)
+        for n in range(1, max(1, max_parts) + 1):
+            rounds = -(-sum(tiles) * cols * n // 256)
+            cost = rounds * -(-nk // n) * step + (n - 1) * int(3e-5 * sum(loads) * N) if max_parts else rounds * step
+            if best is None or cost < best[0]:
+                best = cost, n, sum(tiles) * cols
+    return best[1:]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("most", [240, 320])
 @pytest.mark.parametrize("loads,N,Kd", [((1, 16, 17, 0), 64, 64), ((239, 240, 241, 2), 320, 128), ((15, 241, 480, 481), 288, 192), ((225, 224, 0, 33), 576, 512),
@@ -111,7 +127,7 @@ def test_products_of_few_rows(most, loads, N, Kd):
         splits = torch.zeros(1, dtype=torch.int32, device="cuda")
         K.moe_rows_gemm(x, w2, parts, s, e, post, topk, numel, most, splits=splits)
         n = int(splits)
-        assert 1 <= n <= most_parts
+        assert n == _estimate(loads, N, Kd, most, most_parts, False)[0] and (n > 1 or most_parts == 1)
         assert bool(((parts[:n].double().sum(0) - want).abs() <= bound).all())
         out = torch.empty((M, N), dtype=BF, device="cuda")
         K.moe_sum_parts(parts, splits, tw, out, 0.5)
@@ -122,6 +138,65 @@ def test_products_of_few_rows(most, loads, N, Kd):
         for k in range(topk):
             acc += total.to(BF).float().view(M, topk, N)[:, k] * tw[:, k:k + 1]
         assert torch.equal(out, (acc * 0.5).to(BF))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("most", [240, 320])
+@pytest.mark.parametrize("loads,N,Kd,cut", [((500, 3, 239, 241, 0, 322, 97, 16), 9024, 64, False), ((500, 3, 239, 241, 0, 322, 97, 16), 9024, 128, False),
+                                            ((130, 641, 33, 0, 240, 480, 15, 320), 9024, 192, False), ((700, 650, 0, 5, 720), 9220, 448, False),
+                                            ((30, 17, 0, 48, 16, 5), 7684, 4160, True), ((100, 17, 260, 0, 48, 5), 6404, 4160, True)])
+def test_workgroups_that_take_several_tiles(most, loads, N, Kd, cut):
+    """More tiles than compute units, of uneven experts and of output columns that fill no tile: the next tile's stages behind steps of one, two and three and of odd counts, and from a
+    part of K to the next, which is not as long."""
+    g = torch.Generator(device="cuda").manual_seed(sum(loads) + N + Kd)
+    E, numel = len(loads), sum(loads)
+    ids = _pairs(loads, 1, torch.Generator().manual_seed(numel))
+    flat = ids.flatten().long()
+    s, e, post = K.moe_align_block_size(ids, 256, E)
+    x = torch.randn((numel, Kd), generator=g, device="cuda").to(BF)
+    if N % 32 == 0:
+        parts, tiles = _estimate(loads, N, Kd, most, 0, True)
+        assert tiles > 256
+        w13 = (torch.randn((E, 2 * N, Kd), generator=g, device="cuda") * 0.05).to(BF)
+        up = torch.empty((numel, N), dtype=BF, device="cuda")
+        K.moe_rows_gemm(x, w13, up, s, e, post, 1, numel, most, act=K.SILU)
+        for i in range(E):
+            gu = x[flat == i].double() @ w13[i].double().T.contiguous()
+            want = torch.nn.functional.silu(gu[:, :N]) * gu[:, N:]
+            assert bool(((up[flat == i].double() - want).abs() <= 2.0 ** -6 * want.abs() + 1e-3).all()), i
+        del w13
+    w2 = (torch.randn((E, N, Kd), generator=g, device="cuda") * 0.05).to(BF)
+    most_parts = min(4, Kd // 64)
+    out = torch.full((most_parts, numel, N), float("nan"), device="cuda")
+    splits = torch.zeros(1, dtype=torch.int32, device="cuda")
+    K.moe_rows_gemm(x, w2, out, s, e, post, 1, numel, most, splits=splits)
+    n = int(splits)
+    want_n, tiles = _estimate(loads, N, Kd, most, most_parts, False)
+    assert n == want_n and tiles * n > 256 and (n > 1) == cut, (n, want_n, tiles)
+    got = out[:n].double().sum(0)
+    for i in range(E):
+        a, w = x[flat == i].double(), w2[i].double().T.contiguous()
+        assert bool(((got[flat == i] - a @ w).abs() <= a.abs() @ w.abs() * (Kd + 4) * 2.0 ** -24).all()), i
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,E,N,H,plan", [(520, 8, 7168, 1024, (240, 4)), (2003, 8, 10240, 512, (320, 2)), (1530, 16, 2048, 768, (240, 4))])
+def test_layers_that_take_these_tiles(M, E, N, H, plan):
+    """fused_experts by its own rule, against 64 bits."""
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn((M, H), generator=g, device="cuda").to(BF)
+    w13, w2 = (torch.randn((E, 2 * N, H), generator=g, device="cuda") * 0.03).to(BF), (torch.randn((E, H, N), generator=g, device="cuda") * 0.03).to(BF)
+    tw, ids = (torch.randn((M, E), generator=g, device="cuda") + torch.randn((1, E), generator=g, device="cuda") * 0.5).softmax(-1).topk(2)
+    tw, ids = tw.float().contiguous(), ids.int().contiguous()
+    assert K.moe_weight_bound(2 * M, E, N, H) == plan
+    got, want = K.fused_experts(x, w13, w2, tw, ids, 0.5), torch.zeros((M, H), dtype=torch.float64, device="cuda")
+    for i in range(E):
+        tok, k = (ids == i).nonzero(as_tuple=True)
+        gu = x[tok].double() @ w13[i].double().T.contiguous()
+        want.index_add_(0, tok, (torch.nn.functional.silu(gu[:, :N]) * gu[:, N:]) @ w2[i].double().T.contiguous() * tw[tok, k].double()[:, None] * 0.5)
+    # bf16 roundings of gate and activation, of their product, of a pair's row and of the result, 2^-9 each
+    assert float((got.double() - want).norm() / want.norm()) < 5 * 2.0 ** -9
+    assert torch.equal(got, K.fused_experts(x, w13, w2, tw, ids, 0.5))
 
 
 @pytest.mark.gpu

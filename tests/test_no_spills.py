@@ -115,10 +115,31 @@ def test_moe_256_tile_kernel_keeps_its_registers_and_lds(tmp_path):
     for name, u in rows.items():
         assert u["vgpr_spill_count"] == 0 and u["sgpr_spill_count"] <= 36 and u["vgpr_count"] <= 256, (name, u)
         assert u["group_segment_fixed_size"] == 160 * 1024, (name, u)
+    # moe_weight_bound_kernel: the same walk from another place of K in each XCD, tiles of 240 (three stages of weights) or 320 rows, outputs or parts of K.  Two of the four park 43 scalars
+    bound = {k: v for k, v in usage.items() if "moe_weight_bound_kernel" in k}
+    assert len(bound) == 4, sorted(usage)
+    for name, u in bound.items():
+        assert u["vgpr_spill_count"] == 0 and u["sgpr_spill_count"] <= (43 if "ELb0E" in name else 19), (name, u)
+        assert u["vgpr_count"] <= (224 if "ILi15E" in name else 256) and u["group_segment_fixed_size"] == 160 * 1024, (name, u)
     k128 = {k: v for k, v in usage.items() if "moe_tiled_gemm_kernel" in k}
     assert len(k128) == 1
     for name, u in k128.items():
         assert u["vgpr_spill_count"] == 0 and u["sgpr_spill_count"] == 0 and u["vgpr_count"] <= 128, (name, u)   # two workgroups per CU
+
+
+@pytest.mark.skipif(not Path(HIPCC).exists(), reason="hipcc not installed")
+def test_expert_walks_move_no_parked_scalars(tmp_path):
+    """Scalars parked in lanes of vector registers are fetched between tiles, none of them between a walk's products: no block with products moves a lane."""
+    out = tmp_path / "k.s"
+    res = subprocess.run([HIPCC, *HIPCC_FLAGS, f"-I{ROOT / 'include'}", "--cuda-device-only", "-S", str(ROOT / "sglang_amd" / "csrc" / "moe_tiled_gemm.hip"), "-o", str(out)],
+                         capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr[-2000:]
+    kernels = re.findall(r"^(_ZN\S*(?:moe_rows_kernel|moe_weight_bound_kernel)\S*):[^\n]*\n(.*?)^\.Lfunc_end", out.read_text(), re.S | re.M)
+    assert len(kernels) == 5
+    for name, body in kernels:
+        walks = [b for b in re.split(r"^\.LBB\S+:.*$", body, flags=re.M) if "v_mfma" in b]
+        assert len(walks) == (8 if "ILi15E" in name else 10), name
+        assert not any("v_readlane" in b or "v_writelane" in b for b in walks), name
 
 
 @pytest.mark.skipif(not Path(HIPCC).exists(), reason="hipcc not installed")
