@@ -536,12 +536,12 @@ __device__ __forceinline__ u32x4_t lds_quad(uint32_t addr) {
 // ahead as well, 160 rows a tile: no faster).  And all workgroups at one place of K read rows 8 KiB apart, which few memory channels hold: an XCD's workgroups begin
 // an eighth of K behind those of the XCD in front (a place for each column tile: token rows then miss L2, 1000 tokens 860 -> 888;
 // with 320-row tiles an eighth takes 1 %: 1700 tokens 1220 -> 1209, 3000 1924 -> 1902).
-// Weights that one tile alone reads stay out of the caches (nt): 200 tokens 541 -> 502, 441 587 -> 548, 800 783 -> 766; for all tiles 1000 851 -> 867.
+// Weights that one tile alone reads stay out of the caches (nt): 200 tokens 532 -> 493, 441 567 -> 532, 800 738 -> 726; for all tiles 1000 851 -> 867.
 // PARTS: the down projection of few rows has fewer tiles than there are compute units (8 experts, 16 column tiles of 4096: 128) and the longest K.  K is cut into
 // up to max_splits parts, as many as make the rounds of parts shortest, by the same estimate as the tiles; their sums are left in fp32, and moe_sum_parts
 // adds them, rounds and weighs as the epilogue here would have.
-// us, both products of 8 experts of 14336 / 4096, 128-row tiles or 320 / PARTS with 320 / three stages / and the turn / and nt: 441 tokens 734 / 692 / 621 / 567 / 560,
-// 640 873 / 739 / 657 / 656 / 634, 1000 947 / 880 / 862 / 860 / 860.  The weights alone are 428 us.
+// us, both products of 8 experts of 14336 / 4096, 128-row tiles or 320 / PARTS with 320 / three stages / and the turn / and nt: 441 tokens 734 / 692 / 621 / 567 / 532,
+// 640 873 / 739 / 657 / 649 / 627, 1000 947 / 880 / 862 / 865 / 860.  The weights alone are 428 us.
 __global__ __launch_bounds__(kThreads2, 1) void moe_rows_kernel(TiledParams p) {
   constexpr int UNITS = kWholeUnits;
   constexpr bool PARTS = false, TURN = false;          // (its sums are those of the 128-row tiles, bit by bit)
