@@ -105,8 +105,8 @@ __device__ __forceinline__ T* global_ptr(T* x) {
 // another row's new slot; the plan looks for that once a step (cascade_check_rows), and then every wave stores the rows that it found first (put_rows_first), the later
 // of two with one slot; all rows, where the plan was not made for these slots.  The row of a request without tokens, which no unit reads, is stored by the first
 // workgroup of its kv head.
-// us of attention a step, store launch / this: 64 requests behind shared prefixes, 32 / 8 heads, 8 layers, 233 / 219; 37 of 0.9 to 5.1 k in e4m3, 4 layers,
-// 267 / 258; 21 of 180 in e4m3, 64 / 8 heads, 4 layers, 70 / 61.  What is left of the launch: 1 us a layer in units of 128 tokens (with nothing stored 209).
+// us of attention a step, store launch / this: 64 requests behind shared prefixes, 32 / 8 heads, 8 layers, 232 / 215; 37 of 0.9 to 5.1 k in e4m3, 4 layers,
+// 266 / 256; 21 of 180 in e4m3, 64 / 8 heads, 4 layers, 70 / 61.  What is left of the launch: 0.8 us a layer in units of 128 tokens (with nothing stored 209).
 struct NewRows {
   const uint16_t* k;            // [B, Hkv, D]
   const uint16_t* v;
